@@ -1,89 +1,150 @@
 // Stages 4 and 5a for gfx950: per-tile alpha blending, forward (front to back) and backward
-// (back to front).  Sorted entries are gathered into LDS in batches as two float4 arrays plus
-// one float array, so an entry costs two 128-bit and one 32-bit LDS broadcast read.
+// (back to front).
+//
+// Both directions are bound by the issue of vector instructions, so what counts is how many a (pixel, entry)
+// pair costs and how many pairs are looked at that need not be.  1920x1080 unless noted, us, before (every
+// wavefront walks one list for its 256 pixels) -> now:
+//   forward   2 M faint Gaussians 1097 -> 830, 1.4 M at 1557x1038 384 -> 307, 500 K opaque 130 -> 127,
+//             6 M at 3840x2160 488 -> 450, 16 K at 256x256 58 -> 34
+//   backward  2 M faint 2215 -> 1590, 1.4 M at 1557x1038 658 -> 514, 500 K opaque 251 -> 221, 50 K at 512x512 136 -> 77
 #include "dsx_common.h"
 
 #include <atomic>
+#include <climits>
 #include <cstdlib>
 
 namespace dsx
 {
 
-constexpr float kAlphaThreshold = 1.0f / 255.0f;
-
-// exp through the hardware base-2 exponential (the reference is built with fast-math).  The factor
-// log2(e) is applied to the finished exponent, per pixel: folded into the conic coefficients when an
-// entry is staged it would save that multiply, but every term of the quadratic form would carry one
-// more rounding, and where the terms are large and cancel (thin, long splats far from their centre)
-// the image then moves 1.6 times as far from the reference's as it does now.
-__device__ __forceinline__ float fast_exp(float x)
-{
-    return __builtin_amdgcn_exp2f(x * 1.4426950408889634f);
-}
-
-// The exponent of a splat at a pixel, -1/2 (a dx^2 + c dy^2) - b dx dy with d = pixel - mean, in
-// ONE fixed sequence of roundings (explicit fused multiply-adds, no contraction left to the
-// compiler): the forward and the backward kernel must get the same bits, because both compare the
-// resulting alpha with 1/255 on their own.  If they disagreed on a borderline entry, the backward
-// would rebuild the transmittance of every entry in front of it from a final value that does
-// (or does not) contain its factor: an error of alpha in all their gradients at that pixel.
-// (The halves are taken by the caller: a_half = -a/2 and c_half = c/2, exact scalings, so it does
-// not matter to the bits whether they are applied per entry or once when the entry is staged.)
+// The exponent of a splat at a pixel is -sigma, sigma = 1/2 (a dx^2 + c dy^2) + b dx dy with d = pixel -
+// mean, computed in ONE fixed sequence of roundings (explicit fused multiply-adds, no contraction
+// left to the compiler): the forward and the backward kernel must get the same bits, because both
+// decide on their own whether the splat's alpha reaches 1/255 at the pixel.  If they disagreed on a
+// borderline entry, the backward would rebuild the transmittance of every entry in front of it from a
+// final value that does (or does not) contain its factor: an error of alpha in all their gradients
+// at that pixel.
+//   ax = 1/2 a dx^2, bx = b dx; sigma = (c/2 dy + bx) dy + ax
+// (the halves are exact scalings, taken once when the entry is staged; the forward stages -a/2 and takes
+// -sigma = ax - (c/2 dy + bx) dy: the same bits but for the sign)
 struct ExponentX
 {
-    float ax, bx; // -1/2 a dx^2 and b dx
+    float ax, bx;
 };
 __device__ __forceinline__ ExponentX exponent_x(float a_half, float b, float dx)
 {
 #pragma clang fp contract(off)
     ExponentX r;
     r.bx = b * dx;
-    r.ax = a_half * dx * dx;
+    // (the same rounding as the plain product; a product that is zero becomes +0, never -0)
+    r.ax = __builtin_fmaf(a_half * dx, dx, 0.0f);
     return r;
 }
-__device__ __forceinline__ float exponent_xy(ExponentX x, float c_half, float dy)
+
+// alpha = opacity exp(-sigma) through the hardware base-2 exponential (the reference is built with
+// fast-math), with the opacity as a term of its argument: one fused multiply-add instead of a product
+// before and a product after it.  log2(e) stays a factor of the finished exponent: folded into the
+// conic when an entry is staged it would put one more rounding on every term of the quadratic form, and
+// where the terms are large and cancel (thin, long splats far from their centre) the image would move
+// 1.6 times as far from the reference's as it does.
+constexpr float kLog2E = 1.4426950408889634f;
+constexpr float kLn2 = 0.6931471805599453f;
+constexpr float kLog2Of255 = 7.994353436858858f;
+
+// What an entry's opacity is staged as.
+struct StagedOpacity
+{
+    float log2;  // log2(opacity)
+    // largest sigma with alpha >= 1/255, about ln(255 opacity): the test of alpha is taken on sigma, before
+    // the exponential and with the same bits in both directions
+    float reach;
+};
+// The reach is found as the last float for which opacity * exp2(-sigma log2(e)), evaluated just so, passes: an
+// estimate from the logarithm, one Newton step on that expression, and a bisection of the eight floats around
+// it.  (The logarithm's own rounding alone would move the line between in and out by two or three floats, and with
+// it a few hundred of the 10^9 decisions of a large scene.)
+__device__ __forceinline__ StagedOpacity stage_opacity(float opacity)
 {
 #pragma clang fp contract(off)
-    const float inner = __builtin_fmaf(c_half, dy, x.bx);
-    return __builtin_fmaf(-inner, dy, x.ax);
+    StagedOpacity s;
+    s.log2 = __builtin_amdgcn_logf(opacity);
+    s.reach = (s.log2 + kLog2Of255) * kLn2; // NaN for a negative opacity, and for a NaN
+    auto alpha_at = [&](float sigma) { return opacity * __builtin_amdgcn_exp2f(-sigma * kLog2E); };
+    s.reach += __builtin_fmaf(alpha_at(s.reach), 255.0f, -1.0f);
+    int bits = __float_as_int(s.reach) - 4;
+#pragma unroll
+    for(int step = 4; step > 0; step >>= 1)
+        bits += alpha_at(__int_as_float(bits + step)) >= 1.0f / 255.0f ? step : 0;
+    s.reach = s.reach > 1e-3f ? __int_as_float(bits) : s.reach;
+    return s;
+}
+// Both tests of an entry at a pixel, that sigma has the right sign and that it does not exceed the reach,
+// in one integer compare: the bits of floats of one sign are ordered like their magnitudes.
+// Forward (the reference drops sigma <= 0): the bits of -sigma as a signed number are below zero only if
+// sigma > 0, and grow with it: they must not exceed those of -reach.  -sigma is never -0 (ax is not, and an
+// exact cancellation gives +0).  A NaN of either sign lies above every limit.  (A NaN opacity gives alpha =
+// 0.999 wherever sigma > 0, as in the reference, whose fminf drops the NaN; what is below 1/255, nowhere.)
+__device__ __forceinline__ int reach_limit_fwd(float opacity, float reach)
+{
+    return reach > 0.0f ? __float_as_int(-reach) : (opacity != opacity ? __float_as_int(-__builtin_inff()) : INT_MIN);
+}
+// Backward (which drops sigma < 0 only): the bits of sigma as an unsigned number, up to those of reach.
+__device__ __forceinline__ uint32_t reach_limit_bwd(float opacity, float reach)
+{
+    return reach >= 0.0f ? __float_as_uint(reach) : (opacity != opacity ? 0x7f800000u : 0u);
 }
 
-// Can this entry reach alpha >= 1/255 at ANY pixel of the tile?  The exponent's quadratic form
-// q(d) = 1/2 (a dx^2 + c dy^2) + b dx dy is convex, so its minimum over the box of pixel
-// centres is 0 if the centre lies inside and otherwise sits on one of the four edges, where it
-// is a clamped one-dimensional parabola.  An entry is dropped only if opacity * exp(-qmin)
-// stays below 0.99/255 (one percent of slack against rounding); whatever fails a comparison
-// (NaN, degenerate conic) is kept.  The reference's tile rectangle is the bounding square of a
-// 3-sigma circle, so about half of the (tile, entry) pairs a tile walks touch none of its pixels.
-__device__ __forceinline__ float edge_min(float a, float b, float c, float u, float v0, float v1)
+// The pixels of a wavefront, as four square blocks of kSide x kSide: 8 x 8 (a whole tile, four pixels per
+// lane) or 4 x 4 (a quarter of a tile, one pixel per lane).  Row r of the wavefront's lanes (16 lanes, a
+// DPP row) owns block r and walks ITS OWN list of entries: the four rows blend four different
+// entries at the same time.  An entry of a tile's list that touches the tile at all touches only part of
+// it (dense: 2.5 of its four 8 x 8 blocks, cfg2: 3.2), so a wavefront that walks one list for all
+// of its pixels spends up to half of its lanes on pixels that the entry cannot reach; skipping those
+// on the scalar unit costs as much as it saves, while giving the lanes another entry costs two address
+// instructions.  The rows wait for each other only once per round of staged entries.
+//
+// Which of the four blocks can this entry reach with alpha >= 1/255?  The exponent's quadratic form
+// q(d) = 1/2 (a dx^2 + c dy^2) + b dx dy is convex, so its minimum over a block's box of pixel
+// centres is 0 if the splat's centre lies inside and otherwise sits on an edge that faces the centre,
+// where it is a clamped one-dimensional parabola.  Taking the column and the row of the box that lie nearest to
+// the centre covers both: they are the facing edges where there are any (and points of the box where not).
+// A block is left out only if qmin exceeds the entry's reach by more than 0.01 (one percent of alpha, as slack
+// against rounding); an entry with a degenerate conic or without a limit is kept for all.
+// (x0, y0: the first pixel centre of block 0; bit r of the result: block r, x first)
+template <int kSide>
+__device__ __forceinline__ uint32_t blocks_reached(float mx, float my, float a, float b, float c, float reach,
+                                                   float x0, float y0)
 {
-    // minimum over v in [v0, v1] of 1/2 (a u^2 + c v^2) + b u v   (u fixed, c > 0)
-    const float v = fminf(v1, fmaxf(v0, -b * u * __builtin_amdgcn_rcpf(c)));
-    return 0.5f * (a * u * u + c * v * v) + b * u * v;
-}
-
-// (span_y: last row of pixel centres of the box, 15 for a whole tile, 3 for a band of four rows)
-__device__ __forceinline__ bool entry_reaches_tile(float mx, float my, float a, float b, float c, float opacity,
-                                                   float box_x0, float box_y0, float span_y = 15.0f)
-{
-    const float dx0 = box_x0 - mx, dx1 = box_x0 + 15.0f - mx;
-    const float dy0 = box_y0 - my, dy1 = box_y0 + span_y - my;
-    const bool inside = dx0 <= 0.0f && dx1 >= 0.0f && dy0 <= 0.0f && dy1 >= 0.0f;
-    float qmin = fminf(fminf(edge_min(a, b, c, dx0, dy0, dy1), edge_min(a, b, c, dx1, dy0, dy1)),
-                       fminf(edge_min(c, b, a, dy0, dx0, dx1), edge_min(c, b, a, dy1, dx0, dx1)));
-    qmin = inside ? 0.0f : qmin;
+    const float half_a = 0.5f * a, half_c = 0.5f * c;
+    const float to_v = -b * __builtin_amdgcn_rcpf(c), to_u = -b * __builtin_amdgcn_rcpf(a);
+    const float limit = reach + 0.01f;
     const bool well_formed = a > 0.0f && c > 0.0f;
-    const float limit = __logf(opacity * (255.0f / 0.99f)); // ln(opacity / (0.99/255))
-    return !(well_formed && qmin > limit);
+    const float u_first = x0 - mx, v_first = y0 - my;
+    uint32_t reached = 0;
+    // (a loop, not unrolled: what the blocks could share would hold two dozen registers where few are free)
+#pragma unroll 1
+    for(int r = 0; r < 4; ++r)
+    {
+        const float u0 = u_first + (float)((r & 1) * kSide), v0 = v_first + (float)((r >> 1) * kSide);
+        const float u1 = u0 + (float)(kSide - 1), v1 = v0 + (float)(kSide - 1);
+        const float un = __builtin_amdgcn_fmed3f(0.0f, u0, u1), vn = __builtin_amdgcn_fmed3f(0.0f, v0, v1);
+        // along the nearest column, and along the nearest row
+        const float v = __builtin_amdgcn_fmed3f(to_v * un, v0, v1);
+        const float u = __builtin_amdgcn_fmed3f(to_u * vn, u0, u1);
+        const float qmin = fminf(v * (half_c * v + b * un) + half_a * un * un, u * (half_a * u + b * vn) + half_c * vn * vn);
+        reached |= (well_formed && qmin > limit) ? 0u : 1u << r;
+    }
+    return reached;
 }
 
 // Pixels per lane of the blend kernels: 4 (one wavefront per tile) when the image has enough tiles
-// to occupy the chip (8 wavefronts on each of 1024 SIMDs), else 1 (four wavefronts per tile: more
-// instructions in all, but four times as many wavefronts).  Measured crossover (500 K Gaussians,
-// 640x480 to 1920x1080): about 5000 tiles for the forward, 1600 for the backward, whose
-// one-pixel form also quadruples the atomics.  dsx_set_blend_pixels_per_lane(1 | 4) overrides the
-// choice for the whole process (tests run both forms); DSX_BLEND_PIXELS_PER_LANE=1|4 in the
-// environment gives the override's initial value and is read once.
+// to occupy the chip (8 wavefronts on each of 1024 SIMDs), else 1 (a workgroup of four wavefronts per
+// tile: more instructions in all, but four times as many wavefronts and shorter chains).  Measured, us,
+// wavefront / workgroup form:
+//   forward   256 tiles 107 / 34, 1024 84 / 36, 2170 70 / 48, 3600 169 / 130, 6370 305 / 304, 8160 127 / 141
+//   backward  1024 tiles 154 / 77, 2170 125 / 106, 4056 249 / 280, 6370 514 / 654
+// dsx_set_blend_pixels_per_lane(1 | 4) overrides the choice for the whole process (tests run both
+// forms); DSX_BLEND_PIXELS_PER_LANE=1|4 in the environment gives the override's initial value and is
+// read once.
 static std::atomic<int> g_forced_pixels_per_lane{-1}; // -1: not yet read from the environment, 0: automatic
 
 static int forced_pixels_per_lane()
@@ -185,34 +246,107 @@ __device__ __forceinline__ int bits_below_lane(uint64_t mask)
     return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
 
-constexpr int kFwdFourPixelsFrom = 5000; // tiles
-constexpr int kBwdFourPixelsFrom = 1600;
+constexpr int kFwdFourPixelsFrom = 6400; // tiles
+constexpr int kBwdFourPixelsFrom = 3000;
+
+// -----------------------------------------------------------------------------------------
+// what both directions share: the wavefront's pixels, and the walk through the lists
+// -----------------------------------------------------------------------------------------
+// kPix pixels per lane: 4 (one wavefront per 16x16 tile, its rows of lanes own 8x8 blocks) or 1 (four
+// wavefronts per tile, each one 8x8 quadrant, its rows of lanes own 4x4 blocks).
+template <int kPerLane>
+struct Pixels
+{
+    static constexpr int kSide = kPerLane == 4 ? 8 : 4; // a row's block
+    int tile, part;    // part: which quarter of the tile (0 for the whole)
+    int x0, y0;        // first pixel of the wavefront
+    int x, y;          // this lane's first pixel; the others lie two rows apart
+    float box_x, box_y; // first pixel centre of the wavefront
+    __device__ __forceinline__ Pixels(int block, int ntx, int lane)
+    {
+        tile = kPerLane == 4 ? block : block >> 2;
+        part = kPerLane == 4 ? 0 : block & 3;
+        x0 = (tile % ntx) * kTile + 8 * (part & 1);
+        y0 = (tile / ntx) * kTile + 8 * (part >> 1);
+        const int row = lane >> 4, i = lane & 15;
+        x = x0 + kSide * (row & 1) + (i & (kSide - 1));
+        y = y0 + kSide * (row >> 1) + i / kSide;
+        box_x = (float)x0 + 0.5f;
+        box_y = (float)y0 + 0.5f;
+    }
+    __device__ __forceinline__ int y_of(int p) const { return y + 2 * p; }
+};
+
+// word `i` of a device array (uniform base and a 32-bit byte offset: one address register)
+__device__ __forceinline__ int word_at(const int32_t* base, uint32_t i)
+{
+    return *reinterpret_cast<const int32_t*>(reinterpret_cast<const char*>(base) + 4u * i);
+}
+
+// a wavefront mask of the lanes below `count`
+__device__ __forceinline__ uint64_t lanes_below(int count)
+{
+    return count >= DSX_WAVE ? ~0ull : (1ull << max(count, 0)) - 1;
+}
+
+// the lowest `count` set bits of a mask that has more
+__device__ __forceinline__ uint64_t lowest_bits(uint64_t mask, int count)
+{
+    return __builtin_amdgcn_ballot_w64(bits_below_lane(mask) < count) & mask;
+}
+
+// A side job for the memory system, which the forward leaves idle: every workgroup prepares
+// its share of the backward's gradient accumulator, twelve floats per Gaussian: the nine sums
+// zeroed and, in the three spare places, the conic, which the per-Gaussian backward then has
+// at hand with the sums instead of fetching the splat records for it.  At the end of the
+// kernel, where nothing waits for the stores and the wavefronts arrive spread over time (at
+// the start they would all come at once and hold up the first loads: 0.147 against 0.140 ms).
+__device__ __forceinline__ void prepare_grads_share(const float4* splats, float4* prep, int64_t count, uint8_t* marks,
+                                                    int part, int parts, int tid, int threads)
+{
+    static_assert(DSX_GRAD_FLOATS == 12, "three float4 per Gaussian");
+    const int64_t share = (count + parts - 1) / parts;
+    const int64_t g1 = min((part + 1) * share, count);
+    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+    for(int64_t g = part * share + tid; g < g1; g += threads)
+    {
+        const float4 q1 = splats[3 * g + 1]; // conic a, b, c, opacity
+        prep[3 * g] = zero;
+        prep[3 * g + 1] = zero;
+        prep[3 * g + 2] = make_float4(0.f, q1.x, q1.y, q1.z);
+        if(marks)
+            marks[g] = 0; // "no term added yet"
+    }
+}
 
 // -----------------------------------------------------------------------------------------
 // forward: cpp/rasterizer_kernels.cu:341-431
 // -----------------------------------------------------------------------------------------
-// One wavefront per 16x16 tile, four pixels per lane (lane l owns column l & 15 of rows
-// (l >> 4) + {0, 4, 8, 12}).  Every LDS broadcast read of an entry then feeds 256 pixel
-// updates instead of 64, which moves the kernel from the LDS pipe to the VALU, gives each
-// lane four independent dependency chains, and needs no workgroup barrier at all.
-// Images of few tiles (fewer wavefronts than the chip has slots) take kFwdPix = 1 instead: four
-// wavefronts per tile, each with one band of four rows and one pixel per lane; a tile's walk is
-// then four times shorter in time, which is what counts when the launch cannot fill the chip.
-constexpr int kFwdBatch = 128; // sorted entries staged in LDS per round (two per lane)
+// No workgroup barrier anywhere: a workgroup is one wavefront.  A round takes entries of the tile's
+// list, 64 at a time, until no further 64 would fit: their records are gathered, those that reach any
+// pixel of the wavefront are staged in LDS (packed: what cannot reach leaves no hole), and the place
+// of each goes into the list of every row of lanes whose block it reaches.  Then the rows walk
+// their lists side by side.
+// Images of few tiles (fewer wavefronts than the chip has slots) take kPix = 1: four times
+// as many wavefronts, whose smaller blocks also leave each row fewer entries to walk.
+constexpr int kPix = 4; // pixels per lane of the wavefront forms
+constexpr float kAlphaMax = 0.999f;       // the forward's clamp (the backward's is 0.99)
+constexpr float kLog2AlphaMax = -0.0014434168696687186f; // its base-2 logarithm
+constexpr int kFwdBatch = 96; // staged entries of a round: 5 KB of LDS, 32 wavefronts per compute unit
 constexpr int kScanGroups = 4; // groups of 64 positions of a bin's list whose loads are in flight together
 
-// 8 wavefronts per SIMD (at most 64 VGPRs): all tiles of a 1080p image are resident at once
+typedef float dsx_f32x4 __attribute__((ext_vector_type(4)));
+
 // kBinned: the entries come out of the list of the tile's bin (BinLists).  The wavefront first
 // FILTERS the bin's list: 64 positions at a time it reads the pair's id and key word (two coalesced
-// 4-byte loads, the next 64 already in flight), tests the two bits of its tile in the key's mask,
-// and packs the ids of its own entries into a queue in LDS (the staging arrays' memory, which is
-// free between two rounds) until more than 64 are there or the list ends.  Only those are then gathered,
-// tested for reach and staged as with per-tile lists, so a tile pays a dozen instructions per 64
+// 4-byte loads, those of four groups in flight together), tests the two bits of its tile in the key's mask,
+// and queues the ids of its own entries, one per lane, until 64 are there or the list ends.  Only those
+// are then gathered and tested for reach, so a tile pays a dozen instructions per 64
 // entries of its bin's list instead of a gather and a rectangle test per entry; a scene whose
 // pixels do not saturate early, where every tile reads its bin's whole list, costs a few percent
 // more than with per-tile lists instead of twice as much.  final_idx still receives the
 // reference's index: the tile's range start plus the entry's rank among the tile's own entries.
-template <int kFwdPix, bool kBinned>
+template <bool kBinned>
 __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(8, 8))) void blend_fwd_kernel(const int32_t* __restrict__ ranges,
                                                              const int32_t* __restrict__ ids,
                                                              const float4* __restrict__ splats,
@@ -226,28 +360,442 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(8, 8))
                                                              uint8_t* __restrict__ prep_marks,
                                                              const BinLists lists)
 {
-    __shared__ float4 s_a[kFwdBatch]; // pixel x, pixel y, conic -a/2, conic b
-    __shared__ float4 s_b[kFwdBatch]; // conic c/2, opacity, red, green
-    __shared__ float s_c[kFwdBatch];  // blue
-    // the queue of the tile's own entries (binned lists) lives in s_a between two rounds: up to 128 ids
-    int* const s_queue = reinterpret_cast<int*>(s_a);
+    // the last place is nobody's entry (no exponent passes): rows whose list has ended point at it
+    __shared__ float4 s_a[kFwdBatch + 1]; // pixel x, pixel y, conic -a/2, conic b
+    __shared__ float4 s_b[kFwdBatch + 1]; // conic c/2, log2(opacity / 0.999), limit of the exponent's bits, index in the sorted key array
+    __shared__ float s_c[3 * kFwdBatch + 4]; // red, green, blue
+    __shared__ uint64_t s_list[4 * kFwdBatch / 8 + 1]; // a byte per entry and row: its place (one word more than is used: read ahead)
+    __shared__ int s_queue[DSX_WAVE]; // ids of the tile's own entries, on their way from the scan to the gather
+    static_assert(kFwdBatch % 8 == 0 && kFwdBatch < 256 && kFwdBatch >= DSX_WAVE, "places are bytes, stored by words");
 
     const int lane = threadIdx.x;
-    const int tile = kFwdPix == 4 ? blockIdx.x : blockIdx.x >> 2;
-    const int band = kFwdPix == 4 ? 0 : blockIdx.x & 3; // which four rows of the tile (one-pixel form)
-    const int tx = tile % ntx;
-    const int ty = tile / ntx;
-    const int x = tx * kTile + (lane & 15);
-    const int y0 = ty * kTile + 4 * band + (lane >> 4);
-    const float pxf = (float)x + 0.5f;
-    // first pixel centre and last row of the pixels this wavefront owns
-    const float box_x0 = (float)(tx * kTile) + 0.5f, box_y0 = (float)(ty * kTile + 4 * band) + 0.5f;
-    const float span_y = kFwdPix == 4 ? 15.0f : 3.0f;
+    const int row = lane >> 4;
+    const Pixels<kPix> px(blockIdx.x, ntx, lane);
+    const float pxf = (float)px.x + 0.5f;
+    uint8_t* const list_bytes = reinterpret_cast<uint8_t*>(s_list);
 
     // The lists are data from the device: positions are taken for what they are only inside
     // sorted_ids[0, k), and a `ranges` buffer that was built for another bin size (its header word,
     // which every layout has in the same place, says which) is not read any further; the image is
     // then NaN, like after a sort that gave up.
+    const bool layout_ok = header == nullptr || *header == header_shift;
+    int start = 0, end = 0;
+    TileSource src = {};
+    if(kBinned)
+    {
+        if(layout_ok)
+            src = tile_source(lists, px.tile, ntx);
+        start = src.start;
+        end = src.end;
+    }
+    else if(layout_ok)
+    {
+        start = ranges[px.tile];
+        end = ranges[px.tile + 1];
+    }
+    start = min(max(start, 0), k);
+    end = min(max(end, 0), k);
+
+    // A pixel that has stopped (or lies outside the image) gets NaN as its row coordinate: its
+    // exponent is then NaN, the test of it fails whatever the entry holds, and the loop
+    // needs no per-pixel flag.  `alive` counts the wavefront's live pixels (a scalar: it is kept
+    // from ballots, on the scalar unit, and costs the vector unit nothing).
+    float pyf[kPix], T[kPix];
+    // Colours: the matrix unit's 4x4x1 product in 16 blocks of four lanes adds weight (one pixel per lane)
+    // times (red, green, blue) of each block's own entry in ONE instruction where the vector unit
+    // takes three, with the same fused multiply-add per element.  Register r of lane 4 b + j then
+    // holds channel j of the pixel of lane 4 b + r.
+    dsx_f32x4 colour[kPix];
+    int last[kPix];
+    int alive = 0;
+#pragma unroll
+    for(int p = 0; p < kPix; ++p)
+    {
+        const int y = px.y_of(p);
+        const bool inside = px.x < W && y < H;
+        pyf[p] = inside ? (float)y + 0.5f : __builtin_nanf("");
+        alive += __popcll(__builtin_amdgcn_ballot_w64(inside));
+        T[p] = 1.0f;
+        colour[p] = dsx_f32x4{0.f, 0.f, 0.f, 0.f};
+        last[p] = 0;
+    }
+    if(lane == 0)
+    {
+        s_a[kFwdBatch] = make_float4(0.f, 0.f, 0.f, 0.f);
+        s_b[kFwdBatch] = make_float4(0.f, 0.f, __int_as_float(INT_MIN), 0.f);
+        s_c[3 * kFwdBatch] = s_c[3 * kFwdBatch + 1] = s_c[3 * kFwdBatch + 2] = s_c[3 * kFwdBatch + 3] = 0.f;
+    }
+
+    // binned lists: the scan of the bin's list
+    const uint32_t tile_bits = kBinned ? tile_bits_of(src, lists.shift) << 16 : 0u; // (in the key word's high half)
+    const int32_t* const keys = ids + k; // the pairs' key words lie behind the ids (binned lists)
+    int scan = start;  // next position of the list to look at
+    int seen = 0;      // entries of the tile's own list found so far
+    int index_next = kBinned ? src.fine_base : start; // what final_idx records for the next entry
+    while(alive != 0 && scan < end && (!kBinned || seen < src.count))
+    {
+        // rows with a live pixel
+        uint64_t live = 0;
+#pragma unroll
+        for(int p = 0; p < kPix; ++p)
+            live |= __builtin_amdgcn_ballot_w64(pyf[p] == pyf[p]);
+        uint32_t live_rows = 0;
+#pragma unroll
+        for(int r = 0; r < 4; ++r)
+            live_rows |= (live >> (16 * r)) & 0xffffull ? 1u << r : 0u;
+
+        __syncthreads(); // single wavefront: orders the LDS reads of the last round before these writes
+        if(lane < 4 * kFwdBatch / 8)
+            s_list[lane] = 0x0101010101010101ull * kFwdBatch;
+        int staged = 0;
+        int length[4] = {0, 0, 0, 0};
+        do
+        {
+            int id = 0;
+            int batch; // entries in this gather
+            if(kBinned)
+            {
+                batch = 0;
+                do
+                {
+                    // the loads of four groups of positions are issued together: the scan is bound by
+                    // their latency, not by its dozen instructions per group
+                    int gid[kScanGroups], key[kScanGroups];
+#pragma unroll
+                    for(int j = 0; j < kScanGroups; ++j)
+                    {
+                        const uint32_t e = (uint32_t)min(scan + j * DSX_WAVE + lane, end - 1);
+                        gid[j] = word_at(ids, e);
+                        key[j] = word_at(keys, e);
+                    }
+#pragma unroll
+                    for(int j = 0; j < kScanGroups; ++j)
+                    {
+                        // (uniform; a group that lies behind the end has no members, and moves nothing)
+                        uint64_t m = __builtin_amdgcn_ballot_w64(((uint32_t)key[j] & tile_bits) == tile_bits) &
+                                     lanes_below(end - scan);
+                        int taken = min(end - scan, DSX_WAVE);
+                        const int room = DSX_WAVE - batch;
+                        if(__popcll(m) > room)
+                        {
+                            // not all of the group's members fit: it is taken up to the last one that does
+                            m = lowest_bits(m, room);
+                            taken = room > 0 ? DSX_WAVE - __builtin_clzll(m) : 0;
+                        }
+                        if(m != 0)
+                        {
+                            if(__builtin_amdgcn_inverse_ballot_w64(m))
+                                s_queue[batch + bits_below_lane(m)] = gid[j];
+                            batch += __popcll(m);
+                        }
+                        scan += taken;
+                        if(taken < DSX_WAVE)
+                            break;
+                    }
+                } while(batch < DSX_WAVE && scan < end && seen + batch < src.count);
+                seen += batch;
+                __syncthreads();
+                id = s_queue[lane];
+            }
+            else
+            {
+                batch = min(end - scan, DSX_WAVE);
+                if(lane < batch)
+                    id = ids[scan + lane];
+                scan += batch;
+            }
+            uint32_t reached = 0;
+            float4 q0, q1;
+            StagedOpacity op;
+            const float4* const rec = splats + 3 * (int64_t)min((uint32_t)id, last_id);
+            if(lane < batch)
+            {
+                // (an id is taken for what it is only up to the last Gaussian: lists that a failed sort or a
+                // caller's mix-up left in disorder then give a wrong image, not a fetch outside the records)
+                q0 = rec[0], q1 = rec[1];
+                op = stage_opacity(q1.w);
+                reached = live_rows & blocks_reached<Pixels<kPix>::kSide>(q0.x, q0.y, q1.x, q1.y, q1.z, op.reach,
+                                                                             px.box_x, px.box_y);
+            }
+            const uint64_t m_any = __ballot(reached != 0);
+            const int place = staged + bits_below_lane(m_any);
+            if(reached != 0)
+            {
+                const float4 q2 = rec[2];
+                s_a[place] = make_float4(q0.x, q0.y, q1.x * -0.5f, q1.y);
+                s_b[place] = make_float4(q1.z * 0.5f, q1.w == q1.w ? op.log2 - kLog2AlphaMax : __builtin_inff(),
+                                         __int_as_float(reach_limit_fwd(q1.w, op.reach)),
+                                         __int_as_float(index_next + lane));
+                s_c[3 * place] = q2.x;
+                s_c[3 * place + 1] = q2.y;
+                s_c[3 * place + 2] = q2.z;
+            }
+#pragma unroll
+            for(int r = 0; r < 4; ++r)
+            {
+                const uint64_t m = __ballot((reached >> r) & 1);
+                if((reached >> r) & 1)
+                    list_bytes[r * kFwdBatch + length[r] + bits_below_lane(m)] = (uint8_t)place;
+                length[r] += __popcll(m);
+            }
+            staged += __popcll(m_any);
+            index_next += batch;
+        } while(staged <= kFwdBatch - DSX_WAVE && scan < end && (!kBinned || seen < src.count));
+        __syncthreads();
+
+        const int rounds = max(max(length[0], length[1]), max(length[2], length[3]));
+        const uint8_t* my_list = list_bytes + row * kFwdBatch;
+        int place = *my_list;
+        for(int i = 0; i < rounds; ++i)
+        {
+            if(alive == 0)
+                break;
+            asm("" : "+v"(place)); // (a whole register, as loaded: no masking of the byte)
+            const float4 A = s_a[place];
+            const float4 B = s_b[place];
+            const float channel = s_c[3 * place + (lane & 3)]; // (the fourth lane's is not looked at)
+            const int limit = __float_as_int(B.z);
+            // what final_idx records for this entry: its position in the sorted key array (binned
+            // lists: the tile's range start plus the entry's rank among the tile's own entries)
+            const int entry_index = __float_as_int(B.w);
+            place = *++my_list;
+            const ExponentX ex = exponent_x(A.z, A.w, pxf - A.x);
+            float weight[kPix], Tn[kPix];
+            uint64_t m_pass[kPix], m_low[kPix], m_stop = 0;
+#pragma unroll
+            for(int p = 0; p < kPix; ++p)
+            {
+#pragma clang fp contract(off)
+                const float dy = pyf[p] - A.y;
+                const float power = __builtin_fmaf(-__builtin_fmaf(B.x, dy, ex.bx), dy, ex.ax);
+                // the decisions as wavefront masks (each is its compare's own result register),
+                // combined on the scalar unit and handed back to the lanes as conditions
+                m_pass[p] = __builtin_amdgcn_ballot_w64(__float_as_int(power) <= limit);
+                // alpha / 0.999, at most 1 (the clamp is a modifier of the exponential's result)
+                const float e = __builtin_amdgcn_fmed3f(__builtin_amdgcn_exp2f(__builtin_fmaf(power, kLog2E, B.y)), 0.0f, 1.0f);
+                weight[p] = (__builtin_amdgcn_inverse_ballot_w64(m_pass[p]) ? e : 0.0f) * T[p];
+                Tn[p] = __builtin_fmaf(-kAlphaMax, weight[p], T[p]); // (1 - alpha) T
+                m_low[p] = __builtin_amdgcn_ballot_w64(Tn[p] < 0.0001f);
+                m_stop |= m_low[p];
+            }
+            if(m_stop != 0)
+            {
+                // pixels that this entry would make opaque stop without it
+#pragma unroll
+                for(int p = 0; p < kPix; ++p)
+                {
+                    const bool stop = __builtin_amdgcn_inverse_ballot_w64(m_low[p]);
+                    weight[p] = stop ? 0.0f : weight[p];
+                    pyf[p] = stop ? __builtin_nanf("") : pyf[p];
+                    m_pass[p] &= ~m_low[p];
+                    alive -= __popcll(m_low[p]);
+                }
+            }
+#pragma unroll
+            for(int p = 0; p < kPix; ++p)
+            {
+                colour[p] = __builtin_amdgcn_mfma_f32_4x4x1f32(weight[p], channel, colour[p], 0, 0, 0);
+                T[p] = __builtin_amdgcn_inverse_ballot_w64(m_low[p]) ? T[p] : Tn[p];
+                last[p] = __builtin_amdgcn_inverse_ballot_w64(m_pass[p]) ? entry_index : last[p];
+            }
+        }
+    }
+
+    // A sort pass that gave up waiting on its predecessor (bounded wait, never seen to happen)
+    // leaves its flag set and the tile lists wrong: make that loud instead of plausible.
+    const bool broken = !layout_ok || (sort_flag_a && *sort_flag_a) || (sort_flag_b && *sort_flag_b);
+    const int quad_x = px.x - (lane & 3), channel = lane & 3;
+#pragma unroll
+    for(int p = 0; p < kPix; ++p)
+    {
+        const int y = px.y_of(p);
+        if(px.x < W && y < H)
+        {
+            const int64_t pix = (int64_t)y * W + px.x;
+            final_T[pix] = T[p];
+            final_idx[pix] = last[p];
+        }
+        // (a lane's four neighbours lie in one row of pixels: its registers are one channel of all of them)
+        float* const out = image + 3 * ((int64_t)y * W + quad_x) + channel;
+#pragma unroll
+        for(int r = 0; r < 4; ++r)
+            if(channel < 3 && quad_x + r < W && y < H)
+                out[3 * r] = broken ? __builtin_nanf("") : kAlphaMax * colour[p][r];
+    }
+    if(kBinned && layout_ok)
+    {
+        // for the backward: where this wavefront's scan of the bin's list stopped and how many of the
+        // tile's entries it had met by then (everything that any of its pixels blended lies below).
+        // The other three parts are marked as empty.
+        int32_t* w = lists.walk + (int64_t)px.tile * 8;
+        const int stopped = min(scan, end);
+        if(lane < 8)
+            w[lane] = lane == 0 ? stopped : (lane == 1 ? seen : (lane & 1 ? 0 : -1));
+    }
+    prepare_grads_share(splats, prep, prep_count, prep_marks, blockIdx.x, gridDim.x, lane, DSX_WAVE);
+}
+
+// -----------------------------------------------------------------------------------------
+// the same for images of few tiles: a workgroup of four wavefronts per tile
+// -----------------------------------------------------------------------------------------
+// When the tiles are too few to fill the chip, a wavefront per tile leaves most of it idle and takes as
+// long as its longest dependency chain.  Here four wavefronts share a tile: each owns a quadrant (its
+// rows of lanes the quadrant's four 4x4 blocks, one pixel per lane), the four stage a round
+// of up to kTileBatch entries together (each thread gathers and tests one candidate, against
+// all sixteen blocks), and every wavefront then builds and walks its own rows' lists.  The smaller blocks leave
+// a row a third to a half of the tile's entries, and entries are taken four (backward: two) at a time, with their
+// LDS reads and exponentials in flight together.
+constexpr int kTileBatch = 248;   // (places are bytes; a multiple of 8)
+constexpr int kTileThreads = 256;
+constexpr int kTileWaves = kTileThreads / DSX_WAVE;
+
+// The scan of a bin's list by a workgroup: positions `at`, `at + step`, ... of which `left` lie inside
+// the list; queues up to kTileBatch ids of the entries whose key word has `bits`, after the first `skip` of
+// them.  Returns the number queued; `left` becomes the number of positions that remain, `skip` what remains of it.
+struct TileScan
+{
+    int counts[kScanGroups * kTileWaves]; // members per group of positions and wavefront
+    int taken;                            // positions up to the last accepted member
+};
+template <int kStep>
+__device__ __forceinline__ int tile_scan(TileScan& s, int* queue, const int32_t* ids, const int32_t* keys, int& at, int& left,
+                                         int& skip, uint32_t bits, int wanted)
+{
+    const int tid = threadIdx.x, wave = tid / DSX_WAVE;
+    int batch = 0;
+    while(left > 0 && batch < kTileBatch && batch < wanted)
+    {
+        int id[kScanGroups];
+        uint64_t m[kScanGroups];
+        uint32_t key[kScanGroups];
+#pragma unroll
+        for(int j = 0; j < kScanGroups; ++j)
+        {
+            const int o = min(j * kTileThreads + tid, left - 1);
+            const uint32_t e = (uint32_t)(kStep > 0 ? at + o : at - o);
+            id[j] = word_at(ids, e);
+            key[j] = (uint32_t)word_at(keys, e);
+        }
+#pragma unroll
+        for(int j = 0; j < kScanGroups; ++j)
+        {
+            m[j] = __builtin_amdgcn_ballot_w64((key[j] & bits) == bits) &
+                   lanes_below(left - j * kTileThreads - wave * DSX_WAVE);
+            if((tid & (DSX_WAVE - 1)) == 0)
+                s.counts[j * kTileWaves + wave] = __popcll(m[j]);
+        }
+        if(tid == 0)
+            s.taken = kScanGroups * kTileThreads;
+        __syncthreads();
+        int before = 0, first[kScanGroups] = {};
+#pragma unroll
+        for(int i = 0; i < kScanGroups * kTileWaves; ++i)
+        {
+            const int c = s.counts[i];
+#pragma unroll
+            for(int j = 0; j < kScanGroups; ++j)
+                first[j] += i < j * kTileWaves + wave ? c : 0;
+            before += c;
+        }
+        const int total = __builtin_amdgcn_readfirstlane(before);
+        const int room = kTileBatch - batch;
+#pragma unroll
+        for(int j = 0; j < kScanGroups; ++j)
+        {
+            const int rank = first[j] + bits_below_lane(m[j]) - skip; // among the accepted
+            if(__builtin_amdgcn_inverse_ballot_w64(m[j]) && rank >= 0 && rank < room)
+            {
+                queue[batch + rank] = id[j];
+                if(rank == room - 1)
+                    s.taken = j * kTileThreads + tid + 1;
+            }
+        }
+        __syncthreads();
+        const int taken = min(left, __builtin_amdgcn_readfirstlane(s.taken));
+        at += kStep > 0 ? taken : -taken;
+        left -= taken;
+        batch += min(max(total - skip, 0), room);
+        skip = max(skip - total, 0);
+        __syncthreads(); // s is written again
+    }
+    return batch;
+}
+
+// A wavefront's lists of one round: the places of the staged entries that reach each of its four blocks,
+// padded with the place that is nobody's.  Returns the longest list's length.
+__device__ __forceinline__ int build_lists(uint32_t* list_words, const uint16_t* reach, int staged, int wave, int lane)
+{
+    uint8_t* const bytes = reinterpret_cast<uint8_t*>(list_words + wave * kTileBatch);
+    for(int i = lane; i < kTileBatch; i += DSX_WAVE)
+        list_words[wave * kTileBatch + i] = 0x01010101u * kTileBatch;
+    int length[4] = {0, 0, 0, 0};
+    for(int first = 0; first < staged; first += DSX_WAVE)
+    {
+        const int place = first + lane;
+        const uint32_t mine = place < staged ? (uint32_t)reach[place] >> (4 * wave) : 0u;
+#pragma unroll
+        for(int r = 0; r < 4; ++r)
+        {
+            const uint64_t m = __builtin_amdgcn_ballot_w64((mine >> r) & 1);
+            if(__builtin_amdgcn_inverse_ballot_w64(m))
+                bytes[r * kTileBatch + length[r] + bits_below_lane(m)] = (uint8_t)place;
+            length[r] += __popcll(m);
+        }
+    }
+    return max(max(length[0], length[1]), max(length[2], length[3]));
+}
+
+// this thread's place among the threads of the workgroup whose `m` (a mask per wavefront) is set, and their number
+__device__ __forceinline__ int tile_place(int* counts, uint64_t m, int& total)
+{
+    const int wave = threadIdx.x / DSX_WAVE;
+    if((threadIdx.x & (DSX_WAVE - 1)) == 0)
+        counts[wave] = __popcll(m);
+    __syncthreads();
+    int before = 0, all = 0;
+#pragma unroll
+    for(int w = 0; w < kTileWaves; ++w)
+    {
+        const int c = counts[w];
+        before += w < wave ? c : 0;
+        all += c;
+    }
+    total = __builtin_amdgcn_readfirstlane(all);
+    return before + bits_below_lane(m);
+}
+
+constexpr int kFwdAtOnce = 4; // entries that a row takes at a time
+static_assert(kFwdAtOnce == 4 && kTileBatch % 4 == 0, "a word of the list holds four places");
+
+template <bool kBinned>
+__global__ __launch_bounds__(kTileThreads) void blend_fwd_tile_kernel(const int32_t* __restrict__ ranges, const int32_t* __restrict__ ids,
+                                                                      const float4* __restrict__ splats, float* __restrict__ image,
+                                                                      float* __restrict__ final_T, int32_t* __restrict__ final_idx, int W,
+                                                                      int H, int ntx, uint32_t last_id, int k,
+                                                                      const int32_t* __restrict__ header, int header_shift,
+                                                                      const uint32_t* __restrict__ sort_flag_a,
+                                                                      const uint32_t* __restrict__ sort_flag_b, float4* __restrict__ prep,
+                                                                      int64_t prep_count, uint8_t* __restrict__ prep_marks,
+                                                                      const BinLists lists)
+{
+    // (arrays as in the wavefront form)
+    __shared__ float4 s_a[kTileBatch + 1], s_b[kTileBatch + 1];
+    __shared__ float s_c[3 * kTileBatch + 4];
+    __shared__ uint16_t s_reach[kTileBatch]; // which of the tile's 16 blocks an entry reaches
+    __shared__ uint32_t s_list[kTileWaves * kTileBatch];
+    __shared__ int s_queue[kTileBatch];
+    __shared__ TileScan s_scan;
+    __shared__ int s_counts[kTileWaves];
+    __shared__ uint32_t s_live[kTileWaves];
+
+    const int tid = threadIdx.x, lane = tid & (DSX_WAVE - 1), row = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / DSX_WAVE);
+    const int tile = blockIdx.x;
+    const Pixels<1> px(4 * tile + wave, ntx, lane);
+    const float pxf = (float)px.x + 0.5f;
+    const float tile_x = (float)(tile % ntx * kTile) + 0.5f, tile_y = (float)(tile / ntx * kTile) + 0.5f;
+
+    // (positions and layout are taken for what they are as in the wavefront form)
     const bool layout_ok = header == nullptr || *header == header_shift;
     int start = 0, end = 0;
     TileSource src = {};
@@ -266,236 +814,167 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(8, 8))
     start = min(max(start, 0), k);
     end = min(max(end, 0), k);
 
-    // A pixel that has stopped (or lies outside the image) gets NaN as its row coordinate: its
-    // exponent is then NaN, the test `power < 0` fails whatever the entry holds, and the loop
-    // needs no per-pixel flag.  `alive` counts the wavefront's live pixels (a scalar: it is kept
-    // from ballots, on the scalar unit, and costs the vector unit nothing).
-    float pyf[kFwdPix], T[kFwdPix], cr[kFwdPix], cg[kFwdPix], cb[kFwdPix];
-    int last[kFwdPix];
-    int alive = 0;
-#pragma unroll
-    for(int p = 0; p < kFwdPix; ++p)
+    const bool inside = px.x < W && px.y < H;
+    float pyf = inside ? (float)px.y + 0.5f : __builtin_nanf(""); // (NaN: stopped)
+    float T = 1.0f;
+    dsx_f32x4 colour = {0.f, 0.f, 0.f, 0.f};
+    int last = 0;
+    if(tid == 0)
     {
-        const int y = y0 + 4 * p;
-        const bool inside = x < W && y < H;
-        pyf[p] = inside ? (float)y + 0.5f : __builtin_nanf("");
-        alive += __popcll(__builtin_amdgcn_ballot_w64(inside));
-        T[p] = 1.0f;
-        cr[p] = cg[p] = cb[p] = 0.0f;
-        last[p] = 0;
+        s_a[kTileBatch] = make_float4(0.f, 0.f, 0.f, 0.f);
+        s_b[kTileBatch] = make_float4(0.f, 0.f, __int_as_float(INT_MIN), 0.f);
+        s_c[3 * kTileBatch] = s_c[3 * kTileBatch + 1] = s_c[3 * kTileBatch + 2] = s_c[3 * kTileBatch + 3] = 0.f;
     }
 
-    // per-tile lists: the Gaussian ids of a round are fetched one round ahead: the gather of the
-    // splat records then waits for one memory round trip instead of two in a row
-    int g_ahead[kFwdBatch / DSX_WAVE];
-    // binned lists: the scan of the bin's list
-    const uint32_t tile_bits = kBinned ? tile_bits_of(src, lists.shift) << 16 : 0u; // (in the key word's high half)
-    const int32_t* const keys = ids + k; // the pairs' key words lie behind the ids (binned lists)
-    int scan = start;  // next position of the bin's list to look at
-    int seen = 0;      // entries of the tile's own list found so far
-    if(!kBinned)
+    const uint32_t tile_bits = kBinned ? tile_bits_of(src, lists.shift) << 16 : 0u;
+    const int32_t* const keys = ids + k;
+    int scan = start, left = end - start, seen = 0, no_skip = 0;
+    int index_next = kBinned ? src.fine_base : start;
+    int id_ahead = 0;
+    if(!kBinned && tid < min(left, kTileBatch))
+        id_ahead = ids[scan + tid];
+    while(true)
     {
+        // blocks with a live pixel
+        const uint64_t live = __builtin_amdgcn_ballot_w64(pyf == pyf);
+        uint32_t live_rows = 0;
 #pragma unroll
-        for(int h = 0; h < kFwdBatch / DSX_WAVE; ++h)
-        {
-            const int e = start + h * DSX_WAVE + lane;
-            g_ahead[h] = e < end ? ids[e] : 0;
-        }
-    }
-    int index_base = kBinned ? src.fine_base : start; // what final_idx records for the first entry of the round
-    for(int b = start;; b += kFwdBatch)
-    {
-        if(alive == 0)
+        for(int r = 0; r < 4; ++r)
+            live_rows |= (live >> (16 * r)) & 0xffffull ? 1u << r : 0u;
+        if(lane == 0)
+            s_live[wave] = live_rows << (4 * wave);
+        __syncthreads(); // (and the last round's entries have been walked)
+        const uint32_t live_blocks = __builtin_amdgcn_readfirstlane(s_live[0] | s_live[1] | s_live[2] | s_live[3]);
+        if(live_blocks == 0 || left <= 0 || (kBinned && seen >= src.count))
             break;
-        int batch; // entries of this round
-        __syncthreads(); // single wavefront: orders the LDS reads of the last round before these writes
+        int id, batch;
         if(kBinned)
         {
-            // Another 64 positions are taken only while all of them would still fit the round, and a
-            // tile whose own entries have all been found looks no further.  The loads of four such
-            // groups are issued together (the scan is bound by their latency, not by its dozen
-            // instructions per group); groups that the round has no room for are read again by the next.
-            int count = 0;
-            while(count <= kFwdBatch - DSX_WAVE && scan < end && seen < src.count)
-            {
-                int id[kScanGroups], key[kScanGroups];
-#pragma unroll
-                for(int j = 0; j < kScanGroups; ++j)
-                {
-                    const int e = scan + j * DSX_WAVE + lane;
-                    id[j] = e < end ? ids[e] : 0;
-                    key[j] = e < end ? keys[e] : 0;
-                }
-#pragma unroll
-                for(int j = 0; j < kScanGroups; ++j)
-                {
-                    if(count <= kFwdBatch - DSX_WAVE && scan < end && seen < src.count) // (uniform)
-                    {
-                        const bool member = scan + lane < end && (((uint32_t)key[j]) & tile_bits) == tile_bits;
-                        const uint64_t m = __ballot(member);
-                        if(member)
-                            s_queue[count + bits_below_lane(m)] = id[j];
-                        const int found = __popcll(m);
-                        count += found;
-                        seen += found;
-                        scan += DSX_WAVE;
-                    }
-                }
-            }
-            if(count == 0)
-                break;
-            __syncthreads();
-            batch = count;
-#pragma unroll
-            for(int h = 0; h < kFwdBatch / DSX_WAVE; ++h)
-                g_ahead[h] = h * DSX_WAVE + lane < batch ? s_queue[h * DSX_WAVE + lane] : 0;
-            __syncthreads(); // the queue has been read: its memory now takes the staged records
+            batch = tile_scan<1>(s_scan, s_queue, ids, keys, scan, left, no_skip, tile_bits, src.count - seen);
+            seen += batch;
+            id = tid < batch ? s_queue[tid] : 0;
         }
         else
         {
-            if(b >= end)
-                break;
-            batch = min(end - b, kFwdBatch);
+            batch = min(left, kTileBatch);
+            id = id_ahead;
+            scan += batch;
+            left -= batch;
+            if(tid < min(left, kTileBatch))
+                id_ahead = ids[scan + tid]; // the next round's: in flight meanwhile
         }
-        uint64_t todo[kFwdBatch / DSX_WAVE]; // entries of this round that can touch the tile
-#pragma unroll
-        for(int h = 0; h < kFwdBatch / DSX_WAVE; ++h)
+        uint32_t reached = 0;
+        float4 q0, q1, q2;
+        StagedOpacity op;
+        if(tid < batch)
         {
-            const int slot = h * DSX_WAVE + lane;
-            bool useful = false;
-            // (an id is taken for what it is only up to the last Gaussian: lists that a failed sort or a
-            // caller's mix-up left in disorder then give a wrong image, not a fetch outside the records)
-            const int g = (int)min((uint32_t)g_ahead[h], last_id);
-            if(slot < batch)
-            {
-                const float4* rec = splats + 3 * (int64_t)g;
-                const float4 q0 = rec[0], q1 = rec[1], q2 = rec[2];
-                s_a[slot] = make_float4(q0.x, q0.y, q1.x * -0.5f, q1.y);
-                s_b[slot] = make_float4(q1.z * 0.5f, q1.w, q2.x, q2.y);
-                s_c[slot] = q2.z;
-                useful = entry_reaches_tile(q0.x, q0.y, q1.x, q1.y, q1.z, q1.w, box_x0, box_y0, span_y);
-            }
-            todo[h] = __ballot(useful);
+            const float4* const rec = splats + 3 * (int64_t)min((uint32_t)id, last_id);
+            q0 = rec[0], q1 = rec[1], q2 = rec[2];
+            op = stage_opacity(q1.w);
+#pragma unroll
+            for(int q = 0; q < 4; ++q)
+                reached |= blocks_reached<4>(q0.x, q0.y, q1.x, q1.y, q1.z, op.reach, tile_x + 8.0f * (q & 1), tile_y + 8.0f * (q >> 1)) << (4 * q);
+            reached &= live_blocks;
         }
+        int staged;
+        const int place = tile_place(s_counts, __builtin_amdgcn_ballot_w64(reached != 0), staged);
+        if(reached != 0)
+        {
+            s_a[place] = make_float4(q0.x, q0.y, q1.x * -0.5f, q1.y);
+            s_b[place] = make_float4(q1.z * 0.5f, q1.w == q1.w ? op.log2 - kLog2AlphaMax : __builtin_inff(),
+                                     __int_as_float(reach_limit_fwd(q1.w, op.reach)), __int_as_float(index_next + tid));
+            s_c[3 * place] = q2.x;
+            s_c[3 * place + 1] = q2.y;
+            s_c[3 * place + 2] = q2.z;
+            s_reach[place] = (uint16_t)reached;
+        }
+        index_next += batch;
         __syncthreads();
-        if(!kBinned)
+        if(live_rows == 0)
+            continue; // (nothing left in this quadrant: the others' barriers are met)
+
+        const int rounds = (build_lists(s_list, s_reach, staged, wave, lane) + kFwdAtOnce - 1) / kFwdAtOnce;
+        const uint32_t* my_list = s_list + wave * kTileBatch + row * (kTileBatch / 4);
+        for(int i = 0; i < rounds; ++i)
         {
-            // the next round's ids: in flight while this round's entries are blended
+            const uint32_t places = my_list[i];
+            float4 A[kFwdAtOnce], B[kFwdAtOnce];
+            float channel[kFwdAtOnce], e[kFwdAtOnce], weight[kFwdAtOnce];
+            uint64_t m_pass[kFwdAtOnce];
 #pragma unroll
-            for(int h = 0; h < kFwdBatch / DSX_WAVE; ++h)
+            for(int u = 0; u < kFwdAtOnce; ++u)
             {
-                const int e = b + kFwdBatch + h * DSX_WAVE + lane;
-                g_ahead[h] = e < end ? ids[e] : 0;
+                const uint32_t p = (places >> (8 * u)) & 0xffu;
+                A[u] = s_a[p];
+                B[u] = s_b[p];
+                channel[u] = s_c[3 * p + (lane & 3)];
             }
-        }
+            float Tn = T;
 #pragma unroll
-        for(int h = 0; h < kFwdBatch / DSX_WAVE; ++h)
-        {
-            uint64_t mask = todo[h];
-            while(mask != 0)
+            for(int u = 0; u < kFwdAtOnce; ++u)
             {
-                if(alive == 0)
-                    break;
-                const int bit = __builtin_ctzll(mask);
-                const int i = h * DSX_WAVE + bit;
-                mask &= mask - 1;
-                const float4 A = s_a[i];
-                const float4 B = s_b[i];
-                const float C = s_c[i];
-                // what final_idx records for this entry: its position in the sorted key array (binned
-                // lists: the tile's range start plus the entry's rank among the tile's own entries)
-                const int entry_index = index_base + i;
-                const ExponentX ex = exponent_x(A.z, A.w, pxf - A.x);
+#pragma clang fp contract(off)
+                const ExponentX ex = exponent_x(A[u].z, A[u].w, pxf - A[u].x);
+                const float dy = pyf - A[u].y;
+                const float power = __builtin_fmaf(-__builtin_fmaf(B[u].x, dy, ex.bx), dy, ex.ax);
+                m_pass[u] = __builtin_amdgcn_ballot_w64(__float_as_int(power) <= __float_as_int(B[u].z));
+                const float full = __builtin_amdgcn_fmed3f(__builtin_amdgcn_exp2f(__builtin_fmaf(power, kLog2E, B[u].y)), 0.0f, 1.0f);
+                e[u] = __builtin_amdgcn_inverse_ballot_w64(m_pass[u]) ? full : 0.0f;
+            }
 #pragma unroll
-                for(int p = 0; p < kFwdPix; ++p)
+            for(int u = 0; u < kFwdAtOnce; ++u)
+            {
+                weight[u] = e[u] * Tn;
+                Tn = __builtin_fmaf(-kAlphaMax, weight[u], Tn);
+            }
+            if(__builtin_amdgcn_ballot_w64(Tn < 0.0001f) != 0)
+            {
+                // some pixel becomes opaque within these entries: once more, one entry after the other
+                Tn = T;
+#pragma unroll
+                for(int u = 0; u < kFwdAtOnce; ++u)
                 {
-                    const float power = exponent_xy(ex, B.x, pyf[p] - A.y);
-                    // (a NaN opacity gives alpha = 0.999 here as in the reference: fminf drops the NaN)
-                    const float alpha = fminf(0.999f, B.y * fast_exp(power));
-                    // the three decisions as wavefront masks (each is its compare's own result register),
-                    // combined on the scalar unit and handed back to the lanes as conditions
-                    // (1 - alpha) T in one rounding
-                    const float Tn = __builtin_fmaf(-alpha, T[p], T[p]);
-                    const uint64_t m_pass = __builtin_amdgcn_ballot_w64(power < 0.0f) &
-                                            __builtin_amdgcn_ballot_w64(alpha >= kAlphaThreshold);
-                    const uint64_t m_low = __builtin_amdgcn_ballot_w64(Tn < 0.0001f);
-                    const uint64_t m_stop = m_pass & m_low;
-                    const bool stop = __builtin_amdgcn_inverse_ballot_w64(m_stop);
-                    const bool apply = __builtin_amdgcn_inverse_ballot_w64(m_pass & ~m_low);
-                    const float vis = apply ? alpha * T[p] : 0.0f;
-                    cr[p] += vis * B.z;
-                    cg[p] += vis * B.w;
-                    cb[p] += vis * C;
-                    T[p] = apply ? Tn : T[p];
-                    last[p] = apply ? entry_index : last[p];
-                    pyf[p] = stop ? __builtin_nanf("") : pyf[p];
-                    alive -= __popcll(m_stop);
+                    weight[u] = (pyf == pyf ? e[u] : 0.0f) * Tn;
+                    const float next = __builtin_fmaf(-kAlphaMax, weight[u], Tn);
+                    const uint64_t m_low = __builtin_amdgcn_ballot_w64(next < 0.0001f);
+                    const bool stop = __builtin_amdgcn_inverse_ballot_w64(m_low);
+                    m_pass[u] &= __builtin_amdgcn_ballot_w64(pyf == pyf) & ~m_low;
+                    weight[u] = stop ? 0.0f : weight[u];
+                    Tn = stop ? Tn : next;
+                    pyf = stop ? __builtin_nanf("") : pyf;
                 }
+                if(__builtin_amdgcn_ballot_w64(pyf == pyf) == 0)
+                    i = rounds; // no pixel left
+            }
+            T = Tn;
+#pragma unroll
+            for(int u = 0; u < kFwdAtOnce; ++u)
+            {
+                colour = __builtin_amdgcn_mfma_f32_4x4x1f32(weight[u], channel[u], colour, 0, 0, 0);
+                last = __builtin_amdgcn_inverse_ballot_w64(m_pass[u]) ? __float_as_int(B[u].w) : last;
             }
         }
-        index_base += batch;
     }
 
-    // A sort pass that gave up waiting on its predecessor (bounded wait, never seen to happen)
-    // leaves its flag set and the tile lists wrong: make that loud instead of plausible.
-    if(!layout_ok || (sort_flag_a && *sort_flag_a) || (sort_flag_b && *sort_flag_b))
+    const bool broken = !layout_ok || (sort_flag_a && *sort_flag_a) || (sort_flag_b && *sort_flag_b);
+    const int quad_x = px.x - (lane & 3), channel = lane & 3;
+    if(inside)
     {
+        const int64_t pix = (int64_t)px.y * W + px.x;
+        final_T[pix] = T;
+        final_idx[pix] = last;
+    }
+    float* const out = image + 3 * ((int64_t)px.y * W + quad_x) + channel;
 #pragma unroll
-        for(int p = 0; p < kFwdPix; ++p)
-            cr[p] = cg[p] = cb[p] = __builtin_nanf("");
-    }
-#pragma unroll
-    for(int p = 0; p < kFwdPix; ++p)
+    for(int r = 0; r < 4; ++r)
+        if(channel < 3 && quad_x + r < W && px.y < H)
+            out[3 * r] = broken ? __builtin_nanf("") : kAlphaMax * colour[r];
+    if(kBinned && layout_ok && tid < 8)
     {
-        const int y = y0 + 4 * p;
-        if(x < W && y < H)
-        {
-            const int64_t pix = (int64_t)y * W + x;
-            image[3 * pix] = cr[p];
-            image[3 * pix + 1] = cg[p];
-            image[3 * pix + 2] = cb[p];
-            final_T[pix] = T[p];
-            final_idx[pix] = last[p];
-        }
+        // (as in the wavefront form, which speaks for the whole tile too)
+        lists.walk[(int64_t)tile * 8 + tid] = tid == 0 ? scan : (tid == 1 ? seen : (tid & 1 ? 0 : -1));
     }
-    if(kBinned && layout_ok)
-    {
-        // for the backward: where this wavefront's scan of the bin's list stopped and how many of the
-        // tile's entries it had met by then (everything that any of its pixels blended lies below).
-        // The four-pixel form speaks for the whole tile and marks the other three bands as empty.
-        int32_t* w = lists.walk + (int64_t)tile * 8;
-        const int stopped = min(scan, end);
-        if(kFwdPix == 4)
-        {
-            if(lane < 8)
-                w[lane] = lane == 0 ? stopped : (lane == 1 ? seen : (lane & 1 ? 0 : -1));
-        }
-        else if(lane < 2)
-            w[2 * band + lane] = lane == 0 ? stopped : seen;
-    }
-    // A side job for the memory system, which this kernel leaves idle: every wavefront prepares
-    // its share of the backward's gradient accumulator, twelve floats per Gaussian: the nine sums
-    // zeroed and, in the three spare places, the conic, which the per-Gaussian backward then has
-    // at hand with the sums instead of fetching the splat records for it.  At the end of the
-    // kernel, where nothing waits for the stores and the wavefronts arrive spread over time (at
-    // the start they would all come at once and hold up the first loads: 0.147 against 0.140 ms).
-    if(prep_count > 0)
-    {
-        static_assert(DSX_GRAD_FLOATS == 12, "three float4 per Gaussian");
-        const int64_t share = (prep_count + gridDim.x - 1) / gridDim.x;
-        const int64_t g0 = (int64_t)blockIdx.x * share;
-        const int64_t g1 = min(g0 + share, prep_count);
-        const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-        for(int64_t g = g0 + lane; g < g1; g += DSX_WAVE)
-        {
-            const float4 q1 = splats[3 * g + 1]; // conic a, b, c, opacity
-            prep[3 * g] = zero;
-            prep[3 * g + 1] = zero;
-            prep[3 * g + 2] = make_float4(0.f, q1.x, q1.y, q1.z);
-            if(prep_marks)
-                prep_marks[g] = 0; // "no term added yet"
-        }
-    }
+    prepare_grads_share(splats, prep, prep_count, prep_marks, blockIdx.x, gridDim.x, tid, kTileThreads);
 }
 
 // The BinLists view of a `ranges` buffer in ranges_layout(lg) (lists per bin: lg.shift > 0)
@@ -544,20 +1023,20 @@ int launch_blend_fwd(const dsx_camera& cam, int64_t n, int64_t k, int32_t* range
     {
         DSX_TIMED("blend_fwd_kernel", stream);
         const bool four = blend_pixels_per_lane(ntx * nty, kFwdFourPixelsFrom) == 4;
-        const dim3 grid(four ? ntx * nty : 4 * ntx * nty);
+        const dim3 grid(ntx * nty);
         const float4* sp = reinterpret_cast<const float4*>(splats);
-#define DSX_LAUNCH_FWD(PIX, BINNED)                                                                              \
-    hipLaunchKernelGGL((blend_fwd_kernel<PIX, BINNED>), grid, dim3(DSX_WAVE), 0, stream, ranges, sorted_ids, sp,   \
-                       image, final_T, final_idx, cam.image_width, cam.image_height, ntx, last_id, (int)k, header,  \
-                       lg.shift, sort_flag_a, sort_flag_b, prep, prep_count, prep_marks, L)
+#define DSX_LAUNCH_FWD(KERNEL, THREADS)                                                                          \
+    hipLaunchKernelGGL((KERNEL), grid, dim3(THREADS), 0, stream, ranges, sorted_ids, sp, image, final_T, final_idx,  \
+                       cam.image_width, cam.image_height, ntx, last_id, (int)k, header, lg.shift, sort_flag_a,     \
+                       sort_flag_b, prep, prep_count, prep_marks, L)
         if(four && lg.shift)
-            DSX_LAUNCH_FWD(4, true);
+            DSX_LAUNCH_FWD(blend_fwd_kernel<true>, DSX_WAVE);
         else if(four)
-            DSX_LAUNCH_FWD(4, false);
+            DSX_LAUNCH_FWD(blend_fwd_kernel<false>, DSX_WAVE);
         else if(lg.shift)
-            DSX_LAUNCH_FWD(1, true);
+            DSX_LAUNCH_FWD(blend_fwd_tile_kernel<true>, kTileThreads);
         else
-            DSX_LAUNCH_FWD(1, false);
+            DSX_LAUNCH_FWD(blend_fwd_tile_kernel<false>, kTileThreads);
 #undef DSX_LAUNCH_FWD
     }
     DSX_LAUNCH_CHECK();
@@ -568,125 +1047,151 @@ int launch_blend_fwd(const dsx_camera& cam, int64_t n, int64_t k, int32_t* range
 // backward: cpp/gsplat/backward.cu:25-202
 // -----------------------------------------------------------------------------------------
 
-// Sum over the 64 lanes of a wavefront with data-parallel-primitive adds only (no LDS
-// traffic): two quad permutes, two row mirrors, then the row broadcasts.  The total is valid
-// in lane 63.
-template <int kCtrl, int kRowMask>
-__device__ __forceinline__ float dpp_add(float v)
-{
-    const int moved = __builtin_amdgcn_update_dpp(0, __float_as_int(v), kCtrl, kRowMask, 0xf, false);
-    return v + __int_as_float(moved);
-}
-
-__device__ __forceinline__ float wave_sum_to_lane63(float v)
-{
-    v = dpp_add<0xB1, 0xf>(v);  // quad_perm [1,0,3,2]
-    v = dpp_add<0x4E, 0xf>(v);  // quad_perm [2,3,0,1]
-    v = dpp_add<0x141, 0xf>(v); // row_half_mirror
-    v = dpp_add<0x140, 0xf>(v); // row_mirror: every lane of a row holds the row sum
-    v = dpp_add<0x142, 0xa>(v); // row_bcast:15 into rows 1 and 3
-    v = dpp_add<0x143, 0xc>(v); // row_bcast:31 into rows 2 and 3
-    return v;
-}
-
-typedef unsigned int dsx_u32x2 __attribute__((ext_vector_type(2)));
-
 template <int kCtrl>
 __device__ __forceinline__ float dpp_move(float v)
 {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kCtrl, 0xf, 0xf, false));
 }
-
-// Sums eight per-lane values over the wavefront as a reduce-scatter.  The first two steps use the
-// lane-swap instructions, which halve two registers into one at a time: across the halves of
-// the wavefront (8 -> 4 registers), across neighbouring rows of 16 (4 -> 2); the third step
-// trades between neighbouring lanes (2 -> 1), and three adds over the lanes that differ in bits
-// 1, 2 and 3 finish the rows.  18 instructions where a select-and-add scheme over all three
-// steps took 32.  Every lane ends up with a total: the one of
-// v[4*(lane&1) + 2*((lane>>4)&1) + (lane>>5)].
-__device__ __forceinline__ float pair_sum_halves(float a, float b)
+template <int kCtrl>
+__device__ __forceinline__ float dpp_add(float v)
 {
-    // lanes 0..31 get a summed over the two halves, lanes 32..63 get b
-    const dsx_u32x2 r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-    return __uint_as_float(r.x) + __uint_as_float(r.y);
+    return v + dpp_move<kCtrl>(v);
 }
 
-__device__ __forceinline__ float pair_sum_rows(float a, float b)
+// Sums over the 16 lanes of a row, the four rows at once (their lanes hold four entries' terms), with
+// data-parallel-primitive adds only: no LDS traffic.
+__device__ __forceinline__ float row_sum(float v)
 {
-    // even rows get a summed over each pair of neighbouring rows, odd rows get b
-    const dsx_u32x2 r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-    return __uint_as_float(r.x) + __uint_as_float(r.y);
+    v = dpp_add<0xB1>(v);  // quad_perm [1,0,3,2]
+    v = dpp_add<0x4E>(v);  // quad_perm [2,3,0,1]
+    v = dpp_add<0x124>(v); // row_ror:4
+    v = dpp_add<0x128>(v); // row_ror:8
+    return v;
 }
 
-__device__ __forceinline__ float wave_sum8_scatter(const float (&v)[8], int lane)
+// Eight values at once as a reduce-scatter.  A step takes two registers into one: the lanes of one half
+// keep the first value and add their partner's share of it, the other half the second.  The
+// DPP bank mask (banks of four lanes) chooses the lanes of an add for free where the halves are whole banks,
+// so the first two steps (lanes 8 apart: 8 -> 4 registers; lanes 7 - l of a half row: 4 -> 2) take two
+// instructions per pair; the last pair trades between neighbouring lanes by selects, and one add over lanes
+// two apart finishes: 16 instructions for the eight sums of four entries.
+// Lane l ends up with the total of v[4 * (l & 1) + 2 * ((l >> 2) & 1) + ((l >> 3) & 1)].
+// (In the asm a VALU result may be read through DPP only two wait states after it was written, which the
+// compiler cannot see to inside: hence the s_nop in front; no later instruction of a block reads another's result.)
+__device__ __forceinline__ float row_sum8_scatter(const float (&v)[8], int lane)
 {
-    const float s0 = pair_sum_halves(v[0], v[1]);
-    const float s1 = pair_sum_halves(v[2], v[3]);
-    const float s2 = pair_sum_halves(v[4], v[5]);
-    const float s3 = pair_sum_halves(v[6], v[7]);
-    const float t0 = pair_sum_rows(s0, s1); // v[2 * row parity + half]
-    const float t1 = pair_sum_rows(s2, s3); // v[4 + 2 * row parity + half]
+    float s0, s1, s2, s3;
+    asm("s_nop 1\n\t"
+        "v_add_f32_dpp %0, %4, %4 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+        "v_add_f32_dpp %1, %6, %6 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+        "v_add_f32_dpp %2, %8, %8 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+        "v_add_f32_dpp %3, %10, %10 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+        "v_add_f32_dpp %0, %5, %5 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %1, %7, %7 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %2, %9, %9 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %3, %11, %11 row_ror:8 row_mask:0xf bank_mask:0xc"
+        : "=&v"(s0), "=&v"(s1), "=&v"(s2), "=&v"(s3)
+        : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]), "v"(v[5]), "v"(v[6]), "v"(v[7]));
+    float t0, t1;
+    asm("s_nop 1\n\t"
+        "v_add_f32_dpp %0, %2, %2 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"
+        "v_add_f32_dpp %1, %4, %4 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"
+        "v_add_f32_dpp %0, %3, %3 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
+        "v_add_f32_dpp %1, %5, %5 row_half_mirror row_mask:0xf bank_mask:0xa"
+        : "=&v"(t0), "=&v"(t1)
+        : "v"(s0), "v"(s1), "v"(s2), "v"(s3));
+    // the half mirror pairs lane l with 7 - l: after it a bank's four lanes hold four partial sums of one value
     const bool odd = lane & 1;
     const float keep = odd ? t1 : t0;
     const float send = odd ? t0 : t1;
-    float o = keep + dpp_move<0xB1>(send); // quad_perm [1,0,3,2]: the neighbour's share
-    o = dpp_add<0x4E, 0xf>(o);             // quad_perm [2,3,0,1]: lanes that differ in bit 1
-    o = dpp_add<0x124, 0xf>(o);            // row_ror:4 and
-    o = dpp_add<0x128, 0xf>(o);            // row_ror:8: lanes that differ in bits 2 and 3
-    return o;
+    const float o = keep + dpp_move<0xB1>(send); // quad_perm [1,0,3,2]: the neighbour's share
+    return dpp_add<0x4E>(o);                     // quad_perm [2,3,0,1]: lanes that differ in bit 1
 }
 
-constexpr int kBwdBatch = 128; // sorted entries staged in LDS per round (two per lane)
+// The nine sums of a staged entry, added up in LDS over the rows of lanes: as doubles, because the LDS adds a double
+// in a third of a cycle per lane where a float takes three (36 lanes: 11 cycles against 109, of a unit
+// that the compute unit's wavefronts share).
+constexpr int kSums = 9;
+constexpr int kBwdBatch = 80; // staged entries of a round: 10 KB of LDS with their sums, 16 wavefronts per compute unit
 
-// One wavefront per 16x16 tile, four pixels per lane (same pixel ownership as the forward).
-// The per-Gaussian gradients are first summed over a lane's four pixels, then over the
-// wavefront with DPP adds, and lane 63 issues ONE set of hardware float atomics per
-// (tile, entry).  Compared with four wavefronts of one pixel per lane this does one
-// cross-lane reduction per entry instead of four and needs no LDS accumulators or barriers.
-// (kBwdPix = 1: four wavefronts per tile with one band of four rows each, as in the forward)
+// An entry's sums in LDS, from the moments of w = -v_sigma over its pixels to the gradients:
+// v_x = sum of v_sigma (a dx + b dy) with d = mean - pixel (v_sigma and d both change sign), ...
+__device__ __forceinline__ void moments_to_gradients(double* m, const float4 A, const float4 B)
+{
+    const float half_a = A.z, b = A.w, half_c = B.x;
+    const double w = m[0], wx = m[1], wxx = m[2], wy = m[3], wxy = m[4], wyy = m[5];
+    m[0] = (double)(2.0f * half_a) * wx + (double)b * wy;
+    m[1] = (double)b * wx + (double)(2.0f * half_c) * wy;
+    m[2] = -0.5 * wxx;
+    m[3] = -wxy;
+    m[4] = -0.5 * wyy;
+    m[5] = w * (double)__builtin_amdgcn_exp2f(-B.y); // v_opacity: what w holds as the opacity's factor taken out
+}
+// One set of hardware float atomics per entry and round, and none where no pixel was valid
+__device__ __forceinline__ void flush_sums(const double* sums, const int* ids, int staged, float* grads, uint8_t* marks,
+                                           int tid, int threads)
+{
+    for(int i = tid; i < staged * kSums; i += threads)
+    {
+        const float v = (float)sums[i];
+        if(v != 0.0f)
+        {
+            const int e = i / kSums;
+            const int64_t id = ids[e];
+            unsafeAtomicAdd(grads + id * DSX_GRAD_FLOATS + (i - e * kSums), v);
+            if(marks)
+                marks[id] = 1;
+        }
+    }
+}
+
+// Same shape as the forward: four rows of lanes, each with its block of pixels and its own list of the
+// entries that reach it, back to front from the last entry that any pixel blended.
+// The per-Gaussian gradients are first summed over a lane's four pixels, then over the row's
+// 16 lanes with DPP adds, all four rows' entries at once, and ONE atomic instruction carries the nine
+// sums of up to four entries.
 // kBinned: the entries come out of the list of the tile's bin, filtered into a queue as in the forward
-// but downwards; the forward left, per tile and band, the bin-list position where its scan stopped and
+// but downwards; the forward left, per tile and part, the bin-list position where its scan stopped and
 // the number of the tile's entries it had met by then, from which every entry met on the way down
 // gets its index in the sorted key array (final_idx is compared with those).
-template <int kBwdPix, bool kBinned>
+template <bool kBinned>
 __global__ __launch_bounds__(DSX_WAVE) void blend_bwd_kernel(
     const int32_t* __restrict__ ranges, const int32_t* __restrict__ ids, const float4* __restrict__ splats,
     const float* __restrict__ final_T, const int32_t* __restrict__ final_idx, const float* __restrict__ v_image,
     const float* __restrict__ bg, float* grads, uint8_t* marks, int W, int H, int ntx, uint32_t last_id, int k,
     const int32_t* __restrict__ header, int header_shift, const BinLists lists, const ZeroJobs zeros)
 {
-    __shared__ float4 s_a[kBwdBatch]; // pixel x, pixel y, conic -a/2, conic b
-    __shared__ float4 s_b[kBwdBatch]; // conic c/2, opacity, red, green
-    __shared__ float s_c[kBwdBatch];  // blue
+    // (the last place: nobody's entry, as in the forward)
+    __shared__ float4 s_a[kBwdBatch + 1]; // pixel x, pixel y, conic a/2, conic b
+    __shared__ float4 s_b[kBwdBatch + 1]; // conic c/2, log2(opacity), limit of sigma's bits, index in the sorted key array
+    __shared__ float s_c[3 * (kBwdBatch + 1)]; // red, green, blue
     __shared__ int s_id[kBwdBatch];
-    // the queue of the tile's own entries (binned lists) lives in s_a between two rounds, as in the forward
-    int* const s_queue = reinterpret_cast<int*>(s_a);
+    __shared__ double s_sum[(kBwdBatch + 1) * kSums];
+    __shared__ uint64_t s_list[4 * kBwdBatch / 8 + 1];
+    // ids of the tile's own entries, on their way from the scan to the gather: in the sums' memory, which is
+    // free while a round is staged
+    int* const s_queue = reinterpret_cast<int*>(s_sum);
+    static_assert(kBwdBatch % 8 == 0 && kBwdBatch < 256 && 4 * kBwdBatch / 8 <= DSX_WAVE, "places are bytes, stored by words");
 
     const int lane = threadIdx.x;
-    const int tile = kBwdPix == 4 ? blockIdx.x : blockIdx.x >> 2;
-    const int band = kBwdPix == 4 ? 0 : blockIdx.x & 3;
-    const int tx = tile % ntx;
-    const int ty = tile / ntx;
-    const int x = tx * kTile + (lane & 15);
-    const int y0 = ty * kTile + 4 * band + (lane >> 4);
-    const float pxf = (float)x + 0.5f;
-    // first pixel centre and last row of the pixels this wavefront owns
-    const float box_x0 = (float)(tx * kTile) + 0.5f, box_y0 = (float)(ty * kTile + 4 * band) + 0.5f;
-    const float span_y = kBwdPix == 4 ? 15.0f : 3.0f;
+    const int row = lane >> 4;
+    const Pixels<kPix> px(blockIdx.x, ntx, lane);
+    const float pxf = (float)px.x + 0.5f;
     const float bg0 = bg[0], bg1 = bg[1], bg2 = bg[2];
+    uint8_t* const list_bytes = reinterpret_cast<uint8_t*>(s_list);
 
     // bterm = -T_final * (bg . v_out) - sum over the entries behind of (rgb . v_out) * alpha * T:
     // the three per-channel colour buffers of cpp/gsplat/backward.cu:156-168 only ever appear
     // dotted with v_out, so one scalar carries them
-    float pyf[kBwdPix], T[kBwdPix], vo0[kBwdPix], vo1[kBwdPix], vo2[kBwdPix], bterm[kBwdPix];
-    int bin_final[kBwdPix];
+    float pyf[kPix], T[kPix], vo0[kPix], vo1[kPix], vo2[kPix], bterm[kPix];
+    int bin_final[kPix];
     int m = -1;
 #pragma unroll
-    for(int p = 0; p < kBwdPix; ++p)
+    for(int p = 0; p < kPix; ++p)
     {
-        const int y = y0 + 4 * p;
-        const bool inside = x < W && y < H;
-        const int64_t pix = inside ? (int64_t)y * W + x : 0;
+        const int y = px.y_of(p);
+        const bool inside = px.x < W && y < H;
+        const int64_t pix = inside ? (int64_t)y * W + px.x : 0;
         pyf[p] = (float)y + 0.5f;
         const float Tf = inside ? final_T[pix] : 0.0f;
         T[p] = Tf;
@@ -698,235 +1203,252 @@ __global__ __launch_bounds__(DSX_WAVE) void blend_bwd_kernel(
         m = max(m, bin_final[p]);
     }
 
-    // last entry (as an index in the sorted key array) that any pixel of this wavefront blended
+    // last entry (as an index in the sorted key array) that any pixel of each row, of the wavefront, blended
 #pragma unroll
-    for(int o = 32; o > 0; o >>= 1)
+    for(int o = 8; o > 0; o >>= 1)
         m = max(m, __shfl_xor(m, o, DSX_WAVE));
+    int m_row[4];
+#pragma unroll
+    for(int r = 0; r < 4; ++r)
+        m_row[r] = __builtin_amdgcn_readlane(m, 16 * r);
+    m = max(max(m_row[0], m_row[1]), max(m_row[2], m_row[3]));
+    if(lane == 0)
+    {
+        // (its index, the largest there is, lies behind every pixel's last entry: no pixel takes it)
+        s_a[kBwdBatch] = make_float4(0.f, 0.f, 0.f, 0.f);
+        s_b[kBwdBatch] = make_float4(0.f, 0.f, 0.f, __int_as_float(INT_MAX));
+        s_c[3 * kBwdBatch] = s_c[3 * kBwdBatch + 1] = s_c[3 * kBwdBatch + 2] = 0.f;
+    }
 
     // lists that were built for another bin size than this launch assumes are not read (see the forward)
     const bool layout_ok = header == nullptr || *header == header_shift;
-    int start = 0, hi = -1;
-    TileSource src = {};
-    // binned lists: the scan of the bin's list, downwards from where the forward's scan stopped
-    uint32_t my_bits = 0u; // the two bits of this wavefront's tile in a pair's key word (high half)
-    int pos = -1;       // next position of the bin's list to look at
-    int rank_next = -1; // rank, in the tile's own list, of the next of its entries to be found
+    int start = 0;
+    int pos = -1;       // next position of the list to look at
+    int left = 0;       // entries of the tile's own list that are still to be found (binned lists)
+    int skip = 0;       // those among the next ones that lie behind everything that was blended (binned lists)
     int idx_next = 0;   // index (in the sorted key array) of the next entry that is handed to the blend
+    TileSource src = {};
+    uint32_t my_bits = 0u; // the two bits of this wavefront's tile in a pair's key word (high half)
     if(kBinned && layout_ok)
     {
         // The forward's scan of the bin's list stopped at position w[0] after meeting w[1] of the
-        // tile's entries (the larger of the four bands' figures: both grow together); everything
+        // tile's entries (the larger of the four parts' figures: both grow together); everything
         // that was blended lies below, and the entries are taken from there downwards.  An entry's
         // index is the tile's range start plus its rank; those above the last blended one (m) are
         // not even queued, so the entries that are handed on have consecutive indices.
-        src = tile_source(lists, tile, ntx);
+        src = tile_source(lists, px.tile, ntx);
         my_bits = tile_bits_of(src, lists.shift) << 16;
         start = max(src.start, 0);
-        const int32_t* w = lists.walk + (int64_t)tile * 8;
+        const int32_t* w = lists.walk + (int64_t)px.tile * 8;
         const int stopped = max(max(w[0], w[2]), max(w[4], w[6]));
         const int seen = max(max(w[1], w[3]), max(w[5], w[7]));
         // (positions outside sorted_ids are not followed, as in the forward)
         pos = min(stopped, min(src.end, k)) - 1;
-        rank_next = min(seen, src.count) - 1;
-        idx_next = min(m, src.fine_base + rank_next);
-        if(src.count <= 0 || idx_next < src.fine_base) // nothing of this tile was blended
+        const int last = src.fine_base + min(seen, src.count) - 1;
+        idx_next = min(m, last);
+        skip = last - idx_next;
+        left = idx_next - src.fine_base + 1;
+        if(src.count <= 0 || left <= 0) // nothing of this tile was blended
             pos = start - 1;
     }
     else if(layout_ok)
     {
-        start = max(ranges[tile], 0);
-        const int end = min(ranges[tile + 1], k);
-        hi = min(end - 1, m);
+        start = max(ranges[px.tile], 0);
+        const int end = min(ranges[px.tile + 1], k);
+        pos = min(end - 1, m);
+        idx_next = pos;
     }
 
-    int g_ahead[kBwdBatch / DSX_WAVE];
+    // where this lane's share of an entry's nine sums goes: lanes 0 and 1 of every bank hold the eight totals
+    // of the reduce-scatter (twice: lanes 2 and 3 too), lane 2 of a row takes the ninth
+    const bool carries_blue = (lane & 15) == 2;
+    const bool carries = (lane & 2) == 0 || carries_blue;
+    const int sum_slot = carries_blue ? 8 : 4 * (lane & 1) + 2 * ((lane >> 2) & 1) + ((lane >> 3) & 1);
+
     const int32_t* const keys = ids + k; // the pairs' key words lie behind the ids (binned lists)
-    if(!kBinned)
+    while(pos >= start && (!kBinned || left > 0))
     {
-        // (ids one round ahead, as in the forward)
-#pragma unroll
-        for(int h = 0; h < kBwdBatch / DSX_WAVE; ++h)
-        {
-            const int e = hi - (h * DSX_WAVE + lane);
-            g_ahead[h] = e >= start ? ids[e] : 0;
-        }
-    }
-    for(int top = hi;; top -= kBwdBatch)
-    {
-        int batch;     // entries of this round
-        int idx_first; // index (in the sorted key array) of the round's first entry; the others follow downwards
         __syncthreads(); // single wavefront: orders the LDS reads of the last round before these writes
-        if(kBinned)
+        if(lane < 4 * kBwdBatch / 8)
+            s_list[lane] = 0x0101010101010101ull * kBwdBatch;
+        int staged = 0;
+        int length[4] = {0, 0, 0, 0};
+        do
         {
-            // (four groups of 64 positions in flight at a time, as in the forward)
-            int count = 0;
-            while(count <= kBwdBatch - DSX_WAVE && pos >= start && rank_next >= 0)
+            int id = 0;
+            int batch; // entries in this gather
+            if(kBinned)
             {
-                int id[kScanGroups], key[kScanGroups];
-#pragma unroll
-                for(int j = 0; j < kScanGroups; ++j)
+                // (four groups of 64 positions in flight at a time, as in the forward)
+                batch = 0;
+                do
                 {
-                    const int e = pos - j * DSX_WAVE - lane;
-                    id[j] = e >= start ? ids[e] : 0;
-                    key[j] = e >= start ? keys[e] : 0;
-                }
+                    int gid[kScanGroups], key[kScanGroups];
 #pragma unroll
-                for(int j = 0; j < kScanGroups; ++j)
-                {
-                    if(count <= kBwdBatch - DSX_WAVE && pos >= start && rank_next >= 0) // (uniform)
+                    for(int j = 0; j < kScanGroups; ++j)
                     {
-                        const bool member = pos - lane >= start && (((uint32_t)key[j]) & my_bits) == my_bits;
-                        const uint64_t mm = __ballot(member);
-                        // lower lanes hold higher positions: this entry's rank is the next one less the members before it
-                        const int rank = rank_next - bits_below_lane(mm);
-                        const bool keep = member && src.fine_base + rank <= m;
-                        const uint64_t mk = __ballot(keep);
-                        if(keep)
-                            s_queue[count + bits_below_lane(mk)] = id[j];
-                        count += __popcll(mk);
-                        rank_next -= __popcll(mm);
-                        pos -= DSX_WAVE;
+                        const uint32_t e = (uint32_t)max(pos - j * DSX_WAVE - lane, start);
+                        gid[j] = word_at(ids, e);
+                        key[j] = word_at(keys, e);
                     }
-                }
-            }
-            if(count == 0)
-                break;
-            __syncthreads();
-            batch = count;
 #pragma unroll
-            for(int h = 0; h < kBwdBatch / DSX_WAVE; ++h)
-                g_ahead[h] = h * DSX_WAVE + lane < batch ? s_queue[h * DSX_WAVE + lane] : 0;
-            __syncthreads(); // the queue has been read: its memory now takes the staged records
-            idx_first = idx_next;
+                    for(int j = 0; j < kScanGroups; ++j)
+                    {
+                        // lower lanes hold higher positions
+                        uint64_t m = __builtin_amdgcn_ballot_w64(((uint32_t)key[j] & my_bits) == my_bits) &
+                                     lanes_below(pos - start + 1);
+                        int taken = min(pos - start + 1, DSX_WAVE);
+                        if(skip > 0)
+                        {
+                            const uint64_t skipped = __popcll(m) > skip ? lowest_bits(m, skip) : m;
+                            skip -= __popcll(skipped);
+                            m &= ~skipped;
+                        }
+                        const int room = DSX_WAVE - batch;
+                        if(__popcll(m) > room)
+                        {
+                            // not all of the group's members fit: it is taken down to the last one that does
+                            m = lowest_bits(m, room);
+                            taken = room > 0 ? DSX_WAVE - __builtin_clzll(m) : 0;
+                        }
+                        if(m != 0)
+                        {
+                            if(__builtin_amdgcn_inverse_ballot_w64(m))
+                                s_queue[batch + bits_below_lane(m)] = gid[j];
+                            batch += __popcll(m);
+                        }
+                        pos -= taken;
+                        if(taken < DSX_WAVE)
+                            break;
+                    }
+                } while(batch < DSX_WAVE && pos >= start && batch < left);
+                left -= batch;
+                __syncthreads();
+                id = s_queue[lane];
+            }
+            else
+            {
+                batch = min(pos - start + 1, DSX_WAVE);
+                if(lane < batch)
+                    id = ids[pos - lane];
+                pos -= batch;
+            }
+            uint32_t reached = 0;
+            float4 q0, q1, q2;
+            StagedOpacity op;
+            const int idx = idx_next - lane;
+            if(lane < batch)
+            {
+                id = (int)min((uint32_t)id, last_id); // (as in the forward)
+                const float4* rec = splats + 3 * (int64_t)id;
+                q0 = rec[0], q1 = rec[1], q2 = rec[2];
+                op = stage_opacity(q1.w);
+                reached = blocks_reached<Pixels<kPix>::kSide>(q0.x, q0.y, q1.x, q1.y, q1.z, op.reach, px.box_x, px.box_y);
+#pragma unroll
+                for(int r = 0; r < 4; ++r)
+                    if(idx > m_row[r]) // behind everything that the row's pixels blended
+                        reached &= ~(1u << r);
+            }
+            const uint64_t m_any = __ballot(reached != 0);
+            const int place = staged + bits_below_lane(m_any);
+            if(reached != 0)
+            {
+                s_a[place] = make_float4(q0.x, q0.y, q1.x * 0.5f, q1.y);
+                s_b[place] = make_float4(q1.z * 0.5f, op.log2, __uint_as_float(reach_limit_bwd(q1.w, op.reach)),
+                                         __int_as_float(idx));
+                s_c[3 * place] = q2.x;
+                s_c[3 * place + 1] = q2.y;
+                s_c[3 * place + 2] = q2.z;
+                s_id[place] = id;
+            }
+#pragma unroll
+            for(int r = 0; r < 4; ++r)
+            {
+                const uint64_t mr = __ballot((reached >> r) & 1);
+                if((reached >> r) & 1)
+                    list_bytes[r * kBwdBatch + length[r] + bits_below_lane(mr)] = (uint8_t)place;
+                length[r] += __popcll(mr);
+            }
+            staged += __popcll(m_any);
             idx_next -= batch;
-        }
-        else
-        {
-            if(top < start)
-                break;
-            batch = min(top - start + 1, kBwdBatch);
-            idx_first = top;
-        }
-        uint64_t todo[kBwdBatch / DSX_WAVE]; // entries of this round that can touch the tile
-#pragma unroll
-        for(int h = 0; h < kBwdBatch / DSX_WAVE; ++h)
-        {
-            const int slot = h * DSX_WAVE + lane;
-            bool useful = false;
-            const int g = (int)min((uint32_t)g_ahead[h], last_id); // (as in the forward)
-            if(slot < batch)
-            {
-                const float4* rec = splats + 3 * (int64_t)g;
-                const float4 q0 = rec[0], q1 = rec[1], q2 = rec[2];
-                s_a[slot] = make_float4(q0.x, q0.y, q1.x * -0.5f, q1.y);
-                s_b[slot] = make_float4(q1.z * 0.5f, q1.w, q2.x, q2.y);
-                s_c[slot] = q2.z;
-                s_id[slot] = g;
-                useful = entry_reaches_tile(q0.x, q0.y, q1.x, q1.y, q1.z, q1.w, box_x0, box_y0, span_y);
-            }
-            todo[h] = __ballot(useful);
-        }
+        } while(staged <= kBwdBatch - DSX_WAVE && pos >= start && (!kBinned || left > 0));
         __syncthreads();
-        if(!kBinned)
+        for(int i = lane; i < staged * kSums; i += DSX_WAVE)
+            s_sum[i] = 0.0;
+        __syncthreads();
+
+        const int rounds = max(max(length[0], length[1]), max(length[2], length[3]));
+        const uint8_t* my_list = list_bytes + row * kBwdBatch;
+        int place = *my_list;
+        for(int i = 0; i < rounds; ++i)
         {
-            // the next round's ids: in flight while this round's entries are blended
-#pragma unroll
-            for(int h = 0; h < kBwdBatch / DSX_WAVE; ++h)
-            {
-                const int e = top - kBwdBatch - (h * DSX_WAVE + lane);
-                g_ahead[h] = e >= start ? ids[e] : 0;
-            }
-        }
-#pragma unroll
-        for(int h = 0; h < kBwdBatch / DSX_WAVE; ++h)
-        for(uint64_t mask = todo[h]; mask != 0; mask &= mask - 1)
-        {
-            const int bit = __builtin_ctzll(mask);
-            const int t = h * DSX_WAVE + bit;
-            const int idx = idx_first - t; // the entry's index in the sorted key array (scalar unit)
-            const float4 A = s_a[t];
-            const float4 B = s_b[t];
-            // the exponent exactly as the forward computed it (pixel - mean); sigma = -exponent
-            const float dxf = pxf - A.x;
-            const ExponentX ex = exponent_x(A.z, A.w, dxf);
-            float alpha[kBwdPix], vis[kBwdPix], dy[kBwdPix]; // dy = pixel - mean here
+            asm("" : "+v"(place)); // (a whole register, as loaded: no masking of the byte)
+            const float4 A = s_a[place];
+            const float4 B = s_b[place];
+            const float red = s_c[3 * place], green = s_c[3 * place + 1], blue = s_c[3 * place + 2];
+            const uint32_t limit = __float_as_uint(B.z);
+            const int idx = __float_as_int(B.w);
+            double* const sums = s_sum + place * kSums + sum_slot;
+            place = *++my_list;
+            // sigma exactly as the forward computed it
+            const float dx = pxf - A.x;
+            const ExponentX ex = exponent_x(A.z, A.w, dx);
+            float raw[kPix], dy[kPix]; // alpha before its clamp; dy = pixel - mean
             // which lanes' pixel p takes part: wavefront masks (each compare's own result register),
             // combined on the scalar unit
-            uint64_t m_valid[kBwdPix];
+            uint64_t m_valid[kPix];
             uint64_t m_any = 0;
 #pragma unroll
-            for(int p = 0; p < kBwdPix; ++p)
+            for(int p = 0; p < kPix; ++p)
             {
+#pragma clang fp contract(off)
                 dy[p] = pyf[p] - A.y;
-                const float power = exponent_xy(ex, B.x, dy[p]);
-                vis[p] = fast_exp(power);
-                alpha[p] = fminf(0.99f, B.y * vis[p]);
+                const float sigma = __builtin_fmaf(__builtin_fmaf(B.x, dy[p], ex.bx), dy[p], ex.ax);
                 m_valid[p] = __builtin_amdgcn_ballot_w64(idx <= bin_final[p]) &
-                             __builtin_amdgcn_ballot_w64(!(power > 0.0f)) &
-                             __builtin_amdgcn_ballot_w64(!(alpha[p] < kAlphaThreshold));
+                             __builtin_amdgcn_ballot_w64(__float_as_uint(sigma) <= limit);
                 m_any |= m_valid[p];
+                raw[p] = __builtin_amdgcn_exp2f(__builtin_fmaf(-sigma, kLog2E, B.y));
             }
             if(m_any == 0)
                 continue;
-            const float blue = s_c[t];
-            float g[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}; // v_x, v_y, v_conic a b c, v_opacity, v_red, v_green
-            float g_blue = 0.f;
-            // dx is the same for the lane's four pixels, so the five geometric sums are built from
-            // three moments over dy of vis * v_alpha (v_sigma without its factor -opacity): S0, S1 (times dy), S2 (times dy^2)
-            float S0 = 0.f, S1 = 0.f, S2 = 0.f;
+            // Per lane, over its pixels (which share dx): the weights of the colour's gradient, and three
+            // moments over dy of w = -v_sigma = raw * v_alpha
+            float v_red = 0.f, v_green = 0.f, v_blue = 0.f, S0 = 0.f, S1 = 0.f, S2 = 0.f;
 #pragma unroll
-            for(int p = 0; p < kBwdPix; ++p)
+            for(int p = 0; p < kPix; ++p)
             {
                 if(__builtin_amdgcn_inverse_ballot_w64(m_valid[p]))
                 {
-                    const float ra = __builtin_amdgcn_rcpf(1.0f - alpha[p]);
+                    const float alpha = fminf(0.99f, raw[p]);
+                    const float ra = __builtin_amdgcn_rcpf(1.0f - alpha);
                     T[p] *= ra;
-                    const float fac = alpha[p] * T[p];
-                    g[6] += fac * vo0[p];
-                    g[7] += fac * vo1[p];
-                    g_blue += fac * vo2[p];
-                    const float rv = B.z * vo0[p] + B.w * vo1[p] + blue * vo2[p];
+                    const float fac = alpha * T[p];
+                    v_red += fac * vo0[p];
+                    v_green += fac * vo1[p];
+                    v_blue += fac * vo2[p];
+                    const float rv = red * vo0[p] + green * vo1[p] + blue * vo2[p];
                     const float v_alpha = rv * T[p] + bterm[p] * ra;
                     bterm[p] -= rv * fac;
-                    // v_sigma = -opacity * vis * v_alpha: the moments are taken of vis * v_alpha (which is
-                    // v_opacity's own term) and the common factor -opacity is applied once per entry
-                    const float va = vis[p] * v_alpha;
-                    const float vady = va * dy[p];
-                    S0 += va;
-                    S1 += vady;
-                    S2 += vady * dy[p];
+                    const float w = raw[p] * v_alpha;
+                    const float wdy = w * dy[p];
+                    S0 += w;
+                    S1 += wdy;
+                    S2 += wdy * dy[p];
                 }
             }
-            g[5] = S0; // v_opacity
-            // the gradients are written with d = mean - pixel: dx = -dxf, and S1 changes sign
-            const float dx = -dxf;
-            S0 *= -B.y;
-            S1 *= B.y;
-            // (the staged coefficients are -a/2, b and c/2; A.z * dxf and A.w * dxf are the exponent's own
-            // first products)
-            {
-#pragma clang fp contract(off)
-                g[0] = __builtin_fmaf(A.w, S1, (A.z * dxf) * (S0 * 2.0f));    // v_sigma (a dx + b dy)
-                g[1] = __builtin_fmaf(B.x, S1 * 2.0f, -((A.w * dxf) * S0)); // v_sigma (b dx + c dy)
-            }
-            g[2] = 0.5f * dx * dx * S0;
-            g[3] = dx * S1;
-            g[4] = -0.5f * B.y * S2;
-            const float total = wave_sum8_scatter(g, lane);
-            g_blue = wave_sum_to_lane63(g_blue);
-            // ONE atomic instruction carries all nine sums, each lane its own address: the first
-            // two lanes of every row hold the eight totals of the reduce-scatter (every lane holds
-            // one), lane 63 the ninth
-            if((lane & 14) == 0 || lane == 63)
-            {
-                const int64_t id = s_id[t];
-                float* rec = grads + id * DSX_GRAD_FLOATS;
-                const int slot = lane == 63 ? 8 : 4 * (lane & 1) + 2 * ((lane >> 4) & 1) + (lane >> 5);
-                unsafeAtomicAdd(rec + slot, lane == 63 ? g_blue : total);
-                if(marks)
-                    marks[id] = 1; // (all nine lanes store the same byte: no branch of its own)
-            }
+            // what is summed over the pixels: the moments of w, 1 | dx | dx^2 | dy | dx dy | dy^2, and the colour's three
+            const float S0x = S0 * dx;
+            const float sum8[8] = {S0, S0x, S0x * dx, S1, S1 * dx, S2, v_red, v_green};
+            const float total = row_sum8_scatter(sum8, lane);
+            v_blue = row_sum(v_blue);
+            if(carries)
+                unsafeAtomicAdd(sums, (double)(carries_blue ? v_blue : total));
         }
+        __syncthreads();
+        for(int e = lane; e < staged; e += DSX_WAVE)
+            moments_to_gradients(s_sum + e * kSums, s_a[e], s_b[e]);
+        __syncthreads();
+        flush_sums(s_sum, s_id, staged, grads, marks, lane, DSX_WAVE);
     }
     // A side job for the memory system, as in the forward: the zeros of the per-Gaussian backward's
     // outputs (that kernel writes only the Gaussians that received a term here), every wavefront a
@@ -934,6 +1456,222 @@ __global__ __launch_bounds__(DSX_WAVE) void blend_bwd_kernel(
     // 0.275 ms instead of 0.250; a few stores in every round of the walk instead: no better).
     if(zeros.any)
         zero_share(zeros, blockIdx.x, gridDim.x, lane, DSX_WAVE);
+}
+
+// the workgroup form (see the forward's): the sums of a round's entries are shared by the four wavefronts
+constexpr int kBwdAtOnce = 2; // entries that a row takes at a time
+template <bool kBinned>
+__global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
+    const int32_t* __restrict__ ranges, const int32_t* __restrict__ ids, const float4* __restrict__ splats,
+    const float* __restrict__ final_T, const int32_t* __restrict__ final_idx, const float* __restrict__ v_image,
+    const float* __restrict__ bg, float* grads, uint8_t* marks, int W, int H, int ntx, uint32_t last_id, int k,
+    const int32_t* __restrict__ header, int header_shift, const BinLists lists, const ZeroJobs zeros)
+{
+    __shared__ float4 s_a[kTileBatch + 1], s_b[kTileBatch + 1];
+    __shared__ float s_c[3 * (kTileBatch + 1)];
+    __shared__ int s_id[kTileBatch];
+    __shared__ double s_sum[(kTileBatch + 1) * kSums];
+    __shared__ uint16_t s_reach[kTileBatch];
+    __shared__ uint32_t s_list[kTileWaves * kTileBatch];
+    __shared__ TileScan s_scan;
+    __shared__ int s_counts[kTileWaves];
+    __shared__ int s_last[4 * kTileWaves]; // per block: the last entry that any of its pixels blended
+    int* const s_queue = reinterpret_cast<int*>(s_sum); // (free while a round is staged)
+
+    const int tid = threadIdx.x, lane = tid & (DSX_WAVE - 1), row = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / DSX_WAVE);
+    const int tile = blockIdx.x;
+    const Pixels<1> px(4 * tile + wave, ntx, lane);
+    const float pxf = (float)px.x + 0.5f, pyf = (float)px.y + 0.5f;
+    const float tile_x = (float)(tile % ntx * kTile) + 0.5f, tile_y = (float)(tile / ntx * kTile) + 0.5f;
+
+    const bool inside = px.x < W && px.y < H;
+    const int64_t pix = inside ? (int64_t)px.y * W + px.x : 0;
+    const float Tf = inside ? final_T[pix] : 0.0f;
+    float T = Tf;
+    const int bin_final = inside ? final_idx[pix] : -1;
+    const float vo0 = inside ? v_image[3 * pix] : 0.f, vo1 = inside ? v_image[3 * pix + 1] : 0.f,
+                vo2 = inside ? v_image[3 * pix + 2] : 0.f;
+    float bterm = -Tf * (bg[0] * vo0 + bg[1] * vo1 + bg[2] * vo2);
+    int m = bin_final;
+#pragma unroll
+    for(int o = 8; o > 0; o >>= 1)
+        m = max(m, __shfl_xor(m, o, DSX_WAVE));
+    if((lane & 15) == 0)
+        s_last[4 * wave + row] = m;
+    if(tid == 0)
+    {
+        s_a[kTileBatch] = make_float4(0.f, 0.f, 0.f, 0.f);
+        s_b[kTileBatch] = make_float4(0.f, 0.f, 0.f, __int_as_float(INT_MAX));
+        s_c[3 * kTileBatch] = s_c[3 * kTileBatch + 1] = s_c[3 * kTileBatch + 2] = 0.f;
+    }
+    __syncthreads();
+    m = s_last[0];
+#pragma unroll
+    for(int b = 1; b < 4 * kTileWaves; ++b)
+        m = max(m, s_last[b]);
+    m = __builtin_amdgcn_readfirstlane(m);
+
+    // (where the lists start: as in the wavefront form)
+    const bool layout_ok = header == nullptr || *header == header_shift;
+    int pos = -1, left = 0, skip = 0, idx_next = 0, wanted = 0;
+    TileSource src = {};
+    uint32_t my_bits = 0u;
+    if(kBinned && layout_ok)
+    {
+        src = tile_source(lists, tile, ntx);
+        my_bits = tile_bits_of(src, lists.shift) << 16;
+        const int start = max(src.start, 0);
+        const int32_t* w = lists.walk + (int64_t)tile * 8;
+        const int stopped = max(max(w[0], w[2]), max(w[4], w[6]));
+        const int seen = max(max(w[1], w[3]), max(w[5], w[7]));
+        pos = min(stopped, min(src.end, k)) - 1;
+        const int last = src.fine_base + min(seen, src.count) - 1;
+        idx_next = min(m, last);
+        skip = last - idx_next;
+        wanted = idx_next - src.fine_base + 1;
+        left = src.count <= 0 || wanted <= 0 ? 0 : pos - start + 1;
+    }
+    else if(layout_ok)
+    {
+        const int start = max(ranges[tile], 0);
+        pos = min(min(ranges[tile + 1], k) - 1, m);
+        idx_next = pos;
+        left = pos - start + 1;
+    }
+    left = __builtin_amdgcn_readfirstlane(left);
+
+    const bool carries_blue = (lane & 15) == 2;
+    const bool carries = (lane & 2) == 0 || carries_blue;
+    const int sum_slot = carries_blue ? 8 : 4 * (lane & 1) + 2 * ((lane >> 2) & 1) + ((lane >> 3) & 1);
+
+    const int32_t* const keys = ids + k;
+    int id_ahead = 0;
+    if(!kBinned && tid < min(left, kTileBatch))
+        id_ahead = ids[pos - tid];
+    while(left > 0 && (!kBinned || wanted > 0))
+    {
+        int id, batch;
+        if(kBinned)
+        {
+            batch = tile_scan<-1>(s_scan, s_queue, ids, keys, pos, left, skip, my_bits, wanted);
+            wanted -= batch;
+            id = tid < batch ? s_queue[tid] : 0;
+        }
+        else
+        {
+            batch = min(left, kTileBatch);
+            id = id_ahead;
+            pos -= batch;
+            left -= batch;
+            if(tid < min(left, kTileBatch))
+                id_ahead = ids[pos - tid];
+        }
+        uint32_t reached = 0;
+        float4 q0, q1, q2;
+        StagedOpacity op;
+        const int idx = idx_next - tid;
+        if(tid < batch)
+        {
+            id = (int)min((uint32_t)id, last_id);
+            const float4* const rec = splats + 3 * (int64_t)id;
+            q0 = rec[0], q1 = rec[1], q2 = rec[2];
+            op = stage_opacity(q1.w);
+#pragma unroll
+            for(int q = 0; q < 4; ++q)
+                reached |= blocks_reached<4>(q0.x, q0.y, q1.x, q1.y, q1.z, op.reach, tile_x + 8.0f * (q & 1), tile_y + 8.0f * (q >> 1)) << (4 * q);
+#pragma unroll
+            for(int b = 0; b < 4 * kTileWaves; ++b)
+                if(idx > s_last[b])
+                    reached &= ~(1u << b);
+        }
+        int staged;
+        const int place = tile_place(s_counts, __builtin_amdgcn_ballot_w64(reached != 0), staged);
+        // (the barrier inside: the queue has been read, the last round's sums have been taken)
+        for(int i = tid; i < staged * kSums; i += kTileThreads)
+            s_sum[i] = 0.0;
+        if(reached != 0)
+        {
+            s_a[place] = make_float4(q0.x, q0.y, q1.x * 0.5f, q1.y);
+            s_b[place] = make_float4(q1.z * 0.5f, op.log2, __uint_as_float(reach_limit_bwd(q1.w, op.reach)),
+                                     __int_as_float(idx));
+            s_c[3 * place] = q2.x;
+            s_c[3 * place + 1] = q2.y;
+            s_c[3 * place + 2] = q2.z;
+            s_id[place] = id;
+            s_reach[place] = (uint16_t)reached;
+        }
+        idx_next -= batch;
+        __syncthreads();
+
+        const int rounds = (build_lists(s_list, s_reach, staged, wave, lane) + kBwdAtOnce - 1) / kBwdAtOnce;
+        const uint16_t* my_list = reinterpret_cast<const uint16_t*>(s_list + wave * kTileBatch + row * (kTileBatch / 4));
+        for(int i = 0; i < rounds; ++i)
+        {
+            const uint32_t places = my_list[i];
+            float4 A[kBwdAtOnce], B[kBwdAtOnce];
+            float dx[kBwdAtOnce], dy[kBwdAtOnce], raw[kBwdAtOnce], alpha[kBwdAtOnce], ra[kBwdAtOnce], rv[kBwdAtOnce];
+            double* sums[kBwdAtOnce];
+            uint64_t m_valid[kBwdAtOnce];
+            uint64_t m_any = 0;
+#pragma unroll
+            for(int u = 0; u < kBwdAtOnce; ++u)
+            {
+                const uint32_t p = (places >> (8 * u)) & 0xffu;
+                A[u] = s_a[p];
+                B[u] = s_b[p];
+                rv[u] = s_c[3 * p] * vo0 + s_c[3 * p + 1] * vo1 + s_c[3 * p + 2] * vo2;
+                sums[u] = s_sum + p * kSums + sum_slot;
+            }
+#pragma unroll
+            for(int u = 0; u < kBwdAtOnce; ++u)
+            {
+#pragma clang fp contract(off)
+                dx[u] = pxf - A[u].x;
+                dy[u] = pyf - A[u].y;
+                const ExponentX ex = exponent_x(A[u].z, A[u].w, dx[u]);
+                const float sigma = __builtin_fmaf(__builtin_fmaf(B[u].x, dy[u], ex.bx), dy[u], ex.ax);
+                m_valid[u] = __builtin_amdgcn_ballot_w64(__float_as_int(B[u].w) <= bin_final) &
+                             __builtin_amdgcn_ballot_w64(__float_as_uint(sigma) <= __float_as_uint(B[u].z));
+                m_any |= m_valid[u];
+                raw[u] = __builtin_amdgcn_exp2f(__builtin_fmaf(-sigma, kLog2E, B[u].y));
+                alpha[u] = fminf(0.99f, raw[u]);
+                ra[u] = __builtin_amdgcn_rcpf(1.0f - alpha[u]);
+            }
+            if(m_any == 0)
+                continue;
+#pragma unroll
+            for(int u = 0; u < kBwdAtOnce; ++u)
+            {
+                float w = 0.f, v_red = 0.f, v_green = 0.f, v_blue = 0.f;
+                if(__builtin_amdgcn_inverse_ballot_w64(m_valid[u]))
+                {
+                    T *= ra[u];
+                    const float fac = alpha[u] * T;
+                    v_red = fac * vo0;
+                    v_green = fac * vo1;
+                    v_blue = fac * vo2;
+                    const float v_alpha = rv[u] * T + bterm * ra[u];
+                    bterm -= rv[u] * fac;
+                    w = raw[u] * v_alpha;
+                }
+                const float wx = w * dx[u], wy = w * dy[u];
+                const float sum8[8] = {w, wx, wx * dx[u], wy, wy * dx[u], wy * dy[u], v_red, v_green};
+                const float total = row_sum8_scatter(sum8, lane);
+                v_blue = row_sum(v_blue);
+                if(carries)
+                    unsafeAtomicAdd(sums[u], (double)(carries_blue ? v_blue : total));
+            }
+        }
+        __syncthreads();
+        for(int e = tid; e < staged; e += kTileThreads)
+            moments_to_gradients(s_sum + e * kSums, s_a[e], s_b[e]);
+        __syncthreads();
+        flush_sums(s_sum, s_id, staged, grads, marks, tid, kTileThreads);
+        __syncthreads();
+    }
+    if(zeros.any)
+        zero_share(zeros, blockIdx.x, gridDim.x, tid, kTileThreads);
 }
 
 // ranges, check_header, n, k: as for launch_blend_fwd (the kernel reads the `walk` part that the forward wrote)
@@ -962,20 +1700,20 @@ int launch_blend_bwd(const dsx_camera& cam, int64_t n, int64_t k, const int32_t*
     {
         DSX_TIMED("blend_bwd_kernel", stream);
         const bool four = blend_pixels_per_lane(ntx * nty, kBwdFourPixelsFrom) == 4;
-        const dim3 grid(four ? ntx * nty : 4 * ntx * nty);
+        const dim3 grid(ntx * nty);
         const float4* sp = reinterpret_cast<const float4*>(splats);
-#define DSX_LAUNCH_BWD(PIX, BINNED)                                                                              \
-    hipLaunchKernelGGL((blend_bwd_kernel<PIX, BINNED>), grid, dim3(DSX_WAVE), 0, stream, ranges, sorted_ids, sp,   \
-                       final_T, final_idx, v_image, cam.bg, grads, with_marks ? grad_marks(grads, n) : nullptr,       \
-                       cam.image_width, cam.image_height, ntx, last_id, (int)k, header, lg.shift, L, Z)
+#define DSX_LAUNCH_BWD(KERNEL, THREADS)                                                                          \
+    hipLaunchKernelGGL((KERNEL), grid, dim3(THREADS), 0, stream, ranges, sorted_ids, sp, final_T, final_idx, v_image, \
+                       cam.bg, grads, with_marks ? grad_marks(grads, n) : nullptr, cam.image_width,                 \
+                       cam.image_height, ntx, last_id, (int)k, header, lg.shift, L, Z)
         if(four && lg.shift)
-            DSX_LAUNCH_BWD(4, true);
+            DSX_LAUNCH_BWD(blend_bwd_kernel<true>, DSX_WAVE);
         else if(four)
-            DSX_LAUNCH_BWD(4, false);
+            DSX_LAUNCH_BWD(blend_bwd_kernel<false>, DSX_WAVE);
         else if(lg.shift)
-            DSX_LAUNCH_BWD(1, true);
+            DSX_LAUNCH_BWD(blend_bwd_tile_kernel<true>, kTileThreads);
         else
-            DSX_LAUNCH_BWD(1, false);
+            DSX_LAUNCH_BWD(blend_bwd_tile_kernel<false>, kTileThreads);
 #undef DSX_LAUNCH_BWD
     }
     DSX_LAUNCH_CHECK();
