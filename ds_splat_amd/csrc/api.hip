@@ -513,6 +513,49 @@ static int check_pair_counts(int64_t list_pairs, int64_t tile_pairs)
     return DSX_OK;
 }
 
+// Two words of pinned host memory per host thread (given back when the thread ends), which the device writes.
+namespace
+{
+struct PinnedCounts
+{
+    int64_t* words = nullptr;
+    ~PinnedCounts()
+    {
+        if(words)
+            (void)hipHostFree(words);
+    }
+};
+volatile int64_t* pinned_counts()
+{
+    thread_local PinnedCounts mine;
+    if(mine.words == nullptr)
+    {
+        void* p = nullptr;
+        if(hipHostMalloc(&p, 2 * sizeof(int64_t), hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
+            return nullptr;
+        mine.words = static_cast<int64_t*>(p);
+    }
+    return mine.words;
+}
+// Waits until both words are there.  Every wait ends: when the stream has run dry (or into an error) without them.
+bool wait_for_counts(volatile int64_t* counts, hipStream_t stream)
+{
+    for(int64_t spins = 1;; ++spins)
+    {
+        if(counts[0] >= 0 && counts[1] >= 0)
+            return true;
+        __builtin_ia32_pause();
+        if((spins & 0xffff) == 0)
+        {
+            const hipError_t e = hipStreamQuery(stream);
+            if(e == hipErrorNotReady)
+                continue;
+            return e == hipSuccess && counts[0] >= 0 && counts[1] >= 0;
+        }
+    }
+}
+} // namespace
+
 extern "C" int dsx_forward_project(const dsx_camera* cam, int64_t n, const float* means3d, const float* scales,
                                    const float* quats, const float* opacities, const float* shs,
                                    const float* cov3d_precomp, const float* colors_precomp, float* splats,
@@ -527,21 +570,20 @@ extern "C" int dsx_forward_project(const dsx_camera* cam, int64_t n, const float
                                  splats, radii, cov3d, block_sums, order, order_bytes, stream, true);
     if(rc || n == 0)
         return rc;
-    // The pair counts are sums over the rectangles: the corner-grid kernel, first thing beside the
-    // depth sort, adds them up, and they travel to the host while the depth order is computed.  The
-    // wait below is for that copy only (it overlaps when num_keys is pinned host memory; with
-    // pageable memory the copy is synchronous and nothing is lost).
-    hipEvent_t copied;
-    if(hipEventCreateWithFlags(&copied, hipEventDisableTiming) != hipSuccess)
+    // The pair counts are sums over the rectangles: the kernel that counts the tiles, first thing beside the
+    // depth sort, writes them into pinned host memory, where this thread waits for them while the
+    // depth order is computed (no copy, no event).
+    volatile int64_t* const counts = pinned_counts();
+    if(counts == nullptr)
         return DSX_ERR_RUNTIME;
-    rc = launch_depth_order(*cam, n, order, s, true, num_keys, copied);
-    // (an event that was never recorded counts as complete: no wait after a failed launch)
-    const bool ok = hipEventSynchronize(copied) == hipSuccess;
-    (void)hipEventDestroy(copied);
+    counts[0] = counts[1] = -1;
+    rc = launch_depth_order(*cam, n, order, s, true, const_cast<int64_t*>(counts));
     if(rc)
         return rc;
-    if(!ok)
+    if(!wait_for_counts(counts, s))
         return DSX_ERR_RUNTIME;
+    num_keys[0] = counts[0];
+    num_keys[1] = counts[1];
     // the device wrote (per-tile pairs, bin pairs); the caller gets (pairs of the lists, per-tile pairs)
     const int64_t tile_pairs = num_keys[0], bin_pairs = num_keys[1];
     num_keys[0] = list_grid(*cam).shift ? bin_pairs : tile_pairs;

@@ -97,14 +97,15 @@ __device__ __forceinline__ uint32_t wave_incl_max_scan(uint32_t v)
     return v;
 }
 
-// lanes of the wavefront that hold the same (up to 8-bit) digit; uniform flow only
-__device__ __forceinline__ uint64_t match_digit8(uint32_t d, int bits)
+// lanes of the wavefront that hold the same digit of up to kMaxBits bits; uniform flow only
+template <int kMaxBits>
+__device__ __forceinline__ uint64_t match_digit(uint32_t d, int bits)
 {
     uint32_t lo = 0xffffffffu, hi = 0xffffffffu;
 #pragma unroll
-    for(int b = 0; b < kBits32; ++b)
+    for(int b = 0; b < kMaxBits; ++b)
     {
-        if(b >= bits) // uniform: digits narrower than 8 bits need fewer rounds
+        if(b >= bits) // uniform: narrower digits need fewer rounds
             break;
         uint32_t x = (uint32_t)(((int32_t)(d << (31 - b))) >> 31); // all ones where bit b is set
         asm volatile("" : "+v"(x)); // the ballot tests x itself (one compare), not a second copy of the bit
@@ -312,7 +313,7 @@ __global__ __launch_bounds__(kSort32Threads) void onesweep32_kernel(
     for(int it = 0; it < kSort32Items; ++it)
     {
         const uint32_t d = (key[it] >> shift) & mask;
-        const uint64_t m = match_digit8(d, bits);
+        const uint64_t m = match_digit<kBits32>(d, bits);
         const uint32_t below = (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
         const uint32_t old = wh[d];
         __builtin_amdgcn_wave_barrier();
@@ -711,7 +712,7 @@ OrderLayout order_layout(int64_t n, int image_width, int image_height, int list_
         off += (size_t)((g.nbx + 1) * (g.nby + 1) + 1) * 4;
     off = (off + 7) & ~(size_t)7;
     o.key_count = off; // inside the region that is zeroed with the corner grids
-    off = align(off + 16);
+    off = align(off + 24);
     o.ranges = off;
     off += (size_t)ranges_layout(g).ready * 4;
     o.bytes = align(off);
@@ -771,6 +772,12 @@ __global__ __launch_bounds__(kProjBlock) void ordered_block_sums_kernel(const ui
         block_sums[blockIdx.x] = wave_sums[0] + wave_sums[1] + wave_sums[2] + wave_sums[3];
 }
 
+// a word of pinned host memory that the host polls
+__device__ __forceinline__ void store_to_host(unsigned long long* p, unsigned long long v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // How many pairs each tile receives, straight from the rectangles (no pair is enumerated):
 // a rectangle [sx, ex) x [sy, ey) adds +1, -1, -1, +1 at its four corners of a
 // (nty + 1) x (ntx + 1) grid, and the two-dimensional prefix sum of that grid is the number of
@@ -788,7 +795,8 @@ __global__ __launch_bounds__(kCoverThreads) void tile_cover_kernel(const uint2* 
                                                                    int nty, int shift, int nbx, int nby, int use_lds,
                                                                    int32_t* __restrict__ grid,
                                                                    int32_t* __restrict__ bin_grid,
-                                                                   unsigned long long* __restrict__ key_count)
+                                                                   unsigned long long* __restrict__ key_count,
+                                                                   unsigned long long* k_host)
 {
     extern __shared__ int32_t s_grid[];
     const int tid = threadIdx.x;
@@ -863,13 +871,21 @@ __global__ __launch_bounds__(kCoverThreads) void tile_cover_kernel(const uint2* 
         s_pairs[1][tid >> 6] = bin_pairs;
     }
     __syncthreads();
-    if(tid < 2)
+    if(tid == 0)
     {
-        unsigned long long total = 0;
+        unsigned long long total[2] = {0, 0};
         for(int w = 0; w < kCoverThreads / DSX_WAVE; ++w)
-            total += s_pairs[tid][w];
-        if(total)
-            atomicAdd(key_count + tid, total);
+        {
+            total[0] += s_pairs[0][w];
+            total[1] += s_pairs[1][w];
+        }
+        // The workgroup that is last to add its sums hands them to the waiting host.  The additions have been
+        // performed when their results are back, so the ticket is drawn after them.
+        const unsigned long long before0 = atomicAdd(key_count, total[0]), before1 = atomicAdd(key_count + 1, total[1]);
+        asm volatile("s_waitcnt vmcnt(0)" ::"v"(before0), "v"(before1) : "memory");
+        if(k_host && atomicAdd(key_count + 2, 1ull) == gridDim.x - 1)
+            for(int i = 0; i < 2; ++i)
+                store_to_host(k_host + i, atomicAdd(key_count + i, 0ull));
     }
 }
 
@@ -901,15 +917,13 @@ struct CountsJobs
     CountsJob job[2];
 };
 
-__global__ __launch_bounds__(kCoverThreads) void tile_counts_kernel(const CountsJobs jobs, int use_lds)
+// c: the corner grid, wherever it lies (a workgroup's own copy in LDS, or global memory)
+__device__ __forceinline__ void tile_counts(const CountsJob& J, int32_t* const c)
 {
-    const CountsJob& J = jobs.job[blockIdx.x];
-    int32_t* const grid = J.grid;
     const int ntx = J.ntx, nty = J.nty;
     const Digits32& plan = J.plan;
     uint32_t* const slot_hist = J.slot_hist;
     int32_t* const ranges = J.ranges;
-    extern __shared__ int32_t s_cells[];
     __shared__ uint32_t hist[kMaxPasses32 * kBins32];
     __shared__ __attribute__((aligned(16))) uint32_t wave_tot[kCoverThreads / DSX_WAVE];
     __shared__ uint32_t s_carry;
@@ -919,14 +933,7 @@ __global__ __launch_bounds__(kCoverThreads) void tile_counts_kernel(const Counts
     const int wave = tid >> 6;
     const int pitch = ntx + 1;
     const int cells = pitch * (nty + 1) + 1;
-    const uint32_t negatives = (uint32_t)grid[cells - 1];
-    int32_t* c = grid;
-    if(use_lds)
-    {
-        for(int j = tid; j < cells; j += kCoverThreads)
-            s_cells[j] = grid[j];
-        c = s_cells;
-    }
+    const uint32_t negatives = (uint32_t)c[cells - 1];
     for(int j = tid; j < kMaxPasses32 * kBins32; j += kCoverThreads)
         hist[j] = 0;
     if(tid == 0)
@@ -1038,6 +1045,451 @@ __global__ __launch_bounds__(kCoverThreads) void tile_counts_kernel(const Counts
             slot_hist[j] = hist[j];
 }
 
+__global__ __launch_bounds__(kCoverThreads) void tile_counts_kernel(const CountsJobs jobs, int use_lds)
+{
+    extern __shared__ int32_t s_cells[];
+    const CountsJob& J = jobs.job[blockIdx.x];
+    int32_t* c = J.grid;
+    if(use_lds)
+    {
+        const int cells = (J.ntx + 1) * (J.nty + 1) + 1;
+        for(int j = threadIdx.x; j < cells; j += kCoverThreads)
+            s_cells[j] = J.grid[j];
+        c = s_cells;
+        __syncthreads();
+    }
+    tile_counts(J, c);
+}
+
+// ---------------------------------------------------------------------------------------
+// few Gaussians: depth order and counting in one launch or two
+// ---------------------------------------------------------------------------------------
+// Up to 16384 Gaussians the digit passes, their histogram, the block sums and the scan are eight launches
+// of 3 to 8 us that each do a microsecond's work (2 K Gaussians: 38 us of kernels, 16 K: 50 us).  Here a workgroup
+// sorts 2048 keys in its own LDS and registers (by the digits of the keys' distance from the smallest one, three
+// or fewer for any scene whose depths stay within a factor of eight), and one more (two, for binned lists)
+// fills a corner grid of its own and counts the tiles (and the bins) beside it.  Up to 2048 Gaussians that is
+// all; beyond, a second launch ranks every key among the other workgroups' sorted keys by binary search in LDS.
+// 2 K Gaussians: 10 us, 4 K: 9 + 7, 16 K: 13 + 17 (32 K: 21 + 30, no better than the passes).  (One workgroup for
+// 16 K keys, sixteen to a thread: 51 us.)
+constexpr int kSmallThreads = 1024;
+static_assert(kSmallThreads == kCoverThreads, "tile_counts is written for this many threads");
+constexpr int kSmallItems = 2;
+constexpr int kSmallTile = kSmallThreads * kSmallItems;
+constexpr int kSmallTilesMax = 8;
+constexpr int kSmallMax = kSmallTile * kSmallTilesMax;
+constexpr int kMergeThreads = 256;
+constexpr int kSmallWaves = kSmallThreads / DSX_WAVE;
+constexpr int kSmallDigitBits = 9;
+constexpr int kSmallBins = 1 << kSmallDigitBits;
+
+struct SmallOrder
+{
+    const uint32_t* depth_keys; // by Gaussian
+    const uint2* rects;
+    uint32_t* order; // by depth
+    uint2* rects_sorted;
+    uint32_t* block_sums; // exclusive sums of the list pairs of 256 consecutive Gaussians in depth order, and their total
+    uint32_t *tile_keys, *tile_ids; // several tiles: each one's own order, for the merge
+    unsigned long long* done;       // (merge) workgroups that have added their sums
+    int n, shift, tiles;
+    CountsJobs counts;
+    unsigned long long* k_host;
+};
+
+__device__ __forceinline__ void small_sort(const SmallOrder& J, const int tile, uint32_t* s_mem)
+{
+    constexpr int kItems = kSmallItems;
+    uint32_t* const s_keys = s_mem;
+    uint16_t* const s_ids = reinterpret_cast<uint16_t*>(s_mem + kSmallTile);
+    uint16_t (*const s_whist)[kSmallBins] = reinterpret_cast<uint16_t (*)[kSmallBins]>(s_mem + kSmallTile + kSmallTile / 2);
+    __shared__ uint32_t s_start[kSmallBins];
+    __shared__ __attribute__((aligned(16))) uint32_t s_tot[kSmallWaves];
+    __shared__ uint32_t s_min, s_max;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int base = tile * kSmallTile, n = min(J.n - base, kSmallTile);
+
+    if(tid == 0)
+    {
+        s_min = 0xffffffffu;
+        s_max = 0u;
+    }
+    __syncthreads();
+    // item `it` of a wavefront's lane is input position (wave * kItems + it) * 64 + lane
+    uint32_t key[kItems], id[kItems];
+    uint32_t lo = 0xffffffffu, hi = 0u;
+#pragma unroll
+    for(int it = 0; it < kItems; ++it)
+    {
+        const int i = (wave * kItems + it) * DSX_WAVE + lane;
+        key[it] = i < n ? J.depth_keys[base + i] : kNoPairsKey;
+        id[it] = (uint32_t)i;
+        if(key[it] != kNoPairsKey)
+        {
+            lo = min(lo, key[it]);
+            hi = max(hi, key[it]);
+        }
+    }
+#pragma unroll
+    for(int o = 32; o > 0; o >>= 1)
+    {
+        lo = min(lo, (uint32_t)__shfl_xor(lo, o, DSX_WAVE));
+        hi = max(hi, (uint32_t)__shfl_xor(hi, o, DSX_WAVE));
+    }
+    if(lane == 0)
+    {
+        atomicMin(&s_min, lo);
+        atomicMax(&s_max, hi);
+    }
+    __syncthreads();
+    const uint32_t first = s_min;
+    // distances 0 .. last; those that emit nothing, and the places behind the input, one further
+    const uint32_t last = s_max >= first ? s_max - first : 0u;
+    const uint32_t behind = last < 0xffffffffu ? last + 1u : last; // (keys of all 32-bit values: kNoPairsKey is the largest as it is)
+    const int bits = 32 - __builtin_clz(behind | 1u);
+    const int passes = s_max >= first ? (bits + kSmallDigitBits - 1) / kSmallDigitBits : 0; // nothing emits: in order already
+#pragma unroll
+    for(int it = 0; it < kItems; ++it)
+        key[it] = key[it] == kNoPairsKey ? behind : key[it] - first;
+    for(int p = 0; p < passes; ++p)
+    {
+        const int width = (bits + passes - 1) / passes, shift = p * width;
+        const uint32_t mask = (1u << width) - 1u;
+        for(int j = tid; j < kSmallWaves * kSmallBins / 2; j += kSmallThreads)
+            reinterpret_cast<uint32_t*>(s_whist)[j] = 0;
+        __syncthreads(); // (and the keys and ids of the last pass have been taken)
+        uint32_t place[kItems];
+#pragma unroll
+        for(int it = 0; it < kItems; ++it)
+        {
+            const uint32_t d = (key[it] >> shift) & mask;
+            const uint64_t m = match_digit<kSmallDigitBits>(d, kSmallDigitBits);
+            const uint32_t below = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+            const uint32_t old = s_whist[wave][d];
+            __builtin_amdgcn_wave_barrier();
+            if(below == 0)
+                s_whist[wave][d] = (uint16_t)(old + (uint32_t)__popcll(m));
+            __builtin_amdgcn_wave_barrier();
+            place[it] = old + below;
+        }
+        __syncthreads();
+        uint32_t total = 0;
+        if(tid < kSmallBins)
+        {
+#pragma unroll
+            for(int w = 0; w < kSmallWaves; ++w)
+            {
+                const uint32_t c = s_whist[w][tid];
+                s_whist[w][tid] = (uint16_t)total;
+                total += c;
+            }
+        }
+        const uint32_t incl = wave_incl_scan_u32(total);
+        if(lane == 63)
+            s_tot[wave] = incl;
+        __syncthreads();
+        if(tid < kSmallBins)
+            s_start[tid] = sum_of_waves_before<kSmallBins / DSX_WAVE>(s_tot, wave) + incl - total;
+        __syncthreads();
+#pragma unroll
+        for(int it = 0; it < kItems; ++it)
+        {
+            const uint32_t d = (key[it] >> shift) & mask;
+            const uint32_t at = place[it] + s_start[d] + s_whist[wave][d];
+            s_keys[at] = key[it];
+            s_ids[at] = (uint16_t)id[it];
+        }
+        __syncthreads();
+#pragma unroll
+        for(int it = 0; it < kItems; ++it)
+        {
+            const int i = (wave * kItems + it) * DSX_WAVE + lane;
+            key[it] = s_keys[i];
+            id[it] = s_ids[i];
+        }
+    }
+    if(J.tiles > 1)
+    {
+        // one of several: this tile's order, for the merge (whose block sums start at zero)
+#pragma unroll
+        for(int it = 0; it < kItems; ++it)
+        {
+            const int i = (wave * kItems + it) * DSX_WAVE + lane;
+            if(i < n)
+            {
+                J.tile_keys[base + i] = key[it] == behind ? kNoPairsKey : key[it] + first;
+                J.tile_ids[base + i] = (uint32_t)base + id[it];
+            }
+        }
+        if(tile == 0 && tid <= kSmallMax / kProjBlock && tid <= (J.n + kProjBlock - 1) / kProjBlock)
+            J.block_sums[tid] = 0;
+        return;
+    }
+    // the order, the rectangles in it, and the blocks' sums
+    __syncthreads();
+    uint32_t* const s_groups = s_keys; // pairs of 64 consecutive Gaussians
+#pragma unroll
+    for(int it = 0; it < kItems; ++it)
+    {
+        const int i = (wave * kItems + it) * DSX_WAVE + lane;
+        uint32_t pairs = 0;
+        if(i < n)
+        {
+            const uint2 r = J.rects[id[it]];
+            J.order[i] = id[it];
+            J.rects_sorted[i] = r;
+            pairs = list_count(r, J.shift);
+        }
+        const uint32_t sum = wave_incl_scan_u32(pairs);
+        if(lane == 63)
+            s_groups[wave * kItems + it] = sum;
+    }
+    __syncthreads();
+    if(wave == 0)
+    {
+        const int blocks = (n + kProjBlock - 1) / kProjBlock; // (at most eight)
+        uint32_t sum = 0;
+        if(lane < blocks)
+            for(int g = 0; g < kProjBlock / DSX_WAVE; ++g)
+                sum += s_groups[lane * (kProjBlock / DSX_WAVE) + g];
+        const uint32_t incl = wave_incl_scan_u32(sum);
+        if(lane < blocks)
+            J.block_sums[lane] = incl - sum;
+        if(lane == blocks - 1)
+            J.block_sums[blocks] = incl;
+    }
+    static_assert(kSmallTile / kProjBlock <= DSX_WAVE, "one lane per block");
+}
+
+// The place of every key in the whole order: its place in its own tile and, for every other tile, the number of that
+// tile's keys before it (an equal key of an earlier tile comes first: the order is stable).
+__global__ __launch_bounds__(kMergeThreads) void order_merge_kernel(const SmallOrder J)
+{
+    extern __shared__ uint32_t s_small[]; // all keys, tile after tile
+    __shared__ uint32_t s_sums[kSmallMax / kProjBlock + 1];
+    __shared__ int s_last;
+    const int tid = threadIdx.x;
+    const int blocks = (J.n + kProjBlock - 1) / kProjBlock;
+    for(int j = tid; j < (J.n + 3) / 4; j += kMergeThreads) // (the buffers are padded to 256 bytes)
+        reinterpret_cast<uint4*>(s_small)[j] = reinterpret_cast<const uint4*>(J.tile_keys)[j];
+    for(int j = tid; j < blocks; j += kMergeThreads)
+        s_sums[j] = 0;
+    const int i = blockIdx.x * kMergeThreads + tid;
+    uint32_t id = 0;
+    uint2 r = make_uint2(0u, 0u);
+    if(i < J.n)
+    {
+        id = J.tile_ids[i];
+        r = J.rects[id];
+    }
+    __syncthreads();
+    if(i < J.n)
+    {
+        const uint32_t key = s_small[i];
+        const int mine = i / kSmallTile;
+        int rank = i - mine * kSmallTile;
+        // (four tiles at a time: a search is a chain of a dozen dependent LDS reads)
+        for(int t0 = 0; t0 < J.tiles; t0 += 4)
+        {
+            int before[4] = {0, 0, 0, 0};
+#pragma unroll
+            for(int step = kSmallTile; step > 0; step >>= 1)
+#pragma unroll
+                for(int u = 0; u < 4; ++u)
+                {
+                    // the number of keys of tile t below `key` (or equal to it, for an earlier tile)
+                    const int t = t0 + u, count = min(max(J.n - t * kSmallTile, 0), kSmallTile);
+                    const int at = before[u] + step;
+                    const uint32_t other = s_small[min(t * kSmallTile + at, J.n) - 1];
+                    if(at <= count && (t < mine ? other <= key : other < key))
+                        before[u] = at;
+                }
+#pragma unroll
+            for(int u = 0; u < 4; ++u)
+                rank += t0 + u == mine ? 0 : before[u];
+        }
+        J.order[rank] = id;
+        J.rects_sorted[rank] = r;
+        const uint32_t pairs = list_count(r, J.shift);
+        if(pairs)
+            atomicAdd(&s_sums[rank / kProjBlock], pairs);
+    }
+    __syncthreads();
+    // The blocks' sums over the workgroups; the last one to add its own turns them into exclusive prefixes.
+    // (An addition has been performed when its result is back; every wavefront's are before the barrier.)
+    for(int j = tid; j < blocks; j += kMergeThreads)
+    {
+        const uint32_t before = s_sums[j] ? atomicAdd(&J.block_sums[j], s_sums[j]) : 0u;
+        asm volatile("s_waitcnt vmcnt(0)" ::"v"(before) : "memory");
+    }
+    __syncthreads();
+    if(tid == 0)
+        s_last = atomicAdd(J.done, 1ull) == gridDim.x - 1;
+    __syncthreads();
+    if(s_last && tid < DSX_WAVE)
+    {
+        uint32_t carry = 0;
+        for(int b0 = 0; b0 < blocks; b0 += DSX_WAVE)
+        {
+            const int b = b0 + tid;
+            const uint32_t sum = b < blocks ? atomicAdd(&J.block_sums[b], 0u) : 0u;
+            const uint32_t incl = wave_incl_scan_u32(sum);
+            if(b < blocks)
+                J.block_sums[b] = carry + incl - sum;
+            carry += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+        }
+        if(tid == 0)
+            J.block_sums[blocks] = carry;
+    }
+}
+
+// the corner grid of all rectangles (of their bins when `bins`) in LDS, the pairs' number to the host, the counts
+__device__ __forceinline__ void small_counts(const SmallOrder& J, const bool bins, int32_t* s_grid)
+{
+    __shared__ unsigned long long s_pairs;
+    const CountsJob& C = J.counts.job[bins ? 1 : 0];
+    const int tid = threadIdx.x;
+    const int pitch = C.ntx + 1, cells = pitch * (C.nty + 1) + 1;
+    for(int j = tid; j < cells; j += kSmallThreads)
+        s_grid[j] = 0;
+    if(tid == 0)
+        s_pairs = 0ull;
+    __syncthreads();
+    unsigned long long pairs = 0;
+    for(int g = tid; g < J.n; g += kSmallThreads)
+    {
+        const uint2 r = J.rects[g];
+        int w = (int)(r.y & 0xffffu), h = (int)((r.y >> 16) & 0x7fffu);
+        if(w == 0 || h == 0)
+            continue;
+        int sx = (int)(r.x & 0xffffu), sy = (int)(r.x >> 16);
+        if(r.y >> 31)
+        {
+            pairs += (unsigned long long)(w * h);
+            atomicAdd(&s_grid[cells - 1], w * h);
+            continue;
+        }
+        if(bins)
+        {
+            const BinRect b = bin_rect(r, J.shift);
+            sx = (int)b.bx;
+            sy = (int)b.by;
+            w = (int)b.bw;
+            h = (int)b.bh;
+        }
+        pairs += (unsigned long long)(w * h);
+        atomicAdd(&s_grid[sy * pitch + sx], 1);
+        atomicAdd(&s_grid[sy * pitch + sx + w], -1);
+        atomicAdd(&s_grid[(sy + h) * pitch + sx], -1);
+        atomicAdd(&s_grid[(sy + h) * pitch + sx + w], 1);
+    }
+#pragma unroll
+    for(int o = 32; o > 0; o >>= 1)
+        pairs += __shfl_xor(pairs, o, DSX_WAVE);
+    if((tid & 63) == 0 && pairs)
+        atomicAdd(&s_pairs, pairs);
+    __syncthreads();
+    if(tid == 0 && J.k_host)
+    {
+        store_to_host(J.k_host + (bins ? 1 : 0), s_pairs);
+        if(J.shift == 0)
+            store_to_host(J.k_host + 1, 0ull);
+    }
+    tile_counts(C, s_grid);
+}
+
+__global__ __launch_bounds__(kSmallThreads) void order_small_kernel(const SmallOrder J)
+{
+    extern __shared__ uint32_t s_small[];
+    // (the counting first: the host waits for its sums)
+    const int counting = J.shift ? 2 : 1;
+    if((int)blockIdx.x < counting)
+        small_counts(J, blockIdx.x == 1, reinterpret_cast<int32_t*>(s_small));
+    else
+        small_sort(J, (int)blockIdx.x - counting, s_small);
+}
+
+// true: done (or failed: *rc).  false: too many Gaussians, or a corner grid that does not fit the LDS
+static bool launch_order_small(const ListGrid& lg, int64_t n, char* base, const OrderLayout& o, void* k_host,
+                               const CountsJobs& jobs, hipStream_t stream, int* rc)
+{
+    const int cells = (lg.ntx + 1) * (lg.nty + 1) + 1;
+    if(n > kSmallMax || cells > kCoverLdsCellsLarge - 4096) // (less what the kernel has besides)
+        return false;
+    const size_t sort_bytes = (size_t)kSmallTile * 6 + (size_t)kSmallWaves * kSmallBins * 2;
+    const size_t bytes = std::max(sort_bytes, (size_t)cells * 4), merge_bytes = ((size_t)n * 4 + 15) & ~(size_t)15;
+    auto allow = [](const void* kernel, size_t want) {
+        if(want <= 65536 - 8192 ||
+           hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)want) == hipSuccess)
+            return true;
+        (void)hipGetLastError();
+        return false;
+    };
+    if(!allow(reinterpret_cast<const void*>(order_small_kernel), bytes) ||
+       !allow(reinterpret_cast<const void*>(order_merge_kernel), merge_bytes))
+        return false;
+    SmallOrder J;
+    J.depth_keys = reinterpret_cast<const uint32_t*>(base + o.depth_keys);
+    J.rects = reinterpret_cast<const uint2*>(base + o.rects);
+    J.order = reinterpret_cast<uint32_t*>(base + o.ids_a);
+    J.rects_sorted = reinterpret_cast<uint2*>(base + o.rects_sorted);
+    J.block_sums = reinterpret_cast<uint32_t*>(base + o.block_sums);
+    J.tile_keys = reinterpret_cast<uint32_t*>(base + o.keys_alt);
+    J.tile_ids = reinterpret_cast<uint32_t*>(base + o.ids_b);
+    J.done = reinterpret_cast<unsigned long long*>(base + o.key_count) + 2;
+    J.n = (int)n;
+    J.shift = lg.shift;
+    J.tiles = (int)((n + kSmallTile - 1) / kSmallTile);
+    J.counts = jobs;
+    J.k_host = static_cast<unsigned long long*>(k_host);
+    {
+        DSX_TIMED("order_small_kernel", stream);
+        hipLaunchKernelGGL(order_small_kernel, dim3(J.tiles + (lg.shift ? 2 : 1)), dim3(kSmallThreads), bytes, stream, J);
+    }
+    if(J.tiles > 1)
+    {
+        DSX_TIMED("order_merge_kernel", stream);
+        hipLaunchKernelGGL(order_merge_kernel, dim3((unsigned)((n + kMergeThreads - 1) / kMergeThreads)),
+                           dim3(kMergeThreads), merge_bytes, stream, J);
+    }
+    *rc = hipGetLastError() == hipSuccess ? DSX_OK : DSX_ERR_LAUNCH;
+    return true;
+}
+
+// the counting of the tiles and, for binned lists, of the bins
+static CountsJobs counts_jobs(const ListGrid& lg, char* base, const OrderLayout& o)
+{
+    const RangesLayout rl = ranges_layout(lg);
+    int32_t* const ranges = reinterpret_cast<int32_t*>(base + o.ranges);
+    CountsJobs jobs;
+    CountsJob& fine = jobs.job[0];
+    fine.grid = reinterpret_cast<int32_t*>(base + o.cover);
+    fine.ntx = lg.ntx;
+    fine.nty = lg.nty;
+    fine.plain = 0;
+    fine.plan = digits32(slot_bits(lg.tiles()));
+    fine.slot_hist = lg.shift ? nullptr : reinterpret_cast<uint32_t*>(base + o.slot_hist);
+    fine.ranges = ranges + rl.fine;
+    fine.last = lg.shift ? ranges + rl.last_tile : nullptr;
+    fine.header = ranges + rl.header;
+    fine.header_value = lg.shift;
+    jobs.job[1] = fine;
+    if(lg.shift)
+    {
+        CountsJob& bins = jobs.job[1];
+        bins.grid = reinterpret_cast<int32_t*>(base + o.bin_cover);
+        bins.ntx = lg.nbx;
+        bins.nty = lg.nby;
+        bins.plain = 1;
+        bins.plan = digits32(slot_bits(lg.bins()));
+        bins.slot_hist = reinterpret_cast<uint32_t*>(base + o.slot_hist);
+        bins.ranges = ranges + rl.bins;
+        bins.last = nullptr;
+        bins.header = nullptr;
+    }
+    return jobs;
+}
+
 // order: the buffer of order_layout(n) whose depth_keys and rects the projection has written
 void depth_order_clear_region(const dsx_camera& cam, int64_t n, void* order, uint32_t** words, int64_t* count)
 {
@@ -1048,10 +1500,11 @@ void depth_order_clear_region(const dsx_camera& cam, int64_t n, void* order, uin
     *count = (int64_t)((w.bytes + (o.ranges - o.cover)) / 4);
 }
 
-// k_host (optional, with k_copied): receives the two pair counts (uint64[2]: per-tile lists, bin lists) as
-// soon as the rectangles have been counted; k_copied is recorded behind that copy.
+// k_host (optional): two words of pinned host memory that receive the pair counts (per-tile lists: what the
+// reference calls K, the fine ranges and final_idx index that many pairs; bin lists, zero when the lists
+// are per tile) as soon as the rectangles have been counted, while the sort still runs.
 int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_t stream, bool already_cleared,
-                       void* k_host, hipEvent_t k_copied)
+                       void* k_host)
 {
     if(n <= 0)
         return DSX_OK;
@@ -1074,6 +1527,10 @@ int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_
     if(rc)
         return rc;
 
+    const CountsJobs jobs = counts_jobs(list_grid(cam), base, o);
+    if(launch_order_small(list_grid(cam), n, base, o, k_host, jobs, stream, &rc))
+        return rc;
+
     // pairs per tile: digit histograms of the tile partition and the tile ranges that the second
     // half of the forward needs.  They depend on the rectangles only, not on the depth order,
     // so they run on the helper stream beside the sort (fork after the fill, join at the end).
@@ -1090,17 +1547,14 @@ int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_
             side = nullptr;
         }
     }
-    bool k_copy_ok = true;
     {
         hipStream_t cs = side ? side : stream;
         const ListGrid lg = list_grid(cam);
-        const RangesLayout rl = ranges_layout(lg);
         const int ntx = lg.ntx, nty = lg.nty;
         const int cells = (ntx + 1) * (nty + 1) + 1;
         const int bcells = lg.shift ? (lg.nbx + 1) * (lg.nby + 1) + 1 : 0;
         int32_t* grid = reinterpret_cast<int32_t*>(base + o.cover);
         int32_t* bin_grid = reinterpret_cast<int32_t*>(base + o.bin_cover);
-        int32_t* ranges = reinterpret_cast<int32_t*>(base + o.ranges);
         // The corner grids are privatised in LDS whenever they fit (a 4K image has 32 776 cells =
         // 128 KB: one workgroup per CU); beyond 64 KB a kernel needs its limit raised first.
         // Global atomics are the fallback: correct for any grid, but 24 M same-line atomics
@@ -1124,40 +1578,10 @@ int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_
             hipLaunchKernelGGL(tile_cover_kernel, dim3((unsigned)min((int64_t)kCoverBlocks, want)), dim3(kCoverThreads),
                                use_lds ? (size_t)(cells + bcells) * 4 : 0, cs,
                                reinterpret_cast<const uint2*>(base + o.rects), n, ntx, nty, lg.shift, lg.nbx, lg.nby,
-                               use_lds, grid, bin_grid, reinterpret_cast<unsigned long long*>(base + o.key_count));
+                               use_lds, grid, bin_grid, reinterpret_cast<unsigned long long*>(base + o.key_count),
+                               static_cast<unsigned long long*>(k_host));
         }
-        // both pair counts, 16 bytes: of the per-tile lists (what the reference calls K: the fine ranges
-        // and final_idx index that many pairs) and of the bin lists (zero when the lists are per tile)
-        if(k_host)
-            k_copy_ok = hipMemcpyAsync(k_host, base + o.key_count, 16, hipMemcpyDeviceToHost, cs) == hipSuccess &&
-                        hipEventRecord(k_copied, cs) == hipSuccess;
         {
-            CountsJobs jobs;
-            CountsJob& fine = jobs.job[0];
-            fine.grid = grid;
-            fine.ntx = ntx;
-            fine.nty = nty;
-            fine.plain = 0;
-            fine.plan = digits32(slot_bits(lg.tiles()));
-            fine.slot_hist = lg.shift ? nullptr : reinterpret_cast<uint32_t*>(base + o.slot_hist);
-            fine.ranges = ranges + rl.fine;
-            fine.last = lg.shift ? ranges + rl.last_tile : nullptr;
-            fine.header = ranges + rl.header;
-            fine.header_value = lg.shift;
-            jobs.job[1] = fine;
-            if(lg.shift)
-            {
-                CountsJob& bins = jobs.job[1];
-                bins.grid = bin_grid;
-                bins.ntx = lg.nbx;
-                bins.nty = lg.nby;
-                bins.plain = 1;
-                bins.plan = digits32(slot_bits(lg.bins()));
-                bins.slot_hist = reinterpret_cast<uint32_t*>(base + o.slot_hist);
-                bins.ranges = ranges + rl.bins;
-                bins.last = nullptr;
-                bins.header = nullptr;
-            }
             DSX_TIMED("tile_counts_kernel", cs);
             hipLaunchKernelGGL(tile_counts_kernel, dim3(lg.shift ? 2 : 1), dim3(kCoverThreads),
                                use_lds ? (size_t)cells * 4 : 0, cs, jobs, use_lds);
@@ -1178,8 +1602,6 @@ int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_
     };
     if(hipGetLastError() != hipSuccess)
         return finish(DSX_ERR_LAUNCH);
-    if(!k_copy_ok)
-        return finish(DSX_ERR_RUNTIME);
 
     uint32_t *ko, *vo;
     // 32 key bits = 4 passes: the values (iota in pass 0) go b, a, b, a and end in ids_a

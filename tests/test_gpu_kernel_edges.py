@@ -1,0 +1,38 @@
+"""Kernels that are chosen by size, at the sizes where the choice and their tiles end."""
+import numpy as np
+import pytest
+import torch
+
+from ds_splat_amd.synthetic import make_scene
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+
+
+@pytest.mark.parametrize("depths", ["spread", "equal", "ties", "culled"])
+@pytest.mark.parametrize("n", [1, 255, 2048, 2049, 4097, 16383, 16384, 16385])
+def test_depth_order_of_few_gaussians(n, depths):
+    """The depth order is the stable order of the depth bits, its block offsets are the exclusive sums of the tile
+    counts in that order, whichever kernels make it (one launch up to 2048 Gaussians, two up to 16384)."""
+    from ds_splat_amd import stages
+    sc = make_scene("cfg0", n=n, width=200, height=120, seed=5)
+    means = sc["means_3d"].clone()
+    if depths == "equal":
+        means[:, 2] = 4.0
+    elif depths == "ties":
+        means[::7, 2] = means[::7, 2].round()
+    elif depths == "culled":
+        means[:, 0] += 1e4
+    cam = stages.camera_from_scene(sc, DEV, list_bin=1)
+    order = stages.new_order(cam, n, DEV)
+    splats, radii, _, _ = stages.project_fwd(cam, means.to(DEV), sc["scales"].to(DEV), sc["rotations"].to(DEV),
+                                             sc["opacities"].to(DEV), sc["shs"].to(DEV), order=order)
+    keys = order[:4 * n].cpu().numpy().view(np.uint32).copy()
+    perm, offsets = stages.depth_order(cam, n, order)
+    perm, offsets = perm.cpu().numpy().astype(np.int64), offsets.cpu().numpy().astype(np.int64)
+    assert (keys == 0xffffffff).all() == (depths == "culled" or n == 1)   # (the last Gaussian emits nothing)
+    assert (perm == np.argsort(keys, kind="stable")).all()
+    touched = splats[:, 11].contiguous().view(torch.int32).cpu().numpy().astype(np.int64)
+    touched[keys == 0xffffffff] = 0
+    sums = np.add.reduceat(touched[perm], np.arange(0, n, 256))
+    assert (offsets[:len(sums)] == np.cumsum(sums) - sums).all()
