@@ -128,7 +128,7 @@ extern "C" const char* dsx_error_string(int status)
 
 extern "C" int dsx_version(void)
 {
-    return 300;
+    return 310;
 }
 
 extern "C" int64_t dsx_num_blocks(int64_t n)
@@ -556,39 +556,60 @@ bool wait_for_counts(volatile int64_t* counts, hipStream_t stream)
 }
 } // namespace
 
+extern "C" int dsx_forward_project_begin(const dsx_camera* cam, int64_t n, const float* means3d, const float* scales,
+                                         const float* quats, const float* opacities, const float* shs,
+                                         const float* cov3d_precomp, const float* colors_precomp, float* splats,
+                                         int32_t* radii, float* cov3d, uint32_t* block_sums, void* order,
+                                         size_t order_bytes, void* stream)
+{
+    if(n > 0 && !order)
+        return DSX_ERR_BAD_ARG;
+    int rc = project_fwd_checked(cam, n, means3d, scales, quats, opacities, shs, cov3d_precomp, colors_precomp,
+                                 splats, radii, cov3d, block_sums, order, order_bytes, stream, true);
+    if(rc || n == 0)
+        return rc;
+    // The pair counts are sums over the rectangles: the kernel that counts the tiles, first thing beside the
+    // depth sort, writes them into pinned host memory, where the calling thread finds them while the
+    // depth order is computed (no copy, no event).
+    volatile int64_t* const counts = pinned_counts();
+    if(counts == nullptr)
+        return DSX_ERR_RUNTIME;
+    counts[0] = counts[1] = -1;
+    return launch_depth_order(*cam, n, order, as_stream(stream), true, const_cast<int64_t*>(counts));
+}
+
+extern "C" int dsx_forward_project_counts(const dsx_camera* cam, int64_t n, int64_t* num_keys, void* stream)
+{
+    if(!num_keys)
+        return DSX_ERR_BAD_ARG;
+    num_keys[0] = num_keys[1] = 0;
+    if(int rc = check_camera(cam))
+        return rc;
+    if(n <= 0)
+        return n == 0 ? DSX_OK : DSX_ERR_BAD_ARG;
+    volatile int64_t* const counts = pinned_counts();
+    if(counts == nullptr || !wait_for_counts(counts, as_stream(stream)))
+        return DSX_ERR_RUNTIME;
+    // the device wrote (per-tile pairs, bin pairs); the caller gets (pairs of the lists, per-tile pairs)
+    const int64_t tile_pairs = counts[0], bin_pairs = counts[1];
+    num_keys[0] = list_grid(*cam).shift ? bin_pairs : tile_pairs;
+    num_keys[1] = tile_pairs;
+    return check_pair_counts(num_keys[0], num_keys[1]);
+}
+
 extern "C" int dsx_forward_project(const dsx_camera* cam, int64_t n, const float* means3d, const float* scales,
                                    const float* quats, const float* opacities, const float* shs,
                                    const float* cov3d_precomp, const float* colors_precomp, float* splats,
                                    int32_t* radii, float* cov3d, uint32_t* block_sums, void* order, size_t order_bytes,
                                    int64_t* num_keys, void* stream)
 {
-    if(!num_keys || (n > 0 && !order))
+    if(!num_keys)
         return DSX_ERR_BAD_ARG;
     num_keys[0] = num_keys[1] = 0;
-    hipStream_t s = as_stream(stream);
-    int rc = project_fwd_checked(cam, n, means3d, scales, quats, opacities, shs, cov3d_precomp, colors_precomp,
-                                 splats, radii, cov3d, block_sums, order, order_bytes, stream, true);
-    if(rc || n == 0)
+    if(int rc = dsx_forward_project_begin(cam, n, means3d, scales, quats, opacities, shs, cov3d_precomp, colors_precomp,
+                                          splats, radii, cov3d, block_sums, order, order_bytes, stream))
         return rc;
-    // The pair counts are sums over the rectangles: the kernel that counts the tiles, first thing beside the
-    // depth sort, writes them into pinned host memory, where this thread waits for them while the
-    // depth order is computed (no copy, no event).
-    volatile int64_t* const counts = pinned_counts();
-    if(counts == nullptr)
-        return DSX_ERR_RUNTIME;
-    counts[0] = counts[1] = -1;
-    rc = launch_depth_order(*cam, n, order, s, true, const_cast<int64_t*>(counts));
-    if(rc)
-        return rc;
-    if(!wait_for_counts(counts, s))
-        return DSX_ERR_RUNTIME;
-    num_keys[0] = counts[0];
-    num_keys[1] = counts[1];
-    // the device wrote (per-tile pairs, bin pairs); the caller gets (pairs of the lists, per-tile pairs)
-    const int64_t tile_pairs = num_keys[0], bin_pairs = num_keys[1];
-    num_keys[0] = list_grid(*cam).shift ? bin_pairs : tile_pairs;
-    num_keys[1] = tile_pairs;
-    return check_pair_counts(num_keys[0], num_keys[1]);
+    return dsx_forward_project_counts(cam, n, num_keys, stream);
 }
 
 extern "C" int dsx_forward_finish(const dsx_camera* cam, int64_t n, int64_t k, const float* splats,
@@ -674,6 +695,7 @@ extern "C" int dsx_forward_core(const float* means3d, const float* shs, const fl
     cam.campos = campos;
     cam.bg = campos; // unused by the forward
     cam.list_bin = 0;
+    cam.view_transposed = cam.proj_transposed = cam.planar = 0;
     if(int rc = check_camera(&cam))
         return rc;
     if(n < 0 || !image)

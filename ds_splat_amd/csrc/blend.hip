@@ -295,6 +295,13 @@ __device__ __forceinline__ uint64_t lowest_bits(uint64_t mask, int count)
     return __builtin_amdgcn_ballot_w64(bits_below_lane(mask) < count) & mask;
 }
 
+// the value of one lane of each quad of lanes (quad_perm), in all four
+template <int kCtrl>
+__device__ __forceinline__ float quad_lane(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kCtrl, 0xf, 0xf, false));
+}
+
 // A side job for the memory system, which the forward leaves idle: every workgroup prepares
 // its share of the backward's gradient accumulator, twelve floats per Gaussian: the nine sums
 // zeroed and, in the three spare places, the conic, which the per-Gaussian backward then has
@@ -337,6 +344,23 @@ constexpr int kScanGroups = 4; // groups of 64 positions of a bin's list whose l
 
 typedef float dsx_f32x4 __attribute__((ext_vector_type(4)));
 
+// Stores one pixel per lane: a lane's four neighbours lie in one row of pixels, and its registers are one channel of
+// all of them.  planar: the image is channel-first and has the background composited (the transmittance of
+// the quad's pixels comes from their lanes).
+__device__ __forceinline__ void store_colours(float* image, const dsx_f32x4 colour, float T, int x, int y, int W, int H, int lane,
+                                              bool broken, const float* bg, int planar)
+{
+    const int quad_x = x - (lane & 3), channel = lane & 3;
+    const float back = planar && channel < 3 ? bg[channel] : 0.0f;
+    const float quad_T[4] = {quad_lane<0x00>(T), quad_lane<0x55>(T), quad_lane<0xAA>(T), quad_lane<0xFF>(T)};
+    const int step = planar ? 1 : 3;
+    float* const out = image + (planar ? ((int64_t)channel * H + y) * W + quad_x : 3 * ((int64_t)y * W + quad_x) + channel);
+#pragma unroll
+    for(int r = 0; r < 4; ++r)
+        if(channel < 3 && quad_x + r < W && y < H)
+            out[step * r] = broken ? __builtin_nanf("") : __builtin_fmaf(kAlphaMax, colour[r], planar ? quad_T[r] * back : 0.0f);
+}
+
 // kBinned: the entries come out of the list of the tile's bin (BinLists).  The wavefront first
 // FILTERS the bin's list: 64 positions at a time it reads the pair's id and key word (two coalesced
 // 4-byte loads, those of four groups in flight together), tests the two bits of its tile in the key's mask,
@@ -358,6 +382,7 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(8, 8))
                                                              const uint32_t* __restrict__ sort_flag_b,
                                                              float4* __restrict__ prep, int64_t prep_count,
                                                              uint8_t* __restrict__ prep_marks,
+                                                             const float* __restrict__ bg, int planar,
                                                              const BinLists lists)
 {
     // the last place is nobody's entry (no exponent passes): rows whose list has ended point at it
@@ -604,7 +629,6 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(8, 8))
     // A sort pass that gave up waiting on its predecessor (bounded wait, never seen to happen)
     // leaves its flag set and the tile lists wrong: make that loud instead of plausible.
     const bool broken = !layout_ok || (sort_flag_a && *sort_flag_a) || (sort_flag_b && *sort_flag_b);
-    const int quad_x = px.x - (lane & 3), channel = lane & 3;
 #pragma unroll
     for(int p = 0; p < kPix; ++p)
     {
@@ -615,12 +639,7 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(8, 8))
             final_T[pix] = T[p];
             final_idx[pix] = last[p];
         }
-        // (a lane's four neighbours lie in one row of pixels: its registers are one channel of all of them)
-        float* const out = image + 3 * ((int64_t)y * W + quad_x) + channel;
-#pragma unroll
-        for(int r = 0; r < 4; ++r)
-            if(channel < 3 && quad_x + r < W && y < H)
-                out[3 * r] = broken ? __builtin_nanf("") : kAlphaMax * colour[p][r];
+        store_colours(image, colour[p], T[p], px.x, y, W, H, lane, broken, bg, planar);
     }
     if(kBinned && layout_ok)
     {
@@ -776,6 +795,7 @@ __global__ __launch_bounds__(kTileThreads) void blend_fwd_tile_kernel(const int3
                                                                       const uint32_t* __restrict__ sort_flag_a,
                                                                       const uint32_t* __restrict__ sort_flag_b, float4* __restrict__ prep,
                                                                       int64_t prep_count, uint8_t* __restrict__ prep_marks,
+                                                                      const float* __restrict__ bg, int planar,
                                                                       const BinLists lists)
 {
     // (arrays as in the wavefront form)
@@ -957,18 +977,13 @@ __global__ __launch_bounds__(kTileThreads) void blend_fwd_tile_kernel(const int3
     }
 
     const bool broken = !layout_ok || (sort_flag_a && *sort_flag_a) || (sort_flag_b && *sort_flag_b);
-    const int quad_x = px.x - (lane & 3), channel = lane & 3;
     if(inside)
     {
         const int64_t pix = (int64_t)px.y * W + px.x;
         final_T[pix] = T;
         final_idx[pix] = last;
     }
-    float* const out = image + 3 * ((int64_t)px.y * W + quad_x) + channel;
-#pragma unroll
-    for(int r = 0; r < 4; ++r)
-        if(channel < 3 && quad_x + r < W && px.y < H)
-            out[3 * r] = broken ? __builtin_nanf("") : kAlphaMax * colour[r];
+    store_colours(image, colour, T, px.x, px.y, W, H, lane, broken, bg, planar);
     if(kBinned && layout_ok && tid < 8)
     {
         // (as in the wavefront form, which speaks for the whole tile too)
@@ -1028,7 +1043,7 @@ int launch_blend_fwd(const dsx_camera& cam, int64_t n, int64_t k, int32_t* range
 #define DSX_LAUNCH_FWD(KERNEL, THREADS)                                                                          \
     hipLaunchKernelGGL((KERNEL), grid, dim3(THREADS), 0, stream, ranges, sorted_ids, sp, image, final_T, final_idx,  \
                        cam.image_width, cam.image_height, ntx, last_id, (int)k, header, lg.shift, sort_flag_a,     \
-                       sort_flag_b, prep, prep_count, prep_marks, L)
+                       sort_flag_b, prep, prep_count, prep_marks, cam.bg, cam.planar, L)
         if(four && lg.shift)
             DSX_LAUNCH_FWD(blend_fwd_kernel<true>, DSX_WAVE);
         else if(four)
@@ -1159,7 +1174,7 @@ __global__ __launch_bounds__(DSX_WAVE) void blend_bwd_kernel(
     const int32_t* __restrict__ ranges, const int32_t* __restrict__ ids, const float4* __restrict__ splats,
     const float* __restrict__ final_T, const int32_t* __restrict__ final_idx, const float* __restrict__ v_image,
     const float* __restrict__ bg, float* grads, uint8_t* marks, int W, int H, int ntx, uint32_t last_id, int k,
-    const int32_t* __restrict__ header, int header_shift, const BinLists lists, const ZeroJobs zeros)
+    const int32_t* __restrict__ header, int header_shift, int planar, const BinLists lists, const ZeroJobs zeros)
 {
     // (the last place: nobody's entry, as in the forward)
     __shared__ float4 s_a[kBwdBatch + 1]; // pixel x, pixel y, conic a/2, conic b
@@ -1183,6 +1198,7 @@ __global__ __launch_bounds__(DSX_WAVE) void blend_bwd_kernel(
     // bterm = -T_final * (bg . v_out) - sum over the entries behind of (rgb . v_out) * alpha * T:
     // the three per-channel colour buffers of cpp/gsplat/backward.cu:156-168 only ever appear
     // dotted with v_out, so one scalar carries them
+    const int64_t step = planar ? 1 : 3, plane = planar ? (int64_t)W * H : 1; // of v_image: between pixels, between channels
     float pyf[kPix], T[kPix], vo0[kPix], vo1[kPix], vo2[kPix], bterm[kPix];
     int bin_final[kPix];
     int m = -1;
@@ -1196,9 +1212,9 @@ __global__ __launch_bounds__(DSX_WAVE) void blend_bwd_kernel(
         const float Tf = inside ? final_T[pix] : 0.0f;
         T[p] = Tf;
         bin_final[p] = inside ? final_idx[pix] : -1;
-        vo0[p] = inside ? v_image[3 * pix] : 0.f;
-        vo1[p] = inside ? v_image[3 * pix + 1] : 0.f;
-        vo2[p] = inside ? v_image[3 * pix + 2] : 0.f;
+        vo0[p] = inside ? v_image[step * pix] : 0.f;
+        vo1[p] = inside ? v_image[step * pix + plane] : 0.f;
+        vo2[p] = inside ? v_image[step * pix + 2 * plane] : 0.f;
         bterm[p] = -Tf * (bg0 * vo0[p] + bg1 * vo1[p] + bg2 * vo2[p]);
         m = max(m, bin_final[p]);
     }
@@ -1465,7 +1481,7 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
     const int32_t* __restrict__ ranges, const int32_t* __restrict__ ids, const float4* __restrict__ splats,
     const float* __restrict__ final_T, const int32_t* __restrict__ final_idx, const float* __restrict__ v_image,
     const float* __restrict__ bg, float* grads, uint8_t* marks, int W, int H, int ntx, uint32_t last_id, int k,
-    const int32_t* __restrict__ header, int header_shift, const BinLists lists, const ZeroJobs zeros)
+    const int32_t* __restrict__ header, int header_shift, int planar, const BinLists lists, const ZeroJobs zeros)
 {
     __shared__ float4 s_a[kTileBatch + 1], s_b[kTileBatch + 1];
     __shared__ float s_c[3 * (kTileBatch + 1)];
@@ -1490,8 +1506,9 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
     const float Tf = inside ? final_T[pix] : 0.0f;
     float T = Tf;
     const int bin_final = inside ? final_idx[pix] : -1;
-    const float vo0 = inside ? v_image[3 * pix] : 0.f, vo1 = inside ? v_image[3 * pix + 1] : 0.f,
-                vo2 = inside ? v_image[3 * pix + 2] : 0.f;
+    const int64_t step = planar ? 1 : 3, plane = planar ? (int64_t)W * H : 1; // (between pixels, between channels)
+    const float vo0 = inside ? v_image[step * pix] : 0.f, vo1 = inside ? v_image[step * pix + plane] : 0.f,
+                vo2 = inside ? v_image[step * pix + 2 * plane] : 0.f;
     float bterm = -Tf * (bg[0] * vo0 + bg[1] * vo1 + bg[2] * vo2);
     int m = bin_final;
 #pragma unroll
@@ -1705,7 +1722,7 @@ int launch_blend_bwd(const dsx_camera& cam, int64_t n, int64_t k, const int32_t*
 #define DSX_LAUNCH_BWD(KERNEL, THREADS)                                                                          \
     hipLaunchKernelGGL((KERNEL), grid, dim3(THREADS), 0, stream, ranges, sorted_ids, sp, final_T, final_idx, v_image, \
                        cam.bg, grads, with_marks ? grad_marks(grads, n) : nullptr, cam.image_width,                 \
-                       cam.image_height, ntx, last_id, (int)k, header, lg.shift, L, Z)
+                       cam.image_height, ntx, last_id, (int)k, header, lg.shift, cam.planar, L, Z)
         if(four && lg.shift)
             DSX_LAUNCH_BWD(blend_bwd_kernel<true>, DSX_WAVE);
         else if(four)

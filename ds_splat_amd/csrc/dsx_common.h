@@ -538,6 +538,20 @@ __device__ __forceinline__ void zero_share(const ZeroJobs& jobs, int64_t part, i
         zero_edges(jobs, tid);
 }
 
+// The first kCount elements of a 4x4 matrix, row by row, from memory that holds it row by row or column by column
+// (read whole and in order: one scalar load)
+template <int kCount>
+__device__ __forceinline__ void load_matrix(const float* m, int transposed, float (&out)[kCount])
+{
+    float raw[16];
+#pragma unroll
+    for(int e = 0; e < 16; ++e)
+        raw[e] = m[e];
+#pragma unroll
+    for(int e = 0; e < kCount; ++e)
+        out[e] = transposed ? raw[4 * (e % 4) + e / 4] : raw[e];
+}
+
 struct TileRect
 {
     int sx, ex, sy, ey;

@@ -32,6 +32,7 @@ struct GaussianBwdParams
     const float4* grads;
     const uint8_t* marks; // per Gaussian: did the blend backward add a term? (null: look at the sums)
     const float* view;
+    int view_transposed; // stored column by column
     const float* campos;
     float* v_mean3d;
     float* v_means2d;
@@ -230,7 +231,8 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(3, 3))
             float vc3[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
             if(in.radius > 0)
             {
-                const float* V = p.view;
+                float V[12];
+                load_matrix(p.view, p.view_transposed, V);
                 const float R[3][3] = {{V[0], V[1], V[2]}, {V[4], V[5], V[6]}, {V[8], V[9], V[10]}};
                 const float t[3] = {R[0][0] * mean.x + R[0][1] * mean.y + R[0][2] * mean.z + V[3],
                                     R[1][0] * mean.x + R[1][1] * mean.y + R[1][2] * mean.z + V[7],
@@ -529,6 +531,7 @@ int launch_gaussian_bwd(const dsx_camera& cam, int64_t n, int num_bases, const f
     p.grads = reinterpret_cast<const float4*>(grads);
     p.marks = with_marks ? grad_marks(const_cast<float*>(grads), n) : nullptr;
     p.view = cam.view;
+    p.view_transposed = cam.view_transposed;
     p.campos = cam.campos;
     p.v_mean3d = v_mean3d;
     p.v_means2d = v_means2d;

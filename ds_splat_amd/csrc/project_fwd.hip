@@ -49,6 +49,7 @@ struct ProjectParams
     float focal_x, focal_y, tanfovx, tanfovy, c_x, c_y, scale_modifier;
     int sh_degree, sh_stride; // active degree; floats per shs row
     int ntx, nty;
+    int view_transposed, proj_transposed; // stored column by column
 };
 
 // SH degree 0..3 -> RGB (+0.5, clamped at 0), term order as cpp/rasterizer_kernels.cu:433-554,
@@ -201,7 +202,8 @@ __global__ __launch_bounds__(kProjBlock) void project_fwd_kernel(const ProjectPa
     if(live)
     {
         mean = make_float3(p.means3d[3 * i], p.means3d[3 * i + 1], p.means3d[3 * i + 2]);
-        const float* P = p.proj;
+        float P[16];
+        load_matrix(p.proj, p.proj_transposed, P);
         const float inv_w = 1.0f / (P[12] * mean.x + P[13] * mean.y + P[14] * mean.z + P[15]);
         const float nx = inv_w * (P[0] * mean.x + P[1] * mean.y + P[2] * mean.z + P[3]);
         const float ny = inv_w * (P[4] * mean.x + P[5] * mean.y + P[6] * mean.z + P[7]);
@@ -286,7 +288,8 @@ __global__ __launch_bounds__(kProjBlock) void project_fwd_kernel(const ProjectPa
             rgb = make_float3(p.colors_precomp[3 * i], p.colors_precomp[3 * i + 1], p.colors_precomp[3 * i + 2]);
 
         // view-space position (cpp/rasterizer_kernels.cu:325-330)
-        const float* V = p.view;
+        float V[12];
+        load_matrix(p.view, p.view_transposed, V);
         const float vx = V[0] * mean.x + V[1] * mean.y + V[2] * mean.z + V[3];
         const float vy = V[4] * mean.x + V[5] * mean.y + V[6] * mean.z + V[7];
         const float vz = V[8] * mean.x + V[9] * mean.y + V[10] * mean.z + V[11];
@@ -419,6 +422,8 @@ int launch_project_fwd(const dsx_camera& cam, int64_t n, const float* means3d, c
     p.colors_precomp = colors_precomp;
     p.view = cam.view;
     p.proj = cam.proj;
+    p.view_transposed = cam.view_transposed;
+    p.proj_transposed = cam.proj_transposed;
     p.campos = cam.campos;
     p.splats = reinterpret_cast<float4*>(splats);
     p.radii = radii;

@@ -1,15 +1,17 @@
-// Thin PyTorch binding over the C ABI of libdsx (include/dsx.h): it owns no kernels and no
-// HIP calls.  It plays the role of the reference's pybind module ds_splat_cuda
-// (cpp/rasterizer_python.cpp:3-23) and of the tensor plumbing in cpp/rasterizer_torch.cu:170-316:
-// allocate the outputs as torch tensors, hand raw device pointers and the caller's stream to
-// the library, return the tensors the autograd function keeps for the backward.
+// PyTorch binding over the C ABI of libdsx (include/dsx.h): it owns no kernels.  It plays the role of
+// the reference's pybind module ds_splat_cuda (cpp/rasterizer_python.cpp:3-23), of the tensor
+// plumbing in cpp/rasterizer_torch.cu:170-316 and of the autograd function in ds_splat/rasterizer.py:7-117:
+// check the inputs, allocate the outputs as torch tensors, hand raw device pointers and the current
+// stream to the library.  All of it is native: a small scene's forward takes the device 50 us, and
+// the same steps in Python took the host as long.
 #include <torch/extension.h>
 
 #include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
 
+#include <algorithm>
 #include <stdexcept>
 #include <string>
-#include <tuple>
 #include <vector>
 
 #include "dsx.h"
@@ -17,147 +19,227 @@
 namespace
 {
 
+using OptTensor = c10::optional<at::Tensor>;
+
 void check(int status)
 {
     if(status != DSX_OK)
         throw std::runtime_error(dsx_error_string(status));
 }
 
-const float* fptr(const c10::optional<at::Tensor>& t)
+void require(bool ok, const char* message)
 {
-    return (t.has_value() && t->defined() && t->numel() > 0) ? t->data_ptr<float>() : nullptr;
+    if(!ok)
+        throw std::runtime_error(message);
 }
+
+bool given(const OptTensor& t)
+{
+    return t.has_value() && t->defined() && t->numel() > 0;
+}
+
+const float* fptr(const OptTensor& t)
+{
+    return given(t) ? t->data_ptr<float>() : nullptr;
+}
+
+void* current_stream(const at::Device& dev)
+{
+    return c10::hip::getCurrentHIPStream(dev.index()).stream();
+}
+
+// What a render call is told besides the Gaussians.
+struct Settings
+{
+    int64_t height, width;
+    double tanfovx, tanfovy, scale_modifier;
+    int64_t sh_degree, max_sh_degree;
+    at::Tensor view, proj; // transposed, as the API's users hold them
+    at::Tensor campos, bg;
+    int64_t list_bin; // tiles per side of the bins of the tile lists (0: the library's choice)
+    bool planar;      // [3,H,W] with the background composited instead of [H,W,3] without
+};
 
 struct Camera
 {
-    at::Tensor view, proj, campos, bg; // float32, contiguous, on the device: kept alive for the call
+    at::Tensor view, proj, campos, bg; // float32, on the device: kept alive for the call
     dsx_camera c;
 };
 
-Camera make_camera(int64_t height, int64_t width, double tanfovx, double tanfovy, double scale_modifier,
-                   int64_t sh_degree, int64_t max_sh_degree, const at::Tensor& view, const at::Tensor& proj,
-                   const at::Tensor& campos, const at::Tensor& bg, int64_t list_bin, const at::Device& dev)
+// A matrix as the library takes it: 16 floats and whether they go by columns.  What the user holds is the
+// transpose; a tensor that is itself the transposed view of a contiguous one needs no copy either.
+at::Tensor matrix_of(const at::Tensor& t, const at::Device& dev, int32_t& transposed)
+{
+    at::Tensor m = t.to(dev, at::kFloat);
+    require(m.numel() == 16, "camera tensors must be 4x4, 4x4, [3], [3]");
+    const bool by_columns = m.dim() == 2 && m.stride(0) == 1 && m.stride(1) == 4;
+    transposed = by_columns ? 0 : 1;
+    return by_columns ? m : m.contiguous();
+}
+
+Camera make_camera(const Settings& s, const at::Device& dev)
 {
     Camera cam;
-    auto prep = [&](const at::Tensor& t) { return t.to(dev, at::kFloat).contiguous(); };
-    cam.view = prep(view);
-    cam.proj = prep(proj);
-    cam.campos = prep(campos);
-    cam.bg = prep(bg);
-    TORCH_CHECK(cam.view.numel() == 16 && cam.proj.numel() == 16 && cam.campos.numel() >= 3 && cam.bg.numel() >= 3,
-                "camera tensors must be 4x4, 4x4, [3], [3]");
-    cam.c.image_height = (int32_t)height;
-    cam.c.image_width = (int32_t)width;
-    cam.c.tanfovx = (float)tanfovx;
-    cam.c.tanfovy = (float)tanfovy;
-    cam.c.scale_modifier = (float)scale_modifier;
-    cam.c.sh_degree = (int32_t)sh_degree;
-    cam.c.max_sh_degree = (int32_t)max_sh_degree;
+    cam.view = matrix_of(s.view, dev, cam.c.view_transposed);
+    cam.proj = matrix_of(s.proj, dev, cam.c.proj_transposed);
+    cam.campos = s.campos.to(dev, at::kFloat).contiguous();
+    cam.bg = s.bg.to(dev, at::kFloat).contiguous();
+    require(cam.campos.numel() >= 3 && cam.bg.numel() >= 3, "camera tensors must be 4x4, 4x4, [3], [3]");
+    cam.c.image_height = (int32_t)s.height;
+    cam.c.image_width = (int32_t)s.width;
+    cam.c.tanfovx = (float)s.tanfovx;
+    cam.c.tanfovy = (float)s.tanfovy;
+    cam.c.scale_modifier = (float)s.scale_modifier;
+    cam.c.sh_degree = (int32_t)s.sh_degree;
+    cam.c.max_sh_degree = (int32_t)s.max_sh_degree;
     cam.c.view = cam.view.data_ptr<float>();
     cam.c.proj = cam.proj.data_ptr<float>();
     cam.c.campos = cam.campos.data_ptr<float>();
     cam.c.bg = cam.bg.data_ptr<float>();
-    TORCH_CHECK(list_bin == 0 || list_bin == 1 || list_bin == 2 || list_bin == 4 || list_bin == 8,
-                "list_bin must be 0 (the library's choice), 1, 2, 4 or 8 tiles a side");
-    cam.c.list_bin = (int32_t)list_bin;
+    require(s.list_bin == 0 || s.list_bin == 1 || s.list_bin == 2 || s.list_bin == 4 || s.list_bin == 8,
+            "list_bin must be 0 (the library's choice), 1, 2, 4 or 8 tiles a side");
+    cam.c.list_bin = (int32_t)s.list_bin;
+    cam.c.planar = s.planar ? 1 : 0;
     return cam;
 }
 
-at::Tensor& pinned_key_count()
+// The Gaussians of a call, in the API's order.
+struct Inputs
 {
-    // two pinned int64 per host thread: the landing place of the two pair counts
-    thread_local at::Tensor slot = at::zeros({2}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
-    return slot;
+    at::Tensor means3d, means2d;
+    OptTensor shs, colors;
+    at::Tensor opacities;
+    OptTensor scales, quats, cov3d;
+};
+
+// The checks of rasterizer_forward_deepsense, cpp/rasterizer_torch.cu:176-190 and :124-129, and CHECK_INPUT,
+// cpp/gsplat/bindings.h:9-16.
+void check_input(const at::Tensor& t, const char* name)
+{
+    if(!t.is_cuda())
+        throw std::runtime_error(std::string(name) + " must be a CUDA tensor");
+    if(!t.is_contiguous())
+        throw std::runtime_error(std::string(name) + " must be contiguous");
 }
 
-} // namespace
-
-// list_bin: tiles per side of the bins that the tile lists are built for (0: the library's choice);
-// the backward of this forward must be given the same value.
-// image[H,W,3], radii[N], splats[N,12], sorted_ids[dsx_sorted_ids_count(K)], ranges[dsx_ranges_count], final_T[H,W], final_idx[H,W]
-// (the 3-D covariances are not kept: the backward rebuilds them from scales and rotations, or
-// reads cov3d_precomp) and, when prepare_backward is set, the backward's gradient accumulator
-// (dsx_grads_bytes(N) bytes as float32), which the blend kernel prepares on the side: sums zeroed,
-// conics in the spare places, the byte per Gaussian behind the records cleared (undefined otherwise)
-std::vector<at::Tensor> forward(int64_t height, int64_t width, double tanfovx, double tanfovy, double scale_modifier,
-                                int64_t sh_degree, int64_t max_sh_degree, const at::Tensor& view,
-                                const at::Tensor& proj, const at::Tensor& campos, const at::Tensor& bg,
-                                int64_t list_bin, const at::Tensor& means3d, const c10::optional<at::Tensor>& scales,
-                                const c10::optional<at::Tensor>& quats, const at::Tensor& opacities,
-                                const c10::optional<at::Tensor>& shs, const c10::optional<at::Tensor>& cov3d_precomp,
-                                const c10::optional<at::Tensor>& colors_precomp, bool prepare_backward,
-                                int64_t stream)
+bool usable(const OptTensor& t)
 {
-    const at::Device dev = means3d.device();
-    c10::DeviceGuard guard(dev);
-    Camera cam = make_camera(height, width, tanfovx, tanfovy, scale_modifier, sh_degree, max_sh_degree, view, proj,
-                             campos, bg, list_bin, dev);
-    const int64_t n = means3d.numel() / 3;
+    return t->is_contiguous() && t->is_cuda();
+}
+
+void check_float(const OptTensor& t, const char* name)
+{
+    if(given(t) && t->scalar_type() != at::kFloat)
+        throw std::runtime_error(std::string(name) + " must be float32");
+}
+
+void validate(const Inputs& in, const Settings& s)
+{
+    check_input(in.means3d, "means_3d");
+    check_input(in.means2d, "means_2d");
+    check_input(in.opacities, "opacities");
+    require(!given(in.shs) || usable(in.shs), "shs error");
+    require(!given(in.scales) || usable(in.scales), "scales error");
+    require(!given(in.quats) || usable(in.quats), "rotations error");
+    require(given(in.cov3d) ? usable(in.cov3d)
+                            : given(in.scales) && given(in.quats) && in.scales->size(0) == in.quats->size(0),
+            "cov3D error");
+    require(given(in.colors) ? usable(in.colors) : given(in.shs), "SHS error");
+    check_float(in.means3d, "means_3d");
+    check_float(in.opacities, "opacities");
+    check_float(in.shs, "shs");
+    check_float(in.scales, "scales");
+    check_float(in.quats, "rotations");
+    check_float(in.cov3d, "cov3D_precomp");
+    check_float(in.colors, "colors_precomp");
+    const int64_t n = in.means3d.numel() / 3;
+    require(in.opacities.numel() == n, "opacities must have one entry per Gaussian");
+    if(given(in.shs))
+    {
+        require(s.sh_degree >= 0 && s.sh_degree <= 3 && s.max_sh_degree == 3,
+                "sh_degree must be in [0, 3] and max_sh_degree must be 3");
+        const int64_t coeff = (s.sh_degree + 1) * (s.sh_degree + 1), most = (s.max_sh_degree + 1) * (s.max_sh_degree + 1);
+        require(in.shs->dim() == 3 && in.shs->size(0) == n && in.shs->size(1) >= coeff && in.shs->size(1) == most &&
+                    in.shs->size(2) == 3,
+                "shs must have shape [N, (max_sh_degree+1)^2, 3]");
+    }
+    require(!given(in.scales) || (in.scales->numel() == 3 * n && given(in.quats) && in.quats->numel() == 4 * n),
+            "scales must be [N,3] and rotations [N,4]");
+    require(!given(in.cov3d) || in.cov3d->numel() == 6 * n, "cov3D_precomp must be [N,6]");
+    require(!given(in.colors) || in.colors->numel() == 3 * n, "colors_precomp must be [N,3]");
+}
+
+// What the forward leaves for the backward.
+struct Rendered
+{
+    at::Tensor image, radii;
+    at::Tensor splats;      // f32 [N,12]
+    at::Tensor sorted_ids;  // i32 [dsx_sorted_ids_count(K)]
+    at::Tensor ranges;      // i32 [dsx_ranges_count]
+    at::Tensor final_T, final_idx;
+    at::Tensor grads;       // the backward's accumulator, prepared by the blend kernel (or undefined)
+    int64_t k = 0;
+};
+
+Rendered render(const Camera& cam, const Inputs& in, bool prepare_backward)
+{
+    const at::Device dev = in.means3d.device();
+    const int64_t n = in.means3d.numel() / 3;
+    const int32_t W = cam.c.image_width, H = cam.c.image_height, bin = cam.c.list_bin;
     const auto f32 = at::TensorOptions().dtype(at::kFloat).device(dev);
     const auto i32 = at::TensorOptions().dtype(at::kInt).device(dev);
     const auto u8 = at::TensorOptions().dtype(at::kByte).device(dev);
-    void* s = reinterpret_cast<void*>(stream);
+    void* s = current_stream(dev);
 
-    at::Tensor splats = at::empty({n, DSX_SPLAT_FLOATS}, f32);
-    at::Tensor radii = at::empty({n}, i32);
-    at::Tensor block_sums = at::empty({std::max<int64_t>(dsx_num_blocks(n), 1)}, i32);
-    const size_t order_bytes = dsx_order_bytes(n, (int32_t)width, (int32_t)height, cam.c.list_bin);
-    at::Tensor order = at::empty({(int64_t)std::max<size_t>(order_bytes, 1)}, u8);
-    at::Tensor& k_host = pinned_key_count();
-    uint32_t* bs = reinterpret_cast<uint32_t*>(block_sums.data_ptr<int32_t>());
-    check(dsx_forward_project(&cam.c, n, means3d.data_ptr<float>(), fptr(scales), fptr(quats),
-                              opacities.data_ptr<float>(), fptr(shs), fptr(cov3d_precomp), fptr(colors_precomp),
-                              splats.data_ptr<float>(), radii.data_ptr<int32_t>(), nullptr, bs, order.data_ptr(),
-                              order_bytes, k_host.data_ptr<int64_t>(), s));
-    const int64_t k = *k_host.data_ptr<int64_t>();
-    at::Tensor sorted_ids = at::empty({dsx_sorted_ids_count(k, (int32_t)width, (int32_t)height, cam.c.list_bin)}, i32);
-    at::Tensor ranges = at::empty({dsx_ranges_count((int32_t)width, (int32_t)height, cam.c.list_bin)}, i32);
-    at::Tensor image = at::empty({height, width, 3}, f32);
-    at::Tensor final_T = at::empty({height, width}, f32);
-    at::Tensor final_idx = at::empty({height, width}, i32);
-    const size_t ws_bytes = dsx_workspace_bytes(n, k, (int32_t)width, (int32_t)height, cam.c.list_bin);
+    Rendered r;
+    r.splats = at::empty({n, DSX_SPLAT_FLOATS}, f32);
+    r.radii = at::empty({n}, i32);
+    // scratch of the first half: the projection's block sums and, behind them, the depth order
+    const size_t sums_bytes = ((size_t)std::max<int64_t>(dsx_num_blocks(n), 1) * 4 + 255) & ~(size_t)255;
+    const size_t order_bytes = dsx_order_bytes(n, W, H, bin);
+    at::Tensor scratch = at::empty({(int64_t)(sums_bytes + order_bytes)}, u8);
+    uint32_t* bs = reinterpret_cast<uint32_t*>(scratch.data_ptr());
+    void* order = static_cast<char*>(scratch.data_ptr()) + sums_bytes;
+    check(dsx_forward_project_begin(&cam.c, n, in.means3d.data_ptr<float>(), fptr(in.scales), fptr(in.quats),
+                                    in.opacities.data_ptr<float>(), fptr(in.shs), fptr(in.cov3d), fptr(in.colors),
+                                    r.splats.data_ptr<float>(), r.radii.data_ptr<int32_t>(), nullptr, bs, order,
+                                    order_bytes, s));
+    // (while the device counts the pairs: everything whose size does not depend on their number)
+    r.ranges = at::empty({dsx_ranges_count(W, H, bin)}, i32);
+    r.image = cam.c.planar ? at::empty({3, H, W}, f32) : at::empty({H, W, 3}, f32);
+    r.final_T = at::empty({H, W}, f32);
+    r.final_idx = at::empty({H, W}, i32);
+    if(prepare_backward && n > 0)
+        r.grads = at::empty({(int64_t)(dsx_grads_bytes(n) / 4)}, f32);
+    int64_t counts[2];
+    check(dsx_forward_project_counts(&cam.c, n, counts, s));
+    r.k = counts[0];
+    r.sorted_ids = at::empty({dsx_sorted_ids_count(r.k, W, H, bin)}, i32);
+    const size_t ws_bytes = dsx_workspace_bytes(n, r.k, W, H, bin);
     at::Tensor ws = at::empty({(int64_t)std::max<size_t>(ws_bytes, 1)}, u8);
-    at::Tensor grads = prepare_backward && n > 0 ? at::empty({(int64_t)(dsx_grads_bytes(n) / 4)}, f32) : at::Tensor();
-    check(dsx_forward_finish(&cam.c, n, k, splats.data_ptr<float>(), order.data_ptr(), sorted_ids.data_ptr<int32_t>(),
-                             ranges.data_ptr<int32_t>(), image.data_ptr<float>(), final_T.data_ptr<float>(),
-                             final_idx.data_ptr<int32_t>(), ws.data_ptr(), ws_bytes,
-                             grads.defined() ? grads.data_ptr<float>() : nullptr, s));
-    return {image, radii, splats, sorted_ids, ranges, final_T, final_idx, grads};
+    check(dsx_forward_finish(&cam.c, n, r.k, r.splats.data_ptr<float>(), order, r.sorted_ids.data_ptr<int32_t>(),
+                             r.ranges.data_ptr<int32_t>(), r.image.data_ptr<float>(), r.final_T.data_ptr<float>(),
+                             r.final_idx.data_ptr<int32_t>(), ws.data_ptr(), ws_bytes,
+                             r.grads.defined() ? r.grads.data_ptr<float>() : nullptr, s));
+    return r;
 }
 
 // v_mean3d[N,3], v_means2d[N,3], v_shs[N,B,3] (undefined when num_bases == 0), v_colors[N,3],
 // v_opacity[N,1], v_scale[N,3], v_quat[N,4], v_cov3d[N,6].  Bit i of `wanted` asks for the i-th
-// of them; the others are neither allocated nor written and come back undefined (None).
-std::vector<at::Tensor> backward(int64_t height, int64_t width, double tanfovx, double tanfovy, double scale_modifier,
-                                 int64_t sh_degree, int64_t max_sh_degree, const at::Tensor& view,
-                                 const at::Tensor& proj, const at::Tensor& campos, const at::Tensor& bg,
-                                 int64_t list_bin, int64_t num_bases, const at::Tensor& means3d, const c10::optional<at::Tensor>& scales,
-                                 const c10::optional<at::Tensor>& quats, const at::Tensor& splats,
-                                 const c10::optional<at::Tensor>& cov3d_precomp, const at::Tensor& radii,
-                                 const at::Tensor& ranges,
-                                 const at::Tensor& sorted_ids, const at::Tensor& final_T, const at::Tensor& final_idx,
-                                 const at::Tensor& v_image, const c10::optional<at::Tensor>& prepared_grads,
-                                 int64_t wanted, int64_t stream)
+// of them; the others are neither allocated nor written and come back undefined.
+std::vector<at::Tensor> differentiate(const Camera& cam, int64_t k, int64_t num_bases, const at::Tensor& means3d,
+                                      const OptTensor& scales, const OptTensor& quats, const OptTensor& cov3d,
+                                      const at::Tensor& splats, const at::Tensor& radii, const at::Tensor& ranges,
+                                      const at::Tensor& sorted_ids, const at::Tensor& final_T,
+                                      const at::Tensor& final_idx, const at::Tensor& v_image, at::Tensor prepared,
+                                      int64_t wanted)
 {
     const at::Device dev = means3d.device();
-    c10::DeviceGuard guard(dev);
-    Camera cam = make_camera(height, width, tanfovx, tanfovy, scale_modifier, sh_degree, max_sh_degree, view, proj,
-                             campos, bg, list_bin, dev);
     const int64_t n = means3d.numel() / 3;
     const auto f32 = at::TensorOptions().dtype(at::kFloat).device(dev);
-    TORCH_CHECK(v_image.is_contiguous() && v_image.scalar_type() == at::kFloat && v_image.numel() == height * width * 3,
-                "v_image must be a contiguous float32 [H, W, 3] tensor");
-    // The lists that `ranges` and `sorted_ids` describe are per tile or per bin of tiles, as the forward was
-    // told (list_bin); the library compares the buffer's header word with this call's bin size on the device.
-    TORCH_CHECK(ranges.is_contiguous() && ranges.scalar_type() == at::kInt &&
-                    ranges.numel() == dsx_ranges_count((int32_t)width, (int32_t)height, cam.c.list_bin),
-                "ranges does not have the layout of this image size and bin size (the backward must be given the "
-                "list_bin of its forward)");
-    TORCH_CHECK(sorted_ids.is_contiguous() && sorted_ids.scalar_type() == at::kInt, "sorted_ids must be int32");
-    // pairs in sorted_ids: the buffer holds k ids and, for lists per bin, k more words
-    const int64_t words_per_pair = dsx_sorted_ids_count(1, (int32_t)width, (int32_t)height, cam.c.list_bin);
-    TORCH_CHECK(words_per_pair > 0 && sorted_ids.numel() % words_per_pair == 0, "sorted_ids has the wrong size");
-    const int64_t k = sorted_ids.numel() / words_per_pair;
+    require(v_image.is_contiguous() && v_image.scalar_type() == at::kFloat &&
+                v_image.numel() == (int64_t)cam.c.image_height * cam.c.image_width * 3 && v_image.device() == dev,
+            "v_image must be a float32 tensor of the image's shape, on its device");
     auto out = [&](int bit, std::initializer_list<int64_t> shape) {
         return (wanted >> bit) & 1 ? at::empty(shape, f32) : at::Tensor();
     };
@@ -170,26 +252,136 @@ std::vector<at::Tensor> backward(int64_t height, int64_t width, double tanfovx, 
     at::Tensor v_scale = out(5, {n, 3}), v_quat = out(6, {n, 4}), v_cov3d = out(7, {n, 6});
     // the accumulator that the forward prepared (sums zeroed, conics in place; good for one
     // backward), or a new one that the call fills
-    const bool prepared = prepared_grads.has_value() && prepared_grads->defined();
-    if(prepared)
-        TORCH_CHECK(prepared_grads->is_contiguous() && prepared_grads->scalar_type() == at::kFloat &&
-                        prepared_grads->numel() == (int64_t)(dsx_grads_bytes(n) / 4) && prepared_grads->device() == dev,
-                    "prepared_grads must be the float32 accumulator of this forward (dsx_grads_bytes(N) bytes)");
-    at::Tensor grads = prepared ? *prepared_grads : at::empty({(int64_t)(dsx_grads_bytes(n) / 4)}, f32);
-    check(dsx_backward(&cam.c, n, k, (int32_t)num_bases, means3d.data_ptr<float>(), fptr(scales),
-                       fptr(quats),
-                       splats.data_ptr<float>(), fptr(cov3d_precomp), radii.data_ptr<int32_t>(),
-                       ranges.data_ptr<int32_t>(), sorted_ids.numel() ? sorted_ids.data_ptr<int32_t>() : nullptr,
-                       final_T.data_ptr<float>(), final_idx.data_ptr<int32_t>(), v_image.data_ptr<float>(),
-                       grads.data_ptr<float>(), prepared ? 1 : 0, ptr(v_mean3d), ptr(v_means2d), ptr(v_shs), ptr(v_colors),
-                       ptr(v_opacity), ptr(v_scale), ptr(v_quat), ptr(v_cov3d), reinterpret_cast<void*>(stream)));
+    const bool is_prepared = prepared.defined();
+    at::Tensor grads = is_prepared ? prepared : at::empty({(int64_t)(dsx_grads_bytes(n) / 4)}, f32);
+    check(dsx_backward(&cam.c, n, k, (int32_t)num_bases, means3d.data_ptr<float>(), fptr(scales), fptr(quats),
+                       splats.data_ptr<float>(), fptr(cov3d), radii.data_ptr<int32_t>(), ranges.data_ptr<int32_t>(),
+                       sorted_ids.numel() ? sorted_ids.data_ptr<int32_t>() : nullptr, final_T.data_ptr<float>(),
+                       final_idx.data_ptr<int32_t>(), v_image.data_ptr<float>(), grads.data_ptr<float>(),
+                       is_prepared ? 1 : 0, ptr(v_mean3d), ptr(v_means2d), ptr(v_shs), ptr(v_colors), ptr(v_opacity),
+                       ptr(v_scale), ptr(v_quat), ptr(v_cov3d), current_stream(dev)));
     return {v_mean3d, v_means2d, v_shs, v_colors, v_opacity, v_scale, v_quat, v_cov3d};
 }
+
+// What the autograd node keeps besides its saved tensors.
+struct NodeState : torch::CustomClassHolder
+{
+    Settings settings;
+    Camera camera;
+    at::Tensor prepared; // the accumulator, until a backward has used it
+    int64_t k = 0, num_bases = 0;
+    std::vector<int64_t> opacity_shape;
+    int edge[8]; // which of the node's inputs the i-th of the eight tensors is (-1: not given)
+};
+
+// The reference maps shs.size(-2) in {1,4,9,16} to a degree (anything else to 3), cpp/rasterizer_torch.cu:224-239,
+// and gsplat/sh.cuh:18-29 maps the degree back to the number of bases.
+int64_t bases_of(const OptTensor& shs)
+{
+    if(!given(shs))
+        return 0;
+    const int64_t b = shs->size(-2);
+    return b == 1 || b == 4 || b == 9 || b == 16 ? b : 16;
+}
+
+class Rasterize : public torch::autograd::Function<Rasterize>
+{
+public:
+    static torch::autograd::variable_list forward(torch::autograd::AutogradContext* ctx, const at::Tensor& means3d,
+                                                  const at::Tensor& means2d, const OptTensor& shs,
+                                                  const OptTensor& colors, const at::Tensor& opacities,
+                                                  const OptTensor& scales, const OptTensor& quats,
+                                                  const OptTensor& cov3d, const Settings& settings)
+    {
+        const Inputs in{means3d, means2d, shs, colors, opacities, scales, quats, cov3d};
+        c10::DeviceGuard guard(means3d.device());
+        auto state = c10::make_intrusive<NodeState>();
+        state->camera = make_camera(settings, means3d.device());
+        Rendered r = render(state->camera, in, true);
+        state->settings = settings;
+        state->prepared = r.grads;
+        state->k = r.k;
+        state->num_bases = bases_of(shs);
+        state->opacity_shape = opacities.sizes().vec();
+        const bool present[8] = {true, true, shs.has_value() && shs->defined(), colors.has_value() && colors->defined(), true,
+                                 scales.has_value() && scales->defined(), quats.has_value() && quats->defined(),
+                                 cov3d.has_value() && cov3d->defined()};
+        for(int i = 0, e = 0; i < 8; ++i)
+            state->edge[i] = present[i] ? e++ : -1;
+        // the reference also keeps the 3-D covariances (cpp/rasterizer_torch.cu:207); the backward here
+        // rebuilds them from scales and rotations, or reads the ones that were passed in
+        ctx->save_for_backward({means3d, scales.value_or(at::Tensor()), quats.value_or(at::Tensor()),
+                                cov3d.value_or(at::Tensor()), r.splats, r.radii, r.ranges, r.sorted_ids, r.final_T,
+                                r.final_idx});
+        ctx->saved_data["state"] = c10::IValue::make_capsule(state);
+        ctx->mark_non_differentiable({r.radii});
+        // no zero tensors for outputs that take no gradient (autograd would fill an int32[N] of zeros
+        // for radii before every backward: a kernel launch in the middle of the step)
+        ctx->set_materialize_grads(false);
+        return {r.image, r.radii};
+    }
+
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                   torch::autograd::variable_list grad_outputs)
+    {
+        torch::autograd::variable_list out(9);
+        if(!grad_outputs[0].defined()) // nothing flows into the image (gradients are not materialised)
+            return out;
+        auto holder = ctx->saved_data["state"].toCapsule();
+        NodeState& state = *static_cast<NodeState*>(holder.get());
+        const auto saved = ctx->get_saved_variables();
+        c10::DeviceGuard guard(saved[0].device());
+        // the reference computes all eight gradients and autograd drops those of inputs that take
+        // none (cpp/rasterizer_torch.cu:315, ds_splat/rasterizer.py:112); here the kernel is told
+        // which ones are wanted and writes no others
+        int64_t wanted = 0;
+        for(int i = 0; i < 8; ++i)
+            if(state.edge[i] >= 0 && ctx->needs_input_grad((size_t)state.edge[i]))
+                wanted |= 1ll << i;
+        at::Tensor prepared;
+        std::swap(prepared, state.prepared); // good for one backward: it leaves sums behind
+        std::vector<at::Tensor> g =
+            differentiate(state.camera, state.k, state.num_bases, saved[0], saved[1], saved[2], saved[3], saved[4],
+                          saved[5], saved[6], saved[7], saved[8], saved[9], grad_outputs[0].contiguous(), prepared, wanted);
+        if(g[4].defined() && g[4].sizes() != at::IntArrayRef(state.opacity_shape))
+            g[4] = g[4].reshape(state.opacity_shape);
+        std::copy(g.begin(), g.end(), out.begin());
+        return out;
+    }
+};
+
+// (image, radii).  Optional tensors may be None or empty.
+std::tuple<at::Tensor, at::Tensor> forward(const at::Tensor& means3d, const at::Tensor& means2d, const OptTensor& shs,
+                                           const OptTensor& colors, const at::Tensor& opacities, const OptTensor& scales,
+                                           const OptTensor& quats, const OptTensor& cov3d, int64_t height, int64_t width,
+                                           double tanfovx, double tanfovy, double scale_modifier, int64_t sh_degree,
+                                           int64_t max_sh_degree, const at::Tensor& view, const at::Tensor& proj,
+                                           const at::Tensor& campos, const at::Tensor& bg, int64_t list_bin, bool planar)
+{
+    const Settings settings{height, width, tanfovx, tanfovy, scale_modifier, sh_degree, max_sh_degree, view, proj,
+                            campos, bg, list_bin, planar};
+    const Inputs in{means3d, means2d, shs, colors, opacities, scales, quats, cov3d};
+    validate(in, settings);
+    auto learns = [](const OptTensor& t) { return t.has_value() && t->defined() && t->requires_grad(); };
+    if(!at::GradMode::is_enabled() ||
+       !(learns(means3d) || learns(means2d) || learns(shs) || learns(colors) || learns(opacities) || learns(scales) ||
+         learns(quats) || learns(cov3d)))
+    {
+        c10::DeviceGuard guard(means3d.device());
+        Rendered r = render(make_camera(settings, means3d.device()), in, false);
+        return {r.image, r.radii};
+    }
+    auto out = Rasterize::apply(means3d, means2d, shs, colors, opacities, scales, quats, cov3d, settings);
+    return {out[0], out[1]};
+}
+
+} // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
 {
     m.doc() = "torch binding of libdsx (gfx950 3D-Gaussian-Splatting rasterizer)";
-    m.def("forward", &forward, "projection, tile lists and blend; returns the tensors the backward needs");
-    m.def("backward", &backward, "blend backward and per-Gaussian backward");
+    m.def("forward", &forward, "projection, tile lists and blend; differentiable", py::call_guard<py::gil_scoped_release>());
+    m.def("backward", [](const at::Tensor& image, const at::Tensor& v_image) { image.backward(v_image); },
+          "the backward of an image that forward returned", py::call_guard<py::gil_scoped_release>());
     m.def("version", []() { return dsx_version(); });
 }

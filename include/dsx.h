@@ -16,7 +16,8 @@
  * different streams of one device share it and their forked parts serialise there; (3) the
  * blend-kernel form override of dsx_set_blend_pixels_per_lane, a diagnostic that changes no result
  * of the forward and only the order of the backward's sums; (4) the device address of the
- * built-in scratch of dsx_backward_static, looked up once per device.
+ * built-in scratch of dsx_backward_static, looked up once per device; (5) per host thread, two words of
+ * pinned host memory that the pair counts arrive in, given back when the thread ends.
  *
  * What each entry point replaces in the reference (deepsense-ai/ds-splat) is cited as
  * file:line next to it.  Matrices are row-major, math convention (translation in elements
@@ -70,6 +71,10 @@ typedef struct dsx_camera
     const float* campos;    /* device float[3]                                      */
     const float* bg;        /* device float[3]                                      */
     int32_t list_bin;       /* tiles per side of a list's bin: 0 (automatic), 1, 2, 4, 8 */
+    int32_t view_transposed; /* 1: `view` is stored column by column (what the Python API's users hold) */
+    int32_t proj_transposed; /* 1: the same for `proj`                                     */
+    int32_t planar;         /* 0: image and v_image are [H,W,3], the background is not composited;
+                               1: they are [3,H,W] and the image has final_T * bg added    */
 } dsx_camera;
 
 /*
@@ -89,7 +94,8 @@ typedef struct dsx_camera
  */
 
 const char* dsx_error_string(int status);
-/* 100 * major + minor.  300: the bin size of the tile lists is an argument (dsx_camera::list_bin and
+/* 100 * major + minor.  310: dsx_camera has view_transposed, proj_transposed and planar (0: as before), the
+ * projection's wait for the pair counts is a function of its own.  300: the bin size of the tile lists is an argument (dsx_camera::list_bin and
  * the size helpers) instead of a process-wide setting; the `ranges` buffer carries it in a header word;
  * the blend entry points and the backward are told n and k and follow no id or list position beyond
  * them; dsx_forward_project returns both pair counts.  (200 had dsx_set_list_bin.) */
@@ -285,6 +291,14 @@ int dsx_forward_project(const dsx_camera* cam, int64_t n, const float* means3d,
                         float* splats, int32_t* radii, float* cov3d, uint32_t* block_sums,
                         void* order, size_t order_bytes, int64_t* num_keys /* host */,
                         void* stream);
+/* The same in two halves, for a caller that has something to do (allocations) while the device counts: everything up
+ * to the wait, and the wait for the pair counts of the calling thread's last dsx_forward_project_begin. */
+int dsx_forward_project_begin(const dsx_camera* cam, int64_t n, const float* means3d,
+                        const float* scales, const float* quats, const float* opacities,
+                        const float* shs, const float* cov3d_precomp, const float* colors_precomp,
+                        float* splats, int32_t* radii, float* cov3d, uint32_t* block_sums,
+                        void* order, size_t order_bytes, void* stream);
+int dsx_forward_project_counts(const dsx_camera* cam, int64_t n, int64_t* num_keys /* host */, void* stream);
 
 /* Second half: tile lists (dsx_tile_lists) and blend.  sorted_ids[k] and ranges[T+1] are
  * outputs that backward needs; workspace as dsx_workspace_bytes(n, k, W, H).  If one of the two
