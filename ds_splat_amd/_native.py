@@ -34,6 +34,7 @@ class Camera(C.Structure):
         ("view_transposed", C.c_int32),
         ("proj_transposed", C.c_int32),
         ("planar", C.c_int32),
+        ("view_copy", C.c_void_p),
     ]
 
 

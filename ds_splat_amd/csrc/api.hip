@@ -696,6 +696,7 @@ extern "C" int dsx_forward_core(const float* means3d, const float* shs, const fl
     cam.bg = campos; // unused by the forward
     cam.list_bin = 0;
     cam.view_transposed = cam.proj_transposed = cam.planar = 0;
+    cam.view_copy = nullptr;
     if(int rc = check_camera(&cam))
         return rc;
     if(n < 0 || !image)

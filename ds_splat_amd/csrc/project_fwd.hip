@@ -50,6 +50,7 @@ struct ProjectParams
     int sh_degree, sh_stride; // active degree; floats per shs row
     int ntx, nty;
     int view_transposed, proj_transposed; // stored column by column
+    float* view_copy;                     // (optional) receives the view matrix, row by row
 };
 
 // SH degree 0..3 -> RGB (+0.5, clamped at 0), term order as cpp/rasterizer_kernels.cu:433-554,
@@ -193,6 +194,8 @@ __global__ __launch_bounds__(kProjBlock) void project_fwd_kernel(const ProjectPa
     // instead of by a launch of their own
     for(int64_t j = i; j < p.clear_words; j += (int64_t)gridDim.x * kProjBlock)
         p.clear[j] = 0u;
+    if(p.view_copy && i < 16)
+        p.view_copy[i] = p.view[p.view_transposed ? 4 * (i % 4) + i / 4 : i];
 
     // frustum test on the centre: strict NDC box, z_ndc > 0.1 (cpp/rasterizer_kernels.cu:7-24).
     // It comes first because a Gaussian that fails it is culled whatever its shape is, nothing
@@ -424,6 +427,7 @@ int launch_project_fwd(const dsx_camera& cam, int64_t n, const float* means3d, c
     p.proj = cam.proj;
     p.view_transposed = cam.view_transposed;
     p.proj_transposed = cam.proj_transposed;
+    p.view_copy = cam.view_copy;
     p.campos = cam.campos;
     p.splats = reinterpret_cast<float4*>(splats);
     p.radii = radii;

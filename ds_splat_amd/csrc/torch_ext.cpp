@@ -6,6 +6,7 @@
 // the same steps in Python took the host as long.
 #include <torch/extension.h>
 
+#include <ATen/FuncTorchTLS.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
@@ -72,19 +73,34 @@ at::Tensor matrix_of(const at::Tensor& t, const at::Device& dev, int32_t& transp
 {
     at::Tensor m = t.to(dev, at::kFloat);
     require(m.numel() == 16, "camera tensors must be 4x4, 4x4, [3], [3]");
-    const bool by_columns = m.dim() == 2 && m.stride(0) == 1 && m.stride(1) == 4;
-    transposed = by_columns ? 0 : 1;
-    return by_columns ? m : m.contiguous();
+    const bool square = m.dim() == 2 && m.size(0) == 4;
+    if(square && m.is_contiguous())
+    {
+        transposed = 1;
+        return m;
+    }
+    transposed = 0;
+    if(square && m.stride(0) == 1 && m.stride(1) == 4)
+        return m;
+    return m.t().contiguous(); // (any other shape: what the reference's transposition makes of it, or its error)
 }
 
-Camera make_camera(const Settings& s, const at::Device& dev)
+// kept_view: the forward's copy of the view matrix, for the backward (which does not look at the projection
+// matrix); null: both matrices as the settings hold them
+Camera make_camera(const Settings& s, const at::Device& dev, const float* kept_view = nullptr)
 {
     Camera cam;
-    cam.view = matrix_of(s.view, dev, cam.c.view_transposed);
-    cam.proj = matrix_of(s.proj, dev, cam.c.proj_transposed);
+    if(kept_view == nullptr)
+    {
+        cam.view = matrix_of(s.view, dev, cam.c.view_transposed);
+        cam.proj = matrix_of(s.proj, dev, cam.c.proj_transposed);
+    }
+    else
+        cam.c.view_transposed = cam.c.proj_transposed = 0;
     cam.campos = s.campos.to(dev, at::kFloat).contiguous();
     cam.bg = s.bg.to(dev, at::kFloat).contiguous();
-    require(cam.campos.numel() >= 3 && cam.bg.numel() >= 3, "camera tensors must be 4x4, 4x4, [3], [3]");
+    require(cam.campos.numel() >= 3 && cam.bg.numel() >= 3 && !(s.planar && cam.bg.numel() != 3),
+            "camera tensors must be 4x4, 4x4, [3], [3]");
     cam.c.image_height = (int32_t)s.height;
     cam.c.image_width = (int32_t)s.width;
     cam.c.tanfovx = (float)s.tanfovx;
@@ -92,8 +108,9 @@ Camera make_camera(const Settings& s, const at::Device& dev)
     cam.c.scale_modifier = (float)s.scale_modifier;
     cam.c.sh_degree = (int32_t)s.sh_degree;
     cam.c.max_sh_degree = (int32_t)s.max_sh_degree;
-    cam.c.view = cam.view.data_ptr<float>();
-    cam.c.proj = cam.proj.data_ptr<float>();
+    cam.c.view = kept_view ? kept_view : cam.view.data_ptr<float>();
+    cam.c.proj = kept_view ? kept_view : cam.proj.data_ptr<float>();
+    cam.c.view_copy = nullptr;
     cam.c.campos = cam.campos.data_ptr<float>();
     cam.c.bg = cam.bg.data_ptr<float>();
     require(s.list_bin == 0 || s.list_bin == 1 || s.list_bin == 2 || s.list_bin == 4 || s.list_bin == 8,
@@ -169,11 +186,15 @@ void validate(const Inputs& in, const Settings& s)
     require(!given(in.colors) || in.colors->numel() == 3 * n, "colors_precomp must be [N,3]");
 }
 
+// The user's matrices may be written over between a forward and its backward (one camera buffer for many views):
+// the projection kernel keeps a copy of the one that the backward needs behind its records.
+constexpr int64_t kViewRecords = (16 + DSX_SPLAT_FLOATS - 1) / DSX_SPLAT_FLOATS;
+
 // What the forward leaves for the backward.
 struct Rendered
 {
     at::Tensor image, radii;
-    at::Tensor splats;      // f32 [N,12]
+    at::Tensor splats;      // f32 [N + kViewRecords,12]: the records, then the view matrix that they were made with
     at::Tensor sorted_ids;  // i32 [dsx_sorted_ids_count(K)]
     at::Tensor ranges;      // i32 [dsx_ranges_count]
     at::Tensor final_T, final_idx;
@@ -181,7 +202,7 @@ struct Rendered
     int64_t k = 0;
 };
 
-Rendered render(const Camera& cam, const Inputs& in, bool prepare_backward)
+Rendered render(Camera cam, const Inputs& in, bool prepare_backward)
 {
     const at::Device dev = in.means3d.device();
     const int64_t n = in.means3d.numel() / 3;
@@ -192,7 +213,8 @@ Rendered render(const Camera& cam, const Inputs& in, bool prepare_backward)
     void* s = current_stream(dev);
 
     Rendered r;
-    r.splats = at::empty({n, DSX_SPLAT_FLOATS}, f32);
+    r.splats = at::empty({n + kViewRecords, DSX_SPLAT_FLOATS}, f32);
+    cam.c.view_copy = prepare_backward ? r.splats.data_ptr<float>() + n * DSX_SPLAT_FLOATS : nullptr;
     r.radii = at::empty({n}, i32);
     // scratch of the first half: the projection's block sums and, behind them, the depth order
     const size_t sums_bytes = ((size_t)std::max<int64_t>(dsx_num_blocks(n), 1) * 4 + 255) & ~(size_t)255;
@@ -266,8 +288,7 @@ std::vector<at::Tensor> differentiate(const Camera& cam, int64_t k, int64_t num_
 // What the autograd node keeps besides its saved tensors.
 struct NodeState : torch::CustomClassHolder
 {
-    Settings settings;
-    Camera camera;
+    Settings settings;   // (no address is kept: the tensors' memory may be another one by then)
     at::Tensor prepared; // the accumulator, until a backward has used it
     int64_t k = 0, num_bases = 0;
     std::vector<int64_t> opacity_shape;
@@ -296,9 +317,9 @@ public:
         const Inputs in{means3d, means2d, shs, colors, opacities, scales, quats, cov3d};
         c10::DeviceGuard guard(means3d.device());
         auto state = c10::make_intrusive<NodeState>();
-        state->camera = make_camera(settings, means3d.device());
-        Rendered r = render(state->camera, in, true);
+        Rendered r = render(make_camera(settings, means3d.device()), in, true);
         state->settings = settings;
+        state->settings.view = state->settings.proj = at::Tensor(); // (the records hold the copy)
         state->prepared = r.grads;
         state->k = r.k;
         state->num_bases = bases_of(shs);
@@ -340,8 +361,10 @@ public:
                 wanted |= 1ll << i;
         at::Tensor prepared;
         std::swap(prepared, state.prepared); // good for one backward: it leaves sums behind
+        const Camera camera = make_camera(state.settings, saved[0].device(),
+                                          saved[4].data_ptr<float>() + saved[0].numel() / 3 * DSX_SPLAT_FLOATS);
         std::vector<at::Tensor> g =
-            differentiate(state.camera, state.k, state.num_bases, saved[0], saved[1], saved[2], saved[3], saved[4],
+            differentiate(camera, state.k, state.num_bases, saved[0], saved[1], saved[2], saved[3], saved[4],
                           saved[5], saved[6], saved[7], saved[8], saved[9], grad_outputs[0].contiguous(), prepared, wanted);
         if(g[4].defined() && g[4].sizes() != at::IntArrayRef(state.opacity_shape))
             g[4] = g[4].reshape(state.opacity_shape);
@@ -362,10 +385,16 @@ std::tuple<at::Tensor, at::Tensor> forward(const at::Tensor& means3d, const at::
                             campos, bg, list_bin, planar};
     const Inputs in{means3d, means2d, shs, colors, opacities, scales, quats, cov3d};
     validate(in, settings);
-    auto learns = [](const OptTensor& t) { return t.has_value() && t->defined() && t->requires_grad(); };
-    if(!at::GradMode::is_enabled() ||
-       !(learns(means3d) || learns(means2d) || learns(shs) || learns(colors) || learns(opacities) || learns(scales) ||
-         learns(quats) || learns(cov3d)))
+    // Without a gradient to take the node is passed by; transforms of functions and tangents of forward-mode
+    // differentiation are not: torch refuses them at the node.
+    if(const auto& transforms = at::functorch::functorchTLSAccessor())
+        transforms->checkSupportsCppAutogradFunction();
+    const bool grad_mode = at::GradMode::is_enabled();
+    auto needs_node = [grad_mode](const OptTensor& t) {
+        return t.has_value() && t->defined() && ((grad_mode && t->requires_grad()) || t->_fw_grad(0).defined());
+    };
+    if(!(needs_node(means3d) || needs_node(means2d) || needs_node(shs) || needs_node(colors) || needs_node(opacities) ||
+         needs_node(scales) || needs_node(quats) || needs_node(cov3d)))
     {
         c10::DeviceGuard guard(means3d.device());
         Rendered r = render(make_camera(settings, means3d.device()), in, false);
@@ -380,8 +409,12 @@ std::tuple<at::Tensor, at::Tensor> forward(const at::Tensor& means3d, const at::
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
 {
     m.doc() = "torch binding of libdsx (gfx950 3D-Gaussian-Splatting rasterizer)";
-    m.def("forward", &forward, "projection, tile lists and blend; differentiable", py::call_guard<py::gil_scoped_release>());
-    m.def("backward", [](const at::Tensor& image, const at::Tensor& v_image) { image.backward(v_image); },
-          "the backward of an image that forward returned", py::call_guard<py::gil_scoped_release>());
+    // (torch's own wrappers: errors come back as torch's exceptions, and a Python exception that a hook on saved
+    // tensors raises, as recomputation under checkpointing does, passes through as it is)
+    m.def("forward", torch::wrap_pybind_function_no_gil(forward), "projection, tile lists and blend; differentiable");
+    m.def("backward", torch::wrap_pybind_function_no_gil([](const at::Tensor& image, const at::Tensor& v_image) {
+              image.backward(v_image);
+          }),
+          "the backward of an image that forward returned");
     m.def("version", []() { return dsx_version(); });
 }

@@ -32,6 +32,8 @@ def _render(means_3d, means_2d, shs, colors_precomp, opacities, scales, rotation
             projmatrix, max_sh_degree, planar):
     """``s``: any object with the scalar settings, ``campos`` and ``bg``; the matrices as the API's users hold them
     (transposed).  planar: the image is channel-first and has the background composited."""
+    if torch.jit.is_tracing():  # (nothing but the allocations would be recorded)
+        raise RuntimeError("the rasterizer cannot be recorded by torch.jit.trace")
     return _native.load_torch_ext().forward(
         means_3d, means_2d, shs, colors_precomp, opacities, scales, rotations, cov_3d_precomp, int(s.image_height),
         int(s.image_width), float(s.tanfovx), float(s.tanfovy), float(s.scale_modifier), int(s.sh_degree),

@@ -75,6 +75,8 @@ typedef struct dsx_camera
     int32_t proj_transposed; /* 1: the same for `proj`                                     */
     int32_t planar;         /* 0: image and v_image are [H,W,3], the background is not composited;
                                1: they are [3,H,W] and the image has final_T * bg added    */
+    float* view_copy;       /* device float[16], or null: dsx_forward_project stores `view` there, row by row,
+                               for a backward that runs when the caller's own matrix may be another one    */
 } dsx_camera;
 
 /*
@@ -94,7 +96,7 @@ typedef struct dsx_camera
  */
 
 const char* dsx_error_string(int status);
-/* 100 * major + minor.  310: dsx_camera has view_transposed, proj_transposed and planar (0: as before), the
+/* 100 * major + minor.  310: dsx_camera has view_transposed, proj_transposed, planar and view_copy (0: as before), the
  * projection's wait for the pair counts is a function of its own.  300: the bin size of the tile lists is an argument (dsx_camera::list_bin and
  * the size helpers) instead of a process-wide setting; the `ranges` buffer carries it in a header word;
  * the blend entry points and the backward are told n and k and follow no id or list position beyond

@@ -1,0 +1,133 @@
+"""What torch's autograd machinery and a user's program do around a call: cameras written over, hooks on saved
+tensors, recomputation, tracing, transforms of functions."""
+import pytest
+import torch
+import torch.utils.checkpoint
+
+from ds_splat_amd.synthetic import make_scene
+from helpers import set_camera
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+# image and gradients of two runs of one scene: the same terms, the gradients' added by float atomics in another order
+RTOL, ATOL = 1e-3, 1e-4
+
+
+def scene(camera="rotated"):
+    sc = set_camera(make_scene("cfg0", n=3000, width=96, height=80, sh_degree=2, seed=7), camera)
+    t = {k: (v.to(DEV) if isinstance(v, torch.Tensor) else v) for k, v in sc.items()}
+    leaves = [t["means_3d"], torch.zeros_like(t["means_3d"]), t["shs"], t["opacities"], t["scales"] * 2.0, t["rotations"]]
+    return sc, t, [x.clone().requires_grad_(True) for x in leaves]
+
+
+def rasterizer(t, view=None, proj=None):
+    from ds_splat import GaussianRasterizationSettings, GaussianRasterizer
+    return GaussianRasterizer(GaussianRasterizationSettings(
+        image_height=t["height"], image_width=t["width"], tanfovx=t["tanfovx"], tanfovy=t["tanfovy"], bg=t["bg"],
+        scale_modifier=1.0, viewmatrix=t["viewmatrix"] if view is None else view,
+        projmatrix=t["projmatrix"] if proj is None else proj, sh_degree=2, max_sh_degree=3, campos=t["campos"],
+        prefiltered=False, debug=False))
+
+
+def call(r, leaves):
+    means, means2d, shs, opac, scales, rots = leaves
+    return r(means, means2d, shs, None, opac, scales, rots, None)[0]
+
+
+def wanted():
+    _, t, leaves = scene()
+    image = call(rasterizer(t), leaves)
+    image.backward(t["v_image"])
+    assert all(float(x.grad.abs().max()) > 0 for x in leaves)
+    return image.detach(), [x.grad for x in leaves]
+
+
+def check_grads(got, want):
+    for g, w in zip(got, want):
+        assert torch.allclose(g, w, rtol=RTOL, atol=ATOL * max(1.0, float(w.abs().max())))
+
+
+def test_the_camera_may_be_written_over_before_the_backward():
+    image_w, grads_w = wanted()
+    _, t, leaves = scene()
+    view, proj = t["viewmatrix"].clone(), t["projmatrix"].clone()
+    image = call(rasterizer(t, view, proj), leaves)
+    view.copy_(torch.eye(4))
+    proj.zero_()
+    image.backward(t["v_image"])
+    assert torch.equal(image, image_w)
+    check_grads([x.grad for x in leaves], grads_w)
+
+
+def test_the_backgrounds_memory_may_be_another_one_at_the_backward():
+    image_w, grads_w = wanted()
+    _, t, leaves = scene()
+    image = call(rasterizer(t), leaves)
+    t["bg"].data, t["campos"].data = t["bg"].clone(), t["campos"].clone()
+    image.backward(t["v_image"])
+    check_grads([x.grad for x in leaves], grads_w)
+
+
+@pytest.mark.parametrize("form", ["by_columns", "flat", "strided", "double"])
+def test_forms_of_the_camera_matrices(form):
+    image_w, grads_w = wanted()
+    _, t, leaves = scene()
+
+    def as_form(m):
+        if form == "by_columns":
+            return m.t().contiguous().t()
+        if form == "flat":      # (transposing a vector leaves it: it holds the row-major matrix itself)
+            return m.t().contiguous().view(16)
+        if form == "strided":
+            return torch.stack([m, m], 2)[:, :, 0]
+        return m.double()
+
+    image = call(rasterizer(t, as_form(t["viewmatrix"]), as_form(t["projmatrix"])), leaves)
+    image.backward(t["v_image"])
+    assert torch.equal(image, image_w)
+    check_grads([x.grad for x in leaves], grads_w)
+    with pytest.raises(RuntimeError):
+        call(rasterizer(t, t["viewmatrix"][None]), leaves)
+
+
+def test_saved_tensors_may_be_kept_on_the_host():
+    image_w, grads_w = wanted()
+    _, t, leaves = scene()
+    with torch.autograd.graph.save_on_cpu():
+        image = call(rasterizer(t), leaves)
+    image.backward(t["v_image"])
+    assert torch.equal(image, image_w)
+    check_grads([x.grad for x in leaves], grads_w)
+
+
+@pytest.mark.parametrize("reentrant", [False, True])
+def test_recomputation_under_checkpointing(reentrant):
+    image_w, grads_w = wanted()
+    _, t, leaves = scene()
+    r = rasterizer(t)
+    image = torch.utils.checkpoint.checkpoint(lambda *xs: call(r, xs), *leaves, use_reentrant=reentrant)
+    image.backward(t["v_image"])
+    assert torch.equal(image, image_w)
+    check_grads([x.grad for x in leaves], grads_w)
+
+
+def test_tracing_is_refused():
+    _, t, leaves = scene()
+    with pytest.raises(RuntimeError):
+        torch.jit.trace(lambda *xs: call(rasterizer(t), xs), tuple(x.detach() for x in leaves), check_trace=False)
+
+
+def test_tangents_and_transforms_are_refused():
+    import torch.autograd.forward_ad as fwd
+    _, t, leaves = scene()
+    plain = [x.detach() for x in leaves]
+    r = rasterizer(t)
+    for grad_mode in (True, False):
+        with torch.set_grad_enabled(grad_mode), fwd.dual_level():
+            dual = [fwd.make_dual(plain[0], torch.ones_like(plain[0]))] + plain[1:]
+            with pytest.raises((RuntimeError, NotImplementedError)):
+                call(r, dual)
+    with pytest.raises(RuntimeError):
+        torch.func.grad(lambda m: call(r, [m] + plain[1:]).sum())(plain[0])
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(lambda m: call(r, [m] + plain[1:]))(plain[0][None])
