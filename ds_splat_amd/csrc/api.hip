@@ -2,6 +2,7 @@
 // synchronisation of the forward (read-back of the key count) and error strings.
 #include "dsx_common.h"
 
+#include <algorithm>
 #include <mutex>
 #include <string.h>
 #include <vector>
@@ -513,36 +514,69 @@ static int check_pair_counts(int64_t list_pairs, int64_t tile_pairs)
     return DSX_OK;
 }
 
-// Two words of pinned host memory per host thread (given back when the thread ends), which the device writes.
+// Pinned host memory of a host thread (given back when the thread ends), which the device writes the pair counts
+// into.  A call that was begun and whose counts nobody waited for (an allocation failed in between) may still write
+// its own when the next one is waiting: every call has a ticket, which the words carry, and the next of several slots.
 namespace
 {
+constexpr unsigned kCountSlots = 16;
 struct PinnedCounts
 {
     int64_t* words = nullptr;
+    unsigned calls = 0;
+    unsigned ticket() const
+    {
+        return calls % 0x7fffeu + 1u; // 19 bits: a marked word is never negative, and never zero
+    }
+    volatile int64_t* slot() const
+    {
+        return words + 2 * (calls % kCountSlots);
+    }
     ~PinnedCounts()
     {
         if(words)
             (void)hipHostFree(words);
     }
 };
-volatile int64_t* pinned_counts()
+thread_local PinnedCounts g_counts;
+
+// where the counts of the calling thread's next call arrive (null words: no memory)
+HostCounts next_counts()
 {
-    thread_local PinnedCounts mine;
-    if(mine.words == nullptr)
+    if(g_counts.words == nullptr)
     {
         void* p = nullptr;
-        if(hipHostMalloc(&p, 2 * sizeof(int64_t), hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
-            return nullptr;
-        mine.words = static_cast<int64_t*>(p);
+        if(hipHostMalloc(&p, 2 * kCountSlots * sizeof(int64_t),
+                         hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
+            return {};
+        g_counts.words = static_cast<int64_t*>(p);
+        std::fill_n(g_counts.words, 2 * kCountSlots, 0);
     }
-    return mine.words;
+    ++g_counts.calls;
+    volatile int64_t* const slot = g_counts.slot();
+    slot[0] = slot[1] = 0;
+    return {reinterpret_cast<unsigned long long*>(const_cast<int64_t*>(slot)), g_counts.ticket()};
 }
-// Waits until both words are there.  Every wait ends: when the stream has run dry (or into an error) without them.
-bool wait_for_counts(volatile int64_t* counts, hipStream_t stream)
+// Waits until both words of the calling thread's last call are there.  Every wait ends: when the stream has run dry
+// (or into an error) without them.
+bool wait_for_counts(hipStream_t stream, int64_t (&counts)[2])
 {
+    if(g_counts.words == nullptr)
+        return false;
+    volatile const int64_t* const slot = g_counts.slot();
+    auto arrived = [&] {
+        counts[0] = slot[0];
+        counts[1] = slot[1];
+        const int64_t ticket = g_counts.ticket();
+        if((counts[0] >> kTicketShift) != ticket || (counts[1] >> kTicketShift) != ticket)
+            return false;
+        for(int64_t& c : counts)
+            c &= (1ll << kTicketShift) - 1;
+        return true;
+    };
     for(int64_t spins = 1;; ++spins)
     {
-        if(counts[0] >= 0 && counts[1] >= 0)
+        if(arrived())
             return true;
         __builtin_ia32_pause();
         if((spins & 0xffff) == 0)
@@ -550,7 +584,7 @@ bool wait_for_counts(volatile int64_t* counts, hipStream_t stream)
             const hipError_t e = hipStreamQuery(stream);
             if(e == hipErrorNotReady)
                 continue;
-            return e == hipSuccess && counts[0] >= 0 && counts[1] >= 0;
+            return e == hipSuccess && arrived();
         }
     }
 }
@@ -571,11 +605,10 @@ extern "C" int dsx_forward_project_begin(const dsx_camera* cam, int64_t n, const
     // The pair counts are sums over the rectangles: the kernel that counts the tiles, first thing beside the
     // depth sort, writes them into pinned host memory, where the calling thread finds them while the
     // depth order is computed (no copy, no event).
-    volatile int64_t* const counts = pinned_counts();
-    if(counts == nullptr)
+    const HostCounts to_host = next_counts();
+    if(to_host.words == nullptr)
         return DSX_ERR_RUNTIME;
-    counts[0] = counts[1] = -1;
-    return launch_depth_order(*cam, n, order, as_stream(stream), true, const_cast<int64_t*>(counts));
+    return launch_depth_order(*cam, n, order, as_stream(stream), true, to_host);
 }
 
 extern "C" int dsx_forward_project_counts(const dsx_camera* cam, int64_t n, int64_t* num_keys, void* stream)
@@ -587,8 +620,8 @@ extern "C" int dsx_forward_project_counts(const dsx_camera* cam, int64_t n, int6
         return rc;
     if(n <= 0)
         return n == 0 ? DSX_OK : DSX_ERR_BAD_ARG;
-    volatile int64_t* const counts = pinned_counts();
-    if(counts == nullptr || !wait_for_counts(counts, as_stream(stream)))
+    int64_t counts[2];
+    if(!wait_for_counts(as_stream(stream), counts))
         return DSX_ERR_RUNTIME;
     // the device wrote (per-tile pairs, bin pairs); the caller gets (pairs of the lists, per-tile pairs)
     const int64_t tile_pairs = counts[0], bin_pairs = counts[1];

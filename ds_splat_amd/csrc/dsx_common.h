@@ -268,6 +268,14 @@ struct ListsWorkspace
 ListsWorkspace lists_workspace(int64_t k, int num_tiles, bool binned);
 
 // launchers (each returns a dsx_status)
+// Two words of pinned host memory that receive a call's pair counts (null: none), each marked with the call's ticket.
+struct HostCounts
+{
+    unsigned long long* words = nullptr;
+    unsigned long long ticket = 0;
+};
+constexpr int kTicketShift = 44; // a count is cut off at 2^43: far beyond what a call accepts
+
 int launch_sort32(int64_t count, int key_bits, uint32_t* keys_a, uint32_t* vals_a, uint32_t* keys_b,
                   uint32_t* vals_b, bool iota_values, bool keep_keys, void* sort_ws, hipStream_t stream,
                   uint32_t** keys_out, uint32_t** vals_out, const uint2* gather_src = nullptr,
@@ -275,7 +283,7 @@ int launch_sort32(int64_t count, int key_bits, uint32_t* keys_a, uint32_t* vals_
                   uint32_t* carry_b = nullptr);
 // already_cleared: the words of depth_order_clear_region are zero already (the projection did it)
 int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_t stream,
-                       bool already_cleared = false, void* k_host = nullptr);
+                       bool already_cleared = false, HostCounts to_host = {});
 // the part of an `order` buffer that must be zero when launch_depth_order starts
 void depth_order_clear_region(const dsx_camera& cam, int64_t n, void* order, uint32_t** words, int64_t* count);
 int launch_tile_lists(const dsx_camera& cam, int64_t n, int64_t k, const void* order, int32_t* sorted_ids,

@@ -772,10 +772,12 @@ __global__ __launch_bounds__(kProjBlock) void ordered_block_sums_kernel(const ui
         block_sums[blockIdx.x] = wave_sums[0] + wave_sums[1] + wave_sums[2] + wave_sums[3];
 }
 
-// a word of pinned host memory that the host polls
-__device__ __forceinline__ void store_to_host(unsigned long long* p, unsigned long long v)
+// one of the words of pinned host memory that the host polls
+__device__ __forceinline__ void store_to_host(const HostCounts& to, int word, unsigned long long count)
 {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    constexpr unsigned long long most = 1ull << (kTicketShift - 1);
+    __hip_atomic_store(to.words + word, (to.ticket << kTicketShift) | (count < most ? count : most), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // How many pairs each tile receives, straight from the rectangles (no pair is enumerated):
@@ -796,7 +798,7 @@ __global__ __launch_bounds__(kCoverThreads) void tile_cover_kernel(const uint2* 
                                                                    int32_t* __restrict__ grid,
                                                                    int32_t* __restrict__ bin_grid,
                                                                    unsigned long long* __restrict__ key_count,
-                                                                   unsigned long long* k_host)
+                                                                   const HostCounts to_host)
 {
     extern __shared__ int32_t s_grid[];
     const int tid = threadIdx.x;
@@ -883,9 +885,9 @@ __global__ __launch_bounds__(kCoverThreads) void tile_cover_kernel(const uint2* 
         // performed when their results are back, so the ticket is drawn after them.
         const unsigned long long before0 = atomicAdd(key_count, total[0]), before1 = atomicAdd(key_count + 1, total[1]);
         asm volatile("s_waitcnt vmcnt(0)" ::"v"(before0), "v"(before1) : "memory");
-        if(k_host && atomicAdd(key_count + 2, 1ull) == gridDim.x - 1)
+        if(to_host.words && atomicAdd(key_count + 2, 1ull) == gridDim.x - 1)
             for(int i = 0; i < 2; ++i)
-                store_to_host(k_host + i, atomicAdd(key_count + i, 0ull));
+                store_to_host(to_host, i, atomicAdd(key_count + i, 0ull));
     }
 }
 
@@ -1094,7 +1096,7 @@ struct SmallOrder
     unsigned long long* done;       // (merge) workgroups that have added their sums
     int n, shift, tiles;
     CountsJobs counts;
-    unsigned long long* k_host;
+    HostCounts to_host;
 };
 
 __device__ __forceinline__ void small_sort(const SmallOrder& J, const int tile, uint32_t* s_mem)
@@ -1389,11 +1391,11 @@ __device__ __forceinline__ void small_counts(const SmallOrder& J, const bool bin
     if((tid & 63) == 0 && pairs)
         atomicAdd(&s_pairs, pairs);
     __syncthreads();
-    if(tid == 0 && J.k_host)
+    if(tid == 0 && J.to_host.words)
     {
-        store_to_host(J.k_host + (bins ? 1 : 0), s_pairs);
+        store_to_host(J.to_host, bins ? 1 : 0, s_pairs);
         if(J.shift == 0)
-            store_to_host(J.k_host + 1, 0ull);
+            store_to_host(J.to_host, 1, 0ull);
     }
     tile_counts(C, s_grid);
 }
@@ -1410,7 +1412,7 @@ __global__ __launch_bounds__(kSmallThreads) void order_small_kernel(const SmallO
 }
 
 // true: done (or failed: *rc).  false: too many Gaussians, or a corner grid that does not fit the LDS
-static bool launch_order_small(const ListGrid& lg, int64_t n, char* base, const OrderLayout& o, void* k_host,
+static bool launch_order_small(const ListGrid& lg, int64_t n, char* base, const OrderLayout& o, const HostCounts& to_host,
                                const CountsJobs& jobs, hipStream_t stream, int* rc)
 {
     const int cells = (lg.ntx + 1) * (lg.nty + 1) + 1;
@@ -1441,7 +1443,7 @@ static bool launch_order_small(const ListGrid& lg, int64_t n, char* base, const 
     J.shift = lg.shift;
     J.tiles = (int)((n + kSmallTile - 1) / kSmallTile);
     J.counts = jobs;
-    J.k_host = static_cast<unsigned long long*>(k_host);
+    J.to_host = to_host;
     {
         DSX_TIMED("order_small_kernel", stream);
         hipLaunchKernelGGL(order_small_kernel, dim3(J.tiles + (lg.shift ? 2 : 1)), dim3(kSmallThreads), bytes, stream, J);
@@ -1500,11 +1502,11 @@ void depth_order_clear_region(const dsx_camera& cam, int64_t n, void* order, uin
     *count = (int64_t)((w.bytes + (o.ranges - o.cover)) / 4);
 }
 
-// k_host (optional): two words of pinned host memory that receive the pair counts (per-tile lists: what the
+// to_host (optional): two words of pinned host memory that receive the pair counts (per-tile lists: what the
 // reference calls K, the fine ranges and final_idx index that many pairs; bin lists, zero when the lists
 // are per tile) as soon as the rectangles have been counted, while the sort still runs.
 int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_t stream, bool already_cleared,
-                       void* k_host)
+                       HostCounts to_host)
 {
     if(n <= 0)
         return DSX_OK;
@@ -1528,7 +1530,7 @@ int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_
         return rc;
 
     const CountsJobs jobs = counts_jobs(list_grid(cam), base, o);
-    if(launch_order_small(list_grid(cam), n, base, o, k_host, jobs, stream, &rc))
+    if(launch_order_small(list_grid(cam), n, base, o, to_host, jobs, stream, &rc))
         return rc;
 
     // pairs per tile: digit histograms of the tile partition and the tile ranges that the second
@@ -1579,7 +1581,7 @@ int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_
                                use_lds ? (size_t)(cells + bcells) * 4 : 0, cs,
                                reinterpret_cast<const uint2*>(base + o.rects), n, ntx, nty, lg.shift, lg.nbx, lg.nby,
                                use_lds, grid, bin_grid, reinterpret_cast<unsigned long long*>(base + o.key_count),
-                               static_cast<unsigned long long*>(k_host));
+                               to_host);
         }
         {
             DSX_TIMED("tile_counts_kernel", cs);

@@ -131,3 +131,39 @@ def test_tangents_and_transforms_are_refused():
         torch.func.grad(lambda m: call(r, [m] + plain[1:]).sum())(plain[0])
     with pytest.raises(RuntimeError):
         torch.func.vmap(lambda m: call(r, [m] + plain[1:]))(plain[0][None])
+
+
+def test_counts_belong_to_the_call_that_waits_for_them():
+    """A call that was begun and given up (an allocation failed) writes its counts all the same; the next call of
+    the thread waits for its own."""
+    import ctypes
+    from ds_splat_amd import _native as N, stages
+    lib, stream = N.load(), torch.cuda.current_stream().cuda_stream
+    ptr = lambda x: ctypes.c_void_p(x.data_ptr() if x is not None else None)
+    kept = []
+
+    def begin(n, scale_mul):
+        sc = make_scene("cfg0", n=n, width=256, height=192, seed=3)
+        cam = stages.camera_from_scene(sc, torch.device(DEV), list_bin=2)
+        t = [sc[k].to(DEV) for k in ("means_3d", "scales", "rotations", "opacities", "shs")]
+        t[1] = t[1] * scale_mul
+        order = stages.new_order(cam, n, DEV)
+        bufs = [torch.empty((n, N.SPLAT_FLOATS), device=DEV), torch.empty(n, dtype=torch.int32, device=DEV),
+                torch.empty(int(lib.dsx_num_blocks(n)), dtype=torch.int32, device=DEV)]
+        kept.append((cam, t, order, bufs))
+        N.check(lib.dsx_forward_project_begin(cam.ref, n, *map(ptr, t), ptr(None), ptr(None), ptr(bufs[0]),
+                                              ptr(bufs[1]), ptr(None), ptr(bufs[2]), ptr(order), order.numel(), stream))
+        return cam
+
+    def counts(cam, n):
+        two = (ctypes.c_int64 * 2)()
+        N.check(lib.dsx_forward_project_counts(cam.ref, n, ctypes.byref(two), stream))
+        return two[0], two[1]
+
+    want = counts(begin(5000, 1.0), 5000)
+    other = counts(begin(60000, 2.0), 60000)
+    assert 0 < want[0] <= want[1] < other[0]
+    for _ in range(20):
+        begin(60000, 2.0)
+        assert counts(begin(5000, 1.0), 5000) == want
+    torch.cuda.synchronize()
