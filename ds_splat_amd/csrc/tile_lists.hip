@@ -1633,16 +1633,25 @@ int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_
 
 // ---------------------------------------------------------------------------------------
 // emission in depth order: a workgroup owns a range of OUTPUT pairs and walks the blocks of 256
-// depth-ordered Gaussians that reach into it; one thread per output pair, so the work per
+// depth-ordered Gaussians that reach into it; four output pairs to a thread, so the work per
 // workgroup is bounded and the stores are contiguous however uneven the tile counts are
 // ---------------------------------------------------------------------------------------
 
-#ifndef DSX_EMIT_WINDOWS
-#define DSX_EMIT_WINDOWS 4
-#endif
-constexpr int kEmitWindows = DSX_EMIT_WINDOWS; // windows of 256 outputs per round of the emission
-constexpr int kEmitChunkMax = 4096;            // outputs per workgroup: at most this many ...
-constexpr int kEmitWorkgroups = 4096;          // ... and fewer when that leaves less than this many workgroups
+// Bound by the issue of vector instructions where a Gaussian has many pairs, so a thread makes four consecutive ones:
+// the scan for their owners and the division of the first one's place are paid once, the others advance by one or
+// begin a run, and the stores are 16 bytes wide.  18 M pairs of 1 M Gaussians: 89 instructions a pair and 51 us with
+// one pair to a thread -> 39; 3.4 M of 3 M Gaussians, most of them out of sight, 27 -> 25.  (1024 workgroups: 29 and 40; 4096: 26 and 40.)
+constexpr int kEmitQuad = 4;                        // consecutive outputs of a thread
+constexpr int kEmitRound = kEmitQuad * kProjBlock;  // outputs of a workgroup's round
+constexpr int kEmitChunkMax = 4096;                 // outputs per workgroup: at most this many ...
+constexpr int kEmitWorkgroups = 2048;               // ... and fewer when that leaves less than this many workgroups
+
+// four words at an address that is a multiple of their own size only (the lists may begin anywhere)
+template <typename T>
+struct __attribute__((packed, aligned(alignof(T)))) Quad
+{
+    T v[kEmitQuad];
+};
 
 // kMasks (lists per bin, SlotT = uint32_t): the high half of a pair's slot word says which tiles of the
 // bin the Gaussian's rectangle covers, bit x for the columns and bit 8 + y for the rows of the bin
@@ -1661,22 +1670,23 @@ __global__ __launch_bounds__(kProjBlock) void emit_ordered_kernel(const uint32_t
                                                                   uint32_t* __restrict__ clear, int64_t clear_words,
                                                                   int chunk)
 {
-    __shared__ uint32_t s_off[kProjBlock + 1];
-    // per Gaussian of the block: x = first output, y = slot of the rectangle's first tile (0 for
-    // negative depths), z = width (0 marks a negative depth: every pair goes to slot 0), w = id
+    // per Gaussian of the block: x = first output, y = slot of the rectangle's first tile or bin, z = lists in
+    // a row of the rectangle (16 bits; bit 31: a negative depth, all pairs go to slot 0), with masks also the
+    // rectangle's first column and row (3 bits each) and w = the ones behind its last (16 bits each), all
+    // counted from the first bin's
     __shared__ uint4 s_rec[kProjBlock];
-    __shared__ uint2 s_rect[kMasks ? kProjBlock : 1]; // the tile rectangles themselves (for the masks)
+    __shared__ uint32_t s_id[kProjBlock];
+    __shared__ uint32_t s_total;
     __shared__ __attribute__((aligned(16))) uint32_t wave_tot[kProjBlock / DSX_WAVE];
-    __shared__ uint32_t s_mark[kEmitWindows * kProjBlock];
-    __shared__ __attribute__((aligned(16))) uint32_t s_wave_max[kEmitWindows][kProjBlock / DSX_WAVE];
+    __shared__ __attribute__((aligned(16))) uint32_t s_mark[kEmitRound];
+    __shared__ __attribute__((aligned(16))) uint32_t s_wave_max[kProjBlock / DSX_WAVE];
     static_assert(kProjBlock == 4 * DSX_WAVE, "four wavefronts per workgroup");
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
-#pragma unroll
-    for(int wdw = 0; wdw < kEmitWindows; ++wdw)
-        s_mark[wdw * kProjBlock + tid] = 0;
+    uint4* const my_marks = reinterpret_cast<uint4*>(s_mark) + tid;
+    *my_marks = make_uint4(0u, 0u, 0u, 0u);
 
     // the tile ranges were derived from the rectangles before any pair existed: hand them out
     for(int j = blockIdx.x * kProjBlock + tid; j < range_count; j += gridDim.x * kProjBlock)
@@ -1721,23 +1731,21 @@ __global__ __launch_bounds__(kProjBlock) void emit_ordered_kernel(const uint32_t
         if(p < n)
         {
             // (ntx: lists per row, i.e. bins per row when the lists are binned)
-            const uint32_t g = order[p];
+            s_id[tid] = order[p];
             const uint2 r = rects_sorted[p];
             count = list_count(r, shift);
+            const uint32_t sx = r.x & 0xffffu, sy = r.x >> 16, w = r.y & 0xffffu, h = (r.y >> 16) & 0x7fffu;
             const bool negative = (r.y >> 31) != 0;
-            uint32_t first_x = r.x & 0xffffu, first_y = r.x >> 16, w = r.y & 0xffffu;
-            if(shift && count && !negative)
-            {
-                const BinRect b = bin_rect(r, shift);
-                first_x = b.bx;
-                first_y = b.by;
-                w = b.bw;
-            }
-            rec.y = negative ? 0u : first_y * (uint32_t)ntx + first_x + 1u;
-            rec.z = negative ? 0u : w;
-            rec.w = g;
+            rec.y = (sy >> shift) * (uint32_t)ntx + (sx >> shift) + 1u;
+            rec.z = w;
             if(kMasks)
-                s_rect[tid] = r;
+            {
+                const uint32_t x = sx & ((1u << shift) - 1u), y = sy & ((1u << shift) - 1u);
+                rec.z = (count ? bin_rect(r, shift).bw : 1u) | (x << 16) | (y << 19);
+                rec.w = (x + w) | ((y + h) << 16);
+            }
+            if(negative)
+                rec.z = 0x8000ffffu;
         }
         const uint32_t incl = wave_incl_scan32(count, lane);
         if(lane == 63)
@@ -1745,102 +1753,113 @@ __global__ __launch_bounds__(kProjBlock) void emit_ordered_kernel(const uint32_t
         __syncthreads();
         const uint32_t prefix = sum_of_waves_before<kProjBlock / DSX_WAVE>(wave_tot, wave);
         rec.x = prefix + incl - count;
-        s_off[tid] = rec.x;
         s_rec[tid] = rec;
         if(tid == kProjBlock - 1)
-            s_off[kProjBlock] = prefix + incl;
+            s_total = prefix + incl;
         __syncthreads();
 
-        const uint32_t total = s_off[kProjBlock];
-        const uint32_t my_start = s_off[tid];
+        const int total = (int)s_total, my_start = (int)rec.x; // (fewer than 2^30 pairs in all)
         // the block's outputs that fall into the share: [ja, jb) of its `total`
-        const uint32_t ja = (uint32_t)(max(o0, base) - base);
-        const uint32_t jb = (uint32_t)(min(o1, base + (int64_t)total) - base);
+        const int ja = (int)(max(o0, base) - base);
+        const int jb = (int)(min(o1, base + (int64_t)total) - base);
         if(jb <= ja) // uniform (an empty block, or one that ends before the share)
             continue;
         // Which Gaussian owns output j?  Every Gaussian that emits marks the output where its run
         // starts with (its index + 1); the owner of j is the largest mark at or before j, i.e. an
-        // inclusive max-scan over the outputs (DPP inside the wavefront, LDS across wavefronts
-        // and across rounds of 256 outputs).  Costs a dozen VALU instructions per output
-        // instead of the eight dependent LDS reads of a binary search.
-        // A block of near Gaussians can own tens of thousands of outputs while the workgroup
-        // walks them serially, so a round covers kEmitWindows windows of 256 outputs with two
-        // barriers in all (the kernel's time is the longest such walk).
+        // inclusive max-scan over the outputs: inside a thread's four, over the wavefront (DPP), over the
+        // wavefronts and over the rounds (LDS).
         uint32_t carry = 0; // mark of the owner of the last output before the round
         if(ja > 0)          // uniform: the share starts inside the block
         {
             // the last Gaussian whose run starts before ja (starts are monotone in the thread index)
             const uint64_t early = __ballot(count && my_start < ja);
             if(lane == 0)
-                s_wave_max[0][wave] = early ? (uint32_t)(wave * DSX_WAVE + 64 - __builtin_clzll(early)) : 0u;
+                s_wave_max[wave] = early ? (uint32_t)(wave * DSX_WAVE + 64 - __builtin_clzll(early)) : 0u;
             __syncthreads();
-            carry = max(max(s_wave_max[0][0], s_wave_max[0][1]), max(s_wave_max[0][2], s_wave_max[0][3]));
+            carry = max(max(s_wave_max[0], s_wave_max[1]), max(s_wave_max[2], s_wave_max[3]));
             __syncthreads();
         }
-        for(uint32_t j0 = ja; j0 < jb; j0 += kEmitWindows * kProjBlock) // uniform
+        // (rounds begin at a multiple of four of the whole output: a thread's four lie in one 16-byte word of it)
+        for(int j0 = ja - (int)((base + ja) & (kEmitQuad - 1)); j0 < jb; j0 += kEmitRound) // uniform
         {
-            if(count && my_start >= j0 && my_start < j0 + kEmitWindows * kProjBlock)
+            if(count && my_start >= j0 && my_start < j0 + kEmitRound)
                 s_mark[my_start - j0] = (uint32_t)tid + 1u;
             __syncthreads();
-            uint32_t m[kEmitWindows];
-#pragma unroll
-            for(int wdw = 0; wdw < kEmitWindows; ++wdw)
-            {
-                m[wdw] = s_mark[wdw * kProjBlock + tid];
-                s_mark[wdw * kProjBlock + tid] = 0; // ready for the next round (and the next block)
-                m[wdw] = wave_incl_max_scan(m[wdw]);
-                if(lane == 63)
-                    s_wave_max[wdw][wave] = m[wdw];
-            }
+            const uint4 m = *my_marks;
+            *my_marks = make_uint4(0u, 0u, 0u, 0u); // ready for the next round (and the next block)
+            const uint32_t mark[kEmitQuad] = {m.x, m.y, m.z, m.w};
+            const uint32_t incl_max = wave_incl_max_scan(max(max(m.x, m.y), max(m.z, m.w)));
+            if(lane == 63)
+                s_wave_max[wave] = incl_max;
             __syncthreads();
-            uint32_t before = carry; // largest mark before this thread's output of the current window
-#pragma unroll
-            for(int wdw = 0; wdw < kEmitWindows; ++wdw)
+            const uint4 wm = *reinterpret_cast<const uint4*>(s_wave_max);
+            // the owner of the output before this thread's first (wave_shr:1: the lane below)
+            uint32_t owner = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)incl_max, 0x138, 0xf, 0xf, false);
+            owner = max(max(owner, carry), max(wave > 0 ? wm.x : 0u, max(wave > 1 ? wm.y : 0u, wave > 2 ? wm.z : 0u)));
+            carry = max(carry, max(max(wm.x, wm.y), max(wm.z, wm.w)));
+            const int j = j0 + kEmitQuad * tid;
+            if(j < jb)
             {
-                // the four wavefronts' maxima in one 16-byte read; the earlier wavefronts' count for this one
-                static_assert(kProjBlock / DSX_WAVE == 4, "four wavefronts per emission workgroup");
-                const uint4 wm = *reinterpret_cast<const uint4*>(s_wave_max[wdw]);
-                const uint32_t mine = max(max(before, wave > 0 ? wm.x : 0u), max(wave > 1 ? wm.y : 0u, wave > 2 ? wm.z : 0u));
-                const uint32_t owner = max(m[wdw], mine) - 1u; // every output has an owner: never 0 - 1
-                before = max(before, max(max(wm.x, wm.y), max(wm.z, wm.w)));
-                const uint32_t j = j0 + wdw * kProjBlock + tid;
-                if(j < jb)
+                Quad<SlotT> slot4;
+                Quad<int32_t> id4;
+                uint32_t rx = 0, ry = 0, w = 0, row = 0; // the place in the rectangle, its width, slots of the rows before
+#pragma unroll
+                for(int i = 0; i < kEmitQuad; ++i)
                 {
-                    const uint4 own = s_rec[owner]; // one 16-byte LDS read per output
-                    const uint32_t r = j - own.x;
-                    const uint32_t w = own.z;
-                    uint32_t slot = kMasks ? 0xffff0000u : 0u;
-                    if(w)
+                    owner = max(owner, mark[i]);
+                    const uint4 rec_i = s_rec[(owner - 1u) & (kProjBlock - 1)]; // (every output of the share has an owner)
+                    if(i == 0)
                     {
+                        const uint32_t r = (uint32_t)j - rec_i.x;
+                        w = rec_i.z & 0xffffu;
                         // r / w by a float reciprocal (r < 2^24 tiles per Gaussian), corrected by one step
-                        uint32_t ry = (uint32_t)((float)r * __builtin_amdgcn_rcpf((float)w));
+                        ry = (uint32_t)((float)r * __builtin_amdgcn_rcpf((float)w));
                         if(ry * w > r)
                             --ry;
                         else if((ry + 1) * w <= r)
                             ++ry;
-                        const uint32_t rx = r - ry * w;
-                        slot = own.y + ry * (uint32_t)ntx + rx;
-                        if(kMasks)
-                        {
-                            // the rectangle's columns and rows inside this bin, as bit ranges [lo, hi]
-                            const uint2 tr = s_rect[owner];
-                            const int side = 1 << shift;
-                            const int tsx = (int)(tr.x & 0xffffu), tsy = (int)(tr.x >> 16);
-                            const int tw = (int)(tr.y & 0xffffu), th = (int)((tr.y >> 16) & 0x7fffu);
-                            const int x0 = (int)(((uint32_t)tsx >> shift) + rx) << shift; // the bin's first column
-                            const int y0 = (int)(((uint32_t)tsy >> shift) + ry) << shift;
-                            const int xlo = max(tsx - x0, 0), xhi = min(tsx + tw - 1 - x0, side - 1);
-                            const int ylo = max(tsy - y0, 0), yhi = min(tsy + th - 1 - y0, side - 1);
-                            const uint32_t xm = ((2u << xhi) - 1u) & ~((1u << xlo) - 1u);
-                            const uint32_t ym = ((2u << yhi) - 1u) & ~((1u << ylo) - 1u);
-                            slot |= (xm | (ym << 8)) << 16;
-                        }
+                        rx = r - ry * w;
+                        row = ry * (uint32_t)ntx;
                     }
-                    slots[base + j] = (SlotT)slot;
-                    ids[base + j] = (int32_t)own.w;
+                    else
+                    {
+                        ++rx;
+                        const bool next_row = rx == w, next_run = mark[i] != 0;
+                        rx = next_row || next_run ? 0u : rx;
+                        ry = next_run ? 0u : ry + (next_row ? 1u : 0u);
+                        row = next_run ? 0u : row + (next_row ? (uint32_t)ntx : 0u);
+                        w = rec_i.z & 0xffffu;
+                    }
+                    uint32_t slot = row + rec_i.y + rx;
+                    if(kMasks)
+                    {
+                        // the rectangle's columns and rows inside this bin, as bit ranges [lo, hi)
+                        const int side = 1 << shift, x0 = (int)(rx << shift), y0 = (int)(ry << shift);
+                        const int xlo = max((int)((rec_i.z >> 16) & 7u) - x0, 0), ylo = max((int)((rec_i.z >> 19) & 7u) - y0, 0);
+                        const int xhi = min((int)(rec_i.w & 0xffffu) - x0, side), yhi = min((int)(rec_i.w >> 16) - y0, side);
+                        slot |= ((1u << 16) << xhi) - ((1u << 16) << xlo) + ((1u << 24) << yhi) - ((1u << 24) << ylo);
+                    }
+                    slot = (int)rec_i.z < 0 ? (kMasks ? 0xffff0000u : 0u) : slot;
+                    slot4.v[i] = (SlotT)slot;
+                    id4.v[i] = (int32_t)s_id[(owner - 1u) & (kProjBlock - 1)];
+                }
+                const int64_t out = base + j;
+                if(j >= ja && j + kEmitQuad <= jb)
+                {
+                    *reinterpret_cast<Quad<SlotT>*>(slots + out) = slot4;
+                    *reinterpret_cast<Quad<int32_t>*>(ids + out) = id4;
+                }
+                else
+                {
+#pragma unroll
+                    for(int i = 0; i < kEmitQuad; ++i)
+                        if(j + i >= ja && j + i < jb)
+                        {
+                            slots[out + i] = slot4.v[i];
+                            ids[out + i] = id4.v[i];
+                        }
                 }
             }
-            carry = before;
             // (the next round's marks are written after this round's reads of s_wave_max: the
             // barrier after them orders both)
         }

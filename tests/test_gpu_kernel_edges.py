@@ -3,6 +3,7 @@ import numpy as np
 import pytest
 import torch
 
+import test_gpu_stages
 from ds_splat_amd.synthetic import make_scene
 
 pytestmark = pytest.mark.gpu
@@ -36,3 +37,18 @@ def test_depth_order_of_few_gaussians(n, depths):
     touched[keys == 0xffffffff] = 0
     sums = np.add.reduceat(touched[perm], np.arange(0, n, 256))
     assert (offsets[:len(sums)] == np.cumsum(sums) - sums).all()
+
+
+@pytest.mark.parametrize("bin_side", [1, 2, 8])
+@pytest.mark.parametrize("n,W,H,scale_mul,flip,giants", [
+    (3, 48, 40, 0.1, 0, 0),               # runs shorter than a thread's four outputs
+    (257, 100, 70, 0.2, 5, 0),            # a block of 256 Gaussians and one more
+    (700, 300, 200, 1.0, 90, 2),          # shares that end inside a Gaussian's run, behind the camera and in front
+    (400, 140000, 64, 20.0, 0, 3),        # rectangles of 8750 columns: their ends need more than 13 bits
+])
+def test_emission_of_four_pairs_to_a_thread(oracle, list_bin, bin_side, n, W, H, scale_mul, flip, giants):
+    if bin_side == 1:
+        test_gpu_stages.test_tile_lists_bit_exact(oracle, list_bin, n, W, H, scale_mul, flip, giants=giants)
+    else:
+        test_gpu_stages.test_binned_tile_lists_vs_oracle(oracle, list_bin, bin_side, n, W, H, scale_mul, flip, giants,
+                                                         "identity")
