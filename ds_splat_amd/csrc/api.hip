@@ -234,7 +234,7 @@ static int project_fwd_checked(const dsx_camera* cam, int64_t n, const float* me
     if(!means3d || !opacities || !splats || !radii || !block_sums)
         return DSX_ERR_BAD_ARG; // cov3d may be null: not stored
     uint32_t* depth_keys = nullptr;
-    uint2* rects = nullptr;
+    uint2 *rects = nullptr, *key_ranges = nullptr;
     if(order)
     {
         const OrderLayout o = order_layout(n, cam->image_width, cam->image_height, cam->list_bin);
@@ -242,6 +242,7 @@ static int project_fwd_checked(const dsx_camera* cam, int64_t n, const float* me
             return DSX_ERR_WORKSPACE;
         depth_keys = reinterpret_cast<uint32_t*>(static_cast<char*>(order) + o.depth_keys);
         rects = reinterpret_cast<uint2*>(static_cast<char*>(order) + o.rects);
+        key_ranges = reinterpret_cast<uint2*>(static_cast<char*>(order) + o.key_ranges);
     }
     if(!cov3d_precomp && (!scales || !quats))
         return DSX_ERR_BAD_ARG;
@@ -252,7 +253,8 @@ static int project_fwd_checked(const dsx_camera* cam, int64_t n, const float* me
     if(order && clear_for_depth_order)
         depth_order_clear_region(*cam, n, order, &clear, &clear_words);
     return launch_project_fwd(*cam, n, means3d, scales, quats, opacities, shs, cov3d_precomp, colors_precomp, splats,
-                              radii, cov3d, block_sums, depth_keys, rects, as_stream(stream), clear, clear_words);
+                              radii, cov3d, block_sums, depth_keys, rects, key_ranges, as_stream(stream), clear,
+                              clear_words);
 }
 
 extern "C" int dsx_project_fwd(const dsx_camera* cam, int64_t n, const float* means3d, const float* scales,
@@ -519,18 +521,15 @@ static int check_pair_counts(int64_t list_pairs, int64_t tile_pairs)
 // its own when the next one is waiting: every call has a ticket, which the words carry, and the next of several slots.
 namespace
 {
-constexpr unsigned kCountSlots = 16;
+constexpr unsigned kCountSlots = 16, kSlotWords = 4;
 struct PinnedCounts
 {
     int64_t* words = nullptr;
     unsigned calls = 0;
-    unsigned ticket() const
+    HostCounts current() const
     {
-        return calls % 0x7fffeu + 1u; // 19 bits: a marked word is never negative, and never zero
-    }
-    volatile int64_t* slot() const
-    {
-        return words + 2 * (calls % kCountSlots);
+        // (19 bits: a marked word is never negative, and never zero)
+        return {reinterpret_cast<unsigned long long*>(words + kSlotWords * (calls % kCountSlots)), calls % 0x7fffeu + 1u};
     }
     ~PinnedCounts()
     {
@@ -546,33 +545,31 @@ HostCounts next_counts()
     if(g_counts.words == nullptr)
     {
         void* p = nullptr;
-        if(hipHostMalloc(&p, 2 * kCountSlots * sizeof(int64_t),
+        if(hipHostMalloc(&p, kSlotWords * kCountSlots * sizeof(int64_t),
                          hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
             return {};
         g_counts.words = static_cast<int64_t*>(p);
-        std::fill_n(g_counts.words, 2 * kCountSlots, 0);
+        std::fill_n(g_counts.words, kSlotWords * kCountSlots, 0);
     }
     ++g_counts.calls;
-    volatile int64_t* const slot = g_counts.slot();
-    slot[0] = slot[1] = 0;
-    return {reinterpret_cast<unsigned long long*>(const_cast<int64_t*>(slot)), g_counts.ticket()};
+    const HostCounts next = g_counts.current();
+    for(unsigned i = 0; i < kSlotWords; ++i)
+        static_cast<volatile unsigned long long*>(next.words)[i] = 0;
+    return next;
 }
-// Waits until both words of the calling thread's last call are there.  Every wait ends: when the stream has run dry
-// (or into an error) without them.
-bool wait_for_counts(hipStream_t stream, int64_t (&counts)[2])
+} // namespace
+
+namespace dsx
 {
-    if(g_counts.words == nullptr)
+// Every wait ends: when the stream has run dry (or into an error) without the word.
+bool wait_for_word(const HostCounts& to_host, int word, hipStream_t stream, uint64_t* value)
+{
+    if(to_host.words == nullptr)
         return false;
-    volatile const int64_t* const slot = g_counts.slot();
     auto arrived = [&] {
-        counts[0] = slot[0];
-        counts[1] = slot[1];
-        const int64_t ticket = g_counts.ticket();
-        if((counts[0] >> kTicketShift) != ticket || (counts[1] >> kTicketShift) != ticket)
-            return false;
-        for(int64_t& c : counts)
-            c &= (1ll << kTicketShift) - 1;
-        return true;
+        const uint64_t v = static_cast<const volatile unsigned long long*>(to_host.words)[word];
+        *value = v & ((1ull << kTicketShift) - 1);
+        return (v >> kTicketShift) == to_host.ticket;
     };
     for(int64_t spins = 1;; ++spins)
     {
@@ -588,7 +585,7 @@ bool wait_for_counts(hipStream_t stream, int64_t (&counts)[2])
         }
     }
 }
-} // namespace
+} // namespace dsx
 
 extern "C" int dsx_forward_project_begin(const dsx_camera* cam, int64_t n, const float* means3d, const float* scales,
                                          const float* quats, const float* opacities, const float* shs,
@@ -620,11 +617,14 @@ extern "C" int dsx_forward_project_counts(const dsx_camera* cam, int64_t n, int6
         return rc;
     if(n <= 0)
         return n == 0 ? DSX_OK : DSX_ERR_BAD_ARG;
-    int64_t counts[2];
-    if(!wait_for_counts(as_stream(stream), counts))
+    uint64_t counts[2] = {0, 0};
+    if(g_counts.words == nullptr)
         return DSX_ERR_RUNTIME;
+    for(int i = 0; i < 2; ++i)
+        if(!wait_for_word(g_counts.current(), i, as_stream(stream), counts + i))
+            return DSX_ERR_RUNTIME;
     // the device wrote (per-tile pairs, bin pairs); the caller gets (pairs of the lists, per-tile pairs)
-    const int64_t tile_pairs = counts[0], bin_pairs = counts[1];
+    const int64_t tile_pairs = (int64_t)counts[0], bin_pairs = (int64_t)counts[1];
     num_keys[0] = list_grid(*cam).shift ? bin_pairs : tile_pairs;
     num_keys[1] = tile_pairs;
     return check_pair_counts(num_keys[0], num_keys[1]);

@@ -154,6 +154,47 @@ inline Digits32 digits32(int key_bits)
     }
     return d;
 }
+// The depth sort of a whole forward: the keys' distances from the smallest one, in three digits of up to nine bits
+// instead of four of eight, wherever they fit 27 bits (depths within sixteen octaves of each other, all of one sign).
+// The range comes from the device (rounded outwards to 16 bits), so the host waits for it between the projection
+// and the passes, while the histograms are counted.  us of the passes and the histograms, four digits -> three: 500 K
+// keys 55 + 12 -> 45 + 6, 1 M 68 + 13 -> 56 + 8, 3 M 110 + 19 -> 100 + 17, 6 M 211 + 27 -> 199 + 26.
+constexpr int kDepthBits = 9;
+constexpr int kDepthBins = 1 << kDepthBits;
+constexpr int kDepthPasses = 3;
+constexpr size_t kSortWordsMost = 1536; // of a tile's look-back statuses (and of the histograms): 4 x 256 or 3 x 512
+struct DepthRange
+{
+    bool narrow;            // three digits; else the keys as they are, in four
+    uint32_t first, behind; // smallest key; one more than the largest distance: what a key without pairs becomes
+    Digits32 digits;
+};
+// lowest, highest: upper halves of the smallest and the largest key that emits (lowest > highest: there is none)
+__host__ __device__ inline DepthRange depth_range(uint32_t lowest, uint32_t highest)
+{
+    DepthRange r;
+    if(lowest > highest)
+        lowest = highest = 0;
+    r.first = lowest << 16;
+    r.behind = ((highest - lowest) << 16) + 0x10000u; // (no key that emits has all ones in its upper half: a NaN)
+    const int bits = 32 - __builtin_clz(r.behind);
+    r.narrow = bits <= kDepthPasses * kDepthBits && highest < 0xffffu;
+    if(!r.narrow)
+    {
+        r.first = 0;
+        r.behind = kNoPairsKey;
+    }
+    r.digits.passes = r.narrow ? kDepthPasses : kMaxPasses32;
+    int shift = 0;
+    for(int p = 0; p < kMaxPasses32; ++p)
+    {
+        const int width = r.narrow ? (p < kDepthPasses ? bits / kDepthPasses + (p < bits % kDepthPasses ? 1 : 0) : 0) : kBits32;
+        r.digits.shift[p] = shift;
+        r.digits.mask[p] = (1u << width) - 1u;
+        shift += width;
+    }
+    return r;
+}
 // bits needed for tile slots 0..num_tiles (slot 0 = keys with a negative depth, slot t+1 = tile t)
 inline int slot_bits(int num_tiles)
 {
@@ -243,6 +284,7 @@ struct OrderLayout
     size_t rects_sorted; // uint2[n] the same in depth order
     size_t rects32;    // uint32[n]  packed rectangles on their way through the depth sort
     size_t block_sums; // uint32[blocks + 1] tile counts of 256 consecutive Gaussians IN DEPTH ORDER, scanned
+    size_t key_ranges; // uint2[blocks] of 256 consecutive Gaussians' depth keys, upper halves: 0xffff - smallest, largest (zeros: none emits)
     size_t slot_hist;  // uint32[kMaxPasses32 * 256] digit histograms of the tile slots of all pairs
     size_t cover;      // int32[(ntx + 1) * (nty + 1) + 1] pairs per tile (corner grid, then its 2-D prefix sum)
     size_t bin_cover;  // int32[(nbx + 1) * (nby + 1) + 1] the same per bin (binned lists only)
@@ -268,7 +310,8 @@ struct ListsWorkspace
 ListsWorkspace lists_workspace(int64_t k, int num_tiles, bool binned);
 
 // launchers (each returns a dsx_status)
-// Two words of pinned host memory that receive a call's pair counts (null: none), each marked with the call's ticket.
+// Three words of pinned host memory that receive a call's pair counts and the range of its depth keys (null: none), each
+// marked with the call's ticket.
 struct HostCounts
 {
     unsigned long long* words = nullptr;
@@ -284,6 +327,8 @@ int launch_sort32(int64_t count, int key_bits, uint32_t* keys_a, uint32_t* vals_
 // already_cleared: the words of depth_order_clear_region are zero already (the projection did it)
 int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_t stream,
                        bool already_cleared = false, HostCounts to_host = {});
+// waits for a word of the calling thread's `to_host` (false: the stream has ended without it)
+bool wait_for_word(const HostCounts& to_host, int word, hipStream_t stream, uint64_t* value);
 // the part of an `order` buffer that must be zero when launch_depth_order starts
 void depth_order_clear_region(const dsx_camera& cam, int64_t n, void* order, uint32_t** words, int64_t* count);
 int launch_tile_lists(const dsx_camera& cam, int64_t n, int64_t k, const void* order, int32_t* sorted_ids,
@@ -292,7 +337,8 @@ int launch_project_fwd(const dsx_camera& cam, int64_t n, const float* means3d, c
                        const float* quats, const float* opacities, const float* shs,
                        const float* cov3d_precomp, const float* colors_precomp, float* splats,
                        int32_t* radii, float* cov3d, uint32_t* block_sums, uint32_t* depth_keys,
-                       uint2* rects, hipStream_t stream, uint32_t* clear = nullptr, int64_t clear_words = 0);
+                       uint2* rects, uint2* key_ranges, hipStream_t stream, uint32_t* clear = nullptr,
+                       int64_t clear_words = 0);
 int launch_scan_u32(int64_t count, uint32_t* data, uint32_t* total, hipStream_t stream);
 int launch_emit_keys(const dsx_camera& cam, int64_t n, int64_t k, const float* splats,
                      const uint32_t* block_offsets, int64_t* keys, int32_t* values,
@@ -389,6 +435,26 @@ struct KernelTimer
 __device__ __forceinline__ int lane_id()
 {
     return __lane_id();
+}
+
+// inclusive max-scan over the 64 lanes with data-parallel-primitive moves only (values >= 0,
+// lanes without a source keep 0): four shifts inside each row of 16, then the row broadcasts
+template <int kCtrl, int kRowMask>
+__device__ __forceinline__ uint32_t dpp_max(uint32_t v)
+{
+    const uint32_t moved = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, kRowMask, 0xf, false);
+    return max(v, moved);
+}
+
+__device__ __forceinline__ uint32_t wave_incl_max_scan(uint32_t v)
+{
+    v = dpp_max<0x111, 0xf>(v); // row_shr:1
+    v = dpp_max<0x112, 0xf>(v); // row_shr:2
+    v = dpp_max<0x114, 0xf>(v); // row_shr:4
+    v = dpp_max<0x118, 0xf>(v); // row_shr:8
+    v = dpp_max<0x142, 0xa>(v); // row_bcast:15 into rows 1 and 3
+    v = dpp_max<0x143, 0xc>(v); // row_bcast:31 into rows 2 and 3
+    return v;
 }
 
 // Sum of the first `wave` entries of a 16-byte aligned LDS array of kWaves per-wavefront totals

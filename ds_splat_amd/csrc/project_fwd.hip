@@ -43,6 +43,7 @@ struct ProjectParams
     float* cov3d;
     uint32_t* block_sums;
     uint32_t* depth_keys; // optional: depth bits per Gaussian, the key of the depth order
+    uint2* key_ranges;    // with depth_keys: OrderLayout::key_ranges
     uint2* rects;         // optional: packed tile rectangle per Gaussian (zero when it emits nothing)
     uint32_t* clear;      // optional: words that the kernel zeroes on the side (counters of the sort that follows)
     int64_t clear_words;
@@ -183,6 +184,7 @@ __global__ __launch_bounds__(kProjBlock) void project_fwd_kernel(const ProjectPa
 {
     __shared__ float sh_lds[4][64 * kShPitch];
     __shared__ uint32_t wave_sums[4];
+    __shared__ uint2 wave_ranges[4];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -263,7 +265,7 @@ __global__ __launch_bounds__(kProjBlock) void project_fwd_kernel(const ProjectPa
             rgb = make_float3(fmaxf(rx + 0.5f, 0.0f), fmaxf(ry + 0.5f, 0.0f), fmaxf(rz + 0.5f, 0.0f));
     }
 
-    uint32_t count = 0;
+    uint32_t count = 0, near16 = 0, far16 = 0;
     if(live)
     {
         float c3[6];
@@ -389,6 +391,8 @@ __global__ __launch_bounds__(kProjBlock) void project_fwd_kernel(const ProjectPa
             // its rectangle is empty without a look at it.
             const uint32_t depth_bits = __float_as_uint(vz);
             p.depth_keys[i] = count ? depth_bits : kNoPairsKey;
+            near16 = count ? 0xffffu - (depth_bits >> 16) : 0u;
+            far16 = count ? depth_bits >> 16 : 0u;
             p.rects[i] = count ? make_uint2((uint32_t)r.sx | ((uint32_t)r.sy << 16),
                                             (uint32_t)(r.ex - r.sx) | ((uint32_t)(r.ey - r.sy) << 16) |
                                                 (depth_bits & 0x80000000u))
@@ -397,17 +401,29 @@ __global__ __launch_bounds__(kProjBlock) void project_fwd_kernel(const ProjectPa
     }
 
     const uint32_t ws = wave_sum_u32(count);
-    if(lane == 0)
+    near16 = wave_incl_max_scan(near16);
+    far16 = wave_incl_max_scan(far16);
+    if(lane == 63)
+    {
         wave_sums[wave] = ws;
+        wave_ranges[wave] = make_uint2(near16, far16);
+    }
     __syncthreads();
     if(tid == 0)
+    {
         p.block_sums[blockIdx.x] = wave_sums[0] + wave_sums[1] + wave_sums[2] + wave_sums[3];
+        if(p.depth_keys)
+            p.key_ranges[blockIdx.x] =
+                make_uint2(max(max(wave_ranges[0].x, wave_ranges[1].x), max(wave_ranges[2].x, wave_ranges[3].x)),
+                           max(max(wave_ranges[0].y, wave_ranges[1].y), max(wave_ranges[2].y, wave_ranges[3].y)));
+    }
 }
 
 int launch_project_fwd(const dsx_camera& cam, int64_t n, const float* means3d, const float* scales,
                        const float* quats, const float* opacities, const float* shs,
                        const float* cov3d_precomp, const float* colors_precomp, float* splats, int32_t* radii,
-                       float* cov3d, uint32_t* block_sums, uint32_t* depth_keys, uint2* rects, hipStream_t stream,
+                       float* cov3d, uint32_t* block_sums, uint32_t* depth_keys, uint2* rects,
+                       uint2* key_ranges, hipStream_t stream,
                        uint32_t* clear, int64_t clear_words)
 {
     if(n == 0)
@@ -435,6 +451,7 @@ int launch_project_fwd(const dsx_camera& cam, int64_t n, const float* means3d, c
     p.block_sums = block_sums;
     p.depth_keys = depth_keys;
     p.rects = depth_keys ? rects : nullptr;
+    p.key_ranges = key_ranges;
     // cpp/rasterizer_torch.cu:144-147
     p.focal_y = cam.image_height / (2 * cam.tanfovy);
     p.focal_x = cam.image_width / (2 * cam.tanfovx);

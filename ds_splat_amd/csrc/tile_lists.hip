@@ -77,24 +77,10 @@ __device__ __forceinline__ uint32_t wave_incl_scan32(uint32_t v, int)
     return wave_incl_scan_u32(v);
 }
 
-// inclusive max-scan over the 64 lanes with data-parallel-primitive moves only (values >= 0,
-// lanes without a source keep 0): four shifts inside each row of 16, then the row broadcasts
-template <int kCtrl, int kRowMask>
-__device__ __forceinline__ uint32_t dpp_max(uint32_t v)
+// number of set bits of a wavefront mask below this lane
+__device__ __forceinline__ uint32_t bits_below(uint64_t mask)
 {
-    const uint32_t moved = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, kRowMask, 0xf, false);
-    return max(v, moved);
-}
-
-__device__ __forceinline__ uint32_t wave_incl_max_scan(uint32_t v)
-{
-    v = dpp_max<0x111, 0xf>(v); // row_shr:1
-    v = dpp_max<0x112, 0xf>(v); // row_shr:2
-    v = dpp_max<0x114, 0xf>(v); // row_shr:4
-    v = dpp_max<0x118, 0xf>(v); // row_shr:8
-    v = dpp_max<0x142, 0xa>(v); // row_bcast:15 into rows 1 and 3
-    v = dpp_max<0x143, 0xc>(v); // row_bcast:31 into rows 2 and 3
-    return v;
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
 
 // lanes of the wavefront that hold the same digit of up to kMaxBits bits; uniform flow only
@@ -217,7 +203,7 @@ constexpr int kSpinLimit32 = 1 << 18; // bounded wait: a stuck predecessor ends 
 #endif
 constexpr int kLookBatch32 = DSX_LOOK32;
 
-static_assert(kSortThreads32 >= kBins32, "one thread per digit");
+static_assert(kSortThreads32 >= kDepthBins, "one thread per digit");
 static_assert(kSortThreads32 * kSortItemsMax32 <= 65535, "u16 ranks");
 
 // A tile rectangle as the projection packs it (16-bit fields) in 32 bits: 8 bits each for first
@@ -256,22 +242,30 @@ struct RectJob
 
 // vals_in == nullptr: the values are the input positions (iota).  keys_out == nullptr: the
 // keys are not needed after this pass.  KeyT: uint32_t, or uint16_t for tile slots that fit.
-template <typename KeyT, int kSort32Threads, int kSort32Items, bool kCarry>
+// kBits = 9: a pass of the depth sort over a known range; `range` turns the keys into their distances (the first pass)
+// and names what a key without pairs has become.
+struct KeyRange
+{
+    uint32_t first, behind, no_pairs;
+};
+template <typename KeyT, int kSort32Threads, int kSort32Items, bool kCarry, int kBits>
 __global__ __launch_bounds__(kSort32Threads) void onesweep32_kernel(
     const KeyT* __restrict__ keys_in, const uint32_t* __restrict__ vals_in, KeyT* __restrict__ keys_out,
     uint32_t* __restrict__ vals_out, int64_t count, int shift, uint32_t mask, const uint32_t* __restrict__ hist_counts,
-    uint32_t* status, uint32_t* tile_counter, uint32_t* error_flag, const RectJob rects)
+    uint32_t* status, uint32_t* tile_counter, uint32_t* error_flag, const RectJob rects,
+    const KeyRange range)
 {
     const uint2* __restrict__ gather_src = rects.gather_src;
     uint2* __restrict__ gather_dst = rects.gather_dst;
+    constexpr int kBins = 1 << kBits;
     constexpr int kSort32Tile = kSort32Threads * kSort32Items;
     constexpr int kSort32Waves = kSort32Threads / DSX_WAVE;
     __shared__ uint32_t s_keys[kSort32Tile]; // reused for the values in the second round
-    __shared__ uint16_t s_whist[kSort32Waves][kBins32];
-    __shared__ uint32_t s_digit_start[kBins32];
-    __shared__ uint32_t s_gbase[kBins32];
-    __shared__ __attribute__((aligned(16))) uint32_t s_wave_tot[kBins32 / DSX_WAVE];
-    __shared__ __attribute__((aligned(16))) uint32_t s_hist_tot[kBins32 / DSX_WAVE];
+    __shared__ uint16_t s_whist[kSort32Waves][kBins];
+    __shared__ uint32_t s_digit_start[kBins];
+    __shared__ uint32_t s_gbase[kBins];
+    __shared__ __attribute__((aligned(16))) uint32_t s_wave_tot[kBins / DSX_WAVE];
+    __shared__ __attribute__((aligned(16))) uint32_t s_hist_tot[kBins / DSX_WAVE];
     __shared__ uint32_t s_tile;
 
     const int tid = threadIdx.x;
@@ -280,13 +274,14 @@ __global__ __launch_bounds__(kSort32Threads) void onesweep32_kernel(
 
     if(tid == 0)
         s_tile = atomicAdd(tile_counter, 1u);
-    for(int j = tid; j < kSort32Waves * kBins32; j += kSort32Threads)
+    for(int j = tid; j < kSort32Waves * kBins; j += kSort32Threads)
         (&s_whist[0][0])[j] = 0;
     __syncthreads();
     const int64_t tile = s_tile;
     const int64_t tile_base = tile * kSort32Tile;
     const int tile_n = (int)min((int64_t)kSort32Tile, count - tile_base);
     const int bits = 32 - __builtin_clz(mask); // mask = 2^bits - 1, bits >= 1
+    auto digit_of = [shift, bits](uint32_t k) { return __builtin_amdgcn_ubfe(k, (uint32_t)shift, (uint32_t)bits); };
 
     // ---- load the keys (striped inside each wavefront: coalesced, order = (item, lane)) -----
     // Registers are what limits the blocks per compute unit here, so a thread keeps little per
@@ -304,7 +299,11 @@ __global__ __launch_bounds__(kSort32Threads) void onesweep32_kernel(
         // except the stores (tile position < tile_n).
         key[it] = 0xffffffffu;
         if(local < tile_n)
+        {
             key[it] = (uint32_t)__builtin_nontemporal_load(keys_in + tile_base + local);
+            if(kBits == kDepthBits)
+                key[it] = min(key[it] - range.first, range.behind);
+        }
     }
 
     // ---- wave-local stable rank ------------------------------------------------------------
@@ -312,9 +311,9 @@ __global__ __launch_bounds__(kSort32Threads) void onesweep32_kernel(
 #pragma unroll
     for(int it = 0; it < kSort32Items; ++it)
     {
-        const uint32_t d = (key[it] >> shift) & mask;
-        const uint64_t m = match_digit<kBits32>(d, bits);
-        const uint32_t below = (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+        const uint32_t d = digit_of(key[it]);
+        const uint64_t m = match_digit<kBits>(d, bits);
+        const uint32_t below = (uint32_t)bits_below(m);
         const uint32_t old = wh[d];
         __builtin_amdgcn_wave_barrier();
         if(below == 0)
@@ -331,10 +330,10 @@ __global__ __launch_bounds__(kSort32Threads) void onesweep32_kernel(
     __syncthreads();
 
     // ---- per-digit totals of the tile (thread d <-> digit d), wave offsets, digit starts ----
-    const bool digit_thread = tid < kBins32; // thread d owns digit d (bins above the mask stay empty)
+    const bool digit_thread = tid < kBins; // thread d owns digit d (bins above the mask stay empty)
     uint32_t total = 0;
     uint32_t hist_excl = 0;
-    uint32_t* my_status = status + tile * kBins32 + (digit_thread ? tid : 0);
+    uint32_t* my_status = status + tile * kBins + (digit_thread ? tid : 0);
     if(digit_thread)
     {
 #pragma unroll
@@ -361,13 +360,9 @@ __global__ __launch_bounds__(kSort32Threads) void onesweep32_kernel(
     __syncthreads();
     if(digit_thread)
     {
-        // totals of the digit wavefronts before this one: two 16-byte reads and selects (a loop over
-        // them compiles to dependent 4-byte reads under an exec mask, on every tile's critical path)
-        static_assert(kBins32 / DSX_WAVE == 4, "four digit wavefronts");
-        const uint4 wt = *reinterpret_cast<const uint4*>(s_wave_tot);
-        const uint4 ht = *reinterpret_cast<const uint4*>(s_hist_tot);
-        const uint32_t prefix = (wave > 0 ? wt.x : 0u) + (wave > 1 ? wt.y : 0u) + (wave > 2 ? wt.z : 0u);
-        const uint32_t hprefix = (wave > 0 ? ht.x : 0u) + (wave > 1 ? ht.y : 0u) + (wave > 2 ? ht.z : 0u);
+        // totals of the digit wavefronts before this one
+        const uint32_t prefix = sum_of_waves_before<kBins / DSX_WAVE>(s_wave_tot, wave);
+        const uint32_t hprefix = sum_of_waves_before<kBins / DSX_WAVE>(s_hist_tot, wave);
         s_digit_start[tid] = prefix + s_gbase[tid];
         hist_excl += hprefix;
     }
@@ -377,7 +372,7 @@ __global__ __launch_bounds__(kSort32Threads) void onesweep32_kernel(
 #pragma unroll
     for(int it = 0; it < kSort32Items; ++it)
     {
-        const uint32_t d = (key[it] >> shift) & mask;
+        const uint32_t d = digit_of(key[it]);
         const uint32_t p = ((pos2[it >> 1] >> (16 * (it & 1))) & 0xffffu) + s_digit_start[d] + s_whist[wave][d];
         s_keys[p] = key[it];
         pos2[it >> 1] = (it & 1) ? ((pos2[it >> 1] & 0xffffu) | (p << 16)) : ((pos2[it >> 1] & 0xffff0000u) | p);
@@ -424,7 +419,7 @@ __global__ __launch_bounds__(kSort32Threads) void onesweep32_kernel(
                 {
                     // rows below tile 0 are read as tile 0, whose status is inclusive from the start
                     const int64_t row = t - b > 0 ? t - b : 0;
-                    v[b] = __hip_atomic_load(status + row * kBins32 + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    v[b] = __hip_atomic_load(status + row * kBins + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
 #pragma unroll
                 for(int b = 0; b < kLookBatch32; ++b)
@@ -456,26 +451,22 @@ __global__ __launch_bounds__(kSort32Threads) void onesweep32_kernel(
     __syncthreads();
 
     // ---- scatter keys: consecutive threads -> consecutive addresses inside a digit's run ----
-    uint32_t dig4[(kSort32Items + 3) / 4]; // the digit of the key at tile position it * threads + tid, 8 bits each
+    uint32_t out[kSort32Items];            // where the key at tile position it * threads + tid goes
     uint32_t no_record = 0;                // bit it: that key is kNoPairsKey (its record is known to be zero)
 #pragma unroll
     for(int it = 0; it < kSort32Items; ++it)
     {
         const int j = it * kSort32Threads + tid;
         if((it & 3) == 0)
-        {
             __builtin_amdgcn_sched_barrier(0); // four items in flight at a time: registers, not latency, are scarce
-            dig4[it >> 2] = 0;
-        }
         if(j < tile_n)
         {
             const uint32_t kk = s_keys[j];
-            const uint32_t d = (kk >> shift) & mask;
-            dig4[it >> 2] |= d << (8 * (it & 3));
-            if(gather_src && kk == kNoPairsKey)
+            out[it] = s_gbase[digit_of(kk)] + (uint32_t)j;
+            if(gather_src && kk == (kBits == kDepthBits ? range.no_pairs : kNoPairsKey))
                 no_record |= 1u << it;
             if(keys_out)
-                keys_out[s_gbase[d] + (uint32_t)j] = (KeyT)kk;
+                keys_out[out[it]] = (KeyT)kk;
         }
     }
     __syncthreads();
@@ -496,12 +487,11 @@ __global__ __launch_bounds__(kSort32Threads) void onesweep32_kernel(
         if(j < tile_n)
         {
             const uint32_t v = s_keys[j];
-            const uint32_t out = s_gbase[(dig4[it >> 2] >> (8 * (it & 3))) & 0xffu] + (uint32_t)j;
-            vals_out[out] = v;
+            vals_out[out[it]] = v;
             // optional: a per-value record follows its value to the sorted position (the random
             // gather overlaps with the scatter traffic of the pass)
             if(gather_src)
-                gather_dst[out] = ((no_record >> it) & 1u) ? make_uint2(0u, 0u) : gather_src[v];
+                gather_dst[out[it]] = ((no_record >> it) & 1u) ? make_uint2(0u, 0u) : gather_src[v];
         }
     }
     if(kCarry)
@@ -521,11 +511,10 @@ __global__ __launch_bounds__(kSort32Threads) void onesweep32_kernel(
             if(j < tile_n)
             {
                 const uint32_t v = s_keys[j];
-                const uint32_t out = s_gbase[(dig4[it >> 2] >> (8 * (it & 3))) & 0xffu] + (uint32_t)j;
                 if(rects.unpack_dst)
-                    rects.unpack_dst[out] = rect_from_32(v);
+                    rects.unpack_dst[out[it]] = rect_from_32(v);
                 else
-                    rects.carry_out[out] = v;
+                    rects.carry_out[out[it]] = v;
             }
         }
     }
@@ -538,12 +527,13 @@ Sort32Workspace sort32_workspace(int64_t count, int key_bits, int tile_keys)
     w.passes = digits32(key_bits).passes;
     w.tiles = (count + tile_keys - 1) / tile_keys;
     size_t off = 0;
+    const size_t words = key_bits == 32 ? kSortWordsMost : (size_t)w.passes * kBins32; // (32 bits: perhaps a depth sort)
     w.hist = off;
-    off = align(off + (size_t)w.passes * kBins32 * 4);
+    off = align(off + words * 4);
     w.counters = off;
     off = align(off + (size_t)(w.passes + 1) * 4);
     w.status = off;
-    off = align(off + (size_t)w.passes * (size_t)w.tiles * kBins32 * 4);
+    off = align(off + words * (size_t)w.tiles * 4);
     w.bytes = off;
     return w;
 }
@@ -566,15 +556,17 @@ static int sort32_clear(int64_t count, int key_bits, int tile_keys, void* sort_w
 // gather.  carry_a / carry_b (with gather_src and gather_dst): the records travel through the passes
 // as packed 32-bit values instead, in ping-pong buffers of their own (the first pass packs them from
 // gather_src, the last one unpacks them into gather_dst).
-template <typename KeyT, int kThreads, int kItems, bool kCarry = false>
+// range: a depth sort over a known range (kBits = 9).
+template <typename KeyT, int kThreads, int kItems, bool kCarry = false, int kBits = kBits32>
 static int sort32_passes(int64_t count, int key_bits, KeyT* keys_a, uint32_t* vals_a, KeyT* keys_b, uint32_t* vals_b,
                          bool iota_values, bool keep_keys, void* sort_ws, const char* label, hipStream_t stream,
                          KeyT** keys_out, uint32_t** vals_out, const uint2* gather_src = nullptr,
                          uint2* gather_dst = nullptr, const uint32_t* counts = nullptr, uint32_t* carry_a = nullptr,
-                         uint32_t* carry_b = nullptr)
+                         uint32_t* carry_b = nullptr, const DepthRange* range = nullptr)
 {
+    constexpr int kBins = 1 << kBits;
     const Sort32Workspace w = sort32_workspace(count, key_bits, kThreads * kItems);
-    const Digits32 plan = digits32(key_bits);
+    const Digits32 plan = range ? range->digits : digits32(key_bits);
     char* base = static_cast<char*>(sort_ws);
     uint32_t* hist = reinterpret_cast<uint32_t*>(base + w.hist);
     uint32_t* counters = reinterpret_cast<uint32_t*>(base + w.counters);
@@ -586,9 +578,12 @@ static int sort32_passes(int64_t count, int key_bits, KeyT* keys_a, uint32_t* va
     uint32_t* vout = vals_b;
     uint32_t* cin = carry_a;
     uint32_t* cout = carry_b;
-    for(int p = 0; p < w.passes; ++p)
+    for(int p = 0; p < plan.passes; ++p)
     {
-        const bool last = p == w.passes - 1;
+        const bool last = p == plan.passes - 1;
+        KeyRange keys = {0u, 0xffffffffu, kNoPairsKey};
+        if(range)
+            keys = {p == 0 ? range->first : 0u, p == 0 ? range->behind : 0xffffffffu, range->behind};
         RectJob job = {};
         if(kCarry)
         {
@@ -604,11 +599,11 @@ static int sort32_passes(int64_t count, int key_bits, KeyT* keys_a, uint32_t* va
         }
         {
             DSX_TIMED(label, stream);
-            hipLaunchKernelGGL((onesweep32_kernel<KeyT, kThreads, kItems, kCarry>), dim3((unsigned)w.tiles), dim3(kThreads), 0,
+            hipLaunchKernelGGL((onesweep32_kernel<KeyT, kThreads, kItems, kCarry, kBits>), dim3((unsigned)w.tiles), dim3(kThreads), 0,
                                stream, (const KeyT*)kin, (const uint32_t*)((p == 0 && iota_values) ? nullptr : vin),
                                (last && !keep_keys) ? (KeyT*)nullptr : kout, vout, count, plan.shift[p], plan.mask[p],
-                               raw + p * kBins32, status + (size_t)p * w.tiles * kBins32,
-                               counters + p, counters + w.passes, job);
+                               raw + p * kBins, status + (size_t)p * w.tiles * kBins,
+                               counters + p, counters + w.passes, job, keys);
         }
         DSX_LAUNCH_CHECK();
         KeyT* tk = kin;
@@ -675,6 +670,91 @@ int launch_sort32(int64_t count, int key_bits, uint32_t* keys_a, uint32_t* vals_
     return DSX_ERR_RUNTIME;
 }
 
+// one of the words of pinned host memory that the host polls
+__device__ __forceinline__ void store_to_host(const HostCounts& to, int word, unsigned long long count)
+{
+    constexpr unsigned long long most = 1ull << (kTicketShift - 1);
+    __hip_atomic_store(to.words + word, (to.ticket << kTicketShift) | (count < most ? count : most), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// The histograms of a depth sort whose range only the device knows yet: every workgroup finds it from the projection's
+// blocks, the first one tells the host, and the digits are those of depth_range().
+__global__ __launch_bounds__(kHist32Threads) void depth_hist_kernel(const uint32_t* __restrict__ keys, int64_t count,
+                                                                    const uint2* __restrict__ ranges, int64_t blocks,
+                                                                    uint32_t* __restrict__ global_hist,
+                                                                    const HostCounts to_host)
+{
+    __shared__ uint32_t hist[kSortWordsMost];
+    __shared__ uint2 s_range[kHist32Threads / DSX_WAVE];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    for(int j = tid; j < (int)kSortWordsMost; j += kHist32Threads)
+        hist[j] = 0;
+    uint32_t near16 = 0, far16 = 0;
+    for(int64_t b = tid; b < blocks; b += kHist32Threads)
+    {
+        const uint2 r = ranges[b];
+        near16 = max(near16, r.x);
+        far16 = max(far16, r.y);
+    }
+    near16 = wave_incl_max_scan(near16);
+    far16 = wave_incl_max_scan(far16);
+    if(lane == 63)
+        s_range[wave] = make_uint2(near16, far16);
+    __syncthreads();
+#pragma unroll
+    for(int w = 0; w < kHist32Threads / DSX_WAVE; ++w)
+    {
+        near16 = w == 0 ? s_range[0].x : max(near16, s_range[w].x);
+        far16 = w == 0 ? s_range[0].y : max(far16, s_range[w].y);
+    }
+    const uint32_t lowest = 0xffffu - (uint32_t)__builtin_amdgcn_readfirstlane((int)near16);
+    const uint32_t highest = (uint32_t)__builtin_amdgcn_readfirstlane((int)far16);
+    if(blockIdx.x == 0 && tid == 0)
+        store_to_host(to_host, 2, lowest | ((unsigned long long)highest << 16));
+    const DepthRange range = depth_range(lowest, highest);
+    const int bins = range.narrow ? kDepthBins : kBins32;
+    uint32_t none = 0; // keys without pairs: counted by their thread, added to their bins at the end
+    const int64_t chunk = (int64_t)kHist32Threads * kHist32Items, chunks = (count + chunk - 1) / chunk;
+    for(int64_t c = blockIdx.x; c < chunks; c += gridDim.x)
+    {
+        uint32_t key[kHist32Items];
+        bool valid[kHist32Items];
+#pragma unroll
+        for(int it = 0; it < kHist32Items; ++it)
+        {
+            const int64_t i = c * chunk + it * kHist32Threads + tid;
+            valid[it] = i < count;
+            key[it] = valid[it] ? __builtin_nontemporal_load(keys + i) : 0u;
+        }
+#pragma unroll
+        for(int it = 0; it < kHist32Items; ++it)
+        {
+            if(valid[it] && key[it] == kNoPairsKey)
+            {
+                ++none;
+                valid[it] = false;
+            }
+            // (the top digit takes few values only where the depths span many octaves: the keys go by distance here)
+            if(valid[it])
+#pragma unroll
+                for(int p = 0; p < kMaxPasses32; ++p)
+                    if(p < range.digits.passes)
+                        atomicAdd(&hist[p * bins + (((key[it] - range.first) >> range.digits.shift[p]) & range.digits.mask[p])], 1u);
+        }
+    }
+    none = wave_sum_u32(none);
+    if(lane == 0 && none)
+#pragma unroll
+        for(int p = 0; p < kMaxPasses32; ++p)
+            if(p < range.digits.passes)
+                atomicAdd(&hist[p * bins + ((range.behind >> range.digits.shift[p]) & range.digits.mask[p])], none);
+    __syncthreads();
+    for(int j = tid; j < range.digits.passes * bins; j += kHist32Threads)
+        if(hist[j])
+            atomicAdd(&global_hist[j], hist[j]);
+}
+
 // ---------------------------------------------------------------------------------------
 // depth order of the Gaussians and the scanned tile counts in that order
 // ---------------------------------------------------------------------------------------
@@ -700,6 +780,8 @@ OrderLayout order_layout(int64_t n, int image_width, int image_height, int list_
     off = align(off + (size_t)n * 4);
     o.block_sums = off;
     off = align(off + (size_t)((n + kProjBlock - 1) / kProjBlock + 1) * 4);
+    o.key_ranges = off;
+    off = align(off + (size_t)((n + kProjBlock - 1) / kProjBlock) * 8);
     o.slot_hist = off;
     off = align(off + (size_t)kMaxPasses32 * kBins32 * 4);
     o.sort = off;
@@ -770,14 +852,6 @@ __global__ __launch_bounds__(kProjBlock) void ordered_block_sums_kernel(const ui
     __syncthreads();
     if(tid == 0)
         block_sums[blockIdx.x] = wave_sums[0] + wave_sums[1] + wave_sums[2] + wave_sums[3];
-}
-
-// one of the words of pinned host memory that the host polls
-__device__ __forceinline__ void store_to_host(const HostCounts& to, int word, unsigned long long count)
-{
-    constexpr unsigned long long most = 1ull << (kTicketShift - 1);
-    __hip_atomic_store(to.words + word, (to.ticket << kTicketShift) | (count < most ? count : most), __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // How many pairs each tile receives, straight from the rectangles (no pair is enumerated):
@@ -1502,7 +1576,66 @@ void depth_order_clear_region(const dsx_camera& cam, int64_t n, void* order, uin
     *count = (int64_t)((w.bytes + (o.ranges - o.cover)) / 4);
 }
 
-// to_host (optional): two words of pinned host memory that receive the pair counts (per-tile lists: what the
+// The depth sort of a whole forward (cleared workspace): ids in `ids_a`, rectangles in `rects_sorted`.
+static int launch_depth_sort(int64_t n, char* base, const OrderLayout& o, int64_t blocks, bool carry,
+                             const HostCounts& to_host, hipStream_t stream, uint32_t** vals_out)
+{
+    if(n >= (1ll << 30))
+        return DSX_ERR_TOO_LARGE;
+    uint32_t* const keys_a = reinterpret_cast<uint32_t*>(base + o.depth_keys);
+    uint32_t* const keys_b = reinterpret_cast<uint32_t*>(base + o.keys_alt);
+    uint32_t* const ids_a = reinterpret_cast<uint32_t*>(base + o.ids_a);
+    uint32_t* const ids_b = reinterpret_cast<uint32_t*>(base + o.ids_b);
+    const uint2* const rects = reinterpret_cast<const uint2*>(base + o.rects);
+    uint2* const rects_sorted = reinterpret_cast<uint2*>(base + o.rects_sorted);
+    uint32_t* const packed_a = reinterpret_cast<uint32_t*>(base + o.rects_sorted);
+    uint32_t* const packed_b = reinterpret_cast<uint32_t*>(base + o.rects32);
+    char* const ws = base + o.sort;
+    const Sort32Workspace w = sort32_workspace(n, 32, sort32_tile_keys(n));
+    const int64_t chunks = (n + kHist32Threads * kHist32Items - 1) / (kHist32Threads * kHist32Items);
+    {
+        DSX_TIMED("depth_hist_kernel", stream);
+        hipLaunchKernelGGL(depth_hist_kernel, dim3((unsigned)min((int64_t)DSX_HIST_BLOCKS, chunks)), dim3(kHist32Threads), 0,
+                           stream, (const uint32_t*)keys_a, n, reinterpret_cast<const uint2*>(base + o.key_ranges), blocks,
+                           reinterpret_cast<uint32_t*>(ws + w.hist), to_host);
+    }
+    DSX_LAUNCH_CHECK();
+    uint64_t ends;
+    if(!wait_for_word(to_host, 2, stream, &ends))
+        return DSX_ERR_RUNTIME;
+    const DepthRange range = depth_range((uint32_t)(ends & 0xffffu), (uint32_t)(ends >> 16));
+    uint32_t* ko;
+    const char* const label = "onesweep32_kernel<sort>";
+    // An even number of passes ends where it began, with an odd one the buffers change places: the ids end in ids_a
+    // either way, and the last pass never reads packed rectangles from the memory that it unpacks them into.
+#define DSX_DEPTH_SORT(ITEMS, CARRY)                                                                                    \
+    (range.narrow                                                                                                      \
+         ? sort32_passes<uint32_t, kSortThreads32, ITEMS, CARRY, kDepthBits>(n, 32, keys_a, ids_b, keys_b, ids_a, true, \
+                                                                             false, ws, label, stream, &ko, vals_out,   \
+                                                                             rects, rects_sorted, nullptr,              \
+                                                                             CARRY ? packed_b : nullptr,                \
+                                                                             CARRY ? packed_a : nullptr, &range)        \
+         : sort32_passes<uint32_t, kSortThreads32, ITEMS, CARRY>(n, 32, keys_a, ids_a, keys_b, ids_b, true, false, ws,  \
+                                                                 label, stream, &ko, vals_out, rects, rects_sorted,     \
+                                                                 nullptr, CARRY ? packed_a : nullptr,                   \
+                                                                 CARRY ? packed_b : nullptr))
+#define DSX_DEPTH_SORT_ITEMS(ITEMS) \
+    case ITEMS: return carry ? DSX_DEPTH_SORT(ITEMS, true) : DSX_DEPTH_SORT(ITEMS, false)
+    switch(sort32_items(n))
+    {
+        DSX_DEPTH_SORT_ITEMS(2);
+        DSX_DEPTH_SORT_ITEMS(3);
+        DSX_DEPTH_SORT_ITEMS(4);
+        DSX_DEPTH_SORT_ITEMS(6);
+        DSX_DEPTH_SORT_ITEMS(8);
+        DSX_DEPTH_SORT_ITEMS(kSortItemsMax32);
+    }
+#undef DSX_DEPTH_SORT_ITEMS
+#undef DSX_DEPTH_SORT
+    return DSX_ERR_RUNTIME;
+}
+
+// to_host (optional): words of pinned host memory that receive the pair counts (per-tile lists: what the
 // reference calls K, the fine ranges and final_idx index that many pairs; bin lists, zero when the lists
 // are per tile) as soon as the rectangles have been counted, while the sort still runs.
 int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_t stream, bool already_cleared,
@@ -1606,12 +1739,17 @@ int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_
         return finish(DSX_ERR_LAUNCH);
 
     uint32_t *ko, *vo;
-    // 32 key bits = 4 passes: the values (iota in pass 0) go b, a, b, a and end in ids_a
     // the rectangles travel through the passes when they pack into 32 bits (the passes end in
     // rects_sorted, whose first half holds the packed ones of the passes in between), else the last
     // pass gathers them
     const bool carry = tiles_x(cam.image_width) <= kRect32MaxTiles && tiles_y(cam.image_height) <= kRect32MaxTiles;
-    rc = launch_sort32(n, 32, keys_a, ids_a, keys_b, ids_b, true, false, base + o.sort, stream, &ko, &vo,
+    const int64_t blocks = (n + kProjBlock - 1) / kProjBlock;
+    // (a wait for the range: fewer Gaussians are sorted before the host could have launched the rest; us a step
+    // with four digits / three: 50 K 223 / 230, 100 K 249 / 260, 300 K 493 / 491, 1 M forward 319 / 305)
+    if(to_host.words && sort32_items(n) > 1)
+        rc = launch_depth_sort(n, base, o, blocks, carry, to_host, stream, &vo);
+    else // (four passes: the values, iota in the first, go b, a, b, a and end in ids_a)
+        rc = launch_sort32(n, 32, keys_a, ids_a, keys_b, ids_b, true, false, base + o.sort, stream, &ko, &vo,
                        reinterpret_cast<const uint2*>(base + o.rects), reinterpret_cast<uint2*>(base + o.rects_sorted),
                        true, carry ? reinterpret_cast<uint32_t*>(base + o.rects_sorted) : nullptr,
                        carry ? reinterpret_cast<uint32_t*>(base + o.rects32) : nullptr);
@@ -1619,7 +1757,6 @@ int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_
         return finish(rc);
     if(vo != ids_a)
         return finish(DSX_ERR_RUNTIME);
-    const int64_t blocks = (n + kProjBlock - 1) / kProjBlock;
     {
         DSX_TIMED("ordered_block_sums_kernel", stream);
         hipLaunchKernelGGL(ordered_block_sums_kernel, dim3((unsigned)blocks), dim3(kProjBlock), 0, stream,

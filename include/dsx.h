@@ -16,7 +16,7 @@
  * different streams of one device share it and their forked parts serialise there; (3) the
  * blend-kernel form override of dsx_set_blend_pixels_per_lane, a diagnostic that changes no result
  * of the forward and only the order of the backward's sums; (4) the device address of the
- * built-in scratch of dsx_backward_static, looked up once per device; (5) per host thread, 256 bytes of
+ * built-in scratch of dsx_backward_static, looked up once per device; (5) per host thread, 512 bytes of
  * pinned host memory that the pair counts arrive in, given back when the thread ends.
  *
  * What each entry point replaces in the reference (deepsense-ai/ds-splat) is cited as

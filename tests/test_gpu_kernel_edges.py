@@ -52,3 +52,49 @@ def test_emission_of_four_pairs_to_a_thread(oracle, list_bin, bin_side, n, W, H,
     else:
         test_gpu_stages.test_binned_tile_lists_vs_oracle(oracle, list_bin, bin_side, n, W, H, scale_mul, flip, giants,
                                                          "identity")
+
+
+@pytest.mark.parametrize("depths", ["uniform", "octaves", "too_many_octaves", "equal", "both_signs", "none"])
+@pytest.mark.parametrize("n", [262144, 262145, 530001])
+def test_depth_order_over_a_known_range(n, depths):
+    """The depth order inside a whole forward: three digits where the depths lie within sixteen octaves and have one
+    sign, else four; above and at the size from which the range is asked for."""
+    from ds_splat_amd import stages
+    sc = make_scene("cfg0", n=n, width=64, height=48, seed=9)
+    g = torch.Generator().manual_seed(n)
+    u = torch.rand(n, generator=g)
+    means = torch.zeros(n, 3)
+    means[:, 2] = {"uniform": 2.0 + 18.0 * u, "octaves": 0.02 * 2.0 ** (14.5 * u), "both_signs": 3.0 + u,
+                   "too_many_octaves": 0.015 * 2.0 ** (17.0 * u), "equal": 4.0 + 0.0 * u, "none": 2.0 + u}[depths]
+    if depths == "both_signs":       # (a mirrored point behind the camera passes the frustum test)
+        sc["projmatrix"][2, 2], sc["projmatrix"][3, 2] = -sc["projmatrix"][2, 2].abs(), sc["projmatrix"][3, 2].abs()
+        sc["projmatrix"][:, 2] = torch.tensor([0.0, 0.0, 0.0, 0.5])
+        sc["projmatrix"][:, 3] = torch.tensor([0.0, 0.0, 0.0, 1.0])
+        means[::3, 2] *= -1.0
+    if depths == "none":
+        means[:, 0] = 1e4
+    scales = (means[:, 2:].abs() * 1e-3).expand(n, 3).contiguous()
+    cam = stages.camera_from_scene(sc, DEV, list_bin=1)
+    seen = {}
+
+    def look(order, n_, k):
+        perm, offsets = stages.depth_order_view(n_, order)
+        seen["perm"], seen["offsets"] = perm.cpu().numpy().astype(np.int64), offsets.cpu().numpy().astype(np.int64)
+
+    _, st = stages.forward(cam, means.to(DEV), scales.to(DEV), sc["rotations"].to(DEV), sc["opacities"].to(DEV),
+                           sc["shs"].to(DEV), after_project=look)
+    touched = st.splats[:, 11].contiguous().view(torch.int32).cpu().numpy().astype(np.int64)
+    touched[-1] = 0
+    bits = st.splats[:, 2].contiguous().view(torch.int32).cpu().numpy().view(np.uint32)
+    keys = np.where(touched > 0, bits, np.uint32(0xffffffff))
+    emitting = keys != 0xffffffff
+    assert emitting.sum() == (0 if depths == "none" else n - 1)
+    if depths == "both_signs":
+        assert (keys[emitting] >> 31).any() and not (keys[emitting] >> 31).all()
+    if emitting.any() and depths != "both_signs":
+        span = int(keys[emitting].max() >> 16) - int(keys[emitting].min() >> 16) + 1
+        assert (span << 16 >= 1 << 27) == (depths == "too_many_octaves")
+    perm = np.argsort(keys, kind="stable")
+    assert (seen["perm"] == perm).all()
+    sums = np.add.reduceat(touched[perm], np.arange(0, n, 256))
+    assert (seen["offsets"] == np.concatenate([[0], np.cumsum(sums)])).all()
