@@ -62,7 +62,7 @@ def algorithmic_work(kernel, n, k, pixels, lists, coeffs, counters, marked, carr
         # v_cov3d are not written: the step gives neither colours nor covariances, so nothing takes them).  The
         # zeros of everybody else's outputs are stored by the blend backward's wavefronts (n * (52 + 12c) bytes).
         return "hbm", n + marked * (88 + 52 + 12 * coeffs), "B"
-    if kernel == "hist32_kernel":
+    if kernel in ("hist32_kernel", "depth_hist_kernel"):
         return "hbm", 4 * n, "B"
     if kernel == "onesweep32_kernel<sort>":
         # depth sort of the Gaussians: key + id, in and out; images of at most 255 x 255 tiles also carry each
