@@ -31,10 +31,6 @@ class Camera(C.Structure):
         ("campos", C.c_void_p),
         ("bg", C.c_void_p),
         ("list_bin", C.c_int32),
-        ("view_transposed", C.c_int32),
-        ("proj_transposed", C.c_int32),
-        ("planar", C.c_int32),
-        ("view_copy", C.c_void_p),
     ]
 
 
@@ -68,7 +64,7 @@ SIGNATURES = {
     "dsx_blend_bwd": (C.c_int, [_CAM, _I64, _I64] + [_P] * 7 + [_P]),
     "dsx_gaussian_bwd": (C.c_int, [_CAM, _I64, _I32] + [_P] * 7 + [_P] * 8 + [_P]),
     "dsx_forward_project": (C.c_int, [_CAM, _I64] + [_P] * 7 + [_P] * 4 + [_P, C.c_size_t, _P, _P]),
-    "dsx_forward_project_begin": (C.c_int, [_CAM, _I64] + [_P] * 7 + [_P] * 4 + [_P, C.c_size_t, _P]),
+    "dsx_forward_project_begin": (C.c_int, [_CAM, _I64] + [_P] * 7 + [_P] * 4 + [_P, C.c_size_t, _P, _P]),
     "dsx_forward_project_counts": (C.c_int, [_CAM, _I64, _P, _P]),
     "dsx_forward_finish": (C.c_int, [_CAM, _I64, _I64] + [_P] * 7 + [_P, C.c_size_t, _P, _P]),
     "dsx_backward": (C.c_int, [_CAM, _I64, _I64, _I32] + [_P] * 11 + [_P, _I32] + [_P] * 8 + [_P]),

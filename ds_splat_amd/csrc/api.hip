@@ -101,7 +101,7 @@ int check_camera(const dsx_camera* cam)
     // (cpp/rasterizer_torch.cu:124-129); degree 4 has no forward there, so 0..3 it is
     if(cam->sh_degree < 0 || cam->sh_degree > 3 || cam->max_sh_degree < cam->sh_degree || cam->max_sh_degree > 3)
         return DSX_ERR_BAD_ARG;
-    if(!valid_list_bin(cam->list_bin))
+    if(!valid_list_bin(camera_bin(*cam)))
         return DSX_ERR_BAD_ARG;
     return DSX_OK;
 }
@@ -223,7 +223,7 @@ static int project_fwd_checked(const dsx_camera* cam, int64_t n, const float* me
                                const float* quats, const float* opacities, const float* shs,
                                const float* cov3d_precomp, const float* colors_precomp, float* splats,
                                int32_t* radii, float* cov3d, uint32_t* block_sums, void* order, size_t order_bytes,
-                               void* stream, bool clear_for_depth_order)
+                               void* stream, bool clear_for_depth_order, float* view_copy = nullptr)
 {
     if(int rc = check_camera(cam))
         return rc;
@@ -237,7 +237,7 @@ static int project_fwd_checked(const dsx_camera* cam, int64_t n, const float* me
     uint2 *rects = nullptr, *key_ranges = nullptr;
     if(order)
     {
-        const OrderLayout o = order_layout(n, cam->image_width, cam->image_height, cam->list_bin);
+        const OrderLayout o = order_layout(n, cam->image_width, cam->image_height, camera_bin(*cam));
         if(order_bytes < o.bytes)
             return DSX_ERR_WORKSPACE;
         depth_keys = reinterpret_cast<uint32_t*>(static_cast<char*>(order) + o.depth_keys);
@@ -253,8 +253,8 @@ static int project_fwd_checked(const dsx_camera* cam, int64_t n, const float* me
     if(order && clear_for_depth_order)
         depth_order_clear_region(*cam, n, order, &clear, &clear_words);
     return launch_project_fwd(*cam, n, means3d, scales, quats, opacities, shs, cov3d_precomp, colors_precomp, splats,
-                              radii, cov3d, block_sums, depth_keys, rects, key_ranges, as_stream(stream), clear,
-                              clear_words);
+                              radii, cov3d, block_sums, depth_keys, rects, key_ranges, view_copy, as_stream(stream),
+                              clear, clear_words);
 }
 
 extern "C" int dsx_project_fwd(const dsx_camera* cam, int64_t n, const float* means3d, const float* scales,
@@ -369,7 +369,7 @@ extern "C" int dsx_depth_order(const dsx_camera* cam, int64_t n, void* order, si
         return DSX_OK;
     if(!order)
         return DSX_ERR_BAD_ARG;
-    if(order_bytes < order_layout(n, cam->image_width, cam->image_height, cam->list_bin).bytes)
+    if(order_bytes < order_layout(n, cam->image_width, cam->image_height, camera_bin(*cam)).bytes)
         return DSX_ERR_WORKSPACE;
     return launch_depth_order(*cam, n, order, as_stream(stream));
 }
@@ -591,12 +591,12 @@ extern "C" int dsx_forward_project_begin(const dsx_camera* cam, int64_t n, const
                                          const float* quats, const float* opacities, const float* shs,
                                          const float* cov3d_precomp, const float* colors_precomp, float* splats,
                                          int32_t* radii, float* cov3d, uint32_t* block_sums, void* order,
-                                         size_t order_bytes, void* stream)
+                                         size_t order_bytes, float* view_copy, void* stream)
 {
     if(n > 0 && !order)
         return DSX_ERR_BAD_ARG;
     int rc = project_fwd_checked(cam, n, means3d, scales, quats, opacities, shs, cov3d_precomp, colors_precomp,
-                                 splats, radii, cov3d, block_sums, order, order_bytes, stream, true);
+                                 splats, radii, cov3d, block_sums, order, order_bytes, stream, true, view_copy);
     if(rc || n == 0)
         return rc;
     // The pair counts are sums over the rectangles: the kernel that counts the tiles, first thing beside the
@@ -640,7 +640,7 @@ extern "C" int dsx_forward_project(const dsx_camera* cam, int64_t n, const float
         return DSX_ERR_BAD_ARG;
     num_keys[0] = num_keys[1] = 0;
     if(int rc = dsx_forward_project_begin(cam, n, means3d, scales, quats, opacities, shs, cov3d_precomp, colors_precomp,
-                                          splats, radii, cov3d, block_sums, order, order_bytes, stream))
+                                          splats, radii, cov3d, block_sums, order, order_bytes, nullptr, stream))
         return rc;
     return dsx_forward_project_counts(cam, n, num_keys, stream);
 }
@@ -656,7 +656,7 @@ extern "C" int dsx_forward_finish(const dsx_camera* cam, int64_t n, int64_t k, c
     if(rc)
         return rc;
     const uint32_t *depth_flag = nullptr, *partition_flag = nullptr;
-    rc = dsx_sort_flags(n, k, cam->image_width, cam->image_height, cam->list_bin, order, workspace, &depth_flag,
+    rc = dsx_sort_flags(n, k, cam->image_width, cam->image_height, camera_bin(*cam), order, workspace, &depth_flag,
                         &partition_flag);
     if(rc)
         return rc;
@@ -728,8 +728,6 @@ extern "C" int dsx_forward_core(const float* means3d, const float* shs, const fl
     cam.campos = campos;
     cam.bg = campos; // unused by the forward
     cam.list_bin = 0;
-    cam.view_transposed = cam.proj_transposed = cam.planar = 0;
-    cam.view_copy = nullptr;
     if(int rc = check_camera(&cam))
         return rc;
     if(n < 0 || !image)

@@ -1043,7 +1043,7 @@ int launch_blend_fwd(const dsx_camera& cam, int64_t n, int64_t k, int32_t* range
 #define DSX_LAUNCH_FWD(KERNEL, THREADS)                                                                          \
     hipLaunchKernelGGL((KERNEL), grid, dim3(THREADS), 0, stream, ranges, sorted_ids, sp, image, final_T, final_idx,  \
                        cam.image_width, cam.image_height, ntx, last_id, (int)k, header, lg.shift, sort_flag_a,     \
-                       sort_flag_b, prep, prep_count, prep_marks, cam.bg, cam.planar, L)
+                       sort_flag_b, prep, prep_count, prep_marks, cam.bg, camera_flag(cam, DSX_PLANAR_IMAGE), L)
         if(four && lg.shift)
             DSX_LAUNCH_FWD(blend_fwd_kernel<true>, DSX_WAVE);
         else if(four)
@@ -1722,7 +1722,7 @@ int launch_blend_bwd(const dsx_camera& cam, int64_t n, int64_t k, const int32_t*
 #define DSX_LAUNCH_BWD(KERNEL, THREADS)                                                                          \
     hipLaunchKernelGGL((KERNEL), grid, dim3(THREADS), 0, stream, ranges, sorted_ids, sp, final_T, final_idx, v_image, \
                        cam.bg, grads, with_marks ? grad_marks(grads, n) : nullptr, cam.image_width,                 \
-                       cam.image_height, ntx, last_id, (int)k, header, lg.shift, cam.planar, L, Z)
+                       cam.image_height, ntx, last_id, (int)k, header, lg.shift, camera_flag(cam, DSX_PLANAR_IMAGE), L, Z)
         if(four && lg.shift)
             DSX_LAUNCH_BWD(blend_bwd_kernel<true>, DSX_WAVE);
         else if(four)

@@ -221,9 +221,18 @@ struct ListGrid
 };
 // list_bin: 0: choose by image size; 1, 2, 4, 8: bins of that many tiles a side (dsx_camera::list_bin)
 ListGrid list_grid(int image_width, int image_height, int list_bin);
+constexpr int kCameraFlags = DSX_VIEW_BY_COLUMNS | DSX_PROJ_BY_COLUMNS | DSX_PLANAR_IMAGE;
+inline int camera_bin(const dsx_camera& cam)
+{
+    return cam.list_bin & ~kCameraFlags;
+}
+inline int camera_flag(const dsx_camera& cam, int flag)
+{
+    return cam.list_bin & flag ? 1 : 0;
+}
 inline ListGrid list_grid(const dsx_camera& cam)
 {
-    return list_grid(cam.image_width, cam.image_height, cam.list_bin);
+    return list_grid(cam.image_width, cam.image_height, camera_bin(cam));
 }
 inline bool valid_list_bin(int b)
 {
@@ -337,8 +346,8 @@ int launch_project_fwd(const dsx_camera& cam, int64_t n, const float* means3d, c
                        const float* quats, const float* opacities, const float* shs,
                        const float* cov3d_precomp, const float* colors_precomp, float* splats,
                        int32_t* radii, float* cov3d, uint32_t* block_sums, uint32_t* depth_keys,
-                       uint2* rects, uint2* key_ranges, hipStream_t stream, uint32_t* clear = nullptr,
-                       int64_t clear_words = 0);
+                       uint2* rects, uint2* key_ranges, float* view_copy, hipStream_t stream,
+                       uint32_t* clear = nullptr, int64_t clear_words = 0);
 int launch_scan_u32(int64_t count, uint32_t* data, uint32_t* total, hipStream_t stream);
 int launch_emit_keys(const dsx_camera& cam, int64_t n, int64_t k, const float* splats,
                      const uint32_t* block_offsets, int64_t* keys, int32_t* values,

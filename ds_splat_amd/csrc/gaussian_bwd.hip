@@ -531,7 +531,7 @@ int launch_gaussian_bwd(const dsx_camera& cam, int64_t n, int num_bases, const f
     p.grads = reinterpret_cast<const float4*>(grads);
     p.marks = with_marks ? grad_marks(const_cast<float*>(grads), n) : nullptr;
     p.view = cam.view;
-    p.view_transposed = cam.view_transposed;
+    p.view_transposed = camera_flag(cam, DSX_VIEW_BY_COLUMNS);
     p.campos = cam.campos;
     p.v_mean3d = v_mean3d;
     p.v_means2d = v_means2d;

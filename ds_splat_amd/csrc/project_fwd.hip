@@ -423,7 +423,7 @@ int launch_project_fwd(const dsx_camera& cam, int64_t n, const float* means3d, c
                        const float* quats, const float* opacities, const float* shs,
                        const float* cov3d_precomp, const float* colors_precomp, float* splats, int32_t* radii,
                        float* cov3d, uint32_t* block_sums, uint32_t* depth_keys, uint2* rects,
-                       uint2* key_ranges, hipStream_t stream,
+                       uint2* key_ranges, float* view_copy, hipStream_t stream,
                        uint32_t* clear, int64_t clear_words)
 {
     if(n == 0)
@@ -441,9 +441,9 @@ int launch_project_fwd(const dsx_camera& cam, int64_t n, const float* means3d, c
     p.colors_precomp = colors_precomp;
     p.view = cam.view;
     p.proj = cam.proj;
-    p.view_transposed = cam.view_transposed;
-    p.proj_transposed = cam.proj_transposed;
-    p.view_copy = cam.view_copy;
+    p.view_transposed = camera_flag(cam, DSX_VIEW_BY_COLUMNS);
+    p.proj_transposed = camera_flag(cam, DSX_PROJ_BY_COLUMNS);
+    p.view_copy = view_copy;
     p.campos = cam.campos;
     p.splats = reinterpret_cast<float4*>(splats);
     p.radii = radii;

@@ -1570,7 +1570,7 @@ static CountsJobs counts_jobs(const ListGrid& lg, char* base, const OrderLayout&
 void depth_order_clear_region(const dsx_camera& cam, int64_t n, void* order, uint32_t** words, int64_t* count)
 {
     // the sort's histograms, counters and look-back statuses and, right behind them, the corner grid
-    const OrderLayout o = order_layout(n, cam.image_width, cam.image_height, cam.list_bin);
+    const OrderLayout o = order_layout(n, cam.image_width, cam.image_height, camera_bin(cam));
     const Sort32Workspace w = sort32_workspace(n, 32, sort32_tile_keys(n));
     *words = reinterpret_cast<uint32_t*>(static_cast<char*>(order) + o.sort + w.hist);
     *count = (int64_t)((w.bytes + (o.ranges - o.cover)) / 4);
@@ -1643,7 +1643,7 @@ int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_
 {
     if(n <= 0)
         return DSX_OK;
-    const OrderLayout o = order_layout(n, cam.image_width, cam.image_height, cam.list_bin);
+    const OrderLayout o = order_layout(n, cam.image_width, cam.image_height, camera_bin(cam));
     char* base = static_cast<char*>(order);
     uint32_t* keys_a = reinterpret_cast<uint32_t*>(base + o.depth_keys);
     uint32_t* keys_b = reinterpret_cast<uint32_t*>(base + o.keys_alt);
@@ -2035,7 +2035,7 @@ template <typename SlotT, bool kMasks>
 static int tile_lists_impl(const dsx_camera& cam, int64_t n, int64_t k, int num_tiles, const void* order,
                            int32_t* sorted_ids, int32_t* ranges, void* workspace, hipStream_t stream)
 {
-    const OrderLayout o = order_layout(n, cam.image_width, cam.image_height, cam.list_bin);
+    const OrderLayout o = order_layout(n, cam.image_width, cam.image_height, camera_bin(cam));
     const char* obase = static_cast<const char*>(order);
     const ListGrid lg = list_grid(cam);
     const RangesLayout rl = ranges_layout(lg);

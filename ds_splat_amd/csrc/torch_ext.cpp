@@ -65,21 +65,23 @@ struct Camera
 {
     at::Tensor view, proj, campos, bg; // float32, on the device: kept alive for the call
     dsx_camera c;
+    int32_t bin;  // of c.list_bin, without the flags
+    bool planar;
 };
 
 // A matrix as the library takes it: 16 floats and whether they go by columns.  What the user holds is the
 // transpose; a tensor that is itself the transposed view of a contiguous one needs no copy either.
-at::Tensor matrix_of(const at::Tensor& t, const at::Device& dev, int32_t& transposed)
+at::Tensor matrix_of(const at::Tensor& t, const at::Device& dev, bool& by_columns)
 {
     at::Tensor m = t.to(dev, at::kFloat);
     require(m.numel() == 16, "camera tensors must be 4x4, 4x4, [3], [3]");
     const bool square = m.dim() == 2 && m.size(0) == 4;
     if(square && m.is_contiguous())
     {
-        transposed = 1;
+        by_columns = true;
         return m;
     }
-    transposed = 0;
+    by_columns = false;
     if(square && m.stride(0) == 1 && m.stride(1) == 4)
         return m;
     return m.t().contiguous(); // (any other shape: what the reference's transposition makes of it, or its error)
@@ -90,13 +92,12 @@ at::Tensor matrix_of(const at::Tensor& t, const at::Device& dev, int32_t& transp
 Camera make_camera(const Settings& s, const at::Device& dev, const float* kept_view = nullptr)
 {
     Camera cam;
+    bool view_by_columns = false, proj_by_columns = false;
     if(kept_view == nullptr)
     {
-        cam.view = matrix_of(s.view, dev, cam.c.view_transposed);
-        cam.proj = matrix_of(s.proj, dev, cam.c.proj_transposed);
+        cam.view = matrix_of(s.view, dev, view_by_columns);
+        cam.proj = matrix_of(s.proj, dev, proj_by_columns);
     }
-    else
-        cam.c.view_transposed = cam.c.proj_transposed = 0;
     cam.campos = s.campos.to(dev, at::kFloat).contiguous();
     cam.bg = s.bg.to(dev, at::kFloat).contiguous();
     require(cam.campos.numel() >= 3 && cam.bg.numel() >= 3 && !(s.planar && cam.bg.numel() != 3),
@@ -110,13 +111,14 @@ Camera make_camera(const Settings& s, const at::Device& dev, const float* kept_v
     cam.c.max_sh_degree = (int32_t)s.max_sh_degree;
     cam.c.view = kept_view ? kept_view : cam.view.data_ptr<float>();
     cam.c.proj = kept_view ? kept_view : cam.proj.data_ptr<float>();
-    cam.c.view_copy = nullptr;
     cam.c.campos = cam.campos.data_ptr<float>();
     cam.c.bg = cam.bg.data_ptr<float>();
     require(s.list_bin == 0 || s.list_bin == 1 || s.list_bin == 2 || s.list_bin == 4 || s.list_bin == 8,
             "list_bin must be 0 (the library's choice), 1, 2, 4 or 8 tiles a side");
-    cam.c.list_bin = (int32_t)s.list_bin;
-    cam.c.planar = s.planar ? 1 : 0;
+    cam.c.list_bin = (int32_t)s.list_bin | (view_by_columns ? DSX_VIEW_BY_COLUMNS : 0) |
+                     (proj_by_columns ? DSX_PROJ_BY_COLUMNS : 0) | (s.planar ? DSX_PLANAR_IMAGE : 0);
+    cam.bin = (int32_t)s.list_bin;
+    cam.planar = s.planar;
     return cam;
 }
 
@@ -202,11 +204,11 @@ struct Rendered
     int64_t k = 0;
 };
 
-Rendered render(Camera cam, const Inputs& in, bool prepare_backward)
+Rendered render(const Camera& cam, const Inputs& in, bool prepare_backward)
 {
     const at::Device dev = in.means3d.device();
     const int64_t n = in.means3d.numel() / 3;
-    const int32_t W = cam.c.image_width, H = cam.c.image_height, bin = cam.c.list_bin;
+    const int32_t W = cam.c.image_width, H = cam.c.image_height, bin = cam.bin;
     const auto f32 = at::TensorOptions().dtype(at::kFloat).device(dev);
     const auto i32 = at::TensorOptions().dtype(at::kInt).device(dev);
     const auto u8 = at::TensorOptions().dtype(at::kByte).device(dev);
@@ -214,7 +216,6 @@ Rendered render(Camera cam, const Inputs& in, bool prepare_backward)
 
     Rendered r;
     r.splats = at::empty({n + kViewRecords, DSX_SPLAT_FLOATS}, f32);
-    cam.c.view_copy = prepare_backward ? r.splats.data_ptr<float>() + n * DSX_SPLAT_FLOATS : nullptr;
     r.radii = at::empty({n}, i32);
     // scratch of the first half: the projection's block sums and, behind them, the depth order
     const size_t sums_bytes = ((size_t)std::max<int64_t>(dsx_num_blocks(n), 1) * 4 + 255) & ~(size_t)255;
@@ -225,10 +226,11 @@ Rendered render(Camera cam, const Inputs& in, bool prepare_backward)
     check(dsx_forward_project_begin(&cam.c, n, in.means3d.data_ptr<float>(), fptr(in.scales), fptr(in.quats),
                                     in.opacities.data_ptr<float>(), fptr(in.shs), fptr(in.cov3d), fptr(in.colors),
                                     r.splats.data_ptr<float>(), r.radii.data_ptr<int32_t>(), nullptr, bs, order,
-                                    order_bytes, s));
+                                    order_bytes,
+                                    prepare_backward ? r.splats.data_ptr<float>() + n * DSX_SPLAT_FLOATS : nullptr, s));
     // (while the device counts the pairs: everything whose size does not depend on their number)
     r.ranges = at::empty({dsx_ranges_count(W, H, bin)}, i32);
-    r.image = cam.c.planar ? at::empty({3, H, W}, f32) : at::empty({H, W, 3}, f32);
+    r.image = cam.planar ? at::empty({3, H, W}, f32) : at::empty({H, W, 3}, f32);
     r.final_T = at::empty({H, W}, f32);
     r.final_idx = at::empty({H, W}, i32);
     if(prepare_backward && n > 0)

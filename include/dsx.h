@@ -70,14 +70,14 @@ typedef struct dsx_camera
     const float* proj;      /* device float[16], row-major world->clip              */
     const float* campos;    /* device float[3]                                      */
     const float* bg;        /* device float[3]                                      */
-    int32_t list_bin;       /* tiles per side of a list's bin: 0 (automatic), 1, 2, 4, 8 */
-    int32_t view_transposed; /* 1: `view` is stored column by column (what the Python API's users hold) */
-    int32_t proj_transposed; /* 1: the same for `proj`                                     */
-    int32_t planar;         /* 0: image and v_image are [H,W,3], the background is not composited;
-                               1: they are [3,H,W] and the image has final_T * bg added    */
-    float* view_copy;       /* device float[16], or null: dsx_forward_project stores `view` there, row by row,
-                               for a backward that runs when the caller's own matrix may be another one    */
+    int32_t list_bin;       /* tiles per side of a list's bin: 0 (automatic), 1, 2, 4, 8; plus DSX_* flags */
 } dsx_camera;
+
+/* May be added to dsx_camera::list_bin (not to the list_bin of the size helpers): */
+#define DSX_VIEW_BY_COLUMNS 0x100 /* `view` is stored column by column (what the Python API's users hold) */
+#define DSX_PROJ_BY_COLUMNS 0x200 /* the same for `proj`                                                  */
+#define DSX_PLANAR_IMAGE 0x400    /* image and v_image are [3,H,W] and the image has final_T * bg added;
+                                     without: [H,W,3], the background is not composited                   */
 
 /*
  * Projected record ("splat"), one per Gaussian, DSX_SPLAT_FLOATS floats:
@@ -96,8 +96,8 @@ typedef struct dsx_camera
  */
 
 const char* dsx_error_string(int status);
-/* 100 * major + minor.  310: dsx_camera has view_transposed, proj_transposed, planar and view_copy (0: as before), the
- * projection's wait for the pair counts is a function of its own.  300: the bin size of the tile lists is an argument (dsx_camera::list_bin and
+/* 100 * major + minor.  310: flags beside dsx_camera::list_bin, the projection's wait for the pair
+ * counts is a function of its own.  300: the bin size of the tile lists is an argument (dsx_camera::list_bin and
  * the size helpers) instead of a process-wide setting; the `ranges` buffer carries it in a header word;
  * the blend entry points and the backward are told n and k and follow no id or list position beyond
  * them; dsx_forward_project returns both pair counts.  (200 had dsx_set_list_bin.) */
@@ -293,13 +293,15 @@ int dsx_forward_project(const dsx_camera* cam, int64_t n, const float* means3d,
                         float* splats, int32_t* radii, float* cov3d, uint32_t* block_sums,
                         void* order, size_t order_bytes, int64_t* num_keys /* host */,
                         void* stream);
-/* The same in two halves, for a caller that has something to do (allocations) while the device counts: everything up
- * to the wait, and the wait for the pair counts of the calling thread's last dsx_forward_project_begin. */
+/* The same in two halves, for a caller that has something to do (allocations) while the device sorts: everything up
+ * to the wait, and the wait for the pair counts of the calling thread's last dsx_forward_project_begin.
+ * view_copy: device float[16] that receives `view`, row by row, for a backward that runs when the caller's own matrix
+ * may be another one (null: none). */
 int dsx_forward_project_begin(const dsx_camera* cam, int64_t n, const float* means3d,
                         const float* scales, const float* quats, const float* opacities,
                         const float* shs, const float* cov3d_precomp, const float* colors_precomp,
                         float* splats, int32_t* radii, float* cov3d, uint32_t* block_sums,
-                        void* order, size_t order_bytes, void* stream);
+                        void* order, size_t order_bytes, float* view_copy, void* stream);
 int dsx_forward_project_counts(const dsx_camera* cam, int64_t n, int64_t* num_keys /* host */, void* stream);
 
 /* Second half: tile lists (dsx_tile_lists) and blend.  sorted_ids[k] and ranges[T+1] are

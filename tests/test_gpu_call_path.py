@@ -152,7 +152,8 @@ def test_counts_belong_to_the_call_that_waits_for_them():
                 torch.empty(int(lib.dsx_num_blocks(n)), dtype=torch.int32, device=DEV)]
         kept.append((cam, t, order, bufs))
         N.check(lib.dsx_forward_project_begin(cam.ref, n, *map(ptr, t), ptr(None), ptr(None), ptr(bufs[0]),
-                                              ptr(bufs[1]), ptr(None), ptr(bufs[2]), ptr(order), order.numel(), stream))
+                                              ptr(bufs[1]), ptr(None), ptr(bufs[2]), ptr(order), order.numel(),
+                                              ptr(None), stream))
         return cam
 
     def counts(cam, n):
