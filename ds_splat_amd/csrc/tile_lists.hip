@@ -112,7 +112,9 @@ __device__ __forceinline__ uint64_t match_digit(uint32_t d, int bits)
 // it wants many wavefronts per CU, while every further workgroup adds a flush of up to 1024
 // contended global atomics (256 threads: 0.029 ms, 1024 threads: 0.020 ms at 3 M keys)
 constexpr int kHist32Threads = 1024;
-constexpr int kHist32Items = 8;
+// (keys of a thread: few, so that small inputs are spread over many workgroups; 100 K keys with eight 12 us, with two 6)
+constexpr int kHist32Items = 2;
+constexpr int kDepthHistItems = 4;
 
 template <typename KeyT>
 __global__ __launch_bounds__(kHist32Threads) void hist32_kernel(const KeyT* __restrict__ keys, int64_t count,
@@ -715,20 +717,20 @@ __global__ __launch_bounds__(kHist32Threads) void depth_hist_kernel(const uint32
     const DepthRange range = depth_range(lowest, highest);
     const int bins = range.narrow ? kDepthBins : kBins32;
     uint32_t none = 0; // keys without pairs: counted by their thread, added to their bins at the end
-    const int64_t chunk = (int64_t)kHist32Threads * kHist32Items, chunks = (count + chunk - 1) / chunk;
+    const int64_t chunk = (int64_t)kHist32Threads * kDepthHistItems, chunks = (count + chunk - 1) / chunk;
     for(int64_t c = blockIdx.x; c < chunks; c += gridDim.x)
     {
-        uint32_t key[kHist32Items];
-        bool valid[kHist32Items];
+        uint32_t key[kDepthHistItems];
+        bool valid[kDepthHistItems];
 #pragma unroll
-        for(int it = 0; it < kHist32Items; ++it)
+        for(int it = 0; it < kDepthHistItems; ++it)
         {
             const int64_t i = c * chunk + it * kHist32Threads + tid;
             valid[it] = i < count;
             key[it] = valid[it] ? __builtin_nontemporal_load(keys + i) : 0u;
         }
 #pragma unroll
-        for(int it = 0; it < kHist32Items; ++it)
+        for(int it = 0; it < kDepthHistItems; ++it)
         {
             if(valid[it] && key[it] == kNoPairsKey)
             {
@@ -1592,7 +1594,7 @@ static int launch_depth_sort(int64_t n, char* base, const OrderLayout& o, int64_
     uint32_t* const packed_b = reinterpret_cast<uint32_t*>(base + o.rects32);
     char* const ws = base + o.sort;
     const Sort32Workspace w = sort32_workspace(n, 32, sort32_tile_keys(n));
-    const int64_t chunks = (n + kHist32Threads * kHist32Items - 1) / (kHist32Threads * kHist32Items);
+    const int64_t chunks = (n + kHist32Threads * kDepthHistItems - 1) / (kHist32Threads * kDepthHistItems);
     {
         DSX_TIMED("depth_hist_kernel", stream);
         hipLaunchKernelGGL(depth_hist_kernel, dim3((unsigned)min((int64_t)DSX_HIST_BLOCKS, chunks)), dim3(kHist32Threads), 0,
