@@ -55,7 +55,8 @@ struct StagedOpacity
 {
     float log2;  // log2(opacity)
     // largest sigma with alpha >= 1/255, about ln(255 opacity): the test of alpha is taken on sigma, before
-    // the exponential and with the same bits in both directions
+    // the exponential and with the same bits in both directions.  -infinity for an opacity that no pixel takes,
+    // whose entry is then not even staged; infinity for an infinite one
     float reach;
 };
 // The reach is found as the last float for which opacity * exp2(-sigma log2(e)), evaluated just so, passes: an
@@ -75,6 +76,8 @@ __device__ __forceinline__ StagedOpacity stage_opacity(float opacity)
     for(int step = 4; step > 0; step >>= 1)
         bits += alpha_at(__int_as_float(bits + step)) >= 1.0f / 255.0f ? step : 0;
     s.reach = s.reach > 1e-3f ? __int_as_float(bits) : s.reach;
+    // (masked and pruned Gaussians: zero, denormal and negative opacities have no logarithm to start from)
+    s.reach = opacity < 1.0f / 255.0f ? -__builtin_inff() : (opacity == __builtin_inff() ? opacity : s.reach);
     return s;
 }
 // log2(opacity / mul) as near as a float comes to it: the hardware's logarithm and the difference of two make 1.5 units
@@ -1151,7 +1154,8 @@ __device__ __forceinline__ void moments_to_gradients(double* m, const float4 A, 
     m[2] = -0.5 * wxx;
     m[3] = -wxy;
     m[4] = -0.5 * wyy;
-    m[5] = w * (double)__builtin_amdgcn_exp2f(-B.y); // v_opacity: what w holds as the opacity's factor taken out
+    // v_opacity: what w holds as the opacity's factor taken out (an entry without a pixel has no factor to take)
+    m[5] = w != 0.0 ? w * (double)__builtin_amdgcn_exp2f(-B.y) : 0.0;
 }
 // One set of hardware float atomics per entry and round, and none where no pixel was valid
 __device__ __forceinline__ void flush_sums(const double* sums, const int* ids, int staged, float* grads, uint8_t* marks,
