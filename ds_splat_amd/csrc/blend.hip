@@ -40,56 +40,36 @@ __device__ __forceinline__ ExponentX exponent_x(float a_half, float b, float dx)
     return r;
 }
 
-// alpha = opacity exp(-sigma) through the hardware base-2 exponential (the reference is built with
-// fast-math), with the opacity as a term of its argument: one fused multiply-add instead of a product
-// before and a product after it.  log2(e) stays a factor of the finished exponent: folded into the
-// conic when an entry is staged it would put one more rounding on every term of the quadratic form, and
-// where the terms are large and cancel (thin, long splats far from their centre) the image would move
-// 1.6 times as far from the reference's as it does.
+// alpha = opacity exp(-sigma) through the hardware base-2 exponential (the reference is built with fast-math), the
+// opacity as a factor of it: as a term of the exponential's argument (one instruction less for each pixel and entry)
+// a faint splat's alpha would be off by up to 1.7e-7 of itself, three to four times as much as it is.  log2(e) stays a
+// factor of the finished exponent: folded into the conic when an entry is staged it would put one more rounding on
+// every term of the quadratic form, and where the terms are large and cancel (thin, long splats far from their centre)
+// the image would move 1.6 times as far from the reference's as it does.
 constexpr float kLog2E = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 constexpr float kLog2Of255 = 7.994353436858858f;
 
-// What an entry's opacity is staged as.
-struct StagedOpacity
-{
-    float log2;  // log2(opacity)
-    // largest sigma with alpha >= 1/255, about ln(255 opacity): the test of alpha is taken on sigma, before
-    // the exponential and with the same bits in both directions.  -infinity for an opacity that no pixel takes,
-    // whose entry is then not even staged; infinity for an infinite one
-    float reach;
-};
+// Largest sigma with alpha >= 1/255, about ln(255 opacity): the test of alpha is taken on sigma, before the
+// exponential and with the same bits in both directions.  -infinity for an opacity that no pixel takes, whose entry is
+// then not even staged; infinity for an infinite one; NaN for a NaN.
 // The reach is found as the last float for which opacity * exp2(-sigma log2(e)), evaluated just so, passes: an
 // estimate from the logarithm, one Newton step on that expression, and a bisection of the eight floats around
 // it.  (The logarithm's own rounding alone would move the line between in and out by two or three floats, and with
 // it a few hundred of the 10^9 decisions of a large scene.)
-__device__ __forceinline__ StagedOpacity stage_opacity(float opacity)
+__device__ __forceinline__ float reach_of(float opacity)
 {
 #pragma clang fp contract(off)
-    StagedOpacity s;
-    s.log2 = __builtin_amdgcn_logf(opacity);
-    s.reach = (s.log2 + kLog2Of255) * kLn2; // NaN for a negative opacity, and for a NaN
+    float reach = (__builtin_amdgcn_logf(opacity) + kLog2Of255) * kLn2;
     auto alpha_at = [&](float sigma) { return opacity * __builtin_amdgcn_exp2f(-sigma * kLog2E); };
-    s.reach += __builtin_fmaf(alpha_at(s.reach), 255.0f, -1.0f);
-    int bits = __float_as_int(s.reach) - 4;
+    reach += __builtin_fmaf(alpha_at(reach), 255.0f, -1.0f);
+    int bits = __float_as_int(reach) - 4;
 #pragma unroll
     for(int step = 4; step > 0; step >>= 1)
         bits += alpha_at(__int_as_float(bits + step)) >= 1.0f / 255.0f ? step : 0;
-    s.reach = s.reach > 1e-3f ? __int_as_float(bits) : s.reach;
+    reach = reach > 1e-3f ? __int_as_float(bits) : reach;
     // (masked and pruned Gaussians: zero, denormal and negative opacities have no logarithm to start from)
-    s.reach = opacity < 1.0f / 255.0f ? -__builtin_inff() : (opacity == __builtin_inff() ? opacity : s.reach);
-    return s;
-}
-// log2(opacity / mul) as near as a float comes to it: the hardware's logarithm and the difference of two make 1.5 units
-// in the last place, which for a faint splat is three times what its alpha may be off by otherwise.  One Newton step on
-// the exponential that the value is for (left out where it has no meaning: opacities of zero, infinity, NaN).
-// Root mean square distance of images from a 64-bit evaluation of the same records, faint (opacity 0.035) and ordinary
-// splats: 1.05e-7 and 1.16e-7, as with the product of opacity and exponential; without the step 1.11e-7.
-__device__ __forceinline__ float staged_log2(float log2, float opacity, float mul)
-{
-#pragma clang fp contract(off)
-    const float off = __builtin_fmaf(-mul, __builtin_amdgcn_exp2f(log2), opacity) * __builtin_amdgcn_rcpf(opacity);
-    return fabsf(off) < 1e-3f ? __builtin_fmaf(off, kLog2E, log2) : log2;
+    return opacity < 1.0f / 255.0f ? -__builtin_inff() : (opacity == __builtin_inff() ? opacity : reach);
 }
 // Both tests of an entry at a pixel, that sigma has the right sign and that it does not exceed the reach,
 // in one integer compare: the bits of floats of one sign are ordered like their magnitudes.
@@ -352,7 +332,6 @@ __device__ __forceinline__ void prepare_grads_share(const float4* splats, float4
 // as many wavefronts, whose smaller blocks also leave each row fewer entries to walk.
 constexpr int kPix = 4; // pixels per lane of the wavefront forms
 constexpr float kAlphaMax = 0.999f;       // the forward's clamp (the backward's is 0.99)
-constexpr float kLog2AlphaMax = -0.0014434168696687186f; // its base-2 logarithm
 constexpr int kFwdBatch = 96; // staged entries of a round: 5 KB of LDS, 32 wavefronts per compute unit
 constexpr int kScanGroups = 4; // groups of 64 positions of a bin's list whose loads are in flight together
 
@@ -401,8 +380,8 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(8, 8))
 {
     // the last place is nobody's entry (no exponent passes): rows whose list has ended point at it
     __shared__ float4 s_a[kFwdBatch + 1]; // pixel x, pixel y, conic -a/2, conic b
-    __shared__ float4 s_b[kFwdBatch + 1]; // conic c/2, log2(opacity / 0.999), limit of the exponent's bits, index in the sorted key array
-    __shared__ float s_c[3 * kFwdBatch + 4]; // red, green, blue, times 0.999 (the weights are alpha / 0.999)
+    __shared__ float4 s_b[kFwdBatch + 1]; // conic c/2, opacity, limit of the exponent's bits, index in the sorted key array
+    __shared__ float s_c[3 * kFwdBatch + 4]; // red, green, blue
     __shared__ uint64_t s_list[4 * kFwdBatch / 8 + 1]; // a byte per entry and row: its place (one word more than is used: read ahead)
     __shared__ int s_queue[DSX_WAVE]; // ids of the tile's own entries, on their way from the scan to the gather
     static_assert(kFwdBatch % 8 == 0 && kFwdBatch < 256 && kFwdBatch >= DSX_WAVE, "places are bytes, stored by words");
@@ -545,15 +524,15 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(8, 8))
             }
             uint32_t reached = 0;
             float4 q0, q1;
-            StagedOpacity op;
+            float reach = 0.0f;
             const float4* const rec = splats + 3 * (int64_t)min((uint32_t)id, last_id);
             if(lane < batch)
             {
                 // (an id is taken for what it is only up to the last Gaussian: lists that a failed sort or a
                 // caller's mix-up left in disorder then give a wrong image, not a fetch outside the records)
                 q0 = rec[0], q1 = rec[1];
-                op = stage_opacity(q1.w);
-                reached = live_rows & blocks_reached<Pixels<kPix>::kSide>(q0.x, q0.y, q1.x, q1.y, q1.z, op.reach,
+                reach = reach_of(q1.w);
+                reached = live_rows & blocks_reached<Pixels<kPix>::kSide>(q0.x, q0.y, q1.x, q1.y, q1.z, reach,
                                                                              px.box_x, px.box_y);
             }
             const uint64_t m_any = __ballot(reached != 0);
@@ -562,12 +541,12 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(8, 8))
             {
                 const float4 q2 = rec[2];
                 s_a[place] = make_float4(q0.x, q0.y, q1.x * -0.5f, q1.y);
-                s_b[place] = make_float4(q1.z * 0.5f, q1.w == q1.w ? staged_log2(op.log2 - kLog2AlphaMax, q1.w, kAlphaMax) : __builtin_inff(),
-                                         __int_as_float(reach_limit_fwd(q1.w, op.reach)),
+                s_b[place] = make_float4(q1.z * 0.5f, q1.w,
+                                         __int_as_float(reach_limit_fwd(q1.w, reach)),
                                          __int_as_float(index_next + lane));
-                s_c[3 * place] = kAlphaMax * q2.x;
-                s_c[3 * place + 1] = kAlphaMax * q2.y;
-                s_c[3 * place + 2] = kAlphaMax * q2.z;
+                s_c[3 * place] = q2.x;
+                s_c[3 * place + 1] = q2.y;
+                s_c[3 * place + 2] = q2.z;
             }
 #pragma unroll
             for(int r = 0; r < 4; ++r)
@@ -610,10 +589,11 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(8, 8))
                 // the decisions as wavefront masks (each is its compare's own result register),
                 // combined on the scalar unit and handed back to the lanes as conditions
                 m_pass[p] = __builtin_amdgcn_ballot_w64(__float_as_int(power) <= limit);
-                // alpha / 0.999, at most 1 (the clamp is a modifier of the exponential's result)
-                const float e = __builtin_amdgcn_fmed3f(__builtin_amdgcn_exp2f(__builtin_fmaf(power, kLog2E, B.y)), 0.0f, 1.0f);
-                weight[p] = (__builtin_amdgcn_inverse_ballot_w64(m_pass[p]) ? e : 0.0f) * T[p];
-                Tn[p] = __builtin_fmaf(-kAlphaMax, weight[p], T[p]); // (1 - alpha) T
+                // (a NaN opacity gives 0.999, as in the reference: fminf drops the NaN)
+                const float alpha = fminf(kAlphaMax, B.y * __builtin_amdgcn_exp2f(power * kLog2E));
+                const float taken = __builtin_amdgcn_inverse_ballot_w64(m_pass[p]) ? alpha : 0.0f;
+                weight[p] = taken * T[p];
+                Tn[p] = __builtin_fmaf(-taken, T[p], T[p]); // (1 - alpha) T in one rounding
                 m_low[p] = __builtin_amdgcn_ballot_w64(Tn[p] < 0.0001f);
                 m_stop |= m_low[p];
             }
@@ -899,15 +879,15 @@ __global__ __launch_bounds__(kTileThreads) void blend_fwd_tile_kernel(const int3
         }
         uint32_t reached = 0;
         float4 q0, q1, q2;
-        StagedOpacity op;
+        float reach = 0.0f;
         if(tid < batch)
         {
             const float4* const rec = splats + 3 * (int64_t)min((uint32_t)id, last_id);
             q0 = rec[0], q1 = rec[1], q2 = rec[2];
-            op = stage_opacity(q1.w);
+            reach = reach_of(q1.w);
 #pragma unroll
             for(int q = 0; q < 4; ++q)
-                reached |= blocks_reached<4>(q0.x, q0.y, q1.x, q1.y, q1.z, op.reach, tile_x + 8.0f * (q & 1), tile_y + 8.0f * (q >> 1)) << (4 * q);
+                reached |= blocks_reached<4>(q0.x, q0.y, q1.x, q1.y, q1.z, reach, tile_x + 8.0f * (q & 1), tile_y + 8.0f * (q >> 1)) << (4 * q);
             reached &= live_blocks;
         }
         int staged;
@@ -915,11 +895,11 @@ __global__ __launch_bounds__(kTileThreads) void blend_fwd_tile_kernel(const int3
         if(reached != 0)
         {
             s_a[place] = make_float4(q0.x, q0.y, q1.x * -0.5f, q1.y);
-            s_b[place] = make_float4(q1.z * 0.5f, q1.w == q1.w ? staged_log2(op.log2 - kLog2AlphaMax, q1.w, kAlphaMax) : __builtin_inff(),
-                                     __int_as_float(reach_limit_fwd(q1.w, op.reach)), __int_as_float(index_next + tid));
-            s_c[3 * place] = kAlphaMax * q2.x;
-            s_c[3 * place + 1] = kAlphaMax * q2.y;
-            s_c[3 * place + 2] = kAlphaMax * q2.z;
+            s_b[place] = make_float4(q1.z * 0.5f, q1.w,
+                                     __int_as_float(reach_limit_fwd(q1.w, reach)), __int_as_float(index_next + tid));
+            s_c[3 * place] = q2.x;
+            s_c[3 * place + 1] = q2.y;
+            s_c[3 * place + 2] = q2.z;
             s_reach[place] = (uint16_t)reached;
         }
         index_next += batch;
@@ -933,7 +913,7 @@ __global__ __launch_bounds__(kTileThreads) void blend_fwd_tile_kernel(const int3
         {
             const uint32_t places = my_list[i];
             float4 A[kFwdAtOnce], B[kFwdAtOnce];
-            float channel[kFwdAtOnce], e[kFwdAtOnce], weight[kFwdAtOnce];
+            float channel[kFwdAtOnce], alpha[kFwdAtOnce], weight[kFwdAtOnce];
             uint64_t m_pass[kFwdAtOnce];
 #pragma unroll
             for(int u = 0; u < kFwdAtOnce; ++u)
@@ -952,14 +932,14 @@ __global__ __launch_bounds__(kTileThreads) void blend_fwd_tile_kernel(const int3
                 const float dy = pyf - A[u].y;
                 const float power = __builtin_fmaf(-__builtin_fmaf(B[u].x, dy, ex.bx), dy, ex.ax);
                 m_pass[u] = __builtin_amdgcn_ballot_w64(__float_as_int(power) <= __float_as_int(B[u].z));
-                const float full = __builtin_amdgcn_fmed3f(__builtin_amdgcn_exp2f(__builtin_fmaf(power, kLog2E, B[u].y)), 0.0f, 1.0f);
-                e[u] = __builtin_amdgcn_inverse_ballot_w64(m_pass[u]) ? full : 0.0f;
+                const float full = fminf(kAlphaMax, B[u].y * __builtin_amdgcn_exp2f(power * kLog2E));
+                alpha[u] = __builtin_amdgcn_inverse_ballot_w64(m_pass[u]) ? full : 0.0f;
             }
 #pragma unroll
             for(int u = 0; u < kFwdAtOnce; ++u)
             {
-                weight[u] = e[u] * Tn;
-                Tn = __builtin_fmaf(-kAlphaMax, weight[u], Tn);
+                weight[u] = alpha[u] * Tn;
+                Tn = __builtin_fmaf(-alpha[u], Tn, Tn);
             }
             if(__builtin_amdgcn_ballot_w64(Tn < 0.0001f) != 0)
             {
@@ -968,8 +948,9 @@ __global__ __launch_bounds__(kTileThreads) void blend_fwd_tile_kernel(const int3
 #pragma unroll
                 for(int u = 0; u < kFwdAtOnce; ++u)
                 {
-                    weight[u] = (pyf == pyf ? e[u] : 0.0f) * Tn;
-                    const float next = __builtin_fmaf(-kAlphaMax, weight[u], Tn);
+                    const float taken = pyf == pyf ? alpha[u] : 0.0f;
+                    weight[u] = taken * Tn;
+                    const float next = __builtin_fmaf(-taken, Tn, Tn);
                     const uint64_t m_low = __builtin_amdgcn_ballot_w64(next < 0.0001f);
                     const bool stop = __builtin_amdgcn_inverse_ballot_w64(m_low);
                     m_pass[u] &= __builtin_amdgcn_ballot_w64(pyf == pyf) & ~m_low;
@@ -1143,19 +1124,22 @@ __device__ __forceinline__ float row_sum8_scatter(const float (&v)[8], int lane)
 constexpr int kSums = 9;
 constexpr int kBwdBatch = 80; // staged entries of a round: 10 KB of LDS with their sums, 16 wavefronts per compute unit
 
-// An entry's sums in LDS, from the moments of w = -v_sigma over its pixels to the gradients:
-// v_x = sum of v_sigma (a dx + b dy) with d = mean - pixel (v_sigma and d both change sign), ...
+// An entry's sums in LDS, from the moments of w = vis v_alpha over its pixels (vis = exp(-sigma), and v_sigma =
+// -opacity w) to the gradients: v_x = sum of v_sigma (a dx + b dy) with d = mean - pixel (v_sigma and d both change
+// sign), ...; v_opacity is the sum of w itself
 __device__ __forceinline__ void moments_to_gradients(double* m, const float4 A, const float4 B)
 {
     const float half_a = A.z, b = A.w, half_c = B.x;
+    const double opacity = (double)B.y;
+    // (a sum that is zero stays so whatever the opacity: an infinite or NaN one of an entry that no pixel took)
+    auto scaled = [&](double v) { return v != 0.0 ? opacity * v : 0.0; };
     const double w = m[0], wx = m[1], wxx = m[2], wy = m[3], wxy = m[4], wyy = m[5];
-    m[0] = (double)(2.0f * half_a) * wx + (double)b * wy;
-    m[1] = (double)b * wx + (double)(2.0f * half_c) * wy;
-    m[2] = -0.5 * wxx;
-    m[3] = -wxy;
-    m[4] = -0.5 * wyy;
-    // v_opacity: what w holds as the opacity's factor taken out (an entry without a pixel has no factor to take)
-    m[5] = w != 0.0 ? w * (double)__builtin_amdgcn_exp2f(-B.y) : 0.0;
+    m[0] = scaled((double)(2.0f * half_a) * wx + (double)b * wy);
+    m[1] = scaled((double)b * wx + (double)(2.0f * half_c) * wy);
+    m[2] = scaled(-0.5 * wxx);
+    m[3] = scaled(-wxy);
+    m[4] = scaled(-0.5 * wyy);
+    m[5] = w;
 }
 // One set of hardware float atomics per entry and round, and none where no pixel was valid
 __device__ __forceinline__ void flush_sums(const double* sums, const int* ids, int staged, float* grads, uint8_t* marks,
@@ -1193,7 +1177,7 @@ __global__ __launch_bounds__(DSX_WAVE) void blend_bwd_kernel(
 {
     // (the last place: nobody's entry, as in the forward)
     __shared__ float4 s_a[kBwdBatch + 1]; // pixel x, pixel y, conic a/2, conic b
-    __shared__ float4 s_b[kBwdBatch + 1]; // conic c/2, log2(opacity), limit of sigma's bits, index in the sorted key array
+    __shared__ float4 s_b[kBwdBatch + 1]; // conic c/2, opacity, limit of sigma's bits, index in the sorted key array
     __shared__ float s_c[3 * (kBwdBatch + 1)]; // red, green, blue
     __shared__ int s_id[kBwdBatch];
     __shared__ double s_sum[(kBwdBatch + 1) * kSums];
@@ -1366,15 +1350,15 @@ __global__ __launch_bounds__(DSX_WAVE) void blend_bwd_kernel(
             }
             uint32_t reached = 0;
             float4 q0, q1, q2;
-            StagedOpacity op;
+            float reach = 0.0f;
             const int idx = idx_next - lane;
             if(lane < batch)
             {
                 id = (int)min((uint32_t)id, last_id); // (as in the forward)
                 const float4* rec = splats + 3 * (int64_t)id;
                 q0 = rec[0], q1 = rec[1], q2 = rec[2];
-                op = stage_opacity(q1.w);
-                reached = blocks_reached<Pixels<kPix>::kSide>(q0.x, q0.y, q1.x, q1.y, q1.z, op.reach, px.box_x, px.box_y);
+                reach = reach_of(q1.w);
+                reached = blocks_reached<Pixels<kPix>::kSide>(q0.x, q0.y, q1.x, q1.y, q1.z, reach, px.box_x, px.box_y);
 #pragma unroll
                 for(int r = 0; r < 4; ++r)
                     if(idx > m_row[r]) // behind everything that the row's pixels blended
@@ -1385,7 +1369,7 @@ __global__ __launch_bounds__(DSX_WAVE) void blend_bwd_kernel(
             if(reached != 0)
             {
                 s_a[place] = make_float4(q0.x, q0.y, q1.x * 0.5f, q1.y);
-                s_b[place] = make_float4(q1.z * 0.5f, staged_log2(op.log2, q1.w, 1.0f), __uint_as_float(reach_limit_bwd(q1.w, op.reach)),
+                s_b[place] = make_float4(q1.z * 0.5f, q1.w, __uint_as_float(reach_limit_bwd(q1.w, reach)),
                                          __int_as_float(idx));
                 s_c[3 * place] = q2.x;
                 s_c[3 * place + 1] = q2.y;
@@ -1424,7 +1408,7 @@ __global__ __launch_bounds__(DSX_WAVE) void blend_bwd_kernel(
             // sigma exactly as the forward computed it
             const float dx = pxf - A.x;
             const ExponentX ex = exponent_x(A.z, A.w, dx);
-            float raw[kPix], dy[kPix]; // alpha before its clamp; dy = pixel - mean
+            float vis[kPix], alpha[kPix], dy[kPix]; // dy = pixel - mean
             // which lanes' pixel p takes part: wavefront masks (each compare's own result register),
             // combined on the scalar unit
             uint64_t m_valid[kPix];
@@ -1438,29 +1422,29 @@ __global__ __launch_bounds__(DSX_WAVE) void blend_bwd_kernel(
                 m_valid[p] = __builtin_amdgcn_ballot_w64(idx <= bin_final[p]) &
                              __builtin_amdgcn_ballot_w64(__float_as_uint(sigma) <= limit);
                 m_any |= m_valid[p];
-                raw[p] = __builtin_amdgcn_exp2f(__builtin_fmaf(-sigma, kLog2E, B.y));
+                vis[p] = __builtin_amdgcn_exp2f(-sigma * kLog2E);
+                alpha[p] = fminf(0.99f, B.y * vis[p]);
             }
             if(m_any == 0)
                 continue;
             // Per lane, over its pixels (which share dx): the weights of the colour's gradient, and three
-            // moments over dy of w = -v_sigma = raw * v_alpha
+            // moments over dy of w = vis * v_alpha
             float v_red = 0.f, v_green = 0.f, v_blue = 0.f, S0 = 0.f, S1 = 0.f, S2 = 0.f;
 #pragma unroll
             for(int p = 0; p < kPix; ++p)
             {
                 if(__builtin_amdgcn_inverse_ballot_w64(m_valid[p]))
                 {
-                    const float alpha = fminf(0.99f, raw[p]);
-                    const float ra = __builtin_amdgcn_rcpf(1.0f - alpha);
+                    const float ra = __builtin_amdgcn_rcpf(1.0f - alpha[p]);
                     T[p] *= ra;
-                    const float fac = alpha * T[p];
+                    const float fac = alpha[p] * T[p];
                     v_red += fac * vo0[p];
                     v_green += fac * vo1[p];
                     v_blue += fac * vo2[p];
                     const float rv = red * vo0[p] + green * vo1[p] + blue * vo2[p];
                     const float v_alpha = rv * T[p] + bterm[p] * ra;
                     bterm[p] -= rv * fac;
-                    const float w = raw[p] * v_alpha;
+                    const float w = vis[p] * v_alpha;
                     const float wdy = w * dy[p];
                     S0 += w;
                     S1 += wdy;
@@ -1601,17 +1585,17 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
         }
         uint32_t reached = 0;
         float4 q0, q1, q2;
-        StagedOpacity op;
+        float reach = 0.0f;
         const int idx = idx_next - tid;
         if(tid < batch)
         {
             id = (int)min((uint32_t)id, last_id);
             const float4* const rec = splats + 3 * (int64_t)id;
             q0 = rec[0], q1 = rec[1], q2 = rec[2];
-            op = stage_opacity(q1.w);
+            reach = reach_of(q1.w);
 #pragma unroll
             for(int q = 0; q < 4; ++q)
-                reached |= blocks_reached<4>(q0.x, q0.y, q1.x, q1.y, q1.z, op.reach, tile_x + 8.0f * (q & 1), tile_y + 8.0f * (q >> 1)) << (4 * q);
+                reached |= blocks_reached<4>(q0.x, q0.y, q1.x, q1.y, q1.z, reach, tile_x + 8.0f * (q & 1), tile_y + 8.0f * (q >> 1)) << (4 * q);
 #pragma unroll
             for(int b = 0; b < 4 * kTileWaves; ++b)
                 if(idx > s_last[b])
@@ -1625,7 +1609,7 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
         if(reached != 0)
         {
             s_a[place] = make_float4(q0.x, q0.y, q1.x * 0.5f, q1.y);
-            s_b[place] = make_float4(q1.z * 0.5f, staged_log2(op.log2, q1.w, 1.0f), __uint_as_float(reach_limit_bwd(q1.w, op.reach)),
+            s_b[place] = make_float4(q1.z * 0.5f, q1.w, __uint_as_float(reach_limit_bwd(q1.w, reach)),
                                      __int_as_float(idx));
             s_c[3 * place] = q2.x;
             s_c[3 * place + 1] = q2.y;
@@ -1642,7 +1626,7 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
         {
             const uint32_t places = my_list[i];
             float4 A[kBwdAtOnce], B[kBwdAtOnce];
-            float dx[kBwdAtOnce], dy[kBwdAtOnce], raw[kBwdAtOnce], alpha[kBwdAtOnce], ra[kBwdAtOnce], rv[kBwdAtOnce];
+            float dx[kBwdAtOnce], dy[kBwdAtOnce], vis[kBwdAtOnce], alpha[kBwdAtOnce], ra[kBwdAtOnce], rv[kBwdAtOnce];
             double* sums[kBwdAtOnce];
             uint64_t m_valid[kBwdAtOnce];
             uint64_t m_any = 0;
@@ -1666,8 +1650,8 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
                 m_valid[u] = __builtin_amdgcn_ballot_w64(__float_as_int(B[u].w) <= bin_final) &
                              __builtin_amdgcn_ballot_w64(__float_as_uint(sigma) <= __float_as_uint(B[u].z));
                 m_any |= m_valid[u];
-                raw[u] = __builtin_amdgcn_exp2f(__builtin_fmaf(-sigma, kLog2E, B[u].y));
-                alpha[u] = fminf(0.99f, raw[u]);
+                vis[u] = __builtin_amdgcn_exp2f(-sigma * kLog2E);
+                alpha[u] = fminf(0.99f, B[u].y * vis[u]);
                 ra[u] = __builtin_amdgcn_rcpf(1.0f - alpha[u]);
             }
             if(m_any == 0)
@@ -1685,7 +1669,7 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
                     v_blue = fac * vo2;
                     const float v_alpha = rv[u] * T + bterm * ra[u];
                     bterm -= rv[u] * fac;
-                    w = raw[u] * v_alpha;
+                    w = vis[u] * v_alpha;
                 }
                 const float wx = w * dx[u], wy = w * dy[u];
                 const float sum8[8] = {w, wx, wx * dx[u], wy, wy * dx[u], wy * dy[u], v_red, v_green};

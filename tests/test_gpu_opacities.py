@@ -65,3 +65,79 @@ def test_opacities_that_no_pixel_takes(oracle, blend_form, pixels_per_lane, bins
     bounds = oracle.gradient_bounds(s, 16, A["means_3d"], A["scales"], A["rotations"], S["conic"], S["cov3d"], radii,
                                     B["abs_sums"], rel=1e-4)
     check_grads_against_bounds(got, B, bounds, gok, "opacities")
+
+
+def one_splat_per_tile(opacity, mean, conic, final_T=None, v_image=None, behind=None):
+    """The blend stages on hand-made records: tile t of a square image holds splat t (and, behind it, splat
+    tiles + t, if given).  opacity[T], mean[T, 2] from the tile's first pixel centre, conic[T, 3]; colours are 1."""
+    from ds_splat_amd import stages
+    tiles = opacity.numel()
+    side = int(round(tiles ** 0.5))
+    assert side * side == tiles
+    layers = 1 if behind is None else 2
+    sc = make_scene("cfg0", n=1, width=16 * side, height=16 * side, sh_degree=0)
+    cam = stages.camera_from_scene(sc, DEV, list_bin=1)
+    first = torch.stack([torch.arange(tiles) % side, torch.arange(tiles) // side], 1) * 16.0 + 0.5
+    rec = torch.zeros(layers * tiles, 12)
+    rec[:tiles, 0:2], rec[:tiles, 4:7], rec[:tiles, 7] = first + mean, conic, opacity
+    rec[:, 8:11] = 1.0
+    if behind is not None:
+        rec[tiles:, 0:2], rec[tiles:, 4:7], rec[tiles:, 7] = first + 7.25, torch.tensor([1e-4, 0.0, 1e-4]), behind
+    ids = torch.arange(layers * tiles).view(layers, tiles).t().contiguous().view(-1)
+    rec, ids = rec.to(DEV), ids.to(torch.int32).to(DEV)
+    ranges = torch.arange(0, layers * tiles + 1, layers, dtype=torch.int32, device=DEV)
+    image, T, idx = stages.blend_fwd(cam, ranges, ids, rec)
+    out = {"image": image.cpu(), "T": T.cpu(), "idx": idx.cpu(), "rec": rec.cpu(), "side": side}
+    if v_image is not None:
+        grads = stages.blend_bwd(cam, layers * tiles, ranges, ids, rec, T if final_T is None else final_T.to(DEV), idx,
+                                 v_image.to(DEV))
+        out["grads"] = grads.cpu()
+    torch.cuda.synchronize()
+    return out
+
+
+@pytest.mark.parametrize("pixels_per_lane", [1, 4])
+def test_alpha_is_a_product_with_the_opacity(blend_form, pixels_per_lane):
+    """Half of an opacity gives half of alpha, to the last bit (a pixel's only splat, of colour 1, shows alpha); as a
+    term of the exponential's argument the halves would be rounded on their own."""
+    blend_form(pixels_per_lane)
+    g = torch.Generator().manual_seed(5)
+    rand = lambda *s: torch.rand(*s, generator=g)
+    opacity = 0.02 * 40.0 ** rand(1024)
+    mean = rand(1024, 2) * 16.0 - 0.5
+    a, c = 0.002 * 50.0 ** rand(1024), 0.002 * 50.0 ** rand(1024)
+    conic = torch.stack([a, (rand(1024) - 0.5) * torch.sqrt(a * c), c], 1)
+    whole = one_splat_per_tile(opacity, mean, conic)
+    for k in (1, 2):
+        part = one_splat_per_tile(opacity * 0.5 ** k, mean, conic)
+        seen = part["image"][..., 0] > 0
+        assert seen.float().mean() > 0.2
+        assert torch.equal(part["image"][seen], whole["image"][seen] * 0.5 ** k)
+
+
+@pytest.mark.parametrize("pixels_per_lane", [1, 4])
+def test_opacity_gradient_of_faint_splats(blend_form, pixels_per_lane):
+    """v_opacity of a pixel's only splat, from one pixel, against 64 bits.  Its rounding errors, as root mean squares
+    in 1e-8 of the value: the exponent's product 2, the exponential 4, T = final_T / (1 - alpha) four of 2 to 3.5,
+    two products 2.5 each: 8 together.  With the opacity's logarithm as a term of the exponent (6.6 there: half a
+    unit in its last place is 24) another 9."""
+    blend_form(pixels_per_lane)
+    tiles, side = 1024, 32
+    g = torch.Generator().manual_seed(6)
+    rand = lambda *s: torch.rand(*s, generator=g)
+    opacity = 0.009 + 0.003 * rand(tiles)
+    # sigma = 1/2 a dx^2 with dx = 4: a product of exact factors, the same in any precision
+    mean = torch.stack([torch.full((tiles,), 2.0), torch.full((tiles,), 5.0)], 1)
+    a = 0.02 + 0.06 * rand(tiles)
+    conic = torch.stack([a, torch.zeros(tiles), a], 1)
+    v = torch.zeros(16 * side, 16 * side, 3)
+    v[5::16, 6::16, 0] = 1.0                    # the pixel at (6, 5) of every tile
+    out = one_splat_per_tile(opacity, mean, conic, v_image=v)
+    vis = torch.exp(-0.5 * a.double() * 16.0)
+    alpha = opacity.double() * vis
+    assert (alpha > 1.0 / 255.0).all()
+    want = {5: vis, 6: alpha}                   # (T is 1: nothing lies in front)
+    for column, w in want.items():
+        rms = float(((out["grads"][:, column].double() / w - 1.0) ** 2).mean().sqrt())
+        print("column %d: rms relative error %.2e" % (column, rms))
+        assert rms < 1.0e-7
