@@ -53,10 +53,12 @@ constexpr float kLog2Of255 = 7.994353436858858f;
 // Largest sigma with alpha >= 1/255, about ln(255 opacity): the test of alpha is taken on sigma, before the
 // exponential and with the same bits in both directions.  -infinity for an opacity that no pixel takes, whose entry is
 // then not even staged; infinity for an infinite one; NaN for a NaN.
-// The reach is found as the last float for which opacity * exp2(-sigma log2(e)), evaluated just so, passes: an
-// estimate from the logarithm, one Newton step on that expression, and a bisection of the eight floats around
-// it.  (The logarithm's own rounding alone would move the line between in and out by two or three floats, and with
-// it a few hundred of the 10^9 decisions of a large scene.)
+// The reach is the last float for which opacity * exp2(-sigma log2(e)), evaluated just so, passes: every decision is
+// the one that comparing alpha itself would take (alpha falls with sigma).  For opacities of 2/255 and more it lies
+// within the eight floats around an estimate from the logarithm and one Newton step on that expression.  Below, where
+// sigma is small, hundreds to millions of floats of it share one alpha: there all floats within 1e-6 of the estimate are
+// bisected (its error is a few rounding errors of alpha, 3e-7); far above, where the exponential underflows before
+// alpha does, all floats there are.  Only wavefronts that stage such an entry take those steps.
 __device__ __forceinline__ float reach_of(float opacity)
 {
 #pragma clang fp contract(off)
@@ -67,9 +69,26 @@ __device__ __forceinline__ float reach_of(float opacity)
 #pragma unroll
     for(int step = 4; step > 0; step >>= 1)
         bits += alpha_at(__int_as_float(bits + step)) >= 1.0f / 255.0f ? step : 0;
-    reach = reach > 1e-3f ? __int_as_float(bits) : reach;
-    // (masked and pruned Gaussians: zero, denormal and negative opacities have no logarithm to start from)
-    return opacity < 1.0f / 255.0f ? -__builtin_inff() : (opacity == __builtin_inff() ? opacity : reach);
+    const bool far_off = (opacity >= 1.0f / 255.0f && opacity < 2.0f / 255.0f) || !(opacity <= 1e30f);
+    if(__builtin_amdgcn_ballot_w64(far_off) != 0)
+    {
+        int past = bits; // alpha passes at `bits` and does not at `past`
+        if(far_off && opacity < __builtin_inff())
+        {
+            bits = opacity < 1.0f ? __float_as_int(fmaxf(reach - 1e-6f, 0.0f)) : 0;
+            past = opacity < 1.0f ? __float_as_int(fmaxf(reach, 0.0f) + 1e-6f) : 0x7f800000;
+        }
+        while(past - bits > 1)
+        {
+            const int mid = bits + (past - bits) / 2;
+            const bool passes = alpha_at(__int_as_float(mid)) >= 1.0f / 255.0f;
+            bits = passes ? mid : bits;
+            past = passes ? past : mid;
+        }
+        bits = !(opacity < __builtin_inff()) ? __float_as_int(opacity) : bits;
+    }
+    // (masked and pruned Gaussians: zero, denormal and negative opacities)
+    return opacity < 1.0f / 255.0f ? -__builtin_inff() : __int_as_float(bits);
 }
 // Both tests of an entry at a pixel, that sigma has the right sign and that it does not exceed the reach,
 // in one integer compare: the bits of floats of one sign are ordered like their magnitudes.

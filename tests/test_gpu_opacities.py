@@ -141,3 +141,47 @@ def test_opacity_gradient_of_faint_splats(blend_form, pixels_per_lane):
         rms = float(((out["grads"][:, column].double() / w - 1.0) ** 2).mean().sqrt())
         print("column %d: rms relative error %.2e" % (column, rms))
         assert rms < 1.0e-7
+
+
+@pytest.mark.parametrize("span", ["faint", "ordinary", "huge"])
+@pytest.mark.parametrize("pixels_per_lane", [1, 4])
+def test_a_pixel_is_blended_exactly_where_alpha_reaches_the_threshold(blend_form, pixels_per_lane, span):
+    """The limit on sigma that an entry is staged with is the last float for which alpha, evaluated as the kernels do,
+    is at least 1/255: forward and backward take the pixels that comparing alpha itself takes.  Alpha is read off a
+    run with twice the opacity, whose alpha is twice as large to the last bit.  The splats' centres lie far away, so
+    that sigma changes by a few floats from pixel to pixel and many floats of sigma share one alpha where it is small."""
+    blend_form(pixels_per_lane)
+    tiles, side = 4096, 64
+    g = torch.Generator().manual_seed(7)
+    rand = lambda *s: torch.rand(*s, generator=g, dtype=torch.float64)
+    u = rand(tiles)
+    ratio = {"faint": 1.0 + 10.0 ** (-6.0 * u), "ordinary": 2.0 * 50.0 ** u, "huge": 100.0 * 10.0 ** (38.0 * u)}[span]
+    opacity = (ratio / 255.0).float()
+    r = torch.log(255.0 * opacity.double())
+    far = 10.0 ** (2.0 + 4.0 * rand(tiles))
+    angle = 2.0 * np.pi * rand(tiles)
+    direction = torch.stack([torch.cos(angle), torch.sin(angle)], 1)
+    # sigma reaches r within the tile, at 7.5 pixels from its first centre along both axes
+    mean = (7.5 + far[:, None] * direction).float()
+    a = (2.0 * r / far ** 2).float()
+    conic = torch.stack([a, torch.zeros(tiles), a], 1)
+    whole = one_splat_per_tile(opacity * 2.0, mean, conic)
+    alpha = whole["image"][..., 0] * 0.5
+    # (twice the opacity passes nearly everywhere; the largest ones' exponential underflows first)
+    assert (alpha > 0).float().mean() > (0.8 if span == "huge" else 0.9)
+    takes = alpha >= torch.tensor(1.0) / 255.0
+    per_tile = takes.view(side, 16, side, 16).permute(0, 2, 1, 3).reshape(tiles, 256).float().mean(1)
+    assert ((per_tile > 0) & (per_tile < 1)).float().mean() > 0.5
+    v = torch.ones(16 * side, 16 * side, 3)
+    got = one_splat_per_tile(opacity, mean, conic, v_image=v, behind=torch.full((tiles,), 0.5))
+    # the splat behind is in the lists' odd places and passes everywhere
+    assert (got["idx"] % 2 == 1).all()
+    T = got["T"]
+    back = one_splat_per_tile(torch.zeros(tiles), mean, conic, behind=torch.full((tiles,), 0.5))["T"]
+    assert ((T < back) == takes).all(), "%d pixels" % int(((T < back) != takes).sum())
+    # backward: the sum of alpha over the pixels that it took, against the forward's pixels; one pixel is 1/256 of it
+    # (below the clamps, which differ between the two directions)
+    by_tile = torch.where(takes, alpha, torch.zeros(())).double().view(side, 16, side, 16).permute(0, 2, 1, 3).reshape(tiles, 256)
+    plain = by_tile.max(1).values < 0.4
+    assert plain.float().mean() > 0.9
+    np.testing.assert_allclose(got["grads"][:tiles, 6].double()[plain].numpy(), by_tile.sum(1)[plain].numpy(), rtol=1e-5, atol=1e-7)
