@@ -170,15 +170,16 @@ struct DepthRange
     Digits32 digits;
 };
 // lowest, highest: upper halves of the smallest and the largest key that emits (lowest > highest: there is none)
-__host__ __device__ inline DepthRange depth_range(uint32_t lowest, uint32_t highest)
+__host__ __device__ constexpr DepthRange depth_range(uint32_t lowest, uint32_t highest)
 {
-    DepthRange r;
+    DepthRange r = {};
     if(lowest > highest)
         lowest = highest = 0;
+    const uint32_t halves = highest - lowest + 1; // at most 0x10000: the count of distances is 32 bits with all of them zero
+    const int bits = 16 + 32 - __builtin_clz(halves);
     r.first = lowest << 16;
-    r.behind = ((highest - lowest) << 16) + 0x10000u; // (no key that emits has all ones in its upper half: a NaN)
-    const int bits = 32 - __builtin_clz(r.behind);
-    r.narrow = bits <= kDepthPasses * kDepthBits && highest < 0xffffu;
+    r.behind = halves << 16;
+    r.narrow = bits <= kDepthPasses * kDepthBits && highest < 0xffffu; // (all ones: a NaN, which does not emit)
     if(!r.narrow)
     {
         r.first = 0;
@@ -195,6 +196,10 @@ __host__ __device__ inline DepthRange depth_range(uint32_t lowest, uint32_t high
     }
     return r;
 }
+// (the widest range there is, and the ends of the narrow ones)
+static_assert(!depth_range(0, 0xffffu).narrow && depth_range(0, 0xffffu).behind == kNoPairsKey, "keys as they are");
+static_assert(depth_range(0x4000u, 0x47feu).narrow && depth_range(0x4000u, 0x47feu).behind == 0x07ff0000u, "27 bits");
+static_assert(!depth_range(0x4000u, 0x47ffu).narrow, "28 bits");
 // bits needed for tile slots 0..num_tiles (slot 0 = keys with a negative depth, slot t+1 = tile t)
 inline int slot_bits(int num_tiles)
 {
