@@ -290,7 +290,8 @@ struct Pixels
     __device__ __forceinline__ int y_of(int p) const { return y + 2 * p; }
 };
 
-// word `i` of a device array (uniform base and a 32-bit byte offset: one address register)
+// word `i` of a device array (uniform base and a 32-bit byte offset: one address register; i < 2^30, so a scan of a
+// list passes the place where it stands as the base)
 __device__ __forceinline__ int word_at(const int32_t* base, uint32_t i)
 {
     return *reinterpret_cast<const int32_t*>(reinterpret_cast<const char*>(base) + 4u * i);
@@ -498,12 +499,14 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(8, 8))
                     // the loads of four groups of positions are issued together: the scan is bound by
                     // their latency, not by its dozen instructions per group
                     int gid[kScanGroups], key[kScanGroups];
+                    const int32_t* const ids_here = ids + scan;
+                    const int32_t* const keys_here = keys + scan;
 #pragma unroll
                     for(int j = 0; j < kScanGroups; ++j)
                     {
-                        const uint32_t e = (uint32_t)min(scan + j * DSX_WAVE + lane, end - 1);
-                        gid[j] = word_at(ids, e);
-                        key[j] = word_at(keys, e);
+                        const uint32_t e = (uint32_t)min(j * DSX_WAVE + lane, end - 1 - scan);
+                        gid[j] = word_at(ids_here, e);
+                        key[j] = word_at(keys_here, e);
                     }
 #pragma unroll
                     for(int j = 0; j < kScanGroups; ++j)
@@ -700,13 +703,16 @@ __device__ __forceinline__ int tile_scan(TileScan& s, int* queue, const int32_t*
         int id[kScanGroups];
         uint64_t m[kScanGroups];
         uint32_t key[kScanGroups];
+        const int most = min(left, kScanGroups * kTileThreads) - 1;
+        const int32_t* const ids_here = ids + (kStep > 0 ? at : at - most);
+        const int32_t* const keys_here = keys + (kStep > 0 ? at : at - most);
 #pragma unroll
         for(int j = 0; j < kScanGroups; ++j)
         {
-            const int o = min(j * kTileThreads + tid, left - 1);
-            const uint32_t e = (uint32_t)(kStep > 0 ? at + o : at - o);
-            id[j] = word_at(ids, e);
-            key[j] = (uint32_t)word_at(keys, e);
+            const int o = min(j * kTileThreads + tid, most);
+            const uint32_t e = (uint32_t)(kStep > 0 ? o : most - o);
+            id[j] = word_at(ids_here, e);
+            key[j] = (uint32_t)word_at(keys_here, e);
         }
 #pragma unroll
         for(int j = 0; j < kScanGroups; ++j)
@@ -1318,12 +1324,15 @@ __global__ __launch_bounds__(DSX_WAVE) void blend_bwd_kernel(
                 do
                 {
                     int gid[kScanGroups], key[kScanGroups];
+                    const int most = min(pos - start, kScanGroups * DSX_WAVE - 1);
+                    const int32_t* const ids_here = ids + (pos - most);
+                    const int32_t* const keys_here = keys + (pos - most);
 #pragma unroll
                     for(int j = 0; j < kScanGroups; ++j)
                     {
-                        const uint32_t e = (uint32_t)max(pos - j * DSX_WAVE - lane, start);
-                        gid[j] = word_at(ids, e);
-                        key[j] = word_at(keys, e);
+                        const uint32_t e = (uint32_t)max(most - j * DSX_WAVE - lane, 0);
+                        gid[j] = word_at(ids_here, e);
+                        key[j] = word_at(keys_here, e);
                     }
 #pragma unroll
                     for(int j = 0; j < kScanGroups; ++j)

@@ -98,3 +98,31 @@ def test_depth_order_over_a_known_range(n, depths):
     assert (seen["perm"] == perm).all()
     sums = np.add.reduceat(touched[perm], np.arange(0, n, 256))
     assert (seen["offsets"] == np.concatenate([[0], np.cumsum(sums)])).all()
+
+
+@pytest.mark.parametrize("pixels_per_lane", [1, 4])
+def test_bin_lists_beyond_two_to_the_thirty(blend_form, pixels_per_lane):
+    """Positions of a bin's list that a 32-bit byte offset does not reach: the same lists, moved behind 2^30 others,
+    give the same image and gradients (the places they would be mistaken for hold other Gaussians)."""
+    from ds_splat_amd import stages
+    blend_form(pixels_per_lane)
+    sc = make_scene("cfg0", n=5000, width=160, height=112, sh_degree=0, seed=4)
+    cam = stages.camera_from_scene(sc, DEV, list_bin=4)
+    t = {k: (v.to(DEV) if isinstance(v, torch.Tensor) else v) for k, v in sc.items()}
+    n = sc["n"]
+    image, st = stages.forward(cam, t["means_3d"], t["scales"] * 2.0, t["rotations"], t["opacities"], t["shs"])
+    grads = stages.blend_bwd(cam, n, st.lists, st.sorted_ids, st.splats, st.final_T, st.final_idx, t["v_image"])
+    k, ahead = st.num_keys, 1 << 30
+    if torch.cuda.mem_get_info()[0] < 12 * ahead:
+        pytest.skip("needs 12 GiB of free GPU memory")
+    moved = torch.empty(2 * (ahead + k), dtype=torch.int32, device=DEV)
+    moved[:k], moved[ahead + k:ahead + 2 * k] = st.ids.flip(0), st.sorted_ids[k:].flip(0)
+    moved[ahead:ahead + k], moved[2 * ahead + k:] = st.ids, st.sorted_ids[k:]
+    lists = st.lists.clone()
+    stages.split_lists(cam, lists)["bins"].add_(ahead)
+    image2, T2, idx2 = stages.blend_fwd(cam, lists, moved, st.splats)
+    assert torch.equal(image2, image) and torch.equal(T2, st.final_T) and torch.equal(idx2, st.final_idx)
+    grads2 = stages.blend_bwd(cam, n, lists, moved, st.splats, T2, idx2, t["v_image"])
+    # (the same terms; float atomics add them in another order)
+    assert torch.allclose(grads2[:, :9], grads[:, :9], rtol=1e-3, atol=1e-4 * float(grads[:, :9].abs().max()))
+    assert float(grads[:, :9].abs().max()) > 0
