@@ -406,6 +406,43 @@ std::tuple<at::Tensor, at::Tensor> forward(const at::Tensor& means3d, const at::
     return {out[0], out[1]};
 }
 
+// The two directions for an autograd function written in Python (DsRasterizerFunction and what derives from it): what
+// the forward leaves, and the gradients from it.
+std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor, int64_t>
+render_parts(const at::Tensor& means3d, const at::Tensor& means2d, const OptTensor& shs, const OptTensor& colors,
+             const at::Tensor& opacities, const OptTensor& scales, const OptTensor& quats, const OptTensor& cov3d,
+             int64_t height, int64_t width, double tanfovx, double tanfovy, double scale_modifier, int64_t sh_degree,
+             int64_t max_sh_degree, const at::Tensor& view, const at::Tensor& proj, const at::Tensor& campos,
+             const at::Tensor& bg, int64_t list_bin, bool prepare_backward)
+{
+    const Settings settings{height, width, tanfovx, tanfovy, scale_modifier, sh_degree, max_sh_degree, view, proj,
+                            campos, bg, list_bin, false};
+    const Inputs in{means3d, means2d, shs, colors, opacities, scales, quats, cov3d};
+    validate(in, settings);
+    c10::DeviceGuard guard(means3d.device());
+    Rendered r = render(make_camera(settings, means3d.device()), in, prepare_backward);
+    return {r.image, r.radii, r.splats, r.sorted_ids, r.ranges, r.final_T, r.final_idx, r.grads, r.k};
+}
+
+std::vector<at::Tensor> backward_of_parts(const at::Tensor& means3d, const OptTensor& shs, const OptTensor& scales,
+                                          const OptTensor& quats, const OptTensor& cov3d, const at::Tensor& splats,
+                                          const at::Tensor& radii, const at::Tensor& ranges, const at::Tensor& sorted_ids,
+                                          const at::Tensor& final_T, const at::Tensor& final_idx,
+                                          const at::Tensor& v_image, const OptTensor& prepared, int64_t k, int64_t wanted,
+                                          int64_t height, int64_t width, double tanfovx, double tanfovy,
+                                          double scale_modifier, int64_t sh_degree, int64_t max_sh_degree,
+                                          const at::Tensor& campos, const at::Tensor& bg, int64_t list_bin)
+{
+    const Settings settings{height, width, tanfovx, tanfovy, scale_modifier, sh_degree, max_sh_degree, at::Tensor(),
+                            at::Tensor(), campos, bg, list_bin, false};
+    c10::DeviceGuard guard(means3d.device());
+    require(splats.size(0) == means3d.numel() / 3 + kViewRecords, "splats must be what render returned");
+    const Camera camera = make_camera(settings, means3d.device(),
+                                      splats.data_ptr<float>() + means3d.numel() / 3 * DSX_SPLAT_FLOATS);
+    return differentiate(camera, k, bases_of(shs), means3d, scales, quats, cov3d, splats, radii, ranges, sorted_ids,
+                         final_T, final_idx, v_image, prepared.value_or(at::Tensor()), wanted);
+}
+
 } // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
@@ -414,9 +451,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     // (torch's own wrappers: errors come back as torch's exceptions, and a Python exception that a hook on saved
     // tensors raises, as recomputation under checkpointing does, passes through as it is)
     m.def("forward", torch::wrap_pybind_function_no_gil(forward), "projection, tile lists and blend; differentiable");
-    m.def("backward", torch::wrap_pybind_function_no_gil([](const at::Tensor& image, const at::Tensor& v_image) {
-              image.backward(v_image);
-          }),
-          "the backward of an image that forward returned");
+    m.def("render", torch::wrap_pybind_function_no_gil(render_parts),
+          "the forward without a node: (image, radii, splats, sorted_ids, ranges, final_T, final_idx, grads, k)");
+    m.def("backward", torch::wrap_pybind_function_no_gil(backward_of_parts), "the eight gradients from what render left");
     m.def("version", []() { return dsx_version(); });
 }

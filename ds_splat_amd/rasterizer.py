@@ -17,15 +17,62 @@ import torch
 from . import _native
 
 
-class DsRasterizerFunction:
-    """The differentiable call under ``GaussianRasterizer``: checks, forward and autograd node are native
-    (csrc/torch_ext.cpp).  ``raster_settings`` is what ``GaussianRasterizer.settings_for_cpp_code`` returns."""
+class DsRasterizerFunction(torch.autograd.Function):
+    """The differentiable call under ``GaussianRasterizer``.  ``raster_settings`` is what
+    ``GaussianRasterizer.settings_for_cpp_code`` returns.
+
+    ``DsRasterizerFunction.apply`` itself goes to the native autograd node (csrc/torch_ext.cpp: checks, forward and
+    node without Python).  ``forward`` and ``backward`` are for functions derived from this one, whose ``apply`` is
+    torch's: the same kernels, with the tensors kept on ``ctx``."""
+
+    @classmethod
+    def apply(cls, *args, **kwargs):
+        return _apply(*args, **kwargs) if cls is DsRasterizerFunction else super().apply(*args, **kwargs)
 
     @staticmethod
-    def apply(means_3d, means_2d, shs, colors_precomp, opacities, scales, rotations, cov_3d_precomp, raster_settings):
+    def forward(ctx, means_3d, means_2d, shs, colors_precomp, opacities, scales, rotations, cov_3d_precomp,
+                raster_settings):
+        image, radii, _ = DsRasterizerFunction.run_forward(ctx, means_3d, means_2d, shs, colors_precomp, opacities,
+                                                           scales, rotations, cov_3d_precomp, raster_settings)
+        return image, radii
+
+    @staticmethod
+    def run_forward(ctx, means_3d, means_2d, shs, colors_precomp, opacities, scales, rotations, cov_3d_precomp,
+                    raster_settings):
+        """The forward proper; also returns final_T (for functions that composite a background)."""
         s = raster_settings
-        return _render(means_3d, means_2d, shs, colors_precomp, opacities, scales, rotations, cov_3d_precomp, s,
-                       s.view_matrix.t(), s.proj_matrix.t(), s.max_sh_degree, False)
+        scalars = (int(s.image_height), int(s.image_width), float(s.tanfovx), float(s.tanfovy),
+                   float(s.scale_modifier), int(s.sh_degree), int(s.max_sh_degree))
+        list_bin = _native.default_list_bin()
+        image, radii, splats, sorted_ids, ranges, final_T, final_idx, ctx.prepared_grads, k = \
+            _native.load_torch_ext().render(means_3d, means_2d, shs, colors_precomp, opacities, scales, rotations,
+                                            cov_3d_precomp, *scalars, s.view_matrix.t(), s.proj_matrix.t(), s.campos,
+                                            s.bg, list_bin, any(ctx.needs_input_grad[:8]))
+        ctx.num_keys, ctx.cam = k, scalars + (s.campos, s.bg, list_bin)
+        ctx.save_for_backward(means_3d, shs, scales, rotations, cov_3d_precomp, splats, radii, ranges, sorted_ids,
+                              final_T, final_idx)
+        ctx.opacity_shape = opacities.shape
+        ctx.mark_non_differentiable(radii)
+        ctx.set_materialize_grads(False)
+        return image, radii, final_T
+
+    @staticmethod
+    def backward(ctx, rendered_img_grad, _):
+        if rendered_img_grad is None:   # nothing flows into the image (gradients are not materialised)
+            return (None,) * 9
+        wanted = sum(1 << i for i in range(8) if ctx.needs_input_grad[i])
+        prepared, ctx.prepared_grads = ctx.prepared_grads, None   # good for one backward: it leaves sums behind
+        grads = list(_native.load_torch_ext().backward(*ctx.saved_tensors, rendered_img_grad.contiguous(), prepared,
+                                                       ctx.num_keys, wanted, *ctx.cam))
+        if grads[4] is not None:
+            grads[4] = grads[4].reshape(ctx.opacity_shape)
+        return (*grads, None)
+
+
+def _apply(means_3d, means_2d, shs, colors_precomp, opacities, scales, rotations, cov_3d_precomp, raster_settings):
+    s = raster_settings
+    return _render(means_3d, means_2d, shs, colors_precomp, opacities, scales, rotations, cov_3d_precomp, s,
+                   s.view_matrix.t(), s.proj_matrix.t(), s.max_sh_degree, False)
 
 
 def _render(means_3d, means_2d, shs, colors_precomp, opacities, scales, rotations, cov_3d_precomp, s, viewmatrix,

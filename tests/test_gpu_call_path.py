@@ -168,3 +168,41 @@ def test_counts_belong_to_the_call_that_waits_for_them():
         begin(60000, 2.0)
         assert counts(begin(5000, 1.0), 5000) == want
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("opacity_shape", [(-1, 1), (-1,)])
+def test_functions_derived_from_the_rasterizers(opacity_shape):
+    """DsRasterizerFunction is an autograd function: one derived from it, as it is or with an output more, gives the
+    image and gradients of the call itself."""
+    from ds_splat_amd import DsRasterizerFunction
+
+    class Plain(DsRasterizerFunction):
+        pass
+
+    class WithTransmittance(DsRasterizerFunction):
+        @staticmethod
+        def forward(ctx, *args):
+            image, radii, final_T = DsRasterizerFunction.run_forward(ctx, *args)
+            ctx.mark_non_differentiable(radii, final_T)
+            return image, radii, final_T
+
+        @staticmethod
+        def backward(ctx, v_image, _, __):
+            return DsRasterizerFunction.backward(ctx, v_image, None)
+
+    assert issubclass(DsRasterizerFunction, torch.autograd.Function)
+    image_w, grads_w = wanted()
+    for function in (DsRasterizerFunction, Plain, WithTransmittance):
+        _, t, leaves = scene()
+        means, means2d, shs, opac, scales, rots = leaves
+        none = torch.empty(0, device=DEV)
+        out = function.apply(means, means2d, shs, none, opac.reshape(opacity_shape), scales, rots, none,
+                             rasterizer(t).settings_for_cpp_code)
+        out[0].backward(t["v_image"], retain_graph=True)
+        assert torch.equal(out[0], image_w)
+        check_grads([x.grad for x in leaves], grads_w)
+        out[0].backward(t["v_image"])                         # (the prepared accumulator serves the first one only)
+        check_grads([x.grad for x in leaves], [2.0 * g for g in grads_w])
+        with pytest.raises(RuntimeError):
+            out[0].backward(t["v_image"])
+        assert len(out) == 2 or float((out[2] - 1.0).abs().max()) > 0.01
