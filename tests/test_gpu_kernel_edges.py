@@ -3,8 +3,10 @@ import numpy as np
 import pytest
 import torch
 
+import test_gpu_pipeline
 import test_gpu_stages
 from ds_splat_amd.synthetic import make_scene
+from helpers import comparable_gaussians
 
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda:0")
@@ -126,3 +128,39 @@ def test_bin_lists_beyond_two_to_the_thirty(blend_form, pixels_per_lane):
     # (the same terms; float atomics add them in another order)
     assert torch.allclose(grads2[:, :9], grads[:, :9], rtol=1e-3, atol=1e-4 * float(grads[:, :9].abs().max()))
     assert float(grads[:, :9].abs().max()) > 0
+
+
+@pytest.mark.parametrize("bins", [1, 4])
+@pytest.mark.parametrize("pixels_per_lane", [1, 4])
+@pytest.mark.parametrize("W,H", [(323, 197), (64, 48)])
+def test_channel_first_image_in_every_blend_form(oracle, blend_form, list_bin, pixels_per_lane, bins, W, H):
+    """The adaptor's image and gradients (planes of the image stored and read by the blend kernels, background
+    composited) from both forms of the kernels and both kinds of lists, where planes and rows end inside a quad of
+    lanes and inside a tile, and where they do not."""
+    from ds_splat_amd import inria_compat
+    blend_form(pixels_per_lane)
+    list_bin(bins)
+    bg = np.array([0.3, 0.6, 0.1], np.float32)
+    sc = make_scene("cfg1", n=12000, width=W, height=H, sh_degree=1, seed=31)
+    t = {k: (v.to(DEV) if isinstance(v, torch.Tensor) else v) for k, v in sc.items()}
+    p = dict(means=t["means_3d"].clone(), means2d=torch.zeros_like(t["means_3d"]), shs=t["shs"].clone(),
+             opac=t["opacities"].clone(), scales=t["scales"] * 2.0, rots=t["rotations"].clone())
+    p = {k: v.requires_grad_(True) for k, v in p.items()}
+    settings = inria_compat.GaussianRasterizationSettings(
+        image_height=H, image_width=W, tanfovx=sc["tanfovx"], tanfovy=sc["tanfovy"], bg=torch.from_numpy(bg).to(DEV),
+        scale_modifier=1.0, viewmatrix=t["viewmatrix"], projmatrix=t["projmatrix"], sh_degree=1, campos=t["campos"])
+    color, radii = inria_compat.GaussianRasterizer(settings)(
+        means3D=p["means"], means2D=p["means2d"], opacities=p["opac"], shs=p["shs"], scales=p["scales"],
+        rotations=p["rots"])
+    color.backward(t["v_image"].permute(2, 0, 1))
+    torch.cuda.synchronize()
+    img_o, radii_o, S, B = test_gpu_pipeline.oracle_run(oracle, sc, 2.0, bg=bg)
+    assert color.shape == (3, H, W) and color.is_contiguous() and (radii.cpu().numpy() == radii_o).all()
+    ok = S["margin"] > 1e-4
+    assert ok.mean() > 0.98
+    want = img_o + S["final_T"][..., None] * bg
+    np.testing.assert_allclose(color.detach().permute(1, 2, 0).cpu().numpy()[ok], want[ok], rtol=1e-4, atol=1e-5)
+    fT, fidx, _ = test_gpu_pipeline.gpu_forward_state(sc, 2.0)
+    gok = comparable_gaussians(S, B, W, fT, fidx)
+    assert gok.mean() > 0.8
+    test_gpu_pipeline.check_grads(p, B, gok, "channel first %d %d" % (pixels_per_lane, bins))
