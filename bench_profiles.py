@@ -87,11 +87,12 @@ def trace_name(short):
     """The name the library's own event trace (and bench.py's JSON line) uses for a kernel."""
     base = short.split("<")[0]
     if base == "onesweep32_kernel":
-        # the depth sort of the Gaussians carries their rectangles through the passes (last template argument;
-        # images of more than 255 tiles a side excepted); the tile partition, with 16-bit slots per tile or 32-bit
-        # slot words per bin, carries nothing
-        return "onesweep32_kernel<sort>" if short.rstrip().endswith("true>") else "onesweep32_kernel<tile partition>"
-    return base
+        # <key type, threads, items, carry, bits>: the depth sort of the Gaussians carries their rectangles through the
+        # passes (images of more than 255 tiles a side excepted) or has digits of nine bits (over a known range); the
+        # tile partition, with 16-bit slots per tile or 32-bit slot words per bin, does neither
+        carry, bits = [a.strip() for a in short[short.index("<") + 1:short.rindex(">")].split(",")][3:5]
+        return "onesweep32_kernel<sort>" if carry == "true" or bits != "8" else "onesweep32_kernel<tile partition>"
+    return base.replace("_tile_kernel", "_kernel") if base.startswith("blend_") else base
 
 
 def git_commit():
@@ -167,7 +168,7 @@ def algorithmic_bytes(bench):
     m = re.match(r"(\w+): (\d+) Gaussians, (\d+)x(\d+), SH degree (\d+)", cfg["workload"])
     n, w, h, deg = int(m.group(2)), int(m.group(3)), int(m.group(4)), int(m.group(5))
     out = {}
-    for k in ("project_fwd_kernel", "gaussian_bwd_kernel", "hist32_kernel", "onesweep32_kernel<sort>",
+    for k in ("project_fwd_kernel", "gaussian_bwd_kernel", "hist32_kernel", "depth_hist_kernel", "onesweep32_kernel<sort>",
               "ordered_block_sums_kernel", "emit_ordered_kernel", "onesweep32_kernel<tile partition>"):
         bound, work, _ = bench_module.algorithmic_work(k, n, cfg["num_keys"], w * h, cfg["lists"], (deg + 1) ** 2, None,
                                                        cfg.get("gaussians_with_gradient", 0),
@@ -259,7 +260,7 @@ def cmd_sq(args):
 
 def cmd_mem(args):
     """Vector-memory instructions and atomics per kernel: how many atomic requests the blend backward sends
-    (one instruction per blended (tile, entry) with nine active lanes) and what share of its time they are."""
+    (one for each of a staged entry's nine sums and round) and what share of its time they are."""
     d = counters_per_kernel(args.mem_dir)
     times = kernel_times_ms(args.stats_dir)
     avg = lambda x: sum(x) / len(x) if x else 0.0
@@ -268,9 +269,9 @@ def cmd_mem(args):
              "Commands (on the MI355X box, repository root, after `export TMPDIR=/tmp`):", "",
              "    " + command(MEM_CMD, args.mem_dir, args.workload),
              "    " + command(STATS_CMD, args.stats_dir, args.workload) + "    # the `kernel ms` column", "",
-             "Averages per launch. `VMEM write inst` counts stores and atomics (the blend backward issues one atomic",
-             "instruction per blended (tile, entry), nine lanes active, plus one byte store for the Gaussian's mark, and at",
-             "its end the stores of the zeros); `L2 atomic requests` is TCC_ATOMIC summed over the L2 channels.", "",
+             "Averages per launch. `VMEM write inst` counts stores and atomics (the blend backward adds up a round's entries",
+             "in LDS and issues their nine sums, 64 a wavefront, as atomics, each with a byte store for the Gaussian's mark, and",
+             "at its end the stores of the zeros); `L2 atomic requests` is TCC_ATOMIC summed over the L2 channels.", "",
              "| kernel | waves | VMEM read inst / wave | VMEM write inst / wave | branches / wave | TCP atomic requests | L2 atomic requests | L2 atomics / us | kernel ms |",
              "|---|---|---|---|---|---|---|---|---|"]
     for k in sorted(d, key=lambda k: -avg(d[k]["TCC_ATOMIC_sum"])):

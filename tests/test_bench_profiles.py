@@ -1,0 +1,32 @@
+"""The profile tool's names of kernels: what bench.py's trace calls them, from what rocprofv3 does."""
+import os
+import re
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+sys.path.insert(0, ROOT)
+
+
+@pytest.mark.parametrize("kernel,name", [
+    # key type, threads, items, whether rectangles go along, bits of a digit
+    ("void dsx::onesweep32_kernel<unsigned int, 1024, 4, true, 9>(dsx::Sort32)", "onesweep32_kernel<sort>"),
+    ("void dsx::onesweep32_kernel<unsigned int, 1024, 4, true, 8>(dsx::Sort32)", "onesweep32_kernel<sort>"),
+    ("void dsx::onesweep32_kernel<unsigned int, 1024, 12, false, 9>(dsx::Sort32)", "onesweep32_kernel<sort>"),
+    ("void dsx::onesweep32_kernel<unsigned int, 1024, 12, false, 8>(dsx::Sort32)", "onesweep32_kernel<tile partition>"),
+    ("void dsx::onesweep32_kernel<unsigned short, 1024, 8, false, 8>(dsx::Sort32)", "onesweep32_kernel<tile partition>"),
+    ("void dsx::blend_fwd_tile_kernel<true>(int const*)", "blend_fwd_kernel"),
+    ("void dsx::blend_bwd_kernel<false>(int const*)", "blend_bwd_kernel"),
+    ("dsx::project_fwd_kernel(float)", "project_fwd_kernel"),
+])
+def test_trace_names(kernel, name):
+    import bench_profiles
+    assert bench_profiles.trace_name(bench_profiles.short_name(kernel)) == name
+
+
+def test_the_sorts_template_is_what_the_names_assume():
+    source = open(os.path.join(ROOT, "ds_splat_amd", "csrc", "tile_lists.hip")).read()
+    head = re.search(r"template <([^>]*)>\s*__global__[^;{]*onesweep32_kernel\(", source)
+    assert [p.split("=")[0].split()[-1] for p in head.group(1).split(",")] == ["KeyT", "kSort32Threads", "kSort32Items",
+                                                                              "kCarry", "kBits"]
