@@ -1142,19 +1142,22 @@ __global__ __launch_bounds__(kCoverThreads) void tile_counts_kernel(const Counts
 // ---------------------------------------------------------------------------------------
 // few Gaussians: depth order and counting in one launch or two
 // ---------------------------------------------------------------------------------------
-// Up to 16384 Gaussians the digit passes, their histogram, the block sums and the scan are eight launches
+// Up to 24576 Gaussians the digit passes, their histogram, the block sums and the scan are eight launches
 // of 3 to 8 us that each do a microsecond's work (2 K Gaussians: 38 us of kernels, 16 K: 50 us).  Here a workgroup
 // sorts 2048 keys in its own LDS and registers (by the digits of the keys' distance from the smallest one, three
 // or fewer for any scene whose depths stay within a factor of eight), and one more (two, for binned lists)
 // fills a corner grid of its own and counts the tiles (and the bins) beside it.  Up to 2048 Gaussians that is
 // all; beyond, a second launch ranks every key among the other workgroups' sorted keys by binary search in LDS.
-// 2 K Gaussians: 10 us, 4 K: 9 + 7, 16 K: 13 + 17 (32 K: 21 + 30, no better than the passes).  (One workgroup for
-// 16 K keys, sixteen to a thread: 51 us.)
+// 2 K Gaussians: 10 us, 4 K: 9 + 7, 16 K: 13 + 17.  (One workgroup for 16 K keys, sixteen to a thread: 51 us.)
+// The line lies where a whole forward stops gaining, us, digit passes / merge, at 256x256 and at 1024x768:
+// 3000 Gaussians 89 / 48 and 101 / 60, 8 K 100 / 63 and 106 / 76, 16 K 110 / 92 and 118 / 104, 18000 109 / 98 and
+// 120 / 111, 20 K 112 / 102 and 122 / 116, 24 K 110 / 105 and 126 / 124, 28 K 112 / 112 and 130 / 134, 32 K 112 / 115 and
+// 135 / 142.
 constexpr int kSmallThreads = 1024;
 static_assert(kSmallThreads == kCoverThreads, "tile_counts is written for this many threads");
 constexpr int kSmallItems = 2;
 constexpr int kSmallTile = kSmallThreads * kSmallItems;
-constexpr int kSmallTilesMax = 8;
+constexpr int kSmallTilesMax = 12;
 constexpr int kSmallMax = kSmallTile * kSmallTilesMax;
 constexpr int kMergeThreads = 256;
 constexpr int kSmallWaves = kSmallThreads / DSX_WAVE;

@@ -164,3 +164,10 @@ def test_channel_first_image_in_every_blend_form(oracle, blend_form, list_bin, p
     gok = comparable_gaussians(S, B, W, fT, fidx)
     assert gok.mean() > 0.8
     test_gpu_pipeline.check_grads(p, B, gok, "channel first %d %d" % (pixels_per_lane, bins))
+
+
+@pytest.mark.parametrize("depths", ["spread", "ties"])
+@pytest.mark.parametrize("n", [18433, 24575, 24576, 24577])
+def test_depth_order_up_to_twelve_tiles_of_keys(n, depths):
+    """The merge of more than eight tiles of keys (a third group of four, partly empty), and where the passes take over."""
+    test_depth_order_of_few_gaussians(n, depths)
