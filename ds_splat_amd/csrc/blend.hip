@@ -151,10 +151,20 @@ __device__ __forceinline__ uint32_t blocks_reached(float mx, float my, float a, 
 
 // Pixels per lane of the blend kernels: 4 (one wavefront per tile) when the image has enough tiles
 // to occupy the chip (8 wavefronts on each of 1024 SIMDs), else 1 (a workgroup of four wavefronts per
-// tile: more instructions in all, but four times as many wavefronts and shorter chains).  Measured, us,
-// wavefront / workgroup form:
-//   forward   256 tiles 107 / 34, 1024 84 / 36, 2170 70 / 48, 3600 169 / 130, 6370 305 / 304, 8160 127 / 141
-//   backward  1024 tiles 154 / 77, 2170 125 / 106, 4056 249 / 280, 6370 514 / 654
+// tile: more instructions in all, but four times as many wavefronts and shorter chains).  Measured on scenes of four
+// kinds, us by which a whole forward (a whole training step) is longer with the workgroup form of that kernel:
+//   forward, tiles                            3600  4590  5700  6370  7150  8160
+//     opaque, 0.24 Gaussians a pixel           -13    -8    +5    +6     0   +21   (of 190 to 245)
+//     mixed, 0.9 a pixel                       -37   -25    -9   -15    +3   +39   (of 336 to 520)
+//     faint, 0.6 a pixel                       -36   -23   +12   +20   +58   +64   (of 286 to 722)
+//     large, 0.25 a pixel                       +6   +11   +12    +4   +14   +29   (of 207 to 293)
+//   backward, tiles                           1200  1900  2170  3072  3600  4590
+//     opaque                                   -63   -47   -29    +9   +19   +21   (of 221 to 407)
+//     mixed                                   -159  -121   -88   -42   +40   +70   (of 326 to 900)
+//     faint                                    -86   -77   -56   -49    -9   +43   (of 238 to 903)
+//     large                                     -8    -7    -3   +25   +22   -40   (of 278 to 422)
+// (The kernels run again and again by themselves, with their inputs in the caches, cross at fewer tiles: 4000 in the
+// forward.)  The lines at 6400 and 3000 tiles lie within those crossings.
 // dsx_set_blend_pixels_per_lane(1 | 4) overrides the choice for the whole process (tests run both
 // forms); DSX_BLEND_PIXELS_PER_LANE=1|4 in the environment gives the override's initial value and is
 // read once.
