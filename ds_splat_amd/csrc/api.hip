@@ -1,5 +1,5 @@
-// extern "C" surface of libdsx: argument checks, stage sequencing, the one host
-// synchronisation of the forward (read-back of the key count) and error strings.
+// extern "C" surface of libdsx: argument checks, stage sequencing, the forward's waits of the host
+// (for the pair counts and, above 262144 Gaussians, for the range of the depths) and error strings.
 #include "dsx_common.h"
 
 #include <algorithm>

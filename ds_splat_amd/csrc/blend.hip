@@ -208,7 +208,7 @@ struct BinLists
     const int32_t* fine;      // int32[tiles + 1]
     const int32_t* last_tile; // highest occupied tile (-1: none)
     const int32_t* bins;      // int32[bins + 1]
-    int32_t* walk;            // int32[tiles * 8]: per tile and band of four rows, where the forward's scan of the bin list stopped and how many of the tile's entries it had met by then
+    int32_t* walk;            // int32[tiles * 8]: per tile, where the forward's scan of the bin list stopped and how many of the tile's entries it had met by then
     int shift, nbx, nty;
 };
 
@@ -671,7 +671,7 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(8, 8))
     {
         // for the backward: where this wavefront's scan of the bin's list stopped and how many of the
         // tile's entries it had met by then (everything that any of its pixels blended lies below).
-        // The other three parts are marked as empty.
+        // The tile's other six words are marked as empty.
         int32_t* w = lists.walk + (int64_t)px.tile * 8;
         const int stopped = min(scan, end);
         if(lane < 8)
@@ -1200,7 +1200,7 @@ __device__ __forceinline__ void flush_sums(const double* sums, const int* ids, i
 // 16 lanes with DPP adds, all four rows' entries at once, and ONE atomic instruction carries the nine
 // sums of up to four entries.
 // kBinned: the entries come out of the list of the tile's bin, filtered into a queue as in the forward
-// but downwards; the forward left, per tile and part, the bin-list position where its scan stopped and
+// but downwards; the forward left, per tile, the bin-list position where its scan stopped and
 // the number of the tile's entries it had met by then, from which every entry met on the way down
 // gets its index in the sorted key array (final_idx is compared with those).
 template <bool kBinned>
@@ -1282,7 +1282,7 @@ __global__ __launch_bounds__(DSX_WAVE) void blend_bwd_kernel(
     if(kBinned && layout_ok)
     {
         // The forward's scan of the bin's list stopped at position w[0] after meeting w[1] of the
-        // tile's entries (the larger of the four parts' figures: both grow together); everything
+        // tile's entries (the largest of the four pairs of words, of which three are empty); everything
         // that was blended lies below, and the entries are taken from there downwards.  An entry's
         // index is the tile's range start plus its rank; those above the last blended one (m) are
         // not even queued, so the entries that are handed on have consecutive indices.

@@ -254,9 +254,9 @@ inline bool valid_list_bin(int b)
 // and, when the lists are binned,
 //   last_tile[1]      highest tile that holds a pair of non-negative depth, -1 if none
 //   bins[bins + 1]    ranges of the bin lists inside sorted_ids
-//   walk[tiles * 8]   written by the blend forward for the backward: per tile and band of four
-//                     rows, the position in the bin's list where the forward's scan stopped and
-//                     the number of the tile's own entries it had met by then
+//   walk[tiles * 8]   written by the blend forward for the backward: per tile, the position in the
+//                     bin's list where the forward's scan stopped and the number of the tile's own
+//                     entries it had met by then; the other six words are marked as empty (-1, 0)
 struct RangesLayout
 {
     int fine, header, last_tile, bins, walk, count;

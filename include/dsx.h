@@ -126,8 +126,8 @@ int32_t dsx_sort_passes(int32_t num_tiles);
  * dsx_ranges_count: int32 words of the `ranges` buffer of those entry points: tiles + 1 words of
  * per-tile ranges as the reference defines them (cpp/rasterizer_torch.cu:23-42), one header word
  * (log2 of b: the blend kernels walk nothing when it is not the b they were launched for) and, for
- * b > 1, the highest occupied tile, the bins' ranges and 8 words per tile that the blend forward
- * leaves for the backward.  No counterpart in the reference. */
+ * b > 1, the highest occupied tile, the bins' ranges and 8 words per tile of which the blend forward
+ * leaves two for the backward.  No counterpart in the reference. */
 int32_t dsx_list_bin(int32_t width, int32_t height, int32_t list_bin);
 int64_t dsx_ranges_count(int32_t width, int32_t height, int32_t list_bin);
 /* int32 words of the `sorted_ids` buffer for k pairs: k ids and, for b > 1, behind them one word per
@@ -278,10 +278,11 @@ int dsx_gaussian_bwd(const dsx_camera* cam, int64_t n, int32_t num_bases, const 
 /* ------------------------------------------------------------------------------------ */
 
 /* First half of rasterizer_forward_deepsense (cpp/rasterizer_torch.cu:170-208): projection,
- * the read-back of K (the one host wait of the forward, in place of the reference's block scan
- * and two device drains at cpp/rasterizer_torch.cu:95-104; K is summed from the tile rectangles
- * by the first kernel that runs beside the depth sort) and, overlapping that read-back, the depth
- * order.  block_sums[dsx_num_blocks(n)] receives the tile count of each 256-Gaussian block
+ * the read-back of K (a host wait, in place of the reference's block scan and two device drains at
+ * cpp/rasterizer_torch.cu:95-104; K is summed from the tile rectangles by the first kernel that runs
+ * beside the depth sort) and, overlapping that read-back, the depth order.  Above 262144 Gaussians the
+ * host also waits, between the projection and the sort's passes, for the range of the depths.  Both
+ * waits make the call fail (DSX_ERR_RUNTIME) on a stream that is being captured.  block_sums[dsx_num_blocks(n)] receives the tile count of each 256-Gaussian block
  * (not scanned).  order: device buffer of dsx_order_bytes(n, W, H, cam->list_bin).  num_keys (host,
  * TWO entries; pinned memory lets the copy overlap): [0] receives k, the number of pairs of the lists
  * that dsx_forward_finish will build (entries of sorted_ids); [1] the number of pairs of the per-tile
@@ -294,7 +295,8 @@ int dsx_forward_project(const dsx_camera* cam, int64_t n, const float* means3d,
                         void* order, size_t order_bytes, int64_t* num_keys /* host */,
                         void* stream);
 /* The same in two halves, for a caller that has something to do (allocations) while the device sorts: everything up
- * to the wait, and the wait for the pair counts of the calling thread's last dsx_forward_project_begin.
+ * to the wait for the pair counts (above 262144 Gaussians it waits for the range of the depths itself, see above), and
+ * that wait, for the counts of the calling thread's last dsx_forward_project_begin.
  * view_copy: device float[16] that receives `view`, row by row, for a backward that runs when the caller's own matrix
  * may be another one (null: none). */
 int dsx_forward_project_begin(const dsx_camera* cam, int64_t n, const float* means3d,
