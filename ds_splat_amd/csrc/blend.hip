@@ -54,41 +54,42 @@ constexpr float kLog2Of255 = 7.994353436858858f;
 // exponential and with the same bits in both directions.  -infinity for an opacity that no pixel takes, whose entry is
 // then not even staged; infinity for an infinite one; NaN for a NaN.
 // The reach is the last float for which opacity * exp2(-sigma log2(e)), evaluated just so, passes: every decision is
-// the one that comparing alpha itself would take (alpha falls with sigma).  For opacities of 2/255 and more it lies
-// within the eight floats around an estimate from the logarithm and one Newton step on that expression.  Below, where
-// sigma is small, hundreds to millions of floats of it share one alpha: there all floats within 1e-6 of the estimate are
-// bisected (its error is a few rounding errors of alpha, 3e-7); far above, where the exponential underflows before
-// alpha does, all floats there are.  Only wavefronts that stage such an entry take those steps.
+// the one that comparing alpha itself would take (alpha falls with sigma).  It lies within 2.4e-7 of an estimate from
+// the logarithm and one Newton step on that expression, or within four floats of it where those are further apart, and
+// is found by bisection: three steps for a reach of a half and more, one more for every halving of it (opacities from
+// 1/255 to 2/255, where ever more floats of sigma share one alpha).  All floats are bisected next to 1/255 and beyond
+// 1e30, where the exponential underflows before alpha falls to 1/255.
 __device__ __forceinline__ float reach_of(float opacity)
 {
 #pragma clang fp contract(off)
-    float reach = (__builtin_amdgcn_logf(opacity) + kLog2Of255) * kLn2;
+    const float guess = (__builtin_amdgcn_logf(opacity) + kLog2Of255) * kLn2;
     auto alpha_at = [&](float sigma) { return opacity * __builtin_amdgcn_exp2f(-sigma * kLog2E); };
-    reach += __builtin_fmaf(alpha_at(reach), 255.0f, -1.0f);
-    int bits = __float_as_int(reach) - 4;
-#pragma unroll
-    for(int step = 4; step > 0; step >>= 1)
-        bits += alpha_at(__int_as_float(bits + step)) >= 1.0f / 255.0f ? step : 0;
-    const bool far_off = (opacity >= 1.0f / 255.0f && opacity < 2.0f / 255.0f) || !(opacity <= 1e30f);
-    if(__builtin_amdgcn_ballot_w64(far_off) != 0)
+    int bits = __float_as_int(guess + __builtin_fmaf(alpha_at(guess), 255.0f, -1.0f)) - 4;
+    auto bisect = [&](int step) { bits += alpha_at(__int_as_float(bits + step)) >= 1.0f / 255.0f ? step : 0; };
+    const bool few = opacity >= 1.0f / 255.0f && opacity < 2.0f / 255.0f, many = opacity > 1e30f;
+    // (only wavefronts that stage such an entry take more than the three steps)
+    if(__builtin_amdgcn_ballot_w64(few || many) != 0)
     {
-        int past = bits; // alpha passes at `bits` and does not at `past`
-        if(far_off && opacity < __builtin_inff())
+        constexpr int kHalf = 0x3f000000, kAll = 1 << 30;
+        int step = few && bits < kHalf ? 4 << ((kHalf - bits + 0x7fffff) >> 23) : 4;
+        bits -= step - 4;
+        if(many || (few && bits < 0x35800000)) // (2^-20)
         {
-            bits = opacity < 1.0f ? __float_as_int(fmaxf(reach - 1e-6f, 0.0f)) : 0;
-            past = opacity < 1.0f ? __float_as_int(fmaxf(reach, 0.0f) + 1e-6f) : 0x7f800000;
+            bits = 0;
+            step = kAll;
         }
-        while(past - bits > 1)
-        {
-            const int mid = bits + (past - bits) / 2;
-            const bool passes = alpha_at(__int_as_float(mid)) >= 1.0f / 255.0f;
-            bits = passes ? mid : bits;
-            past = passes ? past : mid;
-        }
-        bits = !(opacity < __builtin_inff()) ? __float_as_int(opacity) : bits;
+        while(__builtin_amdgcn_ballot_w64(step > 4) != 0)
+            if(step > 4)
+            {
+                bisect(step);
+                step >>= 1;
+            }
     }
+    bisect(4);
+    bisect(2);
+    bisect(1);
     // (masked and pruned Gaussians: zero, denormal and negative opacities)
-    return opacity < 1.0f / 255.0f ? -__builtin_inff() : __int_as_float(bits);
+    return opacity < 1.0f / 255.0f ? -__builtin_inff() : (opacity < __builtin_inff() ? __int_as_float(bits) : opacity);
 }
 // Both tests of an entry at a pixel, that sigma has the right sign and that it does not exceed the reach,
 // in one integer compare: the bits of floats of one sign are ordered like their magnitudes.
