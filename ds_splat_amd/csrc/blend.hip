@@ -1,12 +1,13 @@
 // Stages 4 and 5a for gfx950: per-tile alpha blending, forward (front to back) and backward
 // (back to front).
 //
-// Both directions are bound by the issue of vector instructions, so what counts is how many a (pixel, entry)
-// pair costs and how many pairs are looked at that need not be.  1920x1080 unless noted, us, before (every
-// wavefront walks one list for its 256 pixels) -> now:
-//   forward   2 M faint Gaussians 1097 -> 830, 1.4 M at 1557x1038 384 -> 307, 500 K opaque 130 -> 127,
-//             6 M at 3840x2160 488 -> 450, 16 K at 256x256 58 -> 34
-//   backward  2 M faint 2215 -> 1590, 1.4 M at 1557x1038 658 -> 514, 500 K opaque 251 -> 221, 50 K at 512x512 136 -> 77
+// Both directions are bound by the issue of vector instructions (where an entry reaches all of its tile: by latency and
+// the LDS), so what counts is how many a (pixel, entry) pair costs and how many pairs are looked at that need not be.
+// 1920x1080 unless noted, us within a whole pass, before (every wavefront walks one list for its 256 pixels) -> now:
+//   forward   2 M faint Gaussians 1119 -> 896, 1.4 M at 1557x1038 387 -> 331, 500 K opaque 139 -> 150 (3 M: 147 -> 156),
+//             6 M at 3840x2160 510 -> 508, 1 M large ones 104 -> 116, 1 M at 1280x720 184 -> 149, 16 K at 256x256 56 -> 34
+//   backward  2 M faint 2240 -> 1669, 1.4 M at 1557x1038 678 -> 550, 500 K opaque 260 -> 240 (3 M: 293 -> 272),
+//             1 M large ones 259 -> 285, 300 K at 1237x822 346 -> 262, 50 K at 512x512 139 -> 78
 #include "dsx_common.h"
 
 #include <atomic>
