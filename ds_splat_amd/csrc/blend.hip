@@ -65,19 +65,23 @@ __device__ __forceinline__ float reach_of(float opacity)
 #pragma clang fp contract(off)
     const float guess = (__builtin_amdgcn_logf(opacity) + kLog2Of255) * kLn2;
     auto alpha_at = [&](float sigma) { return opacity * __builtin_amdgcn_exp2f(-sigma * kLog2E); };
-    int bits = __float_as_int(guess + __builtin_fmaf(alpha_at(guess), 255.0f, -1.0f)) - 4;
+    int bits = (int)(__float_as_uint(guess + __builtin_fmaf(alpha_at(guess), 255.0f, -1.0f)) - 4u);
     auto bisect = [&](int step) { bits += alpha_at(__int_as_float(bits + step)) >= 1.0f / 255.0f ? step : 0; };
     const bool few = opacity >= 1.0f / 255.0f && opacity < 2.0f / 255.0f, many = opacity > 1e30f;
     // (only wavefronts that stage such an entry take more than the three steps)
     if(__builtin_amdgcn_ballot_w64(few || many) != 0)
     {
-        constexpr int kHalf = 0x3f000000, kAll = 1 << 30;
-        int step = few && bits < kHalf ? 4 << ((kHalf - bits + 0x7fffff) >> 23) : 4;
-        bits -= step - 4;
-        if(many || (few && bits < 0x35800000)) // (2^-20)
+        constexpr int kHalf = 0x3f000000, kLeast = 0x35800000; // 2^-20
+        int step = 4;
+        if(many || (few && bits < kLeast)) // (also where the estimate is below zero)
         {
             bits = 0;
-            step = kAll;
+            step = 1 << 30;
+        }
+        else if(few && bits < kHalf)
+        {
+            step = 4 << ((kHalf - bits + 0x7fffff) >> 23);
+            bits -= step - 4;
         }
         while(__builtin_amdgcn_ballot_w64(step > 4) != 0)
             if(step > 4)
