@@ -1,18 +1,20 @@
 // Stages 4 and 5a for gfx950: per-tile alpha blending, forward (front to back) and backward
 // (back to front).
 //
-// Both directions are bound by the issue of vector instructions (where an entry reaches all of its tile: by latency and
-// the LDS), so what counts is how many a (pixel, entry) pair costs and how many pairs are looked at that need not be.
-// 1920x1080 unless noted, us within a whole pass, before (every wavefront walks one list for its 256 pixels) -> now:
-//   forward   2 M faint Gaussians 1119 -> 896, 1.4 M at 1557x1038 387 -> 331, 500 K opaque 139 -> 150 (3 M: 147 -> 156),
-//             6 M at 3840x2160 510 -> 508, 1 M large ones 104 -> 116, 1 M at 1280x720 184 -> 149, 16 K at 256x256 56 -> 34
-//   backward  2 M faint 2240 -> 1669, 1.4 M at 1557x1038 678 -> 550, 500 K opaque 260 -> 240 (3 M: 293 -> 272),
-//             1 M large ones 259 -> 285, 300 K at 1237x822 346 -> 262, 50 K at 512x512 139 -> 78
+// Both directions are bound by the issue of vector instructions (85 to 90 % of the time where no pixel stops early), so what
+// counts is how many a (pixel, entry) pair costs and how many pairs are looked at that need not be.  The backward of large Gaussians,
+// which every tile adds to, also waits for the memory: 13 ns for each request to one line.
+// 1920x1080 unless noted, us within a whole pass, before (four lists of entries per wavefront) -> now (sixteen):
+//   forward   2 M faint Gaussians 905 -> 717, 1.4 M at 1557x1038 340 -> 285, 500 K opaque 148 -> 130 (3 M: 161 -> 155),
+//             6 M at 3840x2160 519 -> 446, 1 M large ones 118 -> 120, 1 M at 1280x720 148 -> 129, 16 K at 256x256 34 -> 30
+//   backward  2 M faint 1662 -> 1317, 1.4 M at 1557x1038 553 -> 488, 500 K opaque 242 -> 235 (3 M: 279 -> 270),
+//             1 M large ones 290 -> 307, 300 K at 1237x822 263 -> 238, 50 K at 512x512 78 -> 74
 #include "dsx_common.h"
 
 #include <atomic>
 #include <climits>
 #include <cstdlib>
+#include <type_traits>
 
 namespace dsx
 {
@@ -112,65 +114,21 @@ __device__ __forceinline__ uint32_t reach_limit_bwd(float opacity, float reach)
     return reach >= 0.0f ? __float_as_uint(reach) : (opacity != opacity ? 0x7f800000u : 0u);
 }
 
-// The pixels of a wavefront, as four square blocks of kSide x kSide: 8 x 8 (a whole tile, four pixels per
-// lane) or 4 x 4 (a quarter of a tile, one pixel per lane).  Row r of the wavefront's lanes (16 lanes, a
-// DPP row) owns block r and walks ITS OWN list of entries: the four rows blend four different
-// entries at the same time.  An entry of a tile's list that touches the tile at all touches only part of
-// it (dense: 2.5 of its four 8 x 8 blocks, cfg2: 3.2), so a wavefront that walks one list for all
-// of its pixels spends up to half of its lanes on pixels that the entry cannot reach; skipping those
-// on the scalar unit costs as much as it saves, while giving the lanes another entry costs two address
-// instructions.  The rows wait for each other only once per round of staged entries.
-//
-// Which of the four blocks can this entry reach with alpha >= 1/255?  The exponent's quadratic form
-// q(d) = 1/2 (a dx^2 + c dy^2) + b dx dy is convex, so its minimum over a block's box of pixel
-// centres is 0 if the splat's centre lies inside and otherwise sits on an edge that faces the centre,
-// where it is a clamped one-dimensional parabola.  Taking the column and the row of the box that lie nearest to
-// the centre covers both: they are the facing edges where there are any (and points of the box where not).
-// A block is left out only if qmin exceeds the entry's reach by more than 0.01 (one percent of alpha, as slack
-// against rounding); an entry with a degenerate conic or without a limit is kept for all.
-// (x0, y0: the first pixel centre of block 0; bit r of the result: block r, x first)
-template <int kSide>
-__device__ __forceinline__ uint32_t blocks_reached(float mx, float my, float a, float b, float c, float reach,
-                                                   float x0, float y0)
-{
-    const float half_a = 0.5f * a, half_c = 0.5f * c;
-    const float to_v = -b * __builtin_amdgcn_rcpf(c), to_u = -b * __builtin_amdgcn_rcpf(a);
-    const float limit = reach + 0.01f;
-    const bool well_formed = a > 0.0f && c > 0.0f;
-    const float u_first = x0 - mx, v_first = y0 - my;
-    uint32_t reached = 0;
-    // (a loop, not unrolled: what the blocks could share would hold two dozen registers where few are free)
-#pragma unroll 1
-    for(int r = 0; r < 4; ++r)
-    {
-        const float u0 = u_first + (float)((r & 1) * kSide), v0 = v_first + (float)((r >> 1) * kSide);
-        const float u1 = u0 + (float)(kSide - 1), v1 = v0 + (float)(kSide - 1);
-        const float un = __builtin_amdgcn_fmed3f(0.0f, u0, u1), vn = __builtin_amdgcn_fmed3f(0.0f, v0, v1);
-        // along the nearest column, and along the nearest row
-        const float v = __builtin_amdgcn_fmed3f(to_v * un, v0, v1);
-        const float u = __builtin_amdgcn_fmed3f(to_u * vn, u0, u1);
-        const float qmin = fminf(v * (half_c * v + b * un) + half_a * un * un, u * (half_a * u + b * vn) + half_c * vn * vn);
-        reached |= (well_formed && qmin > limit) ? 0u : 1u << r;
-    }
-    return reached;
-}
-
 // Pixels per lane of the blend kernels: 4 (one wavefront per tile) when the image has enough tiles
-// to occupy the chip (8 wavefronts on each of 1024 SIMDs), else 1 (a workgroup of four wavefronts per
+// to occupy the chip, else 1 (a workgroup of four wavefronts per
 // tile: more instructions in all, but four times as many wavefronts and shorter chains).  Measured on scenes of four
 // kinds, us by which a whole forward (a whole training step) is longer with the workgroup form of that kernel:
 //   forward, tiles                            3600  4590  5700  6370  7150  8160
-//     opaque, 0.24 Gaussians a pixel           -13    -8    +5    +6     0   +21   (of 190 to 245)
-//     mixed, 0.9 a pixel                       -37   -25    -9   -15    +3   +39   (of 336 to 520)
-//     faint, 0.6 a pixel                       -36   -23   +12   +20   +58   +64   (of 286 to 722)
-//     large, 0.25 a pixel                       +6   +11   +12    +4   +14   +29   (of 207 to 293)
+//     opaque, 0.24 Gaussians a pixel           -12    -7    +2    +5    -4    +6   (of 177 to 243)
+//     mixed, 0.9 a pixel                       -16   -23    +1    -9   +12   +21   (of 312 to 511)
+//     faint, 0.6 a pixel                       -13    +5   +35   +53   +86  +108   (of 261 to 703)
+//     large, 0.25 a pixel                       +1    +5    +9    -1   +14   +11   (of 202 to 301)
 //   backward, tiles                           1200  1900  2170  3072  3600  4590
-//     opaque                                   -63   -47   -29    +9   +19   +21   (of 221 to 407)
-//     mixed                                   -159  -121   -88   -42   +40   +70   (of 326 to 900)
-//     faint                                    -86   -77   -56   -49    -9   +43   (of 238 to 903)
-//     large                                     -8    -7    -3   +25   +22   -40   (of 278 to 422)
-// (The kernels run again and again by themselves, with their inputs in the caches, cross at fewer tiles: 4000 in the
-// forward.)  The lines at 6400 and 3000 tiles lie within those crossings.
+//     opaque                                   -42   -34   -22   +17   +26   +40   (of 213 to 409)
+//     mixed                                    -93   -55   -27    -2   +70  +125   (of 312 to 919)
+//     faint                                    -48   -35   -15    +9   +58  +122   (of 229 to 888)
+//     large                                    -25   -13   -16   +10    +8   -31   (of 271 to 445)
+// The lines at 5500 and 3000 tiles lie within those crossings.
 // dsx_set_blend_pixels_per_lane(1 | 4) overrides the choice for the whole process (tests run both
 // forms); DSX_BLEND_PIXELS_PER_LANE=1|4 in the environment gives the override's initial value and is
 // read once.
@@ -275,35 +233,25 @@ __device__ __forceinline__ int bits_below_lane(uint64_t mask)
     return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
 
-constexpr int kFwdFourPixelsFrom = 6400; // tiles
+constexpr int kFwdFourPixelsFrom = 5500; // tiles
 constexpr int kBwdFourPixelsFrom = 3000;
 
 // -----------------------------------------------------------------------------------------
-// what both directions share: the wavefront's pixels, and the walk through the lists
+// what both directions share: the pixels, and the walk through the lists
 // -----------------------------------------------------------------------------------------
-// kPix pixels per lane: 4 (one wavefront per 16x16 tile, its rows of lanes own 8x8 blocks) or 1 (four
-// wavefronts per tile, each one 8x8 quadrant, its rows of lanes own 4x4 blocks).
-template <int kPerLane>
+// The pixels of the workgroup forms: wavefront w of a tile owns quadrant w, its rows of 16 lanes a 4 x 4 block each.  Blocks
+// of a tile are numbered as in blocks_reached: row r of the wavefront owns block first_block_of(w) + block_of_row(r).
+__host__ __device__ constexpr int first_block_of(int wave) { return 8 * (wave >> 1) + 2 * (wave & 1); }
+__host__ __device__ constexpr int block_of_row(int row) { return 4 * (row >> 1) + (row & 1); }
 struct Pixels
 {
-    static constexpr int kSide = kPerLane == 4 ? 8 : 4; // a row's block
-    int tile, part;    // part: which quarter of the tile (0 for the whole)
-    int x0, y0;        // first pixel of the wavefront
-    int x, y;          // this lane's first pixel; the others lie two rows apart
-    float box_x, box_y; // first pixel centre of the wavefront
-    __device__ __forceinline__ Pixels(int block, int ntx, int lane)
+    int x, y;
+    __device__ __forceinline__ Pixels(int tile, int wave, int ntx, int lane)
     {
-        tile = kPerLane == 4 ? block : block >> 2;
-        part = kPerLane == 4 ? 0 : block & 3;
-        x0 = (tile % ntx) * kTile + 8 * (part & 1);
-        y0 = (tile / ntx) * kTile + 8 * (part >> 1);
         const int row = lane >> 4, i = lane & 15;
-        x = x0 + kSide * (row & 1) + (i & (kSide - 1));
-        y = y0 + kSide * (row >> 1) + i / kSide;
-        box_x = (float)x0 + 0.5f;
-        box_y = (float)y0 + 0.5f;
+        x = (tile % ntx) * kTile + 8 * (wave & 1) + 4 * (row & 1) + (i & 3);
+        y = (tile / ntx) * kTile + 8 * (wave >> 1) + 4 * (row >> 1) + i / 4;
     }
-    __device__ __forceinline__ int y_of(int p) const { return y + 2 * p; }
 };
 
 // word `i` of a device array (uniform base and a 32-bit byte offset: one address register; i < 2^30, so a scan of a
@@ -323,13 +271,6 @@ __device__ __forceinline__ uint64_t lanes_below(int count)
 __device__ __forceinline__ uint64_t lowest_bits(uint64_t mask, int count)
 {
     return __builtin_amdgcn_ballot_w64(bits_below_lane(mask) < count) & mask;
-}
-
-// the value of one lane of each quad of lanes (quad_perm), in all four
-template <int kCtrl>
-__device__ __forceinline__ float quad_lane(float v)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kCtrl, 0xf, 0xf, false));
 }
 
 // A side job for the memory system, which the forward leaves idle: every workgroup prepares
@@ -360,34 +301,145 @@ __device__ __forceinline__ void prepare_grads_share(const float4* splats, float4
 // forward: cpp/rasterizer_kernels.cu:341-431
 // -----------------------------------------------------------------------------------------
 // No workgroup barrier anywhere: a workgroup is one wavefront.  A round takes entries of the tile's
-// list, 64 at a time, until no further 64 would fit: their records are gathered, those that reach any
-// pixel of the wavefront are staged in LDS (packed: what cannot reach leaves no hole), and the place
-// of each goes into the list of every row of lanes whose block it reaches.  Then the rows walk
-// their lists side by side.
-// Images of few tiles (fewer wavefronts than the chip has slots) take kPix = 1: four times
-// as many wavefronts, whose smaller blocks also leave each row fewer entries to walk.
+// list, 64 at a time: what cannot reach the box around the blocks that still have a live pixel drops out (two words of its record
+// and some forty instructions for 64 of them; two thirds of the faint Gaussians' rectangles touch tiles that they do not reach),
+// and when 64 are left they are staged in LDS, each lane one, and the place of each goes into the list of every quad of
+// lanes whose block it reaches.  Then the quads walk their lists side by side.
 constexpr int kPix = 4; // pixels per lane of the wavefront forms
 constexpr float kAlphaMax = 0.999f;       // the forward's clamp (the backward's is 0.99)
-constexpr int kFwdBatch = 96; // staged entries of a round: 5 KB of LDS, 32 wavefronts per compute unit
 constexpr int kScanGroups = 4; // groups of 64 positions of a bin's list whose loads are in flight together
 
-typedef float dsx_f32x4 __attribute__((ext_vector_type(4)));
+// The 16 blocks of a tile, 4 x 4 pixels each: bit 4 r + c of a mask is the block of the r-th four rows and c-th four
+// columns.  A wavefront that works on a whole tile has a quad of lanes for each block (lane l: quad l >> 2, the column l & 15 of
+// the tile and four pixels, one below the other), and each quad walks ITS OWN list of entries: sixteen entries are blended side by
+// side.  An entry of a tile's list that touches the tile at all touches only part of it, so a wavefront that walks one list
+// for all of its pixels spends most of its lanes on pixels that the entry cannot reach; skipping those on the
+// scalar unit costs as much as it saves, while giving the lanes another entry costs two address instructions.  The quads
+// wait for each other only once per round of staged entries.  Steps of the walk per tile, of four rows of lanes with a list for each
+// 8 x 8 block and of sixteen quads (2 M faint Gaussians at 1920x1080, 1.4 M at 1557x1038, 1 M at 1280x720, 500 K opaque at 1920x1080):
+// 713 -> 570, 258 -> 224, 195 -> 154, 86 -> 82; one list for all pixels takes 1056, 362, 300 and 120.
+constexpr int kQuads = 16;
 
-// Stores one pixel per lane: a lane's four neighbours lie in one row of pixels, and its registers are one channel of
-// all of them.  planar: the image is channel-first and has the background composited (the transmittance of
-// the quad's pixels comes from their lanes).
-__device__ __forceinline__ void store_colours(float* image, const dsx_f32x4 colour, float T, int x, int y, int W, int H, int lane,
-                                              bool broken, const float* bg, int planar)
+// which quads a wavefront mask has a lane of: bit q (uniform)
+__device__ __forceinline__ uint32_t quads_of(uint64_t mask, int lane)
 {
-    const int quad_x = x - (lane & 3), channel = lane & 3;
-    const float back = planar && channel < 3 ? bg[channel] : 0.0f;
-    const float quad_T[4] = {quad_lane<0x00>(T), quad_lane<0x55>(T), quad_lane<0xAA>(T), quad_lane<0xFF>(T)};
-    const int step = planar ? 1 : 3;
-    float* const out = image + (planar ? ((int64_t)channel * H + y) * W + quad_x : 3 * ((int64_t)y * W + quad_x) + channel);
+    return (uint32_t)__builtin_amdgcn_ballot_w64(((mask >> (4 * (lane & 15))) & 15u) != 0) & 0xffffu;
+}
+
+// The box of pixel centres around some blocks of a tile
+struct LiveBox
+{
+    float x0, x1, y0, y1;
+};
+__device__ __forceinline__ LiveBox live_box(uint32_t blocks, float x, float y)
+{
+    const uint32_t columns = (blocks | blocks >> 4 | blocks >> 8 | blocks >> 12) & 15u;
+    LiveBox box;
+    box.x0 = x + (float)(4 * __builtin_ctz(columns | 16u));
+    box.x1 = x + (float)(4 * (31 - __builtin_clz(columns | 1u)) + 3);
+    box.y0 = y + (float)(__builtin_ctz(blocks | 0x10000u) & ~3);
+    box.y1 = y + (float)(((31 - __builtin_clz(blocks | 1u)) & ~3) + 3);
+    return box;
+}
+
+// Can this splat (the first two words of its record) reach a pixel of the box with alpha >= 1/255?
+// The exponent's quadratic form q(d) = 1/2 (a dx^2 + c dy^2) + b dx dy is convex, so its minimum over the box is 0 if the
+// splat's centre lies inside and otherwise sits on an edge that faces the centre, where it is a clamped one-dimensional
+// parabola.  Taking the column and the row of the box that lie nearest to the centre covers both: they are the
+// facing edges where there are any (and points of the box where not).  An entry is left out only if the minimum exceeds
+// ln(255 opacity) by more than 0.01 (one percent of alpha, as slack against rounding); one with a degenerate conic or
+// without a limit is kept.
+__device__ __forceinline__ bool box_reached(const LiveBox& box, const float4 q0, const float4 q1)
+{
+    const float a = q1.x, b = q1.y, c = q1.z, opacity = q1.w;
+    const float half_a = 0.5f * a, half_c = 0.5f * c;
+    const float limit = __builtin_fmaf(__builtin_amdgcn_logf(opacity) + kLog2Of255, kLn2, 0.01f);
+    const float u0 = box.x0 - q0.x, u1 = box.x1 - q0.x, v0 = box.y0 - q0.y, v1 = box.y1 - q0.y;
+    const float un = __builtin_amdgcn_fmed3f(0.0f, u0, u1), vn = __builtin_amdgcn_fmed3f(0.0f, v0, v1);
+    // along the nearest column, and along the nearest row
+    const float v = __builtin_amdgcn_fmed3f(-b * __builtin_amdgcn_rcpf(c) * un, v0, v1);
+    const float u = __builtin_amdgcn_fmed3f(-b * __builtin_amdgcn_rcpf(a) * vn, u0, u1);
+    const float qmin = fminf(v * (half_c * v + b * un) + half_a * un * un, u * (half_a * u + b * vn) + half_c * vn * vn);
+    // (below 1/255: no pixel takes it; a NaN opacity is kept)
+    return !(opacity < 1.0f / 255.0f) && !(a > 0.0f && c > 0.0f && qmin > limit);
+}
+
+// Which of a tile's blocks can this entry reach?  For each four rows of pixels the ellipse q <= limit takes up a range of
+// columns: its right and left extremes lie at v = -+ (b/c) umax (umax: the ellipse's half width) where those rows hold them and
+// at the nearest row otherwise.  The limit is the reach plus 0.01 and plus what q may be off by where its
+// terms are large and cancel (the determinant, too, is one rounding off its value, not off its terms); the range is
+// widened by 1/16 pixel.  All blocks for a degenerate conic or an entry without a limit.
+// (x0, y0: the tile's first pixel centre)
+__device__ __forceinline__ uint32_t blocks_reached(float mx, float my, float a, float b, float c, float reach, float x0, float y0)
+{
+    constexpr float kSlack = 1.0f / 64.0f; // in blocks
+    float det;
+    {
+#pragma clang fp contract(off)
+        const float bb = b * b;
+        det = __builtin_fmaf(a, c, -bb) - __builtin_fmaf(b, b, -bb);
+    }
+    const float u_first = x0 - mx, v_first = y0 - my;
+    const float u_far = fmaxf(fabsf(u_first), fabsf(u_first + (kTile - 1))), v_far = fmaxf(fabsf(v_first), fabsf(v_first + (kTile - 1)));
+    const float limit = reach + 0.01f + 2.5e-7f * (a * u_far * u_far + c * v_far * v_far);
+    const bool all = !(a > 0.0f && c > 0.0f && det > 1e-30f && limit < 1e30f);
+    const float two = 2.0f * limit, inv_a = __builtin_amdgcn_rcpf(a), per_det = two * __builtin_amdgcn_rcpf(det);
+    const float vmax = __builtin_amdgcn_sqrtf(a * per_det);
+    const float v_left = b * __builtin_amdgcn_rcpf(c) * __builtin_amdgcn_sqrtf(c * per_det); // (the right extreme: -v_left)
+    const float from = (u_first + 3.0f) * -0.25f - kSlack, to = u_first * -0.25f + (1.0f + kSlack);
+    const float quarter = 0.25f * inv_a;
+    uint32_t reached = 0;
 #pragma unroll
     for(int r = 0; r < 4; ++r)
-        if(channel < 3 && quad_x + r < W && y < H)
-            out[step * r] = broken ? __builtin_nanf("") : (planar ? __builtin_fmaf(quad_T[r], back, colour[r]) : colour[r]);
+    {
+        const float v0 = fmaxf(v_first + (float)(4 * r), -vmax), v1 = fminf(v_first + (float)(4 * r + 3), vmax);
+        const float vl = __builtin_amdgcn_fmed3f(v_left, v0, v1), vr = __builtin_amdgcn_fmed3f(-v_left, v0, v1);
+        const float left = __builtin_amdgcn_sqrtf(fmaxf(a * two - det * vl * vl, 0.0f)) + b * vl;
+        const float right = __builtin_amdgcn_sqrtf(fmaxf(a * two - det * vr * vr, 0.0f)) - b * vr;
+        // the first block that ends behind the left extreme, the first one that begins behind the right
+        const int first = (int)__builtin_amdgcn_fmed3f(ceilf(from - left * quarter), 0.0f, 4.0f);
+        const int behind = v0 <= v1 ? (int)__builtin_amdgcn_fmed3f(floorf(to + right * quarter), 0.0f, 4.0f) : 0;
+        reached |= ((1u << max(behind - first, 0)) - 1u) << (first + 4 * r);
+    }
+    return all ? 0xffffu : (reach >= 0.0f ? reached : 0u);
+}
+
+// The lists of a round, from which blocks the entry of every lane reaches: the places of the entries of each quad, in order, in
+// bytes that held kPlaces, nobody's place.  Returns the longest list's length.
+constexpr int kBatch = DSX_WAVE; // staged entries of a round
+template <int kPlaces>
+__device__ __forceinline__ int quad_lists(uint8_t* bytes, uint32_t reached, int lane)
+{
+    int longest = 0;
+#pragma unroll
+    for(int q = 0; q < kQuads; ++q)
+    {
+        const uint64_t m = __builtin_amdgcn_ballot_w64((reached & (1u << q)) != 0);
+        if(__builtin_amdgcn_inverse_ballot_w64(m))
+            bytes[__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, q * kPlaces))] = (uint8_t)lane;
+        longest = max(longest, (int)__popcll(m));
+    }
+    return longest;
+}
+
+// a pixel's colour: interleaved, or channel-first with the background composited
+__device__ __forceinline__ void store_pixel(float* image, int64_t pix, int64_t plane, float red, float green, float blue, float T,
+                                            bool broken, const float* bg, int planar)
+{
+    if(broken)
+        red = green = blue = __builtin_nanf("");
+    if(planar)
+    {
+        image[pix] = broken ? red : __builtin_fmaf(T, bg[0], red);
+        image[pix + plane] = broken ? green : __builtin_fmaf(T, bg[1], green);
+        image[pix + 2 * plane] = broken ? blue : __builtin_fmaf(T, bg[2], blue);
+    }
+    else
+    {
+        image[3 * pix] = red;
+        image[3 * pix + 1] = green;
+        image[3 * pix + 2] = blue;
+    }
 }
 
 // kBinned: the entries come out of the list of the tile's bin (BinLists).  The wavefront first
@@ -399,8 +451,10 @@ __device__ __forceinline__ void store_colours(float* image, const dsx_f32x4 colo
 // pixels do not saturate early, where every tile reads its bin's whole list, costs a few percent
 // more than with per-tile lists instead of twice as much.  final_idx still receives the
 // reference's index: the tile's range start plus the entry's rank among the tile's own entries.
+// (seven wavefronts per SIMD: 72 registers; with eight and 64 the walk waits for reloads, 500 K opaque 135 against 130 us, 6 M
+// at 4K 461 against 446; with six the last tiles of a 1080p image start late, 2 M faint 748 against 706)
 template <bool kBinned>
-__global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(8, 8))) void blend_fwd_kernel(const int32_t* __restrict__ ranges,
+__global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(7, 7))) void blend_fwd_kernel(const int32_t* __restrict__ ranges,
                                                              const int32_t* __restrict__ ids,
                                                              const float4* __restrict__ splats,
                                                              float* __restrict__ image, float* __restrict__ final_T,
@@ -414,19 +468,23 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(8, 8))
                                                              const float* __restrict__ bg, int planar,
                                                              const BinLists lists)
 {
-    // the last place is nobody's entry (no exponent passes): rows whose list has ended point at it
-    __shared__ float4 s_a[kFwdBatch + 1]; // pixel x, pixel y, conic -a/2, conic b
-    __shared__ float4 s_b[kFwdBatch + 1]; // conic c/2, opacity, limit of the exponent's bits, index in the sorted key array
-    __shared__ float s_c[3 * kFwdBatch + 4]; // red, green, blue
-    __shared__ uint64_t s_list[4 * kFwdBatch / 8 + 1]; // a byte per entry and row: its place (one word more than is used: read ahead)
-    __shared__ int s_queue[DSX_WAVE]; // ids of the tile's own entries, on their way from the scan to the gather
-    static_assert(kFwdBatch % 8 == 0 && kFwdBatch < 256 && kFwdBatch >= DSX_WAVE, "places are bytes, stored by words");
+    // the last place is nobody's entry (no exponent passes): quads whose list has ended point at it
+    __shared__ float4 s_a[kBatch + 1]; // pixel x, pixel y, conic -a/2, conic b
+    __shared__ float4 s_b[kBatch + 1]; // conic c/2, opacity, limit of the exponent's bits, index in the sorted key array
+    __shared__ float4 s_c[kBatch + 1]; // red, green, blue
+    __shared__ uint4 s_list[kQuads * kBatch / 16 + 1]; // a byte per entry and quad: its place (one word more than is used: read ahead)
+    __shared__ int2 s_left[kBatch]; // candidates (id, index) that did not fit the round
+    // while a round is staged, in the records' memory: the candidates, and ids of the tile's own entries on their way from
+    // the scan to the gather (the last place stays as it is)
+    int2* const s_cand = reinterpret_cast<int2*>(s_a);
+    int* const s_queue = reinterpret_cast<int*>(s_b);
+    static_assert(2 * kBatch * sizeof(int2) <= kBatch * sizeof(float4), "candidates fit the records' memory");
 
     const int lane = threadIdx.x;
-    const int row = lane >> 4;
-    const Pixels<kPix> px(blockIdx.x, ntx, lane);
-    const float pxf = (float)px.x + 0.5f;
-    uint8_t* const list_bytes = reinterpret_cast<uint8_t*>(s_list);
+    const int tile = blockIdx.x;
+    const int x0 = (tile % ntx) * kTile, y0 = (tile / ntx) * kTile;
+    const int x = x0 + (lane & 15), y = y0 + kPix * (lane >> 4); // this lane's column of four pixels
+    const float pxf = (float)x + 0.5f;
 
     // The lists are data from the device: positions are taken for what they are only inside
     // sorted_ids[0, k), and a `ranges` buffer that was built for another bin size (its header word,
@@ -438,14 +496,14 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(8, 8))
     if(kBinned)
     {
         if(layout_ok)
-            src = tile_source(lists, px.tile, ntx);
+            src = tile_source(lists, tile, ntx);
         start = src.start;
         end = src.end;
     }
     else if(layout_ok)
     {
-        start = ranges[px.tile];
-        end = ranges[px.tile + 1];
+        start = ranges[tile];
+        end = ranges[tile + 1];
     }
     start = min(max(start, 0), k);
     end = min(max(end, 0), k);
@@ -454,30 +512,23 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(8, 8))
     // exponent is then NaN, the test of it fails whatever the entry holds, and the loop
     // needs no per-pixel flag.  `alive` counts the wavefront's live pixels (a scalar: it is kept
     // from ballots, on the scalar unit, and costs the vector unit nothing).
-    float pyf[kPix], T[kPix];
-    // Colours: the matrix unit's 4x4x1 product in 16 blocks of four lanes adds weight (one pixel per lane)
-    // times (red, green, blue) of each block's own entry in ONE instruction where the vector unit
-    // takes three, with the same fused multiply-add per element.  Register r of lane 4 b + j then
-    // holds channel j of the pixel of lane 4 b + r.
-    dsx_f32x4 colour[kPix];
+    float pyf[kPix], T[kPix], red[kPix], green[kPix], blue[kPix];
     int last[kPix];
     int alive = 0;
 #pragma unroll
     for(int p = 0; p < kPix; ++p)
     {
-        const int y = px.y_of(p);
-        const bool inside = px.x < W && y < H;
-        pyf[p] = inside ? (float)y + 0.5f : __builtin_nanf("");
+        const bool inside = x < W && y + p < H;
+        pyf[p] = inside ? (float)(y + p) + 0.5f : __builtin_nanf("");
         alive += __popcll(__builtin_amdgcn_ballot_w64(inside));
         T[p] = 1.0f;
-        colour[p] = dsx_f32x4{0.f, 0.f, 0.f, 0.f};
+        red[p] = green[p] = blue[p] = 0.0f;
         last[p] = 0;
     }
     if(lane == 0)
     {
-        s_a[kFwdBatch] = make_float4(0.f, 0.f, 0.f, 0.f);
-        s_b[kFwdBatch] = make_float4(0.f, 0.f, __int_as_float(INT_MIN), 0.f);
-        s_c[3 * kFwdBatch] = s_c[3 * kFwdBatch + 1] = s_c[3 * kFwdBatch + 2] = s_c[3 * kFwdBatch + 3] = 0.f;
+        s_a[kBatch] = s_c[kBatch] = make_float4(0.f, 0.f, 0.f, 0.f);
+        s_b[kBatch] = make_float4(0.f, 0.f, __int_as_float(INT_MIN), 0.f);
     }
 
     // binned lists: the scan of the bin's list
@@ -486,24 +537,24 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(8, 8))
     int scan = start;  // next position of the list to look at
     int seen = 0;      // entries of the tile's own list found so far
     int index_next = kBinned ? src.fine_base : start; // what final_idx records for the next entry
-    while(alive != 0 && scan < end && (!kBinned || seen < src.count))
+    int left = 0;      // candidates that the last round left
+    while(alive != 0 && (left > 0 || (scan < end && (!kBinned || seen < src.count))))
     {
-        // rows with a live pixel
+        // blocks with a live pixel, and the box around them
         uint64_t live = 0;
 #pragma unroll
         for(int p = 0; p < kPix; ++p)
             live |= __builtin_amdgcn_ballot_w64(pyf[p] == pyf[p]);
-        uint32_t live_rows = 0;
-#pragma unroll
-        for(int r = 0; r < 4; ++r)
-            live_rows |= (live >> (16 * r)) & 0xffffull ? 1u << r : 0u;
+        const uint32_t live_blocks = quads_of(live, lane);
+        const LiveBox box = live_box(live_blocks, (float)x0 + 0.5f, (float)y0 + 0.5f);
 
         __syncthreads(); // single wavefront: orders the LDS reads of the last round before these writes
-        if(lane < 4 * kFwdBatch / 8)
-            s_list[lane] = 0x0101010101010101ull * kFwdBatch;
-        int staged = 0;
-        int length[4] = {0, 0, 0, 0};
-        do
+        constexpr uint32_t kNobodies = 0x01010101u * kBatch;
+        s_list[lane] = make_uint4(kNobodies, kNobodies, kNobodies, kNobodies);
+        int found = left;
+        if(lane < left)
+            s_cand[lane] = s_left[lane];
+        while(found < kBatch && scan < end && (!kBinned || seen < src.count))
         {
             int id = 0;
             int batch; // entries in this gather
@@ -552,6 +603,7 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(8, 8))
                 seen += batch;
                 __syncthreads();
                 id = s_queue[lane];
+                __syncthreads();
             }
             else
             {
@@ -560,101 +612,106 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(8, 8))
                     id = ids[scan + lane];
                 scan += batch;
             }
-            uint32_t reached = 0;
-            float4 q0, q1;
-            float reach = 0.0f;
-            const float4* const rec = splats + 3 * (int64_t)min((uint32_t)id, last_id);
+            bool reaches = false;
             if(lane < batch)
             {
                 // (an id is taken for what it is only up to the last Gaussian: lists that a failed sort or a
                 // caller's mix-up left in disorder then give a wrong image, not a fetch outside the records)
-                q0 = rec[0], q1 = rec[1];
-                reach = reach_of(q1.w);
-                reached = live_rows & blocks_reached<Pixels<kPix>::kSide>(q0.x, q0.y, q1.x, q1.y, q1.z, reach,
-                                                                             px.box_x, px.box_y);
+                id = (int)min((uint32_t)id, last_id);
+                const float4* const rec = splats + 3 * (int64_t)id;
+                reaches = box_reached(box, rec[0], rec[1]);
             }
-            const uint64_t m_any = __ballot(reached != 0);
-            const int place = staged + bits_below_lane(m_any);
-            if(reached != 0)
-            {
-                const float4 q2 = rec[2];
-                s_a[place] = make_float4(q0.x, q0.y, q1.x * -0.5f, q1.y);
-                s_b[place] = make_float4(q1.z * 0.5f, q1.w,
-                                         __int_as_float(reach_limit_fwd(q1.w, reach)),
-                                         __int_as_float(index_next + lane));
-                s_c[3 * place] = q2.x;
-                s_c[3 * place + 1] = q2.y;
-                s_c[3 * place + 2] = q2.z;
-            }
-#pragma unroll
-            for(int r = 0; r < 4; ++r)
-            {
-                const uint64_t m = __ballot((reached >> r) & 1);
-                if((reached >> r) & 1)
-                    list_bytes[r * kFwdBatch + length[r] + bits_below_lane(m)] = (uint8_t)place;
-                length[r] += __popcll(m);
-            }
-            staged += __popcll(m_any);
+            const uint64_t m = __builtin_amdgcn_ballot_w64(reaches);
+            if(reaches)
+                s_cand[found + bits_below_lane(m)] = make_int2(id, index_next + lane);
+            found += __popcll(m);
             index_next += batch;
-        } while(staged <= kFwdBatch - DSX_WAVE && scan < end && (!kBinned || seen < src.count));
+        }
+        __syncthreads();
+        const int staged = min(found, kBatch);
+        const int2 mine = s_cand[lane], spare = s_cand[kBatch + lane];
+        left = found - staged;
+        __syncthreads();
+        if(lane < left)
+            s_left[lane] = spare;
+        uint32_t reached = 0;
+        if(lane < staged)
+        {
+            const float4* const rec = splats + 3 * (int64_t)mine.x;
+            const float4 q0 = rec[0], q1 = rec[1], q2 = rec[2];
+            const float reach = reach_of(q1.w);
+            reached = live_blocks & blocks_reached(q0.x, q0.y, q1.x, q1.y, q1.z, reach, (float)x0 + 0.5f, (float)y0 + 0.5f);
+            s_a[lane] = make_float4(q0.x, q0.y, q1.x * -0.5f, q1.y);
+            s_b[lane] = make_float4(q1.z * 0.5f, q1.w, __int_as_float(reach_limit_fwd(q1.w, reach)), __int_as_float(mine.y));
+            s_c[lane] = q2;
+        }
+        const int rounds = quad_lists<kBatch>(reinterpret_cast<uint8_t*>(s_list), reached, lane);
         __syncthreads();
 
-        const int rounds = max(max(length[0], length[1]), max(length[2], length[3]));
-        const uint8_t* my_list = list_bytes + row * kFwdBatch;
-        int place = *my_list;
-        for(int i = 0; i < rounds; ++i)
+        // Two entries at a time, the transmittance going from T to U and back: a pixel that an entry makes opaque keeps the
+        // former (its copy costs nothing where, as nearly always, no pixel stops).
+        const uint16_t* my_list = reinterpret_cast<const uint16_t*>(s_list) + (lane >> 2) * (kBatch / 2);
+        int places = *my_list;
+        for(int i = 0; i < rounds; i += 2)
         {
             if(alive == 0)
                 break;
-            asm("" : "+v"(place)); // (a whole register, as loaded: no masking of the byte)
-            const float4 A = s_a[place];
-            const float4 B = s_b[place];
-            const float channel = s_c[3 * place + (lane & 3)]; // (the fourth lane's is not looked at)
-            const int limit = __float_as_int(B.z);
-            // what final_idx records for this entry: its position in the sorted key array (binned
-            // lists: the tile's range start plus the entry's rank among the tile's own entries)
-            const int entry_index = __float_as_int(B.w);
-            place = *++my_list;
-            const ExponentX ex = exponent_x(A.z, A.w, pxf - A.x);
-            float weight[kPix], Tn[kPix];
-            uint64_t m_pass[kPix], m_low[kPix], m_stop = 0;
-#pragma unroll
-            for(int p = 0; p < kPix; ++p)
-            {
-#pragma clang fp contract(off)
-                const float dy = pyf[p] - A.y;
-                const float power = __builtin_fmaf(-__builtin_fmaf(B.x, dy, ex.bx), dy, ex.ax);
-                // the decisions as wavefront masks (each is its compare's own result register),
-                // combined on the scalar unit and handed back to the lanes as conditions
-                m_pass[p] = __builtin_amdgcn_ballot_w64(__float_as_int(power) <= limit);
-                // (a NaN opacity gives 0.999, as in the reference: fminf drops the NaN)
-                const float alpha = fminf(kAlphaMax, B.y * __builtin_amdgcn_exp2f(power * kLog2E));
-                const float taken = __builtin_amdgcn_inverse_ballot_w64(m_pass[p]) ? alpha : 0.0f;
-                weight[p] = taken * T[p];
-                Tn[p] = __builtin_fmaf(-taken, T[p], T[p]); // (1 - alpha) T in one rounding
-                m_low[p] = __builtin_amdgcn_ballot_w64(Tn[p] < 0.0001f);
-                m_stop |= m_low[p];
-            }
-            if(m_stop != 0)
-            {
-                // pixels that this entry would make opaque stop without it
+            const int here = places;
+            places = *++my_list;
+            float U[kPix];
+            auto blend = [&](int place, const float (&before)[kPix], float (&after)[kPix]) {
+                const float4 A = s_a[place];
+                const float4 B = s_b[place];
+                const float4 C = s_c[place];
+                const int limit = __float_as_int(B.z);
+                // what final_idx records for this entry: its position in the sorted key array (binned
+                // lists: the tile's range start plus the entry's rank among the tile's own entries)
+                const int entry_index = __float_as_int(B.w);
+                const ExponentX ex = exponent_x(A.z, A.w, pxf - A.x);
+                float weight[kPix];
+                uint64_t m_pass[kPix], m_low[kPix], m_stop = 0;
 #pragma unroll
                 for(int p = 0; p < kPix; ++p)
                 {
-                    const bool stop = __builtin_amdgcn_inverse_ballot_w64(m_low[p]);
-                    weight[p] = stop ? 0.0f : weight[p];
-                    pyf[p] = stop ? __builtin_nanf("") : pyf[p];
-                    m_pass[p] &= ~m_low[p];
-                    alive -= __popcll(m_low[p]);
+#pragma clang fp contract(off)
+                    const float dy = pyf[p] - A.y;
+                    const float power = __builtin_fmaf(-__builtin_fmaf(B.x, dy, ex.bx), dy, ex.ax);
+                    // the decisions as wavefront masks (each is its compare's own result register),
+                    // combined on the scalar unit and handed back to the lanes as conditions
+                    m_pass[p] = __builtin_amdgcn_ballot_w64(__float_as_int(power) <= limit);
+                    // (a NaN opacity gives 0.999, as in the reference: fminf drops the NaN)
+                    const float alpha = fminf(kAlphaMax, B.y * __builtin_amdgcn_exp2f(power * kLog2E));
+                    const float taken = __builtin_amdgcn_inverse_ballot_w64(m_pass[p]) ? alpha : 0.0f;
+                    weight[p] = taken * before[p];
+                    after[p] = __builtin_fmaf(-taken, before[p], before[p]); // (1 - alpha) T in one rounding
+                    m_low[p] = __builtin_amdgcn_ballot_w64(after[p] < 0.0001f);
+                    m_stop |= m_low[p];
                 }
-            }
+                if(m_stop != 0)
+                {
+                    // pixels that this entry would make opaque stop without it
 #pragma unroll
-            for(int p = 0; p < kPix; ++p)
-            {
-                colour[p] = __builtin_amdgcn_mfma_f32_4x4x1f32(weight[p], channel, colour[p], 0, 0, 0);
-                T[p] = __builtin_amdgcn_inverse_ballot_w64(m_low[p]) ? T[p] : Tn[p];
-                last[p] = __builtin_amdgcn_inverse_ballot_w64(m_pass[p]) ? entry_index : last[p];
-            }
+                    for(int p = 0; p < kPix; ++p)
+                    {
+                        const bool stop = __builtin_amdgcn_inverse_ballot_w64(m_low[p]);
+                        weight[p] = stop ? 0.0f : weight[p];
+                        after[p] = stop ? before[p] : after[p];
+                        pyf[p] = stop ? __builtin_nanf("") : pyf[p];
+                        m_pass[p] &= ~m_low[p];
+                        alive -= __popcll(m_low[p]);
+                    }
+                }
+#pragma unroll
+                for(int p = 0; p < kPix; ++p)
+                {
+                    red[p] = __builtin_fmaf(weight[p], C.x, red[p]);
+                    green[p] = __builtin_fmaf(weight[p], C.y, green[p]);
+                    blue[p] = __builtin_fmaf(weight[p], C.z, blue[p]);
+                    last[p] = __builtin_amdgcn_inverse_ballot_w64(m_pass[p]) ? entry_index : last[p];
+                }
+            };
+            blend(here & 0xff, T, U);
+            blend(here >> 8, U, T);
         }
     }
 
@@ -663,22 +720,19 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(8, 8))
     const bool broken = !layout_ok || (sort_flag_a && *sort_flag_a) || (sort_flag_b && *sort_flag_b);
 #pragma unroll
     for(int p = 0; p < kPix; ++p)
-    {
-        const int y = px.y_of(p);
-        if(px.x < W && y < H)
+        if(x < W && y + p < H)
         {
-            const int64_t pix = (int64_t)y * W + px.x;
+            const int64_t pix = (int64_t)(y + p) * W + x;
             final_T[pix] = T[p];
             final_idx[pix] = last[p];
+            store_pixel(image, pix, (int64_t)W * H, red[p], green[p], blue[p], T[p], broken, bg, planar);
         }
-        store_colours(image, colour[p], T[p], px.x, y, W, H, lane, broken, bg, planar);
-    }
     if(kBinned && layout_ok)
     {
         // for the backward: where this wavefront's scan of the bin's list stopped and how many of the
         // tile's entries it had met by then (everything that any of its pixels blended lies below).
         // The tile's other six words are marked as empty.
-        int32_t* w = lists.walk + (int64_t)px.tile * 8;
+        int32_t* w = lists.walk + (int64_t)tile * 8;
         const int stopped = min(scan, end);
         if(lane < 8)
             w[lane] = lane == 0 ? stopped : (lane == 1 ? seen : (lane & 1 ? 0 : -1));
@@ -689,7 +743,7 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(8, 8))
 // -----------------------------------------------------------------------------------------
 // the same for images of few tiles: a workgroup of four wavefronts per tile
 // -----------------------------------------------------------------------------------------
-// When the tiles are too few to fill the chip, a wavefront per tile leaves most of it idle and takes as
+// When the tiles are too few to fill the chip, a wavefront per tile leaves much of it idle and takes as
 // long as its longest dependency chain.  Here four wavefronts share a tile: each owns a quadrant (its
 // rows of lanes the quadrant's four 4x4 blocks, one pixel per lane), the four stage a round
 // of up to kTileBatch entries together (each thread gathers and tests one candidate, against
@@ -777,7 +831,7 @@ __device__ __forceinline__ int tile_scan(TileScan& s, int* queue, const int32_t*
 
 // A wavefront's lists of one round: the places of the staged entries that reach each of its four blocks,
 // padded with the place that is nobody's.  Returns the longest list's length.
-__device__ __forceinline__ int build_lists(uint32_t* list_words, const uint16_t* reach, int staged, int wave, int lane)
+__device__ __forceinline__ int build_lists(uint32_t* list_words, const uint16_t* reach, int staged, int wave, int first_block, int lane)
 {
     uint8_t* const bytes = reinterpret_cast<uint8_t*>(list_words + wave * kTileBatch);
     for(int i = lane; i < kTileBatch; i += DSX_WAVE)
@@ -786,11 +840,11 @@ __device__ __forceinline__ int build_lists(uint32_t* list_words, const uint16_t*
     for(int first = 0; first < staged; first += DSX_WAVE)
     {
         const int place = first + lane;
-        const uint32_t mine = place < staged ? (uint32_t)reach[place] >> (4 * wave) : 0u;
+        const uint32_t mine = place < staged ? (uint32_t)reach[place] >> first_block : 0u;
 #pragma unroll
         for(int r = 0; r < 4; ++r)
         {
-            const uint64_t m = __builtin_amdgcn_ballot_w64((mine >> r) & 1);
+            const uint64_t m = __builtin_amdgcn_ballot_w64((mine >> block_of_row(r)) & 1);
             if(__builtin_amdgcn_inverse_ballot_w64(m))
                 bytes[r * kTileBatch + length[r] + bits_below_lane(m)] = (uint8_t)place;
             length[r] += __popcll(m);
@@ -834,8 +888,7 @@ __global__ __launch_bounds__(kTileThreads) void blend_fwd_tile_kernel(const int3
                                                                       const BinLists lists)
 {
     // (arrays as in the wavefront form)
-    __shared__ float4 s_a[kTileBatch + 1], s_b[kTileBatch + 1];
-    __shared__ float s_c[3 * kTileBatch + 4];
+    __shared__ float4 s_a[kTileBatch + 1], s_b[kTileBatch + 1], s_c[kTileBatch + 1];
     __shared__ uint16_t s_reach[kTileBatch]; // which of the tile's 16 blocks an entry reaches
     __shared__ uint32_t s_list[kTileWaves * kTileBatch];
     __shared__ int s_queue[kTileBatch];
@@ -846,7 +899,8 @@ __global__ __launch_bounds__(kTileThreads) void blend_fwd_tile_kernel(const int3
     const int tid = threadIdx.x, lane = tid & (DSX_WAVE - 1), row = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid / DSX_WAVE);
     const int tile = blockIdx.x;
-    const Pixels<1> px(4 * tile + wave, ntx, lane);
+    const int first_block = first_block_of(wave);
+    const Pixels px(tile, wave, ntx, lane);
     const float pxf = (float)px.x + 0.5f;
     const float tile_x = (float)(tile % ntx * kTile) + 0.5f, tile_y = (float)(tile / ntx * kTile) + 0.5f;
 
@@ -872,13 +926,12 @@ __global__ __launch_bounds__(kTileThreads) void blend_fwd_tile_kernel(const int3
     const bool inside = px.x < W && px.y < H;
     float pyf = inside ? (float)px.y + 0.5f : __builtin_nanf(""); // (NaN: stopped)
     float T = 1.0f;
-    dsx_f32x4 colour = {0.f, 0.f, 0.f, 0.f};
+    float red = 0.f, green = 0.f, blue = 0.f;
     int last = 0;
     if(tid == 0)
     {
-        s_a[kTileBatch] = make_float4(0.f, 0.f, 0.f, 0.f);
+        s_a[kTileBatch] = s_c[kTileBatch] = make_float4(0.f, 0.f, 0.f, 0.f);
         s_b[kTileBatch] = make_float4(0.f, 0.f, __int_as_float(INT_MIN), 0.f);
-        s_c[3 * kTileBatch] = s_c[3 * kTileBatch + 1] = s_c[3 * kTileBatch + 2] = s_c[3 * kTileBatch + 3] = 0.f;
     }
 
     const uint32_t tile_bits = kBinned ? tile_bits_of(src, lists.shift) << 16 : 0u;
@@ -895,9 +948,9 @@ __global__ __launch_bounds__(kTileThreads) void blend_fwd_tile_kernel(const int3
         uint32_t live_rows = 0;
 #pragma unroll
         for(int r = 0; r < 4; ++r)
-            live_rows |= (live >> (16 * r)) & 0xffffull ? 1u << r : 0u;
+            live_rows |= (live >> (16 * r)) & 0xffffull ? 1u << block_of_row(r) : 0u;
         if(lane == 0)
-            s_live[wave] = live_rows << (4 * wave);
+            s_live[wave] = live_rows << first_block;
         __syncthreads(); // (and the last round's entries have been walked)
         const uint32_t live_blocks = __builtin_amdgcn_readfirstlane(s_live[0] | s_live[1] | s_live[2] | s_live[3]);
         if(live_blocks == 0 || left <= 0 || (kBinned && seen >= src.count))
@@ -926,10 +979,7 @@ __global__ __launch_bounds__(kTileThreads) void blend_fwd_tile_kernel(const int3
             const float4* const rec = splats + 3 * (int64_t)min((uint32_t)id, last_id);
             q0 = rec[0], q1 = rec[1], q2 = rec[2];
             reach = reach_of(q1.w);
-#pragma unroll
-            for(int q = 0; q < 4; ++q)
-                reached |= blocks_reached<4>(q0.x, q0.y, q1.x, q1.y, q1.z, reach, tile_x + 8.0f * (q & 1), tile_y + 8.0f * (q >> 1)) << (4 * q);
-            reached &= live_blocks;
+            reached = live_blocks & blocks_reached(q0.x, q0.y, q1.x, q1.y, q1.z, reach, tile_x, tile_y);
         }
         int staged;
         const int place = tile_place(s_counts, __builtin_amdgcn_ballot_w64(reached != 0), staged);
@@ -938,9 +988,7 @@ __global__ __launch_bounds__(kTileThreads) void blend_fwd_tile_kernel(const int3
             s_a[place] = make_float4(q0.x, q0.y, q1.x * -0.5f, q1.y);
             s_b[place] = make_float4(q1.z * 0.5f, q1.w,
                                      __int_as_float(reach_limit_fwd(q1.w, reach)), __int_as_float(index_next + tid));
-            s_c[3 * place] = q2.x;
-            s_c[3 * place + 1] = q2.y;
-            s_c[3 * place + 2] = q2.z;
+            s_c[place] = q2;
             s_reach[place] = (uint16_t)reached;
         }
         index_next += batch;
@@ -948,13 +996,13 @@ __global__ __launch_bounds__(kTileThreads) void blend_fwd_tile_kernel(const int3
         if(live_rows == 0)
             continue; // (nothing left in this quadrant: the others' barriers are met)
 
-        const int rounds = (build_lists(s_list, s_reach, staged, wave, lane) + kFwdAtOnce - 1) / kFwdAtOnce;
+        const int rounds = (build_lists(s_list, s_reach, staged, wave, first_block, lane) + kFwdAtOnce - 1) / kFwdAtOnce;
         const uint32_t* my_list = s_list + wave * kTileBatch + row * (kTileBatch / 4);
         for(int i = 0; i < rounds; ++i)
         {
             const uint32_t places = my_list[i];
-            float4 A[kFwdAtOnce], B[kFwdAtOnce];
-            float channel[kFwdAtOnce], alpha[kFwdAtOnce], weight[kFwdAtOnce];
+            float4 A[kFwdAtOnce], B[kFwdAtOnce], C[kFwdAtOnce];
+            float alpha[kFwdAtOnce], weight[kFwdAtOnce];
             uint64_t m_pass[kFwdAtOnce];
 #pragma unroll
             for(int u = 0; u < kFwdAtOnce; ++u)
@@ -962,7 +1010,7 @@ __global__ __launch_bounds__(kTileThreads) void blend_fwd_tile_kernel(const int3
                 const uint32_t p = (places >> (8 * u)) & 0xffu;
                 A[u] = s_a[p];
                 B[u] = s_b[p];
-                channel[u] = s_c[3 * p + (lane & 3)];
+                C[u] = s_c[p];
             }
             float Tn = T;
 #pragma unroll
@@ -1006,7 +1054,9 @@ __global__ __launch_bounds__(kTileThreads) void blend_fwd_tile_kernel(const int3
 #pragma unroll
             for(int u = 0; u < kFwdAtOnce; ++u)
             {
-                colour = __builtin_amdgcn_mfma_f32_4x4x1f32(weight[u], channel[u], colour, 0, 0, 0);
+                red = __builtin_fmaf(weight[u], C[u].x, red);
+                green = __builtin_fmaf(weight[u], C[u].y, green);
+                blue = __builtin_fmaf(weight[u], C[u].z, blue);
                 last = __builtin_amdgcn_inverse_ballot_w64(m_pass[u]) ? __float_as_int(B[u].w) : last;
             }
         }
@@ -1018,8 +1068,8 @@ __global__ __launch_bounds__(kTileThreads) void blend_fwd_tile_kernel(const int3
         const int64_t pix = (int64_t)px.y * W + px.x;
         final_T[pix] = T;
         final_idx[pix] = last;
+        store_pixel(image, pix, (int64_t)W * H, red, green, blue, T, broken, bg, planar);
     }
-    store_colours(image, colour, T, px.x, px.y, W, H, lane, broken, bg, planar);
     if(kBinned && layout_ok && tid < 8)
     {
         // (as in the wavefront form, which speaks for the whole tile too)
@@ -1120,6 +1170,34 @@ __device__ __forceinline__ float row_sum(float v)
     return v;
 }
 
+__host__ __device__ constexpr int block_lane(int block) { return 16 * (block / 4) + block % 4; } // (the first one)
+
+// Sums of eight values over the four lanes of a block (lanes four apart in a row), as a reduce-scatter with the DPP's bank masks, which
+// choose the lanes of an add for free: 12 instructions.  Lane l gets the sums of v[2 * bit 2 of l + bit 3 of l] and of the one four further.
+// (s_nop: as in row_sum8_scatter.)
+__device__ __forceinline__ void bank_sum8_scatter(const float (&v)[8], float& first, float& second)
+{
+    float s0, s1, s2, s3;
+    asm("s_nop 1\n\t"
+        "v_add_f32_dpp %0, %4, %4 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+        "v_add_f32_dpp %1, %6, %6 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+        "v_add_f32_dpp %2, %8, %8 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+        "v_add_f32_dpp %3, %10, %10 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+        "v_add_f32_dpp %0, %5, %5 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %1, %7, %7 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %2, %9, %9 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %3, %11, %11 row_ror:8 row_mask:0xf bank_mask:0xc"
+        : "=&v"(s0), "=&v"(s1), "=&v"(s2), "=&v"(s3)
+        : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]), "v"(v[5]), "v"(v[6]), "v"(v[7]));
+    asm("s_nop 1\n\t"
+        "v_add_f32_dpp %0, %2, %2 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
+        "v_add_f32_dpp %1, %4, %4 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
+        "v_add_f32_dpp %0, %3, %3 row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
+        "v_add_f32_dpp %1, %5, %5 row_shr:4 row_mask:0xf bank_mask:0xa"
+        : "=&v"(first), "=&v"(second)
+        : "v"(s0), "v"(s1), "v"(s2), "v"(s3));
+}
+
 // Eight values at once as a reduce-scatter.  A step takes two registers into one: the lanes of one half
 // keep the first value and add their partner's share of it, the other half the second.  The
 // DPP bank mask (banks of four lanes) chooses the lanes of an add for free where the halves are whole banks,
@@ -1163,77 +1241,95 @@ __device__ __forceinline__ float row_sum8_scatter(const float (&v)[8], int lane)
 // in a third of a cycle per lane where a float takes three (36 lanes: 11 cycles against 109, of a unit
 // that the compute unit's wavefronts share).
 constexpr int kSums = 9;
-constexpr int kBwdBatch = 80; // staged entries of a round: 10 KB of LDS with their sums, 16 wavefronts per compute unit
+constexpr float kAlphaMaxBwd = 0.99f;
+// Where the sums of a place lie: four and four of each place side by side, then the ninths.  An add serves 16 lanes at a time
+// over 16 doubles: four rows' or blocks' lots of four meet only where their places are the same or a multiple of four apart (nine
+// doubles side by side: with 7 of 16 of all other places).
+template <int kPlaces>
+__host__ __device__ constexpr int sum_at(int place, int slot)
+{
+    return slot == 8 ? 8 * kPlaces + place : 4 * (slot & 4 ? kPlaces + place : place) + (slot & 3);
+}
+// staged entries of a round: 7.5 KB of LDS with their sums, 20 wavefronts per compute unit (64 entries and 16 wavefronts: 2 M
+// faint Gaussians 1353 -> 1430 us; 12: 1545, 8: 1815)
+constexpr int kBwdBatch = 56;
 
 // An entry's sums in LDS, from the moments of w = vis v_alpha over its pixels (vis = exp(-sigma), and v_sigma =
 // -opacity w) to the gradients: v_x = sum of v_sigma (a dx + b dy) with d = mean - pixel (v_sigma and d both change
 // sign), ...; v_opacity is the sum of w itself
-__device__ __forceinline__ void moments_to_gradients(double* m, const float4 A, const float4 B)
+template <int kPlaces>
+__device__ __forceinline__ void moments_to_gradients(double* sums, int place, const float4 A, const float4 B, uint8_t* mark)
 {
+    double* const m = sums + 4 * place;
+    double* const n = m + 4 * kPlaces;
     const float half_a = A.z, b = A.w, half_c = B.x;
     const double opacity = (double)B.y;
     // (a sum that is zero stays so whatever the opacity: an infinite or NaN one of an entry that no pixel took)
     auto scaled = [&](double v) { return v != 0.0 ? opacity * v : 0.0; };
-    const double w = m[0], wx = m[1], wxx = m[2], wy = m[3], wxy = m[4], wyy = m[5];
+    const double w = m[0], wx = m[1], wxx = m[2], wy = m[3], wxy = n[0], wyy = n[1];
+    const bool any = w != 0.0 || n[2] != 0.0 || n[3] != 0.0 || sums[8 * kPlaces + place] != 0.0 || wx != 0.0 || wxx != 0.0 ||
+                     wy != 0.0 || wxy != 0.0 || wyy != 0.0;
+    if(any && mark)
+        *mark = 1;
     m[0] = scaled((double)(2.0f * half_a) * wx + (double)b * wy);
     m[1] = scaled((double)b * wx + (double)(2.0f * half_c) * wy);
     m[2] = scaled(-0.5 * wxx);
     m[3] = scaled(-wxy);
-    m[4] = scaled(-0.5 * wyy);
-    m[5] = w;
+    n[0] = scaled(-0.5 * wyy);
+    n[1] = w;
 }
-// One set of hardware float atomics per entry and round, and none where no pixel was valid
-__device__ __forceinline__ void flush_sums(const double* sums, const int* ids, int staged, float* grads, uint8_t* marks,
-                                           int tid, int threads)
+// One set of hardware float atomics per entry and round, and none where no pixel was valid: nine threads for each entry (those
+// that are over sit out: a record's adds leave in one instruction, which takes the memory one or two requests; requests to a
+// line that every tile adds to wait 13 ns for each other).
+template <int kPlaces>
+__device__ __forceinline__ void flush_sums(const double* sums, const int* ids, int ids_step, int staged, float* grads, int tid, int threads)
 {
-    for(int i = tid; i < staged * kSums; i += threads)
-    {
-        const float v = (float)sums[i];
-        if(v != 0.0f)
+    const int at_once = threads / kSums, slot = tid % kSums;
+    if(tid < at_once * kSums)
+        for(int e = tid / kSums; e < staged; e += at_once)
         {
-            const int e = i / kSums;
-            const int64_t id = ids[e];
-            unsafeAtomicAdd(grads + id * DSX_GRAD_FLOATS + (i - e * kSums), v);
-            if(marks)
-                marks[id] = 1;
+            const float v = (float)sums[sum_at<kPlaces>(e, slot)];
+            if(v != 0.0f)
+                unsafeAtomicAdd(grads + (int64_t)ids[ids_step * e] * DSX_GRAD_FLOATS + slot, v);
         }
-    }
 }
 
-// Same shape as the forward: four rows of lanes, each with its block of pixels and its own list of the
+// Same shape as the forward: sixteen quads of lanes, each with its block of pixels and its own list of the
 // entries that reach it, back to front from the last entry that any pixel blended.
-// The per-Gaussian gradients are first summed over a lane's four pixels, then over the row's
-// 16 lanes with DPP adds, all four rows' entries at once, and ONE atomic instruction carries the nine
-// sums of up to four entries.
+// The per-Gaussian gradients are first summed over a lane's four pixels, then over the quad's four lanes, all
+// sixteen quads' entries at once, then in LDS over the quads.
 // kBinned: the entries come out of the list of the tile's bin, filtered into a queue as in the forward
 // but downwards; the forward left, per tile, the bin-list position where its scan stopped and
 // the number of the tile's entries it had met by then, from which every entry met on the way down
 // gets its index in the sorted key array (final_idx is compared with those).
 template <bool kBinned>
-__global__ __launch_bounds__(DSX_WAVE) void blend_bwd_kernel(
+__global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(5, 5))) void blend_bwd_kernel(
     const int32_t* __restrict__ ranges, const int32_t* __restrict__ ids, const float4* __restrict__ splats,
     const float* __restrict__ final_T, const int32_t* __restrict__ final_idx, const float* __restrict__ v_image,
     const float* __restrict__ bg, float* grads, uint8_t* marks, int W, int H, int ntx, uint32_t last_id, int k,
     const int32_t* __restrict__ header, int header_shift, int planar, const BinLists lists, const ZeroJobs zeros)
 {
-    // (the last place: nobody's entry, as in the forward)
-    __shared__ float4 s_a[kBwdBatch + 1]; // pixel x, pixel y, conic a/2, conic b
-    __shared__ float4 s_b[kBwdBatch + 1]; // conic c/2, opacity, limit of sigma's bits, index in the sorted key array
-    __shared__ float s_c[3 * (kBwdBatch + 1)]; // red, green, blue
-    __shared__ int s_id[kBwdBatch];
-    __shared__ double s_sum[(kBwdBatch + 1) * kSums];
-    __shared__ uint64_t s_list[4 * kBwdBatch / 8 + 1];
-    // ids of the tile's own entries, on their way from the scan to the gather: in the sums' memory, which is
-    // free while a round is staged
-    int* const s_queue = reinterpret_cast<int*>(s_sum);
-    static_assert(kBwdBatch % 8 == 0 && kBwdBatch < 256 && 4 * kBwdBatch / 8 <= DSX_WAVE, "places are bytes, stored by words");
+    __shared__ float4 s_records[3 * kBwdBatch + 1];
+    float4* const s_a = s_records;                 // pixel x, pixel y, conic a/2, conic b
+    float4* const s_c = s_records + kBwdBatch;     // red, green, blue, the Gaussian's id
+    float4* const s_b = s_records + 2 * kBwdBatch; // conic c/2, opacity, limit of sigma's bits, index in the sorted key array
+                                                   // (and one more: nobody's entry, as in the forward)
+    __shared__ double s_sum[kBwdBatch * kSums + 1]; // (nobody's zeros are added to others' sums)
+    __shared__ uint4 s_list[kQuads * kBwdBatch / 16 + 1];
+    // while a round is staged, in the records' memory: candidates and the scan's queue, as in the forward
+    int2* const s_cand = reinterpret_cast<int2*>(s_records);
+    int* const s_queue = reinterpret_cast<int*>(s_records + DSX_WAVE);
+    static_assert(DSX_WAVE + DSX_WAVE / 4 <= 3 * kBwdBatch && kBwdBatch % 2 == 0 && (kQuads * kBwdBatch) % 16 == 0 &&
+                      kQuads * kBwdBatch / 16 <= DSX_WAVE, "what the records' memory holds; lists of pairs of bytes, cleared by words");
 
     const int lane = threadIdx.x;
-    const int row = lane >> 4;
-    const Pixels<kPix> px(blockIdx.x, ntx, lane);
-    const float pxf = (float)px.x + 0.5f;
+    const int tile = blockIdx.x;
+    const int x0 = (tile % ntx) * kTile, y0 = (tile / ntx) * kTile;
+    // this lane's column of four pixels: a row of lanes has a row of four blocks, lanes four apart the columns of a block
+    const int block = 4 * (lane >> 4) + (lane & 3);
+    const int x = x0 + 4 * (lane & 3) + ((lane >> 2) & 3), y = y0 + kPix * (lane >> 4);
+    const float pxf = (float)x + 0.5f;
     const float bg0 = bg[0], bg1 = bg[1], bg2 = bg[2];
-    uint8_t* const list_bytes = reinterpret_cast<uint8_t*>(s_list);
 
     // bterm = -T_final * (bg . v_out) - sum over the entries behind of (rgb . v_out) * alpha * T:
     // the three per-channel colour buffers of cpp/gsplat/backward.cu:156-168 only ever appear
@@ -1241,14 +1337,13 @@ __global__ __launch_bounds__(DSX_WAVE) void blend_bwd_kernel(
     const int64_t step = planar ? 1 : 3, plane = planar ? (int64_t)W * H : 1; // of v_image: between pixels, between channels
     float pyf[kPix], T[kPix], vo0[kPix], vo1[kPix], vo2[kPix], bterm[kPix];
     int bin_final[kPix];
-    int m = -1;
+    int m_quad = -1;
 #pragma unroll
     for(int p = 0; p < kPix; ++p)
     {
-        const int y = px.y_of(p);
-        const bool inside = px.x < W && y < H;
-        const int64_t pix = inside ? (int64_t)y * W + px.x : 0;
-        pyf[p] = (float)y + 0.5f;
+        const bool inside = x < W && y + p < H;
+        const int64_t pix = inside ? (int64_t)(y + p) * W + x : 0;
+        pyf[p] = (float)(y + p) + 0.5f;
         const float Tf = inside ? final_T[pix] : 0.0f;
         T[p] = Tf;
         bin_final[p] = inside ? final_idx[pix] : -1;
@@ -1256,24 +1351,21 @@ __global__ __launch_bounds__(DSX_WAVE) void blend_bwd_kernel(
         vo1[p] = inside ? v_image[step * pix + plane] : 0.f;
         vo2[p] = inside ? v_image[step * pix + 2 * plane] : 0.f;
         bterm[p] = -Tf * (bg0 * vo0[p] + bg1 * vo1[p] + bg2 * vo2[p]);
-        m = max(m, bin_final[p]);
+        m_quad = max(m_quad, bin_final[p]);
     }
 
-    // last entry (as an index in the sorted key array) that any pixel of each row, of the wavefront, blended
+    // last entry (as an index in the sorted key array) that any pixel of each block, of the wavefront, blended
+    m_quad = max(m_quad, __shfl_xor(m_quad, 4, DSX_WAVE));
+    m_quad = max(m_quad, __shfl_xor(m_quad, 8, DSX_WAVE));
+    int m = m_quad;
 #pragma unroll
-    for(int o = 8; o > 0; o >>= 1)
+    for(int o = 1; o < DSX_WAVE; o = o == 2 ? 16 : 2 * o)
         m = max(m, __shfl_xor(m, o, DSX_WAVE));
-    int m_row[4];
-#pragma unroll
-    for(int r = 0; r < 4; ++r)
-        m_row[r] = __builtin_amdgcn_readlane(m, 16 * r);
-    m = max(max(m_row[0], m_row[1]), max(m_row[2], m_row[3]));
+    m = __builtin_amdgcn_readfirstlane(m);
     if(lane == 0)
     {
-        // (its index, the largest there is, lies behind every pixel's last entry: no pixel takes it)
-        s_a[kBwdBatch] = make_float4(0.f, 0.f, 0.f, 0.f);
-        s_b[kBwdBatch] = make_float4(0.f, 0.f, 0.f, __int_as_float(INT_MAX));
-        s_c[3 * kBwdBatch] = s_c[3 * kBwdBatch + 1] = s_c[3 * kBwdBatch + 2] = 0.f;
+        // (whatever stands in the other two words, its sigma is NaN: no pixel takes it)
+        s_b[kBwdBatch] = make_float4(__builtin_nanf(""), 0.f, 0.f, __int_as_float(INT_MAX));
     }
 
     // lists that were built for another bin size than this launch assumes are not read (see the forward)
@@ -1292,10 +1384,10 @@ __global__ __launch_bounds__(DSX_WAVE) void blend_bwd_kernel(
         // that was blended lies below, and the entries are taken from there downwards.  An entry's
         // index is the tile's range start plus its rank; those above the last blended one (m) are
         // not even queued, so the entries that are handed on have consecutive indices.
-        src = tile_source(lists, px.tile, ntx);
+        src = tile_source(lists, tile, ntx);
         my_bits = tile_bits_of(src, lists.shift) << 16;
         start = max(src.start, 0);
-        const int32_t* w = lists.walk + (int64_t)px.tile * 8;
+        const int32_t* w = lists.walk + (int64_t)tile * 8;
         const int stopped = max(max(w[0], w[2]), max(w[4], w[6]));
         const int seen = max(max(w[1], w[3]), max(w[5], w[7]));
         // (positions outside sorted_ids are not followed, as in the forward)
@@ -1309,27 +1401,43 @@ __global__ __launch_bounds__(DSX_WAVE) void blend_bwd_kernel(
     }
     else if(layout_ok)
     {
-        start = max(ranges[px.tile], 0);
-        const int end = min(ranges[px.tile + 1], k);
+        start = max(ranges[tile], 0);
+        const int end = min(ranges[tile + 1], k);
         pos = min(end - 1, m);
         idx_next = pos;
     }
 
-    // where this lane's share of an entry's nine sums goes: lanes 0 and 1 of every bank hold the eight totals
-    // of the reduce-scatter (twice: lanes 2 and 3 too), lane 2 of a row takes the ninth
-    const bool carries_blue = (lane & 15) == 2;
-    const bool carries = (lane & 2) == 0 || carries_blue;
-    const int sum_slot = carries_blue ? 8 : 4 * (lane & 1) + 2 * ((lane >> 2) & 1) + ((lane >> 3) & 1);
+    double* const my_sums = s_sum + 2 * ((lane >> 2) & 1) + ((lane >> 3) & 1); // (see bank_sum8_scatter)
+    // Entries up to the smallest last one are behind no pixel's.  (A pixel that blended nothing at all takes no part: its row coordinate
+    // is NaN, and no exponent of it passes.)
+    const int first_index = kBinned ? src.fine_base : start;
+    int m_least = INT_MAX;
+#pragma unroll
+    for(int p = 0; p < kPix; ++p)
+    {
+        const bool none = bin_final[p] < first_index;
+        pyf[p] = none ? __builtin_nanf("") : pyf[p];
+        m_least = none ? m_least : min(m_least, bin_final[p]);
+    }
+#pragma unroll
+    for(int o = 1; o < DSX_WAVE; o <<= 1)
+        m_least = min(m_least, __shfl_xor(m_least, o, DSX_WAVE));
+    m_least = __builtin_amdgcn_readfirstlane(m_least);
 
+    const LiveBox box = {(float)x0 + 0.5f, (float)x0 + 15.5f, (float)y0 + 0.5f, (float)y0 + 15.5f};
     const int32_t* const keys = ids + k; // the pairs' key words lie behind the ids (binned lists)
-    while(pos >= start && (!kBinned || left > 0))
+    int2 spare = make_int2(0, 0);        // candidates that the last round left, and their number
+    int spares = 0;
+    while(spares > 0 || (pos >= start && (!kBinned || left > 0)))
     {
         __syncthreads(); // single wavefront: orders the LDS reads of the last round before these writes
-        if(lane < 4 * kBwdBatch / 8)
-            s_list[lane] = 0x0101010101010101ull * kBwdBatch;
-        int staged = 0;
-        int length[4] = {0, 0, 0, 0};
-        do
+        constexpr uint32_t kNobodies = 0x01010101u * kBwdBatch;
+        if(lane < kQuads * kBwdBatch / 16)
+            s_list[lane] = make_uint4(kNobodies, kNobodies, kNobodies, kNobodies);
+        int found = spares;
+        if(lane < spares)
+            s_cand[lane] = spare;
+        while(found < kBwdBatch && pos >= start && (!kBinned || left > 0))
         {
             int id = 0;
             int batch; // entries in this gather
@@ -1384,6 +1492,7 @@ __global__ __launch_bounds__(DSX_WAVE) void blend_bwd_kernel(
                 left -= batch;
                 __syncthreads();
                 id = s_queue[lane];
+                __syncthreads();
             }
             else
             {
@@ -1392,122 +1501,137 @@ __global__ __launch_bounds__(DSX_WAVE) void blend_bwd_kernel(
                     id = ids[pos - lane];
                 pos -= batch;
             }
-            uint32_t reached = 0;
-            float4 q0, q1, q2;
-            float reach = 0.0f;
-            const int idx = idx_next - lane;
+            bool reaches = false;
             if(lane < batch)
             {
                 id = (int)min((uint32_t)id, last_id); // (as in the forward)
-                const float4* rec = splats + 3 * (int64_t)id;
-                q0 = rec[0], q1 = rec[1], q2 = rec[2];
-                reach = reach_of(q1.w);
-                reached = blocks_reached<Pixels<kPix>::kSide>(q0.x, q0.y, q1.x, q1.y, q1.z, reach, px.box_x, px.box_y);
-#pragma unroll
-                for(int r = 0; r < 4; ++r)
-                    if(idx > m_row[r]) // behind everything that the row's pixels blended
-                        reached &= ~(1u << r);
+                const float4* const rec = splats + 3 * (int64_t)id;
+                reaches = box_reached(box, rec[0], rec[1]);
             }
-            const uint64_t m_any = __ballot(reached != 0);
-            const int place = staged + bits_below_lane(m_any);
-            if(reached != 0)
-            {
-                s_a[place] = make_float4(q0.x, q0.y, q1.x * 0.5f, q1.y);
-                s_b[place] = make_float4(q1.z * 0.5f, q1.w, __uint_as_float(reach_limit_bwd(q1.w, reach)),
-                                         __int_as_float(idx));
-                s_c[3 * place] = q2.x;
-                s_c[3 * place + 1] = q2.y;
-                s_c[3 * place + 2] = q2.z;
-                s_id[place] = id;
-            }
-#pragma unroll
-            for(int r = 0; r < 4; ++r)
-            {
-                const uint64_t mr = __ballot((reached >> r) & 1);
-                if((reached >> r) & 1)
-                    list_bytes[r * kBwdBatch + length[r] + bits_below_lane(mr)] = (uint8_t)place;
-                length[r] += __popcll(mr);
-            }
-            staged += __popcll(m_any);
+            const uint64_t m = __builtin_amdgcn_ballot_w64(reaches);
+            if(reaches)
+                s_cand[found + bits_below_lane(m)] = make_int2(id, idx_next - lane);
+            found += __popcll(m);
             idx_next -= batch;
-        } while(staged <= kBwdBatch - DSX_WAVE && pos >= start && (!kBinned || left > 0));
+        }
         __syncthreads();
-        for(int i = lane; i < staged * kSums; i += DSX_WAVE)
+        const int staged = min(found, kBwdBatch);
+        const int2 mine = s_cand[lane];
+        spare = s_cand[kBwdBatch + lane];
+        spares = found - staged;
+        __syncthreads();
+        uint32_t reached = 0;
+        bool special = false;
+        if(lane < staged)
+        {
+            const float4* const rec = splats + 3 * (int64_t)mine.x;
+            const float4 q0 = rec[0], q1 = rec[1], q2 = rec[2];
+            const float reach = reach_of(q1.w);
+            special = mine.y > m_least || !(q1.w <= kAlphaMaxBwd);
+            reached = blocks_reached(q0.x, q0.y, q1.x, q1.y, q1.z, reach, (float)x0 + 0.5f, (float)y0 + 0.5f);
+            s_a[lane] = make_float4(q0.x, q0.y, q1.x * 0.5f, q1.y);
+            s_b[lane] = make_float4(q1.z * 0.5f, q1.w, __uint_as_float(reach_limit_bwd(q1.w, reach)), __int_as_float(mine.y));
+            s_c[lane] = make_float4(q2.x, q2.y, q2.z, __int_as_float(mine.x));
+        }
+        // (entries behind everything that a quad's pixels blended are not in its list)
+#pragma unroll
+        for(int q = 0; q < kQuads; ++q)
+            if(mine.y > __builtin_amdgcn_readlane(m_quad, block_lane(q)))
+                reached &= ~(1u << q);
+        const int rounds = quad_lists<kBwdBatch>(reinterpret_cast<uint8_t*>(s_list), reached, lane);
+        for(int i = lane; i < kBwdBatch * kSums; i += DSX_WAVE)
             s_sum[i] = 0.0;
         __syncthreads();
 
-        const int rounds = max(max(length[0], length[1]), max(length[2], length[3]));
-        const uint8_t* my_list = list_bytes + row * kBwdBatch;
-        int place = *my_list;
-        for(int i = 0; i < rounds; ++i)
+        // (plain: no pixel's last entry lies among these, and no alpha reaches the clamp: two of 36 instructions a pixel and entry;
+        // 2 M faint Gaussians 1368 -> 1335 us, 1.4 M at 1557x1038 508 -> 493)
+        auto walk = [&](auto plain) {
+        const uint16_t* my_list = reinterpret_cast<const uint16_t*>(s_list) + block * (kBwdBatch / 2);
+        int places = *my_list;
+        for(int i = 0; i < rounds; i += 2)
         {
-            asm("" : "+v"(place)); // (a whole register, as loaded: no masking of the byte)
-            const float4 A = s_a[place];
-            const float4 B = s_b[place];
-            const float red = s_c[3 * place], green = s_c[3 * place + 1], blue = s_c[3 * place + 2];
-            const uint32_t limit = __float_as_uint(B.z);
-            const int idx = __float_as_int(B.w);
-            double* const sums = s_sum + place * kSums + sum_slot;
-            place = *++my_list;
-            // sigma exactly as the forward computed it
-            const float dx = pxf - A.x;
-            const ExponentX ex = exponent_x(A.z, A.w, dx);
-            float vis[kPix], alpha[kPix], dy[kPix]; // dy = pixel - mean
-            // which lanes' pixel p takes part: wavefront masks (each compare's own result register),
-            // combined on the scalar unit
-            uint64_t m_valid[kPix];
-            uint64_t m_any = 0;
+            const int here = places;
+            places = *++my_list;
 #pragma unroll
-            for(int p = 0; p < kPix; ++p)
+            for(int u = 0; u < 2; ++u)
             {
-#pragma clang fp contract(off)
-                dy[p] = pyf[p] - A.y;
-                const float sigma = __builtin_fmaf(__builtin_fmaf(B.x, dy[p], ex.bx), dy[p], ex.ax);
-                m_valid[p] = __builtin_amdgcn_ballot_w64(idx <= bin_final[p]) &
-                             __builtin_amdgcn_ballot_w64(__float_as_uint(sigma) <= limit);
-                m_any |= m_valid[p];
-                vis[p] = __builtin_amdgcn_exp2f(-sigma * kLog2E);
-                alpha[p] = fminf(0.99f, B.y * vis[p]);
-            }
-            if(m_any == 0)
-                continue;
-            // Per lane, over its pixels (which share dx): the weights of the colour's gradient, and three
-            // moments over dy of w = vis * v_alpha
-            float v_red = 0.f, v_green = 0.f, v_blue = 0.f, S0 = 0.f, S1 = 0.f, S2 = 0.f;
+                const int place = u == 0 ? here & 0xff : here >> 8;
+                const float4 A = s_a[place];
+                const float4 B = s_b[place];
+                const float4 C = s_c[place];
+                const uint32_t limit = __float_as_uint(B.z);
+                const int idx = __float_as_int(B.w);
+                // sigma exactly as the forward computed it
+                const float dx = pxf - A.x;
+                const ExponentX ex = exponent_x(A.z, A.w, dx);
+                float vis[kPix], alpha[kPix], dy[kPix]; // dy = pixel - mean
+                // which lanes' pixel p takes part: wavefront masks (each compare's own result register),
+                // combined on the scalar unit
+                uint64_t m_valid[kPix];
+                uint64_t m_any = 0;
 #pragma unroll
-            for(int p = 0; p < kPix; ++p)
-            {
-                if(__builtin_amdgcn_inverse_ballot_w64(m_valid[p]))
+                for(int p = 0; p < kPix; ++p)
                 {
-                    const float ra = __builtin_amdgcn_rcpf(1.0f - alpha[p]);
-                    T[p] *= ra;
-                    const float fac = alpha[p] * T[p];
-                    v_red += fac * vo0[p];
-                    v_green += fac * vo1[p];
-                    v_blue += fac * vo2[p];
-                    const float rv = red * vo0[p] + green * vo1[p] + blue * vo2[p];
-                    const float v_alpha = rv * T[p] + bterm[p] * ra;
-                    bterm[p] -= rv * fac;
-                    const float w = vis[p] * v_alpha;
-                    const float wdy = w * dy[p];
-                    S0 += w;
-                    S1 += wdy;
-                    S2 += wdy * dy[p];
+#pragma clang fp contract(off)
+                    dy[p] = pyf[p] - A.y;
+                    const float sigma = __builtin_fmaf(__builtin_fmaf(B.x, dy[p], ex.bx), dy[p], ex.ax);
+                    m_valid[p] = __builtin_amdgcn_ballot_w64(__float_as_uint(sigma) <= limit);
+                    if(!plain)
+                        m_valid[p] &= __builtin_amdgcn_ballot_w64(idx <= bin_final[p]);
+                    m_any |= m_valid[p];
+                    vis[p] = __builtin_amdgcn_exp2f(-sigma * kLog2E);
+                    alpha[p] = plain ? B.y * vis[p] : fminf(kAlphaMaxBwd, B.y * vis[p]);
                 }
+                if(m_any == 0)
+                    continue;
+                // Per lane, over its pixels (which share dx): the weights of the colour's gradient, and three
+                // moments over dy of w = vis * v_alpha
+                float v_red = 0.f, v_green = 0.f, v_blue = 0.f, S0 = 0.f, S1 = 0.f, S2 = 0.f;
+#pragma unroll
+                for(int p = 0; p < kPix; ++p)
+                {
+                    if(__builtin_amdgcn_inverse_ballot_w64(m_valid[p]))
+                    {
+                        const float ra = __builtin_amdgcn_rcpf(1.0f - alpha[p]);
+                        T[p] *= ra;
+                        const float fac = alpha[p] * T[p];
+                        v_red += fac * vo0[p];
+                        v_green += fac * vo1[p];
+                        v_blue += fac * vo2[p];
+                        const float rv = C.x * vo0[p] + C.y * vo1[p] + C.z * vo2[p];
+                        const float v_alpha = rv * T[p] + bterm[p] * ra;
+                        bterm[p] -= rv * fac;
+                        const float w = vis[p] * v_alpha;
+                        const float wdy = w * dy[p];
+                        S0 += w;
+                        S1 += wdy;
+                        S2 += wdy * dy[p];
+                    }
+                }
+                // what is summed over the pixels: the moments of w, 1 | dx | dx^2 | dy | dx dy | dy^2, and the colour's three
+                const float S0x = S0 * dx;
+                const float sum8[8] = {S0, S0x, S0x * dx, S1, S1 * dx, S2, v_red, v_green};
+                float first, second;
+                bank_sum8_scatter(sum8, first, second);
+                v_blue = dpp_add<0x128>(v_blue); // row_ror:8
+                v_blue = dpp_add<0x104>(v_blue); // row_shl:4 (the sum in every row's first four lanes)
+                double* const sums = my_sums + 4 * place;
+                unsafeAtomicAdd(sums, (double)first);
+                unsafeAtomicAdd(sums + 4 * kBwdBatch, (double)second);
+                if((lane & 12) == 0)
+                    unsafeAtomicAdd(s_sum + 8 * kBwdBatch + place, (double)v_blue);
             }
-            // what is summed over the pixels: the moments of w, 1 | dx | dx^2 | dy | dx dy | dy^2, and the colour's three
-            const float S0x = S0 * dx;
-            const float sum8[8] = {S0, S0x, S0x * dx, S1, S1 * dx, S2, v_red, v_green};
-            const float total = row_sum8_scatter(sum8, lane);
-            v_blue = row_sum(v_blue);
-            if(carries)
-                unsafeAtomicAdd(sums, (double)(carries_blue ? v_blue : total));
         }
+        };
+        if(__builtin_amdgcn_ballot_w64(special) == 0)
+            walk(std::true_type());
+        else
+            walk(std::false_type());
         __syncthreads();
-        for(int e = lane; e < staged; e += DSX_WAVE)
-            moments_to_gradients(s_sum + e * kSums, s_a[e], s_b[e]);
+        if(lane < staged)
+            moments_to_gradients<kBwdBatch>(s_sum, lane, s_a[lane], s_b[lane], marks ? marks + mine.x : nullptr);
         __syncthreads();
-        flush_sums(s_sum, s_id, staged, grads, marks, lane, DSX_WAVE);
+        flush_sums<kBwdBatch>(s_sum, reinterpret_cast<const int*>(s_c) + 3, 4, staged, grads, lane, DSX_WAVE);
     }
     // A side job for the memory system, as in the forward: the zeros of the per-Gaussian backward's
     // outputs (that kernel writes only the Gaussians that received a term here), every wavefront a
@@ -1526,8 +1650,7 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
     const float* __restrict__ bg, float* grads, uint8_t* marks, int W, int H, int ntx, uint32_t last_id, int k,
     const int32_t* __restrict__ header, int header_shift, int planar, const BinLists lists, const ZeroJobs zeros)
 {
-    __shared__ float4 s_a[kTileBatch + 1], s_b[kTileBatch + 1];
-    __shared__ float s_c[3 * (kTileBatch + 1)];
+    __shared__ float4 s_a[kTileBatch + 1], s_b[kTileBatch + 1], s_c[kTileBatch + 1];
     __shared__ int s_id[kTileBatch];
     __shared__ double s_sum[(kTileBatch + 1) * kSums];
     __shared__ uint16_t s_reach[kTileBatch];
@@ -1540,7 +1663,8 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
     const int tid = threadIdx.x, lane = tid & (DSX_WAVE - 1), row = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid / DSX_WAVE);
     const int tile = blockIdx.x;
-    const Pixels<1> px(4 * tile + wave, ntx, lane);
+    const int first_block = first_block_of(wave);
+    const Pixels px(tile, wave, ntx, lane);
     const float pxf = (float)px.x + 0.5f, pyf = (float)px.y + 0.5f;
     const float tile_x = (float)(tile % ntx * kTile) + 0.5f, tile_y = (float)(tile / ntx * kTile) + 0.5f;
 
@@ -1558,12 +1682,11 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
     for(int o = 8; o > 0; o >>= 1)
         m = max(m, __shfl_xor(m, o, DSX_WAVE));
     if((lane & 15) == 0)
-        s_last[4 * wave + row] = m;
+        s_last[first_block + block_of_row(row)] = m;
     if(tid == 0)
     {
-        s_a[kTileBatch] = make_float4(0.f, 0.f, 0.f, 0.f);
+        s_a[kTileBatch] = s_c[kTileBatch] = make_float4(0.f, 0.f, 0.f, 0.f);
         s_b[kTileBatch] = make_float4(0.f, 0.f, 0.f, __int_as_float(INT_MAX));
-        s_c[3 * kTileBatch] = s_c[3 * kTileBatch + 1] = s_c[3 * kTileBatch + 2] = 0.f;
     }
     __syncthreads();
     m = s_last[0];
@@ -1604,6 +1727,8 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
     const bool carries_blue = (lane & 15) == 2;
     const bool carries = (lane & 2) == 0 || carries_blue;
     const int sum_slot = carries_blue ? 8 : 4 * (lane & 1) + 2 * ((lane >> 2) & 1) + ((lane >> 3) & 1);
+    double* const my_sums = s_sum + sum_at<kTileBatch + 1>(0, sum_slot);
+    const int sum_step = carries_blue ? 1 : 4;
 
     const int32_t* const keys = ids + k;
     int id_ahead = 0;
@@ -1637,9 +1762,7 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
             const float4* const rec = splats + 3 * (int64_t)id;
             q0 = rec[0], q1 = rec[1], q2 = rec[2];
             reach = reach_of(q1.w);
-#pragma unroll
-            for(int q = 0; q < 4; ++q)
-                reached |= blocks_reached<4>(q0.x, q0.y, q1.x, q1.y, q1.z, reach, tile_x + 8.0f * (q & 1), tile_y + 8.0f * (q >> 1)) << (4 * q);
+            reached = blocks_reached(q0.x, q0.y, q1.x, q1.y, q1.z, reach, tile_x, tile_y);
 #pragma unroll
             for(int b = 0; b < 4 * kTileWaves; ++b)
                 if(idx > s_last[b])
@@ -1648,23 +1771,23 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
         int staged;
         const int place = tile_place(s_counts, __builtin_amdgcn_ballot_w64(reached != 0), staged);
         // (the barrier inside: the queue has been read, the last round's sums have been taken)
-        for(int i = tid; i < staged * kSums; i += kTileThreads)
-            s_sum[i] = 0.0;
+        for(int i = tid; i < 4 * staged; i += kTileThreads)
+            s_sum[i] = s_sum[sum_at<kTileBatch + 1>(0, 4) + i] = 0.0;
+        if(tid < staged)
+            s_sum[sum_at<kTileBatch + 1>(tid, 8)] = 0.0;
         if(reached != 0)
         {
             s_a[place] = make_float4(q0.x, q0.y, q1.x * 0.5f, q1.y);
             s_b[place] = make_float4(q1.z * 0.5f, q1.w, __uint_as_float(reach_limit_bwd(q1.w, reach)),
                                      __int_as_float(idx));
-            s_c[3 * place] = q2.x;
-            s_c[3 * place + 1] = q2.y;
-            s_c[3 * place + 2] = q2.z;
+            s_c[place] = q2;
             s_id[place] = id;
             s_reach[place] = (uint16_t)reached;
         }
         idx_next -= batch;
         __syncthreads();
 
-        const int rounds = (build_lists(s_list, s_reach, staged, wave, lane) + kBwdAtOnce - 1) / kBwdAtOnce;
+        const int rounds = (build_lists(s_list, s_reach, staged, wave, first_block, lane) + kBwdAtOnce - 1) / kBwdAtOnce;
         const uint16_t* my_list = reinterpret_cast<const uint16_t*>(s_list + wave * kTileBatch + row * (kTileBatch / 4));
         for(int i = 0; i < rounds; ++i)
         {
@@ -1680,8 +1803,9 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
                 const uint32_t p = (places >> (8 * u)) & 0xffu;
                 A[u] = s_a[p];
                 B[u] = s_b[p];
-                rv[u] = s_c[3 * p] * vo0 + s_c[3 * p + 1] * vo1 + s_c[3 * p + 2] * vo2;
-                sums[u] = s_sum + p * kSums + sum_slot;
+                const float4 C = s_c[p];
+                rv[u] = C.x * vo0 + C.y * vo1 + C.z * vo2;
+                sums[u] = my_sums + p * sum_step;
             }
 #pragma unroll
             for(int u = 0; u < kBwdAtOnce; ++u)
@@ -1725,9 +1849,9 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
         }
         __syncthreads();
         for(int e = tid; e < staged; e += kTileThreads)
-            moments_to_gradients(s_sum + e * kSums, s_a[e], s_b[e]);
+            moments_to_gradients<kTileBatch + 1>(s_sum, e, s_a[e], s_b[e], marks ? marks + s_id[e] : nullptr);
         __syncthreads();
-        flush_sums(s_sum, s_id, staged, grads, marks, tid, kTileThreads);
+        flush_sums<kTileBatch + 1>(s_sum, s_id, 1, staged, grads, tid, kTileThreads);
         __syncthreads();
     }
     if(zeros.any)

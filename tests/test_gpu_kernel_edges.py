@@ -171,3 +171,55 @@ def test_channel_first_image_in_every_blend_form(oracle, blend_form, list_bin, p
 def test_depth_order_up_to_twelve_tiles_of_keys(n, depths):
     """The merge of more than eight tiles of keys (a third group of four, partly empty), and where the passes take over."""
     test_depth_order_of_few_gaussians(n, depths)
+
+
+@pytest.mark.parametrize("kind,n,W,H", [
+    ("round", 1, 16, 16),        # (the last Gaussian emits nothing)
+    ("round", 57, 33, 17),       # a round of 56 entries and none; tiles cut off at both edges
+    ("round", 66, 16, 16),       # a round of 64 entries and one more
+    ("round", 250, 64, 64),      # the workgroup form's round of 248 and one more
+    ("thin", 250, 131, 77),      # long splats at all angles: blocks that their middles and their ends reach
+    ("tiny", 6000, 97, 50),      # splats that reach one block or two
+    ("black", 2000, 80, 61),     # colours of zero: an entry that is nobody's must not be taken for one that is
+    ("clamped", 900, 70, 50),    # opacities at and above the clamps of both directions
+])
+@pytest.mark.parametrize("bins", [1, 4])
+@pytest.mark.parametrize("pixels_per_lane", [1, 4])
+def test_entries_in_the_lists_of_the_blocks_that_they_reach(oracle, blend_form, pixels_per_lane, bins, kind, n, W, H):
+    """Image, last indices and gradients of both forms against the oracle, which walks every entry for every pixel: an
+    entry that were missing in a block's list would be missing in its pixels."""
+    import test_gpu_opacities as o
+    blend_form(pixels_per_lane)
+    sc = make_scene("cfg0", n=n, width=W, height=H, sh_degree=0, seed=n)
+    g = torch.Generator().manual_seed(n)
+    sc["scales"] = sc["scales"] * 2.0
+    if kind == "round":
+        sc["opacities"] = sc["opacities"] * 0.1     # (no pixel stops: every entry is walked)
+        sc["means_3d"][:, :2] *= 0.3
+    elif kind == "thin":
+        # (up to 15 pixels, widths below one: the exponent's terms, up to 1/2 3.3 15^2 = 370, cancel and cost alpha
+        # 370 2^-24 = 2e-5 of itself for each rounding)
+        sc["scales"] = torch.exp(torch.randn(n, 1, generator=g) * 0.3 - 1.8) * torch.tensor([[1.0, 0.02, 0.02]])
+    elif kind == "tiny":
+        sc["scales"] = sc["scales"] * 0.1
+    elif kind == "black":
+        sc["shs"][:, 0] = -5.0
+    elif kind == "clamped":
+        sc["opacities"] = torch.tensor([0.98, 0.99, 0.995, 0.999, 1.0])[torch.randint(5, (n, 1), generator=g)]
+    A = o.arrays(sc)
+    s = o.scene_settings(sc)
+    img, radii, ost = oracle.forward(s, A["means_3d"], A["scales"], A["rotations"], A["opacities"], A["shs"])
+    S = oracle.state(s, ost, n)
+    B = oracle.backward(s, ost, 16, A["means_3d"], A["scales"], A["rotations"], A["opacities"], A["v_image"])
+    oracle.free(ost)
+    image, final_T, final_idx, out = o.gpu_run(sc, bins)
+    ok = S["margin"] > 1e-4
+    assert ok.mean() > 0.97
+    assert (final_idx[ok] == S["final_idx"][ok]).all()
+    np.testing.assert_allclose(image[ok], img[ok], rtol=1e-4, atol=1e-5)
+    gok = comparable_gaussians(S, B, W, final_T, final_idx)
+    assert gok.mean() > 0.8
+    bounds = oracle.gradient_bounds(s, 16, A["means_3d"], A["scales"], A["rotations"], S["conic"], S["cov3d"], radii,
+                                    B["abs_sums"], rel=1e-4)
+    got = {k: out[k].cpu().numpy() for k in ("v_mean3d", "v_means2d", "v_shs", "v_opacity", "v_scale", "v_quat")}
+    o.check_grads_against_bounds(got, B, bounds, gok, kind)
