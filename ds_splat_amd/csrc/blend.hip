@@ -233,7 +233,8 @@ __device__ __forceinline__ int bits_below_lane(uint64_t mask)
     return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
 
-constexpr int kFwdFourPixelsFrom = 5500; // tiles
+constexpr int kFwdWideUpTo = 256;        // tiles (a workgroup of sixteen wavefronts for each compute unit)
+constexpr int kFwdFourPixelsFrom = 5500;
 constexpr int kBwdFourPixelsFrom = 3000;
 
 // -----------------------------------------------------------------------------------------
@@ -271,6 +272,13 @@ __device__ __forceinline__ uint64_t lanes_below(int count)
 __device__ __forceinline__ uint64_t lowest_bits(uint64_t mask, int count)
 {
     return __builtin_amdgcn_ballot_w64(bits_below_lane(mask) < count) & mask;
+}
+
+// the values of other lanes of each quad of lanes (quad_perm)
+template <int kCtrl>
+__device__ __forceinline__ float quad_lane(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kCtrl, 0xf, 0xf, true));
 }
 
 // A side job for the memory system, which the forward leaves idle: every workgroup prepares
@@ -1078,6 +1086,208 @@ __global__ __launch_bounds__(kTileThreads) void blend_fwd_tile_kernel(const int3
     prepare_grads_share(splats, prep, prep_count, prep_marks, blockIdx.x, gridDim.x, tid, kTileThreads);
 }
 
+// -----------------------------------------------------------------------------------------
+// the same for images of very few tiles: a workgroup of sixteen wavefronts per tile
+// -----------------------------------------------------------------------------------------
+// Up to a few hundred tiles the chip holds every wavefront of the form above with slots to spare, and a launch lasts as long
+// as its longest tile: 72000 cycles at 256 tiles of 325 entries, 40000 of them the walk (190 an entry, of
+// which a pixel's transmittance needs one multiply-add), the rest four rounds of 248 entries, each with its gather's
+// latency and its barriers.  Here each 4x4 block has a wavefront, each of its pixels a quad of lanes: the
+// four lanes work out four entries' alphas side by side, hand them to each other, take the same four steps of
+// the transmittance (the bits of one lane that takes one entry after the other), and each adds its own entry's colour; and up to
+// 960 entries are staged in one round.  us of the kernel, before -> now: 2 K Gaussians at 64x64 22.3 -> 14.0, 16 K at 256x256
+// 30.4 -> 20.8, 50 K at 512x512 (1024 tiles) 32.7 -> 51.1; whole forwards of four kinds of scenes at 256 tiles 74 -> 71,
+// 108 -> 117, 100 -> 95, 92 -> 88, at 400 tiles 85 -> 85, 118 -> 116, 103 -> 105, 124 -> 132: the line lies at 256.
+// Lists per tile only (images of so few tiles have no others unless the caller asks).
+constexpr int kWideBatch = 960; // (two workgroups' records and lists fit a compute unit's LDS)
+constexpr int kWideThreads = 1024;
+constexpr int kWideWaves = kWideThreads / DSX_WAVE;
+static_assert(kWideWaves == kQuads, "a wavefront for each block");
+
+__global__ __launch_bounds__(kWideThreads) void blend_fwd_wide_kernel(const int32_t* __restrict__ ranges, const int32_t* __restrict__ ids,
+                                                                      const float4* __restrict__ splats, float* __restrict__ image,
+                                                                      float* __restrict__ final_T, int32_t* __restrict__ final_idx, int W,
+                                                                      int H, int ntx, uint32_t last_id, int k,
+                                                                      const int32_t* __restrict__ header, int header_shift,
+                                                                      const uint32_t* __restrict__ sort_flag_a,
+                                                                      const uint32_t* __restrict__ sort_flag_b, float4* __restrict__ prep,
+                                                                      int64_t prep_count, uint8_t* __restrict__ prep_marks,
+                                                                      const float* __restrict__ bg, int planar)
+{
+    // (arrays as in the other forms; eight places more than an entry has blocks: the lists' ends name nobody's place, read ahead)
+    __shared__ float4 s_a[kWideBatch + 1], s_b[kWideBatch + 1], s_c[kWideBatch + 1];
+    __shared__ uint16_t s_reach[kWideBatch];
+    __shared__ uint16_t s_list[kWideWaves][kWideBatch + 8];
+    __shared__ int s_counts[kWideWaves];
+    __shared__ uint32_t s_live[kWideWaves];
+
+    const int tid = threadIdx.x, lane = tid & (DSX_WAVE - 1), slot = lane & 3, pixel = lane >> 2;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / DSX_WAVE);
+    const int tile = blockIdx.x;
+    const int x0 = (tile % ntx) * kTile, y0 = (tile / ntx) * kTile;
+    const int x = x0 + 4 * (wave & 3) + (pixel & 3), y = y0 + 4 * (wave >> 2) + (pixel >> 2);
+    const float pxf = (float)x + 0.5f;
+
+    // (positions and layout are taken for what they are as in the wavefront form)
+    const bool layout_ok = header == nullptr || *header == header_shift;
+    int scan = 0, end = 0;
+    if(layout_ok)
+    {
+        scan = min(max(ranges[tile], 0), k);
+        end = min(max(ranges[tile + 1], 0), k);
+    }
+    int left = end - scan;
+
+    const bool inside = x < W && y < H;
+    float pyf = inside ? (float)y + 0.5f : __builtin_nanf(""); // (NaN: stopped)
+    float T = 1.0f, red = 0.f, green = 0.f, blue = 0.f;        // (the colours of this lane's entries)
+    int last = 0;
+    if(tid == 0)
+    {
+        s_a[kWideBatch] = s_c[kWideBatch] = make_float4(0.f, 0.f, 0.f, 0.f);
+        s_b[kWideBatch] = make_float4(0.f, 0.f, __int_as_float(INT_MIN), 0.f);
+    }
+    int id_ahead = 0;
+    if(tid < min(left, kWideBatch))
+        id_ahead = ids[scan + tid];
+    while(true)
+    {
+        const bool live = __builtin_amdgcn_ballot_w64(pyf == pyf) != 0;
+        if(lane == 0)
+            s_live[wave] = live;
+        __syncthreads(); // (and the last round's entries have been walked)
+        const uint32_t live_blocks = (uint32_t)__builtin_amdgcn_ballot_w64(lane < kWideWaves && s_live[lane & (kWideWaves - 1)] != 0);
+        if(live_blocks == 0 || left <= 0)
+            break;
+        const int batch = min(left, kWideBatch), id = id_ahead, index_next = scan;
+        scan += batch;
+        left -= batch;
+        if(tid < min(left, kWideBatch))
+            id_ahead = ids[scan + tid]; // the next round's: in flight meanwhile
+        uint32_t reached = 0;
+        float4 q0, q1, q2;
+        float reach = 0.0f;
+        if(tid < batch)
+        {
+            const float4* const rec = splats + 3 * (int64_t)min((uint32_t)id, last_id);
+            q0 = rec[0], q1 = rec[1], q2 = rec[2];
+            reach = reach_of(q1.w);
+            reached = live_blocks & blocks_reached(q0.x, q0.y, q1.x, q1.y, q1.z, reach, (float)x0 + 0.5f, (float)y0 + 0.5f);
+        }
+        const uint64_t m = __builtin_amdgcn_ballot_w64(reached != 0);
+        if(lane == 0)
+            s_counts[wave] = __popcll(m);
+        __syncthreads();
+        int staged = 0, place = bits_below_lane(m);
+#pragma unroll
+        for(int w = 0; w < kWideWaves; ++w)
+        {
+            const int c = s_counts[w];
+            place += w < wave ? c : 0;
+            staged += c;
+        }
+        staged = __builtin_amdgcn_readfirstlane(staged);
+        if(reached != 0)
+        {
+            s_a[place] = make_float4(q0.x, q0.y, q1.x * -0.5f, q1.y);
+            s_b[place] = make_float4(q1.z * 0.5f, q1.w, __int_as_float(reach_limit_fwd(q1.w, reach)),
+                                     __int_as_float(index_next + tid));
+            s_c[place] = q2;
+            s_reach[place] = (uint16_t)reached;
+        }
+        __syncthreads();
+        if(!live)
+            continue; // (nothing left in this block: the others' barriers are met)
+
+        uint16_t* const list = s_list[wave];
+        int length = 0;
+        for(int first = 0; first < staged; first += DSX_WAVE)
+        {
+            const int at = first + lane;
+            const uint64_t mine = __builtin_amdgcn_ballot_w64(at < staged && ((uint32_t)s_reach[min(at, kWideBatch - 1)] >> wave & 1) != 0);
+            if(__builtin_amdgcn_inverse_ballot_w64(mine))
+                list[length + bits_below_lane(mine)] = (uint16_t)at;
+            length += __popcll(mine);
+        }
+        if(lane < 8)
+            list[length + lane] = kWideBatch;
+
+        struct Entry
+        {
+            float4 A, B, C;
+        };
+        auto fetch = [&](int at) { return Entry{s_a[at], s_b[at], s_c[at]}; };
+        Entry next = fetch(list[slot]);
+        int after = list[4 + slot];
+        for(int i = 0; i < length; i += 4)
+        {
+            const Entry e = next;
+            next = fetch(after);
+            after = list[min(i + 8, length + 4) + slot];
+            float alpha;
+            uint64_t m_pass;
+            {
+#pragma clang fp contract(off)
+                const ExponentX ex = exponent_x(e.A.z, e.A.w, pxf - e.A.x);
+                const float dy = pyf - e.A.y;
+                const float power = __builtin_fmaf(-__builtin_fmaf(e.B.x, dy, ex.bx), dy, ex.ax);
+                m_pass = __builtin_amdgcn_ballot_w64(__float_as_int(power) <= __float_as_int(e.B.z));
+                const float full = fminf(kAlphaMax, e.B.y * __builtin_amdgcn_exp2f(power * kLog2E));
+                alpha = __builtin_amdgcn_inverse_ballot_w64(m_pass) ? full : 0.0f;
+            }
+            const float alphas[4] = {quad_lane<0x00>(alpha), quad_lane<0x55>(alpha), quad_lane<0xAA>(alpha), quad_lane<0xFF>(alpha)};
+            const float T1 = __builtin_fmaf(-alphas[0], T, T), T2 = __builtin_fmaf(-alphas[1], T1, T1);
+            const float T3 = __builtin_fmaf(-alphas[2], T2, T2), T4 = __builtin_fmaf(-alphas[3], T3, T3);
+            float before = slot & 2 ? (slot & 1 ? T3 : T2) : (slot & 1 ? T1 : T);
+            float Tn = T4;
+            if(__builtin_amdgcn_ballot_w64(T4 < 0.0001f) != 0)
+            {
+                // some pixel becomes opaque within these entries: once more, each lane up to where its pixel stops
+                Tn = T;
+                bool stopped = pyf != pyf, counts = !stopped;
+#pragma unroll
+                for(int u = 0; u < 4; ++u)
+                {
+                    before = slot == u ? Tn : before;
+                    const float further = __builtin_fmaf(-alphas[u], Tn, Tn);
+                    stopped = stopped || further < 0.0001f;
+                    Tn = stopped ? Tn : further;
+                    counts = slot == u ? !stopped : counts;
+                }
+                pyf = stopped ? __builtin_nanf("") : pyf;
+                m_pass &= __builtin_amdgcn_ballot_w64(counts);
+                alpha = counts ? alpha : 0.0f;
+                if(__builtin_amdgcn_ballot_w64(pyf == pyf) == 0)
+                    i = length; // no pixel left
+            }
+            T = Tn;
+            const float weight = alpha * before;
+            red = __builtin_fmaf(weight, e.C.x, red);
+            green = __builtin_fmaf(weight, e.C.y, green);
+            blue = __builtin_fmaf(weight, e.C.z, blue);
+            last = __builtin_amdgcn_inverse_ballot_w64(m_pass) ? __float_as_int(e.B.w) : last;
+        }
+    }
+
+    const bool broken = !layout_ok || (sort_flag_a && *sort_flag_a) || (sort_flag_b && *sort_flag_b);
+    // the quad's four parts of the colour, and the last of its last entries
+    auto sum = [](float v) {
+        v += quad_lane<0xB1>(v);
+        return v + quad_lane<0x4E>(v);
+    };
+    red = sum(red), green = sum(green), blue = sum(blue);
+    last = max(last, __float_as_int(quad_lane<0xB1>(__int_as_float(last))));
+    last = max(last, __float_as_int(quad_lane<0x4E>(__int_as_float(last))));
+    if(inside && slot == 0)
+    {
+        const int64_t pix = (int64_t)y * W + x;
+        final_T[pix] = T;
+        final_idx[pix] = last;
+        store_pixel(image, pix, (int64_t)W * H, red, green, blue, T, broken, bg, planar);
+    }
+    prepare_grads_share(splats, prep, prep_count, prep_marks, blockIdx.x, gridDim.x, tid, kWideThreads);
+}
+
 // The BinLists view of a `ranges` buffer in ranges_layout(lg) (lists per bin: lg.shift > 0)
 static BinLists bin_lists(const ListGrid& lg, int32_t* ranges)
 {
@@ -1124,13 +1334,18 @@ int launch_blend_fwd(const dsx_camera& cam, int64_t n, int64_t k, int32_t* range
     {
         DSX_TIMED("blend_fwd_kernel", stream);
         const bool four = blend_pixels_per_lane(ntx * nty, kFwdFourPixelsFrom) == 4;
+        const bool wide = forced_pixels_per_lane() == 0 && lg.shift == 0 && ntx * nty <= kFwdWideUpTo;
         const dim3 grid(ntx * nty);
         const float4* sp = reinterpret_cast<const float4*>(splats);
+        if(wide)
+            hipLaunchKernelGGL(blend_fwd_wide_kernel, grid, dim3(kWideThreads), 0, stream, ranges, sorted_ids, sp, image, final_T,
+                               final_idx, cam.image_width, cam.image_height, ntx, last_id, (int)k, header, lg.shift, sort_flag_a,
+                               sort_flag_b, prep, prep_count, prep_marks, cam.bg, camera_flag(cam, DSX_PLANAR_IMAGE));
 #define DSX_LAUNCH_FWD(KERNEL, THREADS)                                                                          \
     hipLaunchKernelGGL((KERNEL), grid, dim3(THREADS), 0, stream, ranges, sorted_ids, sp, image, final_T, final_idx,  \
                        cam.image_width, cam.image_height, ntx, last_id, (int)k, header, lg.shift, sort_flag_a,     \
                        sort_flag_b, prep, prep_count, prep_marks, cam.bg, camera_flag(cam, DSX_PLANAR_IMAGE), L)
-        if(four && lg.shift)
+        else if(four && lg.shift)
             DSX_LAUNCH_FWD(blend_fwd_kernel<true>, DSX_WAVE);
         else if(four)
             DSX_LAUNCH_FWD(blend_fwd_kernel<false>, DSX_WAVE);

@@ -178,15 +178,17 @@ def test_depth_order_up_to_twelve_tiles_of_keys(n, depths):
     ("round", 57, 33, 17),       # a round of 56 entries and none; tiles cut off at both edges
     ("round", 66, 16, 16),       # a round of 64 entries and one more
     ("round", 250, 64, 64),      # the workgroup form's round of 248 and one more
+    ("round", 962, 16, 16),      # the round of 960 of sixteen wavefronts and one more
+    ("opaque", 2500, 21, 35),    # pixels that stop in the first round of several, and in the middle of four entries
     ("thin", 250, 131, 77),      # long splats at all angles: blocks that their middles and their ends reach
     ("tiny", 6000, 97, 50),      # splats that reach one block or two
     ("black", 2000, 80, 61),     # colours of zero: an entry that is nobody's must not be taken for one that is
     ("clamped", 900, 70, 50),    # opacities at and above the clamps of both directions
 ])
 @pytest.mark.parametrize("bins", [1, 4])
-@pytest.mark.parametrize("pixels_per_lane", [1, 4])
+@pytest.mark.parametrize("pixels_per_lane", [0, 1, 4])  # (0: sixteen wavefronts per tile, for lists per tile)
 def test_entries_in_the_lists_of_the_blocks_that_they_reach(oracle, blend_form, pixels_per_lane, bins, kind, n, W, H):
-    """Image, last indices and gradients of both forms against the oracle, which walks every entry for every pixel: an
+    """Image, last indices and gradients of every form against the oracle, which walks every entry for every pixel: an
     entry that were missing in a block's list would be missing in its pixels."""
     import test_gpu_opacities as o
     blend_form(pixels_per_lane)
