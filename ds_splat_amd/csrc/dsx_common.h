@@ -159,6 +159,8 @@ inline Digits32 digits32(int key_bits)
 // The range comes from the device (rounded outwards to 16 bits), so the host waits for it between the projection
 // and the passes, while the histograms are counted.  us of the passes and the histograms, four digits -> three: 500 K
 // keys 55 + 12 -> 45 + 6, 1 M 68 + 13 -> 56 + 8, 3 M 110 + 19 -> 100 + 17, 6 M 211 + 27 -> 199 + 26.
+// The host learns how many Gaussians emit at the same time: the first pass leaves the others behind, the second and third run
+// over the rest.  us of the three passes: 3 M Gaussians of which 64 % emit 98 -> 85, 6 M (half) 201 -> 163, 2 M 75 -> 68, 1 M 55 -> 51.
 constexpr int kDepthBits = 9;
 constexpr int kDepthBins = 1 << kDepthBits;
 constexpr int kDepthPasses = 3;
@@ -298,7 +300,7 @@ struct OrderLayout
     size_t rects_sorted; // uint2[n] the same in depth order
     size_t rects32;    // uint32[n]  packed rectangles on their way through the depth sort
     size_t block_sums; // uint32[blocks + 1] tile counts of 256 consecutive Gaussians IN DEPTH ORDER, scanned
-    size_t key_ranges; // uint2[blocks] of 256 consecutive Gaussians' depth keys, upper halves: 0xffff - smallest, largest (zeros: none emits)
+    size_t key_ranges; // uint2[blocks] of 256 consecutive Gaussians: 0xffff - the smallest upper half of a key that emits, and how many emit << 16; the largest one
     size_t slot_hist;  // uint32[kMaxPasses32 * 256] digit histograms of the tile slots of all pairs
     size_t cover;      // int32[(ntx + 1) * (nty + 1) + 1] pairs per tile (corner grid, then its 2-D prefix sum)
     size_t bin_cover;  // int32[(nbx + 1) * (nby + 1) + 1] the same per bin (binned lists only)

@@ -401,21 +401,30 @@ __global__ __launch_bounds__(kProjBlock) void project_fwd_kernel(const ProjectPa
     }
 
     const uint32_t ws = wave_sum_u32(count);
+    const uint32_t emitting = (uint32_t)__popcll(__ballot(count != 0));
     near16 = wave_incl_max_scan(near16);
     far16 = wave_incl_max_scan(far16);
     if(lane == 63)
     {
         wave_sums[wave] = ws;
-        wave_ranges[wave] = make_uint2(near16, far16);
+        wave_ranges[wave] = make_uint2(near16 | emitting << 16, far16);
     }
     __syncthreads();
     if(tid == 0)
     {
         p.block_sums[blockIdx.x] = wave_sums[0] + wave_sums[1] + wave_sums[2] + wave_sums[3];
         if(p.depth_keys)
-            p.key_ranges[blockIdx.x] =
-                make_uint2(max(max(wave_ranges[0].x, wave_ranges[1].x), max(wave_ranges[2].x, wave_ranges[3].x)),
-                           max(max(wave_ranges[0].y, wave_ranges[1].y), max(wave_ranges[2].y, wave_ranges[3].y)));
+        {
+            uint32_t near_all = 0, far_all = 0, emitting_all = 0;
+#pragma unroll
+            for(int w = 0; w < kProjBlock / DSX_WAVE; ++w)
+            {
+                near_all = max(near_all, wave_ranges[w].x & 0xffffu);
+                far_all = max(far_all, wave_ranges[w].y);
+                emitting_all += wave_ranges[w].x >> 16;
+            }
+            p.key_ranges[blockIdx.x] = make_uint2(near_all | emitting_all << 16, far_all);
+        }
     }
 }
 

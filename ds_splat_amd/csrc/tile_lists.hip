@@ -244,14 +244,17 @@ struct RectJob
 
 // vals_in == nullptr: the values are the input positions (iota).  keys_out == nullptr: the
 // keys are not needed after this pass.  KeyT: uint32_t, or uint16_t for tile slots that fit.
-// kBits = 9: a pass of the depth sort over a known range; `range` turns the keys into their distances (the first pass)
-// and names what a key without pairs has become.
+// kBits = 9: a pass of the depth sort over a known range.  The first pass (kFirst) turns the keys into their distances from
+// `first`, of which a key without pairs has none: it becomes `behind`, stands behind the digits in its tile, and its value goes to
+// its final place, behind the `emitting` others in the order of the input (how many lie in the tiles before is those tiles' keys
+// less the sum of the digits' counts that the chained scan brings).  Later passes see the others only.
 struct KeyRange
 {
-    uint32_t first, behind, no_pairs;
+    uint32_t first, behind, emitting;
 };
-template <typename KeyT, int kSort32Threads, int kSort32Items, bool kCarry, int kBits>
-__global__ __launch_bounds__(kSort32Threads) void onesweep32_kernel(
+template <typename KeyT, int kSort32Threads, int kSort32Items, bool kCarry, int kBits, bool kFirst = false>
+// (eight wavefronts per SIMD: two workgroups per compute unit whatever the tile)
+__global__ __launch_bounds__(kSort32Threads) __attribute__((amdgpu_waves_per_eu(8))) void onesweep32_kernel(
     const KeyT* __restrict__ keys_in, const uint32_t* __restrict__ vals_in, KeyT* __restrict__ keys_out,
     uint32_t* __restrict__ vals_out, int64_t count, int shift, uint32_t mask, const uint32_t* __restrict__ hist_counts,
     uint32_t* status, uint32_t* tile_counter, uint32_t* error_flag, const RectJob rects,
@@ -265,6 +268,8 @@ __global__ __launch_bounds__(kSort32Threads) void onesweep32_kernel(
     __shared__ uint32_t s_keys[kSort32Tile]; // reused for the values in the second round
     __shared__ uint16_t s_whist[kSort32Waves][kBins];
     __shared__ uint32_t s_digit_start[kBins];
+    __shared__ uint32_t s_before[kFirst ? kBins / DSX_WAVE : 1]; // keys of the tiles before, by the digits' wavefronts
+    __shared__ uint32_t s_none[kFirst ? kSort32Waves : 1];       // this tile's keys without pairs, by wavefront
     __shared__ uint32_t s_gbase[kBins];
     __shared__ __attribute__((aligned(16))) uint32_t s_wave_tot[kBins / DSX_WAVE];
     __shared__ __attribute__((aligned(16))) uint32_t s_hist_tot[kBins / DSX_WAVE];
@@ -299,26 +304,39 @@ __global__ __launch_bounds__(kSort32Threads) void onesweep32_kernel(
         // highest digit and, being last in tile order, rank behind every real key, so the real
         // keys' positions are what they would be without them and no phase needs a validity test
         // except the stores (tile position < tile_n).
-        key[it] = 0xffffffffu;
+        // (first pass: they are keys without pairs, behind the others of that kind)
+        key[it] = kFirst ? range.behind : 0xffffffffu;
         if(local < tile_n)
         {
             key[it] = (uint32_t)__builtin_nontemporal_load(keys_in + tile_base + local);
-            if(kBits == kDepthBits)
+            if(kFirst)
                 key[it] = min(key[it] - range.first, range.behind);
         }
     }
 
     // ---- wave-local stable rank ------------------------------------------------------------
     uint16_t* wh = s_whist[wave];
+    uint32_t none = 0; // keys without pairs so far
 #pragma unroll
     for(int it = 0; it < kSort32Items; ++it)
     {
         const uint32_t d = digit_of(key[it]);
-        const uint64_t m = match_digit<kBits>(d, bits);
+        uint64_t m = match_digit<kBits>(d, bits);
+        uint64_t m_none = 0;
+        if(kFirst)
+        {
+            m_none = __builtin_amdgcn_ballot_w64(key[it] == range.behind);
+            m = __builtin_amdgcn_inverse_ballot_w64(m_none) ? m_none : m & ~m_none;
+        }
         const uint32_t below = (uint32_t)bits_below(m);
-        const uint32_t old = wh[d];
+        uint32_t old = wh[d];
+        if(kFirst)
+        {
+            old = __builtin_amdgcn_inverse_ballot_w64(m_none) ? none : old;
+            none += (uint32_t)__popcll(m_none);
+        }
         __builtin_amdgcn_wave_barrier();
-        if(below == 0)
+        if(below == 0 && (!kFirst || !__builtin_amdgcn_inverse_ballot_w64(m_none)))
             wh[d] = (uint16_t)(old + (uint32_t)__popcll(m));
         __builtin_amdgcn_wave_barrier();
         if(it & 1)
@@ -329,6 +347,8 @@ __global__ __launch_bounds__(kSort32Threads) void onesweep32_kernel(
         // item's digit, histogram address and old count into the next phase in registers of their own
         asm volatile("" : "+v"(pos2[it >> 1]), "+v"(key[it]));
     }
+    if(kFirst && lane == 0)
+        s_none[wave] = none;
     __syncthreads();
 
     // ---- per-digit totals of the tile (thread d <-> digit d), wave offsets, digit starts ----
@@ -370,12 +390,32 @@ __global__ __launch_bounds__(kSort32Threads) void onesweep32_kernel(
     }
     __syncthreads();
 
+    // places of the tile from `emitters` on (there are none after the first pass) hold what does not emit
+    int emitters = tile_n;
+    uint32_t none_start = 0; // where this wavefront's begin
+    if(kFirst)
+    {
+        uint32_t all = 0;
+#pragma unroll
+        for(int w = 0; w < kSort32Waves; ++w)
+        {
+            const uint32_t c = s_none[w];
+            none_start += w < wave ? c : 0u;
+            all += c;
+        }
+        emitters = kSort32Tile - __builtin_amdgcn_readfirstlane((int)all); // (the places past the end are counted among them)
+        none_start = (uint32_t)emitters + __builtin_amdgcn_readfirstlane(none_start);
+    }
+
     // ---- keys into LDS in tile-sorted order ----------------------------------------------
 #pragma unroll
     for(int it = 0; it < kSort32Items; ++it)
     {
         const uint32_t d = digit_of(key[it]);
-        const uint32_t p = ((pos2[it >> 1] >> (16 * (it & 1))) & 0xffffu) + s_digit_start[d] + s_whist[wave][d];
+        uint32_t start = s_digit_start[d] + s_whist[wave][d];
+        if(kFirst)
+            start = key[it] == range.behind ? none_start : start;
+        const uint32_t p = ((pos2[it >> 1] >> (16 * (it & 1))) & 0xffffu) + start;
         s_keys[p] = key[it];
         pos2[it >> 1] = (it & 1) ? ((pos2[it >> 1] & 0xffffu) | (p << 16)) : ((pos2[it >> 1] & 0xffff0000u) | p);
     }
@@ -449,8 +489,23 @@ __global__ __launch_bounds__(kSort32Threads) void onesweep32_kernel(
                                __HIP_MEMORY_SCOPE_AGENT);
         }
         s_gbase[tid] = hist_excl + excl - s_digit_start[tid];
+        if(kFirst)
+        {
+            const uint32_t before = wave_sum_u32(excl);
+            if(lane == 0)
+                s_before[wave] = before;
+        }
     }
     __syncthreads();
+    uint32_t tail = 0; // place of the tile's first key without pairs, less its position in the tile
+    if(kFirst)
+    {
+        tail = range.emitting + (uint32_t)tile_base - (uint32_t)emitters;
+#pragma unroll
+        for(int w = 0; w < kBins / DSX_WAVE; ++w)
+            tail -= s_before[w];
+        tail = __builtin_amdgcn_readfirstlane(tail);
+    }
 
     // ---- scatter keys: consecutive threads -> consecutive addresses inside a digit's run ----
     uint32_t out[kSort32Items];            // where the key at tile position it * threads + tid goes
@@ -464,10 +519,11 @@ __global__ __launch_bounds__(kSort32Threads) void onesweep32_kernel(
         if(j < tile_n)
         {
             const uint32_t kk = s_keys[j];
-            out[it] = s_gbase[digit_of(kk)] + (uint32_t)j;
-            if(gather_src && kk == (kBits == kDepthBits ? range.no_pairs : kNoPairsKey))
+            const uint32_t digit_base = s_gbase[digit_of(kk)];
+            out[it] = (!kFirst || j < emitters ? digit_base : tail) + (uint32_t)j;
+            if(gather_src && kk == kNoPairsKey)
                 no_record |= 1u << it;
-            if(keys_out)
+            if(keys_out && (!kFirst || j < emitters))
                 keys_out[out[it]] = (KeyT)kk;
         }
     }
@@ -510,7 +566,7 @@ __global__ __launch_bounds__(kSort32Threads) void onesweep32_kernel(
             const int j = it * kSort32Threads + tid;
             if((it & 3) == 0)
                 __builtin_amdgcn_sched_barrier(0);
-            if(j < tile_n)
+            if(kFirst ? j < emitters : j < tile_n)
             {
                 const uint32_t v = s_keys[j];
                 if(rects.unpack_dst)
@@ -558,17 +614,15 @@ static int sort32_clear(int64_t count, int key_bits, int tile_keys, void* sort_w
 // gather.  carry_a / carry_b (with gather_src and gather_dst): the records travel through the passes
 // as packed 32-bit values instead, in ping-pong buffers of their own (the first pass packs them from
 // gather_src, the last one unpacks them into gather_dst).
-// range: a depth sort over a known range (kBits = 9).
-template <typename KeyT, int kThreads, int kItems, bool kCarry = false, int kBits = kBits32>
+template <typename KeyT, int kThreads, int kItems, bool kCarry = false>
 static int sort32_passes(int64_t count, int key_bits, KeyT* keys_a, uint32_t* vals_a, KeyT* keys_b, uint32_t* vals_b,
                          bool iota_values, bool keep_keys, void* sort_ws, const char* label, hipStream_t stream,
                          KeyT** keys_out, uint32_t** vals_out, const uint2* gather_src = nullptr,
                          uint2* gather_dst = nullptr, const uint32_t* counts = nullptr, uint32_t* carry_a = nullptr,
-                         uint32_t* carry_b = nullptr, const DepthRange* range = nullptr)
+                         uint32_t* carry_b = nullptr)
 {
-    constexpr int kBins = 1 << kBits;
     const Sort32Workspace w = sort32_workspace(count, key_bits, kThreads * kItems);
-    const Digits32 plan = range ? range->digits : digits32(key_bits);
+    const Digits32 plan = digits32(key_bits);
     char* base = static_cast<char*>(sort_ws);
     uint32_t* hist = reinterpret_cast<uint32_t*>(base + w.hist);
     uint32_t* counters = reinterpret_cast<uint32_t*>(base + w.counters);
@@ -583,9 +637,6 @@ static int sort32_passes(int64_t count, int key_bits, KeyT* keys_a, uint32_t* va
     for(int p = 0; p < plan.passes; ++p)
     {
         const bool last = p == plan.passes - 1;
-        KeyRange keys = {0u, 0xffffffffu, kNoPairsKey};
-        if(range)
-            keys = {p == 0 ? range->first : 0u, p == 0 ? range->behind : 0xffffffffu, range->behind};
         RectJob job = {};
         if(kCarry)
         {
@@ -601,11 +652,11 @@ static int sort32_passes(int64_t count, int key_bits, KeyT* keys_a, uint32_t* va
         }
         {
             DSX_TIMED(label, stream);
-            hipLaunchKernelGGL((onesweep32_kernel<KeyT, kThreads, kItems, kCarry, kBits>), dim3((unsigned)w.tiles), dim3(kThreads), 0,
+            hipLaunchKernelGGL((onesweep32_kernel<KeyT, kThreads, kItems, kCarry, kBits32>), dim3((unsigned)w.tiles), dim3(kThreads), 0,
                                stream, (const KeyT*)kin, (const uint32_t*)((p == 0 && iota_values) ? nullptr : vin),
                                (last && !keep_keys) ? (KeyT*)nullptr : kout, vout, count, plan.shift[p], plan.mask[p],
-                               raw + p * kBins, status + (size_t)p * w.tiles * kBins,
-                               counters + p, counters + w.passes, job, keys);
+                               raw + p * kBins32, status + (size_t)p * w.tiles * kBins32,
+                               counters + p, counters + w.passes, job, KeyRange{});
         }
         DSX_LAUNCH_CHECK();
         KeyT* tk = kin;
@@ -689,20 +740,26 @@ __global__ __launch_bounds__(kHist32Threads) void depth_hist_kernel(const uint32
 {
     __shared__ uint32_t hist[kSortWordsMost];
     __shared__ uint2 s_range[kHist32Threads / DSX_WAVE];
+    __shared__ uint32_t s_emitting[kHist32Threads / DSX_WAVE];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     for(int j = tid; j < (int)kSortWordsMost; j += kHist32Threads)
         hist[j] = 0;
-    uint32_t near16 = 0, far16 = 0;
+    uint32_t near16 = 0, far16 = 0, emitting = 0;
     for(int64_t b = tid; b < blocks; b += kHist32Threads)
     {
         const uint2 r = ranges[b];
-        near16 = max(near16, r.x);
+        near16 = max(near16, r.x & 0xffffu);
         far16 = max(far16, r.y);
+        emitting += r.x >> 16;
     }
     near16 = wave_incl_max_scan(near16);
     far16 = wave_incl_max_scan(far16);
+    emitting = wave_sum_u32(emitting);
     if(lane == 63)
+    {
         s_range[wave] = make_uint2(near16, far16);
+        s_emitting[wave] = emitting;
+    }
     __syncthreads();
 #pragma unroll
     for(int w = 0; w < kHist32Threads / DSX_WAVE; ++w)
@@ -713,10 +770,16 @@ __global__ __launch_bounds__(kHist32Threads) void depth_hist_kernel(const uint32
     const uint32_t lowest = 0xffffu - (uint32_t)__builtin_amdgcn_readfirstlane((int)near16);
     const uint32_t highest = (uint32_t)__builtin_amdgcn_readfirstlane((int)far16);
     if(blockIdx.x == 0 && tid == 0)
+    {
+        unsigned long long all = 0;
+        for(int w = 0; w < kHist32Threads / DSX_WAVE; ++w)
+            all += s_emitting[w];
         store_to_host(to_host, 2, lowest | ((unsigned long long)highest << 16));
+        store_to_host(to_host, 3, all);
+    }
     const DepthRange range = depth_range(lowest, highest);
     const int bins = range.narrow ? kDepthBins : kBins32;
-    uint32_t none = 0; // keys without pairs: counted by their thread, added to their bins at the end
+    uint32_t none = 0; // keys without pairs: counted by their thread, added to their bins at the end (four digits; three leave them out)
     const int64_t chunk = (int64_t)kHist32Threads * kDepthHistItems, chunks = (count + chunk - 1) / chunk;
     for(int64_t c = blockIdx.x; c < chunks; c += gridDim.x)
     {
@@ -745,7 +808,7 @@ __global__ __launch_bounds__(kHist32Threads) void depth_hist_kernel(const uint32
                         atomicAdd(&hist[p * bins + (((key[it] - range.first) >> range.digits.shift[p]) & range.digits.mask[p])], 1u);
         }
     }
-    none = wave_sum_u32(none);
+    none = range.narrow ? 0u : wave_sum_u32(none);
     if(lane == 0 && none)
 #pragma unroll
         for(int p = 0; p < kMaxPasses32; ++p)
@@ -837,17 +900,20 @@ __device__ __forceinline__ uint32_t list_count(uint2 r, int shift)
 }
 
 // Tile count of each run of 256 Gaussians taken in depth order (the last pass of the depth sort
-// has already put the rectangles into that order).
-__global__ __launch_bounds__(kProjBlock) void ordered_block_sums_kernel(const uint2* __restrict__ rects_sorted,
-                                                                       int64_t n, int shift,
+// has already put the rectangles into that order: those of the first `emitting` Gaussians; the others', as far as the
+// emission looks at them, are cleared here).
+__global__ __launch_bounds__(kProjBlock) void ordered_block_sums_kernel(uint2* __restrict__ rects_sorted,
+                                                                       int64_t n, int64_t emitting, int shift,
                                                                        uint32_t* __restrict__ block_sums)
 {
     __shared__ uint32_t wave_sums[kProjBlock / DSX_WAVE];
     const int tid = threadIdx.x;
     const int64_t p = (int64_t)blockIdx.x * kProjBlock + tid;
     uint32_t count = 0;
-    if(p < n)
+    if(p < emitting)
         count = list_count(rects_sorted[p], shift);
+    else if(p < n && p < (emitting + kProjBlock - 1) / kProjBlock * kProjBlock)
+        rects_sorted[p] = make_uint2(0u, 0u);
     const uint32_t ws = wave_sum_u32(count);
     if((tid & 63) == 0)
         wave_sums[tid >> 6] = ws;
@@ -1581,9 +1647,10 @@ void depth_order_clear_region(const dsx_camera& cam, int64_t n, void* order, uin
     *count = (int64_t)((w.bytes + (o.ranges - o.cover)) / 4);
 }
 
-// The depth sort of a whole forward (cleared workspace): ids in `ids_a`, rectangles in `rects_sorted`.
+// The depth sort of a whole forward (cleared workspace): ids in `ids_a`, the rectangles of the first `emitting` of them in
+// `rects_sorted`.
 static int launch_depth_sort(int64_t n, char* base, const OrderLayout& o, int64_t blocks, bool carry,
-                             const HostCounts& to_host, hipStream_t stream, uint32_t** vals_out)
+                             const HostCounts& to_host, hipStream_t stream, int64_t* emitting)
 {
     if(n >= (1ll << 30))
         return DSX_ERR_TOO_LARGE;
@@ -1605,39 +1672,109 @@ static int launch_depth_sort(int64_t n, char* base, const OrderLayout& o, int64_
                            reinterpret_cast<uint32_t*>(ws + w.hist), to_host);
     }
     DSX_LAUNCH_CHECK();
-    uint64_t ends;
-    if(!wait_for_word(to_host, 2, stream, &ends))
+    uint64_t ends, emitters;
+    if(!wait_for_word(to_host, 2, stream, &ends) || !wait_for_word(to_host, 3, stream, &emitters))
         return DSX_ERR_RUNTIME;
     const DepthRange range = depth_range((uint32_t)(ends & 0xffffu), (uint32_t)(ends >> 16));
-    uint32_t* ko;
     const char* const label = "onesweep32_kernel<sort>";
-    // An even number of passes ends where it began, with an odd one the buffers change places: the ids end in ids_a
-    // either way, and the last pass never reads packed rectangles from the memory that it unpacks them into.
-#define DSX_DEPTH_SORT(ITEMS, CARRY)                                                                                    \
-    (range.narrow                                                                                                      \
-         ? sort32_passes<uint32_t, kSortThreads32, ITEMS, CARRY, kDepthBits>(n, 32, keys_a, ids_b, keys_b, ids_a, true, \
-                                                                             false, ws, label, stream, &ko, vals_out,   \
-                                                                             rects, rects_sorted, nullptr,              \
-                                                                             CARRY ? packed_b : nullptr,                \
-                                                                             CARRY ? packed_a : nullptr, &range)        \
-         : sort32_passes<uint32_t, kSortThreads32, ITEMS, CARRY>(n, 32, keys_a, ids_a, keys_b, ids_b, true, false, ws,  \
-                                                                 label, stream, &ko, vals_out, rects, rects_sorted,     \
-                                                                 nullptr, CARRY ? packed_a : nullptr,                   \
-                                                                 CARRY ? packed_b : nullptr))
-#define DSX_DEPTH_SORT_ITEMS(ITEMS) \
-    case ITEMS: return carry ? DSX_DEPTH_SORT(ITEMS, true) : DSX_DEPTH_SORT(ITEMS, false)
-    switch(sort32_items(n))
+    *emitting = n;
+    if(!range.narrow)
     {
-        DSX_DEPTH_SORT_ITEMS(2);
-        DSX_DEPTH_SORT_ITEMS(3);
-        DSX_DEPTH_SORT_ITEMS(4);
-        DSX_DEPTH_SORT_ITEMS(6);
-        DSX_DEPTH_SORT_ITEMS(8);
-        DSX_DEPTH_SORT_ITEMS(kSortItemsMax32);
-    }
+        // (four passes: the values, iota in the first, go b, a, b, a and end in ids_a)
+        uint32_t *ko, *vo;
+#define DSX_DEPTH_SORT_ITEMS(ITEMS)                                                                                     \
+    case ITEMS:                                                                                                        \
+        return carry ? sort32_passes<uint32_t, kSortThreads32, ITEMS, true>(n, 32, keys_a, ids_a, keys_b, ids_b, true,  \
+                                                                            false, ws, label, stream, &ko, &vo, rects, \
+                                                                            rects_sorted, nullptr, packed_a, packed_b) \
+                     : sort32_passes<uint32_t, kSortThreads32, ITEMS>(n, 32, keys_a, ids_a, keys_b, ids_b, true, false, \
+                                                                      ws, label, stream, &ko, &vo, rects, rects_sorted)
+        switch(sort32_items(n))
+        {
+            DSX_DEPTH_SORT_ITEMS(2);
+            DSX_DEPTH_SORT_ITEMS(3);
+            DSX_DEPTH_SORT_ITEMS(4);
+            DSX_DEPTH_SORT_ITEMS(6);
+            DSX_DEPTH_SORT_ITEMS(8);
+            DSX_DEPTH_SORT_ITEMS(kSortItemsMax32);
+        }
 #undef DSX_DEPTH_SORT_ITEMS
-#undef DSX_DEPTH_SORT
-    return DSX_ERR_RUNTIME;
+        return DSX_ERR_RUNTIME;
+    }
+    // Three passes, of which the first puts the Gaussians that emit nothing into their final places (in ids_a, where its
+    // values and the last pass's go) and the others sort the rest: a third fewer keys where a third of the cloud is out of sight.
+    // The last pass never reads packed rectangles from the memory that it unpacks them into.
+    *emitting = (int64_t)emitters;
+    uint32_t* const counters = reinterpret_cast<uint32_t*>(ws + w.counters);
+    int64_t count = n;
+    int items = sort32_items(n);
+    for(int p = 0; p < kDepthPasses; ++p)
+    {
+        const bool first = p == 0, last = p == kDepthPasses - 1;
+        if(p == 1)
+        {
+            // (as few keys to a thread as the statuses of n Gaussians' tiles have room for)
+            count = *emitting;
+            const int family[] = {1, 2, 3, 4, 6, 8, kSortItemsMax32};
+            for(int i : family)
+                if((items = i) >= sort32_items(count) && (count + (int64_t)i * kSortThreads32 - 1) / ((int64_t)i * kSortThreads32) <= w.tiles)
+                    break;
+        }
+        const unsigned tiles = (unsigned)((count + (int64_t)items * kSortThreads32 - 1) / ((int64_t)items * kSortThreads32));
+        if(tiles == 0)
+            break;
+        RectJob job = {};
+        if(carry)
+        {
+            job.pack_src = first ? rects : nullptr;
+            job.carry_in = p & 1 ? packed_a : packed_b;
+            job.carry_out = p & 1 ? packed_b : packed_a;
+            job.unpack_dst = last ? rects_sorted : nullptr;
+        }
+        else if(last)
+        {
+            job.gather_src = rects;
+            job.gather_dst = rects_sorted;
+        }
+        const KeyRange keys = {first ? range.first : 0u, first ? range.behind : 0xffffffffu, (uint32_t)*emitting};
+        const uint32_t* const keys_in = p & 1 ? keys_b : keys_a;
+        uint32_t* const keys_out = last ? nullptr : (p & 1 ? keys_a : keys_b);
+        const uint32_t* const vals_in = first ? nullptr : (p & 1 ? ids_a : ids_b);
+        uint32_t* const vals_out = p & 1 ? ids_b : ids_a;
+        DSX_TIMED(label, stream);
+#define DSX_DEPTH_PASS(ITEMS, CARRY, FIRST)                                                                             \
+    hipLaunchKernelGGL((onesweep32_kernel<uint32_t, kSortThreads32, ITEMS, CARRY, kDepthBits, FIRST>), dim3(tiles),      \
+                       dim3(kSortThreads32), 0, stream, keys_in, vals_in, keys_out, vals_out, count,                     \
+                       range.digits.shift[p], range.digits.mask[p],                                                    \
+                       reinterpret_cast<const uint32_t*>(ws + w.hist) + p * kDepthBins,                                \
+                       reinterpret_cast<uint32_t*>(ws + w.status) + (size_t)p * w.tiles * kDepthBins, counters + p,     \
+                       counters + w.passes, job, keys)
+#define DSX_DEPTH_PASS_ITEMS(ITEMS)         \
+    case ITEMS:                             \
+        if(carry && first)                  \
+            DSX_DEPTH_PASS(ITEMS, true, true);   \
+        else if(carry)                      \
+            DSX_DEPTH_PASS(ITEMS, true, false);  \
+        else if(first)                      \
+            DSX_DEPTH_PASS(ITEMS, false, true);  \
+        else                                \
+            DSX_DEPTH_PASS(ITEMS, false, false); \
+        break
+        switch(items)
+        {
+            DSX_DEPTH_PASS_ITEMS(1);
+            DSX_DEPTH_PASS_ITEMS(2);
+            DSX_DEPTH_PASS_ITEMS(3);
+            DSX_DEPTH_PASS_ITEMS(4);
+            DSX_DEPTH_PASS_ITEMS(6);
+            DSX_DEPTH_PASS_ITEMS(8);
+            DSX_DEPTH_PASS_ITEMS(kSortItemsMax32);
+        }
+#undef DSX_DEPTH_PASS_ITEMS
+#undef DSX_DEPTH_PASS
+        DSX_LAUNCH_CHECK();
+    }
+    return DSX_OK;
 }
 
 // to_host (optional): words of pinned host memory that receive the pair counts (per-tile lists: what the
@@ -1743,7 +1880,8 @@ int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_
     if(hipGetLastError() != hipSuccess)
         return finish(DSX_ERR_LAUNCH);
 
-    uint32_t *ko, *vo;
+    uint32_t *ko, *vo = ids_a;
+    int64_t emitting = n;
     // the rectangles travel through the passes when they pack into 32 bits (the passes end in
     // rects_sorted, whose first half holds the packed ones of the passes in between), else the last
     // pass gathers them
@@ -1752,7 +1890,7 @@ int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_
     // (a wait for the range: fewer Gaussians are sorted before the host could have launched the rest; us a step
     // with four digits / three: 50 K 223 / 230, 100 K 249 / 260, 300 K 493 / 491, 1 M forward 319 / 305)
     if(to_host.words && sort32_items(n) > 1)
-        rc = launch_depth_sort(n, base, o, blocks, carry, to_host, stream, &vo);
+        rc = launch_depth_sort(n, base, o, blocks, carry, to_host, stream, &emitting);
     else // (four passes: the values, iota in the first, go b, a, b, a and end in ids_a)
         rc = launch_sort32(n, 32, keys_a, ids_a, keys_b, ids_b, true, false, base + o.sort, stream, &ko, &vo,
                        reinterpret_cast<const uint2*>(base + o.rects), reinterpret_cast<uint2*>(base + o.rects_sorted),
@@ -1765,7 +1903,7 @@ int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_
     {
         DSX_TIMED("ordered_block_sums_kernel", stream);
         hipLaunchKernelGGL(ordered_block_sums_kernel, dim3((unsigned)blocks), dim3(kProjBlock), 0, stream,
-                           reinterpret_cast<const uint2*>(base + o.rects_sorted), n,
+                           reinterpret_cast<uint2*>(base + o.rects_sorted), n, emitting,
                            list_grid(cam).shift, block_sums);
     }
     if(hipGetLastError() != hipSuccess)

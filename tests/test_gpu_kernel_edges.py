@@ -102,6 +102,47 @@ def test_depth_order_over_a_known_range(n, depths):
     assert (seen["offsets"] == np.concatenate([[0], np.cumsum(sums)])).all()
 
 
+@pytest.mark.parametrize("out", ["third", "first_half", "last_half", "nearly_all", "in_runs"])
+@pytest.mark.parametrize("n,bins", [(262145, 1), (530001, 1), (3200000, 4)])
+def test_depth_order_of_a_cloud_that_is_partly_out_of_sight(n, bins, out):
+    """The first digit pass of a whole forward puts the Gaussians that emit nothing behind the others, by index, and the
+    others alone go through the rest: the order, the offsets and the pairs that are emitted are what they are without that."""
+    from ds_splat_amd import stages
+    sc = make_scene("cfg0", n=n, width=96, height=64, sh_degree=0, seed=9)
+    g = torch.Generator().manual_seed(n)
+    i = torch.arange(n)
+    gone = {"third": torch.rand(n, generator=g) < 0.35, "first_half": i < n // 2, "last_half": i >= n // 2,
+            "nearly_all": i % 50000 != 7, "in_runs": (i // 5000) % 2 == 0}[out]
+    means = torch.zeros(n, 3)
+    means[:, 2] = 2.0 + 18.0 * torch.rand(n, generator=g)
+    means[::11, 2] = 5.0                                       # ties
+    means[gone, 0] = 1e4
+    scales = (means[:, 2:] * 1e-3).expand(n, 3).contiguous()
+    cam = stages.camera_from_scene(sc, DEV, list_bin=bins)
+    seen = {}
+
+    def look(order, n_, k):
+        perm, offsets = stages.depth_order_view(n_, order)
+        seen["perm"], seen["offsets"] = perm.cpu().numpy().astype(np.int64), offsets.cpu().numpy().astype(np.int64)
+
+    _, st = stages.forward(cam, means.to(DEV), scales.to(DEV), sc["rotations"].to(DEV), sc["opacities"].to(DEV),
+                           sc["shs"].to(DEV), after_project=look)
+    touched = st.splats[:, 11].contiguous().view(torch.int32).cpu().numpy().astype(np.int64)
+    touched[-1] = 0
+    bits = st.splats[:, 2].contiguous().view(torch.int32).cpu().numpy().view(np.uint32)
+    keys = np.where(touched > 0, bits, np.uint32(0xffffffff))
+    emitting = int((keys != 0xffffffff).sum())
+    assert emitting == int((~gone[:-1]).sum()) and 0 < emitting < n - 1
+    perm = np.argsort(keys, kind="stable")
+    assert (seen["perm"] == perm).all()
+    if bins == 1:
+        sums = np.add.reduceat(touched[perm], np.arange(0, n, 256))
+        assert (seen["offsets"] == np.concatenate([[0], np.cumsum(sums)])).all()
+        assert (np.bincount(st.sorted_ids.cpu().numpy(), minlength=n) == touched).all()
+    else:
+        assert set(np.unique(st.ids.cpu().numpy()).tolist()) == set(np.nonzero(touched)[0].tolist())
+
+
 @pytest.mark.parametrize("pixels_per_lane", [1, 4])
 def test_bin_lists_beyond_two_to_the_thirty(blend_form, pixels_per_lane):
     """Positions of a bin's list that a 32-bit byte offset does not reach: the same lists, moved behind 2^30 others,
