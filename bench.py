@@ -68,7 +68,7 @@ def algorithmic_work(kernel, n, k, pixels, lists, coeffs, counters, marked, carr
         # depth sort of the Gaussians: key + id, in and out; images of at most 255 x 255 tiles also carry each
         # Gaussian's packed tile rectangle through the passes (4 bytes in and out) instead of gathering them
         return "hbm", (24 if carries_rects else 16) * n, "B"
-    if kernel == "ordered_block_sums_kernel":
+    if kernel == "ordered_offsets_kernel":
         return "hbm", 8 * n, "B"
     if kernel == "emit_ordered_kernel":
         return "hbm", 12 * n + (slot_bytes + 4) * k, "B"

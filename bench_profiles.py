@@ -169,7 +169,7 @@ def algorithmic_bytes(bench):
     n, w, h, deg = int(m.group(2)), int(m.group(3)), int(m.group(4)), int(m.group(5))
     out = {}
     for k in ("project_fwd_kernel", "gaussian_bwd_kernel", "hist32_kernel", "depth_hist_kernel", "onesweep32_kernel<sort>",
-              "ordered_block_sums_kernel", "emit_ordered_kernel", "onesweep32_kernel<tile partition>"):
+              "ordered_offsets_kernel", "emit_ordered_kernel", "onesweep32_kernel<tile partition>"):
         bound, work, _ = bench_module.algorithmic_work(k, n, cfg["num_keys"], w * h, cfg["lists"], (deg + 1) ** 2, None,
                                                        cfg.get("gaussians_with_gradient", 0),
                                                        (w + 15) // 16 <= 255 and (h + 15) // 16 <= 255,

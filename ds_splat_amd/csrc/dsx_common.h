@@ -305,6 +305,7 @@ struct OrderLayout
     size_t cover;      // int32[(ntx + 1) * (nty + 1) + 1] pairs per tile (corner grid, then its 2-D prefix sum)
     size_t bin_cover;  // int32[(nbx + 1) * (nby + 1) + 1] the same per bin (binned lists only)
     size_t key_count;  // uint64[3]  pairs of the per-tile lists, pairs of the bin lists (summed by the corner-grid kernel), workgroups done
+    size_t offsets;    // uint64[...] what the workgroups of the kernel that fills block_sums tell each other, zeroed with the corner grids
     size_t ranges;     // int32[...] ranges_layout() without its `walk` part, ready before the pairs exist
     size_t sort;       // Sort32Workspace
     size_t bytes;
@@ -326,8 +327,8 @@ struct ListsWorkspace
 ListsWorkspace lists_workspace(int64_t k, int num_tiles, bool binned);
 
 // launchers (each returns a dsx_status)
-// Three words of pinned host memory that receive a call's pair counts and the range of its depth keys (null: none), each
-// marked with the call's ticket.
+// Four words of pinned host memory that receive a call's pair counts, the range of its depth keys and how many of them emit (null:
+// none), each marked with the call's ticket.
 struct HostCounts
 {
     unsigned long long* words = nullptr;
