@@ -93,9 +93,10 @@ __device__ __forceinline__ int sh_basis(int deg, float3 d, float* Y)
 // workgroups are resident at once whenever the list below can hold a run (12 per CU: at most 168
 // VGPRs, 10 KB of LDS): a scene where few Gaussians have work then costs one pass of latency (find the
 // few, do them) instead of one per wave of workgroups, and a scene where all have work gives every
-// wavefront the same share.
+// wavefront the same share.  A run is no longer than that asks for, down to one round of 64: with few Gaussians the rounds of a
+// run, one after another, are the kernel's time (runs of at least 256: 50 K of degree 3 22.4 us, now 8.8; 100 K of degree 0
+// 18.4 -> 11.9; 300 K with colours 13.7 -> 12.3; 500 K and 1 M, of which few have work, 11.5 and 11.2 either way).
 constexpr int kBwdListMax = 2048;  // longest run (its list of Gaussians with work sits in LDS)
-constexpr int kBwdRunMin = 256;
 constexpr int kBwdResidentPerCu = 12;
 
 // does any of the nine sums of an accumulator row differ from zero? (a NaN does)
@@ -554,7 +555,7 @@ int launch_gaussian_bwd(const dsx_camera& cam, int64_t n, int num_bases, const f
     // runs that make all workgroups resident at once, if the list can hold such a run
     const int64_t resident = (int64_t)compute_units() * kBwdResidentPerCu;
     const int64_t even = ((n + resident - 1) / resident + DSX_WAVE - 1) / DSX_WAVE * DSX_WAVE;
-    p.run = (int)max((int64_t)kBwdRunMin, min(even, (int64_t)kBwdListMax));
+    p.run = (int)min(even, (int64_t)kBwdListMax);
     const int64_t blocks = (n + p.run - 1) / p.run;
     {
         DSX_TIMED("gaussian_bwd_kernel", stream);
