@@ -92,7 +92,9 @@ def trace_name(short):
         # tile partition, with 16-bit slots per tile or 32-bit slot words per bin, does neither
         carry, bits = [a.strip() for a in short[short.index("<") + 1:short.rindex(">")].split(",")][3:5]
         return "onesweep32_kernel<sort>" if carry == "true" or bits != "8" else "onesweep32_kernel<tile partition>"
-    return base.replace("_tile_kernel", "_kernel") if base.startswith("blend_") else base
+    if base == "onesweep32_first_kernel":
+        return "onesweep32_kernel<sort>"
+    return re.sub("_(tile|wide)_kernel$", "_kernel", base) if base.startswith("blend_") else base
 
 
 def git_commit():

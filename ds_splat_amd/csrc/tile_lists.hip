@@ -252,9 +252,8 @@ struct KeyRange
 {
     uint32_t first, behind, emitting;
 };
-template <typename KeyT, int kSort32Threads, int kSort32Items, bool kCarry, int kBits, bool kFirst = false>
-// (eight wavefronts per SIMD: two workgroups per compute unit whatever the tile)
-__global__ __launch_bounds__(kSort32Threads) __attribute__((amdgpu_waves_per_eu(8))) void onesweep32_kernel(
+template <typename KeyT, int kSort32Threads, int kSort32Items, bool kCarry, int kBits, bool kFirst>
+__device__ __forceinline__ void onesweep32_pass(
     const KeyT* __restrict__ keys_in, const uint32_t* __restrict__ vals_in, KeyT* __restrict__ keys_out,
     uint32_t* __restrict__ vals_out, int64_t count, int shift, uint32_t mask, const uint32_t* __restrict__ hist_counts,
     uint32_t* status, uint32_t* tile_counter, uint32_t* error_flag, const RectJob rects,
@@ -578,6 +577,28 @@ __global__ __launch_bounds__(kSort32Threads) __attribute__((amdgpu_waves_per_eu(
     }
 }
 
+// (eight wavefronts per SIMD: two workgroups per compute unit whatever the tile)
+template <typename KeyT, int kSort32Threads, int kSort32Items, bool kCarry, int kBits>
+__global__ __launch_bounds__(kSort32Threads) __attribute__((amdgpu_waves_per_eu(8))) void onesweep32_kernel(
+    const KeyT* __restrict__ keys_in, const uint32_t* __restrict__ vals_in, KeyT* __restrict__ keys_out,
+    uint32_t* __restrict__ vals_out, int64_t count, int shift, uint32_t mask, const uint32_t* __restrict__ hist_counts,
+    uint32_t* status, uint32_t* tile_counter, uint32_t* error_flag, const RectJob rects)
+{
+    onesweep32_pass<KeyT, kSort32Threads, kSort32Items, kCarry, kBits, false>(
+        keys_in, vals_in, keys_out, vals_out, count, shift, mask, hist_counts, status, tile_counter, error_flag, rects, KeyRange{});
+}
+
+// the first pass of the depth sort over a known range
+template <int kSort32Items, bool kCarry>
+__global__ __launch_bounds__(kSortThreads32) __attribute__((amdgpu_waves_per_eu(8))) void onesweep32_first_kernel(
+    const uint32_t* __restrict__ keys_in, uint32_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out, int64_t count, int shift,
+    uint32_t mask, const uint32_t* __restrict__ hist_counts, uint32_t* status, uint32_t* tile_counter, uint32_t* error_flag,
+    const RectJob rects, const KeyRange range)
+{
+    onesweep32_pass<uint32_t, kSortThreads32, kSort32Items, kCarry, kDepthBits, true>(
+        keys_in, nullptr, keys_out, vals_out, count, shift, mask, hist_counts, status, tile_counter, error_flag, rects, range);
+}
+
 Sort32Workspace sort32_workspace(int64_t count, int key_bits, int tile_keys)
 {
     auto align = [](size_t x) { return (x + 255) & ~(size_t)255; };
@@ -656,7 +677,7 @@ static int sort32_passes(int64_t count, int key_bits, KeyT* keys_a, uint32_t* va
                                stream, (const KeyT*)kin, (const uint32_t*)((p == 0 && iota_values) ? nullptr : vin),
                                (last && !keep_keys) ? (KeyT*)nullptr : kout, vout, count, plan.shift[p], plan.mask[p],
                                raw + p * kBins32, status + (size_t)p * w.tiles * kBins32,
-                               counters + p, counters + w.passes, job, KeyRange{});
+                               counters + p, counters + w.passes, job);
         }
         DSX_LAUNCH_CHECK();
         KeyT* tk = kin;
@@ -1811,29 +1832,34 @@ static int launch_depth_sort(int64_t n, char* base, const OrderLayout& o, int64_
             job.gather_src = rects;
             job.gather_dst = rects_sorted;
         }
-        const KeyRange keys = {first ? range.first : 0u, first ? range.behind : 0xffffffffu, (uint32_t)*emitting};
+        const KeyRange keys = {range.first, range.behind, (uint32_t)*emitting};
         const uint32_t* const keys_in = p & 1 ? keys_b : keys_a;
         uint32_t* const keys_out = last ? nullptr : (p & 1 ? keys_a : keys_b);
         const uint32_t* const vals_in = first ? nullptr : (p & 1 ? ids_a : ids_b);
         uint32_t* const vals_out = p & 1 ? ids_b : ids_a;
         DSX_TIMED(label, stream);
-#define DSX_DEPTH_PASS(ITEMS, CARRY, FIRST)                                                                             \
-    hipLaunchKernelGGL((onesweep32_kernel<uint32_t, kSortThreads32, ITEMS, CARRY, kDepthBits, FIRST>), dim3(tiles),      \
-                       dim3(kSortThreads32), 0, stream, keys_in, vals_in, keys_out, vals_out, count,                     \
-                       range.digits.shift[p], range.digits.mask[p],                                                    \
-                       reinterpret_cast<const uint32_t*>(ws + w.hist) + p * kDepthBins,                                \
-                       reinterpret_cast<uint32_t*>(ws + w.status) + (size_t)p * w.tiles * kDepthBins, counters + p,     \
-                       counters + w.passes, job, keys)
+        const uint32_t* const counts = reinterpret_cast<const uint32_t*>(ws + w.hist) + p * kDepthBins;
+        uint32_t* const status = reinterpret_cast<uint32_t*>(ws + w.status) + (size_t)p * w.tiles * kDepthBins;
+#define DSX_DEPTH_PASS(ITEMS, CARRY)                                                                                    \
+    if(first)                                                                                                           \
+        hipLaunchKernelGGL((onesweep32_first_kernel<ITEMS, CARRY>), dim3(tiles), dim3(kSortThreads32), 0, stream,        \
+                           keys_in, keys_out, vals_out, count, range.digits.shift[p], range.digits.mask[p], counts,     \
+                           status, counters + p, counters + w.passes, job, keys);                                       \
+    else                                                                                                                \
+        hipLaunchKernelGGL((onesweep32_kernel<uint32_t, kSortThreads32, ITEMS, CARRY, kDepthBits>), dim3(tiles),         \
+                           dim3(kSortThreads32), 0, stream, keys_in, vals_in, keys_out, vals_out, count,                \
+                           range.digits.shift[p], range.digits.mask[p], counts, status, counters + p,                  \
+                           counters + w.passes, job)
 #define DSX_DEPTH_PASS_ITEMS(ITEMS)         \
     case ITEMS:                             \
-        if(carry && first)                  \
-            DSX_DEPTH_PASS(ITEMS, true, true);   \
-        else if(carry)                      \
-            DSX_DEPTH_PASS(ITEMS, true, false);  \
-        else if(first)                      \
-            DSX_DEPTH_PASS(ITEMS, false, true);  \
+        if(carry)                           \
+        {                                   \
+            DSX_DEPTH_PASS(ITEMS, true);    \
+        }                                   \
         else                                \
-            DSX_DEPTH_PASS(ITEMS, false, false); \
+        {                                   \
+            DSX_DEPTH_PASS(ITEMS, false);   \
+        }                                   \
         break
         switch(items)
         {
