@@ -1304,7 +1304,7 @@ __global__ __launch_bounds__(kCoverThreads) void tile_counts_kernel(const Counts
 // ---------------------------------------------------------------------------------------
 // few Gaussians: depth order and counting in one launch or two
 // ---------------------------------------------------------------------------------------
-// Up to 24576 Gaussians the digit passes, their histogram, the block sums and the scan are eight launches
+// Up to 24576 Gaussians the digit passes, their histogram and the offsets (a sum and a scan when this was measured) are launches
 // of 3 to 8 us that each do a microsecond's work (2 K Gaussians: 38 us of kernels, 16 K: 50 us).  Here a workgroup
 // sorts 2048 keys in its own LDS and registers (by the digits of the keys' distance from the smallest one, three
 // or fewer for any scene whose depths stay within a factor of eight), and one more (two, for binned lists)
