@@ -1527,17 +1527,17 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(5, 5))
     const float* __restrict__ bg, float* grads, uint8_t* marks, int W, int H, int ntx, uint32_t last_id, int k,
     const int32_t* __restrict__ header, int header_shift, int planar, const BinLists lists, const ZeroJobs zeros)
 {
-    __shared__ float4 s_records[3 * kBwdBatch + 1];
-    float4* const s_a = s_records;                 // pixel x, pixel y, conic a/2, conic b
-    float4* const s_c = s_records + kBwdBatch;     // red, green, blue
-    float4* const s_b = s_records + 2 * kBwdBatch; // conic c/2, opacity, limit of sigma's bits, index in the sorted key array
-                                                   // (and one more: nobody's entry, as in the forward)
+    // (one place more in two of them: nobody's entry, as in the forward; its colour, which nobody looks at, is another's word)
+    __shared__ float4 s_records[3 * kBwdBatch + 2];
+    float4* const s_c = s_records;                     // red, green, blue
+    float4* const s_a = s_records + kBwdBatch;         // pixel x, pixel y, conic a/2, conic b
+    float4* const s_b = s_records + 2 * kBwdBatch + 1; // conic c/2, opacity, limit of sigma's bits, index in the sorted key array
     __shared__ double s_sum[kBwdBatch * kSums + 1]; // (nobody's zeros are added to others' sums)
     __shared__ uint4 s_list[kQuads * kBwdBatch / 16 + 1];
     // while a round is staged, in the records' memory: candidates and the scan's queue, as in the forward
     int2* const s_cand = reinterpret_cast<int2*>(s_records);
     int* const s_queue = reinterpret_cast<int*>(s_records + DSX_WAVE);
-    static_assert(DSX_WAVE + DSX_WAVE / 4 <= 3 * kBwdBatch && kBwdBatch % 2 == 0 && (kQuads * kBwdBatch) % 16 == 0 &&
+    static_assert(DSX_WAVE + DSX_WAVE / 4 <= 2 * kBwdBatch && kBwdBatch % 2 == 0 && (kQuads * kBwdBatch) % 16 == 0 &&
                       kQuads * kBwdBatch / 16 <= DSX_WAVE, "what the records' memory holds; lists of pairs of bytes, cleared by words");
 
     const int lane = threadIdx.x;
@@ -1582,7 +1582,8 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(5, 5))
     m = __builtin_amdgcn_readfirstlane(m);
     if(lane == 0)
     {
-        // (whatever stands in the other two words, its sigma is NaN: no pixel takes it)
+        // (its sigma is NaN: no pixel takes it.  Its centre is finite, or a pixel's zeros times the distance to it would not be zero)
+        s_a[kBwdBatch] = make_float4(0.f, 0.f, 0.f, 0.f);
         s_b[kBwdBatch] = make_float4(__builtin_nanf(""), 0.f, 0.f, __int_as_float(INT_MAX));
     }
 
