@@ -1,4 +1,4 @@
-"""Records that stretch the blend kernels' arithmetic: colours that are not finite."""
+"""Records that stretch the blend kernels' arithmetic: colours that are not finite, splats of hundreds of pixels' length."""
 import numpy as np
 import pytest
 import torch
@@ -68,3 +68,40 @@ def test_an_infinite_colour_that_no_pixel_takes(blend_form, pixels_per_lane, val
         assert (idx.cpu() == k - 1).any()
         assert (grads[3] == 0.0).all(), (behind, grads[3])
         assert torch.isfinite(grads).all() and (grads[0] != 0.0).any()
+
+
+@pytest.mark.parametrize("length", [150.0, 800.0])
+@pytest.mark.parametrize("pixels_per_lane", [0, 1, 4])
+def test_a_needle_is_blended_wherever_alpha_reaches_the_threshold(blend_form, pixels_per_lane, length):
+    """Splats of hundreds of pixels' length and less than one pixel's width, each in a tile far from its middle: the
+    terms of its exponent, up to 1e6, cancel, so what a test of the whole tile or of a block finds lies further from
+    the pixels' own exponents than a fixed slack.  With an opacity for which alpha reaches 1/255 at a pixel of
+    the tile or a few, both directions take just the pixels that comparing alpha takes (4096 tiles: with the form left
+    to the library, the two directions run different ones)."""
+    tiles, side = 4096, 64
+    g = torch.Generator().manual_seed(11)
+    rand = lambda *s: torch.rand(*s, generator=g, dtype=torch.float64)
+    angle, across, along = 2.0 * np.pi * rand(tiles), 20.0 * rand(tiles) - 10.0, length * (0.1 + 0.9 * rand(tiles))
+    cos, sin = torch.cos(angle), torch.sin(angle)
+    mean = torch.stack([7.5 + along * cos - across * sin, 7.5 + along * sin + across * cos], 1).float()
+    major, minor = 1.0 / length ** 2, 1.0 / (0.3 + 0.3 * rand(tiles))
+    conic = torch.stack([major * cos ** 2 + minor * sin ** 2, (major - minor) * cos * sin,
+                         major * sin ** 2 + minor * cos ** 2], 1).float()
+    by_tile = lambda x: x.view(side, 16, side, 16).permute(0, 2, 1, 3).reshape(tiles, 256)
+    blend_form(1)       # alpha, from an opacity whose reach lies far above
+    alpha = by_tile(o.one_splat_per_tile(torch.full((tiles,), 0.9), mean, conic)["image"][..., 0].contiguous())
+    most = alpha.max(1).values.double()
+    crossed = (most > 2.0 / 255.0) & (most < 0.88)
+    assert crossed.float().mean() > 0.6
+    opacity = torch.where(crossed, 0.9 * (1.0 + 1e-5) / 255.0 / most.clamp_min(1e-3), 0.0).float()
+    twice = by_tile(o.one_splat_per_tile(opacity * 2.0, mean, conic)["image"][..., 0].contiguous()) * 0.5
+    takes = twice >= torch.tensor(1.0) / 255.0
+    assert (takes.any(1) == crossed).all()
+    blend_form(pixels_per_lane)
+    v = torch.ones(16 * side, 16 * side, 3)
+    got = o.one_splat_per_tile(opacity, mean, conic, v_image=v)
+    missed = (by_tile(got["image"][..., 0].contiguous()) > 0) != takes
+    assert not missed.any(), "forward: %d tiles of %d" % (int(missed.any(1).sum()), int(crossed.sum()))
+    want = torch.where(takes, twice, torch.zeros(())).double().sum(1)
+    # (a pixel more or less is 1/255 of colour 1: from sums of up to 16 pixels)
+    np.testing.assert_allclose(got["grads"][:, 6].double().numpy(), want.numpy(), rtol=1e-5, atol=1e-7)
