@@ -129,7 +129,7 @@ extern "C" const char* dsx_error_string(int status)
 
 extern "C" int dsx_version(void)
 {
-    return 310;
+    return 311;
 }
 
 extern "C" int64_t dsx_num_blocks(int64_t n)
@@ -359,7 +359,7 @@ extern "C" int dsx_sort_pairs_u32(int64_t count, int32_t key_bits, uint32_t* key
     return DSX_OK;
 }
 
-extern "C" int dsx_depth_order(const dsx_camera* cam, int64_t n, void* order, size_t order_bytes, void* stream)
+static int check_depth_order(const dsx_camera* cam, int64_t n, const void* order, size_t order_bytes)
 {
     if(int rc = check_camera(cam))
         return rc;
@@ -371,7 +371,13 @@ extern "C" int dsx_depth_order(const dsx_camera* cam, int64_t n, void* order, si
         return DSX_ERR_BAD_ARG;
     if(order_bytes < order_layout(n, cam->image_width, cam->image_height, camera_bin(*cam)).bytes)
         return DSX_ERR_WORKSPACE;
-    return launch_depth_order(*cam, n, order, as_stream(stream));
+    return DSX_OK;
+}
+
+extern "C" int dsx_depth_order(const dsx_camera* cam, int64_t n, void* order, size_t order_bytes, void* stream)
+{
+    const int rc = check_depth_order(cam, n, order, order_bytes);
+    return rc || n == 0 ? rc : launch_depth_order(*cam, n, order, as_stream(stream));
 }
 
 extern "C" int dsx_order_view(int64_t n, const void* order, const uint32_t** depth_order,
@@ -606,6 +612,18 @@ extern "C" int dsx_forward_project_begin(const dsx_camera* cam, int64_t n, const
     if(to_host.words == nullptr)
         return DSX_ERR_RUNTIME;
     return launch_depth_order(*cam, n, order, as_stream(stream), true, to_host);
+}
+
+extern "C" int dsx_depth_order_bounded(const dsx_camera* cam, int64_t n, void* order, size_t order_bytes,
+                                       int32_t offset_polls, void* stream)
+{
+    const int rc = check_depth_order(cam, n, order, order_bytes);
+    if(rc || n == 0)
+        return rc;
+    const HostCounts to_host = next_counts();
+    if(to_host.words == nullptr)
+        return DSX_ERR_RUNTIME;
+    return launch_depth_order(*cam, n, order, as_stream(stream), false, to_host, offset_polls);
 }
 
 extern "C" int dsx_forward_project_counts(const dsx_camera* cam, int64_t n, int64_t* num_keys, void* stream)

@@ -199,7 +199,6 @@ constexpr uint32_t kFlagAggregate32 = 1u << 30;
 constexpr uint32_t kFlagInclusive32 = 2u << 30;
 constexpr uint32_t kFlagMask32 = 3u << 30;
 constexpr uint32_t kValueMask32 = ~kFlagMask32;
-constexpr int kSpinLimit32 = 1 << 18; // bounded wait: a stuck predecessor ends in an error flag, not a hang
 #ifndef DSX_LOOK32
 #define DSX_LOOK32 4
 #endif
@@ -1881,8 +1880,9 @@ static int launch_depth_sort(int64_t n, char* base, const OrderLayout& o, int64_
 // to_host (optional): words of pinned host memory that receive the pair counts (per-tile lists: what the
 // reference calls K, the fine ranges and final_idx index that many pairs; bin lists, zero when the lists
 // are per tile) as soon as the rectangles have been counted, while the sort still runs.
+// offset_polls: how often a workgroup of ordered_offsets_kernel looks for another's word before it does without
 int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_t stream, bool already_cleared,
-                       HostCounts to_host)
+                       HostCounts to_host, int offset_polls)
 {
     if(n <= 0)
         return DSX_OK;
@@ -2005,7 +2005,7 @@ int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_
         DSX_TIMED("ordered_offsets_kernel", stream);
         hipLaunchKernelGGL(ordered_offsets_kernel, dim3((unsigned)((n + kOffsetsShare - 1) / kOffsetsShare)), dim3(kOffsetsThreads), 0, stream,
                            reinterpret_cast<uint2*>(base + o.rects_sorted), n, emitting, list_grid(cam).shift, block_sums,
-                           reinterpret_cast<unsigned long long*>(base + o.offsets), kSpinLimit32);
+                           reinterpret_cast<unsigned long long*>(base + o.offsets), offset_polls);
     }
     return finish(hipGetLastError() != hipSuccess ? DSX_ERR_LAUNCH : DSX_OK);
 }

@@ -116,6 +116,13 @@ def depth_order(cam, n, order):
     return depth_order_view(n, order)
 
 
+def depth_order_bounded(cam, n, order, offset_polls):
+    """The same as a whole forward runs it, with another limit on the block offsets' waits (see dsx.h)."""
+    lib = N.load()
+    N.check(lib.dsx_depth_order_bounded(cam.ref, n, _ptr(order), order.numel(), int(offset_polls), _stream()))
+    return depth_order_view(n, order)
+
+
 def depth_order_view(n, order):
     lib = N.load()
     p_order, p_off = C.c_void_p(), C.c_void_p()

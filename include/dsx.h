@@ -96,7 +96,7 @@ typedef struct dsx_camera
  */
 
 const char* dsx_error_string(int status);
-/* 100 * major + minor.  310: flags beside dsx_camera::list_bin, the projection's wait for the pair
+/* 100 * major + minor.  311: dsx_depth_order_bounded.  310: flags beside dsx_camera::list_bin, the projection's wait for the pair
  * counts is a function of its own.  300: the bin size of the tile lists is an argument (dsx_camera::list_bin and
  * the size helpers) instead of a process-wide setting; the `ranges` buffer carries it in a header word;
  * the blend entry points and the backward are told n and k and follow no id or list position beyond
@@ -393,6 +393,13 @@ int dsx_trace_read(dsx_trace_entry* out /* host */, int max_entries);
  * 1 or 4) or returns the choice to the library (0).  Results of the forward are bit-identical in
  * both forms.  For tests, which run both forms at every size.  No counterpart in the reference. */
 int dsx_set_blend_pixels_per_lane(int pixels);
+
+/* dsx_depth_order as dsx_forward_project runs it (above 262144 Gaussians the host waits for the range of the depths), with
+ * another limit on its waits.  The workgroups that make the block offsets tell each other their sums, and one that has
+ * looked offset_polls times for another's in vain (a negative number: that finds it missing once) sums up the other's
+ * rectangles itself: the offsets are the same.  For tests; the other entry points look 2^18 times. */
+int dsx_depth_order_bounded(const dsx_camera* cam, int64_t n, void* order, size_t order_bytes,
+                            int32_t offset_polls, void* stream);
 
 #ifdef __cplusplus
 }

@@ -143,6 +143,32 @@ def test_depth_order_of_a_cloud_that_is_partly_out_of_sight(n, bins, out):
         assert set(np.unique(st.ids.cpu().numpy()).tolist()) == set(np.nonzero(touched)[0].tolist())
 
 
+@pytest.mark.parametrize("polls", [-1, 3])
+@pytest.mark.parametrize("bins", [1, 4])
+@pytest.mark.parametrize("n,seen", [(24577, 1.0), (28673, 0.5), (262145, 0.3), (530001, 1.0), (1300001, 0.6)])
+def test_block_offsets_of_workgroups_that_do_not_wait(n, seen, bins, polls):
+    """A workgroup that finds another's sum missing adds up the other's rectangles itself: the offsets are those of
+    workgroups that wait, where the last share, the last run and the last Gaussian that emits end anywhere."""
+    from ds_splat_amd import stages
+    sc = make_scene("cfg0", n=n, width=520, height=300, sh_degree=0, seed=9)
+    means = sc["means_3d"].clone()
+    gone = torch.rand(n, generator=torch.Generator().manual_seed(n)) >= seen
+    means[gone, 0] = 1e4
+    cam = stages.camera_from_scene(sc, DEV, list_bin=bins)
+    order = stages.new_order(cam, n, DEV)
+    splats, _, _, _ = stages.project_fwd(cam, means.to(DEV), sc["scales"].to(DEV), sc["rotations"].to(DEV),
+                                         sc["opacities"].to(DEV), sc["shs"].to(DEV), order=order)
+    again = order.clone()
+    perm, offsets = (x.clone() for x in stages.depth_order_bounded(cam, n, order, 1 << 18))
+    perm2, offsets2 = stages.depth_order_bounded(cam, n, again, polls)
+    assert torch.equal(perm, perm2) and torch.equal(offsets, offsets2)
+    assert int(offsets[-1]) > 0 and bool((offsets[1:] >= offsets[:-1]).all())
+    if bins == 1:
+        touched = splats[:, 11].contiguous().view(torch.int32).to(torch.int64)
+        touched[-1] = 0
+        assert int(offsets[-1]) == int(touched.sum())
+
+
 @pytest.mark.parametrize("pixels_per_lane", [1, 4])
 def test_bin_lists_beyond_two_to_the_thirty(blend_form, pixels_per_lane):
     """Positions of a bin's list that a 32-bit byte offset does not reach: the same lists, moved behind 2^30 others,
