@@ -615,7 +615,7 @@ extern "C" int dsx_forward_project_begin(const dsx_camera* cam, int64_t n, const
 }
 
 extern "C" int dsx_depth_order_bounded(const dsx_camera* cam, int64_t n, void* order, size_t order_bytes,
-                                       int32_t offset_polls, void* stream)
+                                       int32_t sort_polls, int32_t offset_polls, void* stream)
 {
     const int rc = check_depth_order(cam, n, order, order_bytes);
     if(rc || n == 0)
@@ -623,7 +623,7 @@ extern "C" int dsx_depth_order_bounded(const dsx_camera* cam, int64_t n, void* o
     const HostCounts to_host = next_counts();
     if(to_host.words == nullptr)
         return DSX_ERR_RUNTIME;
-    return launch_depth_order(*cam, n, order, as_stream(stream), false, to_host, offset_polls);
+    return launch_depth_order(*cam, n, order, as_stream(stream), false, to_host, sort_polls, offset_polls);
 }
 
 extern "C" int dsx_forward_project_counts(const dsx_camera* cam, int64_t n, int64_t* num_keys, void* stream)

@@ -336,15 +336,16 @@ struct HostCounts
 };
 constexpr int kTicketShift = 44; // a count is cut off at 2^43: far beyond what a call accepts
 
+// Of the bounded waits: a stuck predecessor ends in an error flag (a sort's pass) or in doing without it (the block offsets), not in a hang.
+constexpr int kSpinLimit32 = 1 << 18;
 int launch_sort32(int64_t count, int key_bits, uint32_t* keys_a, uint32_t* vals_a, uint32_t* keys_b,
                   uint32_t* vals_b, bool iota_values, bool keep_keys, void* sort_ws, hipStream_t stream,
                   uint32_t** keys_out, uint32_t** vals_out, const uint2* gather_src = nullptr,
                   uint2* gather_dst = nullptr, bool already_cleared = false, uint32_t* carry_a = nullptr,
-                  uint32_t* carry_b = nullptr);
-constexpr int kSpinLimit32 = 1 << 18; // of bounded waits: a stuck predecessor ends in an error flag, or in doing without it, not in a hang
+                  uint32_t* carry_b = nullptr, int polls = kSpinLimit32);
 // already_cleared: the words of depth_order_clear_region are zero already (the projection did it)
 int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_t stream, bool already_cleared = false,
-                       HostCounts to_host = {}, int offset_polls = kSpinLimit32);
+                       HostCounts to_host = {}, int sort_polls = kSpinLimit32, int offset_polls = kSpinLimit32);
 // waits for a word of the calling thread's `to_host` (false: the stream has ended without it)
 bool wait_for_word(const HostCounts& to_host, int word, hipStream_t stream, uint64_t* value);
 // the part of an `order` buffer that must be zero when launch_depth_order starts

@@ -235,6 +235,7 @@ struct RectJob
 {
     const uint2* gather_src;
     uint2* gather_dst;
+    uint32_t last_value; // of those that gather_src has a record for
     const uint2* pack_src;
     const uint32_t* carry_in;
     uint32_t* carry_out;
@@ -247,6 +248,8 @@ struct RectJob
 // `first`, of which a key without pairs has none: it becomes `behind`, stands behind the digits in its tile, and its value goes to
 // its final place, behind the `emitting` others in the order of the input (how many lie in the tiles before is those tiles' keys
 // less the sum of the digits' counts that the chained scan brings).  Later passes see the others only.
+// polls: of a status that is not there, before a tile gives up (below zero: it does not look at all).  Its keys' places are then wrong, and so is what it leaves to later
+// passes: no place is taken beyond the last one, and no value for a record's index beyond the last one.
 struct KeyRange
 {
     uint32_t first, behind, emitting;
@@ -255,7 +258,7 @@ template <typename KeyT, int kSort32Threads, int kSort32Items, bool kCarry, int 
 __device__ __forceinline__ void onesweep32_pass(
     const KeyT* __restrict__ keys_in, const uint32_t* __restrict__ vals_in, KeyT* __restrict__ keys_out,
     uint32_t* __restrict__ vals_out, int64_t count, int shift, uint32_t mask, const uint32_t* __restrict__ hist_counts,
-    uint32_t* status, uint32_t* tile_counter, uint32_t* error_flag, const RectJob rects,
+    uint32_t* status, uint32_t* tile_counter, uint32_t* error_flag, int polls, const RectJob rects,
     const KeyRange range)
 {
     const uint2* __restrict__ gather_src = rects.gather_src;
@@ -450,7 +453,9 @@ __device__ __forceinline__ void onesweep32_pass(
         {
             int64_t t = tile - 1; // next predecessor to account for
             int spins = 0;
-            bool done = false;
+            bool done = polls < 0;
+            if(done)
+                *error_flag = 1u;
             while(!done)
             {
                 uint32_t v[kLookBatch32];
@@ -468,7 +473,7 @@ __device__ __forceinline__ void onesweep32_pass(
                         break;
                     if((v[b] & kFlagMask32) == 0)
                     {
-                        if(++spins > kSpinLimit32)
+                        if(++spins > polls)
                         {
                             *error_flag = 1u;
                             done = true;
@@ -506,6 +511,7 @@ __device__ __forceinline__ void onesweep32_pass(
     }
 
     // ---- scatter keys: consecutive threads -> consecutive addresses inside a digit's run ----
+    const uint32_t last_place = (uint32_t)(count - 1);
     uint32_t out[kSort32Items];            // where the key at tile position it * threads + tid goes
     uint32_t no_record = 0;                // bit it: that key is kNoPairsKey (its record is known to be zero)
 #pragma unroll
@@ -518,7 +524,7 @@ __device__ __forceinline__ void onesweep32_pass(
         {
             const uint32_t kk = s_keys[j];
             const uint32_t digit_base = s_gbase[digit_of(kk)];
-            out[it] = (!kFirst || j < emitters ? digit_base : tail) + (uint32_t)j;
+            out[it] = min((!kFirst || j < emitters ? digit_base : tail) + (uint32_t)j, last_place);
             if(gather_src && kk == kNoPairsKey)
                 no_record |= 1u << it;
             if(keys_out && (!kFirst || j < emitters))
@@ -547,7 +553,7 @@ __device__ __forceinline__ void onesweep32_pass(
             // optional: a per-value record follows its value to the sorted position (the random
             // gather overlaps with the scatter traffic of the pass)
             if(gather_src)
-                gather_dst[out[it]] = ((no_record >> it) & 1u) ? make_uint2(0u, 0u) : gather_src[v];
+                gather_dst[out[it]] = ((no_record >> it) & 1u) ? make_uint2(0u, 0u) : gather_src[min(v, rects.last_value)];
         }
     }
     if(kCarry)
@@ -581,10 +587,11 @@ template <typename KeyT, int kSort32Threads, int kSort32Items, bool kCarry, int 
 __global__ __launch_bounds__(kSort32Threads) __attribute__((amdgpu_waves_per_eu(8))) void onesweep32_kernel(
     const KeyT* __restrict__ keys_in, const uint32_t* __restrict__ vals_in, KeyT* __restrict__ keys_out,
     uint32_t* __restrict__ vals_out, int64_t count, int shift, uint32_t mask, const uint32_t* __restrict__ hist_counts,
-    uint32_t* status, uint32_t* tile_counter, uint32_t* error_flag, const RectJob rects)
+    uint32_t* status, uint32_t* tile_counter, uint32_t* error_flag, int polls, const RectJob rects)
 {
     onesweep32_pass<KeyT, kSort32Threads, kSort32Items, kCarry, kBits, false>(
-        keys_in, vals_in, keys_out, vals_out, count, shift, mask, hist_counts, status, tile_counter, error_flag, rects, KeyRange{});
+        keys_in, vals_in, keys_out, vals_out, count, shift, mask, hist_counts, status, tile_counter, error_flag, polls, rects,
+        KeyRange{});
 }
 
 // the first pass of the depth sort over a known range
@@ -592,10 +599,11 @@ template <int kSort32Items, bool kCarry>
 __global__ __launch_bounds__(kSortThreads32) __attribute__((amdgpu_waves_per_eu(8))) void onesweep32_first_kernel(
     const uint32_t* __restrict__ keys_in, uint32_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out, int64_t count, int shift,
     uint32_t mask, const uint32_t* __restrict__ hist_counts, uint32_t* status, uint32_t* tile_counter, uint32_t* error_flag,
-    const RectJob rects, const KeyRange range)
+    int polls, const RectJob rects, const KeyRange range)
 {
     onesweep32_pass<uint32_t, kSortThreads32, kSort32Items, kCarry, kDepthBits, true>(
-        keys_in, nullptr, keys_out, vals_out, count, shift, mask, hist_counts, status, tile_counter, error_flag, rects, range);
+        keys_in, nullptr, keys_out, vals_out, count, shift, mask, hist_counts, status, tile_counter, error_flag, polls, rects,
+        range);
 }
 
 Sort32Workspace sort32_workspace(int64_t count, int key_bits, int tile_keys)
@@ -639,7 +647,7 @@ static int sort32_passes(int64_t count, int key_bits, KeyT* keys_a, uint32_t* va
                          bool iota_values, bool keep_keys, void* sort_ws, const char* label, hipStream_t stream,
                          KeyT** keys_out, uint32_t** vals_out, const uint2* gather_src = nullptr,
                          uint2* gather_dst = nullptr, const uint32_t* counts = nullptr, uint32_t* carry_a = nullptr,
-                         uint32_t* carry_b = nullptr)
+                         uint32_t* carry_b = nullptr, int polls = kSpinLimit32)
 {
     const Sort32Workspace w = sort32_workspace(count, key_bits, kThreads * kItems);
     const Digits32 plan = digits32(key_bits);
@@ -669,6 +677,7 @@ static int sort32_passes(int64_t count, int key_bits, KeyT* keys_a, uint32_t* va
         {
             job.gather_src = gather_src;
             job.gather_dst = gather_dst;
+            job.last_value = (uint32_t)(count - 1);
         }
         {
             DSX_TIMED(label, stream);
@@ -676,7 +685,7 @@ static int sort32_passes(int64_t count, int key_bits, KeyT* keys_a, uint32_t* va
                                stream, (const KeyT*)kin, (const uint32_t*)((p == 0 && iota_values) ? nullptr : vin),
                                (last && !keep_keys) ? (KeyT*)nullptr : kout, vout, count, plan.shift[p], plan.mask[p],
                                raw + p * kBins32, status + (size_t)p * w.tiles * kBins32,
-                               counters + p, counters + w.passes, job);
+                               counters + p, counters + w.passes, polls, job);
         }
         DSX_LAUNCH_CHECK();
         KeyT* tk = kin;
@@ -698,7 +707,7 @@ static int sort32_passes(int64_t count, int key_bits, KeyT* keys_a, uint32_t* va
 int launch_sort32(int64_t count, int key_bits, uint32_t* keys_a, uint32_t* vals_a, uint32_t* keys_b,
                   uint32_t* vals_b, bool iota_values, bool keep_keys, void* sort_ws, hipStream_t stream,
                   uint32_t** keys_out, uint32_t** vals_out, const uint2* gather_src, uint2* gather_dst,
-                  bool already_cleared, uint32_t* carry_a, uint32_t* carry_b)
+                  bool already_cleared, uint32_t* carry_a, uint32_t* carry_b, int polls)
 {
     *keys_out = keys_a;
     *vals_out = vals_a;
@@ -724,11 +733,12 @@ int launch_sort32(int64_t count, int key_bits, uint32_t* keys_a, uint32_t* vals_
         return carry ? sort32_passes<uint32_t, kSortThreads32, ITEMS, true>(                                          \
                            count, key_bits, keys_a, vals_a, keys_b, vals_b, iota_values, keep_keys, sort_ws,          \
                            "onesweep32_kernel<sort>", stream, keys_out, vals_out, gather_src, gather_dst, nullptr,    \
-                           carry_a, carry_b)                                                                          \
+                           carry_a, carry_b, polls)                                                                   \
                      : sort32_passes<uint32_t, kSortThreads32, ITEMS>(count, key_bits, keys_a, vals_a, keys_b, vals_b, \
                                                                       iota_values, keep_keys, sort_ws,                \
                                                                       "onesweep32_kernel<sort>", stream, keys_out,    \
-                                                                      vals_out, gather_src, gather_dst)
+                                                                      vals_out, gather_src, gather_dst, nullptr,      \
+                                                                      nullptr, nullptr, polls)
     switch(sort32_items(count))
     {
         DSX_SORT32_ITEMS(1);
@@ -979,9 +989,6 @@ __global__ __launch_bounds__(kOffsetsThreads) void ordered_offsets_kernel(uint2*
         unsigned long long v = 0;
         for(int spins = 0;; ++spins)
         {
-            v = __hip_atomic_load(state + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if(v & kReady)
-                break;
             if(spins > patience)
             {
                 v = 0;
@@ -989,6 +996,9 @@ __global__ __launch_bounds__(kOffsetsThreads) void ordered_offsets_kernel(uint2*
                     v += list_count(rects_sorted[p], shift);
                 break;
             }
+            v = __hip_atomic_load(state + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if(v & kReady)
+                break;
             __builtin_amdgcn_s_sleep(1);
         }
         before += v & ~kReady;
@@ -1745,7 +1755,7 @@ void depth_order_clear_region(const dsx_camera& cam, int64_t n, void* order, uin
 // The depth sort of a whole forward (cleared workspace): ids in `ids_a`, the rectangles of the first `emitting` of them in
 // `rects_sorted`.
 static int launch_depth_sort(int64_t n, char* base, const OrderLayout& o, int64_t blocks, bool carry,
-                             const HostCounts& to_host, hipStream_t stream, int64_t* emitting)
+                             const HostCounts& to_host, int polls, hipStream_t stream, int64_t* emitting)
 {
     if(n >= (1ll << 30))
         return DSX_ERR_TOO_LARGE;
@@ -1781,9 +1791,11 @@ static int launch_depth_sort(int64_t n, char* base, const OrderLayout& o, int64_
     case ITEMS:                                                                                                        \
         return carry ? sort32_passes<uint32_t, kSortThreads32, ITEMS, true>(n, 32, keys_a, ids_a, keys_b, ids_b, true,  \
                                                                             false, ws, label, stream, &ko, &vo, rects, \
-                                                                            rects_sorted, nullptr, packed_a, packed_b) \
+                                                                            rects_sorted, nullptr, packed_a, packed_b, \
+                                                                            polls)                                     \
                      : sort32_passes<uint32_t, kSortThreads32, ITEMS>(n, 32, keys_a, ids_a, keys_b, ids_b, true, false, \
-                                                                      ws, label, stream, &ko, &vo, rects, rects_sorted)
+                                                                      ws, label, stream, &ko, &vo, rects, rects_sorted, \
+                                                                      nullptr, nullptr, nullptr, polls)
         switch(sort32_items(n))
         {
             DSX_DEPTH_SORT_ITEMS(2);
@@ -1830,6 +1842,7 @@ static int launch_depth_sort(int64_t n, char* base, const OrderLayout& o, int64_
         {
             job.gather_src = rects;
             job.gather_dst = rects_sorted;
+            job.last_value = (uint32_t)(n - 1);
         }
         const KeyRange keys = {range.first, range.behind, (uint32_t)*emitting};
         const uint32_t* const keys_in = p & 1 ? keys_b : keys_a;
@@ -1843,12 +1856,12 @@ static int launch_depth_sort(int64_t n, char* base, const OrderLayout& o, int64_
     if(first)                                                                                                           \
         hipLaunchKernelGGL((onesweep32_first_kernel<ITEMS, CARRY>), dim3(tiles), dim3(kSortThreads32), 0, stream,        \
                            keys_in, keys_out, vals_out, count, range.digits.shift[p], range.digits.mask[p], counts,     \
-                           status, counters + p, counters + w.passes, job, keys);                                       \
+                           status, counters + p, counters + w.passes, polls, job, keys);                                \
     else                                                                                                                \
         hipLaunchKernelGGL((onesweep32_kernel<uint32_t, kSortThreads32, ITEMS, CARRY, kDepthBits>), dim3(tiles),         \
                            dim3(kSortThreads32), 0, stream, keys_in, vals_in, keys_out, vals_out, count,                \
                            range.digits.shift[p], range.digits.mask[p], counts, status, counters + p,                  \
-                           counters + w.passes, job)
+                           counters + w.passes, polls, job)
 #define DSX_DEPTH_PASS_ITEMS(ITEMS)         \
     case ITEMS:                             \
         if(carry)                           \
@@ -1880,9 +1893,8 @@ static int launch_depth_sort(int64_t n, char* base, const OrderLayout& o, int64_
 // to_host (optional): words of pinned host memory that receive the pair counts (per-tile lists: what the
 // reference calls K, the fine ranges and final_idx index that many pairs; bin lists, zero when the lists
 // are per tile) as soon as the rectangles have been counted, while the sort still runs.
-// offset_polls: how often a workgroup of ordered_offsets_kernel looks for another's word before it does without
 int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_t stream, bool already_cleared,
-                       HostCounts to_host, int offset_polls)
+                       HostCounts to_host, int sort_polls, int offset_polls)
 {
     if(n <= 0)
         return DSX_OK;
@@ -1991,12 +2003,12 @@ int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_
     // (a wait for the range: fewer Gaussians are sorted before the host could have launched the rest; us a step
     // with four digits / three: 50 K 223 / 230, 100 K 249 / 260, 300 K 493 / 491, 1 M forward 319 / 305)
     if(to_host.words && sort32_items(n) > 1)
-        rc = launch_depth_sort(n, base, o, blocks, carry, to_host, stream, &emitting);
+        rc = launch_depth_sort(n, base, o, blocks, carry, to_host, sort_polls, stream, &emitting);
     else // (four passes: the values, iota in the first, go b, a, b, a and end in ids_a)
         rc = launch_sort32(n, 32, keys_a, ids_a, keys_b, ids_b, true, false, base + o.sort, stream, &ko, &vo,
                        reinterpret_cast<const uint2*>(base + o.rects), reinterpret_cast<uint2*>(base + o.rects_sorted),
                        true, carry ? reinterpret_cast<uint32_t*>(base + o.rects_sorted) : nullptr,
-                       carry ? reinterpret_cast<uint32_t*>(base + o.rects32) : nullptr);
+                       carry ? reinterpret_cast<uint32_t*>(base + o.rects32) : nullptr, sort_polls);
     if(rc)
         return finish(rc);
     if(vo != ids_a)

@@ -116,10 +116,11 @@ def depth_order(cam, n, order):
     return depth_order_view(n, order)
 
 
-def depth_order_bounded(cam, n, order, offset_polls):
-    """The same as a whole forward runs it, with another limit on the block offsets' waits (see dsx.h)."""
+def depth_order_bounded(cam, n, order, sort_polls=1 << 18, offset_polls=1 << 18):
+    """The same as a whole forward runs it, with other limits on the kernels' waits (see dsx.h)."""
     lib = N.load()
-    N.check(lib.dsx_depth_order_bounded(cam.ref, n, _ptr(order), order.numel(), int(offset_polls), _stream()))
+    N.check(lib.dsx_depth_order_bounded(cam.ref, n, _ptr(order), order.numel(), int(sort_polls), int(offset_polls),
+                                        _stream()))
     return depth_order_view(n, order)
 
 

@@ -395,11 +395,13 @@ int dsx_trace_read(dsx_trace_entry* out /* host */, int max_entries);
 int dsx_set_blend_pixels_per_lane(int pixels);
 
 /* dsx_depth_order as dsx_forward_project runs it (above 262144 Gaussians the host waits for the range of the depths), with
- * another limit on its waits.  The workgroups that make the block offsets tell each other their sums, and one that has
- * looked offset_polls times for another's in vain (a negative number: that finds it missing once) sums up the other's
- * rectangles itself: the offsets are the same.  For tests; the other entry points look 2^18 times. */
+ * other limits on its waits, in looks for a word that is not there yet (below zero: none).
+ * A tile of a sort's pass that has looked sort_polls times gives up: the sort's flag (dsx_sort_flags) is set and the order wrong,
+ * with every access inside `order`, whatever it held.  The workgroups that make the block offsets tell each other their sums, and one that has
+ * looked offset_polls times for another's sums up the other's rectangles itself: the offsets are the same.  For
+ * tests; the other entry points look 2^18 times. */
 int dsx_depth_order_bounded(const dsx_camera* cam, int64_t n, void* order, size_t order_bytes,
-                            int32_t offset_polls, void* stream);
+                            int32_t sort_polls, int32_t offset_polls, void* stream);
 
 #ifdef __cplusplus
 }

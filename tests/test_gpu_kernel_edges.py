@@ -143,12 +143,12 @@ def test_depth_order_of_a_cloud_that_is_partly_out_of_sight(n, bins, out):
         assert set(np.unique(st.ids.cpu().numpy()).tolist()) == set(np.nonzero(touched)[0].tolist())
 
 
-@pytest.mark.parametrize("polls", [-1, 3])
+@pytest.mark.parametrize("polls", [-1, 0])
 @pytest.mark.parametrize("bins", [1, 4])
 @pytest.mark.parametrize("n,seen", [(24577, 1.0), (28673, 0.5), (262145, 0.3), (530001, 1.0), (1300001, 0.6)])
 def test_block_offsets_of_workgroups_that_do_not_wait(n, seen, bins, polls):
-    """A workgroup that finds another's sum missing adds up the other's rectangles itself: the offsets are those of
-    workgroups that wait, where the last share, the last run and the last Gaussian that emits end anywhere."""
+    """A workgroup that does not look for another's sum, or finds it missing, adds up the other's rectangles itself: the
+    offsets are those of workgroups that wait, where the last share, the last run and the last Gaussian that emits end anywhere."""
     from ds_splat_amd import stages
     sc = make_scene("cfg0", n=n, width=520, height=300, sh_degree=0, seed=9)
     means = sc["means_3d"].clone()
@@ -159,14 +159,36 @@ def test_block_offsets_of_workgroups_that_do_not_wait(n, seen, bins, polls):
     splats, _, _, _ = stages.project_fwd(cam, means.to(DEV), sc["scales"].to(DEV), sc["rotations"].to(DEV),
                                          sc["opacities"].to(DEV), sc["shs"].to(DEV), order=order)
     again = order.clone()
-    perm, offsets = (x.clone() for x in stages.depth_order_bounded(cam, n, order, 1 << 18))
-    perm2, offsets2 = stages.depth_order_bounded(cam, n, again, polls)
+    perm, offsets = (x.clone() for x in stages.depth_order_bounded(cam, n, order))
+    perm2, offsets2 = stages.depth_order_bounded(cam, n, again, offset_polls=polls)
     assert torch.equal(perm, perm2) and torch.equal(offsets, offsets2)
     assert int(offsets[-1]) > 0 and bool((offsets[1:] >= offsets[:-1]).all())
     if bins == 1:
         touched = splats[:, 11].contiguous().view(torch.int32).to(torch.int64)
         touched[-1] = 0
         assert int(offsets[-1]) == int(touched.sum())
+
+
+@pytest.mark.parametrize("n,W", [(24577, 520), (24577, 4200), (530001, 520), (530001, 4200)])
+def test_a_depth_sort_that_gives_up_stays_inside_its_buffer(n, W):
+    """Tiles that do not look at their predecessors' statuses: with four digits and three, rectangles carried and
+    gathered (beyond 255 columns of tiles), the places that their keys take, and those of what later passes make of
+    the places that nobody wrote, lie inside the buffer, and the flag says that the order is wrong."""
+    from ds_splat_amd import stages
+    sc = make_scene("cfg0", n=n, width=W, height=40, sh_degree=0, seed=9)
+    means = sc["means_3d"].clone()
+    means[torch.rand(n, generator=torch.Generator().manual_seed(n)) < 0.6, 0] = 1e4
+    cam = stages.camera_from_scene(sc, DEV, list_bin=1)
+    size, guard = stages.new_order(cam, n, DEV).numel(), 1 << 22
+    buffer = torch.full((size + guard,), 0xfe, dtype=torch.uint8, device=DEV)
+    order = buffer[:size]
+    stages.project_fwd(cam, means.to(DEV), sc["scales"].to(DEV), sc["rotations"].to(DEV), sc["opacities"].to(DEV),
+                       sc["shs"].to(DEV), order=order)
+    keys = order[:4 * n].cpu().numpy().view(np.uint32).copy()
+    perm, _ = stages.depth_order_bounded(cam, n, order, sort_polls=-1)
+    flag = int(order.view(torch.int32)[stages.sort_flag_indices(cam, n, 0, order, None)[0]].item())
+    assert bool((buffer[size:] == 0xfe).all())
+    assert flag == 1 and not (perm.cpu().numpy() == np.argsort(keys, kind="stable")).all()
 
 
 @pytest.mark.parametrize("pixels_per_lane", [1, 4])
