@@ -45,12 +45,14 @@ def measured_traffic(workload, num_keys):
                                     "scale_fetch": rec.get("scale_fetch"), "scale_write": rec.get("scale_write")}
 
 
-def algorithmic_work(kernel, n, k, pixels, lists, coeffs, counters, marked, carries_rects=True, binned=True):
+def algorithmic_work(kernel, n, k, pixels, lists, coeffs, counters, marked, carries_rects=True, binned=True, emitting=None):
     """(bound, work per launch, unit): algorithmic HBM bytes or FP32 operations per launch.
     k: pairs of the tile lists as built (per bin of tiles); lists: how many lists they are partitioned into;
     marked: Gaussians whose accumulator record received a term in the blend backward;
     binned: the lists are per bin of tiles (a pair's slot word then has 32 bits, half of them the mask of the
-    bin's tiles that its Gaussian covers, and the sorted words are kept for the blend kernels)."""
+    bin's tiles that its Gaussian covers, and the sorted words are kept for the blend kernels);
+    emitting: Gaussians that have a pair (None: all)."""
+    emitting = n if emitting is None else emitting
     slot_bytes = 4 if binned else (2 if lists + 1 <= 65535 else 4)
     if kernel == "project_fwd_kernel":
         # inputs 44 + 12c bytes, outputs radii + splat record + depth key + tile rectangle (the 3-D
@@ -67,11 +69,16 @@ def algorithmic_work(kernel, n, k, pixels, lists, coeffs, counters, marked, carr
     if kernel == "onesweep32_kernel<sort>":
         # depth sort of the Gaussians: key + id, in and out; images of at most 255 x 255 tiles also carry each
         # Gaussian's packed tile rectangle through the passes (4 bytes in and out) instead of gathering them
-        return "hbm", (24 if carries_rects else 16) * n, "B"
+        record = 12 if carries_rects else 8
+        if n <= 262144:
+            return "hbm", 2 * record * n, "B"
+        # three passes (average per launch): the first takes all Gaussians and hands the emitting ones on, of the others
+        # it stores the ids only
+        return "hbm", (record * n + 4 * (n - emitting) + 5 * record * emitting) / 3, "B"
     if kernel == "ordered_offsets_kernel":
-        return "hbm", 8 * n, "B"
+        return "hbm", 8 * emitting, "B"
     if kernel == "emit_ordered_kernel":
-        return "hbm", 12 * n + (slot_bytes + 4) * k, "B"
+        return "hbm", 12 * emitting + (slot_bytes + 4) * k, "B"
     if kernel == "onesweep32_kernel<tile partition>":
         # tile partition: slot + id in and out, except that the last pass writes no slots (average per launch)
         passes = 1 if lists + 1 <= 256 else (2 if lists + 1 <= 65536 else 3)
@@ -213,6 +220,7 @@ def main():
     from ds_splat_amd import stages
     cam = stages.camera_from_scene(sc, dev)
     _, st = stages.forward(cam, t["means_3d"], t["scales"], t["rotations"], t["opacities"], t["shs"])
+    emitting = int((st.splats[:-1, 11].contiguous().view(torch.int32) > 0).sum())   # (the last one never does)
     marked = 0
     if do_backward:
         marked = int(stages.backward(cam, st, 16, t["means_3d"], t["scales"], t["rotations"], v_image)["marks"].sum())
@@ -271,7 +279,7 @@ def main():
         launches_per_step = cnt / args.steps
         avg = tot / cnt
         bound, work, unit = algorithmic_work(name, n, k, W * H, lists, coeffs, counters, marked,
-                                             (W + 15) // 16 <= 255 and (H + 15) // 16 <= 255, list_bin > 1)
+                                             (W + 15) // 16 <= 255 and (H + 15) // 16 <= 255, list_bin > 1, emitting)
         table.append((tot / args.steps, name, avg, launches_per_step, bound, work, unit))
     table.sort(reverse=True)
     measured, traffic_source = measured_traffic(spec.name, k) if args.n is None else ({}, None)
@@ -317,7 +325,8 @@ def main():
         "config": {"workload": "%s: %d Gaussians, %dx%d, SH degree %d, %s" %
                                (spec.name, n, W, H, sc["sh_degree"], "forward+backward" if do_backward else "forward"),
                    "num_keys": int(k), "num_keys_per_tile_lists": k_per_tile, "tiles": int(tiles),
-                   "list_bin_tiles": list_bin, "lists": int(lists), "gaussians_with_gradient": marked,
+                   "list_bin_tiles": list_bin, "lists": int(lists), "gaussians_emitting": emitting,
+                   "gaussians_with_gradient": marked,
                    # (from the CPU oracle's counters, when it ran: pixel-entry pairs that the blend kernels
                    # walk, and those among them that are blended)
                    "pairs_walked_fwd": int(counters.pairs_fwd) if counters is not None else None,

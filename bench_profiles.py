@@ -175,7 +175,7 @@ def algorithmic_bytes(bench):
         bound, work, _ = bench_module.algorithmic_work(k, n, cfg["num_keys"], w * h, cfg["lists"], (deg + 1) ** 2, None,
                                                        cfg.get("gaussians_with_gradient", 0),
                                                        (w + 15) // 16 <= 255 and (h + 15) // 16 <= 255,
-                                                       cfg.get("list_bin_tiles", 1) > 1)
+                                                       cfg.get("list_bin_tiles", 1) > 1, cfg.get("gaussians_emitting"))
         if bound == "hbm":
             out[k] = work
     return out, n
@@ -272,8 +272,9 @@ def cmd_mem(args):
              "    " + command(MEM_CMD, args.mem_dir, args.workload),
              "    " + command(STATS_CMD, args.stats_dir, args.workload) + "    # the `kernel ms` column", "",
              "Averages per launch. `VMEM write inst` counts stores and atomics (the blend backward adds up a round's entries",
-             "in LDS and issues their nine sums, 64 a wavefront, as atomics, each with a byte store for the Gaussian's mark, and",
-             "at its end the stores of the zeros); `L2 atomic requests` is TCC_ATOMIC summed over the L2 channels.", "",
+             "in LDS, stores a byte for the mark of each that received a term, issues their nine sums, seven entries a wavefront",
+             "and instruction, as atomics, and at its end the stores of the zeros); `L2 atomic requests` is TCC_ATOMIC summed over",
+             "the L2 channels.", "",
              "| kernel | waves | VMEM read inst / wave | VMEM write inst / wave | branches / wave | TCP atomic requests | L2 atomic requests | L2 atomics / us | kernel ms |",
              "|---|---|---|---|---|---|---|---|---|"]
     for k in sorted(d, key=lambda k: -avg(d[k]["TCC_ATOMIC_sum"])):

@@ -16,7 +16,9 @@ sys.path.insert(0, ROOT)
     ("void dsx::onesweep32_kernel<unsigned int, 1024, 12, false, 9>(dsx::Sort32)", "onesweep32_kernel<sort>"),
     ("void dsx::onesweep32_kernel<unsigned int, 1024, 12, false, 8>(dsx::Sort32)", "onesweep32_kernel<tile partition>"),
     ("void dsx::onesweep32_kernel<unsigned short, 1024, 8, false, 8>(dsx::Sort32)", "onesweep32_kernel<tile partition>"),
+    ("void dsx::onesweep32_first_kernel<12, true>(dsx::Sort32)", "onesweep32_kernel<sort>"),
     ("void dsx::blend_fwd_tile_kernel<true>(int const*)", "blend_fwd_kernel"),
+    ("dsx::blend_fwd_wide_kernel(int const*)", "blend_fwd_kernel"),
     ("void dsx::blend_bwd_kernel<false>(int const*)", "blend_bwd_kernel"),
     ("dsx::project_fwd_kernel(float)", "project_fwd_kernel"),
 ])
