@@ -1,14 +1,16 @@
 // Stages 4 and 5a for gfx950: per-tile alpha blending, forward (front to back) and backward
 // (back to front).
 //
-// Both directions are bound by the issue of vector instructions (85 to 90 % of the time where no pixel stops early), so what
-// counts is how many a (pixel, entry) pair costs and how many pairs are looked at that need not be.  The backward of large Gaussians,
-// which every tile adds to, also waits for the memory: 13 ns for each request to one line.
-// 1920x1080 unless noted, us within a whole pass, before (four lists of entries per wavefront) -> now (sixteen):
-//   forward   2 M faint Gaussians 905 -> 717, 1.4 M at 1557x1038 340 -> 285, 500 K opaque 148 -> 130 (3 M: 161 -> 155),
-//             6 M at 3840x2160 519 -> 446, 1 M large ones 118 -> 120, 1 M at 1280x720 148 -> 129, 16 K at 256x256 34 -> 30
-//   backward  2 M faint 1662 -> 1317, 1.4 M at 1557x1038 553 -> 488, 500 K opaque 242 -> 235 (3 M: 279 -> 270),
-//             1 M large ones 290 -> 307, 300 K at 1237x822 263 -> 238, 50 K at 512x512 78 -> 74
+// Both directions are bound by the issue of vector instructions: these alone take 82 % of the time where no pixel stops early (2 M
+// faint Gaussians; an exponential or a reciprocal, which takes four times as long, counts once there) and 63 to 82 % elsewhere, so
+// what counts is how many a (pixel, entry) pair costs and how many pairs are looked at that need not be.  The backward
+// also waits for its sums: timed without the adds to memory, and then with a place in LDS for each quad of lanes' own sums, 1 M large Gaussians
+// 300 -> 236 -> 209 us, 3 M 253 -> 252 -> 237, 2 M faint 1281 -> 1238 -> 1184.
+// 1920x1080 unless noted, us within a whole pass (medians of a trace), four lists of entries per wavefront -> sixteen:
+//   forward   2 M faint Gaussians 881 -> 686, 1.4 M at 1557x1038 309 -> 266, 500 K opaque 127 -> 118 (3 M: 149 -> 148),
+//             6 M at 3840x2160 509 -> 431, 1 M large ones 123 -> 125, 1 M at 1280x720 138 -> 120, 16 K at 256x256 36 -> 21
+//   backward  2 M faint 1637 -> 1274, 1.4 M at 1557x1038 519 -> 457, 500 K opaque 223 -> 216 (3 M: 254 -> 253),
+//             1 M large ones 302 -> 306, 300 K at 1237x822 244 -> 223, 50 K at 512x512 77 -> 72
 #include "dsx_common.h"
 
 #include <atomic>
@@ -131,7 +133,7 @@ __device__ __forceinline__ uint32_t reach_limit_bwd(float opacity, float reach)
 // The lines at 5500 and 3000 tiles lie within those crossings.
 // dsx_set_blend_pixels_per_lane(1 | 4) overrides the choice for the whole process (tests run both
 // forms); DSX_BLEND_PIXELS_PER_LANE=1|4 in the environment gives the override's initial value and is
-// read once.
+// read once.  The forward's form of sixteen wavefronts per tile is the library's own choice only: either override switches it off.
 static std::atomic<int> g_forced_pixels_per_lane{-1}; // -1: not yet read from the environment, 0: automatic
 
 static int forced_pixels_per_lane()
@@ -1101,9 +1103,15 @@ __global__ __launch_bounds__(kTileThreads) void blend_fwd_tile_kernel(const int3
 // latency and its barriers.  Here each 4x4 block has a wavefront, each of its pixels a quad of lanes: the
 // four lanes work out four entries' alphas side by side, hand them to each other, take the same four steps of
 // the transmittance (the bits of one lane that takes one entry after the other), and each adds its own entry's colour; and up to
-// 960 entries are staged in one round.  us of the kernel, before -> now: 2 K Gaussians at 64x64 22.3 -> 14.0, 16 K at 256x256
-// 30.4 -> 20.8, 50 K at 512x512 (1024 tiles) 32.7 -> 51.1; whole forwards of four kinds of scenes at 256 tiles 74 -> 71,
-// 108 -> 117, 100 -> 95, 92 -> 88, at 400 tiles 85 -> 85, 118 -> 116, 103 -> 105, 124 -> 132: the line lies at 256.
+// 960 entries are staged in one round.  us of the kernel, four wavefronts -> sixteen: 2 K Gaussians at 64x64 23.6 -> 13.6, 16 K at
+// 256x256 35.5 -> 21.2 (1024 tiles of 50 K at 512x512: 32.7 -> 51.1).  Whole forwards of the four kinds of scenes above, and of a mixed one
+// that is nearer:
+//   64 tiles    46 -> 45, 67 -> 60, 57 -> 53, 66 -> 57, 84 -> 71
+//   169 tiles   56 -> 54, 95 -> 92, 92 -> 89, 76 -> 68, 116 -> 102
+//   256 tiles   68 -> 66, 107 -> 102, 99 -> 96, 90 -> 85, 140 -> 121
+//   400 tiles   85 -> 85, 118 -> 116, 103 -> 105, 124 -> 132
+// and at 169 and 256 tiles 40 more of 2 K to 1 M Gaussians, opaque, mixed, faint (322 -> 241) and large (249 -> 246): none is slower.
+// The line lies at 256, a tile for each compute unit; beyond it some units get two.
 // Lists per tile only (images of so few tiles have no others unless the caller asks).
 constexpr int kWideBatch = 960; // (two workgroups' records and lists fit a compute unit's LDS)
 constexpr int kWideThreads = 1024;
@@ -1465,7 +1473,10 @@ constexpr int kSums = 9;
 constexpr float kAlphaMaxBwd = 0.99f;
 // Where the sums of a place lie: four and four of each place side by side, then the ninths.  An add serves 16 lanes at a time
 // over 16 doubles: four rows' or blocks' lots of four meet only where their places are the same or a multiple of four apart (nine
-// doubles side by side: with 7 of 16 of all other places).
+// doubles side by side: with 7 of 16 of all other places).  Blocks that are at the same entry do meet, and where entries
+// reach every block nearly all are: 2.6 to 3.5 conflict cycles an LDS instruction.  The backward's wavefront form without its adds to memory, us,
+// as it is / with a place for each quad's own sums / without adds in LDS: 1 M large Gaussians 236 / 209 / 205, 3 M 252 / 237 / 234, 2 M
+// faint 1238 / 1184 / 1151.
 template <int kPlaces>
 __host__ __device__ constexpr int sum_at(int place, int slot)
 {
@@ -1501,7 +1512,8 @@ __device__ __forceinline__ void moments_to_gradients(double* sums, int place, co
 }
 // One set of hardware float atomics per entry and round, and none where no pixel was valid: nine threads for each entry (those
 // that are over sit out: a record's adds leave in one instruction, which takes the memory one or two requests; requests to a
-// line that every tile adds to wait 13 ns for each other).
+// line that every tile adds to wait 13 ns for each other; all adds together: 64 of 300 us for 1 M large Gaussians, 43 of 1281 for 2 M faint
+// ones, 1 of 253 for 3 M).
 // A load that is issued behind these adds waits for them too, so a round's are issued once the next round's records have arrived, and
 // end during its walk (right after their own walk: 1 M wide Gaussians 306 -> 284 us, 1.4 M at 1557x1038 494 -> 486, 500 K 239 -> 236;
 // tile form: 50 K at 512x512 74.0 -> 71.8, 100 K at 979x546 104.2 -> 103.1).

@@ -206,7 +206,8 @@ __global__ __launch_bounds__(kProjBlock) void project_fwd_kernel(const ProjectPa
     bool in_frustum = false;
     // What the shape needs is on its way before the rows of SH coefficients, not behind them (three dependent loads each); eight more
     // registers, six wavefronts per SIMD instead of seven (held to seven: slower, 164.6).  us before -> now: 3 M 161.5 -> 158.1, 6 M
-    // 285.0 -> 281.0, 1 M 52.8 -> 50.7, 50 K 11.1 -> 10.8; 300 K with colours and covariances 10.5 -> 11.2.
+    // 285.0 -> 281.0, 1 M 52.8 -> 50.7, 50 K 11.1 -> 10.8; with colours and covariances given 300 K 10.5 -> 11.2, 3 M 76.1 -> 75.2 (a kernel of
+    // their own that loads the opacity late and keeps seven: 300 K 9.8 -> 9.4 among the fastest launches, 3 M 76.2; one kernel serves both).
     float sc[3] = {0.f, 0.f, 0.f}, opacity = 0.f;
     float4 quat = make_float4(0.f, 0.f, 0.f, 0.f);
     if(live)

@@ -391,7 +391,9 @@ int dsx_trace_read(dsx_trace_entry* out /* host */, int max_entries);
  * (images with enough tiles to fill the chip) and four wavefronts per tile with one pixel per
  * lane.  The library picks by tile count; this forces one form for the whole process (pixels =
  * 1 or 4) or returns the choice to the library (0).  Results of the forward are bit-identical in
- * both forms.  For tests, which run both forms at every size.  No counterpart in the reference. */
+ * both forms.  For tests, which run both forms at every size.  No counterpart in the reference.
+ * Left to itself the library has a third form of the forward, for lists per tile of images of up to 256 tiles: sixteen
+ * wavefronts per tile, which add up a pixel's colours in four parts (final_T and final_idx are the same bits). */
 int dsx_set_blend_pixels_per_lane(int pixels);
 
 /* dsx_depth_order as dsx_forward_project runs it (above 262144 Gaussians the host waits for the range of the depths), with
