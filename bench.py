@@ -66,15 +66,17 @@ def algorithmic_work(kernel, n, k, pixels, lists, coeffs, counters, marked, carr
         return "hbm", n + marked * (88 + 52 + 12 * coeffs), "B"
     if kernel in ("hist32_kernel", "depth_hist_kernel"):
         return "hbm", 4 * n, "B"
-    if kernel == "onesweep32_kernel<sort>":
+    if kernel.startswith("onesweep32_kernel<sort"):
         # depth sort of the Gaussians: key + id, in and out; images of at most 255 x 255 tiles also carry each
         # Gaussian's packed tile rectangle through the passes (4 bytes in and out) instead of gathering them
         record = 12 if carries_rects else 8
         if n <= 262144:
             return "hbm", 2 * record * n, "B"
-        # three passes (average per launch): the first takes all Gaussians and hands the emitting ones on, of the others
-        # it stores the ids only
-        return "hbm", (record * n + 4 * (n - emitting) + 5 * record * emitting) / 3, "B"
+        # three passes: the first takes all Gaussians and hands the emitting ones on, of the others it stores the ids only
+        # (the passes share a name in the trace, which gives their average)
+        first, later = record * n + 4 * (n - emitting) + record * emitting, 2 * record * emitting
+        return "hbm", {"onesweep32_kernel<sort, first>": first, "onesweep32_kernel<sort, later>": later}.get(
+            kernel, (first + 2 * later) / 3), "B"
     if kernel == "ordered_offsets_kernel":
         return "hbm", 8 * emitting, "B"
     if kernel == "emit_ordered_kernel":

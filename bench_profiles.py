@@ -171,7 +171,8 @@ def algorithmic_bytes(bench):
     n, w, h, deg = int(m.group(2)), int(m.group(3)), int(m.group(4)), int(m.group(5))
     out = {}
     for k in ("project_fwd_kernel", "gaussian_bwd_kernel", "hist32_kernel", "depth_hist_kernel", "onesweep32_kernel<sort>",
-              "ordered_offsets_kernel", "emit_ordered_kernel", "onesweep32_kernel<tile partition>"):
+              "onesweep32_kernel<sort, first>", "onesweep32_kernel<sort, later>", "ordered_offsets_kernel",
+              "emit_ordered_kernel", "onesweep32_kernel<tile partition>"):
         bound, work, _ = bench_module.algorithmic_work(k, n, cfg["num_keys"], w * h, cfg["lists"], (deg + 1) ** 2, None,
                                                        cfg.get("gaussians_with_gradient", 0),
                                                        (w + 15) // 16 <= 255 and (h + 15) // 16 <= 255,
@@ -217,6 +218,8 @@ def cmd_traffic(args):
         tname = trace_name(k)
         tot, cnt = record.get(tname, (0.0, 0))
         record[tname] = (tot + (rb + wb) * 1e6 * len(f), cnt + len(f))      # launch-weighted, per trace name
+        if tname == "onesweep32_kernel<sort>":
+            tname = "onesweep32_kernel<sort, first>" if k.startswith("onesweep32_first") else "onesweep32_kernel<sort, later>"
         a = alg.get(tname)
         lines.append("| %s | %d | %.1f | %.1f | %.1f | %.1f | %.1f | %s | %s |" % (
             k, len(f), fa, wa, rb, wb, rb + wb, "%.1f" % (a / 1e6) if a else "(not HBM-bound)",

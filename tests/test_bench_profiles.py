@@ -32,3 +32,13 @@ def test_the_sorts_template_is_what_the_names_assume():
     head = re.search(r"template <([^>]*)>\s*__global__[^;{]*onesweep32_kernel\(", source)
     assert [p.split("=")[0].split()[-1] for p in head.group(1).split(",")] == ["KeyT", "kSort32Threads", "kSort32Items",
                                                                               "kCarry", "kBits"]
+
+
+@pytest.mark.parametrize("emitting", [300000, 120000, 0])
+def test_bytes_of_the_depth_sorts_passes(emitting):
+    """The first pass and the later two have bytes of their own; the trace's name for all three has their average."""
+    import bench
+    work = [bench.algorithmic_work("onesweep32_kernel<sort%s>" % which, 300000, 0, 0, 0, 0, None, 0, emitting=emitting)[1]
+            for which in (", first", ", later", "")]
+    assert work[0] == 12 * 300000 + 4 * (300000 - emitting) + 12 * emitting and work[1] == 24 * emitting
+    assert work[2] == pytest.approx((work[0] + 2 * work[1]) / 3)
