@@ -6,7 +6,7 @@ and the instruction counters come from separate rocprofv3 runs of the same scrip
 reads their CSV files and writes a short markdown table and, for the traffic, a JSON record that
 bench.py quotes as `roofline.traffic` (with the commit the counters were taken at).
 
-    # on the MI355X box, repository root (each counter set in a run of its own; W = cfg1 .. cfg4, dense):
+    # on the machine with the MI355X, repository root (each counter set in a run of its own; W = cfg1 .. cfg4, dense):
     export TMPDIR=/tmp
     rocprofv3 --kernel-trace --stats --output-format csv -d out/W/prof -o bench -- \\
         python3 bench.py --workload W --steps 20 --warmup 5 --no-cpu-baseline
@@ -149,7 +149,7 @@ def cmd_stats(args):
             med[r["Kernel_Name"]].append(int(r["End_Timestamp"]) - int(r["Start_Timestamp"]))
     lines = ["# Kernel statistics, bench.py (%s)" % workload_title(args.workload), "",
              "Commit: %s" % (args.commit or git_commit()), "",
-             "Command (on the MI355X box, repository root, after `export TMPDIR=/tmp`):", "",
+             "Command (on the machine with the MI355X, repository root, after `export TMPDIR=/tmp`):", "",
              "    " + command(STATS_CMD, args.dir, args.workload), "",
              "rocprofv3 kernel statistics (all launches of the run, warm-up included; the median is taken from the",
              "kernel trace of the same run):", "",
@@ -194,7 +194,7 @@ def cmd_traffic(args):
     cfg = bench["config"]
     lines = ["# HBM traffic per launch (FETCH_SIZE / WRITE_SIZE), %s" % cfg["workload"], "",
              "Commit: %s" % commit, "",
-             "Commands (on the MI355X box, repository root, after `export TMPDIR=/tmp`; one counter per run):", "",
+             "Commands (on the machine with the MI355X, repository root, after `export TMPDIR=/tmp`; one counter per run):", "",
              "    " + command(FETCH_CMD, args.fetch_dir, args.workload),
              "    " + command(WRITE_CMD, args.write_dir, args.workload),
              "    python3 bench_profiles.py traffic %s %s --bench-json <the first run's JSON line> --workload %s --name %s" % (
@@ -241,7 +241,7 @@ def cmd_sq(args):
     avg = lambda x: sum(x) / len(x)
     lines = ["# SQ counters per kernel (VALU issue, LDS bank conflicts), %s" % workload_title(args.workload), "",
              "Commit: %s" % (args.commit or git_commit()), "",
-             "Commands (on the MI355X box, repository root, after `export TMPDIR=/tmp`):", "",
+             "Commands (on the machine with the MI355X, repository root, after `export TMPDIR=/tmp`):", "",
              "    " + command(SQ_CMD, args.sq_dir, args.workload),
              "    " + command(STATS_CMD, args.stats_dir, args.workload) + "    # the `kernel ms` column", "",
              "Averages per launch. A wave64 VALU instruction occupies its SIMD for 4 clocks, so the chip (256 CU x 4 SIMD at 2.4 GHz)",
@@ -271,7 +271,7 @@ def cmd_mem(args):
     avg = lambda x: sum(x) / len(x) if x else 0.0
     lines = ["# Vector-memory instructions and L2 atomics per kernel, %s" % workload_title(args.workload), "",
              "Commit: %s" % (args.commit or git_commit()), "",
-             "Commands (on the MI355X box, repository root, after `export TMPDIR=/tmp`):", "",
+             "Commands (on the machine with the MI355X, repository root, after `export TMPDIR=/tmp`):", "",
              "    " + command(MEM_CMD, args.mem_dir, args.workload),
              "    " + command(STATS_CMD, args.stats_dir, args.workload) + "    # the `kernel ms` column", "",
              "Averages per launch. `VMEM write inst` counts stores and atomics (the blend backward adds up a round's entries",

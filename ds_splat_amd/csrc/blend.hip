@@ -1110,7 +1110,8 @@ __global__ __launch_bounds__(kTileThreads) void blend_fwd_tile_kernel(const int3
 //   169 tiles   56 -> 54, 95 -> 92, 92 -> 89, 76 -> 68, 116 -> 102
 //   256 tiles   68 -> 66, 107 -> 102, 99 -> 96, 90 -> 85, 140 -> 121
 //   400 tiles   85 -> 85, 118 -> 116, 103 -> 105, 124 -> 132
-// and at 169 and 256 tiles 40 more of 2 K to 1 M Gaussians, opaque, mixed, faint (322 -> 241) and large (249 -> 246): none is slower.
+// and at 169 and 256 tiles 40 more of 2 K to 1 M Gaussians, opaque, mixed, faint (322 -> 241) and large (248 -> 246): none is slower
+// by more than its runs differ.
 // The line lies at 256, a tile for each compute unit; beyond it some units get two.
 // Lists per tile only (images of so few tiles have no others unless the caller asks).
 constexpr int kWideBatch = 960; // (two workgroups' records and lists fit a compute unit's LDS)
