@@ -304,8 +304,9 @@ struct OrderLayout
     size_t slot_hist;  // uint32[kMaxPasses32 * 256] digit histograms of the tile slots of all pairs
     size_t cover;      // int32[(ntx + 1) * (nty + 1) + 1] pairs per tile (corner grid, then its 2-D prefix sum)
     size_t bin_cover;  // int32[(nbx + 1) * (nby + 1) + 1] the same per bin (binned lists only)
-    size_t key_count;  // uint64[3]  pairs of the per-tile lists, pairs of the bin lists (summed by the corner-grid kernel), workgroups done
+    size_t key_count;  // uint64[5]  pairs of the per-tile lists, pairs of the bin lists (summed by the corner-grid kernel), workgroups done (of three kinds)
     size_t offsets;    // uint64[...] what the workgroups of the kernel that fills block_sums tell each other, zeroed with the corner grids
+    size_t run_sums;   // uint32[blocks] pairs of 256 consecutive Gaussians in depth order, where one launch makes the order; zeroed too
     size_t ranges;     // int32[...] ranges_layout() without its `walk` part, ready before the pairs exist
     size_t sort;       // Sort32Workspace
     size_t bytes;

@@ -855,6 +855,7 @@ __global__ __launch_bounds__(kHist32Threads) void depth_hist_kernel(const uint32
 // ---------------------------------------------------------------------------------------
 
 constexpr int kOffsetsShare = 16 * kProjBlock; // Gaussians of a workgroup of ordered_offsets_kernel
+constexpr int kRanksMax = 131072;              // Gaussians whose depth order is one launch, order_ranks_kernel
 
 OrderLayout order_layout(int64_t n, int image_width, int image_height, int list_bin)
 {
@@ -891,9 +892,11 @@ OrderLayout order_layout(int64_t n, int image_width, int image_height, int list_
         off += (size_t)((g.nbx + 1) * (g.nby + 1) + 1) * 4;
     off = (off + 7) & ~(size_t)7;
     o.key_count = off; // inside the region that is zeroed with the corner grids
-    off += 24;
+    off += 40;
     o.offsets = off; // so is this
-    off = align(off + 8 * (size_t)((n + kOffsetsShare - 1) / kOffsetsShare));
+    off += 8 * (size_t)((n + kOffsetsShare - 1) / kOffsetsShare);
+    o.run_sums = off; // and this
+    off = align(off + (n <= kRanksMax ? 4 * (size_t)((n + kProjBlock - 1) / kProjBlock) : 0));
     o.ranges = off;
     off += (size_t)ranges_layout(g).ready * 4;
     o.bytes = align(off);
@@ -1311,304 +1314,411 @@ __global__ __launch_bounds__(kCoverThreads) void tile_counts_kernel(const Counts
 }
 
 // ---------------------------------------------------------------------------------------
-// few Gaussians: depth order and counting in one launch or two
+// up to 131072 Gaussians: depth order, block offsets and counting in one launch
 // ---------------------------------------------------------------------------------------
-// Up to 24576 Gaussians the digit passes, their histogram and the offsets (a sum and a scan when this was measured) are launches
-// of 3 to 8 us that each do a microsecond's work (2 K Gaussians: 38 us of kernels, 16 K: 50 us).  Here a workgroup
-// sorts 2048 keys in its own LDS and registers (by the digits of the keys' distance from the smallest one, three
-// or fewer for any scene whose depths stay within a factor of eight), and one more (two, for binned lists)
-// fills a corner grid of its own and counts the tiles (and the bins) beside it.  Up to 2048 Gaussians that is
-// all; beyond, a second launch ranks every key among the other workgroups' sorted keys by binary search in LDS.
-// 2 K Gaussians: 10 us, 4 K: 9 + 7, 16 K: 13 + 17.  (One workgroup for 16 K keys, sixteen to a thread: 51 us.)
-// The line lies where a whole forward stops gaining, us, digit passes / merge, at 256x256 and at 1024x768:
-// 3000 Gaussians 89 / 48 and 101 / 60, 8 K 100 / 63 and 106 / 76, 16 K 110 / 92 and 118 / 104, 18000 109 / 98 and
-// 120 / 111, 20 K 112 / 102 and 122 / 116, 24 K 110 / 105 and 126 / 124, 28 K 112 / 112 and 130 / 134, 32 K 112 / 115 and
-// 135 / 142.
-constexpr int kSmallThreads = 1024;
-static_assert(kSmallThreads == kCoverThreads, "tile_counts is written for this many threads");
-constexpr int kSmallItems = 2;
-constexpr int kSmallTile = kSmallThreads * kSmallItems;
-constexpr int kSmallTilesMax = 12;
-constexpr int kSmallMax = kSmallTile * kSmallTilesMax;
-constexpr int kMergeThreads = 256;
-constexpr int kSmallWaves = kSmallThreads / DSX_WAVE;
-constexpr int kSmallDigitBits = 9;
-constexpr int kSmallBins = 1 << kSmallDigitBits;
+// Few keys are sorted by launches that wait for each other and do a microsecond's work each.  Here every workgroup finds out by
+// itself which ranks are its own: it counts ALL keys into 4096 bins of their range (they lie in the L2), sums the bins up, and
+// the keys between the bin borders next to ranks 512 w and 512 (w + 1) are workgroup w's, some 512 of them.  It reads the keys
+// again, takes those, sorts them in LDS (2048 bins of its own part of the range, and a comparison with the few others in the
+// same bin), and writes them where they belong: nobody waits for anybody.  Workgroups beside them fill corner grids and
+// count the tiles and the bins.
+// What is ordered are the distances of the depth keys from the smallest one with the Gaussian's index behind (all different).  Where a
+// border would be kShareSlack or more ranks off (many equal or nearly equal depths) the bin before it is taken apart by the next
+// twelve bits, if need be down to the index, so a workgroup never has more than 1023 keys, whatever they are.
+// Bound by the two passes over all keys, of every workgroup, at some 35 bytes a cycle and compute unit, and by the chain around them:
+// 2 K Gaussians 10 us (1 for the ranges, 1.5 for the two passes, 3 for borders and barriers, 2.5 in the sort, 2 until the last one has summed up),
+// 16 K 11, 50 K 17.5, 100 K 23.5.  Before, a sort of 2048 keys in LDS and a merge up to 24576 Gaussians, the digit passes beyond: a whole
+// forward of 16 K 78 -> 60 us, a training step of 50 K 199 -> 165, of 100 K 229 -> 198, 2 K 40 as it was.
+constexpr int kRanksThreads = 1024;
+static_assert(kRanksThreads == kCoverThreads, "tile_counts is written for this many threads");
+constexpr int kRanksBinBits = 12;
+constexpr int kRanksBins = 1 << kRanksBinBits;
+constexpr int kShareWanted = 512; // keys of a workgroup
+constexpr int kShareSlack = 512;  // by so many fewer than this may its share begin and end late
+constexpr int kShareMost = 1024;
+constexpr int kShareBinBits = 11;
+constexpr int kRanksWaves = kRanksThreads / DSX_WAVE;
+constexpr int kCountShare = 2048; // rectangles of a counting workgroup, at least
+constexpr int kCountWorkgroupsMost = 32;
+static_assert(kShareWanted + kShareSlack <= kShareMost && kShareMost <= kRanksThreads, "a thread for each key");
+static_assert(kShareWanted == 2 * kProjBlock && kRanksBins == 4 * kRanksThreads, "what the threads take");
+constexpr size_t kRanksLds = (kRanksBins + DSX_WAVE) * 4 + 2 * kShareMost * 8;
 
-struct SmallOrder
+struct RanksJob
 {
     const uint32_t* depth_keys; // by Gaussian
     const uint2* rects;
-    uint32_t* order; // by depth
+    const uint2* key_ranges; // of 256 consecutive Gaussians (see OrderLayout)
+    uint32_t* order;         // by depth
     uint2* rects_sorted;
-    uint32_t* block_sums; // exclusive sums of the list pairs of 256 consecutive Gaussians in depth order, and their total
-    uint32_t *tile_keys, *tile_ids; // several tiles: each one's own order, for the merge
-    unsigned long long* done;       // (merge) workgroups that have added their sums
-    int n, shift, tiles;
+    uint32_t* run_sums;   // pairs of 256 consecutive Gaussians in depth order (zero at first)
+    uint32_t* block_sums; // their exclusive sums, and the total
+    unsigned long long* key_count; // pairs of the tiles, of the bins; workgroups done: the order's, the tiles', the bins' (zero at first)
+    int n, id_bits, shift, shares, counting; // counting: workgroups for each of the grids
     CountsJobs counts;
     HostCounts to_host;
 };
 
-__device__ __forceinline__ void small_sort(const SmallOrder& J, const int tile, uint32_t* s_mem)
+// (the bits of a 64-bit number)
+__device__ __forceinline__ int bits_of(uint64_t v)
 {
-    constexpr int kItems = kSmallItems;
-    uint32_t* const s_keys = s_mem;
-    uint16_t* const s_ids = reinterpret_cast<uint16_t*>(s_mem + kSmallTile);
-    uint16_t (*const s_whist)[kSmallBins] = reinterpret_cast<uint16_t (*)[kSmallBins]>(s_mem + kSmallTile + kSmallTile / 2);
-    __shared__ uint32_t s_start[kSmallBins];
-    __shared__ __attribute__((aligned(16))) uint32_t s_tot[kSmallWaves];
-    __shared__ uint32_t s_min, s_max;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int base = tile * kSmallTile, n = min(J.n - base, kSmallTile);
+    return v ? 64 - __builtin_clzll(v) : 0;
+}
 
-    if(tid == 0)
-    {
-        s_min = 0xffffffffu;
-        s_max = 0u;
-    }
-    __syncthreads();
-    // item `it` of a wavefront's lane is input position (wave * kItems + it) * 64 + lane
-    uint32_t key[kItems], id[kItems];
-    uint32_t lo = 0xffffffffu, hi = 0u;
+// A thread's keys of one step through all of them, sixteen bytes at a time (the buffer is padded to whole lines)
+constexpr int kBatchLoads = 4;
+constexpr int kBatchKeys = 4 * kBatchLoads * kRanksThreads;
+struct KeyBatch
+{
+    uint4 k[kBatchLoads];
+};
+__device__ __forceinline__ KeyBatch load_keys(const uint32_t* keys, int i0, int n)
+{
+    KeyBatch batch;
 #pragma unroll
-    for(int it = 0; it < kItems; ++it)
+    for(int b = 0; b < kBatchLoads; ++b)
     {
-        const int i = (wave * kItems + it) * DSX_WAVE + lane;
-        key[it] = i < n ? J.depth_keys[base + i] : kNoPairsKey;
-        id[it] = (uint32_t)i;
-        if(key[it] != kNoPairsKey)
+        const int i = i0 + 4 * (b * kRanksThreads + (int)threadIdx.x);
+        uint4 k = make_uint4(kNoPairsKey, kNoPairsKey, kNoPairsKey, kNoPairsKey);
+        if(i < n)
+            k = *reinterpret_cast<const uint4*>(keys + i);
+        if(i0 + kBatchKeys > n) // (uniform: the words behind the last key hold anything)
         {
-            lo = min(lo, key[it]);
-            hi = max(hi, key[it]);
+            k.y = i + 1 < n ? k.y : kNoPairsKey;
+            k.z = i + 2 < n ? k.z : kNoPairsKey;
+            k.w = i + 3 < n ? k.w : kNoPairsKey;
         }
+        batch.k[b] = k;
     }
-#pragma unroll
-    for(int o = 32; o > 0; o >>= 1)
+    return batch;
+}
+
+__device__ __forceinline__ void order_share(const RanksJob& J, const int share, uint32_t* const s_mem)
+{
+    uint32_t* const s_hist = s_mem;
+    uint2* const s_rects = reinterpret_cast<uint2*>(s_mem + kRanksBins + DSX_WAVE);
+    uint32_t* const s_taken_ids = reinterpret_cast<uint32_t*>(s_rects); // (before)
+    uint64_t* const s_binned = reinterpret_cast<uint64_t*>(s_rects + kShareMost);
+    __shared__ uint4 s_range[kRanksWaves];
+    __shared__ __attribute__((aligned(16))) uint32_t s_tot[kRanksWaves];
+    __shared__ uint32_t s_found[2][3], s_sums[kShareMost / kProjBlock + 2], s_taken;
+    __shared__ unsigned long long s_all[kRanksWaves];
+    __shared__ int s_last;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int n = J.n, blocks = (n + kProjBlock - 1) / kProjBlock;
+
+    const KeyBatch ahead = load_keys(J.depth_keys, 0, n); // (the first ones, for every pass over the keys)
+    // the keys' range, how many there are, and how many of the Gaussians before this workgroup's 512 emit
+    uint32_t near16 = 0, far16 = 0, emit = 0, emit_before = 0;
+    for(int b = tid; b < blocks; b += kRanksThreads)
     {
-        lo = min(lo, (uint32_t)__shfl_xor(lo, o, DSX_WAVE));
-        hi = max(hi, (uint32_t)__shfl_xor(hi, o, DSX_WAVE));
+        const uint2 r = J.key_ranges[b];
+        near16 = max(near16, r.x & 0xffffu);
+        far16 = max(far16, r.y);
+        emit += r.x >> 16;
+        emit_before += b < 2 * share ? r.x >> 16 : 0u;
     }
-    if(lane == 0)
-    {
-        atomicMin(&s_min, lo);
-        atomicMax(&s_max, hi);
-    }
+    near16 = wave_incl_max_scan(near16);
+    far16 = wave_incl_max_scan(far16);
+    emit = wave_incl_scan_u32(emit);
+    emit_before = wave_incl_scan_u32(emit_before);
+    if(lane == 63)
+        s_range[wave] = make_uint4(near16, far16, emit, emit_before);
+    *reinterpret_cast<uint4*>(s_hist + 4 * tid) = make_uint4(0u, 0u, 0u, 0u);
+    if(tid < kShareMost / kProjBlock + 2)
+        s_sums[tid] = 0;
+    if(tid == 0)
+        s_taken = 0;
     __syncthreads();
-    const uint32_t first = s_min;
-    // distances 0 .. last; those that emit nothing, and the places behind the input, one further
-    const uint32_t last = s_max >= first ? s_max - first : 0u;
-    const uint32_t behind = last < 0xffffffffu ? last + 1u : last; // (keys of all 32-bit values: kNoPairsKey is the largest as it is)
-    const int bits = 32 - __builtin_clz(behind | 1u);
-    const int passes = s_max >= first ? (bits + kSmallDigitBits - 1) / kSmallDigitBits : 0; // nothing emits: in order already
+    near16 = far16 = emit = emit_before = 0;
 #pragma unroll
-    for(int it = 0; it < kItems; ++it)
-        key[it] = key[it] == kNoPairsKey ? behind : key[it] - first;
-    for(int p = 0; p < passes; ++p)
+    for(int w = 0; w < kRanksWaves; ++w)
     {
-        const int width = (bits + passes - 1) / passes, shift = p * width;
-        const uint32_t mask = (1u << width) - 1u;
-        for(int j = tid; j < kSmallWaves * kSmallBins / 2; j += kSmallThreads)
-            reinterpret_cast<uint32_t*>(s_whist)[j] = 0;
-        __syncthreads(); // (and the keys and ids of the last pass have been taken)
-        uint32_t place[kItems];
-#pragma unroll
-        for(int it = 0; it < kItems; ++it)
+        const uint4 r = s_range[w];
+        near16 = max(near16, r.x);
+        far16 = max(far16, r.y);
+        emit += r.z;
+        emit_before += r.w;
+    }
+    const uint32_t emitting = __builtin_amdgcn_readfirstlane(emit), before_mine = __builtin_amdgcn_readfirstlane(emit_before);
+    const uint32_t lowest = 0xffffu - __builtin_amdgcn_readfirstlane(near16), highest = __builtin_amdgcn_readfirstlane(far16);
+    const uint32_t first = emitting ? lowest << 16 : 0u;
+    const int dist_bits = bits_of(emitting ? ((uint64_t)(highest - lowest + 1u) << 16) - 1u : 0xffffull); // (at least 16)
+    const int id_bits = J.id_bits;
+    // the number that is ordered: the distance, then the index
+    auto number_of = [&](uint32_t key, int i) { return ((uint64_t)(key - first) << id_bits) | (uint32_t)i; };
+    // a key that emits nothing has a distance like others only where the range ends at the largest number
+    const bool apart = (uint64_t)first + (1ull << dist_bits) <= kNoPairsKey;
+    // f(sixteen keys, the index of each) for all keys, those that emit nothing among them
+    auto for_all = [&](auto f) {
+        KeyBatch batch = ahead;
+        for(int i0 = 0; i0 < n; i0 += kBatchKeys)
         {
-            const uint32_t d = (key[it] >> shift) & mask;
-            const uint64_t m = match_digit<kSmallDigitBits>(d, kSmallDigitBits);
-            const uint32_t below = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-            const uint32_t old = s_whist[wave][d];
-            __builtin_amdgcn_wave_barrier();
-            if(below == 0)
-                s_whist[wave][d] = (uint16_t)(old + (uint32_t)__popcll(m));
-            __builtin_amdgcn_wave_barrier();
-            place[it] = old + below;
+            const KeyBatch next = load_keys(J.depth_keys, i0 + kBatchKeys, n);
+#pragma unroll
+            for(int b = 0; b < kBatchLoads; b += 4)
+            {
+                uint32_t key[16];
+#pragma unroll
+                for(int u = 0; u < 16; ++u)
+                    key[u] = reinterpret_cast<const uint32_t*>(&batch.k[b + u / 4])[u % 4];
+                f(key, [&](int u) { return i0 + 4 * ((b + u / 4) * kRanksThreads + tid) + u % 4; });
+            }
+            batch = next;
+        }
+    };
+    // Behind a histogram of whole bins, `before` keys of which lie in front of it: for each rank of two, the first bin border at or behind it
+    // (its number, its rank, and the rank of the border before it)
+    auto borders = [&](uint32_t before, const uint32_t (&rank)[2]) {
+        __syncthreads();
+        const uint4 c = *reinterpret_cast<const uint4*>(s_hist + 4 * tid);
+        const uint32_t count[4] = {c.x, c.y, c.z, c.w};
+        const uint32_t sum = c.x + c.y + c.z + c.w, incl = wave_incl_scan_u32(sum);
+        if(lane == 63)
+            s_tot[wave] = incl;
+        if(tid < 6)
+            (&s_found[0][0])[tid] = tid % 3 ? before : 0u; // (rank 0: the first border)
+        __syncthreads();
+        uint32_t at = before + sum_of_waves_before<kRanksWaves>(s_tot, wave) + incl - sum;
+#pragma unroll
+        for(int u = 0; u < 4; ++u)
+        {
+#pragma unroll
+            for(int e = 0; e < 2; ++e)
+                if(at < rank[e] && rank[e] <= at + count[u])
+                {
+                    s_found[e][0] = 4 * tid + u + 1;
+                    s_found[e][1] = at + count[u];
+                    s_found[e][2] = at;
+                }
+            at += count[u];
         }
         __syncthreads();
-        uint32_t total = 0;
-        if(tid < kSmallBins)
-        {
+    };
+
+    const uint32_t rank[2] = {min((uint32_t)(kShareWanted * share), emitting), min((uint32_t)(kShareWanted * (share + 1)), emitting)};
+    uint64_t border[2] = {0, 0};
+    uint32_t place[2] = {0, 0};
+    if(rank[0] < rank[1]) // (uniform; the last workgroups may have none)
+    {
+        // (keys that emit nothing are counted behind the bins, each lane's by themselves)
+        const int top = dist_bits - kRanksBinBits;
+        if(apart)
+            for_all([&](const uint32_t (&key)[16], auto) {
 #pragma unroll
-            for(int w = 0; w < kSmallWaves; ++w)
+                for(int u = 0; u < 16; ++u)
+                    atomicAdd(&s_hist[min((key[u] - first) >> top, (uint32_t)(kRanksBins + lane))], 1u);
+            });
+        else
+            for_all([&](const uint32_t (&key)[16], auto) {
+#pragma unroll
+                for(int u = 0; u < 16; ++u)
+                    atomicAdd(&s_hist[key[u] == kNoPairsKey ? (uint32_t)(kRanksBins + lane) : (key[u] - first) >> top], 1u);
+            });
+        borders(0u, rank);
+        uint32_t found[2][3];
+#pragma unroll
+        for(int e = 0; e < 6; ++e)
+            found[e / 3][e % 3] = __builtin_amdgcn_readfirstlane((&s_found[0][0])[e]);
+#pragma unroll
+        for(int e = 0; e < 2; ++e)
+        {
+            int shift = dist_bits + id_bits - kRanksBinBits; // of the bins' numbers
+            uint64_t low = 0;
+            while(found[e][1] - rank[e] >= (uint32_t)kShareSlack && shift > 0)
             {
-                const uint32_t c = s_whist[w][tid];
-                s_whist[w][tid] = (uint16_t)total;
-                total += c;
+                // the bin in front of the border is a large one: bins of its own
+                const int wide = shift;
+                low += (uint64_t)(found[e][0] - 1u) << wide;
+                shift = max(wide - kRanksBinBits, 0);
+                __syncthreads();
+                *reinterpret_cast<uint4*>(s_hist + 4 * tid) = make_uint4(0u, 0u, 0u, 0u);
+                __syncthreads();
+                for_all([&](const uint32_t (&key)[16], auto index) {
+#pragma unroll
+                    for(int u = 0; u < 16; ++u)
+                    {
+                        const uint64_t d = number_of(key[u], index(u)) - low;
+                        if(key[u] != kNoPairsKey && (d >> wide) == 0)
+                            atomicAdd(&s_hist[(uint32_t)(d >> shift)], 1u);
+                    }
+                });
+                borders(found[e][2], rank);
+#pragma unroll
+                for(int j = 0; j < 3; ++j)
+                    found[e][j] = __builtin_amdgcn_readfirstlane(s_found[e][j]);
             }
+            border[e] = low + ((uint64_t)found[e][0] << shift);
+            place[e] = found[e][1];
         }
-        const uint32_t incl = wave_incl_scan_u32(total);
+        __syncthreads();
+
+        // this workgroup's keys, in any order, and bins of their range
+        // (a lane marks its sixteen keys and then stores the places of the few that are taken; one request for room a wavefront)
+        auto take_all = [&](auto inside) {
+            for_all([&](const uint32_t (&key)[16], auto index) {
+                uint32_t marks = 0;
+#pragma unroll
+                for(int u = 0; u < 16; ++u)
+                    marks += marks + (inside(key[u], index(u)) ? 1u : 0u);
+                if(__builtin_amdgcn_ballot_w64(marks != 0) == 0)
+                    return;
+                const uint32_t taken = (uint32_t)__popc(marks), incl = wave_incl_scan_u32(taken);
+                uint32_t at = 0;
+                if(lane == 63)
+                    at = atomicAdd(&s_taken, incl);
+                at = (uint32_t)__builtin_amdgcn_readlane((int)at, 63) + incl - taken;
+                while(marks != 0)
+                {
+                    const int u = 15 - (31 - __builtin_clz(marks));
+                    marks ^= 0x8000u >> u;
+                    s_taken_ids[min(at++, (uint32_t)kShareMost - 1u)] = (uint32_t)index(u);
+                }
+            });
+        };
+        const uint64_t ids = (1ull << id_bits) - 1;
+        if(apart && ((border[0] | border[1]) & ids) == 0) // (the distances alone tell)
+        {
+            const uint32_t nearest = first + (uint32_t)(border[0] >> id_bits), depth = (uint32_t)((border[1] - border[0]) >> id_bits);
+            take_all([&](uint32_t key, int) { return key - nearest < depth; });
+        }
+        else
+            take_all([&](uint32_t key, int i) {
+                const uint64_t number = number_of(key, i);
+                return key != kNoPairsKey && number >= border[0] && number < border[1];
+            });
+        s_hist[tid] = s_hist[kRanksThreads + tid] = 0;
+        __syncthreads();
+        const int count = (int)(place[1] - place[0]);
+        const int shift = max(bits_of(border[1] - border[0] - 1u) - kShareBinBits, 0);
+        uint64_t mine = 0;
+        uint32_t bin = 0, nth = 0;
+        uint2 rect = make_uint2(0u, 0u);
+        if(tid < count)
+        {
+            const int i = (int)s_taken_ids[tid];
+            rect = J.rects[i]; // (here on time for the end)
+            mine = number_of(J.depth_keys[i], i);
+            bin = (uint32_t)((mine - border[0]) >> shift);
+            nth = atomicAdd(&s_hist[bin], 1u);
+        }
+        __syncthreads();
+        const uint2 c = *reinterpret_cast<const uint2*>(s_hist + 2 * tid);
+        const uint32_t incl = wave_incl_scan_u32(c.x + c.y);
         if(lane == 63)
             s_tot[wave] = incl;
         __syncthreads();
-        if(tid < kSmallBins)
-            s_start[tid] = sum_of_waves_before<kSmallBins / DSX_WAVE>(s_tot, wave) + incl - total;
+        const uint32_t at = sum_of_waves_before<kRanksWaves>(s_tot, wave) + incl - c.x - c.y;
+        *reinterpret_cast<uint2*>(s_hist + 2 * tid) = make_uint2(at, at + c.x);
+        if(tid == 0)
+            s_hist[1 << kShareBinBits] = (uint32_t)count;
         __syncthreads();
-#pragma unroll
-        for(int it = 0; it < kItems; ++it)
+        uint32_t start = 0, end = 0;
+        if(tid < count)
         {
-            const uint32_t d = (key[it] >> shift) & mask;
-            const uint32_t at = place[it] + s_start[d] + s_whist[wave][d];
-            s_keys[at] = key[it];
-            s_ids[at] = (uint16_t)id[it];
+            start = s_hist[bin];
+            end = s_hist[bin + 1];
+            s_binned[start + nth] = mine;
         }
         __syncthreads();
-#pragma unroll
-        for(int it = 0; it < kItems; ++it)
+        uint32_t* const s_ids = s_hist;
+        if(tid < count)
         {
-            const int i = (wave * kItems + it) * DSX_WAVE + lane;
-            key[it] = s_keys[i];
-            id[it] = s_ids[i];
+            uint32_t r = start;
+            for(uint32_t j = start; j < end; ++j)
+                r += s_binned[j] < mine ? 1u : 0u;
+            s_ids[r] = (uint32_t)mine & ((1u << id_bits) - 1u);
+            s_rects[r] = rect;
         }
-    }
-    if(J.tiles > 1)
-    {
-        // one of several: this tile's order, for the merge (whose block sums start at zero)
-#pragma unroll
-        for(int it = 0; it < kItems; ++it)
-        {
-            const int i = (wave * kItems + it) * DSX_WAVE + lane;
-            if(i < n)
-            {
-                J.tile_keys[base + i] = key[it] == behind ? kNoPairsKey : key[it] + first;
-                J.tile_ids[base + i] = (uint32_t)base + id[it];
-            }
-        }
-        if(tile == 0 && tid <= kSmallMax / kProjBlock && tid <= (J.n + kProjBlock - 1) / kProjBlock)
-            J.block_sums[tid] = 0;
-        return;
-    }
-    // the order, the rectangles in it, and the blocks' sums
-    __syncthreads();
-    uint32_t* const s_groups = s_keys; // pairs of 64 consecutive Gaussians
-#pragma unroll
-    for(int it = 0; it < kItems; ++it)
-    {
-        const int i = (wave * kItems + it) * DSX_WAVE + lane;
+        __syncthreads();
+        // the order, the rectangles in it, and the runs' sums
+        const uint32_t p = place[0] + (uint32_t)tid, run0 = place[0] / kProjBlock;
         uint32_t pairs = 0;
-        if(i < n)
+        if(tid < count)
         {
-            const uint2 r = J.rects[id[it]];
-            J.order[i] = id[it];
-            J.rects_sorted[i] = r;
+            const uint2 r = s_rects[tid];
+            J.order[p] = s_ids[tid];
+            J.rects_sorted[p] = r;
             pairs = list_count(r, J.shift);
         }
-        const uint32_t sum = wave_incl_scan_u32(pairs);
-        if(lane == 63)
-            s_groups[wave * kItems + it] = sum;
-    }
-    __syncthreads();
-    if(wave == 0)
-    {
-        const int blocks = (n + kProjBlock - 1) / kProjBlock; // (at most eight)
-        uint32_t sum = 0;
-        if(lane < blocks)
-            for(int g = 0; g < kProjBlock / DSX_WAVE; ++g)
-                sum += s_groups[lane * (kProjBlock / DSX_WAVE) + g];
-        const uint32_t incl = wave_incl_scan_u32(sum);
-        if(lane < blocks)
-            J.block_sums[lane] = incl - sum;
-        if(lane == blocks - 1)
-            J.block_sums[blocks] = incl;
-    }
-    static_assert(kSmallTile / kProjBlock <= DSX_WAVE, "one lane per block");
-}
-
-// The place of every key in the whole order: its place in its own tile and, for every other tile, the number of that
-// tile's keys before it (an equal key of an earlier tile comes first: the order is stable).
-__global__ __launch_bounds__(kMergeThreads) void order_merge_kernel(const SmallOrder J)
-{
-    extern __shared__ uint32_t s_small[]; // all keys, tile after tile
-    __shared__ uint32_t s_sums[kSmallMax / kProjBlock + 1];
-    __shared__ int s_last;
-    const int tid = threadIdx.x;
-    const int blocks = (J.n + kProjBlock - 1) / kProjBlock;
-    for(int j = tid; j < (J.n + 3) / 4; j += kMergeThreads) // (the buffers are padded to 256 bytes)
-        reinterpret_cast<uint4*>(s_small)[j] = reinterpret_cast<const uint4*>(J.tile_keys)[j];
-    for(int j = tid; j < blocks; j += kMergeThreads)
-        s_sums[j] = 0;
-    const int i = blockIdx.x * kMergeThreads + tid;
-    uint32_t id = 0;
-    uint2 r = make_uint2(0u, 0u);
-    if(i < J.n)
-    {
-        id = J.tile_ids[i];
-        r = J.rects[id];
-    }
-    __syncthreads();
-    if(i < J.n)
-    {
-        const uint32_t key = s_small[i];
-        const int mine = i / kSmallTile;
-        int rank = i - mine * kSmallTile;
-        // (four tiles at a time: a search is a chain of a dozen dependent LDS reads)
-        for(int t0 = 0; t0 < J.tiles; t0 += 4)
+        const uint32_t run = p / kProjBlock - run0, other = (uint32_t)__builtin_amdgcn_readlane((int)run, 63);
+        if(__builtin_amdgcn_readfirstlane(run) == other)
         {
-            int before[4] = {0, 0, 0, 0};
-#pragma unroll
-            for(int step = kSmallTile; step > 0; step >>= 1)
-#pragma unroll
-                for(int u = 0; u < 4; ++u)
-                {
-                    // the number of keys of tile t below `key` (or equal to it, for an earlier tile)
-                    const int t = t0 + u, count = min(max(J.n - t * kSmallTile, 0), kSmallTile);
-                    const int at = before[u] + step;
-                    const uint32_t other = s_small[min(t * kSmallTile + at, J.n) - 1];
-                    if(at <= count && (t < mine ? other <= key : other < key))
-                        before[u] = at;
-                }
-#pragma unroll
-            for(int u = 0; u < 4; ++u)
-                rank += t0 + u == mine ? 0 : before[u];
+            const uint32_t sum = wave_sum_u32(pairs);
+            if(lane == 0 && sum)
+                atomicAdd(&s_sums[run], sum);
         }
-        J.order[rank] = id;
-        J.rects_sorted[rank] = r;
-        const uint32_t pairs = list_count(r, J.shift);
-        if(pairs)
-            atomicAdd(&s_sums[rank / kProjBlock], pairs);
+        else if(pairs)
+            atomicAdd(&s_sums[run], pairs);
+        __syncthreads();
+        uint32_t done = 0;
+        if(tid < kShareMost / kProjBlock + 2 && s_sums[tid])
+            done = atomicAdd(&J.run_sums[run0 + tid], s_sums[tid]);
+        asm volatile("s_waitcnt vmcnt(0)" ::"v"(done) : "memory"); // (an addition has been performed when its result is back)
     }
-    __syncthreads();
-    // The blocks' sums over the workgroups; the last one to add its own turns them into exclusive prefixes.
-    // (An addition has been performed when its result is back; every wavefront's are before the barrier.)
-    for(int j = tid; j < blocks; j += kMergeThreads)
+    // of the Gaussians 512 w to 512 w + 511 those that emit nothing: behind the others, by index
     {
-        const uint32_t before = s_sums[j] ? atomicAdd(&J.block_sums[j], s_sums[j]) : 0u;
-        asm volatile("s_waitcnt vmcnt(0)" ::"v"(before) : "memory");
+        const int i = kShareWanted * share + tid;
+        const bool none = tid < kShareWanted && i < n && J.depth_keys[min(i, n - 1)] == kNoPairsKey;
+        const uint64_t m = __builtin_amdgcn_ballot_w64(none);
+        __syncthreads();
+        if(lane == 0)
+            s_tot[wave] = (uint32_t)__popcll(m);
+        __syncthreads();
+        if(none)
+        {
+            const uint32_t at = emitting + (uint32_t)(kShareWanted * share) - before_mine +
+                                sum_of_waves_before<kRanksWaves>(s_tot, wave) + bits_below(m);
+            J.order[at] = (uint32_t)i;
+            J.rects_sorted[at] = make_uint2(0u, 0u);
+        }
     }
-    __syncthreads();
+    // the last workgroup turns the runs' sums into the places where they begin
     if(tid == 0)
-        s_last = atomicAdd(J.done, 1ull) == gridDim.x - 1;
+        s_last = atomicAdd(J.key_count + 2, 1ull) == (unsigned long long)(J.shares - 1);
     __syncthreads();
-    if(s_last && tid < DSX_WAVE)
+    if(!s_last)
+        return;
+    static_assert(kRanksMax / kProjBlock <= kRanksThreads, "a thread for each run");
+    const uint32_t sum = tid < blocks ? atomicAdd(&J.run_sums[tid], 0u) : 0u;
+    const uint32_t incl = wave_incl_scan_u32(sum);
+    unsigned long long all = sum; // (64 bits: what does not fit 32 is refused by the callers, but must not look like less)
+#pragma unroll
+    for(int o = 32; o > 0; o >>= 1)
+        all += __shfl_xor(all, o, DSX_WAVE);
+    if(lane == 63)
     {
-        uint32_t carry = 0;
-        for(int b0 = 0; b0 < blocks; b0 += DSX_WAVE)
-        {
-            const int b = b0 + tid;
-            const uint32_t sum = b < blocks ? atomicAdd(&J.block_sums[b], 0u) : 0u;
-            const uint32_t incl = wave_incl_scan_u32(sum);
-            if(b < blocks)
-                J.block_sums[b] = carry + incl - sum;
-            carry += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
-        }
-        if(tid == 0)
-            J.block_sums[blocks] = carry;
+        s_tot[wave] = incl;
+        s_all[wave] = all;
+    }
+    __syncthreads();
+    if(tid < blocks)
+        J.block_sums[tid] = sum_of_waves_before<kRanksWaves>(s_tot, wave) + incl - sum;
+    if(tid == 0)
+    {
+        all = 0;
+        for(int w = 0; w < kRanksWaves; ++w)
+            all += s_all[w];
+        J.block_sums[blocks] = all > 0xffffffffull ? 0xffffffffu : (uint32_t)all;
     }
 }
 
-// the corner grid of all rectangles (of their bins when `bins`) in LDS, the pairs' number to the host, the counts
-__device__ __forceinline__ void small_counts(const SmallOrder& J, const bool bins, int32_t* s_grid)
+// the corner grid of the rectangles (of their bins when `bins`) in LDS, one of `parts` shares of them; then, by the workgroup
+// that is last to add its own to the whole grid: the pairs' number to the host, the counts
+__device__ __forceinline__ void count_share(const RanksJob& J, const bool bins, const int part, const int parts, int32_t* s_grid)
 {
     __shared__ unsigned long long s_pairs;
+    __shared__ int s_is_last;
     const CountsJob& C = J.counts.job[bins ? 1 : 0];
     const int tid = threadIdx.x;
     const int pitch = C.ntx + 1, cells = pitch * (C.nty + 1) + 1;
-    for(int j = tid; j < cells; j += kSmallThreads)
+    for(int j = tid; j < cells; j += kRanksThreads)
         s_grid[j] = 0;
     if(tid == 0)
         s_pairs = 0ull;
     __syncthreads();
     unsigned long long pairs = 0;
-    for(int g = tid; g < J.n; g += kSmallThreads)
+    for(int g = part * kRanksThreads + tid; g < J.n; g += parts * kRanksThreads)
     {
         const uint2 r = J.rects[g];
         int w = (int)(r.y & 0xffffu), h = (int)((r.y >> 16) & 0x7fffu);
@@ -1641,6 +1751,31 @@ __device__ __forceinline__ void small_counts(const SmallOrder& J, const bool bin
     if((tid & 63) == 0 && pairs)
         atomicAdd(&s_pairs, pairs);
     __syncthreads();
+    if(parts > 1)
+    {
+        // (an addition has been performed when its result is back; every wavefront's are before the barrier)
+        int32_t back = 0;
+        for(int j = tid; j < cells; j += kRanksThreads)
+            if(s_grid[j])
+                back |= atomicAdd(&C.grid[j], s_grid[j]);
+        unsigned long long pairs_back = 0;
+        if(tid == 0)
+            pairs_back = atomicAdd(J.key_count + (bins ? 1 : 0), s_pairs);
+        asm volatile("s_waitcnt vmcnt(0)" ::"v"(back), "v"(pairs_back) : "memory");
+        __syncthreads();
+        if(tid == 0)
+        {
+            s_is_last = atomicAdd(J.key_count + (bins ? 4 : 3), 1ull) == (unsigned long long)(parts - 1);
+            if(s_is_last)
+                s_pairs = atomicAdd(J.key_count + (bins ? 1 : 0), 0ull);
+        }
+        __syncthreads();
+        if(!s_is_last)
+            return;
+        for(int j = tid; j < cells; j += kRanksThreads)
+            s_grid[j] = __hip_atomic_load(C.grid + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+    }
     if(tid == 0 && J.to_host.words)
     {
         store_to_host(J.to_host, bins ? 1 : 0, s_pairs);
@@ -1650,59 +1785,51 @@ __device__ __forceinline__ void small_counts(const SmallOrder& J, const bool bin
     tile_counts(C, s_grid);
 }
 
-__global__ __launch_bounds__(kSmallThreads) void order_small_kernel(const SmallOrder J)
+__global__ __launch_bounds__(kRanksThreads) void order_ranks_kernel(const RanksJob J)
 {
-    extern __shared__ uint32_t s_small[];
+    extern __shared__ __attribute__((aligned(16))) uint32_t s_ranks[];
     // (the counting first: the host waits for its sums)
-    const int counting = J.shift ? 2 : 1;
-    if((int)blockIdx.x < counting)
-        small_counts(J, blockIdx.x == 1, reinterpret_cast<int32_t*>(s_small));
+    const int counting = J.counting * (J.shift ? 2 : 1), w = (int)blockIdx.x;
+    if(w < counting)
+        count_share(J, w >= J.counting, w % J.counting, J.counting, reinterpret_cast<int32_t*>(s_ranks));
     else
-        small_sort(J, (int)blockIdx.x - counting, s_small);
+        order_share(J, w - counting, s_ranks);
 }
 
 // true: done (or failed: *rc).  false: too many Gaussians, or a corner grid that does not fit the LDS
-static bool launch_order_small(const ListGrid& lg, int64_t n, char* base, const OrderLayout& o, const HostCounts& to_host,
+static bool launch_order_ranks(const ListGrid& lg, int64_t n, char* base, const OrderLayout& o, const HostCounts& to_host,
                                const CountsJobs& jobs, hipStream_t stream, int* rc)
 {
     const int cells = (lg.ntx + 1) * (lg.nty + 1) + 1;
-    if(n > kSmallMax || cells > kCoverLdsCellsLarge - 4096) // (less what the kernel has besides)
+    if(n > kRanksMax || cells > kCoverLdsCellsLarge - 4096) // (less what the kernel has besides)
         return false;
-    const size_t sort_bytes = (size_t)kSmallTile * 6 + (size_t)kSmallWaves * kSmallBins * 2;
-    const size_t bytes = std::max(sort_bytes, (size_t)cells * 4), merge_bytes = ((size_t)n * 4 + 15) & ~(size_t)15;
-    auto allow = [](const void* kernel, size_t want) {
-        if(want <= 65536 - 8192 ||
-           hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)want) == hipSuccess)
-            return true;
+    const size_t bytes = std::max(kRanksLds, (size_t)cells * 4);
+    if(bytes > 65536 - 8192 &&
+       hipFuncSetAttribute(reinterpret_cast<const void*>(order_ranks_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                           (int)bytes) != hipSuccess)
+    {
         (void)hipGetLastError();
         return false;
-    };
-    if(!allow(reinterpret_cast<const void*>(order_small_kernel), bytes) ||
-       !allow(reinterpret_cast<const void*>(order_merge_kernel), merge_bytes))
-        return false;
-    SmallOrder J;
+    }
+    RanksJob J;
     J.depth_keys = reinterpret_cast<const uint32_t*>(base + o.depth_keys);
     J.rects = reinterpret_cast<const uint2*>(base + o.rects);
+    J.key_ranges = reinterpret_cast<const uint2*>(base + o.key_ranges);
     J.order = reinterpret_cast<uint32_t*>(base + o.ids_a);
     J.rects_sorted = reinterpret_cast<uint2*>(base + o.rects_sorted);
+    J.run_sums = reinterpret_cast<uint32_t*>(base + o.run_sums);
     J.block_sums = reinterpret_cast<uint32_t*>(base + o.block_sums);
-    J.tile_keys = reinterpret_cast<uint32_t*>(base + o.keys_alt);
-    J.tile_ids = reinterpret_cast<uint32_t*>(base + o.ids_b);
-    J.done = reinterpret_cast<unsigned long long*>(base + o.key_count) + 2;
+    J.key_count = reinterpret_cast<unsigned long long*>(base + o.key_count);
     J.n = (int)n;
+    J.id_bits = std::max(1, 64 - __builtin_clzll((unsigned long long)std::max<int64_t>(n - 1, 1)));
     J.shift = lg.shift;
-    J.tiles = (int)((n + kSmallTile - 1) / kSmallTile);
+    J.shares = (int)((n + kShareWanted - 1) / kShareWanted);
+    J.counting = (int)std::min<int64_t>(kCountWorkgroupsMost, (n + kCountShare - 1) / kCountShare);
     J.counts = jobs;
     J.to_host = to_host;
     {
-        DSX_TIMED("order_small_kernel", stream);
-        hipLaunchKernelGGL(order_small_kernel, dim3(J.tiles + (lg.shift ? 2 : 1)), dim3(kSmallThreads), bytes, stream, J);
-    }
-    if(J.tiles > 1)
-    {
-        DSX_TIMED("order_merge_kernel", stream);
-        hipLaunchKernelGGL(order_merge_kernel, dim3((unsigned)((n + kMergeThreads - 1) / kMergeThreads)),
-                           dim3(kMergeThreads), merge_bytes, stream, J);
+        DSX_TIMED("order_ranks_kernel", stream);
+        hipLaunchKernelGGL(order_ranks_kernel, dim3(J.shares + J.counting * (lg.shift ? 2 : 1)), dim3(kRanksThreads), bytes, stream, J);
     }
     *rc = hipGetLastError() == hipSuccess ? DSX_OK : DSX_ERR_LAUNCH;
     return true;
@@ -1918,7 +2045,9 @@ int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_
         return rc;
 
     const CountsJobs jobs = counts_jobs(list_grid(cam), base, o);
-    if(launch_order_small(list_grid(cam), n, base, o, to_host, jobs, stream, &rc))
+    // (limits of its waits: asked for are the kernels that wait)
+    if(sort_polls == kSpinLimit32 && offset_polls == kSpinLimit32 &&
+       launch_order_ranks(list_grid(cam), n, base, o, to_host, jobs, stream, &rc))
         return rc;
 
     // pairs per tile: digit histograms of the tile partition and the tile ranges that the second

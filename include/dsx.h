@@ -401,7 +401,8 @@ int dsx_set_blend_pixels_per_lane(int pixels);
  * A tile of a sort's pass that has looked sort_polls times gives up: the sort's flag (dsx_sort_flags) is set and the order wrong,
  * with every access inside `order`, whatever it held.  The workgroups that make the block offsets tell each other their sums, and one that has
  * looked offset_polls times for another's sums up the other's rectangles itself: the offsets are the same.  For
- * tests; the other entry points look 2^18 times. */
+ * tests; the other entry points look 2^18 times.  (Up to 131072 Gaussians those order by a launch that waits for nothing; with
+ * other limits than theirs the kernels that wait are what runs, whatever the number.) */
 int dsx_depth_order_bounded(const dsx_camera* cam, int64_t n, void* order, size_t order_bytes,
                             int32_t sort_polls, int32_t offset_polls, void* stream);
 

@@ -314,3 +314,51 @@ def test_entries_in_the_lists_of_the_blocks_that_they_reach(oracle, blend_form, 
                                     B["abs_sums"], rel=1e-4)
     got = {k: out[k].cpu().numpy() for k in ("v_mean3d", "v_means2d", "v_shs", "v_opacity", "v_scale", "v_quat")}
     o.check_grads_against_bounds(got, B, bounds, gok, kind)
+
+
+@pytest.mark.parametrize("depths", ["uniform", "two", "layers", "nearly_equal", "cluster", "seldom", "one", "both_signs"])
+@pytest.mark.parametrize("n", [512, 513, 1537, 40961, 131072, 131073])
+def test_depth_order_and_counts_in_one_launch(n, depths):
+    """Up to 131072 Gaussians a workgroup finds its own 512 ranks: where a bin of the range holds many more keys than that, or keys
+    that differ in the last bits only, or hardly any key emits, or the range goes beyond the largest number there is; and just beyond.
+    Order, offsets, and the lists, ranges and histograms of tiles and of bins are those of the digit passes."""
+    from ds_splat_amd import stages
+    W, H = 200, 120
+    sc = make_scene("cfg0", n=n, width=W, height=H, sh_degree=0, seed=9)
+    u = torch.rand(n, generator=torch.Generator().manual_seed(n))
+    means = torch.zeros(n, 3)
+    means[:, 2] = {"two": torch.where(u < 0.5, 2.0, 19.0), "layers": 2.0 + (u * 20.0).floor(), "nearly_equal": 4.0 + u * 1e-5,
+                   "cluster": torch.where(u < 0.9, 4.0 + u * 1e-4, 2.0 + 18.0 * u)}.get(depths, 2.0 + 18.0 * u)
+    if depths == "both_signs":       # (a mirrored point behind the camera passes the frustum test)
+        sc["projmatrix"][:, 2] = torch.tensor([0.0, 0.0, 0.0, 0.5])
+        sc["projmatrix"][:, 3] = torch.tensor([0.0, 0.0, 0.0, 1.0])
+        means[::3, 2] *= -1.0
+    if depths == "seldom":
+        means[u > 0.01, 0] = 1e4
+    if depths == "one":
+        means[torch.arange(n) != n // 3, 0] = 1e4
+    scales = (means[:, 2:].abs() * 1e-2).expand(n, 3).contiguous()
+    for bins in (1, 4):
+        cam = stages.camera_from_scene(sc, DEV, list_bin=bins)
+        order = stages.new_order(cam, n, DEV)
+        splats, _, _, _ = stages.project_fwd(cam, means.to(DEV), scales.to(DEV), sc["rotations"].to(DEV),
+                                             sc["opacities"].to(DEV), sc["shs"].to(DEV), order=order)
+        keys = order[:4 * n].cpu().numpy().view(np.uint32).copy()
+        again = order.clone()
+        perm, offsets = (x.clone() for x in stages.depth_order(cam, n, order))
+        perm2, offsets2 = stages.depth_order_bounded(cam, n, again, sort_polls=1 << 17)      # (the digit passes)
+        emitting = keys != 0xffffffff
+        assert emitting.any()
+        if depths == "both_signs":
+            assert keys[emitting].max() >> 31 and not keys[emitting].min() >> 31 and not emitting[-1]
+        assert (perm.cpu().numpy() == np.argsort(keys, kind="stable")).all()
+        assert torch.equal(perm, perm2) and torch.equal(offsets, offsets2)
+        if bins == 1:
+            touched = splats[:, 11].contiguous().view(torch.int32).to(torch.int64)
+            touched[-1] = 0
+            assert int(offsets[-1]) == int(touched.sum())
+        k = int(offsets[-1])
+        ids, lists = stages.tile_lists(cam, n, k, order, return_lists=True)
+        ids2, lists2 = stages.tile_lists(cam, n, k, again, return_lists=True)
+        ready = cam.num_tiles + 2 + (0 if bins == 1 else 2 + -(-W // 64) * -(-H // 64))
+        assert torch.equal(ids, ids2) and torch.equal(lists[:ready], lists2[:ready])
