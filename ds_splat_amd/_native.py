@@ -84,6 +84,8 @@ SIGNATURES["dsx_trace_enable"] = (C.c_int, [C.c_int])
 SIGNATURES["dsx_trace_read"] = (C.c_int, [C.POINTER(TraceEntry), C.c_int])
 SIGNATURES["dsx_set_blend_pixels_per_lane"] = (C.c_int, [C.c_int])
 SIGNATURES["dsx_depth_order_bounded"] = (C.c_int, [_CAM, _I64, _P, C.c_size_t, _I32, _I32, _P])
+SIGNATURES["dsx_render_bytes"] = (C.c_size_t, [_I64, _I32, _I32, _I32])
+SIGNATURES["dsx_render"] = (C.c_int, [_CAM, _I64] + [_P] * 7 + [_P, _P, _P, C.c_size_t, _P])
 SIGNATURES["dsx_list_bin"] = (_I32, [_I32, _I32, _I32])
 SIGNATURES["dsx_ranges_count"] = (_I64, [_I32, _I32, _I32])
 SIGNATURES["dsx_sorted_ids_count"] = (_I64, [_I64, _I32, _I32, _I32])

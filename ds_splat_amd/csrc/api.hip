@@ -129,7 +129,7 @@ extern "C" const char* dsx_error_string(int status)
 
 extern "C" int dsx_version(void)
 {
-    return 311;
+    return 312;
 }
 
 extern "C" int64_t dsx_num_blocks(int64_t n)
@@ -681,6 +681,60 @@ extern "C" int dsx_forward_finish(const dsx_camera* cam, int64_t n, int64_t k, c
     return launch_blend_fwd(*cam, n, n > 0 ? k : 0, ranges, sorted_ids, splats, image, final_T, final_idx,
                             as_stream(stream), true, depth_flag, partition_flag, n > 0 ? grads_to_prepare : nullptr,
                             true);
+}
+
+namespace
+{
+// splat records | depth keys | rectangles | the projection's sums and key ranges by block
+struct RenderLayout
+{
+    size_t splats, depth_keys, rects, key_ranges, block_sums, bytes;
+};
+RenderLayout render_layout(int64_t n)
+{
+    auto align = [](size_t x) { return (x + 255) & ~(size_t)255; };
+    const size_t blocks = (size_t)dsx_num_blocks(n);
+    RenderLayout l;
+    l.splats = 0;
+    l.depth_keys = align((size_t)n * DSX_SPLAT_FLOATS * 4);
+    l.rects = align(l.depth_keys + (size_t)n * 4);
+    l.key_ranges = align(l.rects + (size_t)n * 8);
+    l.block_sums = align(l.key_ranges + blocks * 8);
+    l.bytes = align(l.block_sums + blocks * 4);
+    return l;
+}
+} // namespace
+
+extern "C" size_t dsx_render_bytes(int64_t n, int32_t width, int32_t height, int32_t list_bin)
+{
+    if(width <= 0 || height <= 0 || !valid_list_bin(list_bin) || !blends_own_lists(n, list_grid(width, height, list_bin)))
+        return 0;
+    return render_layout(n).bytes;
+}
+
+extern "C" int dsx_render(const dsx_camera* cam, int64_t n, const float* means3d, const float* scales, const float* quats,
+                          const float* opacities, const float* shs, const float* cov3d_precomp, const float* colors_precomp,
+                          int32_t* radii, float* image, void* scratch, size_t scratch_bytes, void* stream)
+{
+    if(int rc = check_camera(cam))
+        return rc;
+    const size_t bytes = dsx_render_bytes(n, cam->image_width, cam->image_height, camera_bin(*cam));
+    if(bytes == 0 || !means3d || !opacities || !radii || !image || !scratch || ((uintptr_t)scratch & 15) != 0)
+        return DSX_ERR_BAD_ARG;
+    if((!cov3d_precomp && (!scales || !quats)) || (!colors_precomp && !shs))
+        return DSX_ERR_BAD_ARG;
+    if(scratch_bytes < bytes)
+        return DSX_ERR_WORKSPACE;
+    const RenderLayout l = render_layout(n);
+    char* const base = static_cast<char*>(scratch);
+    float* const splats = reinterpret_cast<float*>(base + l.splats);
+    uint32_t* const depth_keys = reinterpret_cast<uint32_t*>(base + l.depth_keys);
+    uint2* const rects = reinterpret_cast<uint2*>(base + l.rects);
+    if(int rc = launch_project_fwd(*cam, n, means3d, scales, quats, opacities, shs, cov3d_precomp, colors_precomp, splats, radii,
+                                   nullptr, reinterpret_cast<uint32_t*>(base + l.block_sums), depth_keys, rects,
+                                   reinterpret_cast<uint2*>(base + l.key_ranges), nullptr, as_stream(stream)))
+        return rc;
+    return launch_blend_fwd_own(*cam, n, depth_keys, rects, splats, image, as_stream(stream));
 }
 
 static int backward_impl(const dsx_camera* cam, int64_t n, int64_t k, int32_t num_bases, const float* means3d,

@@ -1119,20 +1119,348 @@ constexpr int kWideThreads = 1024;
 constexpr int kWideWaves = kWideThreads / DSX_WAVE;
 static_assert(kWideWaves == kQuads, "a wavefront for each block");
 
+// Lists that nobody made: a forward without a backward, of few tiles and not too many Gaussians, needs none but each tile's own
+// entries in order, and a workgroup finds them faster than a depth order, pairs and their partition can bring them (and the
+// host need not wait for the pairs' number): it looks at all rectangles, takes those that cover its tile, sorts them
+// by depth and index in LDS, and blends them.  Where more than kOwnMost do, it takes them in windows, nearest first, each found by
+// counting the rest into bins.  Each colour is then a sum in other parts; all else has the same bits.
+struct OwnLists
+{
+    const uint32_t* depth_keys; // by Gaussian, as the projection leaves them
+    const uint2* rects;
+    int n;
+};
+// us of a whole forward, 64x64 / 128x128 / 208x208 / 256x256, four kinds of scenes (small, mixed, faint, large), with lists -> without:
+//   6 K Gaussians   62, 63, 57, 63 -> 47, 48, 42, 46 / 43, 45, 42, 55 -> 25, 28, 23, 36 / 41, 44, 40, 53 -> 22, 24, 21, 34 / 45, 48, 45, 61 -> 21, 23, 20, 33
+//   10 K            81, 84, 72, 66 -> 69, 73, 61, 57 / 52, 55, 49, 56 -> 36, 38, 33, 40 / 45, 49, 43, 57 -> 27, 30, 26, 37 / 48, 54, 49, 67 -> 25, 29, 24, 36
+//   16 K            89, 112, 97, 62 -> 103, 144, 111, 61 / 61, 68, 57, 56 -> 45, 53, 42, 50 / 51, 58, 50, 58 -> 33, 40, 32, 38 / 54, 63, 52, 66 -> 30, 37, 28, 37
+//   24 K            (slower) / 74, 86, 69, 58 -> 59, 72, 56, 59 / 62, 71, 57, 61 -> 45, 53, 40, 60 / 64, 75, 61, 72 -> 40, 49, 37, 58
+//   32 K            (slower) / 77, 90, 81, 60 -> 65, 120, 71, 68 / 68, 81, 65, 63 -> 53, 66, 50, 68 / 72, 85, 68, 73 -> 49, 60, 44, 66
+// 2 K at 64x64 40 -> 24.  What ends it are the windows, each of which costs another three or four looks at everything: the line of
+// 9000 Gaussians and a hundred more for each tile lies below where the first kind of scene loses.
+constexpr int kOwnGaussians = 9000, kOwnGaussiansPerTile = 100;
+constexpr int kOwnMost = 4096; // entries of a window
+constexpr int kOwnBins = 4096;
+constexpr int kOwnBinBits = 12;
+static_assert(kOwnBins == 4 * kWideThreads && kOwnMost == 4 * kWideThreads, "what the threads take");
+constexpr int kOwnGroupMost = 64; // entries in one bin that are compared with each other one by one
+
+// The entries of one tile (sx >= 0), or, one copy for each tile that they touch, all those of negative depth (see TileSource)
+struct OwnSource
+{
+    int sx, sy;
+    __device__ __forceinline__ int copies(uint2 r) const
+    {
+        const uint32_t w = r.y & 0xffffu, h = (r.y >> 16) & 0x7fffu;
+        if(sx < 0)
+            return (int)r.y < 0 ? (int)(w * h) : 0;
+        return (int)r.y >= 0 && (uint32_t)sx - (r.x & 0xffffu) < w && (uint32_t)sy - (r.x >> 16) < h ? 1 : 0;
+    }
+};
+
+// What finding and sorting a window's entries takes of the LDS
+struct OwnScratch
+{
+    uint64_t numbers[kOwnMost]; // depth key, index
+    uint64_t binned[kOwnMost];
+    uint32_t hist[kOwnBins];
+};
+struct OwnShared
+{
+    uint32_t tot[kWideWaves];
+    uint32_t found[3];
+    uint32_t taken, most, nearest, farthest;
+    int highest;
+};
+
+// f(index, copies) for every rectangle of the source with an entry
+template <typename F>
+__device__ __forceinline__ void own_for_all(const OwnLists& L, const OwnSource& src, F f)
+{
+    for(int i0 = 0; i0 < L.n; i0 += 8 * kWideThreads)
+    {
+        uint2 r[8];
+#pragma unroll
+        for(int b = 0; b < 8; ++b)
+        {
+            const int i = i0 + b * kWideThreads + (int)threadIdx.x;
+            r[b] = i < L.n ? L.rects[i] : make_uint2(0u, 0u);
+        }
+        f(i0, r, src);
+    }
+}
+
+// The numbers in [low, high) of the source's entries into scratch.numbers (as far as there is room), in any order; returns how many there
+// are, and their nearest and farthest depth keys.
+__device__ __forceinline__ int own_take(const OwnLists& L, const OwnSource& src, OwnScratch& S, OwnShared& sh, uint64_t low, uint64_t high,
+                                        bool everything)
+{
+    const int tid = threadIdx.x, lane = tid & (DSX_WAVE - 1);
+    __syncthreads();
+    if(tid == 0)
+    {
+        sh.taken = 0;
+        sh.nearest = 0xffffffffu;
+        sh.farthest = 0;
+    }
+    __syncthreads();
+    int highest = 0;
+    uint32_t* const ids = reinterpret_cast<uint32_t*>(S.binned);
+    own_for_all(L, src, [&](int i0, const uint2 (&r)[8], const OwnSource& from) {
+        uint32_t mine = 0, copies[8];
+#pragma unroll
+        for(int b = 0; b < 8; ++b)
+        {
+            // (columns and rows behind the rectangle's last ones, packed: the largest is the highest tile's; below zero behind the camera)
+            highest = max(highest, (int)(r[b].x + r[b].y));
+            copies[b] = (uint32_t)from.copies(r[b]);
+            if(!everything && copies[b])
+            {
+                const uint64_t number = (uint64_t)L.depth_keys[i0 + b * kWideThreads + tid] << 32 | (uint32_t)(i0 + b * kWideThreads + tid);
+                copies[b] = number >= low && number < high ? copies[b] : 0u;
+            }
+            mine += copies[b];
+        }
+        if(__builtin_amdgcn_ballot_w64(mine != 0) == 0)
+            return;
+        const uint32_t incl = wave_incl_scan_u32(mine);
+        uint32_t at = 0;
+        if(lane == DSX_WAVE - 1)
+            at = atomicAdd(&sh.taken, incl);
+        at = (uint32_t)__builtin_amdgcn_readlane((int)at, DSX_WAVE - 1) + incl - mine;
+#pragma unroll
+        for(int b = 0; b < 8; ++b)
+            for(uint32_t c = 0; c < copies[b]; ++c, ++at)
+                if(at < (uint32_t)kOwnMost)
+                    ids[at] = (uint32_t)(i0 + b * kWideThreads + tid);
+    });
+    if(everything)
+    {
+#pragma unroll
+        for(int o = DSX_WAVE / 2; o > 0; o >>= 1)
+            highest = max(highest, __shfl_xor(highest, o, DSX_WAVE));
+        if(lane == 0)
+            atomicMax(&sh.highest, highest);
+    }
+    __syncthreads();
+    const int total = (int)__builtin_amdgcn_readfirstlane((int)sh.taken), count = min(total, kOwnMost);
+    uint32_t nearest = 0xffffffffu, farthest = 0;
+#pragma unroll
+    for(int b = 0; b < kOwnMost / kWideThreads; ++b)
+    {
+        const int at = b * kWideThreads + tid;
+        if(at < count)
+        {
+            const uint32_t id = ids[at], key = L.depth_keys[id];
+            S.numbers[at] = (uint64_t)key << 32 | id;
+            nearest = min(nearest, key);
+            farthest = max(farthest, key);
+        }
+    }
+#pragma unroll
+    for(int o = DSX_WAVE / 2; o > 0; o >>= 1)
+    {
+        nearest = min(nearest, (uint32_t)__shfl_xor((int)nearest, o, DSX_WAVE));
+        farthest = max(farthest, (uint32_t)__shfl_xor((int)farthest, o, DSX_WAVE));
+    }
+    if(lane == 0)
+    {
+        atomicMin(&sh.nearest, nearest);
+        atomicMax(&sh.farthest, farthest);
+    }
+    __syncthreads();
+    return total;
+}
+
+__device__ __forceinline__ int number_bits(uint64_t v)
+{
+    return v ? 64 - __builtin_clzll(v) : 0;
+}
+
+// exclusive sums of the histogram's bins in place of their counts
+__device__ __forceinline__ void own_scan(OwnScratch& S, OwnShared& sh)
+{
+    const int tid = threadIdx.x, lane = tid & (DSX_WAVE - 1), wave = tid / DSX_WAVE;
+    __syncthreads();
+    uint4* const mine = reinterpret_cast<uint4*>(S.hist) + tid;
+    const uint4 c = *mine;
+    const uint32_t sum = c.x + c.y + c.z + c.w, incl = wave_incl_scan_u32(sum);
+    if(lane == DSX_WAVE - 1)
+        sh.tot[wave] = incl;
+    __syncthreads();
+    const uint32_t at = sum_of_waves_before<kWideWaves>(sh.tot, wave) + incl - sum;
+    *mine = make_uint4(at, at + c.x, at + c.x + c.y, at + c.x + c.y + c.z);
+    __syncthreads();
+}
+
+// scratch.numbers [0, count), of depth keys nearest to farthest, in order: their indices into `ids`
+__device__ __forceinline__ void own_sort(OwnScratch& S, OwnShared& sh, int count, uint32_t* ids)
+{
+    constexpr int kItems = kOwnMost / kWideThreads;
+    const int tid = threadIdx.x;
+    const uint64_t from = (uint64_t)sh.nearest << 32, width = ((uint64_t)(sh.farthest - sh.nearest) << 32) | 0xffffffffull;
+    const int shift = max(number_bits(width) - kOwnBinBits, 0);
+    reinterpret_cast<uint4*>(S.hist)[tid] = make_uint4(0u, 0u, 0u, 0u);
+    if(tid == 0)
+        sh.most = 0;
+    __syncthreads();
+    uint64_t mine[kItems];
+    uint32_t bin[kItems], nth[kItems], most = 0;
+#pragma unroll
+    for(int b = 0; b < kItems; ++b)
+    {
+        const int at = b * kWideThreads + tid;
+        bin[b] = nth[b] = 0;
+        mine[b] = ~0ull;
+        if(at < count)
+        {
+            mine[b] = S.numbers[at];
+            bin[b] = (uint32_t)((mine[b] - from) >> shift);
+            nth[b] = atomicAdd(&S.hist[bin[b]], 1u);
+            most = max(most, nth[b]);
+        }
+    }
+    if(__builtin_amdgcn_ballot_w64(most >= kOwnGroupMost) != 0 && (tid & (DSX_WAVE - 1)) == 0)
+        sh.most = 1;
+    own_scan(S, sh);
+    if(__builtin_amdgcn_readfirstlane((int)sh.most) == 0)
+    {
+        uint32_t start[kItems], end[kItems];
+#pragma unroll
+        for(int b = 0; b < kItems; ++b)
+            if(b * kWideThreads + tid < count)
+            {
+                start[b] = S.hist[bin[b]];
+                end[b] = bin[b] + 1 < kOwnBins ? S.hist[bin[b] + 1] : (uint32_t)count;
+                S.binned[start[b] + nth[b]] = mine[b];
+            }
+        __syncthreads();
+#pragma unroll
+        for(int b = 0; b < kItems; ++b)
+            if(b * kWideThreads + tid < count)
+            {
+                uint32_t r = start[b];
+                for(uint32_t j = start[b]; j < end[b]; ++j) // (copies of one entry among them)
+                    r += S.binned[j] < mine[b] || (S.binned[j] == mine[b] && j < start[b] + nth[b]) ? 1u : 0u;
+                ids[r] = (uint32_t)mine[b];
+            }
+    }
+    else
+    {
+        // many depths alike: a bitonic sort
+        int size = kWideThreads;
+        while(size < count)
+            size *= 2;
+        for(int at = tid; at < size; at += kWideThreads)
+            S.binned[at] = at < count ? S.numbers[at] : ~0ull;
+        for(int k = 2; k <= size; k *= 2)
+            for(int j = k / 2; j > 0; j /= 2)
+            {
+                __syncthreads();
+                for(int e = tid; e < size / 2; e += kWideThreads)
+                {
+                    const int i = 2 * e - (e & (j - 1)), l = i + j;
+                    const uint64_t u = S.binned[i], v = S.binned[l];
+                    if((u > v) == ((i & k) == 0))
+                    {
+                        S.binned[i] = v;
+                        S.binned[l] = u;
+                    }
+                }
+            }
+        __syncthreads();
+        for(int at = tid; at < count; at += kWideThreads)
+            ids[at] = (uint32_t)S.binned[at];
+    }
+    __syncthreads();
+}
+
+// Of the source's numbers from `low` on, more than kOwnMost: a border that leaves half as many to kOwnMost of them in front.
+__device__ __forceinline__ uint64_t own_border(const OwnLists& L, const OwnSource& src, OwnScratch& S, OwnShared& sh, uint64_t low)
+{
+    constexpr uint32_t kWanted = kOwnMost / 2;
+    const int tid = threadIdx.x;
+    uint64_t base = low;
+    uint32_t before = 0; // numbers in [low, base)
+    int wide = number_bits(~low), shift = max(wide - kOwnBinBits, 0);
+    while(true)
+    {
+        __syncthreads();
+        reinterpret_cast<uint4*>(S.hist)[tid] = make_uint4(0u, 0u, 0u, 0u);
+        __syncthreads();
+        own_for_all(L, src, [&](int i0, const uint2 (&r)[8], const OwnSource& from) {
+#pragma unroll
+            for(int b = 0; b < 8; ++b)
+            {
+                const int copies = from.copies(r[b]), i = i0 + b * kWideThreads + tid;
+                if(copies)
+                {
+                    const uint64_t number = (uint64_t)L.depth_keys[i] << 32 | (uint32_t)i, d = number - base;
+                    if(number >= base && (wide >= 64 || (d >> wide) == 0))
+                        atomicAdd(&S.hist[(uint32_t)(d >> shift)], (uint32_t)copies);
+                }
+            }
+        });
+        __syncthreads();
+        const uint4 c = reinterpret_cast<const uint4*>(S.hist)[tid];
+        const uint32_t count[4] = {c.x, c.y, c.z, c.w};
+        own_scan(S, sh);
+        // the first bin border with kWanted numbers or more in front
+#pragma unroll
+        for(int u = 0; u < 4; ++u)
+        {
+            const uint32_t at = before + S.hist[4 * tid + u];
+            if(at < kWanted && kWanted <= at + count[u])
+            {
+                sh.found[0] = 4 * tid + u;
+                sh.found[1] = at;
+                sh.found[2] = at + count[u];
+            }
+        }
+        __syncthreads();
+        const uint32_t bin = __builtin_amdgcn_readfirstlane((int)sh.found[0]);
+        const uint32_t front = __builtin_amdgcn_readfirstlane((int)sh.found[1]), behind = __builtin_amdgcn_readfirstlane((int)sh.found[2]);
+        if(behind <= (uint32_t)kOwnMost || shift == 0) // (copies of one entry: a tile each of an image of few)
+            return base + ((uint64_t)(bin + 1) << shift);
+        base += (uint64_t)bin << shift;
+        before = front;
+        wide = shift;
+        shift = max(wide - kOwnBinBits, 0);
+    }
+}
+
+template <bool kOwn>
 __global__ __launch_bounds__(kWideThreads) void blend_fwd_wide_kernel(const int32_t* __restrict__ ranges, const int32_t* __restrict__ ids,
-                                                                      const float4* __restrict__ splats, float* __restrict__ image,
-                                                                      float* __restrict__ final_T, int32_t* __restrict__ final_idx, int W,
-                                                                      int H, int ntx, uint32_t last_id, int k,
+                                                                      const float4* __restrict__ splats,
+                                                                      float* __restrict__ image, float* __restrict__ final_T,
+                                                                      int32_t* __restrict__ final_idx, int W, int H, int ntx,
+                                                                      uint32_t last_id, int k,
                                                                       const int32_t* __restrict__ header, int header_shift,
                                                                       const uint32_t* __restrict__ sort_flag_a,
-                                                                      const uint32_t* __restrict__ sort_flag_b, float4* __restrict__ prep,
-                                                                      int64_t prep_count, uint8_t* __restrict__ prep_marks,
-                                                                      const float* __restrict__ bg, int planar)
+                                                                      const uint32_t* __restrict__ sort_flag_b,
+                                                                      float4* __restrict__ prep, int64_t prep_count,
+                                                                      uint8_t* __restrict__ prep_marks,
+                                                                      const float* __restrict__ bg, int planar, const OwnLists own)
 {
     // (arrays as in the other forms; eight places more than an entry has blocks: the lists' ends name nobody's place, read ahead)
-    __shared__ float4 s_a[kWideBatch + 1], s_b[kWideBatch + 1], s_c[kWideBatch + 1];
-    __shared__ uint16_t s_reach[kWideBatch];
-    __shared__ uint16_t s_list[kWideWaves][kWideBatch + 8];
+    struct Staged
+    {
+        float4 a[kWideBatch + 1], b[kWideBatch + 1], c[kWideBatch + 1];
+        uint16_t list[kWideWaves][kWideBatch + 8];
+        uint16_t reach[kWideBatch];
+    };
+    union Memory // (own lists: a window's entries are found and sorted before they are staged)
+    {
+        Staged staged;
+        OwnScratch scratch;
+    };
+    __shared__ __attribute__((aligned(16))) char s_memory[kOwn ? sizeof(Memory) : sizeof(Staged)];
+    __shared__ uint32_t s_own_ids[kOwn ? kOwnMost : 1];
+    __shared__ __attribute__((aligned(16))) OwnShared s_own;
+    Staged& staged_lds = *reinterpret_cast<Staged*>(s_memory);
+    float4 *const s_a = staged_lds.a, *const s_b = staged_lds.b, *const s_c = staged_lds.c;
+    uint16_t* const s_reach = staged_lds.reach;
+    uint16_t (*const s_list)[kWideBatch + 8] = staged_lds.list;
     __shared__ int s_counts[kWideWaves];
     __shared__ uint32_t s_live[kWideWaves];
 
@@ -1144,9 +1472,9 @@ __global__ __launch_bounds__(kWideThreads) void blend_fwd_wide_kernel(const int3
     const float pxf = (float)x + 0.5f;
 
     // (positions and layout are taken for what they are as in the wavefront form)
-    const bool layout_ok = header == nullptr || *header == header_shift;
+    const bool layout_ok = kOwn || header == nullptr || *header == header_shift;
     int scan = 0, end = 0;
-    if(layout_ok)
+    if(!kOwn && layout_ok)
     {
         scan = min(max(ranges[tile], 0), k);
         end = min(max(ranges[tile + 1], 0), k);
@@ -1157,14 +1485,61 @@ __global__ __launch_bounds__(kWideThreads) void blend_fwd_wide_kernel(const int3
     float pyf = inside ? (float)y + 0.5f : __builtin_nanf(""); // (NaN: stopped)
     float T = 1.0f, red = 0.f, green = 0.f, blue = 0.f;        // (the colours of this lane's entries)
     int last = 0;
+
+    // own lists: whose entries (as tile_source has it), all of them if they fit a window
+    OwnSource src = {tile % ntx, tile / ntx};
+    OwnScratch& scratch = *reinterpret_cast<OwnScratch*>(s_memory);
+    uint64_t low = 0;
+    int remaining = 0;
+    if(kOwn)
+    {
+        if(tid == 0)
+            s_own.highest = 0;
+        remaining = own_take(own, src, scratch, s_own, 0, 0, true);
+        const int highest = __builtin_amdgcn_readfirstlane(s_own.highest); // (0: no tile is occupied)
+        const int last_x = (highest & 0xffff) - 1, last_y = (highest >> 16) - 1;
+        const bool occupied = highest > 0, mine = occupied && src.sx == last_x && src.sy == last_y;
+        if(blockIdx.x == gridDim.x - 1)
+        {
+            if(!mine)
+            {
+                src.sx = occupied ? last_x : -1;
+                src.sy = occupied ? last_y : -1;
+                remaining = own_take(own, src, scratch, s_own, 0, 0, true);
+            }
+        }
+        else if(mine)
+            remaining = 0;
+    }
+    bool first_window = true;
+    while(true) // (windows; one of lists that are there)
+    {
+    if(kOwn)
+    {
+        if(remaining <= 0)
+            break;
+        int count = remaining;
+        if(!first_window || remaining > kOwnMost)
+        {
+            const uint64_t high = remaining > kOwnMost ? own_border(own, src, scratch, s_own, low) : ~0ull;
+            count = min(own_take(own, src, scratch, s_own, low, high, false), kOwnMost);
+            low = high;
+        }
+        own_sort(scratch, s_own, count, s_own_ids);
+        remaining -= count;
+        first_window = false;
+        scan = 0;
+        left = count;
+    }
     if(tid == 0)
     {
         s_a[kWideBatch] = s_c[kWideBatch] = make_float4(0.f, 0.f, 0.f, 0.f);
         s_b[kWideBatch] = make_float4(0.f, 0.f, __int_as_float(INT_MIN), 0.f);
     }
+    const int32_t* const list_ids = kOwn ? reinterpret_cast<const int32_t*>(s_own_ids) : ids;
     int id_ahead = 0;
     if(tid < min(left, kWideBatch))
-        id_ahead = ids[scan + tid];
+        id_ahead = list_ids[scan + tid];
     while(true)
     {
         const bool live = __builtin_amdgcn_ballot_w64(pyf == pyf) != 0;
@@ -1172,13 +1547,15 @@ __global__ __launch_bounds__(kWideThreads) void blend_fwd_wide_kernel(const int3
             s_live[wave] = live;
         __syncthreads(); // (and the last round's entries have been walked)
         const uint32_t live_blocks = (uint32_t)__builtin_amdgcn_ballot_w64(lane < kWideWaves && s_live[lane & (kWideWaves - 1)] != 0);
+        if(live_blocks == 0)
+            remaining = 0;
         if(live_blocks == 0 || left <= 0)
             break;
         const int batch = min(left, kWideBatch), id = id_ahead, index_next = scan;
         scan += batch;
         left -= batch;
         if(tid < min(left, kWideBatch))
-            id_ahead = ids[scan + tid]; // the next round's: in flight meanwhile
+            id_ahead = list_ids[scan + tid]; // the next round's: in flight meanwhile
         uint32_t reached = 0;
         float4 q0, q1, q2;
         float reach = 0.0f;
@@ -1283,6 +1660,9 @@ __global__ __launch_bounds__(kWideThreads) void blend_fwd_wide_kernel(const int3
             last = __builtin_amdgcn_inverse_ballot_w64(m_pass) ? __float_as_int(e.B.w) : last;
         }
     }
+    if(!kOwn)
+        break;
+    }
 
     const bool broken = !layout_ok || (sort_flag_a && *sort_flag_a) || (sort_flag_b && *sort_flag_b);
     // the quad's four parts of the colour, and the last of its last entries
@@ -1296,11 +1676,39 @@ __global__ __launch_bounds__(kWideThreads) void blend_fwd_wide_kernel(const int3
     if(inside && slot == 0)
     {
         const int64_t pix = (int64_t)y * W + x;
-        final_T[pix] = T;
-        final_idx[pix] = last;
+        if(!kOwn)
+        {
+            final_T[pix] = T;
+            final_idx[pix] = last;
+        }
         store_pixel(image, pix, (int64_t)W * H, red, green, blue, T, broken, bg, planar);
     }
-    prepare_grads_share(splats, prep, prep_count, prep_marks, blockIdx.x, gridDim.x, tid, kWideThreads);
+    if(!kOwn)
+        prepare_grads_share(splats, prep, prep_count, prep_marks, blockIdx.x, gridDim.x, tid, kWideThreads);
+}
+
+// Does a forward without a backward find its lists itself?
+bool blends_own_lists(int64_t n, const ListGrid& lg)
+{
+    return n > 0 && lg.shift == 0 && lg.tiles() > 0 && lg.tiles() <= kFwdWideUpTo &&
+           n <= kOwnGaussians + (int64_t)kOwnGaussiansPerTile * lg.tiles() && forced_pixels_per_lane() == 0;
+}
+
+int launch_blend_fwd_own(const dsx_camera& cam, int64_t n, const uint32_t* depth_keys, const uint2* rects, const float* splats, float* image,
+                         hipStream_t stream)
+{
+    const ListGrid lg = list_grid(cam);
+    if(!blends_own_lists(n, lg))
+        return DSX_ERR_BAD_ARG;
+    {
+        DSX_TIMED("blend_fwd_kernel", stream);
+        hipLaunchKernelGGL(blend_fwd_wide_kernel<true>, dim3(lg.tiles()), dim3(kWideThreads), 0, stream, nullptr, nullptr,
+                           reinterpret_cast<const float4*>(splats), image, nullptr, nullptr, cam.image_width, cam.image_height, lg.ntx,
+                           (uint32_t)(n - 1), 0, nullptr, 0, nullptr, nullptr, nullptr, (int64_t)0, nullptr, cam.bg,
+                           camera_flag(cam, DSX_PLANAR_IMAGE), OwnLists{depth_keys, rects, (int)n});
+    }
+    DSX_LAUNCH_CHECK();
+    return DSX_OK;
 }
 
 // The BinLists view of a `ranges` buffer in ranges_layout(lg) (lists per bin: lg.shift > 0)
@@ -1353,9 +1761,9 @@ int launch_blend_fwd(const dsx_camera& cam, int64_t n, int64_t k, int32_t* range
         const dim3 grid(ntx * nty);
         const float4* sp = reinterpret_cast<const float4*>(splats);
         if(wide)
-            hipLaunchKernelGGL(blend_fwd_wide_kernel, grid, dim3(kWideThreads), 0, stream, ranges, sorted_ids, sp, image, final_T,
+            hipLaunchKernelGGL(blend_fwd_wide_kernel<false>, grid, dim3(kWideThreads), 0, stream, ranges, sorted_ids, sp, image, final_T,
                                final_idx, cam.image_width, cam.image_height, ntx, last_id, (int)k, header, lg.shift, sort_flag_a,
-                               sort_flag_b, prep, prep_count, prep_marks, cam.bg, camera_flag(cam, DSX_PLANAR_IMAGE));
+                               sort_flag_b, prep, prep_count, prep_marks, cam.bg, camera_flag(cam, DSX_PLANAR_IMAGE), OwnLists{});
 #define DSX_LAUNCH_FWD(KERNEL, THREADS)                                                                          \
     hipLaunchKernelGGL((KERNEL), grid, dim3(THREADS), 0, stream, ranges, sorted_ids, sp, image, final_T, final_idx,  \
                        cam.image_width, cam.image_height, ntx, last_id, (int)k, header, lg.shift, sort_flag_a,     \

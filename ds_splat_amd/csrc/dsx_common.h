@@ -420,6 +420,10 @@ int launch_blend_fwd(const dsx_camera& cam, int64_t n, int64_t k, int32_t* range
                      const float* splats, float* image, float* final_T, int32_t* final_idx, hipStream_t stream,
                      bool check_header, const uint32_t* sort_flag_a = nullptr, const uint32_t* sort_flag_b = nullptr,
                      float* prepare_grads = nullptr, bool prepare_marks = false);
+// a forward without a backward, of few tiles, from what the projection leaves: each tile finds its own entries (no lists, no final values)
+bool blends_own_lists(int64_t n, const ListGrid& lg);
+int launch_blend_fwd_own(const dsx_camera& cam, int64_t n, const uint32_t* depth_keys, const uint2* rects, const float* splats,
+                         float* image, hipStream_t stream);
 int launch_blend_bwd(const dsx_camera& cam, int64_t n, int64_t k, const int32_t* ranges, const int32_t* sorted_ids,
                      const float* splats, const float* final_T, const int32_t* final_idx, const float* v_image,
                      float* grads, hipStream_t stream, bool check_header, bool grads_prepared = false,

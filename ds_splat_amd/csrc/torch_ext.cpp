@@ -204,7 +204,8 @@ struct Rendered
     int64_t k = 0;
 };
 
-Rendered render(const Camera& cam, const Inputs& in, bool prepare_backward)
+// image_only: what the image and the radii do not need need not be there
+Rendered render(const Camera& cam, const Inputs& in, bool prepare_backward, bool image_only = false)
 {
     const at::Device dev = in.means3d.device();
     const int64_t n = in.means3d.numel() / 3;
@@ -215,8 +216,18 @@ Rendered render(const Camera& cam, const Inputs& in, bool prepare_backward)
     void* s = current_stream(dev);
 
     Rendered r;
-    r.splats = at::empty({n + kViewRecords, DSX_SPLAT_FLOATS}, f32);
     r.radii = at::empty({n}, i32);
+    auto new_image = [&] { return cam.planar ? at::empty({3, H, W}, f32) : at::empty({H, W, 3}, f32); };
+    if(const size_t bytes = image_only ? dsx_render_bytes(n, W, H, bin) : 0)
+    {
+        at::Tensor scratch = at::empty({(int64_t)bytes}, u8);
+        r.image = new_image();
+        check(dsx_render(&cam.c, n, in.means3d.data_ptr<float>(), fptr(in.scales), fptr(in.quats), in.opacities.data_ptr<float>(),
+                         fptr(in.shs), fptr(in.cov3d), fptr(in.colors), r.radii.data_ptr<int32_t>(), r.image.data_ptr<float>(),
+                         scratch.data_ptr(), bytes, s));
+        return r;
+    }
+    r.splats = at::empty({n + kViewRecords, DSX_SPLAT_FLOATS}, f32);
     // scratch of the first half: the projection's block sums and, behind them, the depth order
     const size_t sums_bytes = ((size_t)std::max<int64_t>(dsx_num_blocks(n), 1) * 4 + 255) & ~(size_t)255;
     const size_t order_bytes = dsx_order_bytes(n, W, H, bin);
@@ -230,7 +241,7 @@ Rendered render(const Camera& cam, const Inputs& in, bool prepare_backward)
                                     prepare_backward ? r.splats.data_ptr<float>() + n * DSX_SPLAT_FLOATS : nullptr, s));
     // (while the device counts the pairs: everything whose size does not depend on their number)
     r.ranges = at::empty({dsx_ranges_count(W, H, bin)}, i32);
-    r.image = cam.planar ? at::empty({3, H, W}, f32) : at::empty({H, W, 3}, f32);
+    r.image = new_image();
     r.final_T = at::empty({H, W}, f32);
     r.final_idx = at::empty({H, W}, i32);
     if(prepare_backward && n > 0)
@@ -399,7 +410,7 @@ std::tuple<at::Tensor, at::Tensor> forward(const at::Tensor& means3d, const at::
          needs_node(scales) || needs_node(quats) || needs_node(cov3d)))
     {
         c10::DeviceGuard guard(means3d.device());
-        Rendered r = render(make_camera(settings, means3d.device()), in, false);
+        Rendered r = render(make_camera(settings, means3d.device()), in, false, true);
         return {r.image, r.radii};
     }
     auto out = Rasterize::apply(means3d, means2d, shs, colors, opacities, scales, quats, cov3d, settings);

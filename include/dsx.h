@@ -96,7 +96,7 @@ typedef struct dsx_camera
  */
 
 const char* dsx_error_string(int status);
-/* 100 * major + minor.  311: dsx_depth_order_bounded.  310: flags beside dsx_camera::list_bin, the projection's wait for the pair
+/* 100 * major + minor.  312: dsx_render.  311: dsx_depth_order_bounded.  310: flags beside dsx_camera::list_bin, the projection's wait for the pair
  * counts is a function of its own.  300: the bin size of the tile lists is an argument (dsx_camera::list_bin and
  * the size helpers) instead of a process-wide setting; the `ranges` buffer carries it in a header word;
  * the blend entry points and the backward are told n and k and follow no id or list position beyond
@@ -323,6 +323,19 @@ int dsx_forward_finish(const dsx_camera* cam, int64_t n, int64_t k, const float*
                        const void* order, int32_t* sorted_ids, int32_t* ranges, float* image,
                        float* final_T, int32_t* final_idx, void* workspace,
                        size_t workspace_bytes, float* grads_to_prepare, void* stream);
+
+/* A forward that no backward follows, of an image of few tiles and not too many Gaussians, in two launches: every tile finds and sorts
+ * its own entries, so there are no pairs, no lists and nothing that the host waits for.  The image and the radii are those of
+ * dsx_forward_project and dsx_forward_finish (which take any image and any number): bit for bit, or, where a tile has more than 4096
+ * entries, with each colour added up in other parts.
+ * dsx_render_bytes: bytes of its scratch (16-byte aligned), or 0 where it does not apply: more than 256 tiles, more Gaussians
+ * than 9000 and a hundred for each tile, lists per bin asked for, no Gaussian, or a form of the blend kernels set by
+ * dsx_set_blend_pixels_per_lane.
+ * dsx_render: DSX_ERR_BAD_ARG there. */
+size_t dsx_render_bytes(int64_t n, int32_t width, int32_t height, int32_t list_bin);
+int dsx_render(const dsx_camera* cam, int64_t n, const float* means3d, const float* scales, const float* quats,
+               const float* opacities, const float* shs, const float* cov3d_precomp, const float* colors_precomp,
+               int32_t* radii, float* image, void* scratch, size_t scratch_bytes, void* stream);
 
 /* rasterizer_backward_deepsense, cpp/rasterizer_torch.cu:263-316.  k: entries of sorted_ids (the k
  * of the forward); ranges: the buffer that dsx_forward_finish filled, for the same cam->list_bin (a

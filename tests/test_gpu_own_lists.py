@@ -1,0 +1,106 @@
+"""A forward without a backward, of few tiles: every tile finds its own entries.  The image and the radii against the general
+path's (whose lists, ranges and images are compared with the oracle's elsewhere), which a forward with a backward to follow takes."""
+import pytest
+import torch
+
+from ds_splat import GaussianRasterizationSettings, GaussianRasterizer
+from ds_splat_amd import _native, inria_compat
+from ds_splat_amd.synthetic import make_scene
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+
+
+def render_both(sc, planar=False, precomputed=False):
+    """(image, radii) without and with gradients to take"""
+    t = {k: (v.to(DEV) if isinstance(v, torch.Tensor) else v) for k, v in sc.items()}
+    fields = dict(image_height=sc["height"], image_width=sc["width"], tanfovx=sc["tanfovx"], tanfovy=sc["tanfovy"],
+                  bg=torch.tensor([0.2, 0.5, 0.8], device=DEV), scale_modifier=1.0, viewmatrix=t["viewmatrix"],
+                  projmatrix=t["projmatrix"], sh_degree=sc["sh_degree"], campos=t["campos"], prefiltered=False, debug=False)
+    means2d, colors, cov = torch.zeros_like(t["means_3d"]), None, None
+    if precomputed:
+        colors = t["shs"][:, 0].contiguous().abs()
+        s2 = t["scales"][:, :1] ** 2
+        cov = torch.cat([s2, 0.1 * s2, 0 * s2, s2, 0 * s2, 0.5 * s2], 1).contiguous()
+    shs, scales, rots = (None, None, None) if precomputed else (t["shs"], t["scales"], t["rotations"])
+    got = []
+    for grad in (False, True):
+        means = t["means_3d"].clone().requires_grad_(grad)
+        if planar:
+            r = inria_compat.GaussianRasterizer(inria_compat.GaussianRasterizationSettings(**fields))
+            out = r(means3D=means, means2D=means2d, opacities=t["opacities"], shs=shs, colors_precomp=colors, scales=scales,
+                    rotations=rots, cov3D_precomp=cov)
+        else:
+            r = GaussianRasterizer(GaussianRasterizationSettings(max_sh_degree=3, **fields))
+            out = r(means, means2d, shs, colors, t["opacities"], scales, rots, cov)
+        got.append(tuple(x.detach() for x in out))
+    return got
+
+
+def check(sc, in_parts=False, **options):
+    (image, radii), (want, want_radii) = render_both(sc, **options)
+    assert torch.equal(radii, want_radii)
+    if in_parts:
+        # (a colour is a sum of at most 10200 terms in four parts whose members differ: as many roundings of 2^-24 of at
+        # most the whole sum, of either sign: sqrt(10200) 2^-24 = 6e-6 of the largest colour)
+        assert not torch.isnan(image).any()
+        assert float((image - want).abs().max()) <= 6e-6 * max(1.0, float(want.abs().max()))
+    else:
+        assert torch.equal(image, want)
+    return image
+
+
+def taken(sc):
+    return _native.load().dsx_render_bytes(sc["n"], sc["width"], sc["height"], 0) > 0
+
+
+@pytest.mark.parametrize("n,W,H,applies", [
+    (1, 16, 16, True),             # (the last Gaussian emits nothing)
+    (2, 1, 1, True),
+    (300, 40, 40, True),
+    (5000, 97, 50, True),          # tiles cut off at both edges
+    (16384, 256, 256, True),       # as many tiles as there are compute units
+    (16384, 256, 257, False),
+    (34600, 256, 256, True),
+    (34601, 256, 256, False),
+    (9100, 16, 16, True),
+    (9101, 16, 16, False),
+])
+def test_image_of_tiles_that_find_their_entries(n, W, H, applies):
+    sc = make_scene("cfg0", n=n, width=W, height=H, sh_degree=1, seed=n)
+    assert taken(sc) == applies
+    for options in ({}, {"planar": True}, {"precomputed": True}):
+        check(sc, in_parts=n > 4096 and W * H <= 256, **options)
+
+
+@pytest.mark.parametrize("depths", ["spread", "equal", "layers", "nearly_equal", "two"])
+@pytest.mark.parametrize("n,W,H", [(4096, 16, 16), (4097, 16, 16), (9100, 16, 16), (10200, 64, 48)])
+def test_windows_of_a_tile_with_many_entries(n, W, H, depths):
+    """Faint Gaussians that cover every tile: up to 4096 entries are one window, more are several; depths that are equal or nearly so
+    are told apart by their last bits or by the index, and sorted by comparisons where a bin holds many."""
+    sc = make_scene("cfg0", n=n, width=W, height=H, sh_degree=0, seed=n)
+    g = torch.Generator().manual_seed(n)
+    u = torch.rand(n, generator=g)
+    sc["means_3d"][:, :2] *= 0.05
+    sc["means_3d"][:, 2] = {"spread": 2.0 + 8.0 * u, "equal": 4.0 + 0.0 * u, "layers": 2.0 + (8.0 * u).floor(),
+                            "nearly_equal": 4.0 + 1e-5 * u, "two": torch.where(u < 0.5, 2.0, 9.0)}[depths]
+    sc["scales"] = torch.full((n, 3), 1.0) * (1.0 + torch.rand(n, 1, generator=g))
+    sc["opacities"] = 0.004 + 0.004 * torch.rand(n, 1, generator=g)
+    assert taken(sc)
+    image = check(sc, in_parts=n > 4096)
+    assert float(image.abs().max()) > 0.1
+
+
+@pytest.mark.parametrize("share", [0.0, 0.5, 1.0])
+@pytest.mark.parametrize("n,W,H", [(200, 70, 50), (9000, 70, 50), (3000, 16, 16)])
+def test_entries_behind_the_camera_and_the_highest_tile(n, W, H, share):
+    """The highest occupied tile's entries are blended by the image's last tile, and where no tile is occupied that one blends those
+    of negative depth, once for every tile that they touch (the reference's last run of keys, which nothing ends)."""
+    sc = make_scene("cfg0", n=n, width=W, height=H, sh_degree=0, seed=n)
+    sc["projmatrix"][:, 2] = torch.tensor([0.0, 0.0, 0.0, 0.5])
+    sc["projmatrix"][:, 3] = torch.tensor([0.0, 0.0, 0.0, 1.0])
+    sc["means_3d"][:, :2] = 0.2 * sc["means_3d"][:, :2] - 0.35          # (the upper left of the image: its last tiles are empty)
+    behind = torch.arange(n) < int(share * n)
+    sc["means_3d"][behind] *= -1.0
+    assert taken(sc)
+    check(sc, in_parts=n > 4096)
