@@ -77,6 +77,11 @@ def algorithmic_work(kernel, n, k, pixels, lists, coeffs, counters, marked, carr
         first, later = record * n + 4 * (n - emitting) + record * emitting, 2 * record * emitting
         return "hbm", {"onesweep32_kernel<sort, first>": first, "onesweep32_kernel<sort, later>": later}.get(
             kernel, (first + 2 * later) / 3), "B"
+    if kernel == "depth_scatter_kernel":
+        # key and the emitting ones' rectangle in; a record of 16 bytes out, of the others the ids only
+        return "hbm", 4 * n + 8 * emitting + 16 * emitting + 4 * (n - emitting), "B"
+    if kernel == "order_buckets_kernel":
+        return "hbm", (16 + 12) * emitting, "B"
     if kernel == "ordered_offsets_kernel":
         return "hbm", 8 * emitting, "B"
     if kernel == "emit_ordered_kernel":

@@ -172,6 +172,7 @@ def algorithmic_bytes(bench):
     out = {}
     for k in ("project_fwd_kernel", "gaussian_bwd_kernel", "hist32_kernel", "depth_hist_kernel", "onesweep32_kernel<sort>",
               "onesweep32_kernel<sort, first>", "onesweep32_kernel<sort, later>", "ordered_offsets_kernel",
+              "depth_scatter_kernel", "order_buckets_kernel",
               "emit_ordered_kernel", "onesweep32_kernel<tile partition>"):
         bound, work, _ = bench_module.algorithmic_work(k, n, cfg["num_keys"], w * h, cfg["lists"], (deg + 1) ** 2, None,
                                                        cfg.get("gaussians_with_gradient", 0),

@@ -527,7 +527,7 @@ static int check_pair_counts(int64_t list_pairs, int64_t tile_pairs)
 // its own when the next one is waiting: every call has a ticket, which the words carry, and the next of several slots.
 namespace
 {
-constexpr unsigned kCountSlots = 16, kSlotWords = 4;
+constexpr unsigned kCountSlots = 16, kSlotWords = 8;
 struct PinnedCounts
 {
     int64_t* words = nullptr;

@@ -293,6 +293,7 @@ Sort32Workspace sort32_workspace(int64_t count, int key_bits, int tile_keys);
 struct OrderLayout
 {
     size_t depth_keys; // uint32[n]  depth bits (written by the projection)
+    size_t records;    // uint4[n] where the order is made by buckets: (key, index, rectangle), in the memory of the next three
     size_t keys_alt;   // uint32[n]
     size_t ids_a;      // uint32[n]  the depth order ends here
     size_t ids_b;      // uint32[n]
@@ -328,8 +329,8 @@ struct ListsWorkspace
 ListsWorkspace lists_workspace(int64_t k, int num_tiles, bool binned);
 
 // launchers (each returns a dsx_status)
-// Four words of pinned host memory that receive a call's pair counts, the range of its depth keys and how many of them emit (null:
-// none), each marked with the call's ticket.
+// Five words of pinned host memory that receive a call's pair counts, the range of its depth keys, how many of them emit and whether
+// buckets ordered them (null: none), each marked with the call's ticket.
 struct HostCounts
 {
     unsigned long long* words = nullptr;

@@ -761,30 +761,99 @@ __device__ __forceinline__ void store_to_host(const HostCounts& to, int word, un
                        __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// A thread's keys of one step through all of them, sixteen bytes at a time (the buffer is padded to whole lines)
+constexpr int kBatchLoads = 4;
+constexpr int kBatchKeys = 4 * kBatchLoads * kHist32Threads;
+struct KeyBatch
+{
+    uint4 k[kBatchLoads];
+};
+__device__ __forceinline__ KeyBatch load_keys(const uint32_t* keys, int i0, int n)
+{
+    KeyBatch batch;
+#pragma unroll
+    for(int b = 0; b < kBatchLoads; ++b)
+    {
+        const int i = i0 + 4 * (b * kHist32Threads + (int)threadIdx.x);
+        uint4 k = make_uint4(kNoPairsKey, kNoPairsKey, kNoPairsKey, kNoPairsKey);
+        if(i < n)
+            k = *reinterpret_cast<const uint4*>(keys + i);
+        if(i0 + kBatchKeys > n) // (uniform: the words behind the last key hold anything)
+        {
+            k.y = i + 1 < n ? k.y : kNoPairsKey;
+            k.z = i + 2 < n ? k.z : kNoPairsKey;
+            k.w = i + 3 < n ? k.w : kNoPairsKey;
+        }
+        batch.k[b] = k;
+    }
+    return batch;
+}
+
+// What a thread of `kThreads` finds in its share of the blocks' key ranges: the extremes, and how many keys emit.  Eight loads in flight: one after the other they are most of a short kernel's time.
+struct KeySpan
+{
+    uint32_t near16 = 0, far16 = 0, emitting = 0;
+};
+template <int kThreads>
+__device__ __forceinline__ KeySpan key_span(const uint2* __restrict__ ranges, int blocks)
+{
+    KeySpan s;
+    for(int b0 = threadIdx.x; b0 < blocks; b0 += 8 * kThreads)
+    {
+        uint2 r[8];
+#pragma unroll
+        for(int u = 0; u < 8; ++u)
+            r[u] = b0 + u * kThreads < blocks ? ranges[b0 + u * kThreads] : make_uint2(0u, 0u);
+#pragma unroll
+        for(int u = 0; u < 8; ++u)
+        {
+            s.near16 = max(s.near16, r[u].x & 0xffffu);
+            s.far16 = max(s.far16, r[u].y);
+            s.emitting += r[u].x >> 16;
+        }
+    }
+    return s;
+}
+
+// Bins of equal width over a known range of depths, where that is narrow and more than a thin layer (which would crowd a few buckets);
+// the bin of a distance from its first key
+__host__ __device__ constexpr bool depth_bins(const DepthRange& range)
+{
+    return range.narrow && range.behind >= 16u << 16; // (an eighth of an octave)
+}
+__device__ __forceinline__ uint32_t depth_bin_scale(const DepthRange& range, int bin_bits)
+{
+    return (1u << (bin_bits + 16)) / (range.behind >> 16); // (2^bin_bits bins, 2^32 times, over the distances)
+}
+__device__ __forceinline__ uint32_t depth_bin(uint32_t distance, uint32_t scale)
+{
+    return __umulhi(distance, scale);
+}
+
 // The histograms of a depth sort whose range only the device knows yet: every workgroup finds it from the projection's
-// blocks, the first one tells the host, and the digits are those of depth_range().
+// blocks, the first one tells the host, and the digits are those of depth_range(); with bin_bits, where the range is narrow, one
+// histogram of so many bins of the range, and what depth_scatter_kernel wants to know of the blocks, in `span`: the range's ends (the
+// nearest one's complement), the emitting keys, a spare word, and how many of them lie in front of each of kSpanChunks chunks of blocks.
+// (kBinsWorkgroups: that count bins; each adds them to memory, which takes some 45 additions a clock.  us at 3 M, beside the counting of the
+// tiles: 366 43, 128 17, 64 22)
+constexpr int kBinsWorkgroups = 128;
+constexpr int kSpanWords = 4, kSpanChunks = kHist32Threads;
+__host__ __device__ constexpr int span_chunk(int blocks) { return (blocks + kSpanChunks - 1) / kSpanChunks; }
 __global__ __launch_bounds__(kHist32Threads) void depth_hist_kernel(const uint32_t* __restrict__ keys, int64_t count,
                                                                     const uint2* __restrict__ ranges, int64_t blocks,
-                                                                    uint32_t* __restrict__ global_hist,
-                                                                    const HostCounts to_host)
+                                                                    uint32_t* __restrict__ digit_hist,
+                                                                    uint32_t* __restrict__ bin_hist, int bin_bits,
+                                                                    uint32_t* __restrict__ span, const HostCounts to_host)
 {
-    __shared__ uint32_t hist[kSortWordsMost];
+    extern __shared__ __attribute__((aligned(16))) uint32_t hist[]; // of kSortWordsMost words, or the bins if they are more
     __shared__ uint2 s_range[kHist32Threads / DSX_WAVE];
     __shared__ uint32_t s_emitting[kHist32Threads / DSX_WAVE];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for(int j = tid; j < (int)kSortWordsMost; j += kHist32Threads)
+    for(int j = tid; j < max((int)kSortWordsMost, bin_bits ? 1 << bin_bits : 0); j += kHist32Threads)
         hist[j] = 0;
-    uint32_t near16 = 0, far16 = 0, emitting = 0;
-    for(int64_t b = tid; b < blocks; b += kHist32Threads)
-    {
-        const uint2 r = ranges[b];
-        near16 = max(near16, r.x & 0xffffu);
-        far16 = max(far16, r.y);
-        emitting += r.x >> 16;
-    }
-    near16 = wave_incl_max_scan(near16);
-    far16 = wave_incl_max_scan(far16);
-    emitting = wave_sum_u32(emitting);
+    const KeySpan mine = key_span<kHist32Threads>(ranges, (int)blocks);
+    uint32_t near16 = wave_incl_max_scan(mine.near16), far16 = wave_incl_max_scan(mine.far16);
+    const uint32_t emitting = wave_sum_u32(mine.emitting);
     if(lane == 63)
     {
         s_range[wave] = make_uint2(near16, far16);
@@ -807,10 +876,52 @@ __global__ __launch_bounds__(kHist32Threads) void depth_hist_kernel(const uint32
         store_to_host(to_host, 2, lowest | ((unsigned long long)highest << 16));
         store_to_host(to_host, 3, all);
     }
+    if(blockIdx.x == 0 && bin_bits != 0)
+    {
+        const int chunk = span_chunk((int)blocks);
+        uint32_t mine_emit = 0;
+        for(int b = chunk * tid; b < min(chunk * (tid + 1), (int)blocks); ++b)
+            mine_emit += ranges[b].x >> 16;
+        const uint32_t incl = wave_incl_scan_u32(mine_emit);
+        __syncthreads();
+        if(lane == 63)
+            s_emitting[wave] = incl;
+        __syncthreads();
+        uint32_t before = incl - mine_emit;
+#pragma unroll
+        for(int w = 0; w < kHist32Threads / DSX_WAVE; ++w)
+            before += w < wave ? s_emitting[w] : 0u;
+        span[kSpanWords + tid] = before;
+        if(tid == kHist32Threads - 1)
+        {
+            span[0] = 0xffffu - lowest;
+            span[1] = highest;
+            span[2] = before + mine_emit;
+        }
+    }
     const DepthRange range = depth_range(lowest, highest);
     const int bins = range.narrow ? kDepthBins : kBins32;
+    const bool by_bins = bin_bits != 0 && depth_bins(range);
+    const uint32_t scale = by_bins ? depth_bin_scale(range, bin_bits) : 0u;
     uint32_t none = 0; // keys without pairs: counted by their thread, added to their bins at the end (four digits; three leave them out)
-    const int64_t chunk = (int64_t)kHist32Threads * kDepthHistItems, chunks = (count + chunk - 1) / chunk;
+    const int workgroups = by_bins ? min((int)gridDim.x, kBinsWorkgroups) : (int)gridDim.x;
+    if((int)blockIdx.x >= workgroups)
+        return;
+    if(by_bins)
+        for(int64_t i0 = (int64_t)blockIdx.x * kBatchKeys; i0 < count; i0 += (int64_t)workgroups * kBatchKeys)
+        {
+            const KeyBatch batch = load_keys(keys, (int)i0, (int)count);
+#pragma unroll
+            for(int b = 0; b < kBatchLoads; ++b)
+            {
+                const uint32_t four[4] = {batch.k[b].x, batch.k[b].y, batch.k[b].z, batch.k[b].w};
+#pragma unroll
+                for(int u = 0; u < 4; ++u)
+                    if(four[u] != kNoPairsKey)
+                        atomicAdd(&hist[depth_bin(four[u] - range.first, scale)], 1u);
+            }
+        }
+    const int64_t chunk = (int64_t)kHist32Threads * kDepthHistItems, chunks = by_bins ? 0 : (count + chunk - 1) / chunk;
     for(int64_t c = blockIdx.x; c < chunks; c += gridDim.x)
     {
         uint32_t key[kDepthHistItems];
@@ -845,7 +956,8 @@ __global__ __launch_bounds__(kHist32Threads) void depth_hist_kernel(const uint32
             if(p < range.digits.passes)
                 atomicAdd(&hist[p * bins + ((range.behind >> range.digits.shift[p]) & range.digits.mask[p])], none);
     __syncthreads();
-    for(int j = tid; j < range.digits.passes * bins; j += kHist32Threads)
+    uint32_t* const global_hist = by_bins ? bin_hist : digit_hist;
+    for(int j = tid; j < (by_bins ? 1 << bin_bits : range.digits.passes * bins); j += kHist32Threads)
         if(hist[j])
             atomicAdd(&global_hist[j], hist[j]);
 }
@@ -856,6 +968,11 @@ __global__ __launch_bounds__(kHist32Threads) void depth_hist_kernel(const uint32
 
 constexpr int kOffsetsShare = 16 * kProjBlock; // Gaussians of a workgroup of ordered_offsets_kernel
 constexpr int kRanksMax = 131072;              // Gaussians whose depth order is one launch, order_ranks_kernel
+constexpr int kBucketBitsMost = 11, kBucketsMost = 4096; // wanted keys of a bucket of depth_scatter_kernel, how many buckets there may be
+static bool orders_by_buckets(int64_t n)
+{
+    return n > kRanksMax && n <= (int64_t)kBucketsMost << kBucketBitsMost;
+}
 
 OrderLayout order_layout(int64_t n, int image_width, int image_height, int list_bin)
 {
@@ -864,18 +981,20 @@ OrderLayout order_layout(int64_t n, int image_width, int image_height, int list_
     size_t off = 0;
     o.depth_keys = off;
     off = align(off + (size_t)n * 4);
-    o.keys_alt = off;
-    off = align(off + (size_t)n * 4);
     o.ids_a = off;
-    off = align(off + (size_t)n * 4);
-    o.ids_b = off;
     off = align(off + (size_t)n * 4);
     o.rects = off;
     off = align(off + (size_t)n * 8);
     o.rects_sorted = off;
     off = align(off + (size_t)n * 8);
+    o.records = o.keys_alt = off;
+    off = align(off + (size_t)n * 4);
+    o.ids_b = off;
+    off = align(off + (size_t)n * 4);
     o.rects32 = off;
     off = align(off + (size_t)n * 4);
+    if(orders_by_buckets(n))
+        off = std::max(off, align(o.records + (size_t)n * 16));
     o.block_sums = off;
     off = align(off + (size_t)((n + kProjBlock - 1) / kProjBlock + 1) * 4);
     o.key_ranges = off;
@@ -1030,6 +1149,474 @@ __global__ __launch_bounds__(kOffsetsThreads) void ordered_offsets_kernel(uint2*
     }
 }
 
+// ---------------------------------------------------------------------------------------
+// 131073 to 8388608 Gaussians: the depth order by buckets, and the block offsets with it
+// ---------------------------------------------------------------------------------------
+// Two launches behind a histogram of 2^12 to 2^14 bins of the depths' range.  A bucket is the bins that begin in 1024 or 2048
+// consecutive ranks, so its first rank is known, and a workgroup of the first launch needs no other's ranks: it counts its keys by
+// bucket in LDS, asks for that much room in each (one atomic per bucket and workgroup) and writes (key, index, rectangle) there, in any order.
+// The second launch sorts a bucket at a time in LDS (4096 bins of its own range of (key, index), the few in the same bin compared with
+// each other) and writes order and rectangles; the pairs of a bucket were summed with its room, so the block offsets fall out as well.
+// Nobody waits for another workgroup.
+// Where a bin holds more keys than a bucket has room for beyond the wanted 1024 or 2048 (many equal depths) nothing is written, the
+// host is told, and the digit passes run, 10 to 20 us later than without the attempt; where the range has both signs, or is wide or thin,
+// it sees that beforehand.
+// The first launch is bound by latency (ranges and bins 4 us, the table 3, keys and rectangles 4, room 2, the stores 3 to 10: two rounds
+// of workgroups beyond 3 M) and by its scattered stores, whose partial lines are 69 MB instead of 34 for 3 M (2 M of them emitting); the second
+// by its chain of short steps, four workgroups at a time on a compute unit.  us alone: 300 K 11 + 8, 500 K 14 + 9, 1 M 20 + 14, 3 M 38 + 21,
+// 6 M 77 + 34; the digit passes and the offsets were 42, 47, 57, 97 and 182.  A whole forward, 1280x720, of 150 K Gaussians 120 -> 100 us,
+// 250 K 144 -> 117, 600 K 195 -> 173, 1.5 M 263 -> 240, 4 M 422 -> 384; a training step of 3 M at 1920x1080 752 -> 710.  (Tried: buckets of 1024 and
+// workgroups of 8192 keys, whose two records a bucket and workgroup are nearly all partial lines: 65 us at 3 M; no keys in registers but
+// read twice, by twice the workgroups: 46; buckets of 4096, whose sort takes 27 instead of 21.)
+constexpr int kScatterThreads = 1024;
+constexpr int kScatterWaves = kScatterThreads / DSX_WAVE;
+constexpr int kBucketThreads = 512;
+constexpr int kBucketWaves = kBucketThreads / DSX_WAVE;
+constexpr int kBucketItems = 8;
+constexpr int kBucketKeys = 3840; // that a bucket can have
+constexpr int kBucketBinBits = 12;
+constexpr uint32_t kBucketGroupMost = 64; // keys in one bin that are compared with each other one by one
+constexpr uint64_t kBucketsDone = 1, kBucketsTooFull = 2;
+constexpr int kPairsAt = 24; // bits of a rank
+static_assert(((int64_t)kBucketsMost << kBucketBitsMost) <= 1 << kPairsAt, "ranks");
+
+struct BucketsJob
+{
+    const uint32_t* keys; // by Gaussian
+    const uint2* rects;
+    const uint2* key_ranges; // of 256 consecutive Gaussians (see OrderLayout)
+    const uint32_t* bins;
+    uint32_t* span;              // (see depth_hist_kernel)
+    unsigned long long* cursors; // of each bucket: keys, and their pairs << kPairsAt (zero at first)
+    uint2* starts;               // of each bucket and behind the last: its first rank, the pairs before it
+    uint32_t* done;              // workgroups that have asked for their room; whether there are starts (both zero at first)
+    uint4* records;
+    uint32_t* order; // by depth
+    uint2* rects_sorted;
+    uint32_t* block_sums;
+    int n, shift, buckets, bucket_bits;
+    HostCounts to_host;
+};
+
+// kRuns: of 256 Gaussians, of a wavefront, whose keys and rectangles stay in its registers
+template <int kRuns, int kBinBits>
+__global__ __launch_bounds__(kScatterThreads) void depth_scatter_kernel(const BucketsJob J)
+{
+    constexpr int kBins = 1 << kBinBits, kMine = kBins / kScatterThreads, kEach = kBucketsMost / kScatterThreads;
+    constexpr int kParts = kProjBlock / DSX_WAVE;
+    extern __shared__ __attribute__((aligned(16))) unsigned long long s_taken[]; // this workgroup's keys of the bucket, their pairs << kPairsAt
+    uint32_t* const s_room = reinterpret_cast<uint32_t*>(s_taken + kBucketsMost); // the bucket's first rank, then where its next key goes
+    uint16_t* const s_bucket = reinterpret_cast<uint16_t*>(s_room + kBucketsMost); // of each bin
+    __shared__ uint32_t s_emit[kRuns * kScatterWaves];   // of each of this workgroup's runs: emitting Gaussians before it
+    __shared__ __attribute__((aligned(16))) uint32_t s_tot[kScatterWaves];
+    __shared__ uint2 s_part[kScatterWaves];
+    __shared__ unsigned long long s_all[kScatterWaves];
+    __shared__ uint32_t s_flag, s_front;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int n = J.n, blocks = (n + kProjBlock - 1) / kProjBlock;
+    const int run0 = (int)blockIdx.x * (kRuns * kScatterWaves);
+    auto index_of = [&](int q, int u) { return (run0 + q * kScatterWaves + wave) * kProjBlock + u * DSX_WAVE + lane; };
+
+    uint4 bin4[kMine / 4];
+#pragma unroll
+    for(int q = 0; q < kMine / 4; ++q)
+        bin4[q] = reinterpret_cast<const uint4*>(J.bins)[(kMine / 4) * tid + q];
+    uint32_t key[kRuns][kParts];
+#pragma unroll
+    for(int q = 0; q < kRuns; ++q)
+#pragma unroll
+        for(int u = 0; u < kParts; ++u)
+            key[q][u] = index_of(q, u) < n ? J.keys[index_of(q, u)] : kNoPairsKey;
+    const int chunk = span_chunk(blocks), front = run0 / chunk;
+    const uint32_t emitting = J.span[2], front_emits = J.span[kSpanWords + front];
+    const DepthRange range = depth_range(0xffffu - J.span[0], J.span[1]);
+    // (fewer runs than a wavefront has lanes lie between a chunk's first one and this workgroup's)
+    const uint32_t between = wave == 0 && front * chunk + lane < run0 ? J.key_ranges[front * chunk + lane].x >> 16 : 0u;
+    const uint32_t run_emits = tid < kRuns * kScatterWaves && run0 + tid < blocks ? J.key_ranges[run0 + tid].x >> 16 : 0u;
+    static_assert(((int64_t)kBucketsMost << kBucketBitsMost) / kProjBlock / kSpanChunks <= DSX_WAVE, "a lane for each");
+    if(!depth_bins(range)) // (there are none)
+        return;
+    uint32_t sum = 0, most = 0;
+#pragma unroll
+    for(int q = 0; q < kMine / 4; ++q)
+    {
+        sum += bin4[q].x + bin4[q].y + bin4[q].z + bin4[q].w;
+        most = max(max(max(most, bin4[q].x), max(bin4[q].y, bin4[q].z)), bin4[q].w);
+    }
+    const uint32_t incl = wave_incl_scan_u32(sum), runs_incl = wave_incl_scan_u32(run_emits), between_all = wave_sum_u32(between);
+    if(lane == 63)
+    {
+        s_tot[wave] = incl;
+        s_part[wave].x = runs_incl;
+    }
+    if(tid == 0)
+    {
+        s_flag = 0;
+        s_front = front_emits + between_all;
+    }
+#pragma unroll
+    for(int q = 0; q < kEach; ++q)
+    {
+        s_room[q * kScatterThreads + tid] = 0xffffffffu;
+        s_taken[q * kScatterThreads + tid] = 0;
+    }
+    __syncthreads();
+    if(tid < kRuns * kScatterWaves)
+        s_emit[tid] = s_front + (wave ? s_part[0].x : 0u) + runs_incl - run_emits;
+    static_assert(kRuns * kScatterWaves <= 2 * DSX_WAVE, "two wavefronts' runs");
+    uint32_t at = sum_of_waves_before<kScatterWaves>(s_tot, wave) + incl - sum, last_bucket = 0xffffffffu;
+#pragma unroll
+    for(int q = 0; q < kMine / 4; ++q)
+    {
+        const uint32_t count[4] = {bin4[q].x, bin4[q].y, bin4[q].z, bin4[q].w};
+        uint32_t bucket[4];
+#pragma unroll
+        for(int u = 0; u < 4; ++u)
+        {
+            bucket[u] = min(at >> J.bucket_bits, (uint32_t)J.buckets - 1u);
+            if(count[u] && bucket[u] != last_bucket)
+            {
+                atomicMin(&s_room[bucket[u]], at);
+                last_bucket = bucket[u];
+            }
+            at += count[u];
+        }
+        *reinterpret_cast<uint2*>(s_bucket + kMine * tid + 4 * q) = make_uint2(bucket[0] | bucket[1] << 16, bucket[2] | bucket[3] << 16);
+    }
+    if(most > kBucketKeys - (1u << J.bucket_bits))
+        s_flag = 1;
+    uint2 rect[kRuns][kParts];
+#pragma unroll
+    for(int q = 0; q < kRuns; ++q)
+#pragma unroll
+        for(int u = 0; u < kParts; ++u)
+            rect[q][u] = key[q][u] != kNoPairsKey ? J.rects[index_of(q, u)] : make_uint2(0u, 0u);
+    __syncthreads();
+    const bool too_full = __builtin_amdgcn_readfirstlane((int)s_flag) != 0;
+    if(blockIdx.x == 0 && tid == 0)
+        store_to_host(J.to_host, 4, too_full ? kBucketsTooFull : kBucketsDone);
+    if(too_full) // (every workgroup finds so)
+        return;
+    const uint32_t scale = depth_bin_scale(range, kBinBits);
+    auto bucket_of = [&](uint32_t k) { return s_bucket[min(depth_bin(k - range.first, scale), (uint32_t)(kBins - 1))]; };
+#pragma unroll
+    for(int q = 0; q < kRuns; ++q)
+#pragma unroll
+        for(int u = 0; u < kParts; ++u)
+            if(key[q][u] != kNoPairsKey) // (what a wide rectangle counts is cut off where the callers refuse the sum)
+                atomicAdd(&s_taken[bucket_of(key[q][u])],
+                          (unsigned long long)min(list_count(rect[q][u], J.shift), 1u << 30) << kPairsAt | 1ull);
+    __syncthreads();
+    uint32_t back[kEach];
+#pragma unroll
+    for(int q = 0; q < kEach; ++q)
+    {
+        const int b = q * kScatterThreads + tid;
+        const unsigned long long mine = s_taken[b];
+        back[q] = 0;
+        if(mine)
+            back[q] = (uint32_t)atomicAdd(&J.cursors[b], mine) & ((1u << kPairsAt) - 1u);
+    }
+#pragma unroll
+    for(int q = 0; q < kEach; ++q) // (an addition has been performed when its result is back)
+        s_room[q * kScatterThreads + tid] += back[q];
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if(tid == 0)
+        s_flag = atomicAdd(J.done, 1u) == gridDim.x - 1;
+    const uint32_t kept = (emitting + kProjBlock - 1) / kProjBlock * kProjBlock; // what the emission looks at
+#pragma unroll
+    for(int q = 0; q < kRuns; ++q)
+    {
+        // (those that emit nothing: behind the others, by index)
+        uint32_t behind = emitting + (uint32_t)((run0 + q * kScatterWaves + wave) * kProjBlock) - s_emit[q * kScatterWaves + wave];
+#pragma unroll
+        for(int u = 0; u < kParts; ++u)
+        {
+            const uint32_t i = (uint32_t)index_of(q, u);
+            const uint64_t none = __builtin_amdgcn_ballot_w64(key[q][u] == kNoPairsKey);
+            if(key[q][u] != kNoPairsKey)
+            {
+                const uint32_t p = atomicAdd(&s_room[bucket_of(key[q][u])], 1u);
+                J.records[min(p, (uint32_t)n - 1u)] = make_uint4(key[q][u], i, rect[q][u].x, rect[q][u].y);
+            }
+            else if(i < (uint32_t)n)
+            {
+                const uint32_t p = min(behind + bits_below(none), (uint32_t)n - 1u);
+                J.order[p] = i;
+                if(p < kept)
+                    J.rects_sorted[p] = make_uint2(0u, 0u);
+            }
+            behind += (uint32_t)__popcll(none);
+        }
+    }
+    __syncthreads();
+    // the last workgroup sums the buckets up
+    if(!s_flag)
+        return;
+    uint32_t keys[kEach], own_keys = 0, own_pairs = 0;
+    unsigned long long pairs[kEach], all = 0;
+#pragma unroll
+    for(int q = 0; q < kEach; ++q)
+    {
+        const unsigned long long taken = __hip_atomic_load(J.cursors + kEach * tid + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        keys[q] = (uint32_t)taken & ((1u << kPairsAt) - 1u);
+        pairs[q] = taken >> kPairsAt;
+    }
+#pragma unroll
+    for(int q = 0; q < kEach; ++q)
+    {
+        own_keys += keys[q];
+        own_pairs += (uint32_t)pairs[q];
+        all += pairs[q]; // (64 bits: what does not fit 32 is refused by the callers, but must not look like less)
+    }
+    const uint32_t keys_incl = wave_incl_scan_u32(own_keys), pairs_incl = wave_incl_scan_u32(own_pairs);
+#pragma unroll
+    for(int o = 32; o > 0; o >>= 1)
+        all += __shfl_xor(all, o, DSX_WAVE);
+    if(lane == 63)
+    {
+        s_part[wave] = make_uint2(keys_incl, pairs_incl);
+        s_all[wave] = all;
+    }
+    __syncthreads();
+    uint32_t rank = keys_incl - own_keys, before = pairs_incl - own_pairs;
+    all = 0;
+#pragma unroll
+    for(int w = 0; w < kScatterWaves; ++w)
+    {
+        rank += w < wave ? s_part[w].x : 0u;
+        before += w < wave ? s_part[w].y : 0u;
+        all += s_all[w];
+    }
+#pragma unroll
+    for(int q = 0; q < kEach; ++q)
+    {
+        J.starts[kEach * tid + q] = make_uint2(rank, before);
+        rank += keys[q];
+        before += (uint32_t)pairs[q];
+    }
+    const uint32_t total = all > 0xffffffffull ? 0xffffffffu : (uint32_t)all;
+    for(int run = (int)(kept / kProjBlock) + tid; run <= blocks; run += kScatterThreads)
+        J.block_sums[run] = total;
+    if(tid == 0)
+    {
+        J.starts[kBucketsMost] = make_uint2(emitting, total);
+        J.done[1] = 1u;
+    }
+}
+
+// (39 KB of LDS and 64 registers: four workgroups to a compute unit)
+__global__ __launch_bounds__(kBucketThreads) __attribute__((amdgpu_waves_per_eu(8))) void order_buckets_kernel(const BucketsJob J)
+{
+    constexpr int kBins = 1 << kBucketBinBits;
+    __shared__ __attribute__((aligned(16))) uint64_t s_binned[kBucketKeys];
+    __shared__ __attribute__((aligned(16))) uint16_t s_hist[kBins]; // two in a word
+    __shared__ __attribute__((aligned(16))) uint32_t s_tot[kBucketWaves];
+    __shared__ uint2 s_ends[kBucketWaves];
+    __shared__ uint32_t s_sums[kBucketKeys / kProjBlock + 2];
+    __shared__ uint32_t s_alike;
+    uint32_t* const s_pairs = reinterpret_cast<uint32_t*>(s_hist);
+    static_assert(kBins == 8 * kBucketThreads && kBucketKeys <= kBucketItems * kBucketThreads && kBucketKeys <= kBins, "what the threads take");
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint2 start = J.starts[blockIdx.x];
+    const int count = J.done[1] ? (int)min(J.starts[blockIdx.x + 1].x - start.x, (uint32_t)kBucketKeys) : 0;
+    if(count == 0) // (uniform)
+        return;
+    uint64_t mine[kBucketItems]; // key, index
+    uint2 rect[kBucketItems];
+    uint32_t nearest = 0, farthest = 0; // (the former's complement)
+#pragma unroll
+    for(int it = 0; it < kBucketItems; ++it)
+    {
+        const int at = it * kBucketThreads + tid;
+        mine[it] = ~0ull;
+        rect[it] = make_uint2(0u, 0u);
+        if(at < count)
+        {
+            const uint4 record = J.records[start.x + at];
+            mine[it] = (uint64_t)record.x << 32 | record.y;
+            rect[it] = make_uint2(record.z, record.w);
+            nearest = max(nearest, ~record.x);
+            farthest = max(farthest, record.x);
+        }
+    }
+    nearest = wave_incl_max_scan(nearest);
+    farthest = wave_incl_max_scan(farthest);
+    if(lane == 63)
+        s_ends[wave] = make_uint2(nearest, farthest);
+    reinterpret_cast<uint4*>(s_hist)[tid] = make_uint4(0u, 0u, 0u, 0u);
+    if(tid < kBucketKeys / kProjBlock + 2)
+        s_sums[tid] = 0;
+    if(tid == 0)
+        s_alike = 0;
+    __syncthreads();
+    nearest = farthest = 0;
+#pragma unroll
+    for(int w = 0; w < kBucketWaves; ++w)
+    {
+        nearest = max(nearest, s_ends[w].x);
+        farthest = max(farthest, s_ends[w].y);
+    }
+    nearest = ~(uint32_t)__builtin_amdgcn_readfirstlane((int)nearest);
+    farthest = (uint32_t)__builtin_amdgcn_readfirstlane((int)farthest);
+    const uint64_t from = (uint64_t)nearest << 32;
+    const int to_bin = (farthest == nearest ? 32 : 64 - __builtin_clz(farthest - nearest)) - kBucketBinBits;
+    uint32_t place[kBucketItems]; // bin << 16 | how many came before; then the bin's first place, the one behind its last << 16
+    uint32_t most = 0;
+#pragma unroll
+    for(int it = 0; it < kBucketItems; ++it)
+    {
+        place[it] = 0;
+        if(it * kBucketThreads + tid < count)
+        {
+            const uint32_t bin = (uint32_t)((mine[it] - from) >> to_bin), half = 16 * (bin & 1);
+            const uint32_t nth = atomicAdd(&s_pairs[bin >> 1], 1u << half) >> half & 0xffffu;
+            place[it] = bin << 16 | nth;
+            most = max(most, nth);
+        }
+    }
+    if(__builtin_amdgcn_ballot_w64(most >= kBucketGroupMost) != 0 && lane == 0)
+        s_alike = 1;
+    __syncthreads();
+    // exclusive sums of the bins
+    {
+        uint4* const eight = reinterpret_cast<uint4*>(s_hist) + tid;
+        const uint4 c = *eight;
+        const uint32_t both = c.x + c.y + c.z + c.w, sum = (both & 0xffffu) + (both >> 16), incl = wave_incl_scan_u32(sum);
+        if(lane == 63)
+            s_tot[wave] = incl;
+        __syncthreads();
+        uint32_t at = sum_of_waves_before<kBucketWaves>(s_tot, wave) + incl - sum;
+        auto two = [&](uint32_t w) {
+            const uint32_t first = at, second = at + (w & 0xffffu);
+            at = second + (w >> 16);
+            return first | second << 16;
+        };
+        const uint32_t x = two(c.x), y = two(c.y), z = two(c.z), w = two(c.w);
+        *eight = make_uint4(x, y, z, w);
+    }
+    __syncthreads();
+    const bool alike = __builtin_amdgcn_readfirstlane((int)s_alike) != 0;
+    uint32_t rank[kBucketItems];
+    if(!alike)
+    {
+        uint32_t longest = 0;
+#pragma unroll
+        for(int it = 0; it < kBucketItems; ++it)
+        {
+            rank[it] = 0;
+            if(it * kBucketThreads + tid < count)
+            {
+                const uint32_t bin = place[it] >> 16, first = s_hist[bin];
+                const uint32_t end = bin + 1 < (uint32_t)kBins ? s_hist[bin + 1] : (uint32_t)count;
+                s_binned[first + (place[it] & 0xffffu)] = mine[it];
+                place[it] = first | end << 16;
+                rank[it] = first;
+                longest = max(longest, end - first);
+            }
+        }
+        __syncthreads();
+        for(uint32_t j = 0; __builtin_amdgcn_ballot_w64(j < longest) != 0; ++j)
+#pragma unroll
+            for(int it = 0; it < kBucketItems; ++it)
+                if((place[it] & 0xffffu) + j < place[it] >> 16)
+                    rank[it] += s_binned[(place[it] & 0xffffu) + j] < mine[it] ? 1u : 0u;
+    }
+    else
+    {
+        // many depths alike: a bitonic sort, and everybody looks for its own
+        // (the steps are those of the next power of two; what would lie behind the last key is larger than all)
+        int size = kBucketThreads;
+        while(size < count)
+            size *= 2;
+#pragma unroll
+        for(int it = 0; it < kBucketItems; ++it)
+            if(it * kBucketThreads + tid < count)
+                s_binned[it * kBucketThreads + tid] = mine[it];
+        for(int k = 2; k <= size; k *= 2)
+            for(int j = k / 2; j > 0; j /= 2)
+            {
+                __syncthreads();
+                for(int e = tid; e < size / 2; e += kBucketThreads)
+                {
+                    // (the first step of each size mirrors its second half: the smaller always comes first)
+                    const int i = 2 * e - (e & (j - 1)), l = j == k / 2 ? i + (k - 1 - 2 * (i & (k - 1))) : i + j;
+                    if(l >= count)
+                        continue;
+                    const uint64_t u = s_binned[i], v = s_binned[l];
+                    if(u > v)
+                    {
+                        s_binned[i] = v;
+                        s_binned[l] = u;
+                    }
+                }
+            }
+        __syncthreads();
+#pragma unroll
+        for(int it = 0; it < kBucketItems; ++it)
+        {
+            uint32_t r = 0;
+            if(it * kBucketThreads + tid < count)
+                for(int step = size / 2; step > 0; step /= 2)
+                    if(r + step <= (uint32_t)count && s_binned[r + step - 1] < mine[it])
+                        r += step;
+            rank[it] = r;
+        }
+    }
+    __syncthreads();
+    // the rectangles in order, the runs' sums, and the order
+    uint2* const s_rects = reinterpret_cast<uint2*>(s_binned);
+    uint32_t* const s_ids = reinterpret_cast<uint32_t*>(s_binned);
+#pragma unroll
+    for(int it = 0; it < kBucketItems; ++it)
+        if(it * kBucketThreads + tid < count)
+            s_rects[rank[it]] = rect[it];
+    __syncthreads();
+    const uint32_t run0 = start.x / kProjBlock;
+#pragma unroll
+    for(int it = 0; it < kBucketItems; ++it)
+    {
+        if(it * kBucketThreads >= count) // (uniform)
+            break;
+        const int at = it * kBucketThreads + tid;
+        const uint32_t p = start.x + (uint32_t)at;
+        uint32_t pairs = 0;
+        if(at < count)
+        {
+            const uint2 r = s_rects[at];
+            J.rects_sorted[p] = r;
+            pairs = list_count(r, J.shift);
+        }
+        const uint32_t run = p / kProjBlock - run0, other = (uint32_t)__builtin_amdgcn_readlane((int)run, 63);
+        if(__builtin_amdgcn_readfirstlane(run) == other)
+        {
+            const uint32_t sum = wave_sum_u32(pairs);
+            if(lane == 0 && sum)
+                atomicAdd(&s_sums[run], sum);
+        }
+        else if(pairs)
+            atomicAdd(&s_sums[run], pairs);
+    }
+    __syncthreads();
+#pragma unroll
+    for(int it = 0; it < kBucketItems; ++it)
+        if(it * kBucketThreads + tid < count)
+            s_ids[rank[it]] = (uint32_t)mine[it];
+    __syncthreads();
+    for(int at = tid; at < count; at += kBucketThreads)
+        J.order[start.x + at] = s_ids[at];
+    // (of the runs that begin here)
+    static_assert(kBucketKeys / kProjBlock + 2 <= DSX_WAVE, "a lane for each run");
+    if(wave == 0)
+    {
+        const uint32_t sum = lane < kBucketKeys / kProjBlock + 2 ? s_sums[lane] : 0u, before = start.y + wave_incl_scan_u32(sum) - sum;
+        const uint32_t p = (run0 + (uint32_t)lane) * kProjBlock;
+        if(p >= start.x && p < start.x + (uint32_t)count)
+            J.block_sums[run0 + lane] = before;
+    }
+}
+
 // How many pairs each tile receives, straight from the rectangles (no pair is enumerated):
 // a rectangle [sx, ex) x [sy, ey) adds +1, -1, -1, +1 at its four corners of a
 // (nty + 1) x (ntx + 1) grid, and the two-dimensional prefix sum of that grid is the number of
@@ -1066,9 +1653,18 @@ __global__ __launch_bounds__(kCoverThreads) void tile_cover_kernel(const uint2* 
             s_grid[j] = 0;
         __syncthreads();
     }
-    for(int64_t g = (int64_t)blockIdx.x * kCoverThreads + tid; g < n; g += (int64_t)gridDim.x * kCoverThreads)
+    constexpr int kAhead = 4; // rectangles whose loads are in flight
+    const int64_t stride = (int64_t)gridDim.x * kCoverThreads;
+    for(int64_t g0 = (int64_t)blockIdx.x * kCoverThreads + tid; g0 < n; g0 += kAhead * stride)
     {
-        const uint2 r = rects[g];
+        uint2 ahead[kAhead];
+#pragma unroll
+        for(int u = 0; u < kAhead; ++u)
+            ahead[u] = g0 + u * stride < n ? rects[g0 + u * stride] : make_uint2(0u, 0u);
+#pragma unroll
+        for(int u = 0; u < kAhead; ++u)
+        {
+        const uint2 r = ahead[u];
         const int w = (int)(r.y & 0xffffu), h = (int)((r.y >> 16) & 0x7fffu);
         if(w == 0 || h == 0)
             continue;
@@ -1096,6 +1692,7 @@ __global__ __launch_bounds__(kCoverThreads) void tile_cover_kernel(const uint2* 
             atomicAdd(&bacc[b.by * bpitch + b.bx + b.bw], -1);
             atomicAdd(&bacc[(b.by + b.bh) * bpitch + b.bx], -1);
             atomicAdd(&bacc[(b.by + b.bh) * bpitch + b.bx + b.bw], 1);
+        }
         }
     }
     if(use_lds)
@@ -1330,7 +1927,7 @@ __global__ __launch_bounds__(kCoverThreads) void tile_counts_kernel(const Counts
 // 16 K 11, 50 K 17.5, 100 K 23.5.  Before, a sort of 2048 keys in LDS and a merge up to 24576 Gaussians, the digit passes beyond: a whole
 // forward of 16 K 78 -> 60 us, a training step of 50 K 199 -> 165, of 100 K 229 -> 198, 2 K 40 as it was.
 constexpr int kRanksThreads = 1024;
-static_assert(kRanksThreads == kCoverThreads, "tile_counts is written for this many threads");
+static_assert(kRanksThreads == kCoverThreads && kRanksThreads == kHist32Threads, "tile_counts and load_keys are written for this many threads");
 constexpr int kRanksBinBits = 12;
 constexpr int kRanksBins = 1 << kRanksBinBits;
 constexpr int kShareWanted = 512; // keys of a workgroup
@@ -1363,34 +1960,6 @@ struct RanksJob
 __device__ __forceinline__ int bits_of(uint64_t v)
 {
     return v ? 64 - __builtin_clzll(v) : 0;
-}
-
-// A thread's keys of one step through all of them, sixteen bytes at a time (the buffer is padded to whole lines)
-constexpr int kBatchLoads = 4;
-constexpr int kBatchKeys = 4 * kBatchLoads * kRanksThreads;
-struct KeyBatch
-{
-    uint4 k[kBatchLoads];
-};
-__device__ __forceinline__ KeyBatch load_keys(const uint32_t* keys, int i0, int n)
-{
-    KeyBatch batch;
-#pragma unroll
-    for(int b = 0; b < kBatchLoads; ++b)
-    {
-        const int i = i0 + 4 * (b * kRanksThreads + (int)threadIdx.x);
-        uint4 k = make_uint4(kNoPairsKey, kNoPairsKey, kNoPairsKey, kNoPairsKey);
-        if(i < n)
-            k = *reinterpret_cast<const uint4*>(keys + i);
-        if(i0 + kBatchKeys > n) // (uniform: the words behind the last key hold anything)
-        {
-            k.y = i + 1 < n ? k.y : kNoPairsKey;
-            k.z = i + 2 < n ? k.z : kNoPairsKey;
-            k.w = i + 3 < n ? k.w : kNoPairsKey;
-        }
-        batch.k[b] = k;
-    }
-    return batch;
 }
 
 __device__ __forceinline__ void order_share(const RanksJob& J, const int share, uint32_t* const s_mem)
@@ -1879,10 +2448,96 @@ void depth_order_clear_region(const dsx_camera& cam, int64_t n, void* order, uin
     *count = (int64_t)((w.bytes + (o.ranges - o.cover)) / 4);
 }
 
+// The buckets' launches: their words lie where the passes' look-back statuses would (zero at first); returns the bits of the bins, or 0
+// where these words do not fit.
+static int buckets_job(int64_t n, char* base, const OrderLayout& o, int shift, const HostCounts& to_host, BucketsJob* J)
+{
+    const Sort32Workspace w = sort32_workspace(n, 32, sort32_tile_keys(n));
+    const int bin_bits = n > 1 << 22 ? 14 : (n > 1 << 20 ? 13 : 12);
+    // (a few hundred buckets at least)
+    J->bucket_bits = n > 1 << 19 ? kBucketBitsMost : kBucketBitsMost - 1;
+    J->buckets = (int)((n + (1 << J->bucket_bits) - 1) >> J->bucket_bits);
+    J->n = (int)n;
+    J->shift = shift;
+    J->to_host = to_host;
+    char* at = base + o.sort + w.status;
+    auto take = [&](size_t bytes) {
+        char* const mine = at;
+        at += (bytes + 255) & ~(size_t)255;
+        return mine;
+    };
+    J->bins = reinterpret_cast<const uint32_t*>(take((size_t)4 << bin_bits));
+    J->cursors = reinterpret_cast<unsigned long long*>(take((size_t)kBucketsMost * 8));
+    J->starts = reinterpret_cast<uint2*>(take((size_t)(kBucketsMost + 1) * 8));
+    J->done = reinterpret_cast<uint32_t*>(take(8));
+    J->span = reinterpret_cast<uint32_t*>(take((kSpanWords + kSpanChunks) * 4));
+    if(at > base + o.sort + w.bytes)
+    {
+        *J = {};
+        return 0;
+    }
+    J->keys = reinterpret_cast<const uint32_t*>(base + o.depth_keys);
+    J->rects = reinterpret_cast<const uint2*>(base + o.rects);
+    J->key_ranges = reinterpret_cast<const uint2*>(base + o.key_ranges);
+    J->records = reinterpret_cast<uint4*>(base + o.records);
+    J->order = reinterpret_cast<uint32_t*>(base + o.ids_a);
+    J->rects_sorted = reinterpret_cast<uint2*>(base + o.rects_sorted);
+    J->block_sums = reinterpret_cast<uint32_t*>(base + o.block_sums);
+    if(bin_bits == 14 && hipFuncSetAttribute(reinterpret_cast<const void*>(depth_hist_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             4 << 14) != hipSuccess)
+    {
+        (void)hipGetLastError();
+        *J = {};
+        return 0;
+    }
+    return bin_bits;
+}
+
+static int launch_buckets(const BucketsJob& J, int64_t emitting, hipStream_t stream)
+{
+    int rc = DSX_OK;
+    auto scatter = [&](auto kernel, int runs, int bin_bits) {
+        const int tile = runs * kScatterWaves * kProjBlock;
+        const size_t bytes = (size_t)kBucketsMost * 12 + ((size_t)2 << bin_bits);
+        if(bytes > 65536 - 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                       (int)bytes) != hipSuccess)
+        {
+            (void)hipGetLastError();
+            rc = DSX_ERR_RUNTIME;
+            return;
+        }
+        DSX_TIMED("depth_scatter_kernel", stream);
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((J.n + tile - 1) / tile)), dim3(kScatterThreads), bytes, stream, J);
+    };
+    // (as many Gaussians to a workgroup as leave one for each compute unit)
+    if(J.n <= 1 << 20)
+        scatter(depth_scatter_kernel<1, 12>, 1, 12);
+    else if(J.n <= 2 << 20)
+        scatter(depth_scatter_kernel<2, 13>, 2, 13);
+    else if(J.n <= 3 << 20)
+        scatter(depth_scatter_kernel<3, 13>, 3, 13);
+    else if(J.n <= 4 << 20)
+        scatter(depth_scatter_kernel<4, 13>, 4, 13);
+    else
+        scatter(depth_scatter_kernel<4, 14>, 4, 14);
+    if(rc)
+        return rc;
+    DSX_LAUNCH_CHECK();
+    if(emitting == 0)
+        return DSX_OK;
+    {
+        DSX_TIMED("order_buckets_kernel", stream);
+        hipLaunchKernelGGL(order_buckets_kernel, dim3((unsigned)((emitting + (1 << J.bucket_bits) - 1) >> J.bucket_bits)),
+                           dim3(kBucketThreads), 0, stream, J);
+    }
+    DSX_LAUNCH_CHECK();
+    return DSX_OK;
+}
+
 // The depth sort of a whole forward (cleared workspace): ids in `ids_a`, the rectangles of the first `emitting` of them in
 // `rects_sorted`.
-static int launch_depth_sort(int64_t n, char* base, const OrderLayout& o, int64_t blocks, bool carry,
-                             const HostCounts& to_host, int polls, hipStream_t stream, int64_t* emitting)
+static int launch_depth_sort(int64_t n, char* base, const OrderLayout& o, int64_t blocks, bool carry, bool by_buckets, int list_shift,
+                             const HostCounts& to_host, int polls, hipStream_t stream, int64_t* emitting, bool* offsets_done)
 {
     if(n >= (1ll << 30))
         return DSX_ERR_TOO_LARGE;
@@ -1897,17 +2552,40 @@ static int launch_depth_sort(int64_t n, char* base, const OrderLayout& o, int64_
     char* const ws = base + o.sort;
     const Sort32Workspace w = sort32_workspace(n, 32, sort32_tile_keys(n));
     const int64_t chunks = (n + kHist32Threads * kDepthHistItems - 1) / (kHist32Threads * kDepthHistItems);
-    {
+    // (buckets: only with the waits' own limits, see launch_depth_order)
+    BucketsJob buckets = {};
+    const int bin_bits = polls == kSpinLimit32 && by_buckets ? buckets_job(n, base, o, list_shift, to_host, &buckets) : 0;
+    auto count_keys = [&](uint32_t* bin_hist, int bin_bits) {
+        const size_t bytes = std::max(kSortWordsMost, bin_bits ? (size_t)1 << bin_bits : 0) * 4;
         DSX_TIMED("depth_hist_kernel", stream);
-        hipLaunchKernelGGL(depth_hist_kernel, dim3((unsigned)min((int64_t)DSX_HIST_BLOCKS, chunks)), dim3(kHist32Threads), 0,
-                           stream, (const uint32_t*)keys_a, n, reinterpret_cast<const uint2*>(base + o.key_ranges), blocks,
-                           reinterpret_cast<uint32_t*>(ws + w.hist), to_host);
-    }
+        hipLaunchKernelGGL(depth_hist_kernel, dim3((unsigned)min((int64_t)DSX_HIST_BLOCKS, chunks)), dim3(kHist32Threads), bytes, stream,
+                           (const uint32_t*)keys_a, n, reinterpret_cast<const uint2*>(base + o.key_ranges), blocks,
+                           reinterpret_cast<uint32_t*>(ws + w.hist), bin_hist, bin_bits, buckets.span, to_host);
+    };
+    count_keys(const_cast<uint32_t*>(buckets.bins), bin_bits);
     DSX_LAUNCH_CHECK();
     uint64_t ends, emitters;
     if(!wait_for_word(to_host, 2, stream, &ends) || !wait_for_word(to_host, 3, stream, &emitters))
         return DSX_ERR_RUNTIME;
     const DepthRange range = depth_range((uint32_t)(ends & 0xffffu), (uint32_t)(ends >> 16));
+    if(bin_bits && depth_bins(range))
+    {
+        if(int rc = launch_buckets(buckets, (int64_t)emitters, stream))
+            return rc;
+        uint64_t answer;
+        if(!wait_for_word(to_host, 4, stream, &answer))
+            return DSX_ERR_RUNTIME;
+        if(answer == kBucketsDone)
+        {
+            *offsets_done = true;
+            return DSX_OK;
+        }
+        // too many equal depths: the passes, on a workspace as they want it
+        if(int rc = launch_fill_u32(reinterpret_cast<uint32_t*>(ws + w.hist), (int64_t)((w.bytes - w.hist) / 4), 0u, stream))
+            return rc;
+        count_keys(nullptr, 0);
+        DSX_LAUNCH_CHECK();
+    }
     const char* const label = "onesweep32_kernel<sort>";
     *emitting = n;
     if(!range.narrow)
@@ -1925,6 +2603,7 @@ static int launch_depth_sort(int64_t n, char* base, const OrderLayout& o, int64_
                                                                       nullptr, nullptr, nullptr, polls)
         switch(sort32_items(n))
         {
+            DSX_DEPTH_SORT_ITEMS(1);
             DSX_DEPTH_SORT_ITEMS(2);
             DSX_DEPTH_SORT_ITEMS(3);
             DSX_DEPTH_SORT_ITEMS(4);
@@ -2129,10 +2808,13 @@ int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_
     // pass gathers them
     const bool carry = tiles_x(cam.image_width) <= kRect32MaxTiles && tiles_y(cam.image_height) <= kRect32MaxTiles;
     const int64_t blocks = (n + kProjBlock - 1) / kProjBlock;
-    // (a wait for the range: fewer Gaussians are sorted before the host could have launched the rest; us a step
-    // with four digits / three: 50 K 223 / 230, 100 K 249 / 260, 300 K 493 / 491, 1 M forward 319 / 305)
-    if(to_host.words && sort32_items(n) > 1)
-        rc = launch_depth_sort(n, base, o, blocks, carry, to_host, sort_polls, stream, &emitting);
+    // (a wait for the range: what few Gaussians need is done before the host could have launched the rest.  Beyond those of
+    // launch_order_ranks it pays where buckets order them, a forward of 150 K 120 -> 100 us, and costs 2 of 114 where the range has both signs.)
+    bool offsets_done = false;
+    const bool by_buckets = orders_by_buckets(n) && offset_polls == kSpinLimit32;
+    if(to_host.words && (sort32_items(n) > 1 || (by_buckets && sort_polls == kSpinLimit32)))
+        rc = launch_depth_sort(n, base, o, blocks, carry, by_buckets, list_grid(cam).shift, to_host, sort_polls, stream, &emitting,
+                               &offsets_done);
     else // (four passes: the values, iota in the first, go b, a, b, a and end in ids_a)
         rc = launch_sort32(n, 32, keys_a, ids_a, keys_b, ids_b, true, false, base + o.sort, stream, &ko, &vo,
                        reinterpret_cast<const uint2*>(base + o.rects), reinterpret_cast<uint2*>(base + o.rects_sorted),
@@ -2142,6 +2824,7 @@ int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_
         return finish(rc);
     if(vo != ids_a)
         return finish(DSX_ERR_RUNTIME);
+    if(!offsets_done)
     {
         DSX_TIMED("ordered_offsets_kernel", stream);
         hipLaunchKernelGGL(ordered_offsets_kernel, dim3((unsigned)((n + kOffsetsShare - 1) / kOffsetsShare)), dim3(kOffsetsThreads), 0, stream,

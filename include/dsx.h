@@ -409,13 +409,14 @@ int dsx_trace_read(dsx_trace_entry* out /* host */, int max_entries);
  * wavefronts per tile, which add up a pixel's colours in four parts (final_T and final_idx are the same bits). */
 int dsx_set_blend_pixels_per_lane(int pixels);
 
-/* dsx_depth_order as dsx_forward_project runs it (above 262144 Gaussians the host waits for the range of the depths), with
+/* dsx_depth_order as dsx_forward_project runs it (above 131072 Gaussians the host waits for the range of the depths), with
  * other limits on its waits, in looks for a word that is not there yet (below zero: none).
  * A tile of a sort's pass that has looked sort_polls times gives up: the sort's flag (dsx_sort_flags) is set and the order wrong,
  * with every access inside `order`, whatever it held.  The workgroups that make the block offsets tell each other their sums, and one that has
  * looked offset_polls times for another's sums up the other's rectangles itself: the offsets are the same.  For
- * tests; the other entry points look 2^18 times.  (Up to 131072 Gaussians those order by a launch that waits for nothing; with
- * other limits than theirs the kernels that wait are what runs, whatever the number.) */
+ * tests; the other entry points look 2^18 times.  (Up to 8388608 Gaussians those order by launches that wait for nothing, but for depths of
+ * both signs, of a wide or thin range, or too many equal ones beyond 131072; with other limits than theirs the kernels that wait are
+ * what runs, whatever the number.) */
 int dsx_depth_order_bounded(const dsx_camera* cam, int64_t n, void* order, size_t order_bytes,
                             int32_t sort_polls, int32_t offset_polls, void* stream);
 

@@ -362,3 +362,44 @@ def test_depth_order_and_counts_in_one_launch(n, depths):
         ids2, lists2 = stages.tile_lists(cam, n, k, again, return_lists=True)
         ready = cam.num_tiles + 2 + (0 if bins == 1 else 2 + -(-W // 64) * -(-H // 64))
         assert torch.equal(ids, ids2) and torch.equal(lists[:ready], lists2[:ready])
+
+
+@pytest.mark.parametrize("depths", ["uniform", "layers", "octaves", "seldom", "one", "runs", "two", "thin"])
+@pytest.mark.parametrize("n", [131073, 262145, 524289, 1048577, 2097153, 3145729, 4194305])
+def test_depth_order_by_buckets(n, depths):
+    """From 131073 Gaussians on the order is made by buckets: each number of keys to a workgroup and of bins, where hardly any key
+    emits, whole stretches do not, and where hundreds of depths are equal (which a bucket sorts another way).  Order and offsets are
+    those of the digit passes, which are also what runs where a bin holds too many keys or the range is thin."""
+    from ds_splat_amd import stages
+    W, H = 200, 120
+    sc = make_scene("cfg0", n=64, width=W, height=H, sh_degree=0, seed=9)
+    u = torch.rand(n, generator=torch.Generator().manual_seed(n))
+    layers = n // 700                 # (700 keys to a layer; with the depth, 128 layers at least)
+    means = torch.zeros(n, 3)
+    means[:, 2] = {"two": torch.where(u < 0.5, 2.0, 19.0), "thin": 4.0 + 0.01 * u, "octaves": 0.02 * 2.0 ** (14.5 * u),
+                   "layers": 2.0 + (u * layers).floor() * (18.0 / layers)}.get(depths, 2.0 + 18.0 * u)
+    index = torch.arange(n)
+    gone = {"seldom": index % 100 != 7, "one": index != n // 3, "runs": (index // 3000) % 2 == 0}.get(depths, index < 0)
+    means[gone, 0] = 1e6
+    scales = (means[:, 2:].abs() * 1e-2).expand(n, 3).contiguous()
+    rotations, opacities, shs = torch.zeros(n, 4), torch.full((n, 1), 0.5), torch.zeros(n, 16, 3)
+    rotations[:, 0] = 1.0
+    for bins in (1, 4):
+        cam = stages.camera_from_scene(sc, DEV, list_bin=bins)
+        order = stages.new_order(cam, n, DEV)
+        splats, _, _, _ = stages.project_fwd(cam, means.to(DEV), scales.to(DEV), rotations.to(DEV), opacities.to(DEV),
+                                             shs.to(DEV), order=order)
+        keys = order[:4 * n].view(torch.int32).cpu().numpy().view(np.uint32).copy()
+        again = order.clone()
+        perm, offsets = (x.clone() for x in stages.depth_order_bounded(cam, n, order))
+        # (the tiles of a first digit pass count themselves in the fourth word before the flag)
+        tiles = int(order.view(torch.int32)[stages.sort_flag_indices(cam, n, 0, order, None)[0] - 4].item())
+        assert (tiles == 0) == (depths not in ("two", "thin", "one"))
+        perm2, offsets2 = stages.depth_order_bounded(cam, n, again, sort_polls=1 << 17)      # (the digit passes)
+        assert (keys != 0xffffffff).any()
+        assert torch.equal(perm, perm2) and torch.equal(offsets, offsets2)
+        if bins == 1:
+            assert (perm.cpu().numpy() == np.argsort(keys, kind="stable")).all()
+            touched = splats[:, 11].contiguous().view(torch.int32).to(torch.int64)
+            touched[-1] = 0
+            assert int(offsets[-1]) == int(touched.sum())
