@@ -685,7 +685,7 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(7, 7))
                 const int entry_index = __float_as_int(B.w);
                 const ExponentX ex = exponent_x(A.z, A.w, pxf - A.x);
                 float weight[kPix];
-                uint64_t m_pass[kPix], m_low[kPix], m_stop = 0;
+                uint64_t m_pass[kPix];
 #pragma unroll
                 for(int p = 0; p < kPix; ++p)
                 {
@@ -700,21 +700,23 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(7, 7))
                     const float taken = __builtin_amdgcn_inverse_ballot_w64(m_pass[p]) ? alpha : 0.0f;
                     weight[p] = taken * before[p];
                     after[p] = __builtin_fmaf(-taken, before[p], before[p]); // (1 - alpha) T in one rounding
-                    m_low[p] = __builtin_amdgcn_ballot_w64(after[p] < 0.0001f);
-                    m_stop |= m_low[p];
                 }
-                if(m_stop != 0)
+                // (one compare for the least of the four: three instructions an entry instead of four, and four mask words less; whole passes
+                // of 2 M faint Gaussians 2294 -> 2276 us, 1.4 M 973 -> 966, 6 M at 3840x2160 965 -> 958)
+                static_assert(kPix == 4, "the least of four");
+                if(__builtin_amdgcn_ballot_w64(fminf(fminf(fminf(after[0], after[1]), after[2]), after[3]) < 0.0001f) != 0)
                 {
                     // pixels that this entry would make opaque stop without it
 #pragma unroll
                     for(int p = 0; p < kPix; ++p)
                     {
-                        const bool stop = __builtin_amdgcn_inverse_ballot_w64(m_low[p]);
+                        const uint64_t m_low = __builtin_amdgcn_ballot_w64(after[p] < 0.0001f);
+                        const bool stop = __builtin_amdgcn_inverse_ballot_w64(m_low);
                         weight[p] = stop ? 0.0f : weight[p];
                         after[p] = stop ? before[p] : after[p];
                         pyf[p] = stop ? __builtin_nanf("") : pyf[p];
-                        m_pass[p] &= ~m_low[p];
-                        alive -= __popcll(m_low[p]);
+                        m_pass[p] &= ~m_low;
+                        alive -= __popcll(m_low);
                     }
                 }
 #pragma unroll
