@@ -893,8 +893,10 @@ __device__ __forceinline__ int tile_place(int* counts, uint64_t m, int& total)
 constexpr int kFwdAtOnce = 4; // entries that a row takes at a time
 static_assert(kFwdAtOnce == 4 && kTileBatch % 4 == 0, "a word of the list holds four places");
 
+// (six wavefronts per SIMD: 79 registers instead of the 92 that the scan's loads in flight take; whole passes of 1 M at 1280x720
+// 254 -> 248 us, 300 K at 1237x822 430 -> 423; with seven and 72 the walk reloads, 251 and 426)
 template <bool kBinned>
-__global__ __launch_bounds__(kTileThreads) void blend_fwd_tile_kernel(const int32_t* __restrict__ ranges, const int32_t* __restrict__ ids,
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(6))) void blend_fwd_tile_kernel(const int32_t* __restrict__ ranges, const int32_t* __restrict__ ids,
                                                                       const float4* __restrict__ splats, float* __restrict__ image,
                                                                       float* __restrict__ final_T, int32_t* __restrict__ final_idx, int W,
                                                                       int H, int ntx, uint32_t last_id, int k,
