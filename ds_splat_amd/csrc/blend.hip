@@ -1840,6 +1840,20 @@ __device__ __forceinline__ void bank_sum8_scatter(const float (&v)[8], float& fi
         : "v"(s0), "v"(s1), "v"(s2), "v"(s3));
 }
 
+// The same for one value of each of two entries: lanes 0 to 3 of a row get the first's sums, lanes 8 to 11 the second's.
+__device__ __forceinline__ float bank_sum2(float a, float b)
+{
+    float s, sum;
+    asm("s_nop 1\n\t"
+        "v_add_f32_dpp %0, %2, %2 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+        "v_add_f32_dpp %0, %3, %3 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "s_nop 1\n\t"
+        "v_add_f32_dpp %1, %0, %0 row_shl:4 row_mask:0xf bank_mask:0x5"
+        : "=&v"(s), "=&v"(sum)
+        : "v"(a), "v"(b));
+    return sum;
+}
+
 // Eight values at once as a reduce-scatter.  A step takes two registers into one: the lanes of one half
 // keep the first value and add their partner's share of it, the other half the second.  The
 // DPP bank mask (banks of four lanes) chooses the lanes of an add for free where the halves are whole banks,
@@ -1945,6 +1959,21 @@ __device__ __forceinline__ void flush_sums(const double* sums, const int* ids, i
         }
 }
 
+// Colours and upstream gradients below this keep all products of theirs finite.
+constexpr float kTame = 1e12f;
+// the largest magnitude, infinite if one is NaN
+__device__ __forceinline__ float largest(float a, float b, float c)
+{
+    const float m = fmaxf(fabsf(a), fmaxf(fabsf(b), fabsf(c)));
+    return a == a && b == b && c == c ? m : __builtin_inff();
+}
+
+// Can an entry's product with an alpha of zero be anything but zero, or does its alpha reach the clamp?
+__device__ __forceinline__ bool plain_entry(const float4 q0, const float4 q1, const float4 q2)
+{
+    return q1.w <= kAlphaMaxBwd && largest(q0.x, q0.y, 0.0f) < kTame && largest(q2.x, q2.y, q2.z) < kTame;
+}
+
 // How an entry's gradient at a pixel follows from what lies behind it: with T the transmittance in front of the
 // entry, the reference's v_alpha = T (rgb . v_out) - B / (1 - alpha), B the sum over the entries behind of alpha T (rgb . v_out) and
 // the background's T_final (bg . v_out).  Let `behind` be B over the transmittance behind the entry, T (1 - alpha); then
@@ -1970,16 +1999,26 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(5, 5))
     const float* __restrict__ bg, float* grads, uint8_t* marks, int W, int H, int ntx, uint32_t last_id, int k,
     const int32_t* __restrict__ header, int header_shift, int planar, const BinLists lists, const ZeroJobs zeros)
 {
-    // (one place more in two of them: nobody's entry, as in the forward; its colour, which nobody looks at, is another's word)
-    __shared__ float4 s_records[3 * kBwdBatch + 2];
-    float4* const s_c = s_records;                     // red, green, blue
-    float4* const s_a = s_records + kBwdBatch;         // pixel x, pixel y, conic a/2, conic b
-    float4* const s_b = s_records + 2 * kBwdBatch + 1; // conic c/2, opacity, limit of sigma's bits, index in the sorted key array
-    __shared__ double s_sum[kBwdBatch * kSums + 1]; // (nobody's zeros are added to others' sums)
-    __shared__ uint4 s_list[kQuads * kBwdBatch / 16 + 1];
-    // while a round is staged, in the records' memory: candidates and the scan's queue, as in the forward
-    int2* const s_cand = reinterpret_cast<int2*>(s_records);
-    int* const s_queue = reinterpret_cast<int*>(s_records + DSX_WAVE);
+    // (one place more: nobody's entry, as in the forward.  Side by side, because with what the compiler puts between them the 7672
+    // bytes would not fit 7680, the most of 20 wavefronts per compute unit)
+    __shared__ struct
+    {
+        float4 c[kBwdBatch + 1];              // red, green, blue
+        float4 a[kBwdBatch + 1];              // pixel x, pixel y, conic a/2, conic b
+        float4 b[kBwdBatch + 1];              // conic c/2, opacity, limit of sigma's bits, index in the sorted key array
+        uint4 list[kQuads * kBwdBatch / 16];  // (what follows is read ahead)
+        double sum[kBwdBatch * kSums + 1];    // (nobody's zeros are added to others' sums)
+    } s;
+    static_assert(sizeof(s) <= 7680, "20 wavefronts per compute unit");
+    float4* const s_c = s.c;
+    float4* const s_a = s.a;
+    float4* const s_b = s.b;
+    uint4* const s_list = s.list;
+    double* const s_sum = s.sum;
+    // while a round is staged, in the records' memory: candidates and the scan's queue, as in the forward (nobody's colour, which they
+    // overwrite, is written again for each round)
+    int2* const s_cand = reinterpret_cast<int2*>(&s);
+    int* const s_queue = reinterpret_cast<int*>(&s.a[DSX_WAVE - kBwdBatch - 1]);
     static_assert(DSX_WAVE + DSX_WAVE / 4 <= 2 * kBwdBatch && kBwdBatch % 2 == 0 && (kQuads * kBwdBatch) % 16 == 0 &&
                       kQuads * kBwdBatch / 16 <= DSX_WAVE, "what the records' memory holds; lists of pairs of bytes, cleared by words");
 
@@ -2070,21 +2109,25 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(5, 5))
     }
 
     double* const my_sums = s_sum + 2 * ((lane >> 2) & 1) + ((lane >> 3) & 1); // (see bank_sum8_scatter)
-    // Entries up to the smallest last one are behind no pixel's.  (A pixel that blended nothing at all takes no part: its row coordinate
-    // is NaN, and no exponent of it passes.)
+    // Entries up to the smallest last one are behind no pixel's.  (A pixel that blended nothing at all takes no part: its
+    // transmittance is zero where only that counts, and every index lies behind its last one's.)
     const int first_index = kBinned ? src.fine_base : start;
     int m_least = INT_MAX;
+    bool tame = true;
 #pragma unroll
     for(int p = 0; p < kPix; ++p)
     {
         const bool none = bin_final[p] < first_index;
-        pyf[p] = none ? __builtin_nanf("") : pyf[p];
+        T[p] = none ? 0.0f : T[p];
+        bin_final[p] = none ? INT_MIN : bin_final[p];
+        tame = tame && largest(vo0[p], vo1[p], vo2[p]) < kTame && fabsf(behind[p]) < kTame;
         m_least = none ? m_least : min(m_least, bin_final[p]);
     }
 #pragma unroll
     for(int o = 1; o < DSX_WAVE; o <<= 1)
         m_least = min(m_least, __shfl_xor(m_least, o, DSX_WAVE));
     m_least = __builtin_amdgcn_readfirstlane(m_least);
+    bool wild = __builtin_amdgcn_ballot_w64(!tame) != 0;
 
     const LiveBox box = {(float)x0 + 0.5f, (float)x0 + 15.5f, (float)y0 + 0.5f, (float)y0 + 15.5f};
     const int32_t* const keys = ids + k; // the pairs' key words lie behind the ids (binned lists)
@@ -2182,18 +2225,21 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(5, 5))
         spares = found - staged;
         __syncthreads();
         uint32_t reached = 0;
-        bool special = false;
+        bool special = false, last_here = false;
         if(lane < staged)
         {
             const float4* const rec = splats + 3 * (int64_t)mine.x;
             const float4 q0 = rec[0], q1 = rec[1], q2 = rec[2];
             const float reach = reach_of(q1.w);
-            special = mine.y > m_least || !(q1.w <= kAlphaMaxBwd);
+            last_here = mine.y > m_least;
+            special = !plain_entry(q0, q1, q2);
             reached = blocks_reached(q0.x, q0.y, q1.x, q1.y, q1.z, reach, (float)x0 + 0.5f, (float)y0 + 0.5f);
             s_a[lane] = make_float4(q0.x, q0.y, q1.x * 0.5f, q1.y);
             s_b[lane] = make_float4(q1.z * 0.5f, q1.w, __uint_as_float(reach_limit_bwd(q1.w, reach)), __int_as_float(mine.y));
             s_c[lane] = make_float4(q2.x, q2.y, q2.z, 0.f);
         }
+        if(lane == kBwdBatch)
+            s_c[kBwdBatch] = make_float4(0.f, 0.f, 0.f, 0.f);
         // (entries behind everything that a quad's pixels blended are not in its list)
 #pragma unroll
         for(int q = 0; q < kQuads; ++q)
@@ -2210,9 +2256,118 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(5, 5))
             s_sum[i] = 0.0;
         __syncthreads();
 
-        // (plain: no pixel's last entry lies among these, and no alpha reaches the clamp: two of 36 instructions a pixel and entry;
-        // 2 M faint Gaussians 1368 -> 1335 us, 1.4 M at 1557x1038 508 -> 493)
-        auto walk = [&](auto plain) {
+        // Two entries at a time, without branches: a pixel that does not take an entry gives it the alpha zero.  Both
+        // transmittances come from one reciprocal, and the moments over a lane's four rows from those of two rows each that count
+        // from the upper one, eleven operations instead of sixteen (all four counted from one row: nine, but terms that cancel where a
+        // splat is hardly wider than a pixel: 1.3 times the error there).  A pair's sums are added when the next one's records have been
+        // asked for: the LDS serves a wavefront in order, and behind the adds the reads would wait for them.  117 vector instructions
+        // an entry instead of 132 (of which a seventh was jumped over where no lane took a row).  us, one entry after the other -> pairs, of
+        // which without the late adds: 2 M faint Gaussians 1253 -> 1236 (1235), 1.4 M at 1557x1038 468 -> 451 (457), 500 K 217 -> 205 (210), 3 M 258 -> 243
+        // (255), 300 K at 1237x822 225 -> 215 (221).  Distance of the gradients from a 64-bit evaluation (scenes of 700 records; means, conics,
+        // opacities, 1e-7): ordinary 3.1, 3.0, 3.0 -> 2.9, 2.8, 2.8; opacity 0.9 3.6, 3.5, 3.3 -> 3.2, 3.2, 2.9; large 5.1, 5.4, 6.5 -> 4.6, 3.5, 4.9;
+        // faint 2.1, 2.2, 2.0 -> 2.0, 2.1, 1.9; hardly wider than a pixel 1.2, 1.3, 1.1 -> 1.2, 1.4, 1.1.
+        auto walk_pairs = [&](auto ends) {
+        const uint16_t* my_list = reinterpret_cast<const uint16_t*>(s_list) + block * (kBwdBatch / 2);
+        int places = *my_list;
+        // (zeros at first, for each quad elsewhere; worked out here: kept over the rounds it would be spilled, and the wait for its reload
+        // is one for the last round's adds to memory too)
+        int fresh = lane;
+        asm volatile("" : "+v"(fresh));
+        int summed_places = (fresh >> 2 & 12) | (fresh & 3);
+        summed_places |= summed_places << 8;
+        float sums8[2][2] = {}, sums_blue = 0.0f;
+        auto add_sums = [&]() {
+#pragma unroll
+            for(int u = 0; u < 2; ++u)
+            {
+                double* const sums = my_sums + 4 * (u == 0 ? summed_places & 0xff : summed_places >> 8);
+                unsafeAtomicAdd(sums, (double)sums8[u][0]);
+                unsafeAtomicAdd(sums + 4 * kBwdBatch, (double)sums8[u][1]);
+            }
+            if((lane & 4) == 0)
+                unsafeAtomicAdd(s_sum + 8 * kBwdBatch + ((summed_places >> (lane & 8)) & 0xff), (double)sums_blue);
+        };
+        for(int i = 0; i < rounds; i += 2)
+        {
+            const int here = places;
+            places = *++my_list;
+            const float4 A[2] = {s_a[here & 0xff], s_a[here >> 8]};
+            const float4 B[2] = {s_b[here & 0xff], s_b[here >> 8]};
+            const float4 C[2] = {s_c[here & 0xff], s_c[here >> 8]};
+            asm volatile("" ::: "memory");
+            add_sums();
+            summed_places = here;
+            float alpha[2][kPix], dx[2], dy0[2];
+#pragma unroll
+            for(int u = 0; u < 2; ++u)
+            {
+                dx[u] = pxf - A[u].x;
+                const ExponentX ex = exponent_x(A[u].z, A[u].w, dx[u]);
+#pragma unroll
+                for(int p = 0; p < kPix; ++p)
+                {
+#pragma clang fp contract(off)
+                    // sigma exactly as the forward computed it
+                    const float dy = pyf[p] - A[u].y;
+                    const float sigma = __builtin_fmaf(__builtin_fmaf(B[u].x, dy, ex.bx), dy, ex.ax);
+                    uint64_t m_valid = __builtin_amdgcn_ballot_w64(__float_as_uint(sigma) <= __float_as_uint(B[u].z));
+                    if(ends)
+                        m_valid &= __builtin_amdgcn_ballot_w64(__float_as_int(B[u].w) <= bin_final[p]);
+                    const float full = B[u].y * __builtin_amdgcn_exp2f(-sigma * kLog2E);
+                    alpha[u][p] = __builtin_amdgcn_inverse_ballot_w64(m_valid) ? full : 0.0f;
+                    if(p == 0)
+                        dy0[u] = dy;
+                }
+            }
+            float between[kPix]; // the transmittance in front of the first, T becomes that in front of both
+#pragma unroll
+            for(int p = 0; p < kPix; ++p)
+            {
+                const float through = 1.0f - alpha[0][p];
+                T[p] *= __builtin_amdgcn_rcpf(__builtin_fmaf(-alpha[1][p], through, through));
+                between[p] = __builtin_fmaf(-alpha[1][p], T[p], T[p]);
+            }
+            float blue[2];
+#pragma unroll
+            for(int u = 0; u < 2; ++u)
+            {
+                // per lane, over its pixels (which share dx): the weights of the colour's gradient, and w of every pixel
+                // (opacity * w: alpha holds the opacity)
+                float v_red = 0.f, v_green = 0.f, v_blue = 0.f, w[kPix];
+#pragma unroll
+                for(int p = 0; p < kPix; ++p)
+                {
+                    const float fac = alpha[u][p] * (u == 0 ? between[p] : T[p]);
+                    v_red = p == 0 ? fac * vo0[p] : v_red + fac * vo0[p];
+                    v_green = p == 0 ? fac * vo1[p] : v_green + fac * vo1[p];
+                    v_blue = p == 0 ? fac * vo2[p] : v_blue + fac * vo2[p];
+                    const float ahead = C[u].x * vo0[p] + (C[u].y * vo1[p] + (C[u].z * vo2[p] - behind[p]));
+                    behind[p] += alpha[u][p] * ahead;
+                    w[p] = fac * ahead;
+                }
+                // 1 | dy | dy^2
+                static_assert(kPix == 4, "two times two rows");
+                float of0[2], of1[2], of2[2];
+#pragma unroll
+                for(int h = 0; h < 2; ++h)
+                {
+                    const float dy = dy0[u] + (float)(2 * h), lower = w[2 * h + 1];
+                    of0[h] = w[2 * h] + lower;
+                    of1[h] = __builtin_fmaf(dy, of0[h], lower);
+                    of2[h] = __builtin_fmaf(dy, of1[h] + lower, lower);
+                }
+                const float S0 = of0[0] + of0[1], S1 = of1[0] + of1[1], S2 = of2[0] + of2[1];
+                const float S0x = S0 * dx[u];
+                const float sum8[8] = {S0, S0x, S0x * dx[u], S1, S1 * dx[u], S2, v_red, v_green};
+                bank_sum8_scatter(sum8, sums8[u][0], sums8[u][1]);
+                blue[u] = v_blue;
+            }
+            sums_blue = bank_sum2(blue[0], blue[1]);
+        }
+        add_sums();
+        };
+        // what the walk above leaves out: clamped alphas, and values so large that a product with zero is not zero
+        auto walk_any = [&]() {
         const uint16_t* my_list = reinterpret_cast<const uint16_t*>(s_list) + block * (kBwdBatch / 2);
         int places = *my_list;
         for(int i = 0; i < rounds; i += 2)
@@ -2242,17 +2397,16 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(5, 5))
 #pragma clang fp contract(off)
                     dy[p] = pyf[p] - A.y;
                     const float sigma = __builtin_fmaf(__builtin_fmaf(B.x, dy[p], ex.bx), dy[p], ex.ax);
-                    m_valid[p] = __builtin_amdgcn_ballot_w64(__float_as_uint(sigma) <= limit);
-                    if(!plain)
-                        m_valid[p] &= __builtin_amdgcn_ballot_w64(idx <= bin_final[p]);
+                    m_valid[p] = __builtin_amdgcn_ballot_w64(__float_as_uint(sigma) <= limit) &
+                                 __builtin_amdgcn_ballot_w64(idx <= bin_final[p]);
                     m_any |= m_valid[p];
                     vis[p] = __builtin_amdgcn_exp2f(-sigma * kLog2E);
-                    alpha[p] = plain ? B.y * vis[p] : fminf(kAlphaMaxBwd, B.y * vis[p]);
+                    alpha[p] = fminf(kAlphaMaxBwd, B.y * vis[p]);
                 }
                 if(m_any == 0)
                     continue;
                 // Per lane, over its pixels (which share dx): the weights of the colour's gradient, and three
-                // moments over dy of w = vis * v_alpha (plain: of opacity * w, which the weight already holds)
+                // moments over dy of w = vis * v_alpha
                 float v_red = 0.f, v_green = 0.f, v_blue = 0.f, S0 = 0.f, S1 = 0.f, S2 = 0.f;
 #pragma unroll
                 for(int p = 0; p < kPix; ++p)
@@ -2266,7 +2420,7 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(5, 5))
                         v_blue += fac * vo2[p];
                         const float ahead = C.x * vo0[p] + (C.y * vo1[p] + (C.z * vo2[p] - behind[p]));
                         behind[p] += alpha[p] * ahead;
-                        const float w = (plain ? fac : vis[p] * T[p]) * ahead;
+                        const float w = vis[p] * T[p] * ahead;
                         const float wdy = w * dy[p];
                         S0 += w;
                         S1 += wdy;
@@ -2288,11 +2442,20 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(5, 5))
             }
         }
         };
-        const bool all_plain = __builtin_amdgcn_ballot_w64(special) == 0;
-        if(all_plain)
-            walk(std::true_type());
+        const bool all_plain = !wild && __builtin_amdgcn_ballot_w64(special) == 0;
+        if(!all_plain)
+        {
+            walk_any();
+            bool still = true;
+#pragma unroll
+            for(int p = 0; p < kPix; ++p)
+                still = still && fabsf(behind[p]) < kTame;
+            wild = wild || __builtin_amdgcn_ballot_w64(!still) != 0; // (an infinite colour stays behind all entries in front)
+        }
+        else if(__builtin_amdgcn_ballot_w64(last_here) != 0) // (some pixel's last entry lies among these: one compare a pixel and entry more)
+            walk_pairs(std::true_type());
         else
-            walk(std::false_type());
+            walk_pairs(std::false_type());
         __syncthreads();
         if(lane < staged)
         {

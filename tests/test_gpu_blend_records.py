@@ -105,3 +105,72 @@ def test_a_needle_is_blended_wherever_alpha_reaches_the_threshold(blend_form, pi
     want = torch.where(takes, twice, torch.zeros(())).double().sum(1)
     # (a pixel more or less is 1/255 of colour 1: from sums of up to 16 pixels)
     np.testing.assert_allclose(got["grads"][:, 6].double().numpy(), want.numpy(), rtol=1e-5, atol=1e-7)
+
+
+def sums_in_64_bits(rec, v_image, bg, final_T, final_idx):
+    """The nine sums of every entry, and the sums of their terms' magnitudes, back to front from what the forward
+    left, all entries in the one list of every pixel.  Also the pixels where a decision is closer than 32 bits tell."""
+    h, w = final_T.shape
+    y, x = torch.meshgrid(torch.arange(h) + 0.5, torch.arange(w) + 0.5, indexing="ij")
+    v, T, last = v_image.double(), final_T.double().clone(), final_idx
+    behind = (v * bg.double()).sum(-1)
+    n = rec.shape[0]
+    sums, terms, close = torch.zeros(n, 9).double(), torch.zeros(n, 9).double(), torch.zeros(h, w, dtype=torch.bool)
+    for i in range(n - 1, -1, -1):
+        mx, my, _, _, a, b, c, opacity, red, green, blue, _ = rec[i].double()
+        dx, dy = x - mx, y - my
+        sigma = 0.5 * (a * dx * dx + c * dy * dy) + b * dx * dy
+        vis = torch.exp(-sigma)
+        close |= ((opacity * vis * 255.0 - 1.0).abs() < 1e-4) | (sigma.abs() < 1e-6)
+        takes = (opacity * vis >= 1.0 / 255.0) & (sigma >= 0.0) & (i <= last)
+        alpha = torch.where(takes, (opacity * vis).clamp(max=0.99), torch.zeros(()).double())
+        T = T / (1.0 - alpha)
+        ahead = v @ torch.stack([red, green, blue]) - behind
+        behind = behind + alpha * ahead
+        vw = torch.where(takes, vis * T * ahead, torch.zeros(()).double())
+        s = opacity * vw
+        for j, t in enumerate((s * (a * dx + b * dy), s * (b * dx + c * dy), -0.5 * s * dx * dx, -s * dx * dy,
+                               -0.5 * s * dy * dy, vw, alpha * T * v[..., 0], alpha * T * v[..., 1], alpha * T * v[..., 2])):
+            sums[i, j], terms[i, j] = t.sum(), t.abs().sum()
+    return sums, terms, close
+
+
+@pytest.mark.parametrize("kind", ["faint", "clamped", "stopping", "wild"])
+@pytest.mark.parametrize("n", [1, 2, 55, 57, 113, 247, 249, 500])
+@pytest.mark.parametrize("pixels_per_lane", [1, 4])
+def test_backward_sums_against_64_bits(blend_form, pixels_per_lane, n, kind):
+    """Around the rounds of 56 and of 248 entries, odd and even: rounds that no pixel's last entry lies in, rounds where
+    pixels end or alpha reaches the clamp, and an upstream gradient whose products with zero must stay out of the sums."""
+    from ds_splat_amd import stages
+    blend_form(pixels_per_lane)
+    g = torch.Generator().manual_seed(n)
+    rand = lambda *s: torch.rand(*s, generator=g)
+    h, w = 30, 43
+    rec = torch.zeros(n, 12)
+    rec[:, 0], rec[:, 1], rec[:, 3] = rand(n) * (w + 8) - 4, rand(n) * (h + 8) - 4, 50.0
+    turn, major, minor = rand(n) * 3.14159, 1.0 / (1.0 + 9.0 * rand(n)) ** 2, 1.0 / (0.7 + rand(n)) ** 2
+    cos, sin = torch.cos(turn), torch.sin(turn)
+    rec[:, 4], rec[:, 5] = major * cos ** 2 + minor * sin ** 2, (major - minor) * cos * sin
+    rec[:, 6] = major * sin ** 2 + minor * cos ** 2
+    rec[:, 7] = 0.02 + (0.05 if kind == "faint" else 0.9) * rand(n)
+    if kind == "clamped":
+        rec[:, 7] = torch.where(rand(n) < 0.02, 0.999, 0.05)
+    rec[:, 8:11] = rand(n, 3)
+    v_image = torch.randn(h, w, 3, generator=g)
+    if kind == "wild":
+        v_image[17:, 20:] *= 1e13
+    scene = make_scene("cfg0", n=1, width=w, height=h, sh_degree=0)
+    cam = stages.camera_from_scene(scene, DEV, list_bin=1, bg=torch.tensor([0.3, 0.1, 0.8]))
+    tiles = ((h + 15) // 16) * ((w + 15) // 16)
+    ids = torch.arange(n, dtype=torch.int32).repeat(tiles).to(DEV)
+    ranges = (torch.arange(tiles + 1, dtype=torch.int32) * n).to(DEV)
+    _, final_T, final_idx = stages.blend_fwd(cam, ranges, ids, rec.to(DEV))
+    tile_of = torch.arange(h)[:, None] // 16 * ((w + 15) // 16) + torch.arange(w)[None] // 16
+    args = torch.tensor([0.3, 0.1, 0.8]), final_T.cpu(), final_idx.cpu() - tile_of * n
+    close = sums_in_64_bits(rec, v_image, *args)[2]
+    assert close.float().mean() < 0.2
+    v_image[close] = 0.0
+    want, terms, _ = sums_in_64_bits(rec, v_image, *args)
+    got = stages.blend_bwd(cam, n, ranges, ids, rec.to(DEV), final_T, final_idx, v_image.to(DEV))[:, :9].cpu().double()
+    # (T is rebuilt over up to 500 entries, three roundings of 6e-8 each, and starts from one that the forward left)
+    assert ((got - want).abs() <= 1e-4 * terms + 1e-7).all(), float(((got - want).abs() / (terms + 1e-3)).max())
