@@ -1893,6 +1893,48 @@ __device__ __forceinline__ float row_sum8_scatter(const float (&v)[8], int lane)
     return dpp_add<0x4E>(o);                     // quad_perm [2,3,0,1]: lanes that differ in bit 1
 }
 
+// The same for two entries' eight values each and a ninth of each: `one` is the sum of a[l & 7] for lanes 0 to 7 of a row, of b[l & 7] for
+// lanes 8 to 15, `ninth` that of a8 and b8.  Lanes 8 apart take the two entries apart, half rows mirrored the values four apart, and
+// neighbours and lanes two apart trade by selects: 33 + 5 instructions instead of 2 x 22.
+__device__ __forceinline__ void row_sum16_scatter(const float (&a)[8], const float (&b)[8], float a8, float b8, int lane, float& one,
+                                                  float& ninth)
+{
+    float s[8], t[4], n;
+#pragma unroll
+    for(int h = 0; h < 8; h += 4)
+        asm("s_nop 1\n\t"
+            "v_add_f32_dpp %0, %4, %4 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+            "v_add_f32_dpp %1, %5, %5 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+            "v_add_f32_dpp %2, %6, %6 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+            "v_add_f32_dpp %3, %7, %7 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+            "v_add_f32_dpp %0, %8, %8 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+            "v_add_f32_dpp %1, %9, %9 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+            "v_add_f32_dpp %2, %10, %10 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+            "v_add_f32_dpp %3, %11, %11 row_ror:8 row_mask:0xf bank_mask:0xc"
+            : "=&v"(s[h]), "=&v"(s[h + 1]), "=&v"(s[h + 2]), "=&v"(s[h + 3])
+            : "v"(a[h]), "v"(a[h + 1]), "v"(a[h + 2]), "v"(a[h + 3]), "v"(b[h]), "v"(b[h + 1]), "v"(b[h + 2]), "v"(b[h + 3]));
+    asm("s_nop 1\n\t"
+        "v_add_f32_dpp %4, %13, %13 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+        "v_add_f32_dpp %4, %14, %14 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %0, %5, %5 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"
+        "v_add_f32_dpp %1, %6, %6 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"
+        "v_add_f32_dpp %2, %7, %7 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"
+        "v_add_f32_dpp %3, %8, %8 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"
+        "v_add_f32_dpp %0, %9, %9 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
+        "v_add_f32_dpp %1, %10, %10 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
+        "v_add_f32_dpp %2, %11, %11 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
+        "v_add_f32_dpp %3, %12, %12 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
+        "v_add_f32_dpp %4, %4, %4 row_half_mirror row_mask:0xf bank_mask:0xf"
+        : "=&v"(t[0]), "=&v"(t[1]), "=&v"(t[2]), "=&v"(t[3]), "=&v"(n)
+        : "v"(s[0]), "v"(s[1]), "v"(s[2]), "v"(s[3]), "v"(s[4]), "v"(s[5]), "v"(s[6]), "v"(s[7]), "v"(a8), "v"(b8));
+    const bool odd = lane & 1, upper = lane & 2;
+    const float x = (odd ? t[1] : t[0]) + dpp_move<0xB1, true>(odd ? t[0] : t[1]); // quad_perm [1,0,3,2]
+    const float y = (odd ? t[3] : t[2]) + dpp_move<0xB1, true>(odd ? t[2] : t[3]);
+    one = (upper ? y : x) + dpp_move<0x4E, true>(upper ? x : y);                   // quad_perm [2,3,0,1]
+    n += dpp_move<0xB1, true>(n);
+    ninth = n + dpp_move<0x4E, true>(n);
+}
+
 // The nine sums of a staged entry, added up in LDS over the rows of lanes: as doubles, because the LDS adds a double
 // in a third of a cycle per lane where a float takes three (36 lanes: 11 cycles against 109, of a unit
 // that the compute unit's wavefronts share).
@@ -2487,9 +2529,10 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
     __shared__ int s_id[kTileBatch];
     __shared__ double s_sum[(kTileBatch + 1) * kSums];
     __shared__ uint16_t s_reach[kTileBatch];
-    __shared__ uint32_t s_list[kTileWaves * kTileBatch];
+    __shared__ uint32_t s_list[kTileWaves * kTileBatch + 1]; // (one word more: read ahead)
     __shared__ TileScan s_scan;
     __shared__ int s_counts[kTileWaves];
+    __shared__ uint32_t s_special[kTileWaves]; // per wavefront: does this round need the general walk?
     __shared__ int s_last[4 * kTileWaves]; // per block: the last entry that any of its pixels blended
     int* const s_queue = reinterpret_cast<int*>(s_list); // (free while a round is staged)
 
@@ -2509,9 +2552,9 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
     const int64_t step = planar ? 1 : 3, plane = planar ? (int64_t)W * H : 1; // (between pixels, between channels)
     const float vo0 = inside ? v_image[step * pix] : 0.f, vo1 = inside ? v_image[step * pix + plane] : 0.f,
                 vo2 = inside ? v_image[step * pix + 2 * plane] : 0.f;
-    // (-B, see above: with `behind` in its place an entry's chain is an operation longer, start of a training 97 -> 98 us, 50 K at
-    // 512x512 72.4 -> 72.9)
-    float bterm = -Tf * (bg[0] * vo0 + bg[1] * vo1 + bg[2] * vo2);
+    float behind = bg[0] * vo0 + bg[1] * vo1 + bg[2] * vo2;
+    const bool tame = largest(vo0, vo1, vo2) < kTame && fabsf(behind) < kTame;
+    bool wild = __builtin_amdgcn_ballot_w64(!tame) != 0; // (of this wavefront's pixels)
     int m = bin_final;
 #pragma unroll
     for(int o = 8; o > 0; o >>= 1)
@@ -2564,6 +2607,7 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
     const int sum_slot = carries_blue ? 8 : 4 * (lane & 1) + 2 * ((lane >> 2) & 1) + ((lane >> 3) & 1);
     double* const my_sums = s_sum + sum_at<kTileBatch + 1>(0, sum_slot);
     const int sum_step = carries_blue ? 1 : 4;
+    double* const my_sum = s_sum + sum_at<kTileBatch + 1>(0, lane & 7); // (see row_sum16_scatter)
 
     const int32_t* const keys = ids + k;
     int id_ahead = 0;
@@ -2589,6 +2633,7 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
                 id_ahead = ids[pos - tid];
         }
         uint32_t reached = 0;
+        bool special = wild;
         float4 q0, q1, q2;
         float reach = 0.0f;
         const int idx = idx_next - tid;
@@ -2603,10 +2648,14 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
             for(int b = 0; b < 4 * kTileWaves; ++b)
                 if(idx > s_last[b])
                     reached &= ~(1u << b);
+            special = special || (reached != 0 && !plain_entry(q0, q1, q2));
         }
         if(tid < batch) // (the loads end here: behind the adds they would wait for those)
             asm volatile("" : "+v"(q2.x), "+v"(q2.y), "+v"(q2.z), "+v"(q2.w));
         flush_sums<kTileBatch + 1>(s_sum, s_id, summed, grads, tid, kTileThreads);
+        const bool mine_special = __builtin_amdgcn_ballot_w64(special) != 0;
+        if(lane == 0)
+            s_special[wave] = mine_special;
         int staged;
         const int place = tile_place(s_counts, __builtin_amdgcn_ballot_w64(reached != 0), staged);
         // (the barrier inside: the queue has been read, the last round's sums have been taken)
@@ -2628,67 +2677,130 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
 
         const int rounds = (build_lists(s_list, s_reach, staged, wave, first_block, lane) + kBwdAtOnce - 1) / kBwdAtOnce;
         const uint16_t* my_list = reinterpret_cast<const uint16_t*>(s_list + wave * kTileBatch + row * (kTileBatch / 4));
-        for(int i = 0; i < rounds; ++i)
+        // (one walk for all wavefronts: the sums' unit depends on it)
+        const bool all_plain = __builtin_amdgcn_readfirstlane(s_special[0] | s_special[1] | s_special[2] | s_special[3]) == 0;
+        if(all_plain)
         {
-            const uint32_t places = my_list[i];
-            float4 A[kBwdAtOnce], B[kBwdAtOnce];
-            float dx[kBwdAtOnce], dy[kBwdAtOnce], vis[kBwdAtOnce], alpha[kBwdAtOnce], ra[kBwdAtOnce], rv[kBwdAtOnce];
-            double* sums[kBwdAtOnce];
-            uint64_t m_valid[kBwdAtOnce];
-            uint64_t m_any = 0;
-#pragma unroll
-            for(int u = 0; u < kBwdAtOnce; ++u)
+            // Two entries at a time as in the wavefront form.  Of the sixteen sums of their moments and colours each lane gets one: one add
+            // to LDS of all lanes for two entries instead of two of nine lanes of a row.  us: 50 K at 512x512 71 -> 62, 100 K at
+            // 979x546 98 -> 88; the gradients' distance from a 64-bit evaluation 3 to 30 % less (hardly wider than a pixel: the same).
+            int places = *my_list;
+            int summed_places = 4 * row | 4 * row << 8; // (zeros at first, elsewhere for each row)
+            float sums_one = 0.0f, sums_blue = 0.0f;
+            auto add_sums = [&]() {
+                const int place = (summed_places >> (lane & 8)) & 0xff;
+                unsafeAtomicAdd(my_sum + 4 * place, (double)sums_one);
+                if((lane & 7) == 0)
+                    unsafeAtomicAdd(s_sum + sum_at<kTileBatch + 1>(0, 8) + place, (double)sums_blue);
+            };
+            for(int i = 0; i < rounds; ++i)
             {
-                const uint32_t p = (places >> (8 * u)) & 0xffu;
-                A[u] = s_a[p];
-                B[u] = s_b[p];
-                const float4 C = s_c[p];
-                rv[u] = C.x * vo0 + C.y * vo1 + C.z * vo2;
-                sums[u] = my_sums + p * sum_step;
-            }
+                const int here = places;
+                places = *++my_list;
+                const float4 A[2] = {s_a[here & 0xff], s_a[here >> 8]};
+                const float4 B[2] = {s_b[here & 0xff], s_b[here >> 8]};
+                const float4 C[2] = {s_c[here & 0xff], s_c[here >> 8]};
+                asm volatile("" ::: "memory");
+                add_sums();
+                summed_places = here;
+                float alpha[2], dx[2], dy[2];
 #pragma unroll
-            for(int u = 0; u < kBwdAtOnce; ++u)
-            {
-#pragma clang fp contract(off)
-                dx[u] = pxf - A[u].x;
-                dy[u] = pyf - A[u].y;
-                const ExponentX ex = exponent_x(A[u].z, A[u].w, dx[u]);
-                const float sigma = __builtin_fmaf(__builtin_fmaf(B[u].x, dy[u], ex.bx), dy[u], ex.ax);
-                m_valid[u] = __builtin_amdgcn_ballot_w64(__float_as_int(B[u].w) <= bin_final) &
-                             __builtin_amdgcn_ballot_w64(__float_as_uint(sigma) <= __float_as_uint(B[u].z));
-                m_any |= m_valid[u];
-                vis[u] = __builtin_amdgcn_exp2f(-sigma * kLog2E);
-                alpha[u] = fminf(0.99f, B[u].y * vis[u]);
-                ra[u] = __builtin_amdgcn_rcpf(1.0f - alpha[u]);
-            }
-            if(m_any == 0)
-                continue;
-#pragma unroll
-            for(int u = 0; u < kBwdAtOnce; ++u)
-            {
-                float w = 0.f, v_red = 0.f, v_green = 0.f, v_blue = 0.f;
-                if(__builtin_amdgcn_inverse_ballot_w64(m_valid[u]))
+                for(int u = 0; u < 2; ++u)
                 {
-                    T *= ra[u];
-                    const float fac = alpha[u] * T;
-                    v_red = fac * vo0;
-                    v_green = fac * vo1;
-                    v_blue = fac * vo2;
-                    const float v_alpha = rv[u] * T + bterm * ra[u];
-                    bterm -= rv[u] * fac;
-                    w = vis[u] * v_alpha;
+#pragma clang fp contract(off)
+                    dx[u] = pxf - A[u].x;
+                    dy[u] = pyf - A[u].y;
+                    const ExponentX ex = exponent_x(A[u].z, A[u].w, dx[u]);
+                    const float sigma = __builtin_fmaf(__builtin_fmaf(B[u].x, dy[u], ex.bx), dy[u], ex.ax);
+                    const uint64_t m_valid = __builtin_amdgcn_ballot_w64(__float_as_int(B[u].w) <= bin_final) &
+                                             __builtin_amdgcn_ballot_w64(__float_as_uint(sigma) <= __float_as_uint(B[u].z));
+                    const float full = B[u].y * __builtin_amdgcn_exp2f(-sigma * kLog2E);
+                    alpha[u] = __builtin_amdgcn_inverse_ballot_w64(m_valid) ? full : 0.0f;
                 }
-                const float wx = w * dx[u], wy = w * dy[u];
-                const float sum8[8] = {w, wx, wx * dx[u], wy, wy * dx[u], wy * dy[u], v_red, v_green};
-                const float total = row_sum8_scatter(sum8, lane);
-                v_blue = row_sum(v_blue);
-                if(carries)
-                    unsafeAtomicAdd(sums[u], (double)(carries_blue ? v_blue : total));
+                const float through = 1.0f - alpha[0];
+                T *= __builtin_amdgcn_rcpf(__builtin_fmaf(-alpha[1], through, through));
+                float v[2][8], blue[2];
+#pragma unroll
+                for(int u = 0; u < 2; ++u)
+                {
+                    const float fac = alpha[u] * (u == 0 ? __builtin_fmaf(-alpha[1], T, T) : T);
+                    const float ahead = C[u].x * vo0 + (C[u].y * vo1 + (C[u].z * vo2 - behind));
+                    behind += alpha[u] * ahead;
+                    const float w = fac * ahead, wx = w * dx[u], wy = w * dy[u];
+                    v[u][0] = w, v[u][1] = wx, v[u][2] = wx * dx[u], v[u][3] = wy;
+                    v[u][4] = wy * dx[u], v[u][5] = wy * dy[u], v[u][6] = fac * vo0, v[u][7] = fac * vo1;
+                    blue[u] = fac * vo2;
+                }
+                row_sum16_scatter(v[0], v[1], blue[0], blue[1], lane, sums_one, sums_blue);
             }
+            add_sums();
+        }
+        else
+        {
+            for(int i = 0; i < rounds; ++i)
+            {
+                const uint32_t places = my_list[i];
+                float4 A[kBwdAtOnce], B[kBwdAtOnce];
+                float dx[kBwdAtOnce], dy[kBwdAtOnce], vis[kBwdAtOnce], alpha[kBwdAtOnce], ra[kBwdAtOnce], rv[kBwdAtOnce];
+                double* sums[kBwdAtOnce];
+                uint64_t m_valid[kBwdAtOnce];
+                uint64_t m_any = 0;
+#pragma unroll
+                for(int u = 0; u < kBwdAtOnce; ++u)
+                {
+                    const uint32_t p = (places >> (8 * u)) & 0xffu;
+                    A[u] = s_a[p];
+                    B[u] = s_b[p];
+                    const float4 C = s_c[p];
+                    rv[u] = C.x * vo0 + C.y * vo1 + C.z * vo2;
+                    sums[u] = my_sums + p * sum_step;
+                }
+#pragma unroll
+                for(int u = 0; u < kBwdAtOnce; ++u)
+                {
+#pragma clang fp contract(off)
+                    dx[u] = pxf - A[u].x;
+                    dy[u] = pyf - A[u].y;
+                    const ExponentX ex = exponent_x(A[u].z, A[u].w, dx[u]);
+                    const float sigma = __builtin_fmaf(__builtin_fmaf(B[u].x, dy[u], ex.bx), dy[u], ex.ax);
+                    m_valid[u] = __builtin_amdgcn_ballot_w64(__float_as_int(B[u].w) <= bin_final) &
+                                 __builtin_amdgcn_ballot_w64(__float_as_uint(sigma) <= __float_as_uint(B[u].z));
+                    m_any |= m_valid[u];
+                    vis[u] = __builtin_amdgcn_exp2f(-sigma * kLog2E);
+                    alpha[u] = fminf(0.99f, B[u].y * vis[u]);
+                    ra[u] = __builtin_amdgcn_rcpf(1.0f - alpha[u]);
+                }
+                if(m_any == 0)
+                    continue;
+#pragma unroll
+                for(int u = 0; u < kBwdAtOnce; ++u)
+                {
+                    float w = 0.f, v_red = 0.f, v_green = 0.f, v_blue = 0.f;
+                    if(__builtin_amdgcn_inverse_ballot_w64(m_valid[u]))
+                    {
+                        T *= ra[u];
+                        const float fac = alpha[u] * T;
+                        v_red = fac * vo0;
+                        v_green = fac * vo1;
+                        v_blue = fac * vo2;
+                        const float ahead = rv[u] - behind;
+                        behind += alpha[u] * ahead;
+                        w = vis[u] * T * ahead;
+                    }
+                    const float wx = w * dx[u], wy = w * dy[u];
+                    const float sum8[8] = {w, wx, wx * dx[u], wy, wy * dx[u], wy * dy[u], v_red, v_green};
+                    const float total = row_sum8_scatter(sum8, lane);
+                    v_blue = row_sum(v_blue);
+                    if(carries)
+                        unsafeAtomicAdd(sums[u], (double)(carries_blue ? v_blue : total));
+                }
+            }
+            // (an infinite colour stays behind all entries in front)
+            wild = wild || __builtin_amdgcn_ballot_w64(!(fabsf(behind) < kTame)) != 0;
         }
         __syncthreads();
         for(int e = tid; e < staged; e += kTileThreads)
-            moments_to_gradients<kTileBatch + 1>(s_sum, e, s_a[e], s_b[e], false, marks ? marks + s_id[e] : nullptr);
+            moments_to_gradients<kTileBatch + 1>(s_sum, e, s_a[e], s_b[e], all_plain, marks ? marks + s_id[e] : nullptr);
         __syncthreads();
         summed = staged;
     }
