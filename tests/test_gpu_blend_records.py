@@ -174,3 +174,25 @@ def test_backward_sums_against_64_bits(blend_form, pixels_per_lane, n, kind):
     got = stages.blend_bwd(cam, n, ranges, ids, rec.to(DEV), final_T, final_idx, v_image.to(DEV))[:, :9].cpu().double()
     # (T is rebuilt over up to 500 entries, three roundings of 6e-8 each, and starts from one that the forward left)
     assert ((got - want).abs() <= 1e-4 * terms + 1e-7).all(), float(((got - want).abs() / (terms + 1e-3)).max())
+
+
+@pytest.mark.parametrize("n, where", [(1, 0), (64, 63), (65, 64), (150, 3), (150, 70), (150, 149)])
+def test_alpha_is_clamped_in_the_rounds_that_need_it(blend_form, n, where):
+    """One opaque splat on a pixel's centre among faint ones, in any round of 64 staged entries: the forms of the
+    forward, of which only one leaves the clamp out of the other rounds, give the same bits, and the pixel's
+    transmittance is what 1 - 0.999 leaves of it."""
+    from ds_splat_amd import stages
+    cam = stages.camera_from_scene(make_scene("cfg0", n=1, width=16, height=16, sh_degree=0), DEV, list_bin=1)
+    rec = torch.zeros(n, 12)
+    rec[:, 0:2], rec[:, 4], rec[:, 6], rec[:, 7], rec[:, 8:11] = 8.0, 1e-3, 1e-3, 0.008, 0.5
+    rec[where, 0:2], rec[where, 4], rec[where, 6], rec[where, 7] = 5.51, 0.5, 0.5, 1.0
+    rec, ids = rec.to(DEV), torch.arange(n, dtype=torch.int32, device=DEV)
+    ranges = torch.tensor([0, n], dtype=torch.int32, device=DEV)
+    got = []
+    for form in (1, 4):
+        blend_form(form)
+        got.append([x.cpu() for x in stages.blend_fwd(cam, ranges, ids, rec)])
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+    faint = 0.008 * np.exp(-0.5e-3 * 2 * 2.5 ** 2)
+    # (1 - 0.999 in 32 bits, to a unit in the last place of 0.999)
+    np.testing.assert_allclose(got[1][1][5, 5], 1e-3 * (1.0 - faint) ** (n - 1), rtol=1e-4)
