@@ -129,7 +129,7 @@ extern "C" const char* dsx_error_string(int status)
 
 extern "C" int dsx_version(void)
 {
-    return 312;
+    return 313;
 }
 
 extern "C" int64_t dsx_num_blocks(int64_t n)
@@ -477,12 +477,11 @@ extern "C" int dsx_blend_bwd(const dsx_camera* cam, int64_t n, int64_t k, const 
                             as_stream(stream), false);
 }
 
-// conic_in_grads: places 9..11 of every accumulator record hold the conic (dsx_forward_finish put it there)
 static int gaussian_bwd_checked(const dsx_camera* cam, int64_t n, int32_t num_bases, const float* means3d,
                                 const float* scales, const float* quats, const float* splats, const float* cov3d,
                                 const int32_t* radii, const float* grads, float* v_mean3d, float* v_means2d,
                                 float* v_shs, float* v_colors, float* v_opacity, float* v_scale, float* v_quat,
-                                float* v_cov3d, void* stream, bool conic_in_grads, bool outputs_cleared = false,
+                                float* v_cov3d, void* stream, ConicFrom conic_from, bool outputs_cleared = false,
                                 bool with_marks = false)
 {
     if(int rc = check_camera(cam))
@@ -499,7 +498,7 @@ static int gaussian_bwd_checked(const dsx_camera* cam, int64_t n, int32_t num_ba
         return DSX_ERR_BAD_ARG; // without the stored covariance the kernel rebuilds it from scale and rotation
     return launch_gaussian_bwd(*cam, n, num_bases, means3d, scales, quats, splats, cov3d, radii, grads, v_mean3d,
                                v_means2d, num_bases > 0 ? v_shs : nullptr, v_colors, v_opacity, v_scale, v_quat,
-                               v_cov3d, as_stream(stream), conic_in_grads, outputs_cleared, with_marks);
+                               v_cov3d, as_stream(stream), conic_from, outputs_cleared, with_marks);
 }
 
 extern "C" int dsx_gaussian_bwd(const dsx_camera* cam, int64_t n, int32_t num_bases, const float* means3d,
@@ -509,7 +508,7 @@ extern "C" int dsx_gaussian_bwd(const dsx_camera* cam, int64_t n, int32_t num_ba
                                 float* v_cov3d, void* stream)
 {
     return gaussian_bwd_checked(cam, n, num_bases, means3d, scales, quats, splats, cov3d, radii, grads, v_mean3d,
-                                v_means2d, v_shs, v_colors, v_opacity, v_scale, v_quat, v_cov3d, stream, false);
+                                v_means2d, v_shs, v_colors, v_opacity, v_scale, v_quat, v_cov3d, stream, ConicFrom::kSplats);
 }
 
 // The pair counts a forward can index: the lists that are built are sorted with 30-bit counters, and
@@ -765,7 +764,10 @@ static int backward_impl(const dsx_camera* cam, int64_t n, int64_t k, int32_t nu
         return rc;
     return gaussian_bwd_checked(cam, n, num_bases, means3d, scales, quats, splats, cov3d, radii, grads, v_mean3d,
                                 v_means2d, v_shs, v_colors, v_opacity, v_scale, v_quat, v_cov3d, stream,
-                                grads_prepared != 0, true, true);
+                                zeros_alone(*cam, n)  ? ConicFrom::kInputs
+                                : grads_prepared != 0 ? ConicFrom::kGrads
+                                                      : ConicFrom::kSplats,
+                                true, true);
 }
 
 extern "C" int dsx_backward(const dsx_camera* cam, int64_t n, int64_t k, int32_t num_bases, const float* means3d,

@@ -306,6 +306,17 @@ __device__ __forceinline__ void prepare_grads_share(const float4* splats, float4
             marks[g] = 0; // "no term added yet"
     }
 }
+// The same without the conics, records and bytes as one run of zeros: nothing is read, and what is written is written in order.
+// (Figures at zeros_alone.  A few stores of each thread behind every round's loads, instead of all at the end: 3 M Gaussians the same,
+// 2 M faint +3 us, the workgroup forms +5.  The tiles preparing the records of what they stage, and nobody the others': 3 M 124 us, but 2 M
+// faint 764, whose every Gaussian seven tiles on different XCDs stage.)
+__device__ __forceinline__ void zero_grads_share(float4* prep, int64_t count, int part, int parts, int tid, int threads)
+{
+    const int64_t all = 3 * count + (count + 15) / 16, share = (all + parts - 1) / parts;
+    const int64_t end = min((part + 1) * share, all);
+    for(int64_t i = part * share + tid; i < end; i += threads)
+        prep[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+}
 
 // -----------------------------------------------------------------------------------------
 // forward: cpp/rasterizer_kernels.cu:341-431
@@ -480,7 +491,7 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(7, 7))
                                                              const uint32_t* __restrict__ sort_flag_a,
                                                              const uint32_t* __restrict__ sort_flag_b,
                                                              float4* __restrict__ prep, int64_t prep_count,
-                                                             uint8_t* __restrict__ prep_marks,
+                                                             uint8_t* __restrict__ prep_marks, int prep_zeros,
                                                              const float* __restrict__ bg, int planar,
                                                              const BinLists lists)
 {
@@ -771,7 +782,10 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(7, 7))
         if(lane < 8)
             w[lane] = lane == 0 ? stopped : (lane == 1 ? seen : (lane & 1 ? 0 : -1));
     }
-    prepare_grads_share(splats, prep, prep_count, prep_marks, blockIdx.x, gridDim.x, lane, DSX_WAVE);
+    if(prep_zeros)
+        zero_grads_share(prep, prep_count, blockIdx.x, gridDim.x, lane, DSX_WAVE);
+    else
+        prepare_grads_share(splats, prep, prep_count, prep_marks, blockIdx.x, gridDim.x, lane, DSX_WAVE);
 }
 
 // -----------------------------------------------------------------------------------------
@@ -919,7 +933,7 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(6)
                                                                       const int32_t* __restrict__ header, int header_shift,
                                                                       const uint32_t* __restrict__ sort_flag_a,
                                                                       const uint32_t* __restrict__ sort_flag_b, float4* __restrict__ prep,
-                                                                      int64_t prep_count, uint8_t* __restrict__ prep_marks,
+                                                                      int64_t prep_count, uint8_t* __restrict__ prep_marks, int prep_zeros,
                                                                       const float* __restrict__ bg, int planar,
                                                                       const BinLists lists)
 {
@@ -1111,7 +1125,10 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(6)
         // (as in the wavefront form, which speaks for the whole tile too)
         lists.walk[(int64_t)tile * 8 + tid] = tid == 0 ? scan : (tid == 1 ? seen : (tid & 1 ? 0 : -1));
     }
-    prepare_grads_share(splats, prep, prep_count, prep_marks, blockIdx.x, gridDim.x, tid, kTileThreads);
+    if(prep_zeros)
+        zero_grads_share(prep, prep_count, blockIdx.x, gridDim.x, tid, kTileThreads);
+    else
+        prepare_grads_share(splats, prep, prep_count, prep_marks, blockIdx.x, gridDim.x, tid, kTileThreads);
 }
 
 // -----------------------------------------------------------------------------------------
@@ -1459,7 +1476,7 @@ __global__ __launch_bounds__(kWideThreads) void blend_fwd_wide_kernel(const int3
                                                                       const uint32_t* __restrict__ sort_flag_a,
                                                                       const uint32_t* __restrict__ sort_flag_b,
                                                                       float4* __restrict__ prep, int64_t prep_count,
-                                                                      uint8_t* __restrict__ prep_marks,
+                                                                      uint8_t* __restrict__ prep_marks, int prep_zeros,
                                                                       const float* __restrict__ bg, int planar, const OwnLists own)
 {
     // (arrays as in the other forms; eight places more than an entry has blocks: the lists' ends name nobody's place, read ahead)
@@ -1704,7 +1721,10 @@ __global__ __launch_bounds__(kWideThreads) void blend_fwd_wide_kernel(const int3
         store_pixel(image, pix, (int64_t)W * H, red, green, blue, T, broken, bg, planar);
     }
     if(!kOwn)
-        prepare_grads_share(splats, prep, prep_count, prep_marks, blockIdx.x, gridDim.x, tid, kWideThreads);
+        if(prep_zeros)
+            zero_grads_share(prep, prep_count, blockIdx.x, gridDim.x, tid, kWideThreads);
+        else
+            prepare_grads_share(splats, prep, prep_count, prep_marks, blockIdx.x, gridDim.x, tid, kWideThreads);
 }
 
 // Does a forward without a backward find its lists itself?
@@ -1724,7 +1744,7 @@ int launch_blend_fwd_own(const dsx_camera& cam, int64_t n, const uint32_t* depth
         DSX_TIMED("blend_fwd_kernel", stream);
         hipLaunchKernelGGL(blend_fwd_wide_kernel<true>, dim3(lg.tiles()), dim3(kWideThreads), 0, stream, nullptr, nullptr,
                            reinterpret_cast<const float4*>(splats), image, nullptr, nullptr, cam.image_width, cam.image_height, lg.ntx,
-                           (uint32_t)(n - 1), 0, nullptr, 0, nullptr, nullptr, nullptr, (int64_t)0, nullptr, cam.bg,
+                           (uint32_t)(n - 1), 0, nullptr, 0, nullptr, nullptr, nullptr, (int64_t)0, nullptr, 0, cam.bg,
                            camera_flag(cam, DSX_PLANAR_IMAGE), OwnLists{depth_keys, rects, (int)n});
     }
     DSX_LAUNCH_CHECK();
@@ -1780,14 +1800,15 @@ int launch_blend_fwd(const dsx_camera& cam, int64_t n, int64_t k, int32_t* range
         const bool wide = forced_pixels_per_lane() == 0 && lg.shift == 0 && ntx * nty <= kFwdWideUpTo;
         const dim3 grid(ntx * nty);
         const float4* sp = reinterpret_cast<const float4*>(splats);
+        const int prep_zeros = prep_marks != nullptr && zeros_alone(cam, n);
         if(wide)
             hipLaunchKernelGGL(blend_fwd_wide_kernel<false>, grid, dim3(kWideThreads), 0, stream, ranges, sorted_ids, sp, image, final_T,
                                final_idx, cam.image_width, cam.image_height, ntx, last_id, (int)k, header, lg.shift, sort_flag_a,
-                               sort_flag_b, prep, prep_count, prep_marks, cam.bg, camera_flag(cam, DSX_PLANAR_IMAGE), OwnLists{});
+                               sort_flag_b, prep, prep_count, prep_marks, prep_zeros, cam.bg, camera_flag(cam, DSX_PLANAR_IMAGE), OwnLists{});
 #define DSX_LAUNCH_FWD(KERNEL, THREADS)                                                                          \
     hipLaunchKernelGGL((KERNEL), grid, dim3(THREADS), 0, stream, ranges, sorted_ids, sp, image, final_T, final_idx,  \
                        cam.image_width, cam.image_height, ntx, last_id, (int)k, header, lg.shift, sort_flag_a,     \
-                       sort_flag_b, prep, prep_count, prep_marks, cam.bg, camera_flag(cam, DSX_PLANAR_IMAGE), L)
+                       sort_flag_b, prep, prep_count, prep_marks, prep_zeros, cam.bg, camera_flag(cam, DSX_PLANAR_IMAGE), L)
         else if(four && lg.shift)
             DSX_LAUNCH_FWD(blend_fwd_kernel<true>, DSX_WAVE);
         else if(four)

@@ -228,7 +228,7 @@ struct ListGrid
 };
 // list_bin: 0: choose by image size; 1, 2, 4, 8: bins of that many tiles a side (dsx_camera::list_bin)
 ListGrid list_grid(int image_width, int image_height, int list_bin);
-constexpr int kCameraFlags = DSX_VIEW_BY_COLUMNS | DSX_PROJ_BY_COLUMNS | DSX_PLANAR_IMAGE;
+constexpr int kCameraFlags = DSX_VIEW_BY_COLUMNS | DSX_PROJ_BY_COLUMNS | DSX_PLANAR_IMAGE | DSX_PREPARE_ZEROS;
 inline int camera_bin(const dsx_camera& cam)
 {
     return cam.list_bin & ~kCameraFlags;
@@ -430,12 +430,28 @@ int launch_blend_bwd(const dsx_camera& cam, int64_t n, int64_t k, const int32_t*
                      const float* splats, const float* final_T, const int32_t* final_idx, const float* v_image,
                      float* grads, hipStream_t stream, bool check_header, bool grads_prepared = false,
                      bool with_marks = false, const ZeroJobs* zeros = nullptr);
+// Is the accumulator prepared without the conics (DSX_PREPARE_ZEROS)?  Reading them costs the forward time only where there are
+// many: us with them -> without, the forward and the per-Gaussian backward: 300 K Gaussians 112 -> 112 and 14.4 -> 15.9, 500 K 115 -> 116 and
+// 13.9 -> 14.9, 1.4 M 258 -> 255 and 46.5 -> 47.3, 2 M faint 660 -> 636 and 128 -> 130, 3 M 156 -> 126 and 20.3 -> 20.1.
+constexpr int64_t kZerosAloneFrom = 1000000;
+inline bool zeros_alone(const dsx_camera& cam, int64_t n)
+{
+    return n >= kZerosAloneFrom && camera_flag(cam, DSX_PREPARE_ZEROS);
+}
+// where the per-Gaussian backward finds the conics: in the splat records, in places 9..11 of the accumulator's (dsx_forward_finish put them
+// there), or worked out again, with the projection's own routines (same bits), from what it reads anyway
+enum class ConicFrom
+{
+    kSplats,
+    kGrads,
+    kInputs
+};
 int launch_gaussian_bwd(const dsx_camera& cam, int64_t n, int num_bases, const float* means3d,
                         const float* scales, const float* quats, const float* splats,
                         const float* cov3d, const int32_t* radii, const float* grads,
                         float* v_mean3d, float* v_means2d, float* v_shs, float* v_colors,
                         float* v_opacity, float* v_scale, float* v_quat, float* v_cov3d,
-                        hipStream_t stream, bool conic_in_grads = false, bool outputs_cleared = false,
+                        hipStream_t stream, ConicFrom conic_from = ConicFrom::kSplats, bool outputs_cleared = false,
                         bool with_marks = false);
 // zeros in every output of launch_gaussian_bwd that is not null (it writes only the Gaussians that
 // have something to propagate; outputs_cleared tells it that this has been done)
@@ -530,6 +546,85 @@ __device__ __forceinline__ void cov3d_from_scale_rot(const float* sc, float4 q, 
     out[3] = m10 * m10 + m11 * m11 + m12 * m12;
     out[4] = m10 * m20 + m11 * m21 + m12 * m22;
     out[5] = m20 * m20 + m21 * m21 + m22 * m22;
+}
+
+// The EWA covariance on the image of a 3-D covariance at view position (vx, vy, vz), 0.3 on its diagonal: cpp/rasterizer_kernels.cu:174-231
+// (sums start from 0 and add the three products in index order, zero Jacobian entries included).  V: the view matrix's first three rows.
+struct Cov2d
+{
+    float a, b, c; // xx, xy, yy
+};
+__device__ __forceinline__ Cov2d ewa_cov2d(const float (&V)[12], float vx, float vy, float vz, const float (&c3)[6], float focal_x,
+                                           float focal_y, float tanfovx, float tanfovy)
+{
+#pragma clang fp contract(off) // same bits in every translation unit
+    const float limx = 1.3f * tanfovx;
+    const float limy = 1.3f * tanfovy;
+    const float txtz = vx / vz;
+    const float tytz = vy / vz;
+    const float t0 = fminf(limx, fmaxf(-limx, txtz)) * vz;
+    const float t1 = fminf(limy, fmaxf(-limy, tytz)) * vz;
+    const float t2 = vz;
+    const float J[3][3] = {{focal_x / t2, 0.0f, -(focal_x * t0) / (t2 * t2)},
+                           {0.0f, focal_y / t2, -(focal_y * t1) / (t2 * t2)},
+                           {0.0f, 0.0f, 0.0f}};
+    const float Wm[3][3] = {{V[0], V[4], V[8]}, {V[1], V[5], V[9]}, {V[2], V[6], V[10]}};
+    float T[3][3];
+#pragma unroll
+    for(int a = 0; a < 3; ++a)
+#pragma unroll
+        for(int b = 0; b < 3; ++b)
+        {
+            float acc = 0.0f;
+#pragma unroll
+            for(int k = 0; k < 3; ++k)
+                acc += Wm[a][k] * J[b][k];
+            T[a][b] = acc;
+        }
+    const float S3[3][3] = {{c3[0], c3[1], c3[2]}, {c3[1], c3[3], c3[4]}, {c3[2], c3[4], c3[5]}};
+    float tmp[3][3];
+#pragma unroll
+    for(int a = 0; a < 3; ++a)
+#pragma unroll
+        for(int b = 0; b < 3; ++b)
+        {
+            float acc = 0.0f;
+#pragma unroll
+            for(int k = 0; k < 3; ++k)
+                acc += T[k][a] * S3[k][b];
+            tmp[a][b] = acc;
+        }
+    float cov[2][2];
+#pragma unroll
+    for(int a = 0; a < 2; ++a)
+#pragma unroll
+        for(int b = 0; b < 2; ++b)
+        {
+            float acc = 0.0f;
+#pragma unroll
+            for(int k = 0; k < 3; ++k)
+                acc += tmp[a][k] * T[k][b];
+            cov[a][b] = acc;
+        }
+    return {cov[0][0] + 0.3f, cov[0][1], cov[1][1] + 0.3f};
+}
+// view position (cpp/rasterizer_kernels.cu:325-330), determinant and conic (cpp/rasterizer_kernels.cu:49-55)
+__device__ __forceinline__ float3 view_position(const float (&V)[12], const float3 mean)
+{
+#pragma clang fp contract(off)
+    return make_float3(V[0] * mean.x + V[1] * mean.y + V[2] * mean.z + V[3], V[4] * mean.x + V[5] * mean.y + V[6] * mean.z + V[7],
+                       V[8] * mean.x + V[9] * mean.y + V[10] * mean.z + V[11]);
+}
+__device__ __forceinline__ float det_of(const Cov2d& cov)
+{
+#pragma clang fp contract(off)
+    return cov.a * cov.c - cov.b * cov.b;
+}
+__device__ __forceinline__ float3 conic_of(const Cov2d& cov, float det)
+{
+#pragma clang fp contract(off)
+    const float det_inv = 1.0f / (det + 1e-6f);
+    return make_float3(cov.c * det_inv, -cov.b * det_inv, cov.a * det_inv);
 }
 
 // float -> int32 with the hardware conversion's semantics made explicit (saturate, NaN -> 0).

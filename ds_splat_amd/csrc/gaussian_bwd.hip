@@ -44,7 +44,8 @@ struct GaussianBwdParams
     float* v_cov3d;
     float fx, fy, glob;
     int sh_degree, num_bases;
-    int conic_in_grads; // the accumulator's places 9..11 hold the conic (the forward put it there)
+    ConicFrom conic_from;
+    float fwd_fx, fwd_fy, tanfovx, tanfovy; // the projection's, for ConicFrom::kInputs
     int run;            // Gaussians per workgroup: a multiple of the wavefront, at most kBwdListMax
 };
 
@@ -148,8 +149,10 @@ __device__ __forceinline__ GaussianBwdInputs load_inputs(const GaussianBwdParams
         const float2 c01 = cs[0], c23 = cs[1], c45 = cs[2];
         in.c3[0] = c01.x, in.c3[1] = c01.y, in.c3[2] = c23.x, in.c3[3] = c23.y, in.c3[4] = c45.x, in.c3[5] = c45.y;
     }
-    // the conic: behind the sums when the forward prepared the accumulator, else from the splat record
-    in.conic = p.conic_in_grads ? make_float4(in.g2.y, in.g2.z, in.g2.w, 0.f) : p.splats[3 * i + 1];
+    if(p.conic_from == ConicFrom::kGrads)
+        in.conic = make_float4(in.g2.y, in.g2.z, in.g2.w, 0.f);
+    else if(p.conic_from == ConicFrom::kSplats)
+        in.conic = p.splats[3 * i + 1];
     return in;
 }
 
@@ -247,10 +250,29 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(3, 3))
                     for(int c = 0; c < 3; ++c)
                         vm[c] = R[0][c] * vv[0] + R[1][c] * vv[1] + R[2][c] * vv[2];
                 }
+                // the covariance the forward projected: stored by it, or rebuilt here from scale and
+                // rotation with the forward's own routine (same bits; 24 bytes per Gaussian less to
+                // write there and to read here)
+                float c3[6];
+                if(p.cov3d)
+                {
+#pragma unroll
+                    for(int c = 0; c < 6; ++c)
+                        c3[c] = in.c3[c];
+                }
+                else
+                    cov3d_from_scale_rot(in.sc, in.quat, p.glob, c3);
                 // conic -> cov2d:  v_Sigma = -X G X, X = conic, G = symmetrised v_conic
                 float v_cov2d[3];
                 {
-                    const float4 q1 = in.conic;
+                    float4 q1 = in.conic;
+                    if(p.conic_from == ConicFrom::kInputs)
+                    {
+                        const float3 view = view_position(V, mean);
+                        const Cov2d cov = ewa_cov2d(V, view.x, view.y, view.z, c3, p.fwd_fx, p.fwd_fy, p.tanfovx, p.tanfovy);
+                        const float3 conic = conic_of(cov, det_of(cov));
+                        q1 = make_float4(conic.x, conic.y, conic.z, 0.f);
+                    }
                     const float X[2][2] = {{q1.x, q1.y}, {q1.y, q1.z}};
                     const float G[2][2] = {{vc[0], 0.5f * vc[1]}, {0.5f * vc[1], vc[2]}};
                     float M[2][2], N[2][2];
@@ -279,18 +301,6 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(3, 3))
 #pragma unroll
                         for(int c = 0; c < 3; ++c)
                             T[r][c] = J[r][0] * R[0][c] + J[r][1] * R[1][c] + J[r][2] * R[2][c];
-                    // the covariance the forward projected: stored by it, or rebuilt here from scale and
-                    // rotation with the forward's own routine (same bits; 24 bytes per Gaussian less to
-                    // write there and to read here)
-                    float c3[6];
-                    if(p.cov3d)
-                    {
-#pragma unroll
-                        for(int c = 0; c < 6; ++c)
-                            c3[c] = in.c3[c];
-                    }
-                    else
-                        cov3d_from_scale_rot(in.sc, in.quat, p.glob, c3);
                     const float S[3][3] = {{c3[0], c3[1], c3[2]}, {c3[1], c3[3], c3[4]}, {c3[2], c3[4], c3[5]}};
                     const float Gc[2][2] = {{v_cov2d[0], 0.5f * v_cov2d[1]}, {0.5f * v_cov2d[1], v_cov2d[2]}};
                     // GT = Gc T (2x3)
@@ -512,7 +522,7 @@ int launch_gaussian_bwd(const dsx_camera& cam, int64_t n, int num_bases, const f
                         const float* quats, const float* splats, const float* cov3d, const int32_t* radii,
                         const float* grads, float* v_mean3d, float* v_means2d, float* v_shs, float* v_colors,
                         float* v_opacity, float* v_scale, float* v_quat, float* v_cov3d, hipStream_t stream,
-                        bool conic_in_grads, bool outputs_cleared, bool with_marks)
+                        ConicFrom conic_from, bool outputs_cleared, bool with_marks)
 {
     if(n == 0)
         return DSX_OK;
@@ -551,7 +561,11 @@ int launch_gaussian_bwd(const dsx_camera& cam, int64_t n, int num_bases, const f
     p.glob = cam.scale_modifier;
     p.sh_degree = cam.sh_degree;
     p.num_bases = num_bases;
-    p.conic_in_grads = conic_in_grads ? 1 : 0;
+    p.conic_from = conic_from;
+    p.fwd_fx = cam.image_width / (2 * cam.tanfovx);
+    p.fwd_fy = cam.image_height / (2 * cam.tanfovy);
+    p.tanfovx = cam.tanfovx;
+    p.tanfovy = cam.tanfovy;
     // runs that make all workgroups resident at once, if the list can hold such a run
     const int64_t resident = (int64_t)compute_units() * kBwdResidentPerCu;
     const int64_t even = ((n + resident - 1) / resident + DSX_WAVE - 1) / DSX_WAVE * DSX_WAVE;

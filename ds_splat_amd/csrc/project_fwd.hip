@@ -303,63 +303,11 @@ __global__ __launch_bounds__(kProjBlock) void project_fwd_kernel(const ProjectPa
         // view-space position (cpp/rasterizer_kernels.cu:325-330)
         float V[12];
         load_matrix(p.view, p.view_transposed, V);
-        const float vx = V[0] * mean.x + V[1] * mean.y + V[2] * mean.z + V[3];
-        const float vy = V[4] * mean.x + V[5] * mean.y + V[6] * mean.z + V[7];
-        const float vz = V[8] * mean.x + V[9] * mean.y + V[10] * mean.z + V[11];
+        const float3 view = view_position(V, mean);
+        const float vx = view.x, vy = view.y, vz = view.z;
 
-        // EWA covariance (cpp/rasterizer_kernels.cu:174-231): sums start from 0 and add the
-        // three products in index order, zero Jacobian entries included
-        const float limx = 1.3f * p.tanfovx;
-        const float limy = 1.3f * p.tanfovy;
-        const float txtz = vx / vz;
-        const float tytz = vy / vz;
-        const float t0 = fminf(limx, fmaxf(-limx, txtz)) * vz;
-        const float t1 = fminf(limy, fmaxf(-limy, tytz)) * vz;
-        const float t2 = vz;
-        const float J[3][3] = {{p.focal_x / t2, 0.0f, -(p.focal_x * t0) / (t2 * t2)},
-                               {0.0f, p.focal_y / t2, -(p.focal_y * t1) / (t2 * t2)},
-                               {0.0f, 0.0f, 0.0f}};
-        const float Wm[3][3] = {{V[0], V[4], V[8]}, {V[1], V[5], V[9]}, {V[2], V[6], V[10]}};
-        float T[3][3];
-#pragma unroll
-        for(int a = 0; a < 3; ++a)
-#pragma unroll
-            for(int b = 0; b < 3; ++b)
-            {
-                float acc = 0.0f;
-#pragma unroll
-                for(int k = 0; k < 3; ++k)
-                    acc += Wm[a][k] * J[b][k];
-                T[a][b] = acc;
-            }
-        const float S3[3][3] = {{c3[0], c3[1], c3[2]}, {c3[1], c3[3], c3[4]}, {c3[2], c3[4], c3[5]}};
-        float tmp[3][3];
-#pragma unroll
-        for(int a = 0; a < 3; ++a)
-#pragma unroll
-            for(int b = 0; b < 3; ++b)
-            {
-                float acc = 0.0f;
-#pragma unroll
-                for(int k = 0; k < 3; ++k)
-                    acc += T[k][a] * S3[k][b];
-                tmp[a][b] = acc;
-            }
-        float cov[2][2];
-#pragma unroll
-        for(int a = 0; a < 2; ++a)
-#pragma unroll
-            for(int b = 0; b < 2; ++b)
-            {
-                float acc = 0.0f;
-#pragma unroll
-                for(int k = 0; k < 3; ++k)
-                    acc += tmp[a][k] * T[k][b];
-                cov[a][b] = acc;
-            }
-        const float ca = cov[0][0] + 0.3f;
-        const float cb = cov[0][1];
-        const float cc = cov[1][1] + 0.3f;
+        const Cov2d cov = ewa_cov2d(V, vx, vy, vz, c3, p.focal_x, p.focal_y, p.tanfovx, p.tanfovy);
+        const float ca = cov.a, cc = cov.c;
 
         // pixel mean (cpp/rasterizer_kernels.cu:332-337)
         const float z_inv = 1.0f / (vz + 1e-6f);
@@ -367,7 +315,7 @@ __global__ __launch_bounds__(kProjBlock) void project_fwd_kernel(const ProjectPa
         const float py = p.focal_y * vy * z_inv + p.c_y;
 
         // radius = ceil(3 sigma_max), zero when culled (cpp/rasterizer_kernels.cu:163-172)
-        const float det = ca * cc - cb * cb;
+        const float det = det_of(cov);
         const float mid = 0.5f * (ca + cc);
         const float diff = mid * mid - det;
         const float root = sqrtf(fmaxf(0.1f, diff));
@@ -379,12 +327,11 @@ __global__ __launch_bounds__(kProjBlock) void project_fwd_kernel(const ProjectPa
         const TileRect r = tile_rect(px, py, radius, p.ntx, p.nty);
         const int tiles = (r.ex - r.sx) * (r.ey - r.sy) * (radius > 0 ? 1 : 0);
 
-        // conic (cpp/rasterizer_kernels.cu:49-55)
-        const float det_inv = 1.0f / (det + 1e-6f);
+        const float3 conic = conic_of(cov, det);
 
         float4* rec = p.splats + 3 * i;
         rec[0] = make_float4(px, py, vz, __int_as_float(radius));
-        rec[1] = make_float4(cc * det_inv, -cb * det_inv, ca * det_inv, opacity);
+        rec[1] = make_float4(conic.x, conic.y, conic.z, opacity);
         rec[2] = make_float4(rgb.x, rgb.y, rgb.z, __int_as_float(tiles));
         p.radii[i] = radius;
 

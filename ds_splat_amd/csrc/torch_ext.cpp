@@ -116,7 +116,7 @@ Camera make_camera(const Settings& s, const at::Device& dev, const float* kept_v
     require(s.list_bin == 0 || s.list_bin == 1 || s.list_bin == 2 || s.list_bin == 4 || s.list_bin == 8,
             "list_bin must be 0 (the library's choice), 1, 2, 4 or 8 tiles a side");
     cam.c.list_bin = (int32_t)s.list_bin | (view_by_columns ? DSX_VIEW_BY_COLUMNS : 0) |
-                     (proj_by_columns ? DSX_PROJ_BY_COLUMNS : 0) | (s.planar ? DSX_PLANAR_IMAGE : 0);
+                     (proj_by_columns ? DSX_PROJ_BY_COLUMNS : 0) | (s.planar ? DSX_PLANAR_IMAGE : 0) | DSX_PREPARE_ZEROS;
     cam.bin = (int32_t)s.list_bin;
     cam.planar = s.planar;
     return cam;

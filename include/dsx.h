@@ -78,6 +78,9 @@ typedef struct dsx_camera
 #define DSX_PROJ_BY_COLUMNS 0x200 /* the same for `proj`                                                  */
 #define DSX_PLANAR_IMAGE 0x400    /* image and v_image are [3,H,W] and the image has final_T * bg added;
                                      without: [H,W,3], the background is not composited                   */
+#define DSX_PREPARE_ZEROS 0x800   /* the accumulator that dsx_forward_finish prepares may be zeros alone, without
+                                     the conics (where n is large); dsx_backward is called with the same flag
+                                     and then works them out again from its inputs                        */
 
 /*
  * Projected record ("splat"), one per Gaussian, DSX_SPLAT_FLOATS floats:
@@ -96,7 +99,7 @@ typedef struct dsx_camera
  */
 
 const char* dsx_error_string(int status);
-/* 100 * major + minor.  312: dsx_render.  311: dsx_depth_order_bounded.  310: flags beside dsx_camera::list_bin, the projection's wait for the pair
+/* 100 * major + minor.  313: DSX_PREPARE_ZEROS.  312: dsx_render.  311: dsx_depth_order_bounded.  310: flags beside dsx_camera::list_bin, the projection's wait for the pair
  * counts is a function of its own.  300: the bin size of the tile lists is an argument (dsx_camera::list_bin and
  * the size helpers) instead of a process-wide setting; the `ranges` buffer carries it in a header word;
  * the blend entry points and the backward are told n and k and follow no id or list position beyond

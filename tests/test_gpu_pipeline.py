@@ -5,8 +5,8 @@ import pytest
 import torch
 
 from ds_splat_amd.synthetic import make_scene
-from helpers import (GRAD_KEYS, arrays, check_grads_against_bounds, comparable_gaussians, scene_settings,
-                     set_camera)
+from helpers import (CAMERAS, GRAD_KEYS, arrays, check_grads_against_bounds, comparable_gaussians,
+                     scene_settings, set_camera)
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -915,3 +915,45 @@ def test_stage_entry_points_chain_on_binned_lists(oracle, bins):
     err = np.abs(grads.cpu().numpy()[:, :9].astype(np.float64) - want)[gok]
     bound = (1e-4 * Bb["abs_sums"].astype(np.float64) + 1e-7)[gok]
     assert gok.mean() > 0.5 and (err <= bound).all(), float((err / bound).max())
+
+
+@pytest.mark.parametrize("camera", sorted(CAMERAS))
+@pytest.mark.parametrize("given", [False, True])
+def test_conics_that_the_backward_works_out_again(camera, given):
+    """An accumulator prepared without the conics (DSX_PREPARE_ZEROS, from a million Gaussians on): the per-Gaussian
+    backward's outputs are bit for bit those that it has from the projection's conics, with covariances given or not."""
+    import ctypes as C
+    from ds_splat_amd import _native as N
+    from ds_splat_amd import stages
+    n = 1_000_037
+    sc = set_camera(make_scene("cfg1", n=n, width=70, height=52, sh_degree=1, seed=3), camera)
+    t = {k: (v.to(DEV) if isinstance(v, torch.Tensor) else v) for k, v in sc.items()}
+    cam = stages.camera_from_scene(sc, DEV, list_bin=1)
+    args = t["means_3d"], t["scales"], t["rotations"]
+    _, st = stages.forward(cam, *args, t["opacities"], t["shs"])
+    visible = st.radii > 0
+    assert int(visible.sum()) > 1000
+    sums = torch.randn(n, 9, generator=torch.Generator().manual_seed(4)).to(DEV)
+    st.lists[cam.num_tiles + 1] = 3     # (lists of another bin size are not walked: the sums stay what they are)
+    lib, p = N.load(), lambda x: C.c_void_p(x.data_ptr()) if x is not None else None
+    outs = []
+    for flag in (0, 0x800):
+        grads = stages.new_accumulator(n, DEV)
+        records, marks = stages.accumulator_views(grads, n)
+        records[:, :9] = sums
+        records[:, 9:] = float("nan") if flag else st.splats[:, 4:7]
+        marks.fill_(1)
+        o = {k: torch.full((n, w), float("nan"), device=DEV) for k, w in
+             (("mean", 3), ("means2d", 3), ("shs", 48), ("colors", 3), ("opacity", 1), ("scale", 3), ("quat", 4), ("cov3d", 6))}
+        N.check(lib.dsx_backward(cam.with_list_bin(1 | flag).ref, n, st.num_keys, 16, p(args[0]), None if given else p(args[1]),
+                                 None if given else p(args[2]), p(st.splats), p(st.cov3d) if given else None, p(st.radii),
+                                 p(st.lists), p(st.sorted_ids), p(st.final_T), p(st.final_idx), p(t["v_image"]), p(grads), 1,
+                                 *(None if given and k in ("scale", "quat") else p(o[k]) for k in o),
+                                 C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+        torch.cuda.synchronize()
+        outs.append(o)
+    for k in outs[0]:
+        if not (given and k in ("scale", "quat")):
+            a, b = (o[k].view(torch.int32) for o in outs)
+            assert torch.equal(a, b), k
+    assert bool((outs[1]["cov3d"][visible] != 0).any())
