@@ -149,11 +149,12 @@ extern "C" int32_t dsx_sort_passes(int32_t num_tiles)
 
 extern "C" size_t dsx_workspace_bytes(int64_t n, int64_t k, int32_t width, int32_t height, int32_t list_bin)
 {
-    (void)n;
+    (void)n; // (whatever the number of Gaussians: one wide digit's workspace is the larger one)
     if(!valid_list_bin(list_bin))
         return 0;
     const ListGrid lg = list_grid(width, height, list_bin);
-    return lists_workspace(k < 0 ? 0 : k, lg.lists(), lg.shift != 0).bytes;
+    return std::max(lists_workspace(0, k < 0 ? 0 : k, lg.lists(), lg.shift != 0).bytes,
+                    lists_workspace(INT64_MAX, k < 0 ? 0 : k, lg.lists(), lg.shift != 0).bytes);
 }
 
 extern "C" int32_t dsx_list_bin(int32_t width, int32_t height, int32_t list_bin)
@@ -417,8 +418,8 @@ extern "C" int dsx_sort_flags(int64_t n, int64_t k, int32_t width, int32_t heigh
         {
             const ListGrid lg = list_grid(width, height, list_bin);
             const int tiles = lg.lists();
-            const ListsWorkspace lw = lists_workspace(k, tiles, lg.shift != 0);
-            const Sort32Workspace w = sort32_workspace(k, slot_bits(tiles), sort32_tile_keys(k));
+            const ListsWorkspace lw = lists_workspace(n, k, tiles, lg.shift != 0);
+            const Sort32Workspace w = sort32_workspace(k, slot_bits(tiles), sort32_tile_keys(k), one_wide_digit(slot_bits(tiles), n));
             *partition_flag =
                 reinterpret_cast<const uint32_t*>(static_cast<const char*>(workspace) + lw.sort + w.counters) + w.passes;
         }
@@ -439,7 +440,7 @@ extern "C" int dsx_tile_lists(const dsx_camera* cam, int64_t n, int64_t k, const
     {
         if(!order || !sorted_ids || !workspace)
             return DSX_ERR_BAD_ARG;
-        if(workspace_bytes < lists_workspace(k, list_grid(*cam).lists(), list_grid(*cam).shift != 0).bytes)
+        if(workspace_bytes < lists_workspace(n, k, list_grid(*cam).lists(), list_grid(*cam).shift != 0).bytes)
             return DSX_ERR_WORKSPACE;
     }
     return launch_tile_lists(*cam, n, k, order, sorted_ids, ranges, workspace, as_stream(stream));
@@ -832,7 +833,7 @@ extern "C" int dsx_forward_core(const float* means3d, const float* shs, const fl
     char* buf2 = nullptr;
     if(rc == DSX_OK)
     {
-        const size_t ws = lists_workspace(k, list_grid(cam).lists(), list_grid(cam).shift != 0).bytes;
+        const size_t ws = lists_workspace(n, k, list_grid(cam).lists(), list_grid(cam).shift != 0).bytes;
         const size_t o_ids = align(ws);
         if(hipMallocAsync(reinterpret_cast<void**>(&buf2), o_ids + (size_t)dsx_sorted_ids_count(k, image_width, image_height, 0) * 4 + 256, s) != hipSuccess)
             rc = DSX_ERR_RUNTIME;

@@ -154,6 +154,33 @@ inline Digits32 digits32(int key_bits)
     }
     return d;
 }
+// The digits of the partition by list: one of nine to eleven bits instead of two.  A pass over few pairs lasts as long as one tile's
+// serial work and the chain, whatever its digits; a wide digit costs LDS for the wavefronts' counts (64 KB at eleven bits: one workgroup
+// on a compute unit instead of two) and statuses (8 KB a tile), which many pairs feel.  us of a forward, two digits -> one, with little and with
+// much overlap:
+//   Gaussians                  4 K               30 K             130 K              300 K              1 M            3 M
+//   9 bits   (420 tiles)   42 -> 37, 44 -> 40  56 -> 50, 79 -> 72  109 -> 101, 98 -> 90  156 -> 145, 126 -> 113  198 -> 185  376 -> 360
+//   10 bits  (750 tiles)   41 -> 37, 45 -> 42  54 -> 51, 79 -> 75  95 -> 90, 102 -> 95   144 -> 140, 129 -> 121  196 -> 187  384 -> 377
+//   11 bits (1024 tiles)   41 -> 38, 46 -> 44  55 -> 52, 81 -> 77  98 -> 94, 107 -> 100  152 -> 154, 142 -> 148  201 -> 196  401 -> 398
+//   11 bits (1936 tiles)   46 -> 43, 52 -> 49  60 -> 56, 90 -> 86  98 -> 94, 122 -> 114  152 -> 153, 166 -> 168  222 -> 222  427 -> 433
+//   11 bits (2040 bins, 6 M Gaussians at 3840x2160) 932 -> 936
+constexpr int kWideBits = 11, kWideAlways = 10;
+constexpr int64_t kWideUpTo = 131072; // Gaussians
+inline bool one_wide_digit(int slot_bits, int64_t n)
+{
+    return slot_bits > kBits32 && slot_bits <= (n <= kWideUpTo ? kWideBits : kWideAlways);
+}
+inline Digits32 partition_digits(int slot_bits, int64_t n)
+{
+    Digits32 d = digits32(slot_bits);
+    if(one_wide_digit(slot_bits, n))
+    {
+        d.passes = 1;
+        d.mask[0] = (1u << slot_bits) - 1u;
+        d.mask[1] = 0u;
+    }
+    return d;
+}
 // The depth sort of a whole forward: the keys' distances from the smallest one, in three digits of up to nine bits
 // instead of four of eight, wherever they fit 27 bits (depths within sixteen octaves of each other, all of one sign).
 // The range comes from the device (rounded outwards to 16 bits), so the host waits for it between the projection
@@ -287,7 +314,8 @@ struct Sort32Workspace
     int passes;
     int64_t tiles;
 };
-Sort32Workspace sort32_workspace(int64_t count, int key_bits, int tile_keys);
+// wide: one pass whatever the number of bits (one_wide_digit)
+Sort32Workspace sort32_workspace(int64_t count, int key_bits, int tile_keys, bool wide = false);
 
 // Per-Gaussian buffer that carries the depth order from the projection to the tile lists.
 struct OrderLayout
@@ -327,7 +355,7 @@ struct ListsWorkspace
     int passes;
 };
 // binned: lists per bin (32-bit slot words that carry the tile masks and end in the caller's buffer)
-ListsWorkspace lists_workspace(int64_t k, int num_tiles, bool binned);
+ListsWorkspace lists_workspace(int64_t n, int64_t k, int num_tiles, bool binned);
 
 // launchers (each returns a dsx_status)
 // Five words of pinned host memory that receive a call's pair counts, the range of its depth keys, how many of them emit and whether

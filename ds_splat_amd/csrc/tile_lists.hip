@@ -264,16 +264,20 @@ __device__ __forceinline__ void onesweep32_pass(
     const uint2* __restrict__ gather_src = rects.gather_src;
     uint2* __restrict__ gather_dst = rects.gather_dst;
     constexpr int kBins = 1 << kBits;
+    // digits of a thread, side by side (two from eleven bits on; their statuses are one 64-bit word then, so both are there or neither)
+    constexpr int kOwn = kBins > kSort32Threads ? kBins / kSort32Threads : 1;
+    constexpr int kOwners = kBins / kOwn;
+    static_assert(kOwn <= 2 && (kOwn == 1 || !kFirst), "a status word");
     constexpr int kSort32Tile = kSort32Threads * kSort32Items;
     constexpr int kSort32Waves = kSort32Threads / DSX_WAVE;
     __shared__ uint32_t s_keys[kSort32Tile]; // reused for the values in the second round
-    __shared__ uint16_t s_whist[kSort32Waves][kBins];
+    __shared__ __attribute__((aligned(16))) uint16_t s_whist[kSort32Waves][kBins];
     __shared__ uint32_t s_digit_start[kBins];
     __shared__ uint32_t s_before[kFirst ? kBins / DSX_WAVE : 1]; // keys of the tiles before, by the digits' wavefronts
     __shared__ uint32_t s_none[kFirst ? kSort32Waves : 1];       // this tile's keys without pairs, by wavefront
     __shared__ uint32_t s_gbase[kBins];
-    __shared__ __attribute__((aligned(16))) uint32_t s_wave_tot[kBins / DSX_WAVE];
-    __shared__ __attribute__((aligned(16))) uint32_t s_hist_tot[kBins / DSX_WAVE];
+    __shared__ __attribute__((aligned(16))) uint32_t s_wave_tot[kOwners / DSX_WAVE];
+    __shared__ __attribute__((aligned(16))) uint32_t s_hist_tot[kOwners / DSX_WAVE];
     __shared__ uint32_t s_tile;
 
     const int tid = threadIdx.x;
@@ -282,8 +286,8 @@ __device__ __forceinline__ void onesweep32_pass(
 
     if(tid == 0)
         s_tile = atomicAdd(tile_counter, 1u);
-    for(int j = tid; j < kSort32Waves * kBins; j += kSort32Threads)
-        (&s_whist[0][0])[j] = 0;
+    for(int j = tid; j < kSort32Waves * kBins / 8; j += kSort32Threads)
+        reinterpret_cast<uint4*>(&s_whist[0][0])[j] = make_uint4(0, 0, 0, 0);
     __syncthreads();
     const int64_t tile = s_tile;
     const int64_t tile_base = tile * kSort32Tile;
@@ -353,41 +357,68 @@ __device__ __forceinline__ void onesweep32_pass(
     __syncthreads();
 
     // ---- per-digit totals of the tile (thread d <-> digit d), wave offsets, digit starts ----
-    const bool digit_thread = tid < kBins; // thread d owns digit d (bins above the mask stay empty)
-    uint32_t total = 0;
-    uint32_t hist_excl = 0;
-    uint32_t* my_status = status + tile * kBins + (digit_thread ? tid : 0);
+    const bool digit_thread = tid < kOwners; // thread d owns digit d (bins above the mask stay empty)
+    const int digit0 = kOwn * tid;
+    uint32_t total[kOwn] = {};
+    uint32_t hist_excl[kOwn] = {};
+    auto store_status = [&](const uint32_t (&counts)[kOwn], uint32_t flag) {
+        uint32_t* const mine = status + tile * kBins + digit0;
+        if constexpr(kOwn == 2)
+            __hip_atomic_store(reinterpret_cast<unsigned long long*>(mine),
+                               (unsigned long long)(counts[1] | flag) << 32 | (counts[0] | flag), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else
+            __hip_atomic_store(mine, counts[0] | flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
     if(digit_thread)
     {
 #pragma unroll
         for(int w = 0; w < kSort32Waves; ++w)
+#pragma unroll
+            for(int q = 0; q < kOwn; ++q)
+            {
+                const uint32_t c = s_whist[w][digit0 + q];
+                s_whist[w][digit0 + q] = (uint16_t)total[q];
+                total[q] += c;
+            }
+        store_status(total, tile == 0 ? kFlagInclusive32 : kFlagAggregate32);
+        uint32_t sum = 0, hsum = 0, hcount[kOwn];
+#pragma unroll
+        for(int q = 0; q < kOwn; ++q)
         {
-            const uint32_t c = s_whist[w][tid];
-            s_whist[w][tid] = (uint16_t)total;
-            total += c;
+            // the digit's place in the whole output: exclusive scan of the pass's histogram (every
+            // tile redoes this scan; that is cheaper than a kernel launch of its own)
+            hcount[q] = hist_counts[digit0 + q];
+            sum += total[q];
+            hsum += hcount[q];
         }
-        __hip_atomic_store(my_status, total | (tile == 0 ? kFlagInclusive32 : kFlagAggregate32), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-        const uint32_t incl = wave_incl_scan32(total, lane);
+        const uint32_t incl = wave_incl_scan32(sum, lane);
         if(lane == 63)
             s_wave_tot[wave] = incl;
-        s_gbase[tid] = incl - total; // wave-local exclusive prefix, completed after the barrier
-        // the digit's place in the whole output: exclusive scan of the pass's histogram (every
-        // tile redoes this 256-entry scan; that is cheaper than a kernel launch of its own)
-        const uint32_t hcount = hist_counts[tid];
-        const uint32_t hincl = wave_incl_scan32(hcount, lane);
+        const uint32_t hincl = wave_incl_scan32(hsum, lane);
         if(lane == 63)
             s_hist_tot[wave] = hincl;
-        hist_excl = hincl - hcount;
+        uint32_t before = incl - sum, hbefore = hincl - hsum;
+#pragma unroll
+        for(int q = 0; q < kOwn; ++q)
+        {
+            s_gbase[digit0 + q] = before; // wave-local exclusive prefix, completed after the barrier
+            before += total[q];
+            hist_excl[q] = hbefore;
+            hbefore += hcount[q];
+        }
     }
     __syncthreads();
     if(digit_thread)
     {
         // totals of the digit wavefronts before this one
-        const uint32_t prefix = sum_of_waves_before<kBins / DSX_WAVE>(s_wave_tot, wave);
-        const uint32_t hprefix = sum_of_waves_before<kBins / DSX_WAVE>(s_hist_tot, wave);
-        s_digit_start[tid] = prefix + s_gbase[tid];
-        hist_excl += hprefix;
+        const uint32_t prefix = sum_of_waves_before<kOwners / DSX_WAVE>(s_wave_tot, wave);
+        const uint32_t hprefix = sum_of_waves_before<kOwners / DSX_WAVE>(s_hist_tot, wave);
+#pragma unroll
+        for(int q = 0; q < kOwn; ++q)
+        {
+            s_digit_start[digit0 + q] = prefix + s_gbase[digit0 + q];
+            hist_excl[q] += hprefix;
+        }
     }
     __syncthreads();
 
@@ -448,8 +479,8 @@ __device__ __forceinline__ void onesweep32_pass(
     // ---- chained scan over earlier tiles (decoupled look-back), one thread per digit -------
     if(digit_thread)
     {
-        uint32_t excl = 0;
-        if(tile > 0 && (uint32_t)tid <= mask) // bins above the mask are empty in every tile
+        uint32_t excl[kOwn] = {};
+        if(tile > 0 && (uint32_t)digit0 <= mask) // bins above the mask are empty in every tile
         {
             int64_t t = tile - 1; // next predecessor to account for
             int spins = 0;
@@ -458,20 +489,29 @@ __device__ __forceinline__ void onesweep32_pass(
                 *error_flag = 1u;
             while(!done)
             {
-                uint32_t v[kLookBatch32];
+                uint32_t v[kLookBatch32][kOwn];
 #pragma unroll
                 for(int b = 0; b < kLookBatch32; ++b)
                 {
                     // rows below tile 0 are read as tile 0, whose status is inclusive from the start
                     const int64_t row = t - b > 0 ? t - b : 0;
-                    v[b] = __hip_atomic_load(status + row * kBins + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    uint32_t* const theirs = status + row * kBins + digit0;
+                    if constexpr(kOwn == 2)
+                    {
+                        const unsigned long long both =
+                            __hip_atomic_load(reinterpret_cast<unsigned long long*>(theirs), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        v[b][0] = (uint32_t)both;
+                        v[b][kOwn - 1] = (uint32_t)(both >> 32);
+                    }
+                    else
+                        v[b][0] = __hip_atomic_load(theirs, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
 #pragma unroll
                 for(int b = 0; b < kLookBatch32; ++b)
                 {
                     if(done)
                         break;
-                    if((v[b] & kFlagMask32) == 0)
+                    if((v[b][0] & kFlagMask32) == 0)
                     {
                         if(++spins > polls)
                         {
@@ -482,19 +522,26 @@ __device__ __forceinline__ void onesweep32_pass(
                             __builtin_amdgcn_s_sleep(1);
                         break;
                     }
-                    excl += v[b] & kValueMask32;
+#pragma unroll
+                    for(int q = 0; q < kOwn; ++q)
+                        excl[q] += v[b][q] & kValueMask32;
                     --t;
-                    if(v[b] & kFlagInclusive32)
+                    if(v[b][0] & kFlagInclusive32)
                         done = true;
                 }
             }
-            __hip_atomic_store(my_status, ((excl + total) & kValueMask32) | kFlagInclusive32, __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
+            uint32_t all[kOwn];
+#pragma unroll
+            for(int q = 0; q < kOwn; ++q)
+                all[q] = (excl[q] + total[q]) & kValueMask32;
+            store_status(all, kFlagInclusive32);
         }
-        s_gbase[tid] = hist_excl + excl - s_digit_start[tid];
+#pragma unroll
+        for(int q = 0; q < kOwn; ++q)
+            s_gbase[digit0 + q] = hist_excl[q] + excl[q] - s_digit_start[digit0 + q];
         if(kFirst)
         {
-            const uint32_t before = wave_sum_u32(excl);
+            const uint32_t before = wave_sum_u32(excl[0]);
             if(lane == 0)
                 s_before[wave] = before;
         }
@@ -606,14 +653,15 @@ __global__ __launch_bounds__(kSortThreads32) __attribute__((amdgpu_waves_per_eu(
         range);
 }
 
-Sort32Workspace sort32_workspace(int64_t count, int key_bits, int tile_keys)
+Sort32Workspace sort32_workspace(int64_t count, int key_bits, int tile_keys, bool wide)
 {
     auto align = [](size_t x) { return (x + 255) & ~(size_t)255; };
     Sort32Workspace w;
-    w.passes = digits32(key_bits).passes;
+    w.passes = wide ? 1 : digits32(key_bits).passes;
     w.tiles = (count + tile_keys - 1) / tile_keys;
     size_t off = 0;
-    const size_t words = key_bits == 32 ? kSortWordsMost : (size_t)w.passes * kBins32; // (32 bits: perhaps a depth sort)
+    // (32 bits: perhaps a depth sort)
+    const size_t words = wide ? (size_t)1 << key_bits : (key_bits == 32 ? kSortWordsMost : (size_t)w.passes * kBins32);
     w.hist = off;
     off = align(off + words * 4);
     w.counters = off;
@@ -642,15 +690,16 @@ static int sort32_clear(int64_t count, int key_bits, int tile_keys, void* sort_w
 // gather.  carry_a / carry_b (with gather_src and gather_dst): the records travel through the passes
 // as packed 32-bit values instead, in ping-pong buffers of their own (the first pass packs them from
 // gather_src, the last one unpacks them into gather_dst).
-template <typename KeyT, int kThreads, int kItems, bool kCarry = false>
+template <typename KeyT, int kThreads, int kItems, bool kCarry = false, int kBits = kBits32>
 static int sort32_passes(int64_t count, int key_bits, KeyT* keys_a, uint32_t* vals_a, KeyT* keys_b, uint32_t* vals_b,
                          bool iota_values, bool keep_keys, void* sort_ws, const char* label, hipStream_t stream,
                          KeyT** keys_out, uint32_t** vals_out, const uint2* gather_src = nullptr,
                          uint2* gather_dst = nullptr, const uint32_t* counts = nullptr, uint32_t* carry_a = nullptr,
                          uint32_t* carry_b = nullptr, int polls = kSpinLimit32)
 {
-    const Sort32Workspace w = sort32_workspace(count, key_bits, kThreads * kItems);
-    const Digits32 plan = digits32(key_bits);
+    constexpr bool kWide = kBits > kBits32; // (one digit of kBits bits)
+    const Sort32Workspace w = sort32_workspace(count, key_bits, kThreads * kItems, kWide);
+    const Digits32 plan = kWide ? partition_digits(kBits, 0) : digits32(key_bits);
     char* base = static_cast<char*>(sort_ws);
     uint32_t* hist = reinterpret_cast<uint32_t*>(base + w.hist);
     uint32_t* counters = reinterpret_cast<uint32_t*>(base + w.counters);
@@ -681,7 +730,7 @@ static int sort32_passes(int64_t count, int key_bits, KeyT* keys_a, uint32_t* va
         }
         {
             DSX_TIMED(label, stream);
-            hipLaunchKernelGGL((onesweep32_kernel<KeyT, kThreads, kItems, kCarry, kBits32>), dim3((unsigned)w.tiles), dim3(kThreads), 0,
+            hipLaunchKernelGGL((onesweep32_kernel<KeyT, kThreads, kItems, kCarry, kBits>), dim3((unsigned)w.tiles), dim3(kThreads), 0,
                                stream, (const KeyT*)kin, (const uint32_t*)((p == 0 && iota_values) ? nullptr : vin),
                                (last && !keep_keys) ? (KeyT*)nullptr : kout, vout, count, plan.shift[p], plan.mask[p],
                                raw + p * kBins32, status + (size_t)p * w.tiles * kBins32,
@@ -1016,7 +1065,7 @@ OrderLayout order_layout(int64_t n, int image_width, int image_height, int list_
     o.key_ranges = off;
     off = align(off + (size_t)((n + kProjBlock - 1) / kProjBlock) * 8);
     o.slot_hist = off;
-    off = align(off + (size_t)kMaxPasses32 * kBins32 * 4);
+    off = align(off + std::max((size_t)kMaxPasses32 * kBins32, (size_t)1 << kWideBits) * 4);
     o.sort = off;
     off = align(off + sort32_workspace(n, 32, sort32_tile_keys(n)).bytes);
     const ListGrid g = list_grid(image_width, image_height, list_bin);
@@ -1866,7 +1915,9 @@ __device__ __forceinline__ void tile_counts(const CountsJob& J, int32_t* const c
 {
     const int ntx = J.ntx, nty = J.nty;
     const Digits32& plan = J.plan;
-    uint32_t* const slot_hist = J.slot_hist;
+    // one wide digit: a list's pairs are its own bin's, stored as they are counted
+    uint32_t* const wide_hist = J.plan.mask[0] >= (uint32_t)kBins32 ? J.slot_hist : nullptr;
+    uint32_t* const slot_hist = wide_hist ? nullptr : J.slot_hist;
     int32_t* const ranges = J.ranges;
     __shared__ uint32_t hist[kMaxPasses32 * kBins32];
     __shared__ __attribute__((aligned(16))) uint32_t wave_tot[kTileRounds][kCoverThreads / DSX_WAVE];
@@ -1933,6 +1984,8 @@ __device__ __forceinline__ void tile_counts(const CountsJob& J, int32_t* const c
             // atomics, no conflicts), a higher digit is constant over long runs (one add per run,
             // after a wavefront sum; same-address LDS atomics would serialise)
             const uint32_t slot = (uint32_t)(t0 + u * kCoverThreads + tid) + 1u;
+            if(wide_hist && slot <= plan.mask[0])
+                wide_hist[slot] = cnt[u]; // (zero behind the last list)
             for(int p = 0; slot_hist && p < plan.passes; ++p)
             {
                 const uint32_t d = (slot >> plan.shift[p]) & plan.mask[p];
@@ -1993,6 +2046,8 @@ __device__ __forceinline__ void tile_counts(const CountsJob& J, int32_t* const c
             *J.header = J.header_value;
         for(int p = 0; p < plan.passes; ++p)
             atomicAdd(&hist[p * kBins32], negatives);
+        if(wide_hist)
+            wide_hist[0] = negatives;
     }
     __syncthreads();
     if(slot_hist)
@@ -2540,7 +2595,7 @@ static bool launch_order_ranks(const ListGrid& lg, int64_t n, char* base, const 
 }
 
 // the counting of the tiles and, for binned lists, of the bins
-static CountsJobs counts_jobs(const ListGrid& lg, char* base, const OrderLayout& o)
+static CountsJobs counts_jobs(const ListGrid& lg, int64_t n, char* base, const OrderLayout& o)
 {
     const RangesLayout rl = ranges_layout(lg);
     int32_t* const ranges = reinterpret_cast<int32_t*>(base + o.ranges);
@@ -2550,7 +2605,7 @@ static CountsJobs counts_jobs(const ListGrid& lg, char* base, const OrderLayout&
     fine.ntx = lg.ntx;
     fine.nty = lg.nty;
     fine.plain = 0;
-    fine.plan = digits32(slot_bits(lg.tiles()));
+    fine.plan = partition_digits(slot_bits(lg.tiles()), n);
     fine.slot_hist = lg.shift ? nullptr : reinterpret_cast<uint32_t*>(base + o.slot_hist);
     fine.ranges = ranges + rl.fine;
     fine.last = lg.shift ? ranges + rl.last_tile : nullptr;
@@ -2564,7 +2619,7 @@ static CountsJobs counts_jobs(const ListGrid& lg, char* base, const OrderLayout&
         bins.ntx = lg.nbx;
         bins.nty = lg.nby;
         bins.plain = 1;
-        bins.plan = digits32(slot_bits(lg.bins()));
+        bins.plan = partition_digits(slot_bits(lg.bins()), n);
         bins.slot_hist = reinterpret_cast<uint32_t*>(base + o.slot_hist);
         bins.ranges = ranges + rl.bins;
         bins.last = nullptr;
@@ -2871,7 +2926,7 @@ int launch_depth_order(const dsx_camera& cam, int64_t n, void* order, hipStream_
     if(rc)
         return rc;
 
-    const CountsJobs jobs = counts_jobs(list_grid(cam), base, o);
+    const CountsJobs jobs = counts_jobs(list_grid(cam), n, base, o);
     // (limits of its waits: asked for are the kernels that wait)
     if(sort_polls == kSpinLimit32 && offset_polls == kSpinLimit32 &&
        launch_order_ranks(list_grid(cam), n, base, o, to_host, jobs, stream, &rc))
@@ -3232,12 +3287,13 @@ static bool slots_are_u16(int num_tiles)
 
 // binned: the slot words are 32 bits (slot in the low half, the tile mask in the high half) and the
 // sorted ones end in the caller's buffer, behind the ids
-ListsWorkspace lists_workspace(int64_t k, int num_tiles, bool binned)
+ListsWorkspace lists_workspace(int64_t n, int64_t k, int num_tiles, bool binned)
 {
     auto align = [](size_t x) { return (x + 255) & ~(size_t)255; };
     ListsWorkspace w;
     const size_t slot_bytes = (binned || !slots_are_u16(num_tiles)) ? 4 : 2;
-    w.passes = digits32(slot_bits(num_tiles)).passes;
+    const bool wide = one_wide_digit(slot_bits(num_tiles), n);
+    w.passes = partition_digits(slot_bits(num_tiles), n).passes;
     size_t off = 0;
     w.slots_a = off;
     off = align(off + (size_t)k * slot_bytes);
@@ -3246,7 +3302,7 @@ ListsWorkspace lists_workspace(int64_t k, int num_tiles, bool binned)
     w.ids_alt = off;
     off = align(off + (size_t)k * 4);
     w.sort = off;
-    off += sort32_workspace(k, slot_bits(num_tiles), sort32_tile_keys(k)).bytes;
+    off += sort32_workspace(k, slot_bits(num_tiles), sort32_tile_keys(k), wide).bytes;
     w.bytes = align(off);
     return w;
 }
@@ -3272,8 +3328,9 @@ static int tile_lists_impl(const dsx_camera& cam, int64_t n, int64_t k, int num_
             rc = launch_fill_u32(reinterpret_cast<uint32_t*>(ranges) + rl.last_tile, 1, 0xffffffffu, stream);
         return rc;
     }
-    const ListsWorkspace w = lists_workspace(k, num_tiles, kMasks);
+    const ListsWorkspace w = lists_workspace(n, k, num_tiles, kMasks);
     const int bits = slot_bits(num_tiles);
+    const bool wide = one_wide_digit(bits, n);
     char* base = static_cast<char*>(workspace);
     uint32_t* ids_final = reinterpret_cast<uint32_t*>(sorted_ids);
     uint32_t* ids_other = reinterpret_cast<uint32_t*>(base + w.ids_alt);
@@ -3287,7 +3344,7 @@ static int tile_lists_impl(const dsx_camera& cam, int64_t n, int64_t k, int num_
     SlotT* slots_a = (kMasks && even) ? slots_final : slots_other;
     SlotT* slots_b = (kMasks && even) ? slots_other : slots_final;
     int rc = DSX_OK;
-    const Sort32Workspace sw = sort32_workspace(k, bits, sort32_tile_keys(k));
+    const Sort32Workspace sw = sort32_workspace(k, bits, sort32_tile_keys(k), wide);
     {
         DSX_TIMED("emit_ordered_kernel", stream);
         // outputs per workgroup: a multiple of 256 between 256 and kEmitChunkMax
@@ -3307,12 +3364,17 @@ static int tile_lists_impl(const dsx_camera& cam, int64_t n, int64_t k, int num_
     // per-tile lists: the sorted slots themselves are not needed (the ranges are known already);
     // binned lists: they are kept for their masks
     rc = DSX_ERR_RUNTIME;
-#define DSX_PARTITION_ITEMS(ITEMS)                                                                                    \
-    case ITEMS:                                                                                                       \
-        rc = sort32_passes<SlotT, kSortThreads32, ITEMS>(k, bits, slots_a, vals_a, slots_b, vals_b, false, kMasks,     \
-                                                         base + w.sort, "onesweep32_kernel<tile partition>", stream,  \
-                                                         &ko, &vo, nullptr, nullptr,                                  \
-                                                         reinterpret_cast<const uint32_t*>(obase + o.slot_hist));     \
+    auto partition = [&](auto items, auto digit_bits) {
+        return sort32_passes<SlotT, kSortThreads32, decltype(items)::value, false, decltype(digit_bits)::value>(
+            k, bits, slots_a, vals_a, slots_b, vals_b, false, kMasks, base + w.sort, "onesweep32_kernel<tile partition>", stream, &ko, &vo,
+            nullptr, nullptr, reinterpret_cast<const uint32_t*>(obase + o.slot_hist));
+    };
+#define DSX_PARTITION_ITEMS(ITEMS)                                                                                     \
+    case ITEMS:                                                                                                        \
+        rc = !wide        ? partition(std::integral_constant<int, ITEMS>(), std::integral_constant<int, kBits32>())    \
+             : bits == 9  ? partition(std::integral_constant<int, ITEMS>(), std::integral_constant<int, 9>())          \
+             : bits == 10 ? partition(std::integral_constant<int, ITEMS>(), std::integral_constant<int, 10>())         \
+                          : partition(std::integral_constant<int, ITEMS>(), std::integral_constant<int, kWideBits>());  \
         break
     switch(sort32_items(k))
     {

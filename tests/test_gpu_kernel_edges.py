@@ -56,6 +56,35 @@ def test_emission_of_four_pairs_to_a_thread(oracle, list_bin, bin_side, n, W, H,
                                                          "identity")
 
 
+@pytest.mark.parametrize("n,W,H,scale_mul,flip,bin_side", [
+    (3000, 240, 272, 3.0, 40, 1),         # 255 tiles: eight bits, the last of them; 256: nine
+    (3000, 256, 256, 3.0, 40, 1),
+    (3000, 112, 1168, 3.0, 40, 1),        # 511 and 512: nine and ten
+    (3000, 512, 256, 3.0, 40, 1),
+    (3000, 528, 496, 3.0, 40, 1),         # 1023 and 1024: ten and eleven (two digits a thread)
+    (3000, 512, 512, 3.0, 40, 1),
+    (1, 512, 512, 1.0, 0, 1),
+    (3000, 368, 1424, 3.0, 40, 1),        # 2047: eleven, the last of them
+    (9000, 512, 512, 3.0, 40, 1),         # 2, 4, 8 and 12 keys a thread and more tiles than compute units
+    (20000, 512, 512, 3.0, 40, 1),
+    (40000, 512, 512, 3.0, 40, 1),
+    (90000, 512, 512, 3.0, 40, 1),
+    (131072, 512, 512, 1.0, 40, 1),       # one digit up to here, two beyond
+    (131073, 512, 512, 1.0, 40, 1),
+    (131073, 256, 512, 1.0, 40, 1),
+    (20000, 1920, 1080, 3.0, 40, 4),      # bins: 510, 920 and 2040 lists
+    (20000, 1280, 720, 3.0, 40, 2),
+    (20000, 1920, 1080, 3.0, 40, 2),
+])
+def test_partition_by_one_wide_digit(oracle, list_bin, n, W, H, scale_mul, flip, bin_side):
+    """Lists of nine to eleven bits: one pass where eight bits a pass would take two, at the edges of the widths and of
+    the rule that says for how many Gaussians; ids, ranges and masks bit for bit the oracle's."""
+    if bin_side == 1:
+        test_gpu_stages.test_tile_lists_bit_exact(oracle, list_bin, n, W, H, scale_mul, flip)
+    else:
+        test_gpu_stages.test_binned_tile_lists_vs_oracle(oracle, list_bin, bin_side, n, W, H, scale_mul, flip, 0, "identity")
+
+
 @pytest.mark.parametrize("depths", ["uniform", "octaves", "too_many_octaves", "equal", "both_signs", "none"])
 @pytest.mark.parametrize("n", [262144, 262145, 530001])
 def test_depth_order_over_a_known_range(n, depths):
