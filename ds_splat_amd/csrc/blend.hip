@@ -238,6 +238,7 @@ __device__ __forceinline__ int bits_below_lane(uint64_t mask)
 constexpr int kFwdWideUpTo = 256;        // tiles (a workgroup of sixteen wavefronts for each compute unit)
 constexpr int kFwdFourPixelsFrom = 5500;
 constexpr int kBwdFourPixelsFrom = 3000;
+constexpr int kBwdBlocksUpTo = 256; // (lists per tile only, as kFwdWideUpTo)
 
 // -----------------------------------------------------------------------------------------
 // what both directions share: the pixels, and the walk through the lists
@@ -2846,6 +2847,252 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
         zero_share(zeros, blockIdx.x, gridDim.x, tid, kTileThreads);
 }
 
+// -----------------------------------------------------------------------------------------
+// the same for images of very few tiles: four workgroups per tile, a wavefront for each block
+// -----------------------------------------------------------------------------------------
+// Up to 256 tiles the workgroup form leaves a SIMD one wavefront or none, and the kernel lasts as long as its longest chain: 55
+// instructions an entry, each waiting for the one before.  Here each 4x4 block has a wavefront and each of its pixels a quad of lanes,
+// which work on four entries at a time: they hand each other alphas and colours, each takes the same steps of what they let through and of
+// what lies behind, and keeps its own entry's; sums over the sixteen pixels by twelve DPP adds and two swaps, one add to
+// LDS for all four entries.  86 instructions for four.  A tile's four quadrants are workgroups of their own, so that 64 tiles reach every
+// compute unit; each stages what reaches its quadrant.  us of the kernel, workgroup form -> this:
+//   Gaussians            3 K opaque   15 K mixed   60 K faint   60 K large   400 K mixed
+//   16 tiles             56 -> 34     177 -> 111   712 -> 427   92 -> 52     168 -> 88
+//   64 tiles             27 -> 19     84 -> 54     269 -> 165   57 -> 35     93 -> 52
+//   144 tiles            22 -> 17     58 -> 39     166 -> 106   54 -> 41     76 -> 50
+//   256 tiles            19 -> 15     48 -> 36     124 -> 90    50 -> 51     62 -> 49
+//   324 tiles            18 -> 16     44 -> 30     116 -> 78    58 -> 59     61 -> 59
+//   400 tiles            19 -> 17     41 -> 33     107 -> 78    57 -> 69     60 -> 62
+// The line lies at 256, a compute unit for each tile; beyond it large Gaussians, to which four workgroups a tile add, lose.
+// the two lower halves and the two upper halves of two registers side by side (v_permlane32_swap), and their rows of 16 lanes: the
+// even rows of both and the odd rows of both (v_permlane16_swap)
+__device__ __forceinline__ float add_halves(float a, float b)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float add_rows(float a, float b)
+{
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+constexpr int kBlockThreads = 256;
+constexpr int kBlockAtOnce = 4; // entries that a wavefront takes at a time: one for each lane of a pixel's quad
+__global__ __launch_bounds__(kBlockThreads) void blend_bwd_block_kernel(
+    const int32_t* __restrict__ ranges, const int32_t* __restrict__ ids, const float4* __restrict__ splats,
+    const float* __restrict__ final_T, const int32_t* __restrict__ final_idx, const float* __restrict__ v_image,
+    const float* __restrict__ bg, float* grads, uint8_t* marks, int W, int H, int ntx, uint32_t last_id, int k,
+    const int32_t* __restrict__ header, int header_shift, int planar, const ZeroJobs zeros)
+{
+    static_assert(kBlockThreads == kTileThreads && kTileBatch % kBlockAtOnce == 0, "rounds as in the tile's form");
+    __shared__ float4 s_a[kTileBatch + 1], s_b[kTileBatch + 1], s_c[kTileBatch + 1];
+    __shared__ int s_id[kTileBatch];
+    __shared__ double s_sum[(kTileBatch + 1) * kSums];
+    __shared__ uint16_t s_reach[kTileBatch];
+    __shared__ uint32_t s_list[kTileWaves][kTileBatch / 4 + 1]; // (a word more: read ahead)
+    __shared__ int s_counts[kTileWaves];
+    __shared__ uint32_t s_special[kTileWaves];
+    __shared__ int s_last[kTileWaves]; // per block: the last entry that any of its pixels blended
+
+    const int tid = threadIdx.x, lane = tid & (DSX_WAVE - 1), slot = lane & 3, pixel = lane >> 2;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / DSX_WAVE);
+    const int tile = blockIdx.x / 4, quadrant = blockIdx.x % 4;
+    const int first_block = first_block_of(quadrant), block = first_block + block_of_row(wave);
+    const int x = tile % ntx * kTile + 4 * (block & 3) + (pixel & 3), y = tile / ntx * kTile + 4 * (block >> 2) + (pixel >> 2);
+    const float pxf = (float)x + 0.5f, pyf = (float)y + 0.5f;
+    const float tile_x = (float)(tile % ntx * kTile) + 0.5f, tile_y = (float)(tile / ntx * kTile) + 0.5f;
+
+    const bool inside = x < W && y < H;
+    const int64_t pix = inside ? (int64_t)y * W + x : 0;
+    float T = inside ? final_T[pix] : 0.0f;
+    const int bin_final = inside ? final_idx[pix] : -1;
+    const int64_t step = planar ? 1 : 3, plane = planar ? (int64_t)W * H : 1; // (between pixels, between channels)
+    const float vo0 = inside ? v_image[step * pix] : 0.f, vo1 = inside ? v_image[step * pix + plane] : 0.f,
+                vo2 = inside ? v_image[step * pix + 2 * plane] : 0.f;
+    float behind = bg[0] * vo0 + bg[1] * vo1 + bg[2] * vo2;
+    const bool tame = largest(vo0, vo1, vo2) < kTame && fabsf(behind) < kTame;
+    bool wild = __builtin_amdgcn_ballot_w64(!tame) != 0; // (of this wavefront's pixels)
+    int m = bin_final;
+#pragma unroll
+    for(int o = 4; o < DSX_WAVE; o <<= 1)
+        m = max(m, __shfl_xor(m, o, DSX_WAVE));
+    if(lane == 0)
+        s_last[wave] = m;
+    if(tid == 0)
+    {
+        s_a[kTileBatch] = s_c[kTileBatch] = make_float4(0.f, 0.f, 0.f, 0.f);
+        s_b[kTileBatch] = make_float4(0.f, 0.f, 0.f, __int_as_float(INT_MAX));
+    }
+    __syncthreads();
+    m = s_last[0];
+#pragma unroll
+    for(int w = 1; w < kTileWaves; ++w)
+        m = max(m, s_last[w]);
+    m = __builtin_amdgcn_readfirstlane(m);
+
+    // (where the lists start: as in the wavefront form)
+    int pos = -1, left = 0, idx_next = 0;
+    if(header == nullptr || *header == header_shift)
+    {
+        pos = min(min(ranges[tile + 1], k) - 1, m);
+        idx_next = pos;
+        left = pos - max(ranges[tile], 0) + 1;
+    }
+    left = __builtin_amdgcn_readfirstlane(left);
+
+    // which of an entry's sums this lane adds, and where: rows 0 and 2 the eight that bank_sum8_scatter leaves, the odd rows' first
+    // four lanes halves of the ninth
+    const int row = lane >> 4;
+    const bool carries = (row & 1) == 0 || (lane & 12) == 0;
+    const int sum_shift = row & 1 ? 3 : 5;
+    char* const my_sums = reinterpret_cast<char*>(
+        s_sum + sum_at<kTileBatch + 1>(0, row & 1 ? 8 : 2 * row + 2 * ((lane >> 2) & 1) + ((lane >> 3) & 1)));
+
+    int id_ahead = 0;
+    int summed = 0; // entries of the last round, whose sums are still to be added to memory
+    if(tid < min(left, kTileBatch))
+        id_ahead = ids[pos - tid];
+    while(left > 0)
+    {
+        const int batch = min(left, kTileBatch);
+        int id = id_ahead;
+        pos -= batch;
+        left -= batch;
+        if(tid < min(left, kTileBatch))
+            id_ahead = ids[pos - tid];
+        uint32_t reached = 0;
+        bool special = wild;
+        float4 q0, q1, q2;
+        float reach = 0.0f;
+        const int idx = idx_next - tid;
+        if(tid < batch)
+        {
+            id = (int)min((uint32_t)id, last_id);
+            const float4* const rec = splats + 3 * (int64_t)id;
+            q0 = rec[0], q1 = rec[1], q2 = rec[2];
+            reach = reach_of(q1.w);
+            const uint32_t blocks = blocks_reached(q0.x, q0.y, q1.x, q1.y, q1.z, reach, tile_x, tile_y) >> first_block;
+#pragma unroll
+            for(int w = 0; w < kTileWaves; ++w)
+                if(idx <= s_last[w])
+                    reached |= blocks & (1u << block_of_row(w));
+            special = special || (reached != 0 && !plain_entry(q0, q1, q2));
+        }
+        if(tid < batch) // (the loads end here: behind the adds they would wait for those)
+            asm volatile("" : "+v"(q2.x), "+v"(q2.y), "+v"(q2.z), "+v"(q2.w));
+        flush_sums<kTileBatch + 1>(s_sum, s_id, summed, grads, tid, kBlockThreads);
+        const bool mine_special = __builtin_amdgcn_ballot_w64(special) != 0;
+        if(lane == 0)
+            s_special[wave] = mine_special;
+        int staged;
+        const int place = tile_place(s_counts, __builtin_amdgcn_ballot_w64(reached != 0), staged);
+        // (the barrier inside: the last round's sums have been taken)
+        for(int i = tid; i < 4 * staged; i += kBlockThreads)
+            s_sum[i] = s_sum[sum_at<kTileBatch + 1>(0, 4) + i] = 0.0;
+        if(tid < staged)
+            s_sum[sum_at<kTileBatch + 1>(tid, 8)] = 0.0;
+        if(reached != 0)
+        {
+            s_a[place] = make_float4(q0.x, q0.y, q1.x * 0.5f, q1.y);
+            s_b[place] = make_float4(q1.z * 0.5f, q1.w, __uint_as_float(reach_limit_bwd(q1.w, reach)), __int_as_float(idx));
+            s_c[place] = q2;
+            s_id[place] = id;
+            s_reach[place] = (uint16_t)reached;
+        }
+        idx_next -= batch;
+        __syncthreads();
+
+        // this wavefront's list: the places of the entries that reach its block, and nobody's at the end
+        uint8_t* const bytes = reinterpret_cast<uint8_t*>(s_list[wave]);
+        if(lane < kTileBatch / 4)
+            s_list[wave][lane] = 0x01010101u * kTileBatch;
+        int length = 0;
+        for(int first = 0; first < staged; first += DSX_WAVE)
+        {
+            const int mine = first + lane;
+            const uint64_t reaches = __builtin_amdgcn_ballot_w64(mine < staged && ((s_reach[min(mine, kTileBatch - 1)] >> block_of_row(wave)) & 1));
+            if(__builtin_amdgcn_inverse_ballot_w64(reaches))
+                bytes[length + bits_below_lane(reaches)] = (uint8_t)mine;
+            length += __popcll(reaches);
+        }
+        // (one walk for all wavefronts: the sums' unit depends on it)
+        const bool all_plain = __builtin_amdgcn_readfirstlane(s_special[0] | s_special[1] | s_special[2] | s_special[3]) == 0;
+        auto walk = [&](auto plain) {
+            const int rounds = (length + kBlockAtOnce - 1) / kBlockAtOnce;
+            const uint32_t* my_list = s_list[wave];
+            uint32_t places = *my_list;
+            for(int i = 0; i < rounds; ++i)
+            {
+                const uint32_t here = __builtin_amdgcn_ubfe(places, 8 * slot, 8);
+                places = *++my_list;
+                const float4 A = s_a[here], B = s_b[here], C = s_c[here];
+                float alpha, vis;
+                const float dx = pxf - A.x, dy = pyf - A.y;
+                uint64_t m_valid;
+                {
+#pragma clang fp contract(off)
+                    // sigma exactly as the forward computed it
+                    const ExponentX ex = exponent_x(A.z, A.w, dx);
+                    const float sigma = __builtin_fmaf(__builtin_fmaf(B.x, dy, ex.bx), dy, ex.ax);
+                    m_valid = __builtin_amdgcn_ballot_w64(__float_as_int(B.w) <= bin_final) &
+                              __builtin_amdgcn_ballot_w64(__float_as_uint(sigma) <= __float_as_uint(B.z));
+                    vis = __builtin_amdgcn_exp2f(-sigma * kLog2E);
+                    const float full = plain ? B.y * vis : fminf(kAlphaMaxBwd, B.y * vis);
+                    alpha = __builtin_amdgcn_inverse_ballot_w64(m_valid) ? full : 0.0f;
+                }
+                const float colour = C.x * vo0 + (C.y * vo1 + C.z * vo2);
+                // the quad's four entries from the farthest one on: what they let through, and what lies behind each
+                const float a[4] = {quad_lane<0x00>(alpha), quad_lane<0x55>(alpha), quad_lane<0xaa>(alpha), quad_lane<0xff>(alpha)};
+                const float q[4] = {quad_lane<0x00>(colour), quad_lane<0x55>(colour), quad_lane<0xaa>(colour), quad_lane<0xff>(colour)};
+                const float through0 = 1.0f - a[0], through1 = __builtin_fmaf(-a[1], through0, through0);
+                const float through2 = __builtin_fmaf(-a[2], through1, through1), through3 = __builtin_fmaf(-a[3], through2, through2);
+                const float T_here =
+                    T * __builtin_amdgcn_rcpf(slot == 0 ? through0 : (slot == 1 ? through1 : (slot == 2 ? through2 : through3)));
+                T = quad_lane<0xff>(T_here); // in front of all four
+                float behind_here = behind;
+#pragma unroll
+                for(int u = 0; u < 4; ++u)
+                {
+                    behind_here = slot == u ? behind : behind_here;
+                    const float next = behind + a[u] * (q[u] - behind);
+                    behind = plain || a[u] != 0.0f ? next : behind; // (zero times infinity)
+                }
+                const float fac = alpha * T_here, ahead = colour - behind_here;
+                float w = (plain ? fac : vis * T_here) * ahead;
+                if(!plain)
+                    w = __builtin_amdgcn_inverse_ballot_w64(m_valid) ? w : 0.0f;
+                const float wx = w * dx, wy = w * dy;
+                const float sum8[8] = {w, wx, wx * dx, wy, wy * dx, wy * dy, fac * vo0, fac * vo1};
+                float first, second;
+                bank_sum8_scatter(sum8, first, second);
+                float v_blue = dpp_add<0x128>(fac * vo2); // row_ror:8
+                v_blue += dpp_move<0x104, true>(v_blue);  // row_shl:4 (the sum in every row's first four lanes)
+                // (v_blue's two upper rows are the lower ones' other halves)
+                const float halves = add_halves(first, second);
+                const float total = add_rows(halves, v_blue);
+                if(carries)
+                    unsafeAtomicAdd(reinterpret_cast<double*>(my_sums + (here << sum_shift)), (double)total);
+            }
+        };
+        if(all_plain)
+            walk(std::true_type());
+        else
+        {
+            walk(std::false_type());
+            // (an infinite colour stays behind all entries in front)
+            wild = wild || __builtin_amdgcn_ballot_w64(!(fabsf(behind) < kTame)) != 0;
+        }
+        __syncthreads();
+        for(int e = tid; e < staged; e += kBlockThreads)
+            moments_to_gradients<kTileBatch + 1>(s_sum, e, s_a[e], s_b[e], all_plain, marks ? marks + s_id[e] : nullptr);
+        __syncthreads();
+        summed = staged;
+    }
+    flush_sums<kTileBatch + 1>(s_sum, s_id, summed, grads, tid, kBlockThreads);
+    if(zeros.any)
+        zero_share(zeros, blockIdx.x, gridDim.x, tid, kBlockThreads);
+}
+
 // ranges, check_header, n, k: as for launch_blend_fwd (the kernel reads the `walk` part that the forward wrote)
 int launch_blend_bwd(const dsx_camera& cam, int64_t n, int64_t k, const int32_t* ranges, const int32_t* sorted_ids,
                      const float* splats, const float* final_T, const int32_t* final_idx, const float* v_image,
@@ -2878,7 +3125,12 @@ int launch_blend_bwd(const dsx_camera& cam, int64_t n, int64_t k, const int32_t*
     hipLaunchKernelGGL((KERNEL), grid, dim3(THREADS), 0, stream, ranges, sorted_ids, sp, final_T, final_idx, v_image, \
                        cam.bg, grads, with_marks ? grad_marks(grads, n) : nullptr, cam.image_width,                 \
                        cam.image_height, ntx, last_id, (int)k, header, lg.shift, camera_flag(cam, DSX_PLANAR_IMAGE), L, Z)
-        if(four && lg.shift)
+        const bool blocks = forced_pixels_per_lane() == 0 && lg.shift == 0 && ntx * nty <= kBwdBlocksUpTo;
+        if(blocks)
+            hipLaunchKernelGGL(blend_bwd_block_kernel, dim3(4 * ntx * nty), dim3(kBlockThreads), 0, stream, ranges, sorted_ids, sp, final_T,
+                               final_idx, v_image, cam.bg, grads, with_marks ? grad_marks(grads, n) : nullptr, cam.image_width,
+                               cam.image_height, ntx, last_id, (int)k, header, lg.shift, camera_flag(cam, DSX_PLANAR_IMAGE), Z);
+        else if(four && lg.shift)
             DSX_LAUNCH_BWD(blend_bwd_kernel<true>, DSX_WAVE);
         else if(four)
             DSX_LAUNCH_BWD(blend_bwd_kernel<false>, DSX_WAVE);

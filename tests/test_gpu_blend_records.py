@@ -137,7 +137,7 @@ def sums_in_64_bits(rec, v_image, bg, final_T, final_idx):
 
 @pytest.mark.parametrize("kind", ["faint", "clamped", "stopping", "wild"])
 @pytest.mark.parametrize("n", [1, 2, 55, 57, 113, 247, 249, 500])
-@pytest.mark.parametrize("pixels_per_lane", [1, 4])
+@pytest.mark.parametrize("pixels_per_lane", [0, 1, 4])
 def test_backward_sums_against_64_bits(blend_form, pixels_per_lane, n, kind):
     """Around the rounds of 56 and of 248 entries, odd and even: rounds that no pixel's last entry lies in, rounds where
     pixels end or alpha reaches the clamp, and an upstream gradient whose products with zero must stay out of the sums."""
