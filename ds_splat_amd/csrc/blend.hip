@@ -15,6 +15,7 @@
 
 #include <atomic>
 #include <climits>
+#include <cstddef>
 #include <cstdlib>
 #include <type_traits>
 
@@ -236,6 +237,7 @@ __device__ __forceinline__ int bits_below_lane(uint64_t mask)
 }
 
 constexpr int kFwdWideUpTo = 256;        // tiles (a workgroup of sixteen wavefronts for each compute unit)
+constexpr int kWideSplitUpTo = 64;        // (a compute unit for each quadrant)
 constexpr int kFwdFourPixelsFrom = 5500;
 constexpr int kBwdFourPixelsFrom = 3000;
 constexpr int kBwdBlocksUpTo = 256; // (lists per tile only, as kFwdWideUpTo)
@@ -1151,6 +1153,9 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(6)
 // and at 169 and 256 tiles 40 more of 2 K to 1 M Gaussians, opaque, mixed, faint (322 -> 241) and large (248 -> 246): none is slower
 // by more than its runs differ.
 // The line lies at 256, a tile for each compute unit; beyond it some units get two.
+// Up to 64 tiles a workgroup for each quadrant, sixteen wavefronts to find and stage its entries and four to walk, one to a SIMD.  us of the
+// kernel, a workgroup for each tile -> four: 16 tiles of 60 K faint Gaussians 258 -> 176, of 400 K mixed ones 94 -> 52, 36 tiles 150 -> 104 and 62 -> 38, 64
+// tiles 100 -> 70 and 45 -> 31.
 // Lists per tile only (images of so few tiles have no others unless the caller asks).
 constexpr int kWideBatch = 960; // (two workgroups' records and lists fit a compute unit's LDS)
 constexpr int kWideThreads = 1024;
@@ -1161,12 +1166,16 @@ static_assert(kWideWaves == kQuads, "a wavefront for each block");
 // entries in order, and a workgroup finds them faster than a depth order, pairs and their partition can bring them (and the
 // host need not wait for the pairs' number): it looks at all rectangles, takes those that cover its tile, sorts them
 // by depth and index in LDS, and blends them.  Where more than kOwnMost do, it takes them in windows, nearest first, each found by
-// counting the rest into bins.  Each colour is then a sum in other parts; all else has the same bits.
+// counting the rest into bins.  Each colour is then a sum in other parts; all else has the same bits.  Up to 960 entries (a round) take the
+// short way: a thread for each fetches its record and its depth together, drops it if it reaches no block of the workgroup's, and puts it where it belongs
+// among the others.  us of a forward, found, sorted and then staged -> this -> and by quadrants up to 64 tiles: 2 K Gaussians at 64x64 25.5 -> 22.7 -> 18.7, 2 K
+// at 128x128 19.8 -> 17.2 -> 16.2, 6 K at 128x128 27.0 -> 23.8 -> 21.2, 10 K at 208x208 29.1 -> 26.9, 16 K at 256x256 37.4 -> 35.1.
 struct OwnLists
 {
     const uint32_t* depth_keys; // by Gaussian, as the projection leaves them
     const uint2* rects;
     int n;
+    int last_tile; // of the image
 };
 // us of a whole forward, 64x64 / 128x128 / 208x208 / 256x256, four kinds of scenes (small, mixed, faint, large), with lists -> without:
 //   6 K Gaussians   62, 63, 57, 63 -> 47, 48, 42, 46 / 43, 45, 42, 55 -> 25, 28, 23, 36 / 41, 44, 40, 53 -> 22, 24, 21, 34 / 45, 48, 45, 61 -> 21, 23, 20, 33
@@ -1208,29 +1217,40 @@ struct OwnShared
     uint32_t tot[kWideWaves];
     uint32_t found[3];
     uint32_t taken, most, nearest, farthest;
+    uint32_t reaching, reaching_near, reaching_far; // of own_stage: how many, and their extreme keys (the nearest one's complement)
     int highest;
 };
 
-// f(index, copies) for every rectangle of the source with an entry
+// f(first index, this thread's eight rectangles, source) for all of them, eight thousand at a time with the next ones in flight
 template <typename F>
 __device__ __forceinline__ void own_for_all(const OwnLists& L, const OwnSource& src, F f)
 {
-    for(int i0 = 0; i0 < L.n; i0 += 8 * kWideThreads)
-    {
-        uint2 r[8];
+    auto load = [&](int i0, uint2 (&r)[8]) {
 #pragma unroll
         for(int b = 0; b < 8; ++b)
         {
             const int i = i0 + b * kWideThreads + (int)threadIdx.x;
             r[b] = i < L.n ? L.rects[i] : make_uint2(0u, 0u);
         }
+    };
+    uint2 next[8];
+    load(0, next);
+    for(int i0 = 0; i0 < L.n; i0 += 8 * kWideThreads)
+    {
+        uint2 r[8];
+#pragma unroll
+        for(int b = 0; b < 8; ++b)
+            r[b] = next[b];
+        if(i0 + 8 * kWideThreads < L.n)
+            load(i0 + 8 * kWideThreads, next);
         f(i0, r, src);
     }
 }
 
-// The numbers in [low, high) of the source's entries into scratch.numbers (as far as there is room), in any order; returns how many there
-// are, and their nearest and farthest depth keys.
-__device__ __forceinline__ int own_take(const OwnLists& L, const OwnSource& src, OwnScratch& S, OwnShared& sh, uint64_t low, uint64_t high,
+// The source's entries with numbers in [low, high): their indices (as far as there is room), in any order, where own_found has them;
+// returns how many there are.
+__device__ __forceinline__ const uint32_t* own_found(const OwnScratch& S) { return reinterpret_cast<const uint32_t*>(S.binned); }
+__device__ __forceinline__ int own_find(const OwnLists& L, const OwnSource& src, OwnScratch& S, OwnShared& sh, uint64_t low, uint64_t high,
                                         bool everything)
 {
     const int tid = threadIdx.x, lane = tid & (DSX_WAVE - 1);
@@ -1240,6 +1260,7 @@ __device__ __forceinline__ int own_take(const OwnLists& L, const OwnSource& src,
         sh.taken = 0;
         sh.nearest = 0xffffffffu;
         sh.farthest = 0;
+        sh.reaching = sh.reaching_near = sh.reaching_far = 0;
     }
     __syncthreads();
     int highest = 0;
@@ -1274,15 +1295,20 @@ __device__ __forceinline__ int own_take(const OwnLists& L, const OwnSource& src,
     });
     if(everything)
     {
-#pragma unroll
-        for(int o = DSX_WAVE / 2; o > 0; o >>= 1)
-            highest = max(highest, __shfl_xor(highest, o, DSX_WAVE));
-        if(lane == 0)
+        highest = (int)wave_incl_max_scan((uint32_t)highest); // (it begins with zero)
+        if(lane == DSX_WAVE - 1)
             atomicMax(&sh.highest, highest);
     }
     __syncthreads();
-    const int total = (int)__builtin_amdgcn_readfirstlane((int)sh.taken), count = min(total, kOwnMost);
-    uint32_t nearest = 0xffffffffu, farthest = 0;
+    return (int)__builtin_amdgcn_readfirstlane((int)sh.taken);
+}
+
+// the numbers of `total` found entries, and their nearest and farthest depth keys
+__device__ __forceinline__ void own_numbers(const OwnLists& L, OwnScratch& S, OwnShared& sh, int total)
+{
+    const int tid = threadIdx.x, lane = tid & (DSX_WAVE - 1), count = min(total, kOwnMost);
+    const uint32_t* const ids = own_found(S);
+    uint32_t nearest = 0, farthest = 0; // (the nearest one's complement)
 #pragma unroll
     for(int b = 0; b < kOwnMost / kWideThreads; ++b)
     {
@@ -1291,23 +1317,18 @@ __device__ __forceinline__ int own_take(const OwnLists& L, const OwnSource& src,
         {
             const uint32_t id = ids[at], key = L.depth_keys[id];
             S.numbers[at] = (uint64_t)key << 32 | id;
-            nearest = min(nearest, key);
+            nearest = max(nearest, ~key);
             farthest = max(farthest, key);
         }
     }
-#pragma unroll
-    for(int o = DSX_WAVE / 2; o > 0; o >>= 1)
+    nearest = wave_incl_max_scan(nearest);
+    farthest = wave_incl_max_scan(farthest);
+    if(lane == DSX_WAVE - 1)
     {
-        nearest = min(nearest, (uint32_t)__shfl_xor((int)nearest, o, DSX_WAVE));
-        farthest = max(farthest, (uint32_t)__shfl_xor((int)farthest, o, DSX_WAVE));
-    }
-    if(lane == 0)
-    {
-        atomicMin(&sh.nearest, nearest);
+        atomicMin(&sh.nearest, ~nearest);
         atomicMax(&sh.farthest, farthest);
     }
     __syncthreads();
-    return total;
 }
 
 __device__ __forceinline__ int number_bits(uint64_t v)
@@ -1316,11 +1337,11 @@ __device__ __forceinline__ int number_bits(uint64_t v)
 }
 
 // exclusive sums of the histogram's bins in place of their counts
-__device__ __forceinline__ void own_scan(OwnScratch& S, OwnShared& sh)
+__device__ __forceinline__ void own_scan(uint32_t* hist, OwnShared& sh)
 {
     const int tid = threadIdx.x, lane = tid & (DSX_WAVE - 1), wave = tid / DSX_WAVE;
     __syncthreads();
-    uint4* const mine = reinterpret_cast<uint4*>(S.hist) + tid;
+    uint4* const mine = reinterpret_cast<uint4*>(hist) + tid;
     const uint4 c = *mine;
     const uint32_t sum = c.x + c.y + c.z + c.w, incl = wave_incl_scan_u32(sum);
     if(lane == DSX_WAVE - 1)
@@ -1331,13 +1352,25 @@ __device__ __forceinline__ void own_scan(OwnScratch& S, OwnShared& sh)
     __syncthreads();
 }
 
+// where a number's bin begins to matter: the range of keys in 2^kOwnBinBits bins
+struct OwnBinning
+{
+    uint64_t from;
+    int shift;
+    __device__ __forceinline__ OwnBinning(uint32_t nearest, uint32_t farthest)
+        : from((uint64_t)nearest << 32),
+          shift(max(number_bits(((uint64_t)(farthest - nearest) << 32) | 0xffffffffull) - kOwnBinBits, 0))
+    {
+    }
+    __device__ __forceinline__ uint32_t operator()(uint64_t number) const { return (uint32_t)((number - from) >> shift); }
+};
+
 // scratch.numbers [0, count), of depth keys nearest to farthest, in order: their indices into `ids`
 __device__ __forceinline__ void own_sort(OwnScratch& S, OwnShared& sh, int count, uint32_t* ids)
 {
     constexpr int kItems = kOwnMost / kWideThreads;
     const int tid = threadIdx.x;
-    const uint64_t from = (uint64_t)sh.nearest << 32, width = ((uint64_t)(sh.farthest - sh.nearest) << 32) | 0xffffffffull;
-    const int shift = max(number_bits(width) - kOwnBinBits, 0);
+    const OwnBinning bin_of(sh.nearest, sh.farthest);
     reinterpret_cast<uint4*>(S.hist)[tid] = make_uint4(0u, 0u, 0u, 0u);
     if(tid == 0)
         sh.most = 0;
@@ -1353,14 +1386,14 @@ __device__ __forceinline__ void own_sort(OwnScratch& S, OwnShared& sh, int count
         if(at < count)
         {
             mine[b] = S.numbers[at];
-            bin[b] = (uint32_t)((mine[b] - from) >> shift);
+            bin[b] = bin_of(mine[b]);
             nth[b] = atomicAdd(&S.hist[bin[b]], 1u);
             most = max(most, nth[b]);
         }
     }
     if(__builtin_amdgcn_ballot_w64(most >= kOwnGroupMost) != 0 && (tid & (DSX_WAVE - 1)) == 0)
         sh.most = 1;
-    own_scan(S, sh);
+    own_scan(S.hist, sh);
     if(__builtin_amdgcn_readfirstlane((int)sh.most) == 0)
     {
         uint32_t start[kItems], end[kItems];
@@ -1442,7 +1475,7 @@ __device__ __forceinline__ uint64_t own_border(const OwnLists& L, const OwnSourc
         __syncthreads();
         const uint4 c = reinterpret_cast<const uint4*>(S.hist)[tid];
         const uint32_t count[4] = {c.x, c.y, c.z, c.w};
-        own_scan(S, sh);
+        own_scan(S.hist, sh);
         // the first bin border with kWanted numbers or more in front
 #pragma unroll
         for(int u = 0; u < 4; ++u)
@@ -1478,7 +1511,7 @@ __global__ __launch_bounds__(kWideThreads) void blend_fwd_wide_kernel(const int3
                                                                       const uint32_t* __restrict__ sort_flag_b,
                                                                       float4* __restrict__ prep, int64_t prep_count,
                                                                       uint8_t* __restrict__ prep_marks, int prep_zeros,
-                                                                      const float* __restrict__ bg, int planar, const OwnLists own)
+                                                                      const float* __restrict__ bg, int planar, int split, const OwnLists own)
 {
     // (arrays as in the other forms; eight places more than an entry has blocks: the lists' ends name nobody's place, read ahead)
     struct Staged
@@ -1504,9 +1537,12 @@ __global__ __launch_bounds__(kWideThreads) void blend_fwd_wide_kernel(const int3
 
     const int tid = threadIdx.x, lane = tid & (DSX_WAVE - 1), slot = lane & 3, pixel = lane >> 2;
     const int wave = __builtin_amdgcn_readfirstlane(tid / DSX_WAVE);
-    const int tile = blockIdx.x;
+    // (split: a workgroup for each quadrant of a tile, of which four wavefronts have a block and the others help to find and stage)
+    const int tile = split ? blockIdx.x / 4 : blockIdx.x, quadrant = blockIdx.x % 4;
+    const bool has_block = !split || wave < 4;
+    const int block = split ? first_block_of(quadrant) + block_of_row(wave & 3) : wave;
     const int x0 = (tile % ntx) * kTile, y0 = (tile / ntx) * kTile;
-    const int x = x0 + 4 * (wave & 3) + (pixel & 3), y = y0 + 4 * (wave >> 2) + (pixel >> 2);
+    const int x = x0 + 4 * (block & 3) + (pixel & 3), y = y0 + 4 * (block >> 2) + (pixel >> 2);
     const float pxf = (float)x + 0.5f;
 
     // (positions and layout are taken for what they are as in the wavefront form)
@@ -1519,11 +1555,87 @@ __global__ __launch_bounds__(kWideThreads) void blend_fwd_wide_kernel(const int3
     }
     int left = end - scan;
 
-    const bool inside = x < W && y < H;
+    const bool inside = has_block && x < W && y < H;
     float pyf = inside ? (float)y + 0.5f : __builtin_nanf(""); // (NaN: stopped)
     float T = 1.0f, red = 0.f, green = 0.f, blue = 0.f;        // (the colours of this lane's entries)
     int last = 0;
 
+    // this wavefront's list of what is staged, and its walk
+    auto blend_staged = [&](int staged) {
+        uint16_t* const list = s_list[wave];
+        int length = 0;
+        for(int first = 0; first < staged; first += DSX_WAVE)
+        {
+            const int at = first + lane;
+            const uint64_t mine = __builtin_amdgcn_ballot_w64(at < staged && ((uint32_t)s_reach[min(at, kWideBatch - 1)] >> block & 1) != 0);
+            if(__builtin_amdgcn_inverse_ballot_w64(mine))
+                list[length + bits_below_lane(mine)] = (uint16_t)at;
+            length += __popcll(mine);
+        }
+        if(lane < 8)
+            list[length + lane] = kWideBatch;
+
+        struct Entry
+        {
+            float4 A, B, C;
+        };
+        auto fetch = [&](int at) { return Entry{s_a[at], s_b[at], s_c[at]}; };
+        Entry next = fetch(list[slot]);
+        int after = list[4 + slot];
+        for(int i = 0; i < length; i += 4)
+        {
+            const Entry e = next;
+            next = fetch(after);
+            after = list[min(i + 8, length + 4) + slot];
+            float alpha;
+            uint64_t m_pass;
+            {
+#pragma clang fp contract(off)
+                const ExponentX ex = exponent_x(e.A.z, e.A.w, pxf - e.A.x);
+                const float dy = pyf - e.A.y;
+                const float power = __builtin_fmaf(-__builtin_fmaf(e.B.x, dy, ex.bx), dy, ex.ax);
+                m_pass = __builtin_amdgcn_ballot_w64(__float_as_int(power) <= __float_as_int(e.B.z));
+                const float full = fminf(kAlphaMax, e.B.y * __builtin_amdgcn_exp2f(power * kLog2E));
+                alpha = __builtin_amdgcn_inverse_ballot_w64(m_pass) ? full : 0.0f;
+            }
+            const float alphas[4] = {quad_lane<0x00>(alpha), quad_lane<0x55>(alpha), quad_lane<0xAA>(alpha), quad_lane<0xFF>(alpha)};
+            const float T1 = __builtin_fmaf(-alphas[0], T, T), T2 = __builtin_fmaf(-alphas[1], T1, T1);
+            const float T3 = __builtin_fmaf(-alphas[2], T2, T2), T4 = __builtin_fmaf(-alphas[3], T3, T3);
+            float before = slot & 2 ? (slot & 1 ? T3 : T2) : (slot & 1 ? T1 : T);
+            float Tn = T4;
+            if(__builtin_amdgcn_ballot_w64(T4 < 0.0001f) != 0)
+            {
+                // some pixel becomes opaque within these entries: once more, each lane up to where its pixel stops
+                Tn = T;
+                bool stopped = pyf != pyf, counts = !stopped;
+#pragma unroll
+                for(int u = 0; u < 4; ++u)
+                {
+                    before = slot == u ? Tn : before;
+                    const float further = __builtin_fmaf(-alphas[u], Tn, Tn);
+                    stopped = stopped || further < 0.0001f;
+                    Tn = stopped ? Tn : further;
+                    counts = slot == u ? !stopped : counts;
+                }
+                pyf = stopped ? __builtin_nanf("") : pyf;
+                m_pass &= __builtin_amdgcn_ballot_w64(counts);
+                alpha = counts ? alpha : 0.0f;
+                if(__builtin_amdgcn_ballot_w64(pyf == pyf) == 0)
+                    i = length; // no pixel left
+            }
+            T = Tn;
+            const float weight = alpha * before;
+            red = __builtin_fmaf(weight, e.C.x, red);
+            green = __builtin_fmaf(weight, e.C.y, green);
+            blue = __builtin_fmaf(weight, e.C.z, blue);
+            last = __builtin_amdgcn_inverse_ballot_w64(m_pass) ? __float_as_int(e.B.w) : last;
+        }
+    };
+
+    if(tid < kWideWaves)
+        s_live[tid] = 0;
+    if(!kOwn) // (own lists: there are barriers before it is written)
+        __syncthreads();
     // own lists: whose entries (as tile_source has it), all of them if they fit a window
     OwnSource src = {tile % ntx, tile / ntx};
     OwnScratch& scratch = *reinterpret_cast<OwnScratch*>(s_memory);
@@ -1533,21 +1645,92 @@ __global__ __launch_bounds__(kWideThreads) void blend_fwd_wide_kernel(const int3
     {
         if(tid == 0)
             s_own.highest = 0;
-        remaining = own_take(own, src, scratch, s_own, 0, 0, true);
+        remaining = own_find(own, src, scratch, s_own, 0, 0, true);
         const int highest = __builtin_amdgcn_readfirstlane(s_own.highest); // (0: no tile is occupied)
         const int last_x = (highest & 0xffff) - 1, last_y = (highest >> 16) - 1;
         const bool occupied = highest > 0, mine = occupied && src.sx == last_x && src.sy == last_y;
-        if(blockIdx.x == gridDim.x - 1)
+        if(tile == own.last_tile)
         {
             if(!mine)
             {
                 src.sx = occupied ? last_x : -1;
                 src.sy = occupied ? last_y : -1;
-                remaining = own_take(own, src, scratch, s_own, 0, 0, true);
+                remaining = own_find(own, src, scratch, s_own, 0, 0, true);
             }
         }
         else if(mine)
             remaining = 0;
+    }
+    if(kOwn && remaining > 0 && remaining <= kWideBatch)
+    {
+        // A thread for each: what reaches no block is dropped before it is sorted, and the rest goes to its place at once.  (In the
+        // lists' memory: the bins, and the numbers by bin.)
+        uint32_t* const hist = reinterpret_cast<uint32_t*>(s_list);
+        uint64_t* const binned = reinterpret_cast<uint64_t*>(hist + kOwnBins);
+        static_assert(kOwnBins * 4 + kWideThreads * 8 <= sizeof(staged_lds.list) && offsetof(Staged, list) % 16 == 0, "room");
+        static_assert(offsetof(OwnScratch, binned) + kWideThreads * 4 <= offsetof(Staged, list), "the bins leave the found indices alone");
+        uint32_t reached = 0, key = 0;
+        uint64_t number = 0;
+        float4 q0, q1, q2;
+        float reach = 0.0f;
+        if(tid < remaining)
+        {
+            const uint32_t id = own_found(scratch)[tid];
+            const float4* const rec = splats + 3 * (int64_t)id;
+            q0 = rec[0], q1 = rec[1], q2 = rec[2];
+            key = own.depth_keys[id];
+            reach = reach_of(q1.w);
+            reached = blocks_reached(q0.x, q0.y, q1.x, q1.y, q1.z, reach, (float)x0 + 0.5f, (float)y0 + 0.5f);
+            if(split)
+                reached &= 0x33u << first_block_of(quadrant);
+            number = (uint64_t)key << 32 | id;
+        }
+        reinterpret_cast<uint4*>(hist)[tid] = make_uint4(0u, 0u, 0u, 0u);
+        const uint32_t near = wave_incl_max_scan(reached ? ~key : 0u), far = wave_incl_max_scan(reached ? key : 0u);
+        const int reaching = __popcll(__builtin_amdgcn_ballot_w64(reached != 0));
+        if(lane == DSX_WAVE - 1 && reaching)
+        {
+            atomicAdd(&s_own.reaching, (uint32_t)reaching);
+            atomicMax(&s_own.reaching_near, near);
+            atomicMax(&s_own.reaching_far, far);
+        }
+        __syncthreads();
+        const int count = __builtin_amdgcn_readfirstlane((int)s_own.reaching);
+        const OwnBinning bin_of(~s_own.reaching_near, s_own.reaching_far);
+        uint32_t bin = 0, nth = 0;
+        if(reached)
+        {
+            bin = bin_of(number);
+            nth = atomicAdd(&hist[bin], 1u);
+        }
+        own_scan(hist, s_own);
+        uint32_t start = 0, end = 0;
+        if(reached)
+        {
+            start = hist[bin];
+            end = bin + 1 < kOwnBins ? hist[bin + 1] : (uint32_t)count;
+            binned[start + nth] = number;
+        }
+        __syncthreads();
+        if(reached)
+        {
+            uint32_t place = start;
+            for(uint32_t j = start; j < end; ++j) // (copies of one entry among them)
+                place += binned[j] < number || (binned[j] == number && j < start + nth) ? 1u : 0u;
+            s_a[place] = make_float4(q0.x, q0.y, q1.x * -0.5f, q1.y);
+            s_b[place] = make_float4(q1.z * 0.5f, q1.w, __int_as_float(reach_limit_fwd(q1.w, reach)), 0.0f);
+            s_c[place] = q2;
+            s_reach[place] = (uint16_t)reached;
+        }
+        if(tid == 0)
+        {
+            s_a[kWideBatch] = s_c[kWideBatch] = make_float4(0.f, 0.f, 0.f, 0.f);
+            s_b[kWideBatch] = make_float4(0.f, 0.f, __int_as_float(INT_MIN), 0.f);
+        }
+        __syncthreads();
+        if(has_block)
+            blend_staged(count);
+        remaining = 0;
     }
     bool first_window = true;
     while(true) // (windows; one of lists that are there)
@@ -1560,9 +1743,10 @@ __global__ __launch_bounds__(kWideThreads) void blend_fwd_wide_kernel(const int3
             if(!first_window || remaining > kOwnMost)
             {
                 const uint64_t high = remaining > kOwnMost ? own_border(own, src, scratch, s_own, low) : ~0ull;
-                count = min(own_take(own, src, scratch, s_own, low, high, false), kOwnMost);
+                count = min(own_find(own, src, scratch, s_own, low, high, false), kOwnMost);
                 low = high;
             }
+            own_numbers(own, scratch, s_own, count);
             own_sort(scratch, s_own, count, s_own_ids);
             remaining -= count;
             first_window = false;
@@ -1581,8 +1765,8 @@ __global__ __launch_bounds__(kWideThreads) void blend_fwd_wide_kernel(const int3
         while(true)
         {
             const bool live = __builtin_amdgcn_ballot_w64(pyf == pyf) != 0;
-            if(lane == 0)
-                s_live[wave] = live;
+            if(lane == 0 && has_block)
+                s_live[block] = live;
             __syncthreads(); // (and the last round's entries have been walked)
             const uint32_t live_blocks = (uint32_t)__builtin_amdgcn_ballot_w64(lane < kWideWaves && s_live[lane & (kWideWaves - 1)] != 0);
             if(live_blocks == 0)
@@ -1629,74 +1813,7 @@ __global__ __launch_bounds__(kWideThreads) void blend_fwd_wide_kernel(const int3
             if(!live)
                 continue; // (nothing left in this block: the others' barriers are met)
 
-            uint16_t* const list = s_list[wave];
-            int length = 0;
-            for(int first = 0; first < staged; first += DSX_WAVE)
-            {
-                const int at = first + lane;
-                const uint64_t mine = __builtin_amdgcn_ballot_w64(at < staged && ((uint32_t)s_reach[min(at, kWideBatch - 1)] >> wave & 1) != 0);
-                if(__builtin_amdgcn_inverse_ballot_w64(mine))
-                    list[length + bits_below_lane(mine)] = (uint16_t)at;
-                length += __popcll(mine);
-            }
-            if(lane < 8)
-                list[length + lane] = kWideBatch;
-
-            struct Entry
-            {
-                float4 A, B, C;
-            };
-            auto fetch = [&](int at) { return Entry{s_a[at], s_b[at], s_c[at]}; };
-            Entry next = fetch(list[slot]);
-            int after = list[4 + slot];
-            for(int i = 0; i < length; i += 4)
-            {
-                const Entry e = next;
-                next = fetch(after);
-                after = list[min(i + 8, length + 4) + slot];
-                float alpha;
-                uint64_t m_pass;
-                {
-#pragma clang fp contract(off)
-                    const ExponentX ex = exponent_x(e.A.z, e.A.w, pxf - e.A.x);
-                    const float dy = pyf - e.A.y;
-                    const float power = __builtin_fmaf(-__builtin_fmaf(e.B.x, dy, ex.bx), dy, ex.ax);
-                    m_pass = __builtin_amdgcn_ballot_w64(__float_as_int(power) <= __float_as_int(e.B.z));
-                    const float full = fminf(kAlphaMax, e.B.y * __builtin_amdgcn_exp2f(power * kLog2E));
-                    alpha = __builtin_amdgcn_inverse_ballot_w64(m_pass) ? full : 0.0f;
-                }
-                const float alphas[4] = {quad_lane<0x00>(alpha), quad_lane<0x55>(alpha), quad_lane<0xAA>(alpha), quad_lane<0xFF>(alpha)};
-                const float T1 = __builtin_fmaf(-alphas[0], T, T), T2 = __builtin_fmaf(-alphas[1], T1, T1);
-                const float T3 = __builtin_fmaf(-alphas[2], T2, T2), T4 = __builtin_fmaf(-alphas[3], T3, T3);
-                float before = slot & 2 ? (slot & 1 ? T3 : T2) : (slot & 1 ? T1 : T);
-                float Tn = T4;
-                if(__builtin_amdgcn_ballot_w64(T4 < 0.0001f) != 0)
-                {
-                    // some pixel becomes opaque within these entries: once more, each lane up to where its pixel stops
-                    Tn = T;
-                    bool stopped = pyf != pyf, counts = !stopped;
-#pragma unroll
-                    for(int u = 0; u < 4; ++u)
-                    {
-                        before = slot == u ? Tn : before;
-                        const float further = __builtin_fmaf(-alphas[u], Tn, Tn);
-                        stopped = stopped || further < 0.0001f;
-                        Tn = stopped ? Tn : further;
-                        counts = slot == u ? !stopped : counts;
-                    }
-                    pyf = stopped ? __builtin_nanf("") : pyf;
-                    m_pass &= __builtin_amdgcn_ballot_w64(counts);
-                    alpha = counts ? alpha : 0.0f;
-                    if(__builtin_amdgcn_ballot_w64(pyf == pyf) == 0)
-                        i = length; // no pixel left
-                }
-                T = Tn;
-                const float weight = alpha * before;
-                red = __builtin_fmaf(weight, e.C.x, red);
-                green = __builtin_fmaf(weight, e.C.y, green);
-                blue = __builtin_fmaf(weight, e.C.z, blue);
-                last = __builtin_amdgcn_inverse_ballot_w64(m_pass) ? __float_as_int(e.B.w) : last;
-            }
+            blend_staged(staged);
         }
         if(!kOwn)
             break;
@@ -1721,11 +1838,10 @@ __global__ __launch_bounds__(kWideThreads) void blend_fwd_wide_kernel(const int3
         }
         store_pixel(image, pix, (int64_t)W * H, red, green, blue, T, broken, bg, planar);
     }
-    if(!kOwn)
-        if(prep_zeros)
-            zero_grads_share(prep, prep_count, blockIdx.x, gridDim.x, tid, kWideThreads);
-        else
-            prepare_grads_share(splats, prep, prep_count, prep_marks, blockIdx.x, gridDim.x, tid, kWideThreads);
+    if(!kOwn && prep_zeros)
+        zero_grads_share(prep, prep_count, blockIdx.x, gridDim.x, tid, kWideThreads);
+    else if(!kOwn)
+        prepare_grads_share(splats, prep, prep_count, prep_marks, blockIdx.x, gridDim.x, tid, kWideThreads);
 }
 
 // Does a forward without a backward find its lists itself?
@@ -1743,10 +1859,11 @@ int launch_blend_fwd_own(const dsx_camera& cam, int64_t n, const uint32_t* depth
         return DSX_ERR_BAD_ARG;
     {
         DSX_TIMED("blend_fwd_kernel", stream);
-        hipLaunchKernelGGL(blend_fwd_wide_kernel<true>, dim3(lg.tiles()), dim3(kWideThreads), 0, stream, nullptr, nullptr,
+        const int split = lg.tiles() <= kWideSplitUpTo;
+        hipLaunchKernelGGL(blend_fwd_wide_kernel<true>, dim3(split ? 4 * lg.tiles() : lg.tiles()), dim3(kWideThreads), 0, stream, nullptr, nullptr,
                            reinterpret_cast<const float4*>(splats), image, nullptr, nullptr, cam.image_width, cam.image_height, lg.ntx,
                            (uint32_t)(n - 1), 0, nullptr, 0, nullptr, nullptr, nullptr, (int64_t)0, nullptr, 0, cam.bg,
-                           camera_flag(cam, DSX_PLANAR_IMAGE), OwnLists{depth_keys, rects, (int)n});
+                           camera_flag(cam, DSX_PLANAR_IMAGE), split, OwnLists{depth_keys, rects, (int)n, lg.tiles() - 1});
     }
     DSX_LAUNCH_CHECK();
     return DSX_OK;
@@ -1802,10 +1919,11 @@ int launch_blend_fwd(const dsx_camera& cam, int64_t n, int64_t k, int32_t* range
         const dim3 grid(ntx * nty);
         const float4* sp = reinterpret_cast<const float4*>(splats);
         const int prep_zeros = prep_marks != nullptr && zeros_alone(cam, n);
+        const int split = lg.tiles() <= kWideSplitUpTo;
         if(wide)
-            hipLaunchKernelGGL(blend_fwd_wide_kernel<false>, grid, dim3(kWideThreads), 0, stream, ranges, sorted_ids, sp, image, final_T,
+            hipLaunchKernelGGL(blend_fwd_wide_kernel<false>, dim3(split ? 4 * lg.tiles() : lg.tiles()), dim3(kWideThreads), 0, stream, ranges, sorted_ids, sp, image, final_T,
                                final_idx, cam.image_width, cam.image_height, ntx, last_id, (int)k, header, lg.shift, sort_flag_a,
-                               sort_flag_b, prep, prep_count, prep_marks, prep_zeros, cam.bg, camera_flag(cam, DSX_PLANAR_IMAGE), OwnLists{});
+                               sort_flag_b, prep, prep_count, prep_marks, prep_zeros, cam.bg, camera_flag(cam, DSX_PLANAR_IMAGE), split, OwnLists{});
 #define DSX_LAUNCH_FWD(KERNEL, THREADS)                                                                          \
     hipLaunchKernelGGL((KERNEL), grid, dim3(THREADS), 0, stream, ranges, sorted_ids, sp, image, final_T, final_idx,  \
                        cam.image_width, cam.image_height, ntx, last_id, (int)k, header, lg.shift, sort_flag_a,     \

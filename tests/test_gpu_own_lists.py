@@ -156,3 +156,23 @@ def test_a_captured_forward_without_lists_follows_its_inputs():
             assert torch.equal(image, want) and torch.equal(radii, want_radii)
             seen.append(want.clone())
         assert not torch.equal(seen[0], seen[3])
+
+
+@pytest.mark.parametrize("n,W,H", [(960, 16, 16), (961, 16, 16), (962, 16, 16), (2500, 128, 128), (2500, 208, 80), (3000, 127, 113)])
+@pytest.mark.parametrize("depths", ["spread", "equal"])
+def test_quadrants_and_entries_that_a_round_holds(blend_form, n, W, H, depths):
+    """Up to 960 entries of a tile are tested, sorted and staged in one go, and up to 64 tiles have a workgroup for each quadrant: at the edges
+    of both, the image that the tiles' own lists give, that of the general path, and the four-wavefront form's agree."""
+    sc = make_scene("cfg0", n=n, width=W, height=H, sh_degree=0, seed=n)
+    if W * H == 256:
+        sc["means_3d"][:, :2] *= 0.05
+        sc["scales"] = torch.full((n, 3), 1.0) * (1.0 + torch.rand(n, 1, generator=torch.Generator().manual_seed(n)))
+        sc["opacities"] = 0.004 + 0.02 * torch.rand(n, 1, generator=torch.Generator().manual_seed(n))
+    if depths == "equal":
+        sc["means_3d"][:, 2] = 4.0
+    assert taken(sc)
+    image = check(sc)
+    (_, _), (four, _) = (blend_form(1), render_both(sc))[1]
+    # (the sums' parts differ: as above)
+    assert float((image - four).abs().max()) <= 6e-6 * max(1.0, float(four.abs().max()))
+    assert float(image.abs().max()) > 0.1
