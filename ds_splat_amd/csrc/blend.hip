@@ -4,13 +4,14 @@
 // Both directions are bound by the issue of vector instructions: these alone take 82 % of the time where no pixel stops early (2 M
 // faint Gaussians; an exponential or a reciprocal, which takes four times as long, counts once there) and 63 to 82 % elsewhere, so
 // what counts is how many a (pixel, entry) pair costs and how many pairs are looked at that need not be.  The backward
-// also waits for its sums: timed without the adds to memory, and then with a place in LDS for each quad of lanes' own sums, 1 M large Gaussians
-// 300 -> 236 -> 209 us, 3 M 253 -> 252 -> 237, 2 M faint 1281 -> 1238 -> 1184.
-// 1920x1080 unless noted, us within a whole pass (medians of a trace), four lists of entries per wavefront -> sixteen:
-//   forward   2 M faint Gaussians 881 -> 686, 1.4 M at 1557x1038 309 -> 266, 500 K opaque 127 -> 118 (3 M: 149 -> 148),
-//             6 M at 3840x2160 509 -> 431, 1 M large ones 123 -> 125, 1 M at 1280x720 138 -> 120, 16 K at 256x256 36 -> 21
-//   backward  2 M faint 1637 -> 1274, 1.4 M at 1557x1038 519 -> 457, 500 K opaque 223 -> 216 (3 M: 254 -> 253),
-//             1 M large ones 302 -> 306, 300 K at 1237x822 244 -> 223, 50 K at 512x512 77 -> 72
+// also waits for its sums: timed without the adds to memory, and then with a place in LDS for each quad of lanes' own sums, one entry at a time,
+// 1 M large Gaussians 300 -> 236 -> 209 us, 3 M 253 -> 252 -> 237, 2 M faint 1281 -> 1238 -> 1184.
+// 1920x1080 unless noted, us within a whole pass (medians of a trace), four lists of entries per wavefront -> sixteen -> with the clamp of alpha where it
+// is needed and plain zeros beside the forward, and two entries at a time in the backward:
+//   forward   2 M faint Gaussians 881 -> 686 -> 630, 1.4 M at 1557x1038 309 -> 266 -> 254, 500 K opaque 127 -> 118 -> 115 (3 M: 149 -> 148 -> 124),
+//             6 M at 3840x2160 509 -> 431 -> 383, 1 M large ones 123 -> 125 -> 106, 1 M at 1280x720 138 -> 120 -> 115
+//   backward  2 M faint 1637 -> 1274 -> 1237, 1.4 M at 1557x1038 519 -> 457 -> 452, 500 K opaque 223 -> 216 -> 207 (3 M: 254 -> 253 -> 243),
+//             1 M large ones 302 -> 306 -> 252, 300 K at 1237x822 244 -> 223 -> 220, 50 K at 512x512 77 -> 72 -> 63
 #include "dsx_common.h"
 
 #include <atomic>
@@ -131,6 +132,8 @@ __device__ __forceinline__ uint32_t reach_limit_bwd(float opacity, float reach)
 //     mixed                                    -93   -55   -27    -2   +70  +125   (of 312 to 919)
 //     faint                                    -48   -35   -15    +9   +58  +122   (of 229 to 888)
 //     large                                    -25   -13   -16   +10    +8   -31   (of 271 to 445)
+//   the backward's kernel alone, since both take entries by pairs: 1920, 2170, 3072, 3600, 4590 tiles
+//     opaque -37, -22, +3, +8, +15; mixed -65, -38, +2, +2, +32; faint -81, -41, -68, -24, +32; large +5, -13, +22, +26, +41
 // The lines at 5500 and 3000 tiles lie within those crossings.
 // dsx_set_blend_pixels_per_lane(1 | 4) overrides the choice for the whole process (tests run both
 // forms); DSX_BLEND_PIXELS_PER_LANE=1|4 in the environment gives the override's initial value and is
@@ -1183,7 +1186,11 @@ struct OwnLists
 //   16 K            89, 112, 97, 62 -> 103, 144, 111, 61 / 61, 68, 57, 56 -> 45, 53, 42, 50 / 51, 58, 50, 58 -> 33, 40, 32, 38 / 54, 63, 52, 66 -> 30, 37, 28, 37
 //   24 K            (slower) / 74, 86, 69, 58 -> 59, 72, 56, 59 / 62, 71, 57, 61 -> 45, 53, 40, 60 / 64, 75, 61, 72 -> 40, 49, 37, 58
 //   32 K            (slower) / 77, 90, 81, 60 -> 65, 120, 71, 68 / 68, 81, 65, 63 -> 53, 66, 50, 68 / 72, 85, 68, 73 -> 49, 60, 44, 66
-// 2 K at 64x64 40 -> 24.  What ends it are the windows, each of which costs another three or four looks at everything: the line of
+// Without, since a round's entries are tested and placed in one go and quadrants have workgroups:
+//   6 K             39, 41, 36, 33 / 21, 22, 21, 28 / 21, 24, 21, 33 / 20, 22, 20, 33
+//   10 K            53, 53, 54, 42 / 32, 36, 32, 41 / 27, 32, 27, 44 / 25, 30, 26, 36
+//   16 K            70, 68, 85, 60 / 56, 60, 56, 55 / 39, 42, 39, 51 / 32, 41, 37, 51
+// 2 K at 64x64 40 -> 24 -> 18.  What ends it are the windows, each of which costs another three or four looks at everything: the line of
 // 9000 Gaussians and a hundred more for each tile lies below where the first kind of scene loses.
 constexpr int kOwnGaussians = 9000, kOwnGaussiansPerTile = 100;
 constexpr int kOwnMost = 4096; // entries of a window
