@@ -3184,13 +3184,21 @@ __global__ __launch_bounds__(kBlockThreads) void blend_bwd_block_kernel(
                 }
                 const float fac = alpha * T_here, ahead = colour - behind_here;
                 float w = (plain ? fac : vis * T_here) * ahead;
+                float v_red = fac * vo0, v_green = fac * vo1, v_blue = fac * vo2;
                 if(!plain)
-                    w = __builtin_amdgcn_inverse_ballot_w64(m_valid) ? w : 0.0f;
+                {
+                    // (a pixel that does not take the entry adds nothing, whatever its gradient: zero times infinity again)
+                    const bool takes = __builtin_amdgcn_inverse_ballot_w64(m_valid);
+                    w = takes ? w : 0.0f;
+                    v_red = takes ? v_red : 0.0f;
+                    v_green = takes ? v_green : 0.0f;
+                    v_blue = takes ? v_blue : 0.0f;
+                }
                 const float wx = w * dx, wy = w * dy;
-                const float sum8[8] = {w, wx, wx * dx, wy, wy * dx, wy * dy, fac * vo0, fac * vo1};
+                const float sum8[8] = {w, wx, wx * dx, wy, wy * dx, wy * dy, v_red, v_green};
                 float first, second;
                 bank_sum8_scatter(sum8, first, second);
-                float v_blue = dpp_add<0x128>(fac * vo2); // row_ror:8
+                v_blue = dpp_add<0x128>(v_blue);         // row_ror:8
                 v_blue += dpp_move<0x104, true>(v_blue);  // row_shl:4 (the sum in every row's first four lanes)
                 // (v_blue's two upper rows are the lower ones' other halves)
                 const float halves = add_halves(first, second);

@@ -48,7 +48,7 @@ def test_colour_gradients_where_colours_are_not_finite(oracle, blend_form, pixel
 
 
 @pytest.mark.parametrize("value", [float("inf"), float("nan")])
-@pytest.mark.parametrize("pixels_per_lane", [1, 4])
+@pytest.mark.parametrize("pixels_per_lane", [0, 1, 4])
 def test_an_infinite_colour_that_no_pixel_takes(blend_form, pixels_per_lane, value):
     """A splat between four pixels of one block, too narrow for any, gets no gradient whatever its colour and wherever it stands
     in its round of staged entries (the wide splats behind it fill the rounds of 56 and of 248)."""
@@ -109,7 +109,8 @@ def test_a_needle_is_blended_wherever_alpha_reaches_the_threshold(blend_form, pi
 
 def sums_in_64_bits(rec, v_image, bg, final_T, final_idx):
     """The nine sums of every entry, and the sums of their terms' magnitudes, back to front from what the forward
-    left, all entries in the one list of every pixel.  Also the pixels where a decision is closer than 32 bits tell."""
+    left, all entries in the one list of every pixel; a pixel has a term in the entries that it took and in no other,
+    whatever its gradient.  Also the pixels where a decision is closer than 32 bits tell."""
     h, w = final_T.shape
     y, x = torch.meshgrid(torch.arange(h) + 0.5, torch.arange(w) + 0.5, indexing="ij")
     v, T, last = v_image.double(), final_T.double().clone(), final_idx
@@ -126,11 +127,13 @@ def sums_in_64_bits(rec, v_image, bg, final_T, final_idx):
         alpha = torch.where(takes, (opacity * vis).clamp(max=0.99), torch.zeros(()).double())
         T = T / (1.0 - alpha)
         ahead = v @ torch.stack([red, green, blue]) - behind
-        behind = behind + alpha * ahead
-        vw = torch.where(takes, vis * T * ahead, torch.zeros(()).double())
+        zero = torch.zeros(()).double()
+        behind = torch.where(takes, behind + alpha * ahead, behind)
+        vw = torch.where(takes, vis * T * ahead, zero)
         s = opacity * vw
+        colour = [torch.where(takes, alpha * T * v[..., channel], zero) for channel in range(3)]
         for j, t in enumerate((s * (a * dx + b * dy), s * (b * dx + c * dy), -0.5 * s * dx * dx, -s * dx * dy,
-                               -0.5 * s * dy * dy, vw, alpha * T * v[..., 0], alpha * T * v[..., 1], alpha * T * v[..., 2])):
+                               -0.5 * s * dy * dy, vw, *colour)):
             sums[i, j], terms[i, j] = t.sum(), t.abs().sum()
     return sums, terms, close
 
@@ -140,7 +143,8 @@ def sums_in_64_bits(rec, v_image, bg, final_T, final_idx):
 @pytest.mark.parametrize("pixels_per_lane", [0, 1, 4])
 def test_backward_sums_against_64_bits(blend_form, pixels_per_lane, n, kind):
     """Around the rounds of 56 and of 248 entries, odd and even: rounds that no pixel's last entry lies in, rounds where
-    pixels end or alpha reaches the clamp, and an upstream gradient whose products with zero must stay out of the sums."""
+    pixels end or alpha reaches the clamp, and an upstream gradient too large for the walk that multiplies by zeros (one
+    that is not finite: below)."""
     from ds_splat_amd import stages
     blend_form(pixels_per_lane)
     g = torch.Generator().manual_seed(n)
@@ -174,6 +178,48 @@ def test_backward_sums_against_64_bits(blend_form, pixels_per_lane, n, kind):
     got = stages.blend_bwd(cam, n, ranges, ids, rec.to(DEV), final_T, final_idx, v_image.to(DEV))[:, :9].cpu().double()
     # (T is rebuilt over up to 500 entries, three roundings of 6e-8 each, and starts from one that the forward left)
     assert ((got - want).abs() <= 1e-4 * terms + 1e-7).all(), float(((got - want).abs() / (terms + 1e-3)).max())
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+@pytest.mark.parametrize("n", [57, 130, 300])
+@pytest.mark.parametrize("pixels_per_lane", [0, 1, 4])
+def test_a_pixels_gradient_that_is_not_finite(blend_form, pixels_per_lane, n, value):
+    """An infinite or NaN upstream gradient at a pixel that some entries took and at one that none took: it is in the sums
+    of those that took it; those of all others, in the same block's list or not, are what they are without it."""
+    from ds_splat_amd import stages
+    blend_form(pixels_per_lane)
+    g = torch.Generator().manual_seed(n)
+    rand = lambda *s: torch.rand(*s, generator=g)
+    h, w = 30, 43
+    rec = torch.zeros(n, 12)
+    rec[:, 0], rec[:, 1], rec[:, 3] = rand(n) * 0.7 * w, rand(n) * 0.7 * h, 50.0
+    rec[:, 4] = rec[:, 6] = 0.6 + rand(n)                               # (a pixel or two wide)
+    rec[:, 7], rec[:, 8:11] = 0.02 + 0.3 * rand(n), rand(n, 3)
+    # one in the empty part, which takes some pixels of its block and not the one at (36, 26)
+    rec[n // 2, :2], rec[n // 2, 4], rec[n // 2, 6], rec[n // 2, 7] = torch.tensor([38.3, 26.3]), 3.0, 3.0, 0.5
+    cam = stages.camera_from_scene(make_scene("cfg0", n=1, width=w, height=h, sh_degree=0), DEV, list_bin=1,
+                                   bg=torch.tensor([0.3, 0.1, 0.8]))
+    tiles = ((h + 15) // 16) * ((w + 15) // 16)
+    ids = torch.arange(n, dtype=torch.int32).repeat(tiles).to(DEV)
+    ranges = (torch.arange(tiles + 1, dtype=torch.int32) * n).to(DEV)
+    _, final_T, final_idx = stages.blend_fwd(cam, ranges, ids, rec.to(DEV))
+    tile_of = torch.arange(h)[:, None] // 16 * ((w + 15) // 16) + torch.arange(w)[None] // 16
+    args = torch.tensor([0.3, 0.1, 0.8]), final_T.cpu(), final_idx.cpu() - tile_of * n
+    v_image = torch.randn(h, w, 3, generator=g)
+    close = sums_in_64_bits(rec, v_image, *args)[2]
+    assert close.float().mean() < 0.2
+    v_image[close] = 0.0
+    untouched, touched = (final_T.cpu() == 1.0) & ~close, (final_T.cpu() < 0.99) & ~close
+    assert untouched[26, 36] and final_T[26, 38] < 1.0
+    y, x = torch.nonzero(touched)[len(torch.nonzero(touched)) // 2].tolist()
+    v_image[26, 36], v_image[y, x] = value, value                       # (the first: by nobody)
+    want, terms, _ = sums_in_64_bits(rec, v_image, *args)
+    got = stages.blend_bwd(cam, n, ranges, ids, rec.to(DEV), final_T, final_idx, v_image.to(DEV))[:, :9].cpu().double()
+    others = torch.isfinite(want).all(1)
+    assert 0 < int((~others).sum()) < n // 2 and others[n // 2]
+    # (T over up to 300 entries, as above)
+    assert ((got - want).abs() <= 1e-4 * terms + 1e-7)[others].all(), int((~torch.isfinite(got[others])).any(1).sum())
+    assert not torch.isfinite(got[~others]).all(1).any()
 
 
 @pytest.mark.parametrize("n, where", [(1, 0), (64, 63), (65, 64), (150, 3), (150, 70), (150, 149)])
