@@ -176,3 +176,54 @@ def test_quadrants_and_entries_that_a_round_holds(blend_form, n, W, H, depths):
     # (the sums' parts differ: as above)
     assert float((image - four).abs().max()) <= 6e-6 * max(1.0, float(four.abs().max()))
     assert float(image.abs().max()) > 0.1
+
+
+@pytest.mark.parametrize("n", [128, 129, 130, 500, 960])
+@pytest.mark.parametrize("depths", ["equal", "two", "outlier"])
+def test_entries_of_one_round_whose_depths_are_alike(n, depths):
+    """Up to 128 entries of a bin of depths are compared with each other, more are sorted: at the edges of both, all in one bin, in two,
+    and all but one, the image is the general path's."""
+    g = torch.Generator().manual_seed(n)
+    sc = make_scene("cfg0", n=n, width=16, height=16, sh_degree=0, seed=n)
+    sc["means_3d"][:, :2] *= 0.05
+    sc["scales"] = torch.ones(n, 3) * (1.0 + torch.rand(n, 1, generator=g))
+    sc["opacities"] = 0.004 + 0.02 * torch.rand(n, 1, generator=g)
+    sc["means_3d"][:, 2] = 4.0
+    if depths == "two":
+        sc["means_3d"][::3, 2] = 6.0
+    if depths == "outlier":
+        sc["means_3d"][n // 2, 2] = 9.0
+    assert taken(sc)
+    assert float(check(sc).abs().max()) > 0.01
+
+
+def test_depths_that_are_alike_take_no_longer():
+    """A plane of Gaussians that faces the camera, of which each tile has hundreds of one depth, against the same ones a little apart: the
+    same work but for the order (1.9 times as long where each entry is compared with all others of its depth, 1.3 as it is)."""
+    n = 12000
+    sc = make_scene("cfg0", n=n, width=176, height=160, sh_degree=0, seed=1)
+    assert taken(sc)
+    t = {k: (v.to(DEV) if isinstance(v, torch.Tensor) else v) for k, v in sc.items()}
+    settings = GaussianRasterizationSettings(
+        image_height=sc["height"], image_width=sc["width"], tanfovx=sc["tanfovx"], tanfovy=sc["tanfovy"], bg=t["bg"], scale_modifier=1.0,
+        viewmatrix=t["viewmatrix"], projmatrix=t["projmatrix"], sh_degree=0, max_sh_degree=3, campos=t["campos"], prefiltered=False,
+        debug=False)
+    rasterizer = GaussianRasterizer(settings)
+    apart = t["means_3d"].clone()
+    apart[:, 2] = 4.0 + 0.2 * torch.rand(n, generator=torch.Generator().manual_seed(2)).to(DEV)
+    plane = apart.clone()
+    plane[:, 2] = 4.1
+    means2d = torch.zeros_like(plane)
+    best = {}
+    with torch.no_grad():
+        for _ in range(8):
+            for name, means in (("apart", apart), ("plane", plane)):
+                begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+                begin.record()
+                for _ in range(50):
+                    rasterizer(means, means2d, t["shs"], None, t["opacities"], t["scales"], t["rotations"], None)
+                end.record()
+                end.synchronize()
+                best[name] = min(best.get(name, 1e9), begin.elapsed_time(end) / 50)
+    print("us: apart %.1f, alike %.1f" % (1e3 * best["apart"], 1e3 * best["plane"]))
+    assert best["plane"] < 1.6 * best["apart"], best
