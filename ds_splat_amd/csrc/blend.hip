@@ -2218,10 +2218,14 @@ __device__ __forceinline__ uint32_t made_here(uint32_t v)
     return v;
 }
 
-// Can an entry's product with an alpha of zero be anything but zero, or does its alpha reach the clamp?
-__device__ __forceinline__ bool plain_entry(const float4 q0, const float4 q1, const float4 q2)
+// What an entry asks of the walk: may its product with an alpha of zero be anything but zero (kAnyEntry), does its alpha reach the
+// clamp (kClampedEntry), or neither (0)?  An opacity beyond 2, which no training gives, is left to the general walk: its moments are
+// not taken times the opacity before they are summed.
+constexpr uint32_t kClampedEntry = 1, kAnyEntry = 2;
+__device__ __forceinline__ uint32_t entry_kind(const float4 q0, const float4 q1, const float4 q2)
 {
-    return q1.w <= kAlphaMaxBwd && largest(q0.x, q0.y, 0.0f) < kTame && largest(q2.x, q2.y, q2.z) < kTame;
+    const bool tame = q1.w <= 2.0f && largest(q0.x, q0.y, 0.0f) < kTame && largest(q2.x, q2.y, q2.z) < kTame;
+    return !tame ? kAnyEntry : (q1.w <= kAlphaMaxBwd ? 0 : kClampedEntry);
 }
 
 // How an entry's gradient at a pixel follows from what lies behind it: with T the transmittance in front of the
@@ -2475,14 +2479,15 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(5, 5))
         spares = found - staged;
         __syncthreads();
         uint32_t reached = 0;
-        bool special = false, last_here = false;
+        uint32_t kind = 0;
+        bool last_here = false;
         if(lane < staged)
         {
             const float4* const rec = splats + 3 * (int64_t)mine.x;
             const float4 q0 = rec[0], q1 = rec[1], q2 = rec[2];
             const float reach = reach_of(q1.w);
             last_here = mine.y > m_least;
-            special = !plain_entry(q0, q1, q2);
+            kind = entry_kind(q0, q1, q2);
             reached = blocks_reached(q0.x, q0.y, q1.x, q1.y, q1.z, reach, (float)x0 + 0.5f, (float)y0 + 0.5f);
             s_a[lane] = make_float4(q0.x, q0.y, q1.x * 0.5f, q1.y);
             s_b[lane] = make_float4(q1.z * 0.5f, q1.w, __uint_as_float(reach_limit_bwd(q1.w, reach)), __int_as_float(mine.y));
@@ -2491,7 +2496,7 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(5, 5))
         if(lane == kBwdBatch)
         {
             const float zero = __uint_as_float(made_here(0u));
-            s_c[kBwdBatch] = make_float4(zero, zero, zero, zero);
+            s_c[made_here(kBwdBatch)] = make_float4(zero, zero, zero, zero);
         }
         // (entries behind everything that a quad's pixels blended are not in its list)
 #pragma unroll
@@ -2507,8 +2512,9 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(5, 5))
         }
         __syncthreads();
         const int rounds = quad_lists<kBwdBatch>(reinterpret_cast<uint8_t*>(s_list), reached, lane);
+        const int zero = (int)made_here(0u);
         for(int i = lane; i < kBwdBatch * kSums; i += DSX_WAVE)
-            s_sum[i] = 0.0;
+            s_sum[i] = __hiloint2double(zero, zero);
         __syncthreads();
 
         // Two entries at a time, without branches: a pixel that does not take an entry gives it the alpha zero.  Both
@@ -2521,7 +2527,11 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(5, 5))
         // (255), 300 K at 1237x822 225 -> 215 (221).  Distance of the gradients from a 64-bit evaluation (scenes of 700 records; means, conics,
         // opacities, 1e-7): ordinary 3.1, 3.0, 3.0 -> 2.9, 2.8, 2.8; opacity 0.9 3.6, 3.5, 3.3 -> 3.2, 3.2, 2.9; large 5.1, 5.4, 6.5 -> 4.6, 3.5, 4.9;
         // faint 2.1, 2.2, 2.0 -> 2.0, 2.1, 1.9; hardly wider than a pixel 1.2, 1.3, 1.1 -> 1.2, 1.4, 1.1.
-        auto walk_pairs = [&](auto ends) {
+        // clamps: some entry's alpha may reach the clamp, which the moments do not see: three instructions more a pixel and entry.  One such
+        // entry in a round is the rule where a scene has been trained for long; us, the general walk for these rounds (one entry at
+        // a time) -> this, half of the opacities beyond the clamp: 1.4 M at 1557x1038 143 -> 123, 500 K 157 -> 145, 3 M 215 -> 200, 300 K at 1237x822 142 ->
+        // 132.  (The distance from 64 bits: as before for conics, opacities and colours, 0 to 15 % less for means.)
+        auto walk_pairs = [&](auto ends, auto clamps) {
         const uint16_t* my_list = reinterpret_cast<const uint16_t*>(s_list) + made_here(block) * (kBwdBatch / 2);
         int places = *my_list;
         // (zeros at first, for each quad elsewhere)
@@ -2550,7 +2560,8 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(5, 5))
             asm volatile("" ::: "memory");
             add_sums();
             summed_places = here;
-            float alpha[2][kPix], dx[2], dy0[2];
+            float unclamped[2][kPix], dx[2], dy0[2];
+            auto clamped = [&](float alpha) { return clamps ? fminf(kAlphaMaxBwd, alpha) : alpha; };
 #pragma unroll
             for(int u = 0; u < 2; ++u)
             {
@@ -2567,7 +2578,7 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(5, 5))
                     if(ends)
                         m_valid &= __builtin_amdgcn_ballot_w64(__float_as_int(B[u].w) <= bin_final[p]);
                     const float full = B[u].y * __builtin_amdgcn_exp2f(-sigma * kLog2E);
-                    alpha[u][p] = __builtin_amdgcn_inverse_ballot_w64(m_valid) ? full : 0.0f;
+                    unclamped[u][p] = __builtin_amdgcn_inverse_ballot_w64(m_valid) ? full : 0.0f;
                     if(p == 0)
                         dy0[u] = dy;
                 }
@@ -2576,9 +2587,9 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(5, 5))
 #pragma unroll
             for(int p = 0; p < kPix; ++p)
             {
-                const float through = 1.0f - alpha[0][p];
-                T[p] *= __builtin_amdgcn_rcpf(__builtin_fmaf(-alpha[1][p], through, through));
-                between[p] = __builtin_fmaf(-alpha[1][p], T[p], T[p]);
+                const float alpha1 = clamped(unclamped[1][p]), through = 1.0f - clamped(unclamped[0][p]);
+                T[p] *= __builtin_amdgcn_rcpf(__builtin_fmaf(-alpha1, through, through));
+                between[p] = __builtin_fmaf(-alpha1, T[p], T[p]);
             }
             float blue[2];
 #pragma unroll
@@ -2590,13 +2601,13 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(5, 5))
 #pragma unroll
                 for(int p = 0; p < kPix; ++p)
                 {
-                    const float fac = alpha[u][p] * (u == 0 ? between[p] : T[p]);
+                    const float alpha = clamped(unclamped[u][p]), T_here = u == 0 ? between[p] : T[p], fac = alpha * T_here;
                     v_red = p == 0 ? fac * vo0[p] : v_red + fac * vo0[p];
                     v_green = p == 0 ? fac * vo1[p] : v_green + fac * vo1[p];
                     v_blue = p == 0 ? fac * vo2[p] : v_blue + fac * vo2[p];
                     const float ahead = C[u].x * vo0[p] + (C[u].y * vo1[p] + (C[u].z * vo2[p] - behind[p]));
-                    behind[p] += alpha[u][p] * ahead;
-                    w[p] = fac * ahead;
+                    behind[p] += alpha * ahead;
+                    w[p] = (clamps ? unclamped[u][p] * T_here : fac) * ahead;
                 }
                 // 1 | dy | dy^2
                 static_assert(kPix == 4, "two times two rows");
@@ -2619,7 +2630,7 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(5, 5))
         }
         add_sums();
         };
-        // what the walk above leaves out: clamped alphas, and values so large that a product with zero is not zero
+        // what the walk above leaves out: values so large that a product with zero is not zero
         auto walk_any = [&]() {
         const uint16_t* my_list = reinterpret_cast<const uint16_t*>(s_list) + made_here(block) * (kBwdBatch / 2);
         int places = *my_list;
@@ -2695,8 +2706,8 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(5, 5))
             }
         }
         };
-        const bool all_plain = !wild && __builtin_amdgcn_ballot_w64(special) == 0;
-        if(!all_plain)
+        const bool in_pairs = !wild && __builtin_amdgcn_ballot_w64((kind & kAnyEntry) != 0) == 0;
+        if(!in_pairs)
         {
             walk_any();
             bool still = true;
@@ -2705,15 +2716,17 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(5, 5))
                 still = still && fabsf(behind[p]) < kTame;
             wild = wild || __builtin_amdgcn_ballot_w64(!still) != 0; // (an infinite colour stays behind all entries in front)
         }
+        else if(__builtin_amdgcn_ballot_w64((kind & kClampedEntry) != 0) != 0)
+            walk_pairs(std::true_type(), std::true_type());
         else if(__builtin_amdgcn_ballot_w64(last_here) != 0) // (some pixel's last entry lies among these: one compare a pixel and entry more)
-            walk_pairs(std::true_type());
+            walk_pairs(std::true_type(), std::false_type());
         else
-            walk_pairs(std::false_type());
+            walk_pairs(std::false_type(), std::false_type());
         __syncthreads();
         if(lane < staged)
         {
             s_ids[lane] = mine.x;
-            moments_to_gradients<kBwdBatch>(s_sum, lane, s_a[lane], s_b[lane], all_plain, marks ? marks + mine.x : nullptr);
+            moments_to_gradients<kBwdBatch>(s_sum, lane, s_a[lane], s_b[lane], in_pairs, marks ? marks + mine.x : nullptr);
         }
         summed = staged;
     }
@@ -2743,7 +2756,7 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
     __shared__ uint32_t s_list[kTileWaves * kTileBatch + 1]; // (one word more: read ahead)
     __shared__ TileScan s_scan;
     __shared__ int s_counts[kTileWaves];
-    __shared__ uint32_t s_special[kTileWaves]; // per wavefront: does this round need the general walk?
+    __shared__ uint32_t s_special[kTileWaves]; // per wavefront: the kinds of its entries (entry_kind)
     __shared__ int s_last[4 * kTileWaves]; // per block: the last entry that any of its pixels blended
     int* const s_queue = reinterpret_cast<int*>(s_list); // (free while a round is staged)
 
@@ -2844,7 +2857,7 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
                 id_ahead = ids[pos - tid];
         }
         uint32_t reached = 0;
-        bool special = wild;
+        uint32_t kind = wild ? kAnyEntry : 0;
         float4 q0, q1, q2;
         float reach = 0.0f;
         const int idx = idx_next - tid;
@@ -2859,14 +2872,15 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
             for(int b = 0; b < 4 * kTileWaves; ++b)
                 if(idx > s_last[b])
                     reached &= ~(1u << b);
-            special = special || (reached != 0 && !plain_entry(q0, q1, q2));
+            kind |= reached != 0 ? entry_kind(q0, q1, q2) : 0;
         }
         if(tid < batch) // (the loads end here: behind the adds they would wait for those)
             asm volatile("" : "+v"(q2.x), "+v"(q2.y), "+v"(q2.z), "+v"(q2.w));
         flush_sums<kTileBatch + 1>(s_sum, s_id, summed, grads, tid, kTileThreads);
-        const bool mine_special = __builtin_amdgcn_ballot_w64(special) != 0;
+        const uint32_t kinds = (__builtin_amdgcn_ballot_w64((kind & kClampedEntry) != 0) != 0 ? kClampedEntry : 0) |
+                               (__builtin_amdgcn_ballot_w64((kind & kAnyEntry) != 0) != 0 ? kAnyEntry : 0);
         if(lane == 0)
-            s_special[wave] = mine_special;
+            s_special[wave] = kinds;
         int staged;
         const int place = tile_place(s_counts, __builtin_amdgcn_ballot_w64(reached != 0), staged);
         // (the barrier inside: the queue has been read, the last round's sums have been taken)
@@ -2889,12 +2903,14 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
         const int rounds = (build_lists(s_list, s_reach, staged, wave, first_block, lane) + kBwdAtOnce - 1) / kBwdAtOnce;
         const uint16_t* my_list = reinterpret_cast<const uint16_t*>(s_list + wave * kTileBatch + row * (kTileBatch / 4));
         // (one walk for all wavefronts: the sums' unit depends on it)
-        const bool all_plain = __builtin_amdgcn_readfirstlane(s_special[0] | s_special[1] | s_special[2] | s_special[3]) == 0;
-        if(all_plain)
-        {
+        const uint32_t all_kinds = __builtin_amdgcn_readfirstlane(s_special[0] | s_special[1] | s_special[2] | s_special[3]);
+        const bool in_pairs = all_kinds < kAnyEntry;
+        auto walk_pairs = [&](auto clamps) {
             // Two entries at a time as in the wavefront form.  Of the sixteen sums of their moments and colours each lane gets one: one add
             // to LDS of all lanes for two entries instead of two of nine lanes of a row.  us: 50 K at 512x512 71 -> 62, 100 K at
             // 979x546 98 -> 88; the gradients' distance from a 64-bit evaluation 3 to 30 % less (hardly wider than a pixel: the same).
+            // Where alphas may reach the clamp (general walk -> this, half of the opacities beyond it): 50 K at 512x512 39 -> 35, 200 K
+            // 70 -> 62, 100 K at 979x546 88 -> 78, 400 K 92 -> 80.
             int places = *my_list;
             int summed_places = 4 * row | 4 * row << 8; // (zeros at first, elsewhere for each row)
             float sums_one = 0.0f, sums_blue = 0.0f;
@@ -2914,7 +2930,7 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
                 asm volatile("" ::: "memory");
                 add_sums();
                 summed_places = here;
-                float alpha[2], dx[2], dy[2];
+                float reached_alpha[2], alpha[2], dx[2], dy[2]; // (before and after the clamp)
 #pragma unroll
                 for(int u = 0; u < 2; ++u)
                 {
@@ -2926,7 +2942,8 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
                     const uint64_t m_valid = __builtin_amdgcn_ballot_w64(__float_as_int(B[u].w) <= bin_final) &
                                              __builtin_amdgcn_ballot_w64(__float_as_uint(sigma) <= __float_as_uint(B[u].z));
                     const float full = B[u].y * __builtin_amdgcn_exp2f(-sigma * kLog2E);
-                    alpha[u] = __builtin_amdgcn_inverse_ballot_w64(m_valid) ? full : 0.0f;
+                    reached_alpha[u] = __builtin_amdgcn_inverse_ballot_w64(m_valid) ? full : 0.0f;
+                    alpha[u] = clamps ? fminf(kAlphaMaxBwd, reached_alpha[u]) : reached_alpha[u];
                 }
                 const float through = 1.0f - alpha[0];
                 T *= __builtin_amdgcn_rcpf(__builtin_fmaf(-alpha[1], through, through));
@@ -2934,10 +2951,12 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
 #pragma unroll
                 for(int u = 0; u < 2; ++u)
                 {
-                    const float fac = alpha[u] * (u == 0 ? __builtin_fmaf(-alpha[1], T, T) : T);
+                    const float T_here = u == 0 ? __builtin_fmaf(-alpha[1], T, T) : T;
+                    const float fac = alpha[u] * T_here;
                     const float ahead = C[u].x * vo0 + (C[u].y * vo1 + (C[u].z * vo2 - behind));
                     behind += alpha[u] * ahead;
-                    const float w = fac * ahead, wx = w * dx[u], wy = w * dy[u];
+                    // (of the unclamped alpha: the opacity times vis)
+                    const float w = (clamps ? reached_alpha[u] * T_here : fac) * ahead, wx = w * dx[u], wy = w * dy[u];
                     v[u][0] = w, v[u][1] = wx, v[u][2] = wx * dx[u], v[u][3] = wy;
                     v[u][4] = wy * dx[u], v[u][5] = wy * dy[u], v[u][6] = fac * vo0, v[u][7] = fac * vo1;
                     blue[u] = fac * vo2;
@@ -2945,7 +2964,11 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
                 row_sum16_scatter(v[0], v[1], blue[0], blue[1], lane, sums_one, sums_blue);
             }
             add_sums();
-        }
+        };
+        if(all_kinds == 0)
+            walk_pairs(std::false_type());
+        else if(in_pairs)
+            walk_pairs(std::true_type());
         else
         {
             for(int i = 0; i < rounds; ++i)
@@ -3011,7 +3034,7 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
         }
         __syncthreads();
         for(int e = tid; e < staged; e += kTileThreads)
-            moments_to_gradients<kTileBatch + 1>(s_sum, e, s_a[e], s_b[e], all_plain, marks ? marks + s_id[e] : nullptr);
+            moments_to_gradients<kTileBatch + 1>(s_sum, e, s_a[e], s_b[e], in_pairs, marks ? marks + s_id[e] : nullptr);
         __syncthreads();
         summed = staged;
     }
@@ -3149,7 +3172,7 @@ __global__ __launch_bounds__(kBlockThreads) void blend_bwd_block_kernel(
             for(int w = 0; w < kTileWaves; ++w)
                 if(idx <= s_last[w])
                     reached |= blocks & (1u << block_of_row(w));
-            special = special || (reached != 0 && !plain_entry(q0, q1, q2));
+            special = special || (reached != 0 && entry_kind(q0, q1, q2) != 0);
         }
         if(tid < batch) // (the loads end here: behind the adds they would wait for those)
             asm volatile("" : "+v"(q2.x), "+v"(q2.y), "+v"(q2.z), "+v"(q2.w));

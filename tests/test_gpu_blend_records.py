@@ -227,6 +227,38 @@ def test_a_pixels_gradient_that_is_not_finite(blend_form, pixels_per_lane, n, va
     assert not torch.isfinite(got[~others]).all(1).any()
 
 
+@pytest.mark.parametrize("opacity", [0.99, 0.9900001, 1.0, 2.0, 2.5, 300.0])
+@pytest.mark.parametrize("n, where", [(2, 1), (57, 3), (250, 249)])
+@pytest.mark.parametrize("pixels_per_lane", [0, 1, 4])
+def test_sums_where_one_opacity_lies_at_a_limit_of_the_walks(blend_form, pixels_per_lane, n, where, opacity):
+    """Rounds of the backward whose alphas stay below the clamp, rounds that reach it, and rounds with an opacity beyond 2 take different
+    walks: one opacity on either side of each limit among ordinary ones, in the first round and in a later one."""
+    from ds_splat_amd import stages
+    blend_form(pixels_per_lane)
+    g = torch.Generator().manual_seed(n)
+    rand = lambda *s: torch.rand(*s, generator=g)
+    h, w = 16, 16
+    rec = torch.zeros(n, 12)
+    rec[:, 0], rec[:, 1], rec[:, 3] = rand(n) * w, rand(n) * h, 50.0
+    rec[:, 4] = rec[:, 6] = 0.02 + 0.2 * rand(n)
+    rec[:, 7], rec[:, 8:11] = 0.01 + 0.03 * rand(n), rand(n, 3)
+    rec[where, :2], rec[where, 7] = torch.tensor([8.5, 7.5]), opacity    # (on a pixel's centre but for the sign of sigma)
+    bg = torch.tensor([0.3, 0.1, 0.8])
+    cam = stages.camera_from_scene(make_scene("cfg0", n=1, width=w, height=h, sh_degree=0), DEV, list_bin=1, bg=bg)
+    ids, ranges = torch.arange(n, dtype=torch.int32).to(DEV), torch.tensor([0, n], dtype=torch.int32).to(DEV)
+    _, final_T, final_idx = stages.blend_fwd(cam, ranges, ids, rec.to(DEV))
+    v_image = torch.randn(h, w, 3, generator=g)
+    args = bg, final_T.cpu(), final_idx.cpu()
+    close = sums_in_64_bits(rec, v_image, *args)[2]
+    assert close.float().mean() < 0.2
+    v_image[close] = 0.0
+    want, terms, _ = sums_in_64_bits(rec, v_image, *args)
+    assert (terms[where] > 0).all()
+    got = stages.blend_bwd(cam, n, ranges, ids, rec.to(DEV), final_T, final_idx, v_image.to(DEV))[:, :9].cpu().double()
+    # (as above: T over up to 250 entries)
+    assert ((got - want).abs() <= 1e-4 * terms + 1e-7).all(), float(((got - want).abs() / (terms + 1e-3)).max())
+
+
 @pytest.mark.parametrize("n, where", [(1, 0), (64, 63), (65, 64), (150, 3), (150, 70), (150, 149)])
 def test_alpha_is_clamped_in_the_rounds_that_need_it(blend_form, n, where):
     """One opaque splat on a pixel's centre among faint ones, in any round of 64 staged entries: the forms of the
