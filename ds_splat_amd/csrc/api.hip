@@ -149,12 +149,23 @@ extern "C" int32_t dsx_sort_passes(int32_t num_tiles)
 
 extern "C" size_t dsx_workspace_bytes(int64_t n, int64_t k, int32_t width, int32_t height, int32_t list_bin)
 {
-    (void)n; // (whatever the number of Gaussians: one wide digit's workspace is the larger one)
+    (void)n; // (enough for any number of Gaussians)
     if(!valid_list_bin(list_bin))
         return 0;
     const ListGrid lg = list_grid(width, height, list_bin);
-    return std::max(lists_workspace(0, k < 0 ? 0 : k, lg.lists(), lg.shift != 0).bytes,
-                    lists_workspace(INT64_MAX, k < 0 ? 0 : k, lg.lists(), lg.shift != 0).bytes);
+    const bool binned = lg.shift != 0;
+    k = std::max<int64_t>(k, 0);
+    // and for any smaller number of pairs: one wide digit, or smaller tiles of keys, take more statuses than what lies behind their limits
+    size_t bytes = 0;
+    auto with = [&](int64_t pairs) {
+        for(const int64_t gaussians : {(int64_t)0, INT64_MAX})
+            bytes = std::max(bytes, lists_workspace(gaussians, pairs, lg.lists(), binned).bytes);
+    };
+    with(k);
+    with(std::min(k, wide_digit_most(slot_bits(lg.lists()), 0, binned)));
+    for(int items = 1; items < kSortItemsMax32; ++items)
+        with(std::min(k, (int64_t)items * kSortThreads32 * kSortTilesWanted32));
+    return bytes;
 }
 
 extern "C" int32_t dsx_list_bin(int32_t width, int32_t height, int32_t list_bin)
@@ -419,7 +430,7 @@ extern "C" int dsx_sort_flags(int64_t n, int64_t k, int32_t width, int32_t heigh
             const ListGrid lg = list_grid(width, height, list_bin);
             const int tiles = lg.lists();
             const ListsWorkspace lw = lists_workspace(n, k, tiles, lg.shift != 0);
-            const Sort32Workspace w = sort32_workspace(k, slot_bits(tiles), sort32_tile_keys(k), one_wide_digit(slot_bits(tiles), n));
+            const Sort32Workspace w = sort32_workspace(k, slot_bits(tiles), sort32_tile_keys(k), one_wide_digit(slot_bits(tiles), n, k, lg.shift != 0));
             *partition_flag =
                 reinterpret_cast<const uint32_t*>(static_cast<const char*>(workspace) + lw.sort + w.counters) + w.passes;
         }

@@ -154,26 +154,36 @@ inline Digits32 digits32(int key_bits)
     }
     return d;
 }
-// The digits of the partition by list: one of nine to eleven bits instead of two.  A pass over few pairs lasts as long as one tile's
-// serial work and the chain, whatever its digits; a wide digit costs LDS for the wavefronts' counts (64 KB at eleven bits: one workgroup
-// on a compute unit instead of two) and statuses (8 KB a tile), which many pairs feel.  us of a forward, two digits -> one, with little and with
-// much overlap:
-//   Gaussians                  4 K               30 K             130 K              300 K              1 M            3 M
-//   9 bits   (420 tiles)   42 -> 37, 44 -> 40  56 -> 50, 79 -> 72  109 -> 101, 98 -> 90  156 -> 145, 126 -> 113  198 -> 185  376 -> 360
-//   10 bits  (750 tiles)   41 -> 37, 45 -> 42  54 -> 51, 79 -> 75  95 -> 90, 102 -> 95   144 -> 140, 129 -> 121  196 -> 187  384 -> 377
-//   11 bits (1024 tiles)   41 -> 38, 46 -> 44  55 -> 52, 81 -> 77  98 -> 94, 107 -> 100  152 -> 154, 142 -> 148  201 -> 196  401 -> 398
-//   11 bits (1936 tiles)   46 -> 43, 52 -> 49  60 -> 56, 90 -> 86  98 -> 94, 122 -> 114  152 -> 153, 166 -> 168  222 -> 222  427 -> 433
-//   11 bits (2040 bins, 6 M Gaussians at 3840x2160) 932 -> 936
-constexpr int kWideBits = 11, kWideAlways = 10;
-constexpr int64_t kWideUpTo = 131072; // Gaussians
-inline bool one_wide_digit(int slot_bits, int64_t n)
+// The partition by list takes one digit of nine to eleven bits instead of two where the pairs are not too many.  A pass over few pairs lasts
+// as long as one tile's serial work and the chain, whatever its digits; a wide digit costs LDS for the wavefronts' counts (one
+// workgroup on a compute unit instead of two with eleven bits, and with ten and tiles of 12 keys a thread) and statuses (8 KB a tile at eleven
+// bits), which many pairs feel.  us of a forward, two digits -> one, by bits and lists; 10 K, 60 K, 250 K and 1 M Gaussians of growing size:
+//   Million pairs    0.3         0.8 to 1.2   2 to 3       4 to 5       6 to 8       10 to 12     16 to 20     30 to 57
+//   9,  441 tiles    65 -> 57    78 -> 70     84 -> 73     139 -> 122                127 -> 104   165 -> 130
+//   10, 800 tiles    81 -> 76    84 -> 78     91 -> 82     101 -> 89    204 -> 198   132 -> 129   171 -> 174   245 -> 255
+//   10, 1000 tiles   82 -> 77    85 -> 79     90 -> 82     107 -> 102   95 -> 90     140 -> 139   189 -> 194   265 -> 290
+//   11, 1024 tiles   82 -> 78    88 -> 83     94 -> 87     108 -> 104   116 -> 107   143 -> 146   205 -> 216   314 -> 340
+//   11, 1444 tiles   83 -> 79    75 -> 71     86 -> 80     100 -> 96    132 -> 128   126 -> 127   174 -> 186   248 -> 286
+//   11, 1936 tiles   88 -> 84    88 -> 82     104 -> 97    118 -> 117   121 -> 119   150 -> 153   208 -> 226   320 -> 381
+//   11, 2040 bins    160 -> 156  315 -> 309   361 -> 354   347 -> 348   261 -> 265   353 -> 356   377 -> 410   518 -> 597
+// With more Gaussians eleven bits gain nothing: 300 K of 1024 tiles 152 -> 154 and 142 -> 148, 1 M of 1936 tiles 222 -> 222, 3 M 427 -> 433.
+constexpr int kWideBits = 11;
+constexpr int64_t kWideUpTo = 131072; // Gaussians, for eleven bits
+// the most pairs that are partitioned by one digit (0: none).  binned: lists per bin, whose slot words are twice as wide
+inline int64_t wide_digit_most(int slot_bits, int64_t n, bool binned)
 {
-    return slot_bits > kBits32 && slot_bits <= (n <= kWideUpTo ? kWideBits : kWideAlways);
+    if(slot_bits <= kBits32 || slot_bits > kWideBits || (slot_bits == kWideBits && n > kWideUpTo))
+        return 0;
+    return slot_bits == 9 ? 1ll << 30 : (slot_bits == 10 ? 12000000 : (binned ? 3500000 : 8000000));
 }
-inline Digits32 partition_digits(int slot_bits, int64_t n)
+inline bool one_wide_digit(int slot_bits, int64_t n, int64_t k, bool binned)
+{
+    return k <= wide_digit_most(slot_bits, n, binned);
+}
+inline Digits32 partition_digits(int slot_bits, bool wide)
 {
     Digits32 d = digits32(slot_bits);
-    if(one_wide_digit(slot_bits, n))
+    if(wide)
     {
         d.passes = 1;
         d.mask[0] = (1u << slot_bits) - 1u;
@@ -330,7 +340,7 @@ struct OrderLayout
     size_t rects32;    // uint32[n]  packed rectangles on their way through the depth sort
     size_t block_sums; // uint32[blocks + 1] tile counts of 256 consecutive Gaussians IN DEPTH ORDER, scanned
     size_t key_ranges; // uint2[blocks] of 256 consecutive Gaussians: 0xffff - the smallest upper half of a key that emits, and how many emit << 16; the largest one
-    size_t slot_hist;  // uint32[kMaxPasses32 * 256] digit histograms of the tile slots of all pairs
+    size_t slot_hist;  // uint32[2048] digit histograms of the tile slots of all pairs (one wide digit's, or 256 words for each of the others)
     size_t cover;      // int32[(ntx + 1) * (nty + 1) + 1] pairs per tile (corner grid, then its 2-D prefix sum)
     size_t bin_cover;  // int32[(nbx + 1) * (nby + 1) + 1] the same per bin (binned lists only)
     size_t key_count;  // uint64[5]  pairs of the per-tile lists, pairs of the bin lists (summed by the corner-grid kernel), workgroups done (of three kinds)

@@ -699,7 +699,7 @@ static int sort32_passes(int64_t count, int key_bits, KeyT* keys_a, uint32_t* va
 {
     constexpr bool kWide = kBits > kBits32; // (one digit of kBits bits)
     const Sort32Workspace w = sort32_workspace(count, key_bits, kThreads * kItems, kWide);
-    const Digits32 plan = kWide ? partition_digits(kBits, 0) : digits32(key_bits);
+    const Digits32 plan = kWide ? partition_digits(kBits, true) : digits32(key_bits);
     char* base = static_cast<char*>(sort_ws);
     uint32_t* hist = reinterpret_cast<uint32_t*>(base + w.hist);
     uint32_t* counters = reinterpret_cast<uint32_t*>(base + w.counters);
@@ -1065,7 +1065,8 @@ OrderLayout order_layout(int64_t n, int image_width, int image_height, int list_
     o.key_ranges = off;
     off = align(off + (size_t)((n + kProjBlock - 1) / kProjBlock) * 8);
     o.slot_hist = off;
-    off = align(off + std::max((size_t)kMaxPasses32 * kBins32, (size_t)1 << kWideBits) * 4);
+    static_assert(kMaxPasses32 * kBins32 <= 1 << kWideBits, "either");
+    off = align(off + ((size_t)1 << kWideBits) * 4);
     o.sort = off;
     off = align(off + sort32_workspace(n, 32, sort32_tile_keys(n)).bytes);
     const ListGrid g = list_grid(image_width, image_height, list_bin);
@@ -2605,7 +2606,7 @@ static CountsJobs counts_jobs(const ListGrid& lg, int64_t n, char* base, const O
     fine.ntx = lg.ntx;
     fine.nty = lg.nty;
     fine.plain = 0;
-    fine.plan = partition_digits(slot_bits(lg.tiles()), n);
+    fine.plan = partition_digits(slot_bits(lg.tiles()), wide_digit_most(slot_bits(lg.tiles()), n, false) > 0);
     fine.slot_hist = lg.shift ? nullptr : reinterpret_cast<uint32_t*>(base + o.slot_hist);
     fine.ranges = ranges + rl.fine;
     fine.last = lg.shift ? ranges + rl.last_tile : nullptr;
@@ -2619,7 +2620,7 @@ static CountsJobs counts_jobs(const ListGrid& lg, int64_t n, char* base, const O
         bins.ntx = lg.nbx;
         bins.nty = lg.nby;
         bins.plain = 1;
-        bins.plan = partition_digits(slot_bits(lg.bins()), n);
+        bins.plan = partition_digits(slot_bits(lg.bins()), wide_digit_most(slot_bits(lg.bins()), n, true) > 0);
         bins.slot_hist = reinterpret_cast<uint32_t*>(base + o.slot_hist);
         bins.ranges = ranges + rl.bins;
         bins.last = nullptr;
@@ -3066,6 +3067,33 @@ struct __attribute__((packed, aligned(alignof(T)))) Quad
     T v[kEmitQuad];
 };
 
+// The histograms of two digits (256 words each) from that of one digit of both, where more pairs were found than one digit is taken for.
+// (Not where the slots are counted: there it made the counting of 32400 tiles 43 -> 48 us, whose loop the compiler then laid out
+// otherwise; as a launch of its own it takes 3 us.)
+struct NarrowJob
+{
+    const uint32_t* wide;
+    uint32_t* two; // null: none
+    int slots;     // of `wide`; what lies behind them is not counted
+    int shift;     // bits of the first digit
+};
+__device__ __forceinline__ void narrow_digits(const NarrowJob& J, uint32_t* hist, int tid)
+{
+    __syncthreads();
+    for(int j = tid; j < 2 * kBins32; j += kProjBlock)
+        hist[j] = 0;
+    __syncthreads();
+    for(int slot = tid; slot < J.slots; slot += kProjBlock)
+    {
+        const uint32_t count = J.wide[slot];
+        atomicAdd(&hist[slot & ((1 << J.shift) - 1)], count);
+        atomicAdd(&hist[kBins32 + (slot >> J.shift)], count);
+    }
+    __syncthreads();
+    for(int j = tid; j < 2 * kBins32; j += kProjBlock)
+        J.two[j] = hist[j];
+}
+
 // kMasks (lists per bin, SlotT = uint32_t): the high half of a pair's slot word says which tiles of the
 // bin the Gaussian's rectangle covers, bit x for the columns and bit 8 + y for the rows of the bin
 // (a rectangle is the product of a column range and a row range).  The partition sorts by the low bits
@@ -3081,7 +3109,7 @@ __global__ __launch_bounds__(kProjBlock) void emit_ordered_kernel(const uint32_t
                                                                   const int32_t* __restrict__ ranges_in,
                                                                   int32_t* __restrict__ ranges_out, int range_count,
                                                                   uint32_t* __restrict__ clear, int64_t clear_words,
-                                                                  int chunk)
+                                                                  int chunk, const NarrowJob narrow)
 {
     // per Gaussian of the block: x = first output, y = slot of the rectangle's first tile or bin, z = lists in
     // a row of the rectangle (16 bits; bit 31: a negative depth, all pairs go to slot 0), with masks also the
@@ -3107,11 +3135,16 @@ __global__ __launch_bounds__(kProjBlock) void emit_ordered_kernel(const uint32_t
     // housekeeping for the partition that follows: its counters and look-back statuses start at zero
     for(int64_t j = (int64_t)blockIdx.x * kProjBlock + tid; j < clear_words; j += (int64_t)gridDim.x * kProjBlock)
         clear[j] = 0u;
+    if(narrow.two && blockIdx.x == 0) // (a workgroup more than there are shares, and the first to start)
+    {
+        narrow_digits(narrow, reinterpret_cast<uint32_t*>(s_rec), tid);
+        return;
+    }
 
     // This workgroup's share: outputs [o0, o1).  The work is cut by OUTPUTS, not by Gaussians: a
     // block of 256 near Gaussians can own a hundred thousand pairs and a block of far ones a few
     // hundred, and a workgroup that walked a whole heavy block alone set the kernel's time.
-    const int64_t o0 = (int64_t)blockIdx.x * chunk;
+    const int64_t o0 = (int64_t)(blockIdx.x - (narrow.two ? 1u : 0u)) * chunk;
     const int64_t o1 = min(o0 + chunk, k);
     if(o0 >= o1) // uniform
         return;
@@ -3292,8 +3325,8 @@ ListsWorkspace lists_workspace(int64_t n, int64_t k, int num_tiles, bool binned)
     auto align = [](size_t x) { return (x + 255) & ~(size_t)255; };
     ListsWorkspace w;
     const size_t slot_bytes = (binned || !slots_are_u16(num_tiles)) ? 4 : 2;
-    const bool wide = one_wide_digit(slot_bits(num_tiles), n);
-    w.passes = partition_digits(slot_bits(num_tiles), n).passes;
+    const bool wide = one_wide_digit(slot_bits(num_tiles), n, k, binned);
+    w.passes = partition_digits(slot_bits(num_tiles), wide).passes;
     size_t off = 0;
     w.slots_a = off;
     off = align(off + (size_t)k * slot_bytes);
@@ -3330,7 +3363,7 @@ static int tile_lists_impl(const dsx_camera& cam, int64_t n, int64_t k, int num_
     }
     const ListsWorkspace w = lists_workspace(n, k, num_tiles, kMasks);
     const int bits = slot_bits(num_tiles);
-    const bool wide = one_wide_digit(bits, n);
+    const bool wide = one_wide_digit(bits, n, k, kMasks);
     char* base = static_cast<char*>(workspace);
     uint32_t* ids_final = reinterpret_cast<uint32_t*>(sorted_ids);
     uint32_t* ids_other = reinterpret_cast<uint32_t*>(base + w.ids_alt);
@@ -3345,18 +3378,28 @@ static int tile_lists_impl(const dsx_camera& cam, int64_t n, int64_t k, int num_
     SlotT* slots_b = (kMasks && even) ? slots_other : slots_final;
     int rc = DSX_OK;
     const Sort32Workspace sw = sort32_workspace(k, bits, sort32_tile_keys(k), wide);
+    const uint32_t* counts = reinterpret_cast<const uint32_t*>(obase + o.slot_hist);
+    NarrowJob narrow = {};
+    if(!wide && wide_digit_most(bits, n, kMasks) > 0) // (counted for one digit before the number of pairs was known)
+    {
+        static_assert(kWideBits <= 2 * kBits32 && sizeof(uint4) * kProjBlock >= 2 * kBins32 * 4, "two digits, in the records' memory");
+        narrow = {counts, reinterpret_cast<uint32_t*>(base + w.sort + sw.hist), num_tiles + 1, digits32(bits).shift[1]};
+        counts = narrow.two;
+    }
+    // (what lies behind the histogram starts at zero)
+    const size_t clear_from = narrow.two ? sw.counters : sw.hist;
     {
         DSX_TIMED("emit_ordered_kernel", stream);
         // outputs per workgroup: a multiple of 256 between 256 and kEmitChunkMax
         const int64_t want = (k + kEmitWorkgroups - 1) / kEmitWorkgroups;
         const int chunk = (int)min((int64_t)kEmitChunkMax, ((want + kProjBlock - 1) / kProjBlock) * kProjBlock);
-        hipLaunchKernelGGL((emit_ordered_kernel<SlotT, kMasks>), dim3((unsigned)((k + chunk - 1) / chunk)),
+        hipLaunchKernelGGL((emit_ordered_kernel<SlotT, kMasks>), dim3((unsigned)((k + chunk - 1) / chunk) + (narrow.two ? 1 : 0)),
                            dim3(kProjBlock), 0, stream, reinterpret_cast<const uint32_t*>(obase + o.ids_a),
                            reinterpret_cast<const uint2*>(obase + o.rects_sorted),
                            reinterpret_cast<const uint32_t*>(obase + o.block_sums), n, k,
                            lg.shift ? lg.nbx : lg.ntx, lg.shift, slots_a, reinterpret_cast<int32_t*>(vals_a),
                            reinterpret_cast<const int32_t*>(obase + o.ranges), ranges, ready_words,
-                           reinterpret_cast<uint32_t*>(base + w.sort + sw.hist), (int64_t)(sw.bytes / 4), chunk);
+                           reinterpret_cast<uint32_t*>(base + w.sort + clear_from), (int64_t)((sw.bytes - (clear_from - sw.hist)) / 4), chunk, narrow);
     }
     DSX_LAUNCH_CHECK();
     SlotT* ko;
@@ -3367,7 +3410,7 @@ static int tile_lists_impl(const dsx_camera& cam, int64_t n, int64_t k, int num_
     auto partition = [&](auto items, auto digit_bits) {
         return sort32_passes<SlotT, kSortThreads32, decltype(items)::value, false, decltype(digit_bits)::value>(
             k, bits, slots_a, vals_a, slots_b, vals_b, false, kMasks, base + w.sort, "onesweep32_kernel<tile partition>", stream, &ko, &vo,
-            nullptr, nullptr, reinterpret_cast<const uint32_t*>(obase + o.slot_hist));
+            nullptr, nullptr, counts);
     };
 #define DSX_PARTITION_ITEMS(ITEMS)                                                                                     \
     case ITEMS:                                                                                                        \

@@ -138,7 +138,8 @@ int64_t dsx_ranges_count(int32_t width, int32_t height, int32_t list_bin);
  * a tile's entries out of its bin's list by it): 2 k words.  Wherever this header says sorted_ids[k],
  * the buffer has this many words and k is still the number of pairs. */
 int64_t dsx_sorted_ids_count(int64_t k, int32_t width, int32_t height, int32_t list_bin);
-/* bytes of `workspace` dsx_forward_finish / dsx_tile_lists need for k keys */
+/* bytes of `workspace` dsx_forward_finish / dsx_tile_lists need for k keys; enough for any smaller number of keys, and for
+ * any number of Gaussians */
 size_t dsx_workspace_bytes(int64_t n, int64_t k, int32_t width, int32_t height, int32_t list_bin);
 /* bytes of `workspace` dsx_sort_pairs needs for k keys, and dsx_sort_pairs_u32 for count pairs */
 size_t dsx_sort_workspace_bytes(int64_t k, int32_t num_tiles);
