@@ -244,6 +244,8 @@ constexpr int kWideSplitUpTo = 64;        // (a compute unit for each quadrant)
 constexpr int kFwdFourPixelsFrom = 5500;
 constexpr int kBwdFourPixelsFrom = 3000;
 constexpr int kBwdBlocksUpTo = 256; // (lists per tile only, as kFwdWideUpTo)
+constexpr int kBwdBlocksAlways = 100;
+constexpr int64_t kBwdBlocksShared = 3700; // (beyond that many tiles: pairs times tiles, by Gaussian)
 
 // -----------------------------------------------------------------------------------------
 // what both directions share: the pixels, and the walk through the lists
@@ -3051,15 +3053,17 @@ __global__ __launch_bounds__(kTileThreads) void blend_bwd_tile_kernel(
 // which work on four entries at a time: they hand each other alphas and colours, each takes the same steps of what they let through and of
 // what lies behind, and keeps its own entry's; sums over the sixteen pixels by twelve DPP adds and two swaps, one add to
 // LDS for all four entries.  86 instructions for four.  A tile's four quadrants are workgroups of their own, so that 64 tiles reach every
-// compute unit; each stages what reaches its quadrant.  us of the kernel, workgroup form -> this:
-//   Gaussians            3 K opaque   15 K mixed   60 K faint   60 K large   400 K mixed
-//   16 tiles             56 -> 34     177 -> 111   712 -> 427   92 -> 52     168 -> 88
-//   64 tiles             27 -> 19     84 -> 54     269 -> 165   57 -> 35     93 -> 52
-//   144 tiles            22 -> 17     58 -> 39     166 -> 106   54 -> 41     76 -> 50
-//   256 tiles            19 -> 15     48 -> 36     124 -> 90    50 -> 51     62 -> 49
-//   324 tiles            18 -> 16     44 -> 30     116 -> 78    58 -> 59     61 -> 59
-//   400 tiles            19 -> 17     41 -> 33     107 -> 78    57 -> 69     60 -> 62
-// The line lies at 256, a compute unit for each tile; beyond it large Gaussians, to which four workgroups a tile add, lose.
+// compute unit; each stages what reaches its quadrant.  What it costs are four times the adds to memory, which wait for each other where many tiles share
+// a Gaussian.  us of the kernel, workgroup form -> this, 20 K Gaussians, opaque / mixed / faint, by the tiles that one covers:
+//    64 tiles   13  17 -> 14, 44 -> 26, 196 -> 105   28  16 -> 14, 31 -> 21, 181 -> 96
+//   100          9  23 -> 16, 52 -> 34, 146 -> 88    19  17 -> 16, 43 -> 33, 170 -> 104   41  16 -> 15, 28 -> 22, 167 -> 99
+//   144         12  22 -> 19, 50 -> 36, 135 -> 86    25  17 -> 19, 43 -> 36, 163 -> 105   58  15 -> 20, 27 -> 29, 160 -> 111
+//   196         15  22 -> 21, 46 -> 41, 126 -> 80    33  17 -> 23, 41 -> 38, 163 -> 121   77  15 -> 24, 28 -> 35, 152 -> 150
+//   256          8  27 -> 24, 67 -> 48, 57 -> 43     18  22 -> 24, 46 -> 46, 123 -> 90    42  17 -> 27, 39 -> 43, 154 -> 134
+//   324          9  27 -> 26, 63 -> 47, 53 -> 41     22  22 -> 33, 51 -> 58, 115 -> 85    52  19 -> 32, 43 -> 57, 162 -> 157
+//   100 K of 18 at 256 tiles 21 -> 27, 41 -> 51, 183 -> 160; 400 K of 9 at 324 33 -> 37, 63 -> 67, 239 -> 239
+// Up to 100 tiles it is taken always; up to 256, a compute unit for each tile, where pairs times tiles are at most 3700 a Gaussian (14 tiles
+// covered of 256, 26 of 144), between the second and the third column.
 // the two lower halves and the two upper halves of two registers side by side (v_permlane32_swap), and their rows of 16 lanes: the
 // even rows of both and the odd rows of both (v_permlane16_swap)
 __device__ __forceinline__ float add_halves(float a, float b)
@@ -3329,7 +3333,9 @@ int launch_blend_bwd(const dsx_camera& cam, int64_t n, int64_t k, const int32_t*
     hipLaunchKernelGGL((KERNEL), grid, dim3(THREADS), 0, stream, ranges, sorted_ids, sp, final_T, final_idx, v_image, \
                        cam.bg, grads, with_marks ? grad_marks(grads, n) : nullptr, cam.image_width,                 \
                        cam.image_height, ntx, last_id, (int)k, header, lg.shift, camera_flag(cam, DSX_PLANAR_IMAGE), L, Z)
-        const bool blocks = forced_pixels_per_lane() == 0 && lg.shift == 0 && ntx * nty <= kBwdBlocksUpTo;
+        const int tiles = ntx * nty;
+        const bool blocks = forced_pixels_per_lane() == 0 && lg.shift == 0 && tiles <= kBwdBlocksUpTo &&
+                            (tiles <= kBwdBlocksAlways || k * tiles <= kBwdBlocksShared * n);
         if(blocks)
             hipLaunchKernelGGL(blend_bwd_block_kernel, dim3(4 * ntx * nty), dim3(kBlockThreads), 0, stream, ranges, sorted_ids, sp, final_T,
                                final_idx, v_image, cam.bg, grads, with_marks ? grad_marks(grads, n) : nullptr, cam.image_width,

@@ -35,6 +35,13 @@ def test_api_forward_backward_vs_oracle(oracle, blend_form, list_bin, n, W, H, d
                                                           list_bin)
 
 
+@pytest.mark.parametrize("n,W,H,scale_mul", [(1500, 250, 246, 0.1), (1500, 250, 246, 0.5), (1500, 170, 90, 0.5)])
+def test_large_gaussians_vs_oracle(oracle, blend_form, list_bin, n, W, H, scale_mul):
+    """Gaussians that cover some tiles or many: on both sides of the pairs up to which each block has a wavefront."""
+    test_gpu_pipeline.test_api_forward_backward_vs_oracle(oracle, "cfg4", n, W, H, 2, scale_mul, None, "identity", 1, 0, blend_form,
+                                                          list_bin)
+
+
 @pytest.mark.parametrize("W,H", [(211, 197), (64, 48)])
 def test_channel_first_image(oracle, blend_form, list_bin, W, H):
     test_gpu_kernel_edges.test_channel_first_image_in_every_blend_form(oracle, blend_form, list_bin, 0, 1, W, H)
