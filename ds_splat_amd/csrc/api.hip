@@ -776,7 +776,7 @@ static int backward_impl(const dsx_camera* cam, int64_t n, int64_t k, int32_t nu
         return rc;
     return gaussian_bwd_checked(cam, n, num_bases, means3d, scales, quats, splats, cov3d, radii, grads, v_mean3d,
                                 v_means2d, v_shs, v_colors, v_opacity, v_scale, v_quat, v_cov3d, stream,
-                                zeros_alone(*cam, n)  ? ConicFrom::kInputs
+                                conics_again(*cam, n)  ? ConicFrom::kInputs
                                 : grads_prepared != 0 ? ConicFrom::kGrads
                                                       : ConicFrom::kSplats,
                                 true, true);

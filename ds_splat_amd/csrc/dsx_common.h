@@ -468,13 +468,23 @@ int launch_blend_bwd(const dsx_camera& cam, int64_t n, int64_t k, const int32_t*
                      const float* splats, const float* final_T, const int32_t* final_idx, const float* v_image,
                      float* grads, hipStream_t stream, bool check_header, bool grads_prepared = false,
                      bool with_marks = false, const ZeroJobs* zeros = nullptr);
-// Is the accumulator prepared without the conics (DSX_PREPARE_ZEROS)?  Reading them costs the forward time only where there are
-// many: us with them -> without, the forward and the per-Gaussian backward: 300 K Gaussians 112 -> 112 and 14.4 -> 15.9, 500 K 115 -> 116 and
-// 13.9 -> 14.9, 1.4 M 258 -> 255 and 46.5 -> 47.3, 2 M faint 660 -> 636 and 128 -> 130, 3 M 156 -> 126 and 20.3 -> 20.1.
-constexpr int64_t kZerosAloneFrom = 1000000;
+// Does the forward prepare the accumulator without the conics (DSX_PREPARE_ZEROS)?  Reading them costs it time only where there are many.  us of
+// a whole step at 1920x1080, with them -> without, opaque / mixed / faint / large Gaussians, and mixed ones at 1280x720 (runs differ by 1 to 3):
+//   1 M    378 -> 380, 543 -> 546, 1120 -> 1121, 604 -> 606, 533 -> 533    1.7 M  458 -> 444, 584 -> 581, 1877 -> 1869, 640 -> 635, 588 -> 584
+//   1.2 M  400 -> 402, 552 -> 557, 1330 -> 1328, 652 -> 653, 558 -> 558    2 M    497 -> 484, 611 -> 600, 2213 -> 2201, 682 -> 676, 618 -> 608
+//   1.4 M  420 -> 416, 564 -> 565, 1553 -> 1549, 664 -> 662, 571 -> 571    3 M    645 -> 610, 708 -> 681, 3360 -> 3346, 807 -> 790, 723 -> 700
+constexpr int64_t kZerosAloneFrom = 1400000;
+// From how many on the backward does not look for them there, so that an accumulator of zeros alone serves it (0.5 to 1.5 us for working
+// them out again, of 14 to 65)
+constexpr int64_t kConicsAgainFrom = 1000000;
+static_assert(kConicsAgainFrom <= kZerosAloneFrom, "what the forward leaves out the backward does not look for");
 inline bool zeros_alone(const dsx_camera& cam, int64_t n)
 {
     return n >= kZerosAloneFrom && camera_flag(cam, DSX_PREPARE_ZEROS);
+}
+inline bool conics_again(const dsx_camera& cam, int64_t n)
+{
+    return n >= kConicsAgainFrom && camera_flag(cam, DSX_PREPARE_ZEROS);
 }
 // where the per-Gaussian backward finds the conics: in the splat records, in places 9..11 of the accumulator's (dsx_forward_finish put them
 // there), or worked out again, with the projection's own routines (same bits), from what it reads anyway
