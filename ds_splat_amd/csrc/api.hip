@@ -155,16 +155,16 @@ extern "C" size_t dsx_workspace_bytes(int64_t n, int64_t k, int32_t width, int32
     const ListGrid lg = list_grid(width, height, list_bin);
     const bool binned = lg.shift != 0;
     k = std::max<int64_t>(k, 0);
-    // and for any smaller number of pairs: one wide digit, or smaller tiles of keys, take more statuses than what lies behind their limits
-    size_t bytes = 0;
-    auto with = [&](int64_t pairs) {
-        for(const int64_t gaussians : {(int64_t)0, INT64_MAX})
-            bytes = std::max(bytes, lists_workspace(gaussians, pairs, lg.lists(), binned).bytes);
-    };
-    with(k);
-    with(std::min(k, wide_digit_most(slot_bits(lg.lists()), 0, binned)));
-    for(int items = 1; items < kSortItemsMax32; ++items)
-        with(std::min(k, (int64_t)items * kSortThreads32 * kSortTilesWanted32));
+    // and for any smaller number of pairs: one wide digit, or smaller tiles of keys, take more statuses than what lies behind their limits (which
+    // lie beyond the last border of the tiles; at those all have as many tiles, so that the nearest one is the largest)
+    const int lists = lg.lists();
+    const int64_t unit = (int64_t)kSortThreads32 * kSortTilesWanted32, most = wide_digit_most(slot_bits(lists), 0, binned);
+    int64_t border = 0;
+    for(int64_t items = 1; items <= kSortItemsMax32 && items * unit <= k; ++items)
+        border = sort32_items(items * unit) == items ? items * unit : border;
+    size_t bytes = lists_workspace(0, k, lists, binned).bytes;
+    for(const int64_t fewer : {border, std::min(k, most)})
+        bytes = fewer > 0 && fewer < k ? std::max(bytes, lists_workspace(0, fewer, lists, binned).bytes) : bytes;
     return bytes;
 }
 
