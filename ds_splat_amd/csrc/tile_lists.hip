@@ -297,8 +297,8 @@ __device__ __forceinline__ void onesweep32_pass(
 
     // ---- load the keys (striped inside each wavefront: coalesced, order = (item, lane)) -----
     // Registers are what limits the blocks per compute unit here, so a thread keeps little per
-    // item: the key while it is ranked, the rank as 16 bits, the digit as 8 bits; the value is
-    // fetched only once the key registers are free.
+    // item: the key while it is ranked and the rank as 16 bits; the value is fetched only once the key registers are
+    // free.
     uint32_t key[kSort32Items];
     uint32_t pos2[(kSort32Items + 1) / 2]; // two 16-bit positions per register
 #pragma unroll
@@ -629,7 +629,8 @@ __device__ __forceinline__ void onesweep32_pass(
     }
 }
 
-// (eight wavefronts per SIMD: two workgroups per compute unit whatever the tile)
+// (eight wavefronts per SIMD: two workgroups per compute unit with digits of eight and nine bits, whatever the tile, and of ten with up to eight
+// keys a thread; 88 KB of LDS with ten bits and twelve keys, and what eleven bits take, leave room for one)
 template <typename KeyT, int kSort32Threads, int kSort32Items, bool kCarry, int kBits>
 __global__ __launch_bounds__(kSort32Threads) __attribute__((amdgpu_waves_per_eu(8))) void onesweep32_kernel(
     const KeyT* __restrict__ keys_in, const uint32_t* __restrict__ vals_in, KeyT* __restrict__ keys_out,

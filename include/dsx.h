@@ -91,7 +91,7 @@ typedef struct dsx_camera
  *
  * Gradient accumulator record, DSX_GRAD_FLOATS floats:
  *   [0] v_x [1] v_y [2] v_conic_a [3] v_conic_b [4] v_conic_c [5] v_opacity
- *   [6] v_red [7] v_green [8] v_blue [9..11] unused (the conic, once dsx_forward_finish has prepared it)
+ *   [6] v_red [7] v_green [8] v_blue [9..11] unused (the conic or zeros, once dsx_forward_finish has prepared it)
  * The accumulator of the whole backward (dsx_forward_finish's grads_to_prepare, dsx_backward's
  * grads) is a buffer of dsx_grads_bytes(n) bytes, 16-byte aligned: the n records and, behind
  * them, one byte per Gaussian that the blend backward sets when it adds a term to the record.
@@ -111,7 +111,7 @@ size_t dsx_grads_bytes(int64_t n);
 
 /* number of workgroups of the per-Gaussian kernels = entries of `block_sums` */
 int64_t dsx_num_blocks(int64_t n);
-/* tiles of an image, and radix passes the sort runs for that many tiles */
+/* tiles of an image, and radix passes that dsx_sort_pairs runs for that many tiles (dsx_tile_lists sorts otherwise) */
 int32_t dsx_num_tiles(int32_t width, int32_t height);
 int32_t dsx_sort_passes(int32_t num_tiles);
 /* The tile lists of the whole forward (dsx_forward_project / dsx_forward_finish / dsx_backward,
@@ -323,7 +323,8 @@ int dsx_forward_project_counts(const dsx_camera* cam, int64_t n, int64_t* num_ke
  * prepares it on the side (the nine sums zeroed, each Gaussian's conic in the three spare places,
  * the byte per Gaussian behind the records cleared), and that
  * dsx_backward is then called with grads_prepared = 1: it needs no fill of its own and its
- * per-Gaussian kernel does not fetch the splat records for the conic. */
+ * per-Gaussian kernel does not fetch the splat records for the conic.  With DSX_PREPARE_ZEROS the spare places may
+ * be zeros too, where n is large; dsx_backward with the same flag does not read them there. */
 int dsx_forward_finish(const dsx_camera* cam, int64_t n, int64_t k, const float* splats,
                        const void* order, int32_t* sorted_ids, int32_t* ranges, float* image,
                        float* final_T, int32_t* final_idx, void* workspace,
