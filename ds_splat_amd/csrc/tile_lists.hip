@@ -3136,19 +3136,18 @@ __global__ __launch_bounds__(kProjBlock) void emit_ordered_kernel(const uint32_t
     // housekeeping for the partition that follows: its counters and look-back statuses start at zero
     for(int64_t j = (int64_t)blockIdx.x * kProjBlock + tid; j < clear_words; j += (int64_t)gridDim.x * kProjBlock)
         clear[j] = 0u;
-    if(narrow.two && blockIdx.x == 0) // (a workgroup more than there are shares, and the first to start)
-    {
-        narrow_digits(narrow, reinterpret_cast<uint32_t*>(s_rec), tid);
-        return;
-    }
 
     // This workgroup's share: outputs [o0, o1).  The work is cut by OUTPUTS, not by Gaussians: a
     // block of 256 near Gaussians can own a hundred thousand pairs and a block of far ones a few
     // hundred, and a workgroup that walked a whole heavy block alone set the kernel's time.
-    const int64_t o0 = (int64_t)(blockIdx.x - (narrow.two ? 1u : 0u)) * chunk;
+    const int64_t o0 = (int64_t)blockIdx.x * chunk;
     const int64_t o1 = min(o0 + chunk, k);
     if(o0 >= o1) // uniform
+    {
+        if(narrow.two) // (a workgroup more than there are shares)
+            narrow_digits(narrow, reinterpret_cast<uint32_t*>(s_rec), tid);
         return;
+    }
     const int64_t blocks = (n + kProjBlock - 1) / kProjBlock;
     // first block of 256 Gaussians (in depth order) whose outputs reach into the share: the largest
     // b with block_offsets[b] <= o0, by a 64-way search (every wavefront does it for itself)
