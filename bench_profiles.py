@@ -245,11 +245,11 @@ def cmd_sq(args):
              "Commands (on the machine with the MI355X, repository root, after `export TMPDIR=/tmp`):", "",
              "    " + command(SQ_CMD, args.sq_dir, args.workload),
              "    " + command(STATS_CMD, args.stats_dir, args.workload) + "    # the `kernel ms` column", "",
-             "Averages per launch. A wave64 VALU instruction occupies its SIMD for 4 clocks, so the chip (256 CU x 4 SIMD at 2.4 GHz)",
-             "issues at most 614 G wave-instructions/s: `VALU floor` = SQ_INSTS_VALU / 614e9 is the time the kernel's VALU",
-             "instructions alone need (quarter-rate instructions such as exp and rcp count once here, so the true floor is higher);",
-             "`kernel ms` is the launch average of the kernel-trace run.", "",
-             "| kernel | waves | VALU inst / wave | SALU inst / wave | LDS inst / wave | LDS bank-conflict cycles / LDS inst | SQ_INSTS_VALU | VALU floor ms | kernel ms | floor / kernel |",
+             "Averages per launch. `VALU / busy` = SQ_ACTIVE_INST_VALU / SQ_BUSY_CYCLES, both summed over the chip, the one over its 1024 SIMDs and",
+             "the other over its 32 shader engines of 32 SIMDs; `per SIMD` is an eighth of it: vector instructions that a SIMD has",
+             "under way every 4 clocks, the time one of 64 lanes takes at 16 lanes a clock. More than 1 has been read, so 1 is no limit; it",
+             "says how densely a kernel issues, not how fast it could. `kernel ms` is the launch average of the kernel-trace run.", "",
+             "| kernel | waves | VALU inst / wave | SALU inst / wave | LDS inst / wave | LDS bank-conflict cycles / LDS inst | SQ_INSTS_VALU | VALU / busy | per SIMD | kernel ms |",
              "|---|---|---|---|---|---|---|---|---|---|"]
     for k in sorted(d, key=lambda k: -avg(d[k]["SQ_INSTS_VALU"]) if d[k]["SQ_INSTS_VALU"] else 0):
         c = d[k]
@@ -257,10 +257,9 @@ def cmd_sq(args):
             continue
         waves, valu, salu, lds = avg(c["SQ_WAVES"]), avg(c["SQ_INSTS_VALU"]), avg(c["SQ_INSTS_SALU"]), avg(c["SQ_INSTS_LDS"])
         bank = avg(c["SQ_LDS_BANK_CONFLICT"])
-        floor = valu / 614e9 * 1e3
-        lines.append("| %s | %d | %d | %d | %d | %.2f | %.3g | %.3f | %.3f | %.0f %% |" % (
-            k, waves, valu / waves, salu / waves, lds / waves, bank / max(lds, 1), valu, floor, times[k],
-            100 * floor / times[k]))
+        issue = avg(c["SQ_ACTIVE_INST_VALU"]) / avg(c["SQ_BUSY_CYCLES"])
+        lines.append("| %s | %d | %d | %d | %d | %.2f | %.3g | %.2f | %.2f | %.3f |" % (
+            k, waves, valu / waves, salu / waves, lds / waves, bank / max(lds, 1), valu, issue, issue / 8, times[k]))
     write(args.name, lines)
 
 

@@ -1,17 +1,16 @@
 // Stages 4 and 5a for gfx950: per-tile alpha blending, forward (front to back) and backward
 // (back to front).
 //
-// Both directions are bound by the issue of vector instructions: these alone take 82 % of the time where no pixel stops early (2 M
-// faint Gaussians; an exponential or a reciprocal, which takes four times as long, counts once there) and 63 to 82 % elsewhere, so
-// what counts is how many a (pixel, entry) pair costs and how many pairs are looked at that need not be.  The backward
+// What counts is how many vector instructions a (pixel, entry) pair costs and how many pairs are looked at that need not be: the forward has
+// 0.99 to 1.30 of them under way in a SIMD every four clocks, the backward 0.74 to 0.93, and fewer have meant less time.  The backward
 // also waits for its sums: timed without the adds to memory, and then with a place in LDS for each quad of lanes' own sums, one entry at a time,
 // 1 M large Gaussians 300 -> 236 -> 209 us, 3 M 253 -> 252 -> 237, 2 M faint 1281 -> 1238 -> 1184.
 // 1920x1080 unless noted, us within a whole pass (medians of a trace), four lists of entries per wavefront -> sixteen -> with the clamp of alpha where it
-// is needed and plain zeros beside the forward, and two entries at a time in the backward:
-//   forward   2 M faint Gaussians 881 -> 686 -> 630, 1.4 M at 1557x1038 309 -> 266 -> 254, 500 K opaque 127 -> 118 -> 115 (3 M: 149 -> 148 -> 124),
-//             6 M at 3840x2160 509 -> 431 -> 383, 1 M large ones 123 -> 125 -> 106, 1 M at 1280x720 138 -> 120 -> 115
-//   backward  2 M faint 1637 -> 1274 -> 1237, 1.4 M at 1557x1038 519 -> 457 -> 452, 500 K opaque 223 -> 216 -> 207 (3 M: 254 -> 253 -> 243),
-//             1 M large ones 302 -> 306 -> 252, 300 K at 1237x822 244 -> 223 -> 220, 50 K at 512x512 77 -> 72 -> 63
+// is needed and plain zeros beside the forward, and two entries at a time in the backward, without spills:
+//   forward   2 M faint Gaussians 881 -> 686 -> 639, 1.4 M at 1557x1038 309 -> 266 -> 254, 500 K opaque 127 -> 118 -> 115 (3 M: 149 -> 148 -> 125),
+//             6 M at 3840x2160 509 -> 431 -> 380, 1 M large ones 123 -> 125 -> 109, 1 M at 1280x720 138 -> 120 -> 115
+//   backward  2 M faint 1637 -> 1274 -> 1212, 1.4 M at 1557x1038 519 -> 457 -> 438, 500 K opaque 223 -> 216 -> 201 (3 M: 254 -> 253 -> 234),
+//             1 M large ones 302 -> 306 -> 252 to 302, 300 K at 1237x822 244 -> 223 -> 206, 50 K at 512x512 77 -> 72 -> 61
 #include "dsx_common.h"
 
 #include <atomic>
@@ -721,7 +720,8 @@ __global__ __launch_bounds__(DSX_WAVE) __attribute__((amdgpu_waves_per_eu(7, 7))
                 }
                 // (only where an entry of the round can reach the clamp: four of some 66 instructions an entry.  A branch costs less here than
                 // a second walk without the clamp, which does not fit the registers; 6 M Gaussians at 3840x2160 401 -> 381 us, 1.4 M at
-                // 1557x1038 266 -> 257, 500 K opaque 122 -> 117, 2 M faint 671 -> 660)
+                // 1557x1038 266 -> 257, 500 K opaque 122 -> 117, 2 M faint 671 -> 660.  Where nearly every round has one, against a clamp without the
+                // branch: 500 K of which half reach beyond 0.99 91 -> 94, all 82 -> 84, 6 M 182 -> 188, 1.4 M 79 -> 82)
                 if(__builtin_expect(clamps, 0))
                 {
                     // (a NaN opacity gives 0.999, as in the reference: fminf drops the NaN)
